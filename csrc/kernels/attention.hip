@@ -1029,7 +1029,8 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
                                long long k_st, long long k_sh, long long v_sb, long long v_st,
                                long long v_sh, long long o_sb, long long o_st, long long o_sh,
                                int B, int Sq, int Sk, int H, int Hkv, int d, int causal,
-                               float scale, int rowsum_col, int max_col, int* flags, hipStream_t stream);
+                               float scale, const float* alibi, const int* kv_len, int window, int rowsum_col,
+                               int max_col, int* flags, hipStream_t stream);
 
 // workspace: >= 4 * ceil(Sq/128) * B * H ints for the full-tile fast path of
 // attention_tiled.hip (its overflow flags), or null for the generic kernel.
@@ -1052,10 +1053,10 @@ KCA_API int kca_attn_fwd(const void* q, const void* k, const void* v, void* o,
                q_sb, q_st, q_sh, k_sb, k_st, k_sh, v_sb, v_st, v_sh, o_sb, o_st, o_sh,
                B, Sq, Sk, H, Hkv, d_real, causal, scale, alibi, kv_len, nullptr,
                window, key_mask, (Sk + 31) / 32};
-  if (g_attn_tiled && workspace && !alibi && !kv_len && !window && !key_mask &&
+  if (g_attn_tiled && workspace && !key_mask &&
       kca_attn_fwd_tiled(q, k, v, o, lse, q_sb, q_st, q_sh, k_sb, k_st, k_sh, v_sb, v_st, v_sh,
-                         o_sb, o_st, o_sh, B, Sq, Sk, H, Hkv, d_real, causal, scale, rowsum_col, max_col,
-                         workspace, stream) == 0)
+                         o_sb, o_st, o_sh, B, Sq, Sk, H, Hkv, d_real, causal, scale, alibi, kv_len, window,
+                         rowsum_col, max_col, workspace, stream) == 0)
     p.fix_flags = workspace;  // fixup launch below: only flagged blocks do work
   dim3 grid(((Sq + 127) / 128) * B * H);
   ATTN_D_DISPATCH(D, {
@@ -1093,7 +1094,8 @@ KCA_API int kca_attn_bwd_tiled(const void* q, const void* k, const void* v, cons
                                long long dq_sb, long long dq_st, long long dq_sh, long long dk_sb,
                                long long dk_st, long long dk_sh, long long dv_sb, long long dv_st,
                                long long dv_sh, int B, int Sq, int Sk, int H, int Hkv, int d,
-                               int causal, float scale, hipStream_t stream);
+                               int causal, float scale, const float* alibi, const int* kv_len, int window,
+                               hipStream_t stream);
 
 KCA_API int kca_attn_bwd(const void* q, const void* k, const void* v,
                          const void* o, const void* dout, void* dq, void* dk,
@@ -1109,11 +1111,11 @@ KCA_API int kca_attn_bwd(const void* q, const void* k, const void* v,
                          int causal, float scale, const float* alibi,
                          const int* kv_len, int window, const unsigned* key_mask, hipStream_t stream) {
   if (d_real % 8 || H % Hkv || window < 0) return 1;
-  if (g_attn_tiled && !alibi && !kv_len && !window && !key_mask &&
+  if (g_attn_tiled && !key_mask &&
       kca_attn_bwd_tiled(q, k, v, dout, dq, dk, dv, lse, delta, q_sb, q_st, q_sh, k_sb, k_st, k_sh,
                          v_sb, v_st, v_sh, do_sb, do_st, do_sh, dq_sb, dq_st, dq_sh, dk_sb, dk_st,
-                         dk_sh, dv_sb, dv_st, dv_sh, B, Sq, Sk, H, Hkv, d_real, causal, scale,
-                         stream) == 0)
+                         dk_sh, dv_sb, dv_st, dv_sh, B, Sq, Sk, H, Hkv, d_real, causal, scale, alibi, kv_len,
+                         window, stream) == 0)
     return 0;
   const int D = pick_d(d_real);
   AttnBwdParams p{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)o,

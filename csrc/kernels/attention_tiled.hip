@@ -1,10 +1,13 @@
-// Flash attention forward + backward, full-tile fast path for head_dim 64 / 96 / 128 / 160 / 256 (K2).
+// Flash attention forward + backward, fast path for head_dim 64 / 96 / 128 / 160 / 256 (K2).
 //
-// The generic kernels in attention.hip handle every shape (ALiBi, per-batch
-// key lengths, ragged tiles, padded head dims). This file holds the path the
-// GPT-J / NeoX-class training step actually runs -- causal or not, Sq % 128 ==
-// 0, Sk % 32 == 0, d == D -- written around one rule: no per-tile address
-// arithmetic and no guards inside the key loop.
+// The generic kernels in attention.hip handle every shape (key bitmaps, padded head dims). This file holds
+// the path that training and prompts actually run, written around one rule: no per-tile address arithmetic
+// and no guards inside the key loop. Two forms of every kernel (template argument G):
+//   0  causal or not, Sq % 128 == 0, Sk % 32 (backward: 128) == 0, no other mask
+//   1  any number of queries and keys, per-batch key lengths, a sliding window;  2  the same with ALiBi
+// The general forms keep the loop free of guards by other means: K / V (dK/dV: Q / dO) tiles come through
+// buffer resources that end with the sequence's last valid row, so that what lies beyond reads as zeros; and
+// only tiles at the edges of a workgroup's band run the masked body.
 //
 // LDS image (cdna_hip_programming.md §5.5 T10, image (a)): a tile of 32 rows x
 // D bf16 is stored as 8-row x 32-column sub-tiles of 512 B,
@@ -74,15 +77,44 @@ struct FastFwdParams {
   long long o_sb, o_st, o_sh;
   int B, Sq, Sk, H, Hkv;
   float scale;
+  const float* alibi;  // [H] slopes (G = 2)
+  const int* kv_len;   // [B] or null (G > 0)
+  int window;          // > 0: key visible only if key > q + off - window (G > 0)
 };
 
+constexpr int kAllRows = 0x7fffffff;
+
 // buffer resource over one (batch, head) slice; the base is workgroup-uniform (readfirstlane'd so
-// the descriptor is provably scalar: no waterfall loop, T20)
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t head_rsrc(const bf16_t* b) {
+// the descriptor is provably scalar: no waterfall loop, T20). `bytes`: loads at or past it return zeros.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t head_rsrc(const bf16_t* b, int bytes = kAllRows) {
   const unsigned long long a = (unsigned long long)b;
   const unsigned long long au = ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(a >> 32)) << 32) |
                                 (unsigned)__builtin_amdgcn_readfirstlane((unsigned)a);
-  return __builtin_amdgcn_make_buffer_rsrc((void*)au, (short)0, 0x7fffffff, 0x00020000);
+  return __builtin_amdgcn_make_buffer_rsrc((void*)au, (short)0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+}
+// bytes of `rows` rows of D elements, `st` elements apart
+__device__ __forceinline__ int rows_bytes(int rows, long long st, int D) {
+  return rows > 0 ? (int)(((rows - 1) * st + D) * 2) : 0;
+}
+
+// The 32-key tiles of a workgroup's query rows [r0, r0 + BM) in the general forms: it walks tiles [lo, hi),
+// of which [f_lo, f_hi] need no mask. A row's last visible key lies in a tile above f_hi. At least one tile,
+// also where no key is visible (a length of 0): its mask gives zeros.
+struct TileSpan { int lo, hi, f_lo, f_hi; };
+template <int BM, bool CAUSAL>
+__device__ __forceinline__ TileSpan tile_span(int r0, int off, int kv_end, int window) {
+  TileSpan s;
+  s.hi = max(1, ((CAUSAL ? min(kv_end, r0 + BM + off) : kv_end) + 31) / 32);
+  s.f_hi = (CAUSAL ? min(r0 + off, kv_end - 1) : kv_end - 1) / 32 - 1;
+  s.lo = s.f_lo = 0;
+  if (window > 0) {
+    s.lo = min(s.hi - 1, max(0, r0 + off - window + 1) / 32);
+    s.f_lo = max(0, r0 + BM + off - window + 31) / 32;
+  }
+  return s;
+}
+__device__ __forceinline__ int batch_keys(const int* kv_len, int b, int Sk) {
+  return kv_len ? max(0, min(Sk, kv_len[b])) : Sk;
 }
 
 // Staging of a 32-row x D tile by the 256 threads of a workgroup: chunk idx = tid + 256*i is
@@ -110,18 +142,20 @@ struct Stager<D, true> {
   }
   // kb / vb: the (batch, kv head) base pointers -- workgroup-uniform (readfirstlane'd so the
   // descriptor is provably scalar: no waterfall loop, T20). Offsets stay < 2^31 bytes per head slice.
-  __device__ __forceinline__ void bind(const bf16_t* kb, const bf16_t* vb, long long k_st, long long v_st) {
+  __device__ __forceinline__ void bind(const bf16_t* kb, const bf16_t* vb, long long k_st, long long v_st,
+                                       int kn = kAllRows, int vn = kAllRows) {
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
       vok_[i] = (int)((ok_ + (long long)i * RPI * k_st) * 2);
       vov_[i] = (int)((ov_ + (long long)i * RPI * v_st) * 2);
     }
-    set_base(kb, vb);
+    set_base(kb, vb, kn, vn);
   }
   // scalar work only: a kernel whose base changes per tile (dK/dV over GQA query heads) rebinds it
-  __device__ __forceinline__ void set_base(const bf16_t* kb, const bf16_t* vb) {
-    rk_ = head_rsrc(kb);
-    rv_ = head_rsrc(vb);
+  // (kn, vn: bytes of the valid rows)
+  __device__ __forceinline__ void set_base(const bf16_t* kb, const bf16_t* vb, int kn = kAllRows, int vn = kAllRows) {
+    rk_ = head_rsrc(kb, kn);
+    rv_ = head_rsrc(vb, vn);
   }
   __device__ __forceinline__ void load(u32x4 (&sk)[CPT], u32x4 (&sv)[CPT], const bf16_t* kb, const bf16_t* vb,
                                        int k0, long long k_st, long long v_st) const {
@@ -152,30 +186,39 @@ template <int D>
 struct Stager<D, false> {
   static constexpr int NCH = D / 8, TOT = 32 * NCH, CPT = (TOT + 255) / 256;
   static_assert(D % 32 == 0 && TOT % 64 == 0, "tiled attention: D multiple of 32");
-  long long ok_[CPT], ov_[CPT];
+  int vok_[CPT], vov_[CPT];
   int lds_[CPT];
   bool tail_;  // this thread owns a chunk in the last, partial round
+  __amdgpu_buffer_rsrc_t rk_, rv_;
   __device__ __forceinline__ Stager(int tid, long long k_st, long long v_st) {
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
       const int idx = min(tid + 256 * i, TOT - 1);
       const int row = idx / NCH, ch = idx % NCH;
-      ok_[i] = (long long)row * k_st + ch * 8;
-      ov_[i] = (long long)row * v_st + ch * 8;
+      vok_[i] = (int)(((long long)row * k_st + ch * 8) * 2);
+      vov_[i] = (int)(((long long)row * v_st + ch * 8) * 2);
       lds_[i] = img_off<D>(row, ch);
     }
     tail_ = tid + 256 * (CPT - 1) < TOT;
   }
-  __device__ __forceinline__ void bind(const bf16_t*, const bf16_t*, long long, long long) {}
-  __device__ __forceinline__ void set_base(const bf16_t*, const bf16_t*) {}
-  __device__ __forceinline__ void load(u32x4 (&sk)[CPT], u32x4 (&sv)[CPT], const bf16_t* kb, const bf16_t* vb,
+  __device__ __forceinline__ void bind(const bf16_t* kb, const bf16_t* vb, long long, long long, int kn = kAllRows,
+                                       int vn = kAllRows) {
+    set_base(kb, vb, kn, vn);
+  }
+  __device__ __forceinline__ void set_base(const bf16_t* kb, const bf16_t* vb, int kn = kAllRows, int vn = kAllRows) {
+    rk_ = head_rsrc(kb, kn);
+    rv_ = head_rsrc(vb, vn);
+  }
+  __device__ __forceinline__ void load(u32x4 (&sk)[CPT], u32x4 (&sv)[CPT], const bf16_t*, const bf16_t*,
                                        int k0, long long k_st, long long v_st) const {
-    const bf16_t* kr = kb + (long long)k0 * k_st;
-    const bf16_t* vr = vb + (long long)k0 * v_st;
+    const int sok = __builtin_amdgcn_readfirstlane((int)(k0 * k_st * 2));
+    const int sov = __builtin_amdgcn_readfirstlane((int)(k0 * v_st * 2));
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {  // a clamped tail chunk re-reads a valid chunk (never stored)
-      sk[i] = *reinterpret_cast<const u32x4*>(kr + ok_[i]);
-      sv[i] = *reinterpret_cast<const u32x4*>(vr + ov_[i]);
+      const auto a = __builtin_amdgcn_raw_buffer_load_b128(rk_, vok_[i], sok, 0);
+      const auto b = __builtin_amdgcn_raw_buffer_load_b128(rv_, vov_[i], sov, 0);
+      sk[i] = *reinterpret_cast<const u32x4*>(&a);
+      sv[i] = *reinterpret_cast<const u32x4*>(&b);
     }
   }
   __device__ __forceinline__ void store(const u32x4 (&sk)[CPT], const u32x4 (&sv)[CPT], char* buf) const {
@@ -207,10 +250,13 @@ struct StagerNarrow {
     lds_ = img_off<D>(row, ch);
     on_ = tid < TOT;
   }
-  __device__ __forceinline__ void bind(const bf16_t* kb, const bf16_t* vb, long long, long long) { set_base(kb, vb); }
-  __device__ __forceinline__ void set_base(const bf16_t* kb, const bf16_t* vb) {
-    rk_ = head_rsrc(kb);
-    rv_ = head_rsrc(vb);
+  __device__ __forceinline__ void bind(const bf16_t* kb, const bf16_t* vb, long long, long long, int kn = kAllRows,
+                                       int vn = kAllRows) {
+    set_base(kb, vb, kn, vn);
+  }
+  __device__ __forceinline__ void set_base(const bf16_t* kb, const bf16_t* vb, int kn = kAllRows, int vn = kAllRows) {
+    rk_ = head_rsrc(kb, kn);
+    rv_ = head_rsrc(vb, vn);
   }
   __device__ __forceinline__ void load(u32x4 (&sk)[1], u32x4 (&sv)[1], const bf16_t*, const bf16_t*, int k0,
                                        long long k_st, long long v_st) const {
@@ -237,9 +283,10 @@ using StagerFor = std::conditional_t<DS == D, Stager<D>, StagerNarrow<D, DS>>;
 // so the per-lane 8-B writes and the row-contiguous 16-B reads are both conflict-free -- and every
 // store instruction then writes two whole rows with 16-B stores, instead of 8-B stores that each
 // touch 64 rows. `mul` is the lane's row scale. The LDS must be free (after the loop's barrier).
-template <int D, int DS = D>
+// EDGE: only the first `rows` rows exist.
+template <int D, int DS = D, bool EDGE = false>
 __device__ __forceinline__ void store_tile_lds(bf16_t* row0, long long st, const f32x16 (&acc)[D / 32], int lane,
-                                               float mul, char* lds) {
+                                               float mul, char* lds, int rows = 32) {
   constexpr int NCH = D / 8, RB = D * 2, NCS = DS / 8;  // NCS: stored chunks per row
   const int l32 = lane & 31, hh = lane >> 5;
 #pragma unroll
@@ -258,7 +305,7 @@ __device__ __forceinline__ void store_tile_lds(bf16_t* row0, long long st, const
   for (int j = 0; j < 32 * NCS / 64; ++j) {
     const int idx = j * 64 + lane, r = idx / NCS, c = idx % NCS;
     const uint4 v = *reinterpret_cast<const uint4*>(lds + r * RB + ((c + r) % NCH) * 16);
-    *reinterpret_cast<uint4*>(row0 + (long long)r * st + c * 8) = v;
+    if (!EDGE || r < rows) *reinterpret_cast<uint4*>(row0 + (long long)r * st + c * 8) = v;
   }
   asm volatile("" ::: "memory");
 }
@@ -272,8 +319,12 @@ __device__ __forceinline__ void store_tile_lds(bf16_t* row0, long long st, const
 // column MC set to 1.0 (the SD UNet folds both into its padded QKV weights), and the kernel writes
 // -m into Q's column MC in registers once m is known, so the S MFMAs return s * log2(e) - m and
 // P = exp2(S) needs no per-element FMA: the D <= 64 loop is bound by that VALU work, not the MFMAs.
-template <int D, bool CAUSAL, int OC = -1, int DS = D, int MC = -1>
+// G > 0 walks the tiles from the last to the first: every row's last visible key -- with ALiBi the one with the
+// least bias, with a window or a length one that surely exists -- then lies in one of the first, masked tiles,
+// whose row max is the reference (below).
+template <int D, bool CAUSAL, int OC = -1, int DS = D, int MC = -1, int G = 0>
 __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1)) attn_fwd_tiled_kernel(FastFwdParams p) {
+  static_assert(G == 0 || (OC < 0 && MC < 0 && DS == D && D < 256), "general form: plain heads");
   constexpr int BM = 128, BN = 32;
   constexpr int TILE = BN * D * 2;           // bytes per K or V tile (LDS image)
   constexpr int KS = DS / 16;                // S MFMA steps
@@ -284,7 +335,7 @@ __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1)) attn_fwd_tiled_kernel
   ASTAMP_DECL
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5, gi = lane & 15;
-  const int nqb = p.Sq / BM;
+  const int nqb = (p.Sq + BM - 1) / BM;
   const int lid = xcd_remap(blockIdx.x, gridDim.x);
   const int qi = lid % nqb;
   const int qb = CAUSAL ? (nqb - 1 - qi) : qi;
@@ -294,9 +345,13 @@ __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1)) attn_fwd_tiled_kernel
   const int off = p.Sk - p.Sq;
   const int q0 = qb * BM + wave * 32;
   const int qrow = q0 + l32;
-  int kv_hi = p.Sk;
+  const int kv_end = G ? batch_keys(p.kv_len, b, p.Sk) : p.Sk;
+  int kv_hi = kv_end;
   if (CAUSAL) kv_hi = min(kv_hi, qb * BM + BM + off);
-  const int ntiles = kv_hi > 0 ? (kv_hi + BN - 1) / BN : 0;
+  TileSpan sp{};
+  if constexpr (G > 0) sp = tile_span<BM, CAUSAL>(qb * BM, off, kv_end, p.window);
+  const int ntiles = G ? sp.hi - sp.lo : kv_hi > 0 ? (kv_hi + BN - 1) / BN : 0;
+  auto key0 = [&](int t) { return G ? (sp.hi - 1 - t) * BN : t * BN; };  // first key of the t-th tile walked
   static_assert(MC < 0 || (!CAUSAL && OC >= 0 && MC < DS), "max column: non-causal, with the row-sum column");
   const float sl2 = MC >= 0 ? 1.f : p.scale * kLog2e;
 
@@ -309,18 +364,21 @@ __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1)) attn_fwd_tiled_kernel
   bf16x8 qf[KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s)
-    qf[s] = *reinterpret_cast<const bf16x8*>(qp + (long long)qrow * p.q_st + 16 * s + 8 * hh);
+    qf[s] = *reinterpret_cast<const bf16x8*>(qp + (long long)(G ? min(qrow, p.Sq - 1) : qrow) * p.q_st + 16 * s + 8 * hh);
 
   f32x16 oacc[D / 32];
 #pragma unroll
   for (int i = 0; i < D / 32; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[i][r] = 0.f;
-  float m = 0.f, lsum = 0.f;  // m: reference max (log2 units), set by tile 0
+  // m: reference max (log2 units), set by tile 0 (G: by a row's first tile with a visible key)
+  float m = G ? -INFINITY : 0.f, lsum = 0.f;
+  const float slope = G == 2 ? p.alibi[h] * kLog2e : 0.f;
 
   // staging: thread handles chunks idx = tid + i*256 (Stager)
   Stg stg(tid, p.k_st, p.v_st);
-  stg.bind(kp, vp, p.k_st, p.v_st);
+  if constexpr (G > 0) stg.bind(kp, vp, p.k_st, p.v_st, rows_bytes(kv_end, p.k_st, D), rows_bytes(kv_end, p.v_st, D));
+  else stg.bind(kp, vp, p.k_st, p.v_st);
   u32x4 sk[CPT], sv[CPT];
   if constexpr (DS < D) {  // V image chunks DS/8.. (read by the PV d-blocks, never loaded): zero once
     constexpr int PC = D / 8 - DS / 8, NZ = 3 * 32 * PC;
@@ -338,7 +396,7 @@ __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1)) attn_fwd_tiled_kernel
   const int vb_1 = 64 * (4 * hh + (gi >> 2)) + 16 * (c3 ^ hh) + 8 * (gi & 1);
   const int vb_2 = 16 * D + 64 * (4 * hh + (gi >> 2)) + 16 * (c3 ^ hh ^ 2) + 8 * (gi & 1);
 
-  // ntiles >= 1 on this path (Sk >= 32; causal: Sk >= Sq)
+  // ntiles >= 1 on this path (Sk >= 32; causal: Sk >= Sq; G: tile_span)
   // Software pipeline over 32-key tiles, three LDS buffers: while the softmax
   // of tile t runs on the VALU, the S^T MFMAs of tile t+1 run on the matrix
   // pipe (independent instructions the scheduler interleaves, T15), then
@@ -367,29 +425,33 @@ __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1)) attn_fwd_tiled_kernel
   // causal: keys past this lane's query -> -inf. sacc[r] holds key
   // k0 + (r&3) + 8(r>>2) + 4hh of query qrow. Tiles wholly above a wave's rows
   // are masked, not skipped (a skip puts O in a conditional region: spills).
+  const int last = G ? (CAUSAL ? min(qrow + off, kv_end - 1) : kv_end - 1) : qrow + off;  // row's last visible key
+  const int before = G && p.window > 0 ? qrow + off - p.window : -(1 << 30);              // key before its first
   auto mask = [&](f32x16& acc, int k0) {
-    const int lim = qrow + off - k0 - 4 * hh;
+    const int lim = last - k0 - 4 * hh, lo = before - k0 - 4 * hh;
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-      if ((r & 3) + 8 * (r >> 2) > lim) acc[r] = -INFINITY;
+    for (int r = 0; r < 16; ++r) {
+      const int c = (r & 3) + 8 * (r >> 2);
+      if (c > lim || (G && c <= lo)) acc[r] = -INFINITY;
+    }
   };
 
-  stg.load(sk, sv, kp, vp, 0, p.k_st, p.v_st);
+  stg.load(sk, sv, kp, vp, key0(0), p.k_st, p.v_st);
   stg.store(sk, sv, smem);
-  stg.load(sk, sv, kp, vp, min(BN, (ntiles - 1) * BN), p.k_st, p.v_st);
+  stg.load(sk, sv, kp, vp, key0(min(1, ntiles - 1)), p.k_st, p.v_st);
   stg.store(sk, sv, smem + 2 * TILE);
   // D = 256 (one wave per SIMD, no other wave to cover a load): two tiles of K/V loads in flight
   // in registers; tile 2 goes into set 0 before the loop (stored at the end of iteration 0).
   // GPT-J fwd 0.563 -> 0.535 ms; at D = 160 it measured 3-4 % slower (profiles/attn_stamps_r2.md)
   constexpr bool PF2 = D >= 256;
   u32x4 sk2[CPT], sv2[CPT];
-  if constexpr (PF2) stg.load(sk, sv, kp, vp, min(2 * BN, (ntiles - 1) * BN), p.k_st, p.v_st);
+  if constexpr (PF2) stg.load(sk, sv, kp, vp, key0(min(2, ntiles - 1)), p.k_st, p.v_st);
   __syncthreads();
 
   const int nfree = CAUSAL ? ntiles - 4 : ntiles;  // tiles no wave needs masked
   f32x16 sa = qk(smem);
-  if (CAUSAL && nfree <= 0) mask(sa, 0);
-  {
+  if (!G && CAUSAL && nfree <= 0) mask(sa, 0);
+  if constexpr (G == 0) {
     // No running max and no O rescale: the reference max m is the row max of
     // the first tile and stays fixed. Floating point is scale invariant, so
     // P = 2^(s - m) only needs to stay finite -- it can exceed 1 when a later
@@ -412,7 +474,7 @@ __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1)) attn_fwd_tiled_kernel
 #pragma unroll
     for (int r = 0; r < 16; ++r) sa[r] -= m;
   }
-  const float nm = -m;
+  float nm = G ? 0.f : -m;
   ASTAMP(0);
 
   auto tile_step = [&](int t, auto masked, auto par) {
@@ -428,20 +490,42 @@ __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1)) attn_fwd_tiled_kernel
     u32x4(&ldv)[CPT] = (PF2 && !ODD) ? sv2 : sv;
     u32x4(&stk)[CPT] = ODD ? sk2 : sk;
     u32x4(&stv)[CPT] = ODD ? sv2 : sv;
-    stg.load(ldk, ldv, kp, vp, min((t + (PF2 ? 3 : 2)) * BN, (ntiles - 1) * BN), p.k_st, p.v_st);
+    stg.load(ldk, ldv, kp, vp, key0(min(t + (PF2 ? 3 : 2), ntiles - 1)), p.k_st, p.v_st);
     ASTAMP(1);
     // keep the staging loads above and the LDS stores below on their own
     // sides of the MFMAs (without the fences hipcc stores each load right
     // after it, behind a vmcnt(0))
     asm volatile("" ::: "memory");
     f32x16 sb = qk(Kn);  // S of tile t+1 (stale buffer on the last tile: unused)
-    if constexpr (MASKED) mask(sa, t * BN);
+    float sl = sl2, bias[16];  // P = exp2(s * sl + bias)
+    if constexpr (G == 2) {
+      const float b0 = slope * (float)(key0(t) + 4 * hh - qrow - off) + (MASKED ? 0.f : nm);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bias[r] = fmaf(slope, (float)((r & 3) + 8 * (r >> 2)), b0);
+    }
+    if constexpr (MASKED) mask(sa, key0(t));
+    if constexpr (G > 0 && MASKED) {
+      float mt = -INFINITY;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        sa[r] = G == 2 ? fmaf(sa[r], sl2, bias[r]) : sa[r] * sl2;
+        mt = fmaxf(mt, sa[r]);
+      }
+      mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+      m = m == -INFINITY ? mt : m;
+      nm = m == -INFINITY ? 0.f : -m;
+      sl = 1.f;
+    }
+    if constexpr (G < 2 || MASKED) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bias[r] = nm;
+    }
     float ps = 0.f;
     bf16x8 pf0, pf1;
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-      const float e0 = __builtin_amdgcn_exp2f(MC >= 0 ? sa[r] : fmaf(sa[r], sl2, nm));
-      const float e1 = __builtin_amdgcn_exp2f(MC >= 0 ? sa[r + 8] : fmaf(sa[r + 8], sl2, nm));
+      const float e0 = __builtin_amdgcn_exp2f(MC >= 0 ? sa[r] : fmaf(sa[r], sl, bias[r]));
+      const float e1 = __builtin_amdgcn_exp2f(MC >= 0 ? sa[r + 8] : fmaf(sa[r + 8], sl, bias[r + 8]));
       if constexpr (OC < 0) ps += e0 + e1;
       pf0[r] = (__bf16)e0;
       pf1[r] = (__bf16)e1;
@@ -492,6 +576,11 @@ __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1)) attn_fwd_tiled_kernel
     tile_step(t + 1, std::true_type{}, std::true_type{});
   }
   if (t < ntiles) tile_step(t, std::true_type{}, std::false_type{});
+  } else if constexpr (G > 0) {
+    const int top = min(ntiles, sp.hi - 1 - sp.f_hi), low = max(top, min(ntiles, sp.hi - sp.f_lo));
+    for (int t = 0; t < top; ++t) tile_step(t, std::true_type{}, std::false_type{});
+    for (int t = top; t < low; ++t) tile_step(t, std::false_type{}, std::false_type{});
+    for (int t = low; t < ntiles; ++t) tile_step(t, std::true_type{}, std::false_type{});
   } else {
   for (int t = 0; t < nfree; ++t) tile_step(t, std::false_type{}, std::false_type{});
   for (int t = max(nfree, 0); t < ntiles; ++t) tile_step(t, std::true_type{}, std::false_type{});
@@ -510,14 +599,14 @@ __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1)) attn_fwd_tiled_kernel
   }
   // row sums past 2^100 (or inf / NaN) mean P may have overflowed: flag the
   // wave for the generic-kernel fixup (which then rewrites O and lse)
-  const bool bad = !(ltot < 1.2676506e30f);
+  const bool bad = !(ltot < 1.2676506e30f) && (!G || qrow < p.Sq);
   const int any_bad = __any(bad);
   if (lane == 0) p.flags[lid * 4 + wave] = any_bad;
   const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
-  if (hh == 0 && p.lse)
+  if (hh == 0 && p.lse && (!G || qrow < p.Sq))
     p.lse[((long long)b * p.H + h) * p.Sq + qrow] = ltot > 0.f ? (m + log2f(ltot)) * kLn2 : INFINITY;
-  store_tile_lds<D, DS>(p.o + b * p.o_sb + h * p.o_sh + (long long)q0 * p.o_st, p.o_st, oacc, lane, inv,
-                        smem + wave * 32 * D * 2);
+  store_tile_lds<D, DS, (G > 0)>(p.o + b * p.o_sb + h * p.o_sh + (long long)q0 * p.o_st, p.o_st, oacc, lane, inv,
+                                 smem + wave * 32 * D * 2, p.Sq - q0);
   ASTAMP(5);
   ASTAMP_FLUSH(0);
 }
@@ -591,7 +680,7 @@ __device__ __forceinline__ bf16x8 as_bf8(u32x2 lo, u32x2 hi) {
 // SIMD, O^T = 256 registers, Q^T fragments 128; two 64-KiB stages, the next tile's DMA in flight
 // under the current tile). Inference only: the overflow flags go back to the caller, which has no
 // generic D = 512 kernel to fix rows up with and reruns flagged calls on the GEMM path.
-template <int D, bool CAUSAL, int NW = 8, int NBUF = 4>
+template <int D, bool CAUSAL, int NW = 8, int NBUF = 4, int G = 0>
 __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p) {
   constexpr int BM = NW * 32, BN = 32;
   constexpr int TILE = BN * D * 2;            // one K or V image
@@ -610,7 +699,7 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hh = lane >> 5;
-  const int nqb = p.Sq / BM;
+  const int nqb = (p.Sq + BM - 1) / BM;
   const int lid = xcd_remap(blockIdx.x, gridDim.x);
   const int qi = lid % nqb;
   const int qb = CAUSAL ? (nqb - 1 - qi) : qi;
@@ -620,9 +709,16 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
   const int off = p.Sk - p.Sq;
   const int q0 = qb * BM + wave * 32;
   const int qrow = q0 + l32;
-  int kv_hi = p.Sk;
+  const int kv_end = G ? batch_keys(p.kv_len, b, p.Sk) : p.Sk;
+  int kv_hi = kv_end;
   if (CAUSAL) kv_hi = min(kv_hi, qb * BM + BM + off);
-  const int ntiles = kv_hi / BN;
+  TileSpan sp{}, own{};  // G: of the workgroup, of this wave's rows (which walk the same order, tile_span)
+  if constexpr (G > 0) {
+    sp = tile_span<BM, CAUSAL>(qb * BM, off, kv_end, p.window);
+    own = tile_span<32, CAUSAL>(q0, off, kv_end, p.window);
+    if (q0 >= p.Sq) own.hi = 0;
+  }
+  const int ntiles = G ? sp.hi - sp.lo : kv_hi / BN;
   const int mytiles = CAUSAL ? min(ntiles, (q0 + 32 + off) / BN) : ntiles;
   const float sl2 = p.scale * kLog2e;
 
@@ -630,13 +726,15 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
   bf16x8 qf[KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s)
-    qf[s] = *reinterpret_cast<const bf16x8*>(qp + (long long)qrow * p.q_st + 16 * s + 8 * hh);
+    qf[s] = *reinterpret_cast<const bf16x8*>(qp + (long long)(G ? min(qrow, p.Sq - 1) : qrow) * p.q_st + 16 * s + 8 * hh);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // Q landed before any DMA is counted
 
   // LDS-DMA sources: piece j of an image covers image bytes [1024 j, 1024 j + 1024); lane L writes
   // byte 1024 j + 16 L, i.e. (row, chunk) = img_off^-1 of it
-  const __amdgpu_buffer_rsrc_t rk = head_rsrc(p.k + b * p.k_sb + hk * p.k_sh);
-  const __amdgpu_buffer_rsrc_t rv = head_rsrc(p.v + b * p.v_sb + hk * p.v_sh);
+  const __amdgpu_buffer_rsrc_t rk =
+      head_rsrc(p.k + b * p.k_sb + hk * p.k_sh, G ? rows_bytes(kv_end, p.k_st, D) : kAllRows);
+  const __amdgpu_buffer_rsrc_t rv =
+      head_rsrc(p.v + b * p.v_sb + hk * p.v_sh, G ? rows_bytes(kv_end, p.v_st, D) : kAllRows);
   // A wave's PPW pieces lie in one 8-row group (D / 64 pieces per group), piece i of them 2 sub-tiles
   // = 8 chunks = 128 source bytes after piece 0: one per-lane offset, the rest a scalar add
   static_assert((D / 64) % PPW == 0, "a wave's pieces within one row group");
@@ -653,7 +751,8 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
   typedef __attribute__((address_space(3))) char lds_char;
   lds_char* lsm = (lds_char*)smem;
   auto issue = [&](int tile, int buf) {
-    const int kt = min(tile, ntiles - 1);  // clamped: the last tiles re-load a tile nobody reads
+    int kt = min(tile, ntiles - 1);  // clamped: the last tiles re-load a tile nobody reads
+    if constexpr (G > 0) kt = sp.hi - 1 - kt;
     const int sok = __builtin_amdgcn_readfirstlane(kt * BN * (int)p.k_st * 2);
     const int sov = __builtin_amdgcn_readfirstlane(kt * BN * (int)p.v_st * 2);
 #if defined(__HIP_DEVICE_COMPILE__)  // (the host pass drops the launch stub over this builtin)
@@ -672,7 +771,8 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
   for (int i = 0; i < D / 32; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[i][r] = 0.f;
-  float m = 0.f, lsum = 0.f;
+  float m = G ? -INFINITY : 0.f, lsum = 0.f;
+  const float slope = G == 2 ? p.alibi[h] * kLog2e : 0.f;
 
   // per-lane LDS read bases (bytes, relative to a stage)
   const unsigned sbase = (unsigned)(size_t)lsm;
@@ -708,24 +808,37 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
       sa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(fk[s % 3]), qf[s], sa, 0, 0, 0);
     });
     ASTAMP(3);
+    if constexpr (G == 2) {
+      const float b0 = slope * (float)(t * BN + 4 * hh - qrow - off);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) sa[r] = fmaf(sa[r], sl2, fmaf(slope, (float)((r & 3) + 8 * (r >> 2)), b0));
+    }
     if constexpr (MASKED) {
-      const int lim = qrow + off - t * BN - 4 * hh;
+      const int lim = (G ? (CAUSAL ? min(qrow + off, kv_end - 1) : kv_end - 1) : qrow + off) - t * BN - 4 * hh;
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         if ((r & 3) + 8 * (r >> 2) > lim) sa[r] = -INFINITY;
+      if (G && t < own.f_lo) {
+        const int lo = qrow + off - p.window - t * BN - 4 * hh;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if ((r & 3) + 8 * (r >> 2) <= lo) sa[r] = -INFINITY;
+      }
     }
-    if (t == 0) {  // reference max = the first tile's row max (see attn_fwd_tiled_kernel)
+    // reference max = the first tile's row max (see attn_fwd_tiled_kernel)
+    if (G ? t > own.f_hi : t == 0) {
       float mt = sa[0];
 #pragma unroll
       for (int r = 1; r < 16; ++r) mt = fmaxf(mt, sa[r]);
-      m = fmaxf(mt, __shfl_xor(mt, 32, 64)) * sl2;
+      mt = fmaxf(mt, __shfl_xor(mt, 32, 64)) * (G == 2 ? 1.f : sl2);
+      m = !G || m == -INFINITY ? mt : m;
     }
-    const float nm = -m;
+    const float nm = G && m == -INFINITY ? 0.f : -m;
     float ps = 0.f;
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-      const float e0 = __builtin_amdgcn_exp2f(fmaf(sa[r], sl2, nm));
-      const float e1 = __builtin_amdgcn_exp2f(fmaf(sa[r + 8], sl2, nm));
+      const float e0 = __builtin_amdgcn_exp2f(G == 2 ? sa[r] + nm : fmaf(sa[r], sl2, nm));
+      const float e1 = __builtin_amdgcn_exp2f(G == 2 ? sa[r + 8] + nm : fmaf(sa[r + 8], sl2, nm));
       ps += e0 + e1;
       pf0[r] = (__bf16)e0;
       pf1[r] = (__bf16)e1;
@@ -775,31 +888,32 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
   };
   // causal: the mask is applied on every tile (16 selects that change nothing before the diagonal):
   // separate masked / mask-free bodies made hipcc spill ~170 registers
-  constexpr auto CM = std::integral_constant<bool, CAUSAL>{};
+  constexpr auto CM = std::integral_constant<bool, (CAUSAL || G > 0)>{};
   for (int t = 0; t < ntiles; ++t) {
     sync_issue(t);
-    if (t < mytiles) {
-      sm_part(t % NBUF, CM, t);
+    const int tile = sp.hi - 1 - t;
+    if (G ? tile < own.hi && tile >= own.lo : t < mytiles) {
+      sm_part(t % NBUF, CM, G ? tile : t);
       pv_part(t % NBUF);
     }
   }
 
   const float ltot = lsum + __shfl_xor(lsum, 32, 64);
-  const bool bad = !(ltot < 1.2676506e30f);
+  const bool bad = !(ltot < 1.2676506e30f) && (!G || qrow < p.Sq);
   const int any_bad = __any(bad);
   // overflow flags in the 4-wave kernel's layout (4 per 128-row block, lid order of the generic fixup)
   {
-    const int nqb128 = p.Sq / 128, qb128 = q0 / 128, w128 = (q0 % 128) / 32;
+    const int nqb128 = (p.Sq + 127) / 128, qb128 = q0 / 128, w128 = (q0 % 128) / 32;
     const int lid128 = bh * nqb128 + (CAUSAL ? nqb128 - 1 - qb128 : qb128);
-    if (lane == 0) p.flags[lid128 * 4 + w128] = any_bad;
+    if (lane == 0 && (!G || qb128 < nqb128)) p.flags[lid128 * 4 + w128] = any_bad;
   }
   const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
-  if (hh == 0 && p.lse)
+  if (hh == 0 && p.lse && (!G || qrow < p.Sq))
     p.lse[((long long)b * p.H + h) * p.Sq + qrow] = ltot > 0.f ? (m + log2f(ltot)) * kLn2 : INFINITY;
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // the clamped tail DMAs
   __syncthreads();  // the tile buffers become the epilogue images
-  store_tile_lds<D, D>(p.o + b * p.o_sb + h * p.o_sh + (long long)q0 * p.o_st, p.o_st, oacc, lane, inv,
-                       smem + wave * 32 * D * 2);
+  store_tile_lds<D, D, (G > 0)>(p.o + b * p.o_sb + h * p.o_sh + (long long)q0 * p.o_st, p.o_st, oacc, lane, inv,
+                                smem + wave * 32 * D * 2, p.Sq - q0);
   ASTAMP(6);
   ASTAMP_FLUSH(48);
 }
@@ -825,6 +939,9 @@ struct FastBwdParams {
   long long dq_sb, dq_st, dq_sh, dk_sb, dk_st, dk_sh, dv_sb, dv_st, dv_sh;
   int B, Sq, Sk, H, Hkv;
   float scale;
+  const float* alibi;  // as in FastFwdParams
+  const int* kv_len;
+  int window;
 };
 
 // A operand (32 rows x 16 k) read by rows from an image: lane (row l32, half hh)
@@ -873,8 +990,8 @@ __device__ __forceinline__ void store_acc_t(bf16_t* rowp, const f32x16 (&acc)[D 
 // steps, the dQ (dK, dV) tiles are stored DS wide.
 // 64-wide heads without a causal mask (SD): registers capped for 4 waves per SIMD instead of 3 (a 16-byte
 // spill in the 48-wide form; DreamBooth +1.5-2.8 % same box, profiles/decode_launch_structure_ab_r5.txt)
-template <int D, bool CAUSAL, int DS = D>
-__global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 4 : 1) attn_bwd_dq_tiled_kernel(FastBwdParams p) {
+template <int D, bool CAUSAL, int DS = D, int G = 0>
+__global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 4 : 1) attn_bwd_dq_tiled_kernel(FastBwdParams p) {
   constexpr int BM = 128, BN = 32;
   constexpr int TILE = BN * D * 2;
   using Stg = StagerFor<D, DS>;
@@ -885,7 +1002,7 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 4 : 1) attn_bwd_dq
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5;
-  const int nqb = p.Sq / BM;
+  const int nqb = (p.Sq + BM - 1) / BM;
   const int lid = xcd_remap(blockIdx.x, gridDim.x);
   const int qi = lid % nqb;
   const int qb = CAUSAL ? (nqb - 1 - qi) : qi;
@@ -895,20 +1012,25 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 4 : 1) attn_bwd_dq
   const int off = p.Sk - p.Sq;
   const int q0 = qb * BM + wave * 32;
   const int qrow = q0 + l32;
-  int kv_hi = p.Sk;
+  const int kv_end = G ? batch_keys(p.kv_len, b, p.Sk) : p.Sk;
+  int kv_hi = kv_end;
   if (CAUSAL) kv_hi = min(kv_hi, qb * BM + BM + off);
-  const int ntiles = (kv_hi + BN - 1) / BN;
+  TileSpan sp{};
+  if constexpr (G > 0) sp = tile_span<BM, CAUSAL>(qb * BM, off, kv_end, p.window);
+  const int ntiles = G ? sp.hi : (kv_hi + BN - 1) / BN, t0 = G ? sp.lo : 0;
   const float sl2 = p.scale * kLog2e;
 
-  const bf16_t* qp = p.q + b * p.q_sb + h * p.q_sh + (long long)qrow * p.q_st;
-  const bf16_t* gp = p.dout + b * p.do_sb + h * p.do_sh + (long long)qrow * p.do_st;
+  const int qr = G ? min(qrow, p.Sq - 1) : qrow;
+  const bf16_t* qp = p.q + b * p.q_sb + h * p.q_sh + (long long)qr * p.q_st;
+  const bf16_t* gp = p.dout + b * p.do_sb + h * p.do_sh + (long long)qr * p.do_st;
   bf16x8 qf[KSD], gf[KSD];
 #pragma unroll
   for (int s = 0; s < KSD; ++s) {
     qf[s] = *reinterpret_cast<const bf16x8*>(qp + 16 * s + 8 * hh);
     gf[s] = *reinterpret_cast<const bf16x8*>(gp + 16 * s + 8 * hh);
   }
-  const long long li = ((long long)b * p.H + h) * p.Sq + qrow;
+  const float slope = G == 2 ? p.alibi[h] * kLog2e : 0.f;
+  const long long li = ((long long)b * p.H + h) * p.Sq + qr;
   const float nlse = -p.lse[li] * kLog2e;
   const float dl = p.delta[li];
   f32x16 dq[D / 32];
@@ -920,7 +1042,8 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 4 : 1) attn_bwd_dq
   const bf16_t* kst = p.k + b * p.k_sb + hk * p.k_sh;
   const bf16_t* vst = p.v + b * p.v_sb + hk * p.v_sh;
   Stg stg(tid, p.k_st, p.v_st);
-  stg.bind(kst, vst, p.k_st, p.v_st);
+  if constexpr (G > 0) stg.bind(kst, vst, p.k_st, p.v_st, rows_bytes(kv_end, p.k_st, D), rows_bytes(kv_end, p.v_st, D));
+  else stg.bind(kst, vst, p.k_st, p.v_st);
   u32x4 sk[CPT], sv[CPT];
   int be, bo, b1, b2;
   row_bases<D>(l32, hh, be, bo);
@@ -933,8 +1056,8 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 4 : 1) attn_bwd_dq
     }
   }
 
-  stg.load(sk, sv, kst, vst, 0, p.k_st, p.v_st);
-  stg.store(sk, sv, smem);
+  stg.load(sk, sv, kst, vst, t0 * BN, p.k_st, p.v_st);
+  stg.store(sk, sv, smem + (t0 & 1) * 2 * TILE);
   __syncthreads();
   ASTAMP(0);
   // the last 4 tiles hold the four waves' diagonals; earlier tiles run the
@@ -975,15 +1098,19 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 4 : 1) attn_bwd_dq
       }
     }
     ASTAMP(2);
-    const int lim = qrow + off - k0 - 4 * hh;  // visible key offsets (r&3)+8(r>>2) <= lim
+    // visible key offsets (r&3)+8(r>>2): lo < offset <= lim
+    const int lim = (G ? (CAUSAL ? min(qrow + off, kv_end - 1) : kv_end - 1) : qrow + off) - k0 - 4 * hh;
+    const int lo = G && p.window > 0 ? qrow + off - p.window - k0 - 4 * hh : -(1 << 30);
+    const float b0 = G == 2 ? fmaf(slope, (float)(k0 + 4 * hh - qrow - off), nlse) : nlse;
     bf16x8 d0, d1;
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-      float p0 = __builtin_amdgcn_exp2f(fmaf(st[r], sl2, nlse));
-      float p1 = __builtin_amdgcn_exp2f(fmaf(st[r + 8], sl2, nlse));
+      const int c = (r & 3) + 8 * (r >> 2);
+      float p0 = __builtin_amdgcn_exp2f(fmaf(st[r], sl2, G == 2 ? fmaf(slope, (float)c, b0) : b0));
+      float p1 = __builtin_amdgcn_exp2f(fmaf(st[r + 8], sl2, G == 2 ? fmaf(slope, (float)(c + 16), b0) : b0));
       if constexpr (MASKED) {
-        if ((r & 3) + 8 * (r >> 2) > lim) p0 = 0.f;
-        if ((r & 3) + 8 * (r >> 2) + 16 > lim) p1 = 0.f;
+        if (c > lim || (G && c <= lo)) p0 = 0.f;
+        if (c + 16 > lim || (G && c + 16 <= lo)) p1 = 0.f;
       }
       d0[r] = (__bf16)(p0 * (dpt[r] - dl));
       d1[r] = (__bf16)(p1 * (dpt[r + 8] - dl));
@@ -1012,11 +1139,18 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 4 : 1) attn_bwd_dq
     __syncthreads();
     ASTAMP(5);
   };
-  const int nfree = CAUSAL ? ntiles - 4 : ntiles;
-  for (int t = 0; t < nfree; ++t) tile_step(t, std::false_type{});
-  for (int t = max(nfree, 0); t < ntiles; ++t) tile_step(t, std::true_type{});
-  store_tile_lds<D, DS>(p.dq + b * p.dq_sb + h * p.dq_sh + (long long)q0 * p.dq_st, p.dq_st, dq, lane, p.scale,
-                        smem + wave * 32 * D * 2);
+  if constexpr (G > 0) {
+    const int low = min(ntiles, max(t0, sp.f_lo)), top = max(low, min(ntiles, sp.f_hi + 1));
+    for (int t = t0; t < low; ++t) tile_step(t, std::true_type{});
+    for (int t = low; t < top; ++t) tile_step(t, std::false_type{});
+    for (int t = top; t < ntiles; ++t) tile_step(t, std::true_type{});
+  } else {
+    const int nfree = CAUSAL ? ntiles - 4 : ntiles;
+    for (int t = 0; t < nfree; ++t) tile_step(t, std::false_type{});
+    for (int t = max(nfree, 0); t < ntiles; ++t) tile_step(t, std::true_type{});
+  }
+  store_tile_lds<D, DS, (G > 0)>(p.dq + b * p.dq_sb + h * p.dq_sh + (long long)q0 * p.dq_st, p.dq_st, dq, lane, p.scale,
+                                 smem + wave * 32 * D * 2, p.Sq - q0);
   ASTAMP(6);
   ASTAMP_FLUSH(16);
 }
@@ -1024,8 +1158,8 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 4 : 1) attn_bwd_dq
 // 64-wide heads without a causal mask (SD-1.5's 40-wide heads in narrow storage): registers capped for
 // 3 waves per SIMD (165 VGPRs, no spill) instead of 2 -- DreamBooth 61.1 -> 62.3 samples/s same box
 // (the causal D = 64 form spills at that cap and keeps 2)
-template <int D, bool CAUSAL, int DS = D>
-__global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 3 : 1) attn_bwd_dkdv_tiled_kernel(FastBwdParams p) {
+template <int D, bool CAUSAL, int DS = D, int G = 0>
+__global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 3 : 1) attn_bwd_dkdv_tiled_kernel(FastBwdParams p) {
   constexpr int BK = 128, BQ = 32;
   constexpr int TILE = BQ * D * 2;                  // one 32-row image
   using Stg = StagerFor<D, DS>;
@@ -1038,7 +1172,7 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 3 : 1) attn_bwd_dk
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5;
-  const int nkb = p.Sk / BK;
+  const int nkb = (p.Sk + BK - 1) / BK;
   const int lid = xcd_remap(blockIdx.x, gridDim.x);
   const int kb = lid % nkb, bh = lid / nkb;
   const int b = bh / p.Hkv, hk = bh % p.Hkv;
@@ -1046,21 +1180,25 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 3 : 1) attn_bwd_dk
   const int off = p.Sk - p.Sq;
   const int kw = kb * BK + wave * 32;
   const int key = kw + l32;
+  const int kv_end = G ? batch_keys(p.kv_len, b, p.Sk) : p.Sk;
   const float sl2 = p.scale * kLog2e;
 
   const bf16_t* kp = p.k + b * p.k_sb + hk * p.k_sh;
   const bf16_t* vp = p.v + b * p.v_sb + hk * p.v_sh;
   bf16x8 kf[KSD];
 #pragma unroll
-  for (int s = 0; s < KSD; ++s)
-    kf[s] = *reinterpret_cast<const bf16x8*>(kp + (long long)key * p.k_st + 16 * s + 8 * hh);
+  for (int s = 0; s < KSD; ++s) {
+    kf[s] = *reinterpret_cast<const bf16x8*>(kp + (long long)(G ? min(key, p.Sk - 1) : key) * p.k_st + 16 * s + 8 * hh);
+    if (G && key >= kv_end) kf[s] = bf16x8{};
+  }
   // this wave's 32 V rows -> its own image (read back by rows for dP; pad chunks zero)
   char* vimg = smem + VOFF + wave * TILE;
 #pragma unroll
   for (int i = 0; i < 32 * NCH / 64; ++i) {
     const int idx = lane + 64 * i, row = idx / NCH, ch = idx % NCH;
     *reinterpret_cast<u32x4*>(vimg + img_off<D>(row, ch)) =
-        ch < NCS ? *reinterpret_cast<const u32x4*>(vp + (long long)(kw + row) * p.v_st + ch * 8) : u32x4{0, 0, 0, 0};
+        ch < NCS && (!G || kw + row < kv_end) ? *reinterpret_cast<const u32x4*>(vp + (long long)(kw + row) * p.v_st + ch * 8)
+                                              : u32x4{0, 0, 0, 0};
   }
   if constexpr (DS < D) {  // Q / dO image chunks DS/8.. are never loaded: zero them in both buffers once
     constexpr int PC = NCH - NCS, NZ = 2 * 2 * 32 * PC;
@@ -1077,11 +1215,14 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 3 : 1) attn_bwd_dk
 
   int q_lo = 0;
   if (CAUSAL) q_lo = max(0, kb * BK - off) & ~(BQ - 1);
-  const int nqt = (p.Sq - q_lo) / BQ;
-  const int total = nqt * grp;
+  // G: no query sees a block past the length; past the last key's window no query sees the block
+  const int q_end = G && p.window > 0 ? min(p.Sq, kb * BK + BK - 1 - off + p.window) : p.Sq;
+  const int nqt = G ? max(0, q_end - q_lo + BQ - 1) / BQ : (p.Sq - q_lo) / BQ;
+  const int total = !G || kb * BK < kv_end ? nqt * grp : 0;
+  const int qn = G ? rows_bytes(p.Sq, p.q_st, D) : kAllRows, gn = G ? rows_bytes(p.Sq, p.do_st, D) : kAllRows;
 
   Stg stg(tid, p.q_st, p.do_st);
-  stg.bind(p.q + b * p.q_sb + hk * grp * p.q_sh, p.dout + b * p.do_sb + hk * grp * p.do_sh, p.q_st, p.do_st);
+  stg.bind(p.q + b * p.q_sb + hk * grp * p.q_sh, p.dout + b * p.do_sb + hk * grp * p.do_sh, p.q_st, p.do_st, qn, gn);
   u32x4 sq[CPT], sg[CPT];
   float lreg = 0.f;
   int be, bo, b1, b2;
@@ -1091,12 +1232,14 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 3 : 1) attn_bwd_dk
 #define KCA_DKDV_LOAD(it_)                                                                     \
   {                                                                                            \
     const int hq_ = hk * grp + (it_) / nqt, qt_ = q_lo + ((it_) % nqt) * BQ;                   \
-    if (grp > 1) stg.set_base(p.q + b * p.q_sb + hq_ * p.q_sh, p.dout + b * p.do_sb + hq_ * p.do_sh); \
+    if (grp > 1) stg.set_base(p.q + b * p.q_sb + hq_ * p.q_sh, p.dout + b * p.do_sb + hq_ * p.do_sh, qn, gn); \
     stg.load(sq, sg, p.q + b * p.q_sb + hq_ * p.q_sh, p.dout + b * p.do_sb + hq_ * p.do_sh, qt_,   \
              p.q_st, p.do_st);                                                                 \
     if (tid < 64) {                                                                            \
-      const long long li_ = ((long long)b * p.H + hq_) * p.Sq + qt_ + (tid & 31);              \
+      const int qr_ = qt_ + (tid & 31);                                                        \
+      const long long li_ = ((long long)b * p.H + hq_) * p.Sq + (G ? min(qr_, p.Sq - 1) : qr_); \
       lreg = tid < 32 ? p.lse[li_] * kLog2e : p.delta[li_];                                    \
+      if (G && qr_ >= p.Sq) lreg = tid < 32 ? INFINITY : 0.f;  /* P = 0 */                     \
     }                                                                                          \
   }
 #define KCA_DKDV_STORE(buf_)                                                                   \
@@ -1158,7 +1301,14 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 3 : 1) attn_bwd_dk
     ASTAMP(2);
     // rows q = qt + 8g + 4hh + j (g = r>>2, j = r&3): lse / delta as float4;
     // visible iff key <= q + off, i.e. 8g + j >= key - qt - off - 4hh
-    const int lim = key - qt - off - 4 * hh;
+    int lim = G && !CAUSAL ? -(1 << 30) : key - qt - off - 4 * hh;
+    if (G && key >= kv_end) lim = 1 << 30;
+    const int ul = G && p.window > 0 ? key + p.window - off - qt - 4 * hh : 1 << 30;  // G: and 8g + j < ul
+    float slope = 0.f, b0 = 0.f;
+    if constexpr (G == 2) {
+      slope = p.alibi[hk * grp + it / nqt] * kLog2e;
+      b0 = slope * (float)(key - qt - off - 4 * hh);
+    }
     bf16x8 p0, p1, s0, s1;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
@@ -1167,9 +1317,10 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 3 : 1) attn_bwd_dk
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int r = 4 * g + j;
-        float pr = __builtin_amdgcn_exp2f(fmaf(sacc[r], sl2, -lq[j]));
+        const float bl = G == 2 ? fmaf(-slope, (float)(8 * g + j), b0) - lq[j] : -lq[j];
+        float pr = __builtin_amdgcn_exp2f(fmaf(sacc[r], sl2, bl));
         if constexpr (MASKED) {
-          if (8 * g + j < lim) pr = 0.f;
+          if (8 * g + j < lim || (G && 8 * g + j >= ul)) pr = 0.f;
         }
         const float ds = pr * (dpacc[r] - dq4[j]);
         if (r < 8) { p0[r] = (__bf16)pr; s0[r] = (__bf16)ds; }
@@ -1217,17 +1368,19 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 3 : 1) attn_bwd_dk
   // One flat loop with the (cheap, select-only) causal mask on every tile:
   // splitting into masked / mask-free bodies -- by a per-tile branch or by
   // two loops per head -- pushed the 256 dK/dV accumulators into spills.
-  for (int it = 0; it < total; ++it) tile_step(it, std::integral_constant<bool, CAUSAL>{});
+  for (int it = 0; it < total; ++it) tile_step(it, std::integral_constant<bool, (CAUSAL || G > 0)>{});
 #undef KCA_DKDV_LOAD
 #undef KCA_DKDV_STORE
   if constexpr (D == 96) {  // the LDS staging's registers push this one past 256 (2 -> 1 wave per SIMD)
-    store_acc_t<D>(p.dk + b * p.dk_sb + hk * p.dk_sh + (long long)key * p.dk_st, dk, hh, p.scale);
-    store_acc_t<D>(p.dv + b * p.dv_sb + hk * p.dv_sh + (long long)key * p.dv_st, dv, hh, 1.f);
+    if (!G || key < p.Sk) {
+      store_acc_t<D>(p.dk + b * p.dk_sb + hk * p.dk_sh + (long long)key * p.dk_st, dk, hh, p.scale);
+      store_acc_t<D>(p.dv + b * p.dv_sb + hk * p.dv_sh + (long long)key * p.dv_st, dv, hh, 1.f);
+    }
   } else {
-    store_tile_lds<D, DS>(p.dk + b * p.dk_sb + hk * p.dk_sh + (long long)kw * p.dk_st, p.dk_st, dk, lane, p.scale,
-                      smem + wave * 32 * D * 2);
-    store_tile_lds<D, DS>(p.dv + b * p.dv_sb + hk * p.dv_sh + (long long)kw * p.dv_st, p.dv_st, dv, lane, 1.f,
-                      smem + wave * 32 * D * 2);
+    store_tile_lds<D, DS, (G > 0)>(p.dk + b * p.dk_sb + hk * p.dk_sh + (long long)kw * p.dk_st, p.dk_st, dk, lane, p.scale,
+                                   smem + wave * 32 * D * 2, p.Sk - kw);
+    store_tile_lds<D, DS, (G > 0)>(p.dv + b * p.dv_sb + hk * p.dv_sh + (long long)kw * p.dv_st, p.dv_st, dv, lane, 1.f,
+                                   smem + wave * 32 * D * 2, p.Sk - kw);
   }
   ASTAMP(6);
   ASTAMP_FLUSH(32);
@@ -1236,6 +1389,32 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL) ? 3 : 1) attn_bwd_dk
 // the staged K/V (dK/dV: Q/dO) rows are addressed as 32-bit byte offsets from a
 // per-head buffer resource; longer rows fall back to the generic kernel
 inline bool offsets_fit(long long rows, long long stride) { return (rows + 128) * stride * 2 < (1ll << 31); }
+
+// 16-byte rows: what the general forms ask of a call (any other one runs the generic kernels, which it ran before)
+inline bool rows16(const void* p, long long sb, long long st, long long sh) {
+  return (uintptr_t)p % 16 == 0 && (sb | st | sh) % 8 == 0;
+}
+
+// Calls f(D, causal, G) with the general forms' constants; false: there is no such form. ALiBi comes with a causal
+// mask only (without one the least bias is not at a row's last key).
+template <class F>
+bool general_form(int d, bool causal, bool alibi, F&& f) {
+  if (alibi && !causal) return false;
+  auto mask = [&](auto D) {
+    if (!causal) f(D, std::false_type{}, std::integral_constant<int, 1>{});
+    else if (!alibi) f(D, std::true_type{}, std::integral_constant<int, 1>{});
+    else f(D, std::true_type{}, std::integral_constant<int, 2>{});
+    return true;
+  };
+  switch (d) {
+    case 64: return mask(std::integral_constant<int, 64>{});
+    case 96: return mask(std::integral_constant<int, 96>{});
+    case 128: return mask(std::integral_constant<int, 128>{});
+    case 160: return mask(std::integral_constant<int, 160>{});
+    case 256: return mask(std::integral_constant<int, 256>{});
+  }
+  return false;
+}
 
 }  // namespace
 
@@ -1255,20 +1434,41 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
                                long long k_st, long long k_sh, long long v_sb, long long v_st,
                                long long v_sh, long long o_sb, long long o_st, long long o_sh,
                                int B, int Sq, int Sk, int H, int Hkv, int d, int causal,
-                               float scale, int rowsum_col, int max_col, int* flags, hipStream_t stream) {
-  if ((d != 48 && d != 64 && d != 96 && d != 128 && d != 160 && d != 256) || Sq % 128 || Sk % 32 || Sq <= 0 ||
-      H % Hkv || !flags)
-    return 1;
-  if (max_col >= 0 && (max_col != 40 || rowsum_col != 40 || d != 48)) return 1;  // instantiated variant
-  if (d == 48 && causal) return 1;  // narrow storage: SD-1.5's (non-causal) 40-wide heads
-  if (rowsum_col >= 0 && (rowsum_col != 40 || (d != 64 && d != 48) || causal)) return 1;  // instantiated variants
+                               float scale, const float* alibi, const int* kv_len, int window, int rowsum_col,
+                               int max_col, int* flags, hipStream_t stream) {
+  if (Sq <= 0 || Sk <= 0 || H % Hkv || !flags) return 1;
   if (causal && Sk < Sq) return 1;
   if (!offsets_fit(Sk, k_st) || !offsets_fit(Sk, v_st)) return 1;  // buffer-load byte offsets are 32-bit
   FastFwdParams p{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (bf16_t*)o, lse, flags,
                   q_sb, q_st, q_sh, k_sb, k_st, k_sh, v_sb, v_st, v_sh, o_sb, o_st, o_sh,
-                  B, Sq, Sk, H, Hkv, scale};
-  dim3 grid((Sq / 128) * B * H);
+                  B, Sq, Sk, H, Hkv, scale, alibi, kv_len, window};
+  dim3 grid(((Sq + 127) / 128) * B * H);
   (void)hipGetLastError();
+  // The general forms against the generic kernels, which took these calls before (one MI355X; forward, forward's and
+  // backward's kernels in us, generic -> general):
+  //   2 x 2048, 14 heads of 128, ALiBi       198 -> 80, 345 -> 303    1 x 1500, 64 heads of 96       177 -> 66, 366 -> 234
+  //   4 x 1100, 16 heads of 256              194 -> 77, 685 -> 307    8 x 1000, 12 heads of 64        59 -> 36, 181 -> 145
+  //   4 x 2048, 16 heads of 256, lengths     528 -> 203, 1870 -> 815  2 x 2048, 20 of 128, window 256  68 -> 39, 148 -> 137
+  // Full tiles without another mask keep the plain form, whose loops have no edge to test: 4 x 2048 of 256 179 us
+  // against 203 forward and 760 against 815 backward, 8 x 1024 of 64 36 and 137 against 36 and 146.
+  if (alibi || kv_len || window || Sq % 128 || Sk % 32) {
+    if (!rows16(q, q_sb, q_st, q_sh) || !rows16(k, k_sb, k_st, k_sh) || !rows16(v, v_sb, v_st, v_sh) ||
+        !rows16(o, o_sb, o_st, o_sh))
+      return 1;
+    const bool done = general_form(d, causal, alibi, [&](auto D_, auto C_, auto G_) {
+      constexpr int D = decltype(D_)::value, G = decltype(G_)::value;
+      constexpr bool C = decltype(C_)::value;
+      if constexpr (D == 256)
+        hipLaunchKernelGGL((attn_fwd_w8_kernel<D, C, 8, 4, G>), dim3(((Sq + 255) / 256) * B * H), dim3(512), 0, stream, p);
+      else
+        hipLaunchKernelGGL((attn_fwd_tiled_kernel<D, C, -1, D, -1, G>), grid, dim3(256), 0, stream, p);
+    });
+    return !done ? 1 : hipGetLastError() == hipSuccess ? 0 : 3;
+  }
+  if ((d != 48 && d != 64 && d != 96 && d != 128 && d != 160 && d != 256)) return 1;
+  if (max_col >= 0 && (max_col != 40 || rowsum_col != 40 || d != 48)) return 1;  // instantiated variant
+  if (d == 48 && causal) return 1;  // narrow storage: SD-1.5's (non-causal) 40-wide heads
+  if (rowsum_col >= 0 && (rowsum_col != 40 || (d != 64 && d != 48) || causal)) return 1;  // instantiated variants
   if (d == 256 && (g_attn_variant & 1) && Sq % 256 == 0) {
     dim3 g8((Sq / 256) * B * H);
     if (causal) hipLaunchKernelGGL((attn_fwd_w8_kernel<256, true>), g8, dim3(512), 0, stream, p);
@@ -1325,19 +1525,32 @@ KCA_API int kca_attn_bwd_tiled(const void* q, const void* k, const void* v, cons
                                long long dq_sb, long long dq_st, long long dq_sh, long long dk_sb,
                                long long dk_st, long long dk_sh, long long dv_sb, long long dv_st,
                                long long dv_sh, int B, int Sq, int Sk, int H, int Hkv, int d,
-                               int causal, float scale, hipStream_t stream) {
-  if ((d != 48 && d != 64 && d != 96 && d != 128 && d != 160 && d != 256) || Sq % 128 || Sk % 128 || Sq <= 0 ||
-      H % Hkv)
-    return 1;
-  if (d == 48 && causal) return 1;  // narrow storage: SD-1.5's (non-causal) 40-wide heads
+                               int causal, float scale, const float* alibi, const int* kv_len, int window,
+                               hipStream_t stream) {
+  if (Sq <= 0 || Sk <= 0 || H % Hkv) return 1;
   if (causal && Sk < Sq) return 1;
   if (!offsets_fit(Sk, k_st) || !offsets_fit(Sk, v_st) || !offsets_fit(Sq, q_st) || !offsets_fit(Sq, do_st)) return 1;
   FastBwdParams p{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)dout,
                   (bf16_t*)dq, (bf16_t*)dk, (bf16_t*)dv, lse, delta,
                   q_sb, q_st, q_sh, k_sb, k_st, k_sh, v_sb, v_st, v_sh, do_sb, do_st, do_sh,
                   dq_sb, dq_st, dq_sh, dk_sb, dk_st, dk_sh, dv_sb, dv_st, dv_sh,
-                  B, Sq, Sk, H, Hkv, scale};
-  dim3 g1((Sk / 128) * B * Hkv), g2((Sq / 128) * B * H);
+                  B, Sq, Sk, H, Hkv, scale, alibi, kv_len, window};
+  dim3 g1(((Sk + 127) / 128) * B * Hkv), g2(((Sq + 127) / 128) * B * H);
+  if (alibi || kv_len || window || Sq % 128 || Sk % 128) {
+    if (!rows16(q, q_sb, q_st, q_sh) || !rows16(k, k_sb, k_st, k_sh) || !rows16(v, v_sb, v_st, v_sh) ||
+        !rows16(dout, do_sb, do_st, do_sh) || !rows16(dq, dq_sb, dq_st, dq_sh) || !rows16(dk, dk_sb, dk_st, dk_sh) ||
+        !rows16(dv, dv_sb, dv_st, dv_sh))
+      return 1;
+    const bool done = general_form(d, causal, alibi, [&](auto D_, auto C_, auto G_) {
+      constexpr int D = decltype(D_)::value, G = decltype(G_)::value;
+      constexpr bool C = decltype(C_)::value;
+      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<D, C, D, G>), g1, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((attn_bwd_dq_tiled_kernel<D, C, D, G>), g2, dim3(256), 0, stream, p);
+    });
+    return done ? 0 : 1;
+  }
+  if (d != 48 && d != 64 && d != 96 && d != 128 && d != 160 && d != 256) return 1;
+  if (d == 48 && causal) return 1;  // narrow storage: SD-1.5's (non-causal) 40-wide heads
   if (d == 48) {  // heads stored 48 wide in D = 64 images (the UNet's 40-wide heads, training)
     hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<64, false, 48>), g1, dim3(256), 0, stream, p);
     hipLaunchKernelGGL((attn_bwd_dq_tiled_kernel<64, false, 48>), g2, dim3(256), 0, stream, p);
