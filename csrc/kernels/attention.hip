@@ -59,6 +59,7 @@ struct AttnParams {
   int window;                 // > 0: key visible only if key > q + off - window (GPT-Neo local layers)
   const unsigned* key_mask;   // [B, km_words] bitmap of attended keys (masks with holes) or null
   int km_words;
+  const int* cu;  // [B + 1] or null: packed sequences, batch b is rows cu[b] .. cu[b + 1] (batch strides 0, lse null)
 };
 
 struct AttnBwdParams {
@@ -191,6 +192,15 @@ __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1)) attn_fwd_kernel(AttnP
   const int bh = lid / nqb;
   const int b = bh / p.H, h = bh % p.H;
   const int hk = h / (p.H / p.Hkv);
+  if (p.cu) {  // (Sq was the longest sequence's length)
+    const int c0 = p.cu[b];
+    p.Sq = p.Sk = p.cu[b + 1] - c0;
+    if (qb * BM >= p.Sq) return;
+    p.q += c0 * p.q_st;
+    p.k += c0 * p.k_st;
+    p.v += c0 * p.v_st;
+    p.o += c0 * p.o_st;
+  }
   const int off = p.Sk - p.Sq;
   int kv_end = p.Sk;
   KCA_DASSERT(!p.kv_len || (p.kv_len[b] >= 0 && p.kv_len[b] <= p.Sk));
@@ -1029,8 +1039,27 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
                                long long k_st, long long k_sh, long long v_sb, long long v_st,
                                long long v_sh, long long o_sb, long long o_st, long long o_sh,
                                int B, int Sq, int Sk, int H, int Hkv, int d, int causal,
-                               float scale, const float* alibi, const int* kv_len, int window, int rowsum_col,
-                               int max_col, int* flags, hipStream_t stream);
+                               float scale, const float* alibi, const int* kv_len, int window, const int* cu,
+                               int rowsum_col, int max_col, int* flags, hipStream_t stream);
+
+static int attn_fwd_go(AttnParams p, int rowsum_col, int max_col, int* workspace, hipStream_t stream) {
+  if (p.d_real % 8 || p.H % p.Hkv || p.window < 0) return 1;
+  const int D = pick_d(p.d_real);
+  p.km_words = (p.Sk + 31) / 32;
+  if (g_attn_tiled && workspace && !p.key_mask &&
+      kca_attn_fwd_tiled(p.q, p.k, p.v, p.o, p.lse, p.q_sb, p.q_st, p.q_sh, p.k_sb, p.k_st, p.k_sh, p.v_sb, p.v_st,
+                         p.v_sh, p.o_sb, p.o_st, p.o_sh, p.B, p.Sq, p.Sk, p.H, p.Hkv, p.d_real, p.causal, p.scale,
+                         p.alibi, p.kv_len, p.window, p.cu, rowsum_col, max_col, workspace, stream) == 0)
+    p.fix_flags = workspace;  // fixup launch below: only flagged blocks do work
+  dim3 grid(((p.Sq + 127) / 128) * p.B * p.H);
+  ATTN_D_DISPATCH(D, {
+    if (p.causal)
+      hipLaunchKernelGGL((attn_fwd_kernel<DD, true>), grid, dim3(256), 0, stream, p);
+    else
+      hipLaunchKernelGGL((attn_fwd_kernel<DD, false>), grid, dim3(256), 0, stream, p);
+  });
+  return 0;
+}
 
 // workspace: >= 4 * ceil(Sq/128) * B * H ints for the full-tile fast path of
 // attention_tiled.hip (its overflow flags), or null for the generic kernel.
@@ -1047,25 +1076,26 @@ KCA_API int kca_attn_fwd(const void* q, const void* k, const void* v, void* o,
                          int d_real, int causal, float scale,
                          const float* alibi, const int* kv_len, int window, const unsigned* key_mask,
                          int rowsum_col, int max_col, int* workspace, hipStream_t stream) {
-  if (d_real % 8 || H % Hkv || window < 0) return 1;
-  const int D = pick_d(d_real);
-  AttnParams p{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (bf16_t*)o, lse,
-               q_sb, q_st, q_sh, k_sb, k_st, k_sh, v_sb, v_st, v_sh, o_sb, o_st, o_sh,
-               B, Sq, Sk, H, Hkv, d_real, causal, scale, alibi, kv_len, nullptr,
-               window, key_mask, (Sk + 31) / 32};
-  if (g_attn_tiled && workspace && !key_mask &&
-      kca_attn_fwd_tiled(q, k, v, o, lse, q_sb, q_st, q_sh, k_sb, k_st, k_sh, v_sb, v_st, v_sh,
-                         o_sb, o_st, o_sh, B, Sq, Sk, H, Hkv, d_real, causal, scale, alibi, kv_len, window,
-                         rowsum_col, max_col, workspace, stream) == 0)
-    p.fix_flags = workspace;  // fixup launch below: only flagged blocks do work
-  dim3 grid(((Sq + 127) / 128) * B * H);
-  ATTN_D_DISPATCH(D, {
-    if (causal)
-      hipLaunchKernelGGL((attn_fwd_kernel<DD, true>), grid, dim3(256), 0, stream, p);
-    else
-      hipLaunchKernelGGL((attn_fwd_kernel<DD, false>), grid, dim3(256), 0, stream, p);
-  });
-  return 0;
+  return attn_fwd_go(AttnParams{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (bf16_t*)o, lse,
+                                q_sb, q_st, q_sh, k_sb, k_st, k_sh, v_sb, v_st, v_sh, o_sb, o_st, o_sh,
+                                B, Sq, Sk, H, Hkv, d_real, causal, scale, alibi, kv_len, nullptr,
+                                window, key_mask, 0, nullptr},
+                     rowsum_col, max_col, workspace, stream);
+}
+
+// Sequences of any lengths one after another in [T, H, D] rows: sequence b is rows cu[b] .. cu[b + 1] (at most
+// max_len of them) and attends to itself. Inference (no lse). workspace as above, with Sq = max_len, B = n.
+KCA_API int kca_attn_fwd_packed(const void* q, const void* k, const void* v, void* o, long long q_st, long long q_sh,
+                                long long k_st, long long k_sh, long long v_st, long long v_sh, long long o_st,
+                                long long o_sh, int n, int max_len, int H, int Hkv, int d_real, int causal,
+                                float scale, const float* alibi, int window, const int* cu, int* workspace,
+                                hipStream_t stream) {
+  if (n < 1 || max_len < 1 || !cu) return 1;
+  return attn_fwd_go(AttnParams{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (bf16_t*)o, nullptr,
+                                0, q_st, q_sh, 0, k_st, k_sh, 0, v_st, v_sh, 0, o_st, o_sh,
+                                n, max_len, max_len, H, Hkv, d_real, causal, scale, alibi, nullptr, nullptr,
+                                window, nullptr, 0, cu},
+                     -1, -1, workspace, stream);
 }
 
 KCA_API int kca_attn_bwd_preprocess(const void* o, const void* dout,

@@ -80,7 +80,18 @@ struct FastFwdParams {
   const float* alibi;  // [H] slopes (G = 2)
   const int* kv_len;   // [B] or null (G > 0)
   int window;          // > 0: key visible only if key > q + off - window (G > 0)
+  const int* cu;       // [B + 1] or null (G > 0): packed sequences -- batch b is rows cu[b] .. cu[b + 1], the batch
+                       // strides are 0, Sq is the longest's length and lse null
 };
+
+__device__ __forceinline__ void own_sequence(FastFwdParams& p, int b) {
+  const int c0 = p.cu[b];
+  p.Sq = p.Sk = p.cu[b + 1] - c0;
+  p.q += c0 * p.q_st;
+  p.k += c0 * p.k_st;
+  p.v += c0 * p.v_st;
+  p.o += c0 * p.o_st;
+}
 
 constexpr int kAllRows = 0x7fffffff;
 
@@ -342,6 +353,15 @@ __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1)) attn_fwd_tiled_kernel
   const int bh = lid / nqb;
   const int b = bh / p.H, h = bh % p.H;
   const int hk = h / (p.H / p.Hkv);
+  if constexpr (G > 0) {
+    if (p.cu) {
+      own_sequence(p, b);
+      if (qb * BM >= p.Sq) {
+        if (lane == 0) p.flags[lid * 4 + wave] = 0;
+        return;
+      }
+    }
+  }
   const int off = p.Sk - p.Sq;
   const int q0 = qb * BM + wave * 32;
   const int qrow = q0 + l32;
@@ -706,6 +726,18 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
   const int bh = lid / nqb;
   const int b = bh / p.H, h = bh % p.H;
   const int hk = h / (p.H / p.Hkv);
+  // overflow flags in the 4-wave kernel's layout (4 per 128-row block, lid order of the generic fixup)
+  const int nqb128 = (p.Sq + 127) / 128, qb128 = (qb * BM + wave * 32) / 128;
+  int* flag = p.flags + (bh * nqb128 + (CAUSAL ? nqb128 - 1 - qb128 : qb128)) * 4 + wave % 4;
+  if constexpr (G > 0) {
+    if (p.cu) {
+      own_sequence(p, b);
+      if (qb * BM >= p.Sq) {
+        if (lane == 0 && qb128 < nqb128) *flag = 0;
+        return;
+      }
+    }
+  }
   const int off = p.Sk - p.Sq;
   const int q0 = qb * BM + wave * 32;
   const int qrow = q0 + l32;
@@ -901,12 +933,7 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
   const float ltot = lsum + __shfl_xor(lsum, 32, 64);
   const bool bad = !(ltot < 1.2676506e30f) && (!G || qrow < p.Sq);
   const int any_bad = __any(bad);
-  // overflow flags in the 4-wave kernel's layout (4 per 128-row block, lid order of the generic fixup)
-  {
-    const int nqb128 = (p.Sq + 127) / 128, qb128 = q0 / 128, w128 = (q0 % 128) / 32;
-    const int lid128 = bh * nqb128 + (CAUSAL ? nqb128 - 1 - qb128 : qb128);
-    if (lane == 0 && (!G || qb128 < nqb128)) p.flags[lid128 * 4 + w128] = any_bad;
-  }
+  if (lane == 0 && (!G || qb128 < nqb128)) *flag = any_bad;
   const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
   if (hh == 0 && p.lse && (!G || qrow < p.Sq))
     p.lse[((long long)b * p.H + h) * p.Sq + qrow] = ltot > 0.f ? (m + log2f(ltot)) * kLn2 : INFINITY;
@@ -1434,14 +1461,14 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
                                long long k_st, long long k_sh, long long v_sb, long long v_st,
                                long long v_sh, long long o_sb, long long o_st, long long o_sh,
                                int B, int Sq, int Sk, int H, int Hkv, int d, int causal,
-                               float scale, const float* alibi, const int* kv_len, int window, int rowsum_col,
-                               int max_col, int* flags, hipStream_t stream) {
+                               float scale, const float* alibi, const int* kv_len, int window, const int* cu,
+                               int rowsum_col, int max_col, int* flags, hipStream_t stream) {
   if (Sq <= 0 || Sk <= 0 || H % Hkv || !flags) return 1;
   if (causal && Sk < Sq) return 1;
   if (!offsets_fit(Sk, k_st) || !offsets_fit(Sk, v_st)) return 1;  // buffer-load byte offsets are 32-bit
   FastFwdParams p{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (bf16_t*)o, lse, flags,
                   q_sb, q_st, q_sh, k_sb, k_st, k_sh, v_sb, v_st, v_sh, o_sb, o_st, o_sh,
-                  B, Sq, Sk, H, Hkv, scale, alibi, kv_len, window};
+                  B, Sq, Sk, H, Hkv, scale, alibi, kv_len, window, cu};
   dim3 grid(((Sq + 127) / 128) * B * H);
   (void)hipGetLastError();
   // The general forms against the generic kernels, which took these calls before (one MI355X; forward, forward's and
@@ -1451,7 +1478,7 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
   //   4 x 2048, 16 heads of 256, lengths     528 -> 203, 1870 -> 815  2 x 2048, 20 of 128, window 256  68 -> 39, 148 -> 137
   // Full tiles without another mask keep the plain form, whose loops have no edge to test: 4 x 2048 of 256 179 us
   // against 203 forward and 760 against 815 backward, 8 x 1024 of 64 36 and 137 against 36 and 146.
-  if (alibi || kv_len || window || Sq % 128 || Sk % 32) {
+  if (alibi || kv_len || window || cu || Sq % 128 || Sk % 32) {
     if (!rows16(q, q_sb, q_st, q_sh) || !rows16(k, k_sb, k_st, k_sh) || !rows16(v, v_sb, v_st, v_sh) ||
         !rows16(o, o_sb, o_st, o_sh))
       return 1;

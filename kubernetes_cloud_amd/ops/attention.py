@@ -203,6 +203,24 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: b
     return o
 
 
+def packed_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu: torch.Tensor, max_len: int,
+                     scale: float | None = None, alibi: torch.Tensor | None = None, window: int = 0) -> torch.Tensor:
+    """Causal self-attention of sequences that lie one after another in [T, H, D] rows (inference): sequence i is rows
+    ``cu[i]`` .. ``cu[i + 1]`` (int32, on the device), none longer than ``max_len``."""
+    T, H, D = q.shape
+    _check(*(t.unsqueeze(0) for t in (q, k, v)))
+    n = cu.shape[0] - 1
+    o = torch.empty(T, H, D, device=q.device, dtype=q.dtype)
+    flags = torch.empty(4 * ((max_len + 127) // 128) * n * H, device=q.device, dtype=torch.int32)
+    scale = scale if scale is not None else 1.0 / math.sqrt(D)
+    if alibi is not None:
+        alibi = alibi.to(device=q.device, dtype=torch.float32).contiguous()
+    _lib.call("kca_attn_fwd_packed", q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), q.stride(0), q.stride(1),
+              k.stride(0), k.stride(1), v.stride(0), v.stride(1), o.stride(0), o.stride(1), n, max_len, H, k.shape[1], D,
+              1, float(scale), _lib.ptr(alibi), int(window), cu.data_ptr(), flags.data_ptr(), _lib.stream())
+    return o
+
+
 def wide_head_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float):
     """Single-head attention over [B, S, 512] bf16 rows (the VAE mid-block, inference) on the
     LDS-DMA flash kernel (attention_tiled.hip ``kca_attn_fwd_wide``). Returns None when the shape is

@@ -88,6 +88,23 @@ def apply_rotary_(q: torch.Tensor, k: torch.Tensor, rot: int, seq: int, interlea
             t.copy_(out.view(t.shape))
 
 
+def rope_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, rot: int, interleaved: bool, cos, sin,
+                pos: torch.Tensor, page: torch.Tensor, off: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor) -> bool:
+    """Prompt rows [T, H, D] (views of a fused projection): rotates q and k in place and writes k and v to row ``off`` of
+    page ``page`` (< 0: nowhere) of a cache [pages, Hkv, rows, D]. ``pos``, ``page``, ``off``: int32 [T]. One launch
+    (``csrc/kernels/rope_append.hip``); False, and nothing done, for tensors it does not take."""
+    code = {torch.bfloat16: 1, torch.float16: 2}.get(q.dtype)
+    T, H, D = q.shape
+    if (code is None or not q.is_cuda or any(t.dtype != q.dtype for t in (k, v, kc, vc))
+            or any(t.stride(2) != 1 for t in (q, k, v)) or not (kc.is_contiguous() and vc.is_contiguous())
+            or vc.shape != kc.shape or kc.shape[1] != k.shape[1] or kc.shape[3] != D or v.shape != k.shape):
+        return False
+    return _lib.call_rc("kca_rope_append", code, q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), q.stride(1),
+                        k.stride(0), k.stride(1), v.stride(0), v.stride(1), T, H, k.shape[1], D, rot, int(interleaved),
+                        _lib.ptr(cos), _lib.ptr(sin), pos.data_ptr(), page.data_ptr(), off.data_ptr(), kc.data_ptr(),
+                        vc.data_ptr(), kc.shape[2], _lib.stream()) == 0
+
+
 def rotary_reference(x: torch.Tensor, rot: int, interleaved: bool, base: float = 10000.0):
     """Out-of-place reference for tests: x [B, S, H, D]."""
     B, S, H, D = x.shape
@@ -97,4 +114,4 @@ def rotary_reference(x: torch.Tensor, rot: int, interleaved: bool, base: float =
     return out.view(B, S, H, D)
 
 
-__all__ = ["apply_rotary_", "rope_tables", "rotary_reference", "math"]
+__all__ = ["apply_rotary_", "rope_append", "rope_tables", "rotary_reference", "math"]
