@@ -1098,12 +1098,9 @@ KCA_API int kca_attn_fwd_packed(const void* q, const void* k, const void* v, voi
                      -1, -1, workspace, stream);
 }
 
-KCA_API int kca_attn_bwd_preprocess(const void* o, const void* dout,
-                                    float* delta, long long o_sb,
-                                    long long o_st, long long o_sh,
-                                    long long do_sb, long long do_st,
-                                    long long do_sh, int B, int S, int H,
-                                    int d_real, hipStream_t stream) {
+static int attn_bwd_preprocess(const void* o, const void* dout, float* delta, long long o_sb, long long o_st,
+                               long long o_sh, long long do_sb, long long do_st, long long do_sh, int B, int S, int H,
+                               int d_real, hipStream_t stream) {
   int nc = (d_real + 7) / 8;
   int tpr = 1;
   while (tpr < nc && tpr < 64) tpr <<= 1;
@@ -1116,8 +1113,9 @@ KCA_API int kca_attn_bwd_preprocess(const void* o, const void* dout,
   return 0;
 }
 
-KCA_API int kca_attn_bwd_tiled(const void* q, const void* k, const void* v, const void* dout,
-                               void* dq, void* dk, void* dv, const float* lse, const float* delta,
+KCA_API int kca_attn_bwd_tiled(const void* q, const void* k, const void* v, const void* o, long long o_sb,
+                               long long o_st, long long o_sh, const void* dout,
+                               void* dq, void* dk, void* dv, const float* lse, float* delta,
                                long long q_sb, long long q_st, long long q_sh, long long k_sb,
                                long long k_st, long long k_sh, long long v_sb, long long v_st,
                                long long v_sh, long long do_sb, long long do_st, long long do_sh,
@@ -1127,12 +1125,14 @@ KCA_API int kca_attn_bwd_tiled(const void* q, const void* k, const void* v, cons
                                int causal, float scale, const float* alibi, const int* kv_len, int window,
                                hipStream_t stream);
 
+// delta: scratch [B, H, Sq]
 KCA_API int kca_attn_bwd(const void* q, const void* k, const void* v,
                          const void* o, const void* dout, void* dq, void* dk,
-                         void* dv, const float* lse, const float* delta,
+                         void* dv, const float* lse, float* delta,
                          long long q_sb, long long q_st, long long q_sh,
                          long long k_sb, long long k_st, long long k_sh,
                          long long v_sb, long long v_st, long long v_sh,
+                         long long o_sb, long long o_st, long long o_sh,
                          long long do_sb, long long do_st, long long do_sh,
                          long long dq_sb, long long dq_st, long long dq_sh,
                          long long dk_sb, long long dk_st, long long dk_sh,
@@ -1142,11 +1142,12 @@ KCA_API int kca_attn_bwd(const void* q, const void* k, const void* v,
                          const int* kv_len, int window, const unsigned* key_mask, hipStream_t stream) {
   if (d_real % 8 || H % Hkv || window < 0) return 1;
   if (g_attn_tiled && !key_mask &&
-      kca_attn_bwd_tiled(q, k, v, dout, dq, dk, dv, lse, delta, q_sb, q_st, q_sh, k_sb, k_st, k_sh,
+      kca_attn_bwd_tiled(q, k, v, o, o_sb, o_st, o_sh, dout, dq, dk, dv, lse, delta, q_sb, q_st, q_sh, k_sb, k_st, k_sh,
                          v_sb, v_st, v_sh, do_sb, do_st, do_sh, dq_sb, dq_st, dq_sh, dk_sb, dk_st,
                          dk_sh, dv_sb, dv_st, dv_sh, B, Sq, Sk, H, Hkv, d_real, causal, scale, alibi, kv_len,
                          window, stream) == 0)
     return 0;
+  attn_bwd_preprocess(o, dout, delta, o_sb, o_st, o_sh, do_sb, do_st, do_sh, B, Sq, H, d_real, stream);
   const int D = pick_d(d_real);
   AttnBwdParams p{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)o,
                   (const bf16_t*)dout, (bf16_t*)dq, (bf16_t*)dk, (bf16_t*)dv, lse, delta,

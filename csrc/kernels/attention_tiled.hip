@@ -949,7 +949,10 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
 // Same image and fragment conventions as the forward. Two kernels, no float
 // atomics, deterministic:
 //   dQ kernel  : wave = 32 queries; Q, dO fragments resident, dQ^T in AGPRs;
-//                sweeps 32-key K/V tiles (double-buffered images).
+//                sweeps 32-key K/V tiles (double-buffered images). Runs first and leaves
+//                delta = rowsum(dO * O) for the other: its dO rows are at hand, so the pass of
+//                its own over O and dO goes (backward, us: 4 x 2048, 16 heads of 256 760 -> 746;
+//                8 x 1000, 12 heads of 64 145 -> 140).
 //                S^T = K.Q^T, dP^T = V.dO^T (keys on registers, query on the
 //                lane), dS^T = P^T (dP^T - delta), dQ^T += K^T.dS^T with K^T
 //                from the K image by transposed reads.
@@ -961,7 +964,7 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
 struct FastBwdParams {
   const bf16_t* q; const bf16_t* k; const bf16_t* v; const bf16_t* dout;
   bf16_t* dq; bf16_t* dk; bf16_t* dv;
-  const float* lse; const float* delta;
+  const float* lse; float* delta;
   long long q_sb, q_st, q_sh, k_sb, k_st, k_sh, v_sb, v_st, v_sh, do_sb, do_st, do_sh;
   long long dq_sb, dq_st, dq_sh, dk_sb, dk_st, dk_sh, dv_sb, dv_st, dv_sh;
   int B, Sq, Sk, H, Hkv;
@@ -969,6 +972,8 @@ struct FastBwdParams {
   const float* alibi;  // as in FastFwdParams
   const int* kv_len;
   int window;
+  const bf16_t* o;
+  long long o_sb, o_st, o_sh;
 };
 
 // A operand (32 rows x 16 k) read by rows from an image: lane (row l32, half hh)
@@ -1059,7 +1064,18 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 4 : 1) attn_
   const float slope = G == 2 ? p.alibi[h] * kLog2e : 0.f;
   const long long li = ((long long)b * p.H + h) * p.Sq + qr;
   const float nlse = -p.lse[li] * kLog2e;
-  const float dl = p.delta[li];
+  float dl = 0.f;
+  {
+    const bf16_t* op = p.o + b * p.o_sb + h * p.o_sh + (long long)qr * p.o_st;
+#pragma unroll
+    for (int s = 0; s < KSD; ++s) {
+      const bf16x8 of = *reinterpret_cast<const bf16x8*>(op + 16 * s + 8 * hh);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) dl = fmaf((float)of[j], (float)gf[s][j], dl);
+    }
+    dl += __shfl_xor(dl, 32, 64);
+    if (hh == 0 && (!G || qrow < p.Sq)) p.delta[li] = dl;
+  }
   f32x16 dq[D / 32];
 #pragma unroll
   for (int i = 0; i < D / 32; ++i)
@@ -1544,8 +1560,9 @@ KCA_API int kca_attn_fwd_wide(const void* q, const void* k, const void* v, void*
   return hipGetLastError() == hipSuccess ? 0 : 3;
 }
 
-KCA_API int kca_attn_bwd_tiled(const void* q, const void* k, const void* v, const void* dout,
-                               void* dq, void* dk, void* dv, const float* lse, const float* delta,
+KCA_API int kca_attn_bwd_tiled(const void* q, const void* k, const void* v, const void* o, long long o_sb,
+                               long long o_st, long long o_sh, const void* dout,
+                               void* dq, void* dk, void* dv, const float* lse, float* delta,
                                long long q_sb, long long q_st, long long q_sh, long long k_sb,
                                long long k_st, long long k_sh, long long v_sb, long long v_st,
                                long long v_sh, long long do_sb, long long do_st, long long do_sh,
@@ -1561,65 +1578,65 @@ KCA_API int kca_attn_bwd_tiled(const void* q, const void* k, const void* v, cons
                   (bf16_t*)dq, (bf16_t*)dk, (bf16_t*)dv, lse, delta,
                   q_sb, q_st, q_sh, k_sb, k_st, k_sh, v_sb, v_st, v_sh, do_sb, do_st, do_sh,
                   dq_sb, dq_st, dq_sh, dk_sb, dk_st, dk_sh, dv_sb, dv_st, dv_sh,
-                  B, Sq, Sk, H, Hkv, scale, alibi, kv_len, window};
+                  B, Sq, Sk, H, Hkv, scale, alibi, kv_len, window, (const bf16_t*)o, o_sb, o_st, o_sh};
   dim3 g1(((Sk + 127) / 128) * B * Hkv), g2(((Sq + 127) / 128) * B * H);
   if (alibi || kv_len || window || Sq % 128 || Sk % 128) {
     if (!rows16(q, q_sb, q_st, q_sh) || !rows16(k, k_sb, k_st, k_sh) || !rows16(v, v_sb, v_st, v_sh) ||
-        !rows16(dout, do_sb, do_st, do_sh) || !rows16(dq, dq_sb, dq_st, dq_sh) || !rows16(dk, dk_sb, dk_st, dk_sh) ||
+        !rows16(o, o_sb, o_st, o_sh) || !rows16(dout, do_sb, do_st, do_sh) || !rows16(dq, dq_sb, dq_st, dq_sh) || !rows16(dk, dk_sb, dk_st, dk_sh) ||
         !rows16(dv, dv_sb, dv_st, dv_sh))
       return 1;
     const bool done = general_form(d, causal, alibi, [&](auto D_, auto C_, auto G_) {
       constexpr int D = decltype(D_)::value, G = decltype(G_)::value;
       constexpr bool C = decltype(C_)::value;
-      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<D, C, D, G>), g1, dim3(256), 0, stream, p);
       hipLaunchKernelGGL((attn_bwd_dq_tiled_kernel<D, C, D, G>), g2, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<D, C, D, G>), g1, dim3(256), 0, stream, p);
     });
     return done ? 0 : 1;
   }
   if (d != 48 && d != 64 && d != 96 && d != 128 && d != 160 && d != 256) return 1;
   if (d == 48 && causal) return 1;  // narrow storage: SD-1.5's (non-causal) 40-wide heads
   if (d == 48) {  // heads stored 48 wide in D = 64 images (the UNet's 40-wide heads, training)
-    hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<64, false, 48>), g1, dim3(256), 0, stream, p);
     hipLaunchKernelGGL((attn_bwd_dq_tiled_kernel<64, false, 48>), g2, dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<64, false, 48>), g1, dim3(256), 0, stream, p);
   } else if (d == 256) {
     if (causal) {
-      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<256, true>), g1, dim3(256), 0, stream, p);
       hipLaunchKernelGGL((attn_bwd_dq_tiled_kernel<256, true>), g2, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<256, true>), g1, dim3(256), 0, stream, p);
     } else {
-      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<256, false>), g1, dim3(256), 0, stream, p);
       hipLaunchKernelGGL((attn_bwd_dq_tiled_kernel<256, false>), g2, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<256, false>), g1, dim3(256), 0, stream, p);
     }
   } else if (d == 160) {
     if (causal) {
-      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<160, true>), g1, dim3(256), 0, stream, p);
       hipLaunchKernelGGL((attn_bwd_dq_tiled_kernel<160, true>), g2, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<160, true>), g1, dim3(256), 0, stream, p);
     } else {
-      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<160, false>), g1, dim3(256), 0, stream, p);
       hipLaunchKernelGGL((attn_bwd_dq_tiled_kernel<160, false>), g2, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<160, false>), g1, dim3(256), 0, stream, p);
     }
   } else if (d == 96) {
     if (causal) {
-      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<96, true>), g1, dim3(256), 0, stream, p);
       hipLaunchKernelGGL((attn_bwd_dq_tiled_kernel<96, true>), g2, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<96, true>), g1, dim3(256), 0, stream, p);
     } else {
-      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<96, false>), g1, dim3(256), 0, stream, p);
       hipLaunchKernelGGL((attn_bwd_dq_tiled_kernel<96, false>), g2, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<96, false>), g1, dim3(256), 0, stream, p);
     }
   } else if (d == 128) {
     if (causal) {
-      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<128, true>), g1, dim3(256), 0, stream, p);
       hipLaunchKernelGGL((attn_bwd_dq_tiled_kernel<128, true>), g2, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<128, true>), g1, dim3(256), 0, stream, p);
     } else {
-      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<128, false>), g1, dim3(256), 0, stream, p);
       hipLaunchKernelGGL((attn_bwd_dq_tiled_kernel<128, false>), g2, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<128, false>), g1, dim3(256), 0, stream, p);
     }
   } else {
     if (causal) {
-      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<64, true>), g1, dim3(256), 0, stream, p);
       hipLaunchKernelGGL((attn_bwd_dq_tiled_kernel<64, true>), g2, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<64, true>), g1, dim3(256), 0, stream, p);
     } else {
-      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<64, false>), g1, dim3(256), 0, stream, p);
       hipLaunchKernelGGL((attn_bwd_dq_tiled_kernel<64, false>), g2, dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<64, false>), g1, dim3(256), 0, stream, p);
     }
   }
   return 0;

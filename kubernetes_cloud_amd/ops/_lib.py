@@ -67,8 +67,7 @@ _SIGS = {
     "kca_adamw8bit": [P, P, P, P, P, P, P, LL, P, F, F, F, F, F, F, F, P, P, P],
     "kca_clip_coef": [P, F, F, P, P, P, P],
     "kca_attn_fwd": [P] * 5 + [LL] * 12 + [I] * 7 + [F, P, P, I, P, I, I, P, P],
-    "kca_attn_bwd_preprocess": [P, P, P, LL, LL, LL, LL, LL, LL, I, I, I, I, P],
-    "kca_attn_bwd": [P] * 10 + [LL] * 21 + [I] * 7 + [F, P, P, I, P, P],
+    "kca_attn_bwd": [P] * 10 + [LL] * 24 + [I] * 7 + [F, P, P, I, P, P],
     "kca_attn_fwd_packed": [P] * 4 + [LL] * 8 + [I] * 6 + [F, P, I, P, P, P],
     "kca_rope_append": [I, P, P, P] + [LL] * 6 + [I] * 6 + [P] * 7 + [I, P],
     "kca_attn_fwd_wide": [P] * 5 + [LL] * 12 + [I] * 6 + [F, P, P],

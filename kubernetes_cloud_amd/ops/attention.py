@@ -125,11 +125,9 @@ def _bwd(q, k, v, o, do, lse, dq, dk, dv, causal, scale, kv_len, alibi, window: 
     B, Sq, H, D = q.shape
     Sk, Hkv = k.shape[1], k.shape[2]
     delta = torch.empty(B, H, Sq, device=q.device, dtype=torch.float32)
-    _lib.call("kca_attn_bwd_preprocess", o.data_ptr(), do.data_ptr(), delta.data_ptr(),
-              *_strides(o), *_strides(do), B, Sq, H, D, _lib.stream())
     _lib.call("kca_attn_bwd", q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(),
               dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), lse.data_ptr(), delta.data_ptr(),
-              *_strides(q), *_strides(k), *_strides(v), *_strides(do),
+              *_strides(q), *_strides(k), *_strides(v), *_strides(o), *_strides(do),
               *_strides(dq), *_strides(dk), *_strides(dv),
               B, Sq, Sk, H, Hkv, D, int(causal), float(scale), _lib.ptr(alibi), _lib.ptr(_masks(kv_len)[0]),
               int(window), _lib.ptr(_masks(kv_len)[1]), _lib.stream())
