@@ -83,7 +83,7 @@ def set_variant(v: int) -> int:
 
 
 def _strides(t):
-    return t.stride(0), t.stride(1), t.stride(2)
+    return t.stride()[:3]
 
 
 def pack_key_mask(mask: torch.Tensor) -> torch.Tensor:
