@@ -13,6 +13,7 @@
 //   group   assignments sorted by expert and cut in row tiles that hold one expert each
 //   gemv    expert products of tiles of up to 8 rows: streams the weight rows on the vector units
 //           (decode; any dims, fp32 too)
+//   stream  expert products of tiles of up to 32 rows on the matrix cores (large decode batches, short prompts)
 //   gemm    expert products of tiles of up to 128 rows on the matrix cores (prompts)
 // Expert weights are stacked: gate-and-up [E][2F][d] (gate rows first), down [E][d][F]. The sorted rows'
 // activations are [n][F], their outputs [n][d]; the residual pass (rms_shift.hip) sums a token's outputs
@@ -455,6 +456,136 @@ __global__ void __launch_bounds__(256) expert_gemv_kernel(ExpertArgs p) {
   }
 }
 
+// ---------------------------------------------------------------------------------------------- stream
+// bf16, tiles of up to 32 rows x 128 weight rows (up: 64 gate rows and the 64 up rows beside them) x 64 per stage,
+// 4 waves of 32 weight rows. Bound by the weight stream: a stage's 16 KiB of weights and 4 KiB of activations go
+// straight to LDS (no registers, so three stages a workgroup and two workgroups a CU are in flight, 120 KiB), and
+// the products (16x16x32 tiles, weights as the A operand: a lane holds one activation row and four outputs) hide
+// under it. Beside the gemv kernel, whose vector products a row cost more than its weights from about 4 rows an
+// expert on, and the 128-row gemm, which computes and stages mostly padding: both products of 32 tokens, 16 experts of
+// 3 x 4096 x 2048, top 3: 190 us (gemv), 192 (gemm), 172 (4.7 TB/s); 100 tokens 450, 197, 175 (tile_rows in ops/moe.py).
+// K % 64 == 0 and N % 16 == 0; an LDS-DMA instruction fills 8 rows of 128 bytes lane by lane, so the 16-byte pieces
+// are swizzled (by row pair: 16 rows x one piece cover all 64 banks) on the source address.
+constexpr int SROWS = 32, SK = 64, SWN = 128, SST = (SWN + SROWS) * SK * 2, SNB = 4, STREAM_LDS = SNB * SST;
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rsrc(const void* p) {
+  const unsigned long long a = (unsigned long long)p;
+  const unsigned long long u = ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(a >> 32)) << 32) |
+                               (unsigned)__builtin_amdgcn_readfirstlane((unsigned)a);
+  return __builtin_amdgcn_make_buffer_rsrc((void*)u, (short)0, 0x7fffffff, 0x00020000);
+}
+
+// four 16-byte LDS reads and their wait in one piece (hipcc would drain every LDS-DMA in flight before a read it sees)
+__device__ __forceinline__ void lds_read4(unsigned a0, unsigned a1, unsigned a2, unsigned a3, u32x4& r0, u32x4& r1,
+                                          u32x4& r2, u32x4& r3) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile(
+      "ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %6\n\tds_read_b128 %3, %7\n\ts_waitcnt lgkmcnt(0)"
+      : "=&v"(r0), "=&v"(r1), "=&v"(r2), "=&v"(r3)
+      : "v"(a0), "v"(a1), "v"(a2), "v"(a3)
+      : "memory");
+#endif
+}
+
+template <bool UP>
+__global__ void __launch_bounds__(256, 2) expert_stream_kernel(ExpertArgs p) {
+  extern __shared__ __attribute__((aligned(1024))) char sl[];  // [SNB][128 weight rows | 32 activation rows][128 B]
+  constexpr int NB = UP ? SWN / 2 : SWN;
+  const int nt = *p.ntiles, nb = (p.N + NB - 1) / NB;
+  if ((int)blockIdx.x >= nt * nb) return;
+  const int id = xcd_remap(blockIdx.x, nt * nb);  // the order of expert_gemm_kernel
+  const int* t0 = p.tiles + id / nb * 5;
+  const int in = id - t0[3] * nb, tile = t0[3] + in % t0[4], bn = in / t0[4];
+  const int* tl = p.tiles + tile * 5;
+  const int ex = tl[0], lo = tl[1], nr = tl[2], K = p.K, N = p.N, n0 = bn * NB;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
+  // sources: a wave fills its own 32 weight rows (4 pieces of 8) and 8 of the activation rows
+  const __amdgpu_buffer_rsrc_t rw =
+      uniform_rsrc(reinterpret_cast<const bf16_t*>(p.w) + (long long)ex * (UP ? 2 * N : N) * K);
+  const __amdgpu_buffer_rsrc_t rx = uniform_rsrc(p.x);
+  int wo[4], xo;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = 8 * i + (lane >> 3);  // of the wave's 32
+    const int n = UP ? (r < 16 ? 0 : N) + min(n0 + wv * 16 + (r & 15), N - 1) : min(n0 + wv * 32 + r, N - 1);
+    wo[i] = (n * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
+  }
+  {
+    const int r = wv * 8 + (lane >> 3), xr = lo + min(r, nr - 1);
+    xo = ((UP ? p.perm[xr] / p.top : xr) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
+  }
+  typedef __attribute__((address_space(3))) char lds_char;
+  lds_char* lsm = (lds_char*)sl;
+  const int nk = K / SK;
+  auto issue = [&](int t) {
+    const int k = __builtin_amdgcn_readfirstlane(min(t, nk - 1) * SK * 2);  // the last stages repeat one that nobody reads
+    lds_char* st = lsm + (t % SNB) * SST;
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (void __attribute__((address_space(3)))*)(st + (wv * 4 + i) * 1024), 16,
+                                               wo[i], k, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (void __attribute__((address_space(3)))*)(st + (16 + wv) * 1024), 16, xo,
+                                             k, 0, 0);
+#endif
+  };
+  f32x4 acc[2][2];  // [gate, up | two runs of 16 outputs][16 rows]
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i][j][e] = 0.f;
+  const unsigned base = (unsigned)(size_t)lsm, sw = (r16 >> 1) & 7;
+  const unsigned aw = (wv * 32 + r16) * 128, ax = (SWN + r16) * 128;
+#pragma unroll
+  for (int t = 0; t < SNB - 1; ++t) issue(t);
+  for (int t = 0; t < nk; ++t) {
+    // this wave's pieces of stage t have landed (two younger stages may be in flight), then everybody's
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SNB - 2) * 5) : "memory");
+    __builtin_amdgcn_s_barrier();
+    issue(t + SNB - 1);  // into the buffer of stage t - 1, which all waves have left
+    const unsigned st = base + (t % SNB) * SST;
+#pragma unroll
+    for (int s = 0; s < SK / 32; ++s) {
+      const unsigned c = ((4 * s + g) ^ sw) * 16;
+      u32x4 a0, a1, x0, x1;
+      lds_read4(st + aw + c, st + aw + 16 * 128 + c, st + ax + c, st + ax + 16 * 128 + c, a0, a1, x0, x1);
+      const bf16x8 A0 = __builtin_bit_cast(bf16x8, a0), A1 = __builtin_bit_cast(bf16x8, a1);
+      const bf16x8 X0 = __builtin_bit_cast(bf16x8, x0), X1 = __builtin_bit_cast(bf16x8, x1);
+      acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A0, X0, acc[0][0], 0, 0, 0);
+      acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A1, X0, acc[1][0], 0, 0, 0);
+      acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A0, X1, acc[0][1], 0, 0, 0);
+      acc[1][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A1, X1, acc[1][1], 0, 0, 0);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the repeated stages, before the LDS is given back
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int r = 16 * j + r16;
+    if (r >= nr) continue;
+    const float s = p.scale ? p.wts[p.perm[lo + r]] : 1.f;
+    bf16_t* y = reinterpret_cast<bf16_t*>(p.y) + (long long)(lo + r) * N;
+#pragma unroll
+    for (int i = 0; i < (UP ? 1 : 2); ++i) {
+      const int n = n0 + wv * (UP ? 16 : 32) + 16 * i + 4 * g;
+      if (n >= N) continue;
+      float o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (UP) {
+          const float gt = acc[0][j][e] * s, up = acc[1][j][e] * s;
+          o[e] = gt * __builtin_amdgcn_rcpf(1.f + __expf(-gt)) * up;
+        } else {
+          o[e] = acc[i][j][e] * s;
+        }
+      }
+      *reinterpret_cast<uint2*>(y + n) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+    }
+  }
+}
+
 // ------------------------------------------------------------------------------------------------ gemm
 // bf16, 128 rows x 256 weight rows x 64 per step, 8 waves of 64 x 64 (32x32x16 tiles); weights are the A
 // operand, so a lane holds one activation row and runs of four outputs. up: a workgroup covers 128 gate
@@ -689,13 +820,14 @@ KCA_API int kca_moe_route_group(const void* h, const void* wr, const void* wsg, 
   return route_go<16, true>(a, g, s);
 }
 
-// One expert product of every tile. mt: the tiles' row limit (1, 2, 4, 8: gemv; 128: gemm, bf16 with
-// K % 8 == 0 and N % 4 == 0). ws: a shared expert's product over all tokens beside them (gemv; nullable).
+// One expert product of every tile. mt: the tiles' row limit (1, 2, 4, 8: gemv; 32: stream, bf16 with K % 64 == 0 and
+// N % 16 == 0; 128: gemm, bf16 with K % 8 == 0 and N % 4 == 0). x_rows: rows of x. ws: a shared expert's product over all tokens beside them (gemv; nullable).
 KCA_API int kca_moe_expert(int dtype, const void* x, const void* w, void* y, const void* perm, const void* wts,
                            const void* tiles, const void* ntiles, int max_tiles, int mt, int top, int N, int K, int up,
-                           int scale, const void* xs, const void* ws, void* ys, int tokens, int Ns, int Ks, hipStream_t s) {
+                           int scale, const void* xs, const void* ws, void* ys, int tokens, int Ns, int Ks, int x_rows,
+                           hipStream_t s) {
   if (max_tiles < 1 || max_tiles > 32767 || N < 1 || K < 1 || top < 1 || !x || !w || !y || !perm || !wts || !tiles || !ntiles) return 1;
-  if (ws && (!xs || !ys || tokens < 1 || tokens > 32767 || Ns < 1 || Ks < 1 || mt == 128)) return 1;
+  if (ws && (!xs || !ys || tokens < 1 || tokens > 32767 || Ns < 1 || Ks < 1 || mt > 8)) return 1;
   const ExpertArgs a{x, w, y, (const int*)perm, (const float*)wts, (const int*)tiles, (const int*)ntiles, top, N, K, up, scale,
                      xs, ws, ys, tokens, Ns, Ks};
   if (mt == 128) {
@@ -704,6 +836,16 @@ KCA_API int kca_moe_expert(int dtype, const void* x, const void* w, void* y, con
     if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS) != hipSuccess) return 5;
     if (up) hipLaunchKernelGGL(expert_gemm_kernel<true>, dim3((N + 127) / 128 * max_tiles), dim3(512), GEMM_LDS, s, a);
     else hipLaunchKernelGGL(expert_gemm_kernel<false>, dim3((N + 255) / 256 * max_tiles), dim3(512), GEMM_LDS, s, a);
+    return hipGetLastError() == hipSuccess ? 0 : 4;
+  }
+  if (mt == SROWS) {
+    if (dtype != 1 || K % SK || N % 16 || !al16(x) || !al16(w) || (uintptr_t)y % 8 || 2ll * (up ? 2 * N : N) * K >= 1ll << 31 ||
+        2ll * x_rows * K >= 1ll << 31)  // (32-bit byte offsets)
+      return 10;
+    const void* kern = up ? (const void*)expert_stream_kernel<true> : (const void*)expert_stream_kernel<false>;
+    if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, STREAM_LDS) != hipSuccess) return 5;
+    if (up) hipLaunchKernelGGL(expert_stream_kernel<true>, dim3((N + SWN / 2 - 1) / (SWN / 2) * max_tiles), dim3(256), STREAM_LDS, s, a);
+    else hipLaunchKernelGGL(expert_stream_kernel<false>, dim3((N + SWN - 1) / SWN * max_tiles), dim3(256), STREAM_LDS, s, a);
     return hipGetLastError() == hipSuccess ? 0 : 4;
   }
   const int v = dtype == 1 ? 8 : 4;

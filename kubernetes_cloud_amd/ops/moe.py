@@ -15,6 +15,7 @@ from . import _lib
 from .rms_shift import native_dt
 
 GEMM_ROWS = 128
+STREAM_ROWS = 32
 SHARED_ROWS = 16  # tokens up to which a shared expert's weights stream beside the routed ones'
 
 
@@ -80,11 +81,27 @@ class Groups:
 
 
 def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
-    """Row limit of an expert tile: the matrix-core product (128) once an active expert expects enough rows
-    to be worth a tile, else a streaming product of 1 .. 8 rows."""
-    gemm = dtype == torch.bfloat16 and d % 8 == 0 and F % 8 == 0
-    if gemm and T * top > 16 * min(E, T * top):
-        return GEMM_ROWS
+    """Row limit of an expert tile, by the rows that an expert expects: a streaming vector product (1 .. 8), the weight
+    stream on the matrix cores (32), or the prompts' product (128).
+
+    Both products, us, vector / stream / prompts' product (width, experts, top, inner size):
+
+        4096, 16, 2, 4096   24 tokens 270 / 273 / 285   32: 312 / 291 / 304   100: 716 / 296 / 310   250: - / 322 / 315
+        2048, 32, 4, 1024   12 tokens  71 /  74 /  86   16:  84 /  79 /  93   100: 265 /  89 / 101   250: - /  99 / 107
+        4096, 20, 3, 2048   24 tokens 165 / 166 / 189   32: 190 / 172 / 192   100: 450 / 175 / 197   250: - / 197 / 205
+        2048, 32, 5, 768    12 tokens  53 /  51 /  63   32:  83 /  61 /  62   100: 205 /  62 /  71   250: - /  70 /  74
+
+    so the matrix cores take over at about 3 rows an expert, at 2 where a row is short (a wave's reduction is then a
+    larger part of its stream); up to 16 tokens the vector product also carries the shared expert. A stream tile
+    holds 32 rows: past that an expert's weights are read again."""
+    n = T * top
+    used = min(E, n)
+    if dtype == torch.bfloat16 and d % 8 == 0 and F % 8 == 0:
+        stream = d % 64 == 0 and F % 64 == 0 and max(4 * F * d, 2 * n * max(d, F)) < 2 ** 31
+        if n > (32 if stream else 4) * used:
+            return GEMM_ROWS
+        if stream and T > SHARED_ROWS and n > (3 if d > 2048 else 2) * used:
+            return STREAM_ROWS
     return 1 if T == 1 else 2 if T == 2 else 4 if T <= 4 else 8
 
 
@@ -136,7 +153,7 @@ def group(ids: torch.Tensor, E: int, mt: int) -> Groups:
 
 def shared_ok(T: int, mt: int) -> bool:
     """Whether a shared expert streams beside the routed ones' (``experts``): few tokens, streaming products."""
-    return mt != GEMM_ROWS and T <= SHARED_ROWS
+    return mt <= 8 and T <= SHARED_ROWS
 
 
 def experts(h: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor,
@@ -175,9 +192,9 @@ def experts(h: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, gate_up: 
         up_s = (h.data_ptr(), w_up.data_ptr(), act_s.data_ptr(), T, Fs, d)
         down_s = (act_s.data_ptr(), w_down.data_ptr(), y_s.data_ptr(), T, d, Fs)
     _lib.call("kca_moe_expert", code, h.data_ptr(), gate_up.data_ptr(), act.data_ptr(), *common, F, d, 1,
-              int(scale_in), *up_s, _lib.stream())
+              int(scale_in), *up_s, T, _lib.stream())
     _lib.call("kca_moe_expert", code, act.data_ptr(), down.data_ptr(), y.data_ptr(), *common, d, F, 0,
-              int(not scale_in), *down_s, _lib.stream())
+              int(not scale_in), *down_s, n, _lib.stream())
     return y if shared is None else (y, y_s)
 
 

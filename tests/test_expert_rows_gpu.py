@@ -1,0 +1,39 @@
+"""Expert products on the matrix cores where their tiles can go wrong: rows an expert from none to one past a tile, one and
+many stages, output blocks that end early -- against fp32 products of the same bf16 operands."""
+import pytest
+import torch
+
+from kubernetes_cloud_amd.ops import moe
+
+pytestmark = pytest.mark.gpu
+# the activation and the result are rounded to bf16 once each (2^-9), the products are summed in fp32
+TOL = 2.5 * 2.0 ** -9
+
+
+def _case(counts, top, d, F, seed=0):
+    """Ids with ``counts[e]`` rows of expert e, shuffled."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    flat = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])
+    assert flat.numel() % top == 0
+    ids = flat[torch.randperm(flat.numel(), generator=torch.Generator().manual_seed(seed))].view(-1, top).int().cuda()
+    T, E = ids.shape[0], len(counts)
+    r = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    return (r(T, d).bfloat16(), ids, torch.rand(T, top, device="cuda", generator=g), (r(E, 2 * F, d) * d ** -0.5).bfloat16(),
+            (r(E, d, F) * F ** -0.5).bfloat16())
+
+
+@pytest.mark.parametrize("mt", [moe.STREAM_ROWS, moe.GEMM_ROWS])
+@pytest.mark.parametrize("scale_in", [True, False])
+@pytest.mark.parametrize("counts,top,d,F", [([0, 1, 16, 17, 32, 33, 15], 2, 64, 64), ([31, 64, 65, 0, 8], 3, 320, 192),
+                                            ([1], 1, 128, 64), ([129, 127, 256, 2], 2, 192, 320), ([40, 40], 4, 64, 576)])
+def test_products(mt, scale_in, counts, top, d, F):
+    h, ids, wts, gu, dn = _case(counts, top, d, F)
+    g = moe.group(ids, len(counts), mt)
+    y = moe.experts(h, ids, wts, gu, dn, g, scale_in)[g.inv.long()]
+    e = ids.long()
+    u = torch.einsum("td,tkfd->tkf", h.float(), gu.float()[e])
+    w = wts[..., None]
+    u = u * w if scale_in else u
+    a = (torch.nn.functional.silu(u[..., :F]) * u[..., F:]).bfloat16().float()
+    want = torch.einsum("tkf,tkdf->tkd", a, dn.float()[e]) * (1 if scale_in else w)
+    assert (y.float() - want).norm() <= TOL * want.norm()
