@@ -14,7 +14,7 @@
 //   gemv    expert products of tiles of up to 8 rows: streams the weight rows on the vector units
 //           (decode; any dims, fp32 too)
 //   stream  expert products of tiles of up to 32 rows on the matrix cores (large decode batches, short prompts)
-//   gemm    expert products of tiles of up to 128 rows on the matrix cores (prompts)
+//   gemm    expert products of tiles of up to 256 rows on the matrix cores (prompts)
 // Expert weights are stacked: gate-and-up [E][2F][d] (gate rows first), down [E][d][F]. The sorted rows'
 // activations are [n][F], their outputs [n][d]; the residual pass (rms_shift.hip) sums a token's outputs
 // through `inv`.
@@ -462,17 +462,18 @@ __global__ void __launch_bounds__(256) expert_gemv_kernel(ExpertArgs p) {
 // straight to LDS (no registers, so three stages a workgroup and two workgroups a CU are in flight, 120 KiB), and
 // the products (16x16x32 tiles, weights as the A operand: a lane holds one activation row and four outputs) hide
 // under it. Beside the gemv kernel, whose vector products a row cost more than its weights from about 4 rows an
-// expert on, and the 128-row gemm, which computes and stages mostly padding: both products of 32 tokens, 16 experts of
+// expert on, and the gemm, which computes and stages mostly padding: both products of 32 tokens, 16 experts of
 // 3 x 4096 x 2048, top 3: 190 us (gemv), 192 (gemm), 172 (4.7 TB/s); 100 tokens 450, 197, 175 (tile_rows in ops/moe.py).
 // K % 64 == 0 and N % 16 == 0; an LDS-DMA instruction fills 8 rows of 128 bytes lane by lane, so the 16-byte pieces
 // are swizzled (by row pair: 16 rows x one piece cover all 64 banks) on the source address.
 constexpr int SROWS = 32, SK = 64, SWN = 128, SST = (SWN + SROWS) * SK * 2, SNB = 4, STREAM_LDS = SNB * SST;
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rsrc(const void* p) {
+// `bytes`: loads past them return zeros
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rsrc(const void* p, unsigned bytes = ~0u) {
   const unsigned long long a = (unsigned long long)p;
   const unsigned long long u = ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(a >> 32)) << 32) |
                                (unsigned)__builtin_amdgcn_readfirstlane((unsigned)a);
-  return __builtin_amdgcn_make_buffer_rsrc((void*)u, (short)0, 0x7fffffff, 0x00020000);
+  return __builtin_amdgcn_make_buffer_rsrc((void*)u, (short)0, (int)bytes, 0x00020000);
 }
 
 // four 16-byte LDS reads and their wait in one piece (hipcc would drain every LDS-DMA in flight before a read it sees)
@@ -503,17 +504,17 @@ __global__ void __launch_bounds__(256, 2) expert_stream_kernel(ExpertArgs p) {
   // sources: a wave fills its own 32 weight rows (4 pieces of 8) and 8 of the activation rows
   const __amdgpu_buffer_rsrc_t rw =
       uniform_rsrc(reinterpret_cast<const bf16_t*>(p.w) + (long long)ex * (UP ? 2 * N : N) * K);
-  const __amdgpu_buffer_rsrc_t rx = uniform_rsrc(p.x);
-  int wo[4], xo;
+  const __amdgpu_buffer_rsrc_t rx = uniform_rsrc(reinterpret_cast<const bf16_t*>(p.x) + (UP ? 0ll : (long long)lo * K));
+  unsigned wo[4], xo;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = 8 * i + (lane >> 3);  // of the wave's 32
     const int n = UP ? (r < 16 ? 0 : N) + min(n0 + wv * 16 + (r & 15), N - 1) : min(n0 + wv * 32 + r, N - 1);
-    wo[i] = (n * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
+    wo[i] = ((unsigned)n * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
   }
   {
-    const int r = wv * 8 + (lane >> 3), xr = lo + min(r, nr - 1);
-    xo = ((UP ? p.perm[xr] / p.top : xr) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
+    const int r = wv * 8 + (lane >> 3), xr = min(r, nr - 1);
+    xo = ((unsigned)(UP ? p.perm[lo + xr] / p.top : xr) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
   }
   typedef __attribute__((address_space(3))) char lds_char;
   lds_char* lsm = (lds_char*)sl;
@@ -587,138 +588,154 @@ __global__ void __launch_bounds__(256, 2) expert_stream_kernel(ExpertArgs p) {
 }
 
 // ------------------------------------------------------------------------------------------------ gemm
-// bf16, 128 rows x 256 weight rows x 64 per step, 8 waves of 64 x 64 (32x32x16 tiles); weights are the A
-// operand, so a lane holds one activation row and runs of four outputs. up: a workgroup covers 128 gate
-// and the matching 128 up rows, each wave 32 of both.
-constexpr int GBK = 64, GN = 256, GM = 128, GEMM_LDS = 2 * (GN + GM) * GBK * 2;
+// bf16, tiles of up to 256 rows x 256 weight rows (up: 128 gate rows and the 128 up rows beside them) x 64 per stage;
+// weights are the A operand, so a lane holds one activation row and runs of four outputs.
+// Bound by the LDS: 8 waves of 64 x 64 (the form before, 128 rows x 256) read a fragment per product, 128 bytes a cycle
+// beside the stores; 4 waves of 128 x 128, one a SIMD, read half a fragment per product. A wave alone on its SIMD has to
+// hide everything itself: fragments one sub-step ahead, loads two stages ahead, loads and LDS stores spread over the
+// products (pinned: hipcc requests everything at a stage's end, 1182 us instead of 904 below), the barrier before the
+// last sub-step. Tiles of fewer rows run 4 waves of 64 weight rows x all rows instead, in steps of 32.
+// Narrow blocks (128 weight rows, tiles to 192 rows, two workgroups a CU) fill the chip with a quarter of the work.
+// Both products of 4096 tokens, 16 experts of 3 x 4096 x 4096, top 2: 1143 -> 904 us (913 TFLOP/s without padding);
+// 16 experts of 3 x 4096 x 2048, top 3: 764 -> 541; 1000 tokens, 32 experts of 3 x 2048 x 1024, top 4: 148 -> 116.
+constexpr int GBK = 64, GN = 256, GM = 256, GEMM_LDS = 2 * (GN + GM) * GBK * 2;
 
-template <bool UP>
-__global__ void __launch_bounds__(512, 2) expert_gemm_kernel(ExpertArgs p) {
-  constexpr int BK = GBK;
-  extern __shared__ __attribute__((aligned(16))) bf16_t gl[];  // [2][GN + GM][BK]: weight rows, then activation rows
-  bf16_t *const sw[2] = {gl, gl + (GN + GM) * BK}, *const sx[2] = {gl + GN * BK, gl + (2 * GN + GM) * BK};
-  // order: an XCD works a contiguous run of (expert, weight block, row tile), so the row tiles that share a
-  // weight block are on one XCD at one time
-  const int nt = *p.ntiles, nb = (p.N + (UP ? 127 : 255)) / (UP ? 128 : 256);
-  if ((int)blockIdx.x >= nt * nb) return;
-  const int id = xcd_remap(blockIdx.x, nt * nb);
-  const int* t0 = p.tiles + id / nb * 5;
-  const int in = id - t0[3] * nb, tile = t0[3] + in % t0[4], bn = in / t0[4];
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, l32 = lane & 31, hh = lane >> 5;
-  const int wn = wv >> 1, wm = wv & 1;
-  const int* tl = p.tiles + tile * 5;
-  const int ex = tl[0], lo = tl[1], nr = tl[2], K = p.K, N = p.N;
-  const int n0 = bn * (UP ? 128 : 256);
-  // staging: thread tid owns 16-B chunk tid % 8 of rows tid / 8 + 64 i
+// WN x WM waves, each with AI runs of 32 weight rows and BJ of 32 rows
+template <bool UP, int WN, int AI, int WM, int BJ>
+__device__ __forceinline__ void expert_gemm_tile(const ExpertArgs& p, bf16_t* gl, int ex, int lo, int nr, int n0) {
+  constexpr int WP = WN * AI, RP = WM * BJ, NP = WP + RP;  // staging passes of 32 rows: weights, activations
+  constexpr int STG = NP * 32 * GBK;                       // one stage (elements)
+  static_assert(WN * WM == 4 && AI % 2 == 0, "four waves, gate runs beside up runs");
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), wn = wv % WN, wm = wv / WN;
+  const int K = p.K, N = p.N;
+  // staging: thread tid owns the 16-byte piece tid % 8 of rows tid / 8 + 32 i
   const int ch = tid & 7, sr = tid >> 3;
-  const bf16_t *wp[4], *xp[2];
+  const __amdgpu_buffer_rsrc_t rw =
+      uniform_rsrc(reinterpret_cast<const bf16_t*>(p.w) + (long long)ex * (UP ? 2 * N : N) * K);
+  constexpr unsigned OUT = 1u << 31;  // past the activations: a stage past K multiplies zeros
+  const __amdgpu_buffer_rsrc_t rx = uniform_rsrc(reinterpret_cast<const bf16_t*>(p.x) + (UP ? 0ll : (long long)lo * K), OUT);
+  unsigned wo[WP], xo[RP];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = sr + 64 * i;
-    long long wr;
-    if constexpr (UP) wr = (r < 128 ? 0 : N) + min(n0 + (r & 127), N - 1);
-    else wr = min(n0 + r, N - 1);
-    wp[i] = reinterpret_cast<const bf16_t*>(p.w) + ((long long)ex * (UP ? 2 * N : N) + wr) * K;
+  for (int i = 0; i < WP; ++i) {
+    const int r = sr + 32 * i;
+    // (up: a wave's rows are AI / 2 runs of 32 gate rows, then the same up rows)
+    const int run = r / 32, wrun = run % AI, base = run / AI * (AI / 2) * 32;
+    const int n = UP ? (wrun < AI / 2 ? 0 : N) + min(n0 + base + wrun % (AI / 2) * 32 + (r & 31), N - 1) : min(n0 + r, N - 1);
+    wo[i] = (unsigned)n * K * 2;
   }
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int r = sr + 64 * i, xr = lo + min(r, nr - 1);
-    const long long src = UP ? p.perm[xr] / p.top : xr;
-    xp[i] = reinterpret_cast<const bf16_t*>(p.x) + src * K;
+  for (int i = 0; i < RP; ++i) {
+    const int xr = min(sr + 32 * i, nr - 1);
+    xo[i] = (unsigned)(UP ? p.perm[lo + xr] / p.top : xr) * K * 2;
   }
-  // Two k steps in flight in registers (a step's products alone do not cover a trip past L2). No load or
-  // store of the loop is conditional -- a branch between them would make every wait a full drain: loads
-  // past K repeat valid columns, and such columns of the activation are stored as zeros.
-  u32x4 ra[2][4], rb[2][2];
-  auto load = [&](int t, u32x4 (&rw)[4], u32x4 (&rx)[2]) {
-    const int k = min(t * BK + ch * 8, K - 8);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) rw[i] = *reinterpret_cast<const u32x4*>(wp[i] + k);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) rx[i] = *reinterpret_cast<const u32x4*>(xp[i] + k);
+  u32x4 ra[2][NP];
+  const int so = sr * GBK + ((ch ^ ((sr >> 1) & 7)) << 3);  // 16 rows x one piece cover all 64 banks
+  auto load = [&](int t, int i, u32x4 (&r)[NP]) {
+    const int k = t * GBK + ch * 8;
+    const unsigned kw = min(k, K - 8) * 2, kx = k < K ? k * 2 : OUT;
+    const auto v = i < WP ? __builtin_amdgcn_raw_buffer_load_b128(rw, wo[i < WP ? i : 0] + kw, 0, 0)
+                          : __builtin_amdgcn_raw_buffer_load_b128(rx, xo[i < WP ? 0 : i - WP] + kx, 0, 0);
+    r[i] = *reinterpret_cast<const u32x4*>(&v);
   };
-  const int so = sr * BK + ((ch ^ ((sr >> 1) & 7)) << 3);  // 16 rows x one chunk, or 2 x 8: all 64 banks
-  auto store = [&](int t, int b, const u32x4 (&rw)[4], const u32x4 (&rx)[2]) {
-    const uint32_t keep = t * BK + ch * 8 < K ? ~0u : 0u;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(sw[b] + so + 64 * i * BK) = rw[i];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4*>(sx[b] + so + 64 * i * BK) = rx[i] & u32x4{keep, keep, keep, keep};
+  auto store = [&](int i, bf16_t* buf, const u32x4 (&r)[NP]) {
+    *reinterpret_cast<u32x4*>(buf + so + 32 * i * GBK) = r[i];
   };
-  f32x16 acc[2][2];
+  f32x16 acc[AI][BJ];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < AI; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < BJ; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-  int ar[2], br[2];
+  const int sw = (l32 >> 1) & 7;
+  const int ar = (wn * AI * 32 + l32) * GBK, br = (WP * 32 + wm * BJ * 32 + l32) * GBK;
+  const int nk = ((K + GBK - 1) / GBK + 1) & ~1;  // (an odd count's extra stage multiplies zeros)
+  bf16x8 a[2][AI], x[2][BJ];
+  auto frag = [&](const bf16_t* st, int s) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    ar[i] = (UP ? i * 128 + wn * 32 : wn * 64 + i * 32) + l32;
-    br[i] = wm * 64 + i * 32 + l32;
-  }
-  const int nk = ((K + BK - 1) / BK + 1) & ~1;  // (an odd count's extra step multiplies zeros)
-  const bool live = __builtin_amdgcn_readfirstlane(wm) * 64 < nr;
-  // step t: LDS buffer t & 1 holds it, register set (t + 1) & 1 the next, the other set is requested
-  auto step = [&](int t, auto par) {
-    constexpr int b = decltype(par)::value;
-    load(t + 2, ra[b], rb[b]);
-    asm volatile("" ::: "memory");
-    if (live) {
-      bf16x8 a[2][2], x[2][2];
-      auto frag = [&](int s, int f) {
+    for (int i = 0; i < AI; ++i)
+      a[s & 1][i] = *reinterpret_cast<const bf16x8*>(st + ar + i * 32 * GBK + (((2 * s + hh) ^ sw) << 3));
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          a[f][i] = *reinterpret_cast<const bf16x8*>(sw[b] + ar[i] * BK + (((2 * s + hh) ^ ((ar[i] >> 1) & 7)) << 3));
-          x[f][i] = *reinterpret_cast<const bf16x8*>(sx[b] + br[i] * BK + (((2 * s + hh) ^ ((br[i] >> 1) & 7)) << 3));
-        }
-      };
-      frag(0, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-#pragma unroll
-      for (int s = 0; s < BK / 16; ++s) {  // fragments one sub-step ahead of their products
-        if (s + 1 < BK / 16) {
-          frag(s + 1, (s + 1) & 1);
-          __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-        }
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s & 1][i], x[s & 1][j], acc[i][j], 0, 0, 0);
-        __builtin_amdgcn_sched_group_barrier(0x8, 4, 0);
-      }
-    }
-    asm volatile("" ::: "memory");
-    store(t + 1, b ^ 1, ra[b ^ 1], rb[b ^ 1]);
-    __syncthreads();
+    for (int j = 0; j < BJ; ++j)
+      x[s & 1][j] = *reinterpret_cast<const bf16x8*>(st + br + j * 32 * GBK + (((2 * s + hh) ^ sw) << 3));
   };
-  load(0, ra[0], rb[0]);
-  store(0, 0, ra[0], rb[0]);
-  load(1, ra[1], rb[1]);
+  auto products = [&](int s) {
+#pragma unroll
+    for (int i = 0; i < AI; ++i)
+#pragma unroll
+      for (int j = 0; j < BJ; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s & 1][i], x[s & 1][j], acc[i][j], 0, 0, 0);
+  };
+  constexpr int NM = AI * BJ, NF = AI + BJ;  // products of a sub-step, its fragments
+  // stage t: LDS buffer t & 1 holds it, register set (t + 1) & 1 the next, the other set the one after; a piece that is
+  // stored makes room for its successor two stages on. The barrier
+  // stands before the last sub-step, whose fragments are in registers: its products cover the first reads after it.
+  auto stage = [&](int t, auto par) {
+    constexpr int b = decltype(par)::value;
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      constexpr int PP = (NP + 2) / 3;
+      frag(gl + b * STG, s + 1);
+#pragma unroll
+      for (int i = s * PP; i < (s + 1) * PP && i < NP; ++i) {
+        store(i, gl + (b ^ 1) * STG, ra[b ^ 1]);
+        load(t + 3, i, ra[b ^ 1]);
+      }
+      products(s);
+#pragma unroll
+      for (int i = 0; i < NF; ++i) {  // (hipcc by itself requests everything at a stage's end)
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+      }
+#pragma unroll
+      for (int i = s * PP; i < (s + 1) * PP && i < NP; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x8, NM, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    frag(gl + (b ^ 1) * STG, 0);
+    products(3);
+    __builtin_amdgcn_sched_group_barrier(0x100, NF, 0);
+    __builtin_amdgcn_sched_group_barrier(0x8, NM, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int i = 0; i < NP; ++i) load(0, i, ra[0]);
+#pragma unroll
+  for (int i = 0; i < NP; ++i) load(1, i, ra[1]);
+#pragma unroll
+  for (int i = 0; i < NP; ++i) store(i, gl, ra[0]);
+#pragma unroll
+  for (int i = 0; i < NP; ++i) load(2, i, ra[0]);
   __syncthreads();
+  frag(gl, 0);
   for (int t = 0; t < nk; t += 2) {
-    step(t, std::integral_constant<int, 0>{});
-    step(t + 1, std::integral_constant<int, 1>{});
+    stage(t, std::integral_constant<int, 0>{});
+    stage(t + 1, std::integral_constant<int, 1>{});
   }
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int r = br[j];
+  for (int j = 0; j < BJ; ++j) {
+    const int r = wm * BJ * 32 + j * 32 + l32;
     if (r >= nr) continue;
     const float s = p.scale ? p.wts[p.perm[lo + r]] : 1.f;
     bf16_t* y = reinterpret_cast<bf16_t*>(p.y) + (long long)(lo + r) * N;
 #pragma unroll
-    for (int i = 0; i < (UP ? 1 : 2); ++i)
+    for (int i = 0; i < (UP ? AI / 2 : AI); ++i)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int n = n0 + (UP ? wn * 32 : wn * 64 + i * 32) + 8 * q + 4 * hh;
+        const int n = n0 + (wn * (UP ? AI / 2 : AI) + i) * 32 + 8 * q + 4 * hh;
         if (n >= N) continue;  // (N % 4 == 0)
         float o[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           if constexpr (UP) {
-            const float gt = acc[0][j][4 * q + e] * s, up = acc[1][j][4 * q + e] * s;
+            const float gt = acc[i][j][4 * q + e] * s, up = acc[AI / 2 + i][j][4 * q + e] * s;
             o[e] = gt * __builtin_amdgcn_rcpf(1.f + __expf(-gt)) * up;
           } else {
             o[e] = acc[i][j][4 * q + e] * s;
@@ -727,6 +744,43 @@ __global__ void __launch_bounds__(512, 2) expert_gemm_kernel(ExpertArgs p) {
         *reinterpret_cast<uint2*>(y + n) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
       }
   }
+}
+
+// NARROW: tiles of up to 192 rows x 128 weight rows
+template <bool UP, bool NARROW>
+__global__ void __launch_bounds__(256, NARROW ? 2 : 1) expert_gemm_kernel(ExpertArgs p) {
+  extern __shared__ __attribute__((aligned(16))) bf16_t gl[];  // [2][weight rows, then activation rows][GBK]
+  // order: an XCD works a contiguous run of (expert, weight block, row tile), so the row tiles that share a
+  // weight block are on one XCD at one time
+  constexpr int NB = (NARROW ? 128 : 256) / (UP ? 2 : 1);
+  const int nt = *p.ntiles, nb = (p.N + NB - 1) / NB;
+  if ((int)blockIdx.x >= nt * nb) return;
+  const int id = xcd_remap(blockIdx.x, nt * nb);
+  const int* t0 = p.tiles + id / nb * 5;
+  const int in = id - t0[3] * nb, tile = t0[3] + in % t0[4], bn = in / t0[4];
+  const int* tl = p.tiles + tile * 5;
+  const int nr = tl[2], n0 = bn * NB;
+  if constexpr (NARROW) {
+    if (nr > 128) expert_gemm_tile<UP, 2, 2, 2, 3>(p, gl, tl[0], tl[1], nr, n0);
+    else if (nr > 64) expert_gemm_tile<UP, 2, 2, 2, 2>(p, gl, tl[0], tl[1], nr, n0);
+    else expert_gemm_tile<UP, 2, 2, 2, 1>(p, gl, tl[0], tl[1], nr, n0);
+  } else {
+    if (nr > 192) expert_gemm_tile<UP, 2, 4, 2, 4>(p, gl, tl[0], tl[1], nr, n0);
+    else if (nr > 160) expert_gemm_tile<UP, 4, 2, 1, 6>(p, gl, tl[0], tl[1], nr, n0);
+    else if (nr > 128) expert_gemm_tile<UP, 4, 2, 1, 5>(p, gl, tl[0], tl[1], nr, n0);
+    else if (nr > 96) expert_gemm_tile<UP, 4, 2, 1, 4>(p, gl, tl[0], tl[1], nr, n0);
+    else if (nr > 64) expert_gemm_tile<UP, 4, 2, 1, 3>(p, gl, tl[0], tl[1], nr, n0);
+    else expert_gemm_tile<UP, 4, 2, 1, 2>(p, gl, tl[0], tl[1], nr, n0);
+  }
+}
+
+template <bool UP, bool NARROW>
+int gemm_go(const ExpertArgs& a, int max_tiles, hipStream_t s) {
+  constexpr int NB = (NARROW ? 128 : 256) / (UP ? 2 : 1), LDS = NARROW ? GEMM_LDS / 8 * 5 : GEMM_LDS;
+  auto kern = expert_gemm_kernel<UP, NARROW>;
+  if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess) return 5;
+  hipLaunchKernelGGL(kern, dim3((a.N + NB - 1) / NB * max_tiles), dim3(256), LDS, s, a);
+  return hipGetLastError() == hipSuccess ? 0 : 4;
 }
 
 template <typename E, bool VEC>
@@ -821,7 +875,7 @@ KCA_API int kca_moe_route_group(const void* h, const void* wr, const void* wsg, 
 }
 
 // One expert product of every tile. mt: the tiles' row limit (1, 2, 4, 8: gemv; 32: stream, bf16 with K % 64 == 0 and
-// N % 16 == 0; 128: gemm, bf16 with K % 8 == 0 and N % 4 == 0). x_rows: rows of x. ws: a shared expert's product over all tokens beside them (gemv; nullable).
+// N % 16 == 0; 128, 192, 256: gemm, bf16 with K % 8 == 0 and N % 4 == 0). x_rows: rows of x. ws: a shared expert's product over all tokens beside them (gemv; nullable).
 KCA_API int kca_moe_expert(int dtype, const void* x, const void* w, void* y, const void* perm, const void* wts,
                            const void* tiles, const void* ntiles, int max_tiles, int mt, int top, int N, int K, int up,
                            int scale, const void* xs, const void* ws, void* ys, int tokens, int Ns, int Ks, int x_rows,
@@ -830,17 +884,16 @@ KCA_API int kca_moe_expert(int dtype, const void* x, const void* w, void* y, con
   if (ws && (!xs || !ys || tokens < 1 || tokens > 32767 || Ns < 1 || Ks < 1 || mt > 8)) return 1;
   const ExpertArgs a{x, w, y, (const int*)perm, (const float*)wts, (const int*)tiles, (const int*)ntiles, top, N, K, up, scale,
                      xs, ws, ys, tokens, Ns, Ks};
-  if (mt == 128) {
-    if (dtype != 1 || K % 8 || N % 4 || !al16(x) || !al16(w) || (uintptr_t)y % 8) return 10;
-    const void* kern = up ? (const void*)expert_gemm_kernel<true> : (const void*)expert_gemm_kernel<false>;
-    if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, GEMM_LDS) != hipSuccess) return 5;
-    if (up) hipLaunchKernelGGL(expert_gemm_kernel<true>, dim3((N + 127) / 128 * max_tiles), dim3(512), GEMM_LDS, s, a);
-    else hipLaunchKernelGGL(expert_gemm_kernel<false>, dim3((N + 255) / 256 * max_tiles), dim3(512), GEMM_LDS, s, a);
-    return hipGetLastError() == hipSuccess ? 0 : 4;
+  if (mt == GM || mt == 128 || mt == 192) {
+    if (dtype != 1 || K % 8 || N % 4 || !al16(x) || !al16(w) || (uintptr_t)y % 8 || 2ll * (up ? 2 * N : N) * K >= 1ll << 32 ||
+        (up && 2ll * x_rows * K >= 1ll << 31))  // (32-bit byte offsets)
+      return 10;
+    if (mt == GM) return up ? gemm_go<true, false>(a, max_tiles, s) : gemm_go<false, false>(a, max_tiles, s);
+    return up ? gemm_go<true, true>(a, max_tiles, s) : gemm_go<false, true>(a, max_tiles, s);
   }
   if (mt == SROWS) {
-    if (dtype != 1 || K % SK || N % 16 || !al16(x) || !al16(w) || (uintptr_t)y % 8 || 2ll * (up ? 2 * N : N) * K >= 1ll << 31 ||
-        2ll * x_rows * K >= 1ll << 31)  // (32-bit byte offsets)
+    if (dtype != 1 || K % SK || N % 16 || !al16(x) || !al16(w) || (uintptr_t)y % 8 || 2ll * (up ? 2 * N : N) * K >= 1ll << 32 ||
+        (up && 2ll * x_rows * K >= 1ll << 31))  // (32-bit byte offsets)
       return 10;
     const void* kern = up ? (const void*)expert_stream_kernel<true> : (const void*)expert_stream_kernel<false>;
     if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, STREAM_LDS) != hipSuccess) return 5;

@@ -14,7 +14,7 @@ import torch
 from . import _lib
 from .rms_shift import native_dt
 
-GEMM_ROWS = 128
+GEMM_ROWS = 256
 STREAM_ROWS = 32
 SHARED_ROWS = 16  # tokens up to which a shared expert's weights stream beside the routed ones'
 
@@ -81,26 +81,38 @@ class Groups:
 
 
 def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
-    """Row limit of an expert tile, by the rows that an expert expects: a streaming vector product (1 .. 8), the weight
-    stream on the matrix cores (32), or the prompts' product (128).
+    """Row limit of an expert tile, by the rows ``r`` that an expert expects: a streaming vector product (1 .. 8), the
+    weight stream on the matrix cores (32), the prompts' product in narrow blocks (128 or 192 rows x 128 weight rows) or
+    wide ones (256 x 256). Both products of a layer, us (width, experts, top, inner size; - not measured):
 
-    Both products, us, vector / stream / prompts' product (width, experts, top, inner size):
+        4096, 16, 2, 4096   tokens   24: vector 270, stream 273     32: 312, 291             100: 716, 296, narrow 302
+                                    160: stream 298, narrow 296    250: 322, 302             800: 340 - 346, wide 337
+                                   1000: narrow 374, wide 347     2000: 609 - 632, 578      4096: 946, 904
+        2048, 32, 4, 1024   tokens   12: vector 71, stream 74       32: 111, 87, narrow -    100: 265, 89, 91
+                                    250: stream 99, narrow 92     1000: 128 rows 132, 192 rows 116, wide 120
+                                   1500: 143, 162, 140            4096: 302, 267, 301       8192: -, 551, 540
+        4096, 20, 3, 2048   tokens   24: vector 165, stream 166     32: 190, 172             160: 450 (100), 183, 178
+                                    600: 128 rows 226, 192 rows 197    1500: 309, 312, wide 332    4096: 645, 634, 558
+        2048, 32, 5, 768    tokens   12: vector 53, stream 51       32: 83, 61               250: -, 70, narrow 77
+                                    400: stream 76, narrow 79      600: 94, 128 rows 77      8192: -, 382, wide 445
 
-        4096, 16, 2, 4096   24 tokens 270 / 273 / 285   32: 312 / 291 / 304   100: 716 / 296 / 310   250: - / 322 / 315
-        2048, 32, 4, 1024   12 tokens  71 /  74 /  86   16:  84 /  79 /  93   100: 265 /  89 / 101   250: - /  99 / 107
-        4096, 20, 3, 2048   24 tokens 165 / 166 / 189   32: 190 / 172 / 192   100: 450 / 175 / 197   250: - / 197 / 205
-        2048, 32, 5, 768    12 tokens  53 /  51 /  63   32:  83 /  61 /  62   100: 205 /  62 /  71   250: - /  70 /  74
-
-    so the matrix cores take over at about 3 rows an expert, at 2 where a row is short (a wave's reduction is then a
-    larger part of its stream); up to 16 tokens the vector product also carries the shared expert. A stream tile
-    holds 32 rows: past that an expert's weights are read again."""
+    The stream takes over at about 3 rows, at 2 where a row is short (a vector wave's reduction is then a larger part of
+    its work), but up to 16 tokens the vector product also carries the shared expert. A stream tile holds 32 rows, past
+    which weights are read again, so it ends at 16 rows -- at 64 where narrow blocks are too few to fill the chip. A
+    narrow tile of 192 rows saves a second tile a little over 128 rows, if there are blocks enough without it, and costs
+    one a little over 192. A wide block is
+    alone on its CU and pays its ramps in full: it needs a long contraction, or many rows."""
     n = T * top
     used = min(E, n)
-    if dtype == torch.bfloat16 and d % 8 == 0 and F % 8 == 0:
-        stream = d % 64 == 0 and F % 64 == 0 and max(4 * F * d, 2 * n * max(d, F)) < 2 ** 31
-        if n > (32 if stream else 4) * used:
-            return GEMM_ROWS
-        if stream and T > SHARED_ROWS and n > (3 if d > 2048 else 2) * used:
+    fits = 4 * F * d < 2 ** 32 and 2 * T * d < 2 ** 31  # 32-bit offsets into an expert's weights and the token rows
+    if dtype == torch.bfloat16 and d % 8 == 0 and F % 8 == 0 and fits:
+        stream = d % 64 == 0 and F % 64 == 0
+        r, short, full = n / used, min(d, F), used * (F // 64) >= 512
+        if r > ((16 if full else 64) if stream else 4):
+            if r > 96 and (short >= 4096 or (short >= 1024 and r > 512)):
+                return GEMM_ROWS
+            return 192 if (full and 100 < r <= 160) or r > 240 else 128
+        if stream and T > SHARED_ROWS and r > (3 if d > 2048 else 2):
             return STREAM_ROWS
     return 1 if T == 1 else 2 if T == 2 else 4 if T <= 4 else 8
 
