@@ -37,9 +37,14 @@ class Branch:
     inv: torch.Tensor | None = None
 
 
-def rows_per_block(T: int) -> int:
-    """Rows a workgroup walks: a longer walk recomputes fewer left neighbours, a short batch needs the spread."""
-    return 8 if T >= 4096 else 4 if T >= 1024 else 2 if T >= 512 else 1
+def rows_per_block(T: int, shift: bool = True, routed: bool = False) -> int:
+    """Rows a workgroup walks. With a shift a longer walk recomputes fewer left neighbours, a short batch needs the spread;
+    without one nothing is recomputed. Width 4096, shift, us for 1 / 2 / 4 / 8 rows, two routed rows a token (none):
+    777 tokens 29 / 24 / 32 / 53 (17 / 19 / 25 / 40), 4096 tokens 107 / 93 / 105 / 107 (69 / 61 / 57 / 75), 8192 tokens
+    - / 179 / 177 / 206 (- / 118 / 115 / 112)."""
+    if not shift:
+        return 1
+    return 8 if T >= 8192 and not routed else 4 if T >= 4096 else 2 if T >= 512 else 1
 
 
 def rms_shift(x: torch.Tensor | None, branch: Branch | None, m: float, gain: torch.Tensor, eps: float, *,
@@ -81,7 +86,8 @@ def rms_shift(x: torch.Tensor | None, branch: Branch | None, m: float, gain: tor
     _lib.call("kca_rms_shift", code, p(x), p(embed if x is None else None), p(tokens), p(a),
               a.stride(0) if a is not None else 0, p(y), p(inv), inv.shape[1] if inv is not None else 0, float(m),
               p(gain), int(gain.numel() > 1), float(eps), p(shift), p(prev), p(prev_idx), p(pos), p(flags), p(state),
-              p(slots), p(rows), p(x_out), p(h), p(hs), T, d, rows_per_block(T), _lib.stream())
+              p(slots), p(rows), p(x_out), p(h), p(hs), T, d, rows_per_block(T, shift is not None, y is not None),
+              _lib.stream())
     return x_out, h, hs
 
 
