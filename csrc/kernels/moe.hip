@@ -311,16 +311,18 @@ __global__ void __launch_bounds__(NW * 64) route_mfma_kernel(RouteArgs p, GroupA
     else if (nt == 2) steps(std::integral_constant<int, 2>{});
     else steps(std::integral_constant<int, 4>{});
     __syncthreads();
+    // (16-byte pieces swizzled by row: 16 rows x one piece cover all 64 banks)
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) part[(wv * 16 + r16) * 64 + i * 16 + g * 4 + r] = acc[i][r];
+      if (i < nt) *reinterpret_cast<f32x4*>(part + (wv * 16 + r16) * 64 + (((i * 4 + g) ^ r16) << 2)) = acc[i];
     __syncthreads();
-    for (int i = tid; i < 1024; i += NW * 64) {
-      float s = 0.f;
+    for (int i = tid; i < 256; i += NW * 64) {  // (row, piece)
+      const int r = i >> 4, q = i & 15;
+      if (q >= nt * 4) continue;
+      f32x4 s{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int w8 = 0; w8 < NW; ++w8) s += part[w8 * 1024 + i];
-      z[(i >> 6) * zs + e0 + (i & 63)] = s;
+      for (int w8 = 0; w8 < NW; ++w8) s += *reinterpret_cast<const f32x4*>(part + (w8 * 16 + r) * 64 + ((q ^ r) << 2));
+      *reinterpret_cast<f32x4*>(z + r * zs + e0 + q * 4) = s;
     }
   }
   __syncthreads();
