@@ -11,9 +11,12 @@ CPU tensors and inference use plain ``F.linear``.
 """
 from __future__ import annotations
 
+import math
+
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -131,10 +134,64 @@ class TLinear(nn.Linear):
         if self._tn and torch.is_grad_enabled() and (x.requires_grad or self.weight.requires_grad) \
                 and x.is_cuda and x.dtype == torch.bfloat16:
             return _LinearTN.apply(x, self.weight, self.bias, self)
-        return F.linear(x, self.weight, self.bias)
+        return linear_rows(x, self.weight, self.bias)
 
 
-__all__ = ["TLinear", "transpose", "param_linear"]
+__all__ = ["TLinear", "transpose", "param_linear", "linear_rows"]
+
+
+# ---------------------------------------------------------------- long prompts: whole waves, then the rest
+_CUS, _TILE = 256, 256
+
+
+def wave_rows(rows: int, n: int, k: int) -> int:
+    """Rows of ``x[rows, k] W[n, k]^T`` for a first launch, the others go in a second; ``rows`` itself: one launch.
+
+    hipBLASLt's output blocks are 256 x 256 at these sizes, one a CU. A product whose blocks fill whole waves of the 256
+    CUs runs at 1500 to 1600 TFLOP/s; one with a last wave of a few blocks at 690 to 1200, for the chip waits on it, or
+    on the smaller blocks that the library then takes for all rows. So the rows that fill whole waves are one launch.
+    Measured, us, one launch against two: 5400 rows of 16384 x 4096 621 : 483, of 4096 x 16384 982 : 502, of
+    12288 x 4096 419 : 387; 4209 rows 422 : 374, 844 : 382, 398 : 282; 7333 rows 694 : 652, 1172 : 709; 5762 rows of
+    8192 x 2048 210 : 143. The worst: 6800 rows of 4096 x 4096 159 : 164, 3189 rows of 8192 x 2048 87 : 89.
+
+    Left in one launch: up to 2048 rows (1700 of 16384 x 4096 165 : 172), k below 2048 (a second launch costs as
+    much as the idle CUs), widths whose blocks fill a wave only at more rows (6144 and 2048 wide: 8192; there a
+    first part of nearly whole waves loses, 7344 rows of 6144 x 2048 134 : 142). A rest of 1536 to 2048 rows takes
+    a quarter of a wave more: the library runs 1600 to 1850 rows of 4096 x 16384 at 560 TFLOP/s (5888 rows: 570 in one
+    launch, 755 as 4096 + 1792, 570 as 3072 + 2816)."""
+    across = -(-n // _TILE)
+    wave = _TILE * (_CUS // math.gcd(across, _CUS))  # the fewest rows whose blocks fill whole waves
+    first = rows // wave * wave
+    if first < 2048 or first == rows or k < 2048:
+        return rows
+    if 1536 < rows - first < 2048:
+        first -= wave // 4
+    return first
+
+
+def linear_rows(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """``F.linear`` without gradients, in two launches where ``wave_rows`` says so; ``F.linear`` itself for all else (a
+    gradient or a tangent recorded, a transform or autocast at work, tensor subclasses, strided rows, other types)."""
+    n, k = weight.shape
+    if (torch.is_grad_enabled() or not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16)
+            or x.numel() <= 2048 * k):
+        return F.linear(x, weight, bias)
+    rows = x.numel() // k
+    first = wave_rows(rows, n, k)
+    if (first == rows or x.shape[-1] != k or (bias is not None and bias.shape != (n,)) or not x.is_contiguous() or type(x) is not torch.Tensor
+            or any(t is not None and (t.dtype != x.dtype or t.device != x.device
+                                      or type(t) not in (torch.Tensor, nn.Parameter)) for t in (weight, bias))
+            or torch.is_autocast_enabled("cuda") or torch._C._are_functorch_transforms_active()
+            or forward_ad._current_level >= 0 or torch.jit.is_tracing() or torch.compiler.is_compiling()):
+        return F.linear(x, weight, bias)
+    x2, wt = x.view(rows, k), weight.t()
+    y = torch.empty(rows, n, device=x.device, dtype=x.dtype)
+    for part in (slice(0, first), slice(first, rows)):
+        if bias is None:
+            torch.mm(x2[part], wt, out=y[part])
+        else:
+            torch.addmm(bias, x2[part], wt, out=y[part])
+    return y.view(*x.shape[:-1], n)
 
 
 # ---------------------------------------------------------------- split-K weight gradients
