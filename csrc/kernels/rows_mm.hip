@@ -1,0 +1,258 @@
+// y[M, N] = x[M, K] . W[N, K]^T (+ bias), bf16 or fp16, for the few rows of a short prompt.
+#include "common.h"
+
+namespace {
+
+bool al16(const void* p) { return (uintptr_t)p % 16 == 0; }
+
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int NB = 64, SK = 64, ROWS = 128;  // weight rows a block, K a stage, activation rows at most
+
+struct RowsArgs {
+  const void *x, *w, *bias;
+  void* y;
+  float* ws;      // ks > 1: [block][slice][product tile][2][256 threads][2]
+  unsigned* cnt;  // ks > 1: one arrival counter a block, zero before and after
+  int M, N, K, ks;
+};
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rsrc(const void* p) {
+  const unsigned long long a = (unsigned long long)p;
+  const unsigned long long u = ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(a >> 32)) << 32) |
+                               (unsigned)__builtin_amdgcn_readfirstlane((unsigned)a);
+  return __builtin_amdgcn_make_buffer_rsrc((void*)u, (short)0, -1, 0x00020000);
+}
+
+// both sub-steps' fragments of a stage and their wait in one piece (hipcc would drain every LDS-DMA in flight before a
+// read it sees): runs of 16 rows at a0 and, for the second sub-step, at a1
+__device__ __forceinline__ void read_frags(unsigned a0, unsigned a1, u32x4 (&r)[2][1]) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
+               : "=&v"(r[0][0]), "=&v"(r[1][0])
+               : "v"(a0), "v"(a1)
+               : "memory");
+#endif
+}
+__device__ __forceinline__ void read_frags(unsigned a0, unsigned a1, u32x4 (&r)[2][2]) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile(
+      "ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:2048\n\t"
+      "ds_read_b128 %2, %5\n\tds_read_b128 %3, %5 offset:2048\n\ts_waitcnt lgkmcnt(0)"
+      : "=&v"(r[0][0]), "=&v"(r[0][1]), "=&v"(r[1][0]), "=&v"(r[1][1])
+      : "v"(a0), "v"(a1)
+      : "memory");
+#endif
+}
+__device__ __forceinline__ void read_frags(unsigned a0, unsigned a1, u32x4 (&r)[2][4]) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile(
+      "ds_read_b128 %0, %8\n\tds_read_b128 %1, %8 offset:2048\n\t"
+      "ds_read_b128 %2, %8 offset:4096\n\tds_read_b128 %3, %8 offset:6144\n\t"
+      "ds_read_b128 %4, %9\n\tds_read_b128 %5, %9 offset:2048\n\t"
+      "ds_read_b128 %6, %9 offset:4096\n\tds_read_b128 %7, %9 offset:6144\n\ts_waitcnt lgkmcnt(0)"
+      : "=&v"(r[0][0]), "=&v"(r[0][1]), "=&v"(r[0][2]), "=&v"(r[0][3]), "=&v"(r[1][0]), "=&v"(r[1][1]), "=&v"(r[1][2]),
+        "=&v"(r[1][3])
+      : "v"(a0), "v"(a1)
+      : "memory");
+#endif
+}
+
+template <bool F16>
+__device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
+  if constexpr (F16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// Bound by the weight stream. A block is 64 weight rows x all activation rows (rounded up to XR); a stage's weights and
+// activations, 64 of K each, go straight to LDS (no registers), so 60 to 64 KiB a workgroup and two workgroups a CU are in flight;
+// the products (weights as the A operand: a lane holds one activation row and four outputs) hide under it. Blocks of 64 rows
+// rather than 128 keep the CUs busy with fewer slices of K, whose partial sums (4 bytes beside 2 of a weight, for every
+// activation row) cost more than reading the activations once a block from L2: 61 rows of 12288 x 4096 26.5 us against 30.1,
+// of 16384 x 4096 32.2 : 36.1, of 4096 x 4096 13.0 : 16.6. Where the blocks are fewer than the CUs, slices of K write partial
+// sums and the last to arrive adds them in slice order. Deeper pipelines with one workgroup a CU were slower (33.2, 27.6).
+// An LDS-DMA instruction fills 8 rows of 128 bytes lane by lane, so the 16-byte pieces are swizzled (by row pair: 16 rows x one
+// piece cover all 64 banks) on the source address.
+// us, hipBLASLt : this (weights cold; at the copy rate 20.9, 27.8, 7.0, 27.8):
+//   rows   12288 x 4096   16384 x 4096   4096 x 4096   4096 x 16384
+//     16    27.2 : 22.3    31.6 : 30.0   15.6 : 11.5   29.9 : 32.1
+//     64    25.3 : 26.8    33.0 : 32.4   15.4 : 13.0   39.1 : 33.8
+//    128    32.2 : 34.2    36.3 : 38.0   24.4 : 17.6   81.5 : 42.2
+// A call costs the host 14 us, the library's through the tuned table 20 to 26: four GPT-J layers on 61 tokens 944 -> 769 us.
+// XR activation rows; 4 waves, WM of them across the activation rows; SNB stages.
+template <bool F16, int XR, int WM, int SNB>
+__global__ void __launch_bounds__(256, 2) rows_mm_kernel(RowsArgs p) {
+  constexpr int WN = 4 / WM, A = NB / WN / 16, B = XR / WM / 16;  // a wave's runs of 16 weight and activation rows
+  constexpr int STG = (NB + XR) * SK * 2, WI = NB / 32, XI = XR / 32, PER = WI + XI;
+  extern __shared__ __attribute__((aligned(1024))) char sl[];  // [SNB][128 weight rows | XR activation rows][128 B]
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wn = wv % WN, wm = wv / WN;
+  const int r16 = lane & 15, g = lane >> 4;
+  const int id = xcd_remap(blockIdx.x, gridDim.x);  // the slices of a block on one XCD, beside their partial sums
+  const int blk = id / p.ks, z = id % p.ks, n0 = blk * NB, K = p.K;
+  const int nk = K / SK, t0 = (int)((long long)nk * z / p.ks), t1 = (int)((long long)nk * (z + 1) / p.ks);
+  const __amdgpu_buffer_rsrc_t rw = uniform_rsrc(p.w), rx = uniform_rsrc(p.x);
+  unsigned wo[WI], xo[XI];
+#pragma unroll
+  for (int i = 0; i < WI; ++i) {
+    const int r = wv * 8 * WI + 8 * i + (lane >> 3);
+    wo[i] = ((unsigned)min(n0 + r, p.N - 1) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
+  }
+#pragma unroll
+  for (int i = 0; i < XI; ++i) {
+    const int r = wv * 8 * XI + 8 * i + (lane >> 3);
+    xo[i] = ((unsigned)min(r, p.M - 1) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
+  }
+  typedef __attribute__((address_space(3))) char lds_char;
+  lds_char* lsm = (lds_char*)sl;
+  auto issue = [&](int t) {
+    const int k = __builtin_amdgcn_readfirstlane(min(t, t1 - 1) * SK * 2);  // the last stages repeat one that nobody reads
+    lds_char* st = lsm + ((t - t0) % SNB) * STG;
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+    for (int i = 0; i < WI; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (void __attribute__((address_space(3)))*)(st + (wv * WI + i) * 1024), 16,
+                                               wo[i], k, 0, 0);
+#pragma unroll
+    for (int i = 0; i < XI; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rx, (void __attribute__((address_space(3)))*)(st + (NB / 8 + wv * XI + i) * 1024), 16, xo[i], k, 0, 0);
+#endif
+  };
+  f32x4 acc[A][B];
+#pragma unroll
+  for (int i = 0; i < A; ++i)
+#pragma unroll
+    for (int j = 0; j < B; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const unsigned base = (unsigned)(size_t)lsm, sw = (r16 >> 1) & 7;
+  const unsigned aw = (wn * A * 16 + r16) * 128, ax = (NB + wm * B * 16 + r16) * 128;
+  const unsigned c0 = (g ^ sw) * 16, c1 = ((4 + g) ^ sw) * 16;
+#pragma unroll
+  for (int t = 0; t < SNB - 1; ++t) issue(t0 + t);
+  for (int t = t0; t < t1; ++t) {
+    // this wave's pieces of stage t have landed (SNB - 2 younger stages may be in flight), then everybody's
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SNB - 2) * PER) : "memory");
+    __builtin_amdgcn_s_barrier();
+    issue(t + SNB - 1);  // into the buffer of stage t - 1, which all waves have left
+    const unsigned st = base + ((t - t0) % SNB) * STG;
+    u32x4 wf[2][A], xf[2][B];
+    read_frags(st + aw + c0, st + aw + c1, wf);
+    read_frags(st + ax + c0, st + ax + c1, xf);
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int j = 0; j < B; ++j)
+#pragma unroll
+        for (int i = 0; i < A; ++i) acc[i][j] = mma<F16>(wf[s][i], xf[s][j], acc[i][j]);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the repeated stages, before the LDS is given back
+  if (p.ks > 1) {
+    unsigned long long* part = reinterpret_cast<unsigned long long*>(p.ws) + (long long)blk * p.ks * A * B * 512 + threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < A; ++i)
+#pragma unroll
+      for (int j = 0; j < B; ++j)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          __hip_atomic_store(part + (z * A * B + i * B + j) * 512 + h * 256,
+                             __builtin_bit_cast(unsigned long long, f32x2{acc[i][j][2 * h], acc[i][j][2 * h + 1]}),
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const int last = __hip_atomic_fetch_add(p.cnt + blk, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)p.ks - 1;
+      if (last) {
+        __hip_atomic_store(p.cnt + blk, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
+      *(int*)sl = last;  // (the stages are done)
+    }
+    __syncthreads();
+    if (!*(volatile int*)sl) return;
+    // all slices in slice order, whichever came last: the sum does not depend on the order of arrival
+    f32x4 sum[A][B];
+#pragma unroll
+    for (int i = 0; i < A; ++i)
+#pragma unroll
+      for (int j = 0; j < B; ++j) sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+    for (int s = 0; s < p.ks; ++s) {
+#pragma unroll
+      for (int i = 0; i < A; ++i)
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+          const auto* q = part + (s * A * B + i * B + j) * 512;
+          const f32x2 lo = __builtin_bit_cast(f32x2, q[0]), hi = __builtin_bit_cast(f32x2, q[256]);
+          sum[i][j] += f32x4{lo[0], lo[1], hi[0], hi[1]};
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < A; ++i)
+#pragma unroll
+      for (int j = 0; j < B; ++j) acc[i][j] = sum[i][j];
+  }
+#pragma unroll
+  for (int i = 0; i < A; ++i) {
+    const int n = n0 + (wn * A + i) * 16 + 4 * g;
+    if (n >= p.N) continue;
+    float b[4] = {0.f, 0.f, 0.f, 0.f};
+    if (p.bias) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const unsigned short v = reinterpret_cast<const unsigned short*>(p.bias)[n + e];
+        b[e] = F16 ? (float)__builtin_bit_cast(_Float16, v) : bf2f(v);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < B; ++j) {
+      const int m = (wm * B + j) * 16 + r16;
+      if (m >= p.M) continue;
+      float o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = acc[i][j][e] + b[e];
+      uint2 v;
+      if constexpr (F16) {
+        const _Float16 h[4] = {(_Float16)o[0], (_Float16)o[1], (_Float16)o[2], (_Float16)o[3]};
+        v = __builtin_bit_cast(uint2, h);
+      } else {
+        v = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+      }
+      *reinterpret_cast<uint2*>(reinterpret_cast<unsigned short*>(p.y) + (long long)m * p.N + n) = v;
+    }
+  }
+}
+
+template <bool F16, int XR, int WM, int SNB>
+int go(const RowsArgs& a, hipStream_t s) {
+  constexpr int lds = SNB * (NB + XR) * SK * 2;
+  if (hipFuncSetAttribute((const void*)rows_mm_kernel<F16, XR, WM, SNB>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) !=
+      hipSuccess)
+    return 5;
+  hipLaunchKernelGGL((rows_mm_kernel<F16, XR, WM, SNB>), dim3((a.N + NB - 1) / NB * a.ks), dim3(256), lds, s, a);
+  return hipGetLastError() == hipSuccess ? 0 : 4;
+}
+
+}  // namespace
+
+// dtype 1 bf16, 2 fp16. x [M, K], W [N, K], y [M, N] contiguous, x and W 16-byte aligned; bias [N] or null; ks > 1: slices of
+// K, with ws of ks * blocks * 64 * (M rounded up to 32, 64 or 128) floats and cnt of `blocks` zeroed counters (left zeroed),
+// blocks = ceil(N / 64). Other sizes return a status and launch nothing.
+KCA_API int kca_rows_mm(int dtype, const void* x, const void* w, const void* bias, void* y, float* ws, unsigned* cnt,
+                        long long ws_floats, int cnt_n, int M, int N, int K, int ks, hipStream_t s) {
+  if ((dtype != 1 && dtype != 2) || !x || !w || !y || M < 1 || M > ROWS || N < 16 || N % 16 || K < SK || K % SK || ks < 1 ||
+      ks > K / SK)
+    return 1;
+  if (!al16(x) || !al16(w) || (uintptr_t)y % 8) return 2;
+  if (2ll * N * K >= 1ll << 32) return 3;  // (32-bit byte offsets)
+  const long long blocks = (N + NB - 1) / NB, xr = M <= 32 ? 32 : M <= 64 ? 64 : 128;
+  if (blocks * ks >= 1ll << 31) return 3;
+  if (ks > 1 && (!ws || !cnt || !al16(ws) || ws_floats < blocks * ks * NB * xr || cnt_n < blocks)) return 6;
+  const RowsArgs a{x, w, bias, y, ws, cnt, M, N, K, ks};
+  if (xr == 32) return dtype == 2 ? go<true, 32, 1, 6>(a, s) : go<false, 32, 1, 6>(a, s);
+  if (xr == 64) return dtype == 2 ? go<true, 64, 1, 5>(a, s) : go<false, 64, 1, 5>(a, s);
+  return dtype == 2 ? go<true, 128, 2, 3>(a, s) : go<false, 128, 2, 3>(a, s);
+}

@@ -125,6 +125,7 @@ _SIGS.update({
     "kca_moe_group": [P, I, I, I, P, P, P, I, P, P],
     "kca_moe_route_group": [P, P, P, P, P, P, I, I, I, I, I, I, P, I, I, I, P, P, P, I, P, P],
     "kca_moe_expert": [I, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P, P, P, I, I, I, I, P],
+    "kca_rows_mm": [I, P, P, P, P, P, P, LL, I, I, I, I, I, P],
     "kca_act_rows": [I, I, P, LL, P, P, P, LL, I, I, F, P],
     "kca_norm_residual": [I, P, P, P, P, LL, P, P, P, P, F, P, P, P, I, I, I, P],
 })
@@ -243,6 +244,13 @@ def stream() -> int:
     if _raw_stream is None or _current_device is None:
         return torch.cuda.current_stream().cuda_stream
     return _raw_stream(_current_device())
+
+
+def stream_on(device: torch.device) -> int:
+    """The current stream's handle on a device (``stream``: on the current one)."""
+    if _raw_stream is None or device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

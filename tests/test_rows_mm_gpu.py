@@ -1,0 +1,76 @@
+"""Products of few rows on the weight-streaming kernel (csrc/kernels/rows_mm.hip) against float32."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from kubernetes_cloud_amd.ops import _lib
+from kubernetes_cloud_amd.ops.linear import _k_slices, _rows_mm, linear_rows
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(rows, n, k, dtype, bias, seed=3):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.empty(rows, k, device="cuda", dtype=dtype).normal_(generator=g)
+    w = torch.empty(n, k, device="cuda", dtype=dtype).normal_(std=k ** -0.5, generator=g)
+    b = torch.empty(n, device="cuda", dtype=dtype).normal_(generator=g) if bias else None
+    return x, w, b, F.linear(x.float(), w.float(), None if b is None else b.float())
+
+
+def _close(y, ref):
+    # one rounding to the type; the 32-bit sums of terms of size k^-1/2 are good to well below 1e-4
+    eps = 2.0 ** -8 if y.dtype is torch.bfloat16 else 2.0 ** -11
+    return ((y.float() - ref).abs() <= eps * ref.abs() + 1e-4).all().item()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [1, 15, 32, 33, 64, 65, 127, 128])
+@pytest.mark.parametrize("n,k,bias", [(16, 64, True), (80, 192, False), (4096, 1024, True), (2048, 4160, True), (12304, 512, False)])
+def test_rows_against_float32(dtype, rows, n, k, bias):
+    x, w, b, ref = _inputs(rows, n, k, dtype, bias)
+    before = _lib.LAUNCHES[0]
+    with torch.no_grad():
+        y = linear_rows(x, w, b)
+        again = linear_rows(x, w, b)
+    assert _lib.LAUNCHES[0] == before + 2 and _close(y, ref) and torch.equal(y, again)
+
+
+@pytest.mark.parametrize("rows,n,k", [(61, 4096, 4096), (128, 2048, 2048)])
+def test_slices_under_capture_and_on_streams(rows, n, k):
+    """The slices' counters: two streams at once, and a graph beside eager calls of its stream."""
+    assert _k_slices(n, k) > 1
+    x, w, b, ref = _inputs(rows, n, k, torch.bfloat16, True)
+    main, side = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.no_grad():
+        outs = []
+        for _ in range(20):
+            for s in (main, side):
+                with torch.cuda.stream(s):
+                    outs.append(linear_rows(x, w, b))
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, outs[0]) for o in outs) and _close(outs[0], ref)
+        for s in (main, torch.cuda.Stream()):  # a stream with a workspace, and one that has none yet
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=s):
+                y = linear_rows(x, w, b)
+            for _ in range(3):
+                y.zero_()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(y, outs[0])
+                assert torch.equal(linear_rows(x, w, b), outs[0])
+
+
+def test_what_it_does_not_take():
+    x, w, b, _ = _inputs(8, 96, 128, torch.bfloat16, True)
+    with torch.no_grad():
+        before = _lib.LAUNCHES[0]
+        for args in ((x, w[:90], b[:90]), (x[:, :120], w[:, :120], b), (x.float(), w.float(), b.float()), (x[:0], w, b)):
+            assert torch.allclose(linear_rows(*args).float(), F.linear(*args).float(), atol=0.05)
+        assert _lib.LAUNCHES[0] == before
+        assert _rows_mm(x, w[:90], b[:90]) is None
+    p = torch.nn.Parameter(w)
+    assert linear_rows(x, p, b).requires_grad
+    with pytest.raises(RuntimeError):
+        _lib.call("kca_rows_mm", 1, x.data_ptr(), w.data_ptr(), None, x.data_ptr(), None, None, 0, 0, 129, 96, 128, 1, _lib.stream())
