@@ -119,23 +119,34 @@ __device__ __forceinline__ float lane_of(float v, int j) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
 }
 
-// Both rules for up to 64 outputs, one a lane: choices by rank, all at once. (NaN counts as the least; ties go to the
-// lower index, so ranks are distinct.)
+// largest over the wave, in every lane (rows of 16 by DPP, the four rows by lane reads)
+__device__ __forceinline__ float lanes_max(float x) {
+  x = lanes_reduce<16>(x, [](float a, float b) { return fmaxf(a, b); });
+  return fmaxf(fmaxf(lane_of(x, 0), lane_of(x, 16)), fmaxf(lane_of(x, 32), lane_of(x, 48)));
+}
+
+// Both rules for up to 64 outputs, one a lane. (NaN counts as the least; ties go to the lower index.) The largest is
+// taken `top` times, or, where that is more than half of the outputs, all ranks are counted at once: 16 instructions a
+// choice, 8 an output (1 token, top 2 of 16, one workgroup: counting 11.7 us, taking 8.9).
 __device__ __forceinline__ void pick_lanes(const RouteArgs& p, const float* z, float fix, int t, int lane, int* ids_lds) {
   const bool on = lane < p.E;
   float s = on ? z[lane] : -INFINITY, c;
   if (p.softmax) {
     auto add = [](float a, float b) { return a + b; };
-    auto big = [](float a, float b) { return fmaxf(a, b); };
-    const float mx = lanes_reduce<64>(s, big), e = on ? expf(s - mx) : 0.f;
+    const float mx = lanes_max(s), e = on ? expf(s - mx) : 0.f;
     s = e / lanes_reduce<64>(e, add);
     c = on ? s + fix : -INFINITY;
     if (c != c) c = -INFINITY;
     if (p.keep < p.groups) {
       const int size = p.E / p.groups, g = lane / size;
-      float best = -INFINITY;
+      auto big = [](float a, float b) { return fmaxf(a, b); };
+      float best = c;
+      if (size == 8) best = lanes_reduce<8>(c, big);
+      else if (size == 16) best = lanes_reduce<16>(c, big);
+      else if (size == 4) best = lanes_reduce<4>(c, big);
+      else
+        for (int j = 0; j < size; ++j) best = fmaxf(best, __shfl(c, g * size + j, 64));
       int ahead = 0;  // groups before this lane's
-      for (int j = 0; j < size; ++j) best = fmaxf(best, __shfl(c, g * size + j, 64));
       for (int j = 0; j < p.groups; ++j) {
         const float o = lane_of(best, j * size);
         ahead += o > best || (o == best && j < g);
@@ -145,10 +156,22 @@ __device__ __forceinline__ void pick_lanes(const RouteArgs& p, const float* z, f
   } else {
     c = s != s ? -INFINITY : s;
   }
-  int rank = 0;
-  for (int j = 0; j < p.E; ++j) {
-    const float o = lane_of(c, j);
-    rank += o > c || (o == c && j < lane);
+  int rank = 64;
+  if (2 * p.top <= p.E) {
+    unsigned long long left = p.E == 64 ? ~0ull : (1ull << p.E) - 1;
+    float m = on ? c : -INFINITY;
+    for (int k = 0; k < p.top; ++k) {
+      const float best = lanes_max(m);
+      const int at = __builtin_ctzll(__ballot(c == best) & left);
+      left &= ~(1ull << at);
+      if (lane == at) rank = k, m = -INFINITY;
+    }
+  } else {
+    rank = 0;
+    for (int j = 0; j < p.E; ++j) {
+      const float o = lane_of(c, j);
+      rank += o > c || (o == c && j < lane);
+    }
   }
   const bool take = on && rank < p.top;
   float w = sigmoid(s);
@@ -335,6 +358,111 @@ __global__ void __launch_bounds__(NW * 64) route_mfma_kernel(RouteArgs p, GroupA
     __syncthreads();
     gr.ids = sids;
     group_rows<NW * 64>(gr, reinterpret_cast<int*>(part));
+  }
+}
+
+// bf16, up to 64 outputs and 1024 tokens: the 16 cuts of K that one workgroup of the kernel above takes, over four
+// workgroups of four waves. Bound by a CU's loads: 16 token rows and 32 output rows of 2048 are 192 KiB, which one CU
+// fetched in 11 us, its 16 waves' registers too few to request everything at once; a quarter of it is in flight whole.
+// The last of the four adds the cuts (in the same order, so the logits are those of the kernel above, bit for bit),
+// chooses and, GROUP, groups. parts: [token block][16 cuts][16 tokens][16 nt], cnt: a zeroed counter a token block.
+// Sixteen waves although four of them load: one a token chooses (four tokens a wave, side by side, took twice as long).
+// Routing and grouping, us, one workgroup a token block : this (launches back to back; 32 outputs of 2048, 16 of 4096, sigmoid):
+//   1 token 12.4 : 7.2, 8.9 : 7.0; 16 tokens 15.9 : 8.2, 11.9 : 8.1; 128 tokens 17.6 : 10.2, 13.4 : 10.0;
+//   1024 tokens 19.6 : 14.1, 14.5 : 13.0 (the blocks alone come near filling the chip)
+template <bool GROUP>
+__global__ void __launch_bounds__(1024) route_split_kernel(RouteArgs p, GroupArgs gr, float* parts, unsigned* cnt) {
+  __shared__ __attribute__((aligned(16))) float z[16 * 64];
+  __shared__ int sids[GROUP ? 16 * 64 : 1], sh[GROUP ? 3 * 64 + 2 : 1], s_last;
+  const int n = p.E + (p.wsg ? 1 : 0), nt = (n + 15) / 16, d = p.d, nk = (d + 31) / 32;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, r16 = lane & 15, g = lane >> 4;
+  const int tb = blockIdx.x / 4, cut = blockIdx.x % 4 * 4 + (wv & 3), t0 = tb * 16;
+  const bf16_t* h = reinterpret_cast<const bf16_t*>(p.h) + (long long)min(t0 + r16, p.T - 1) * d;
+  const float fix = lane_fix(p, lane);
+  const bf16_t* w[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int e = min(16 * i + r16, n - 1);
+    w[i] = e < p.E ? reinterpret_cast<const bf16_t*>(p.wr) + (long long)e * d : reinterpret_cast<const bf16_t*>(p.wsg);
+  }
+  f32x4 acc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto steps = [&](auto ntc, auto ahead) {
+    constexpr int NTC = decltype(ntc)::value, AH = decltype(ahead)::value;
+    for (int k0 = cut * 2; k0 < nk; k0 += 16 * AH) {  // 64 columns at a time: whole cache lines of every row
+      u32x4 a[AH][NTC], b[AH];
+#pragma unroll
+      for (int j = 0; j < AH; ++j) {  // (no load is conditional; columns past d multiply zeros)
+        const int c = (k0 + (j & 1) + (j >> 1) * 32) * 32 + g * 8, cc = min(c, d - 8);
+        b[j] = *reinterpret_cast<const u32x4*>(h + cc);
+#pragma unroll
+        for (int i = 0; i < NTC; ++i) a[j][i] = *reinterpret_cast<const u32x4*>(w[i] + cc);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // all requested before the first is waited for
+#pragma unroll
+      for (int j = 0; j < AH; ++j) {
+        const int c = (k0 + (j & 1) + (j >> 1) * 32) * 32 + g * 8;
+        const uint32_t keep = c < d ? ~0u : 0u;
+        const u32x4 x = b[j] & u32x4{keep, keep, keep, keep};
+#pragma unroll
+        for (int i = 0; i < NTC; ++i)
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[j][i]), __builtin_bit_cast(bf16x8, x),
+                                                           acc[i], 0, 0, 0);
+      }
+    }
+  };
+  auto store = [&] {
+    auto* to = reinterpret_cast<unsigned long long*>(parts + ((long long)(tb * 16 + cut) * 16 + r16) * (16 * nt) + 4 * g);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i < nt) {
+        const unsigned long long* v = reinterpret_cast<const unsigned long long*>(&acc[i]);
+        __hip_atomic_store(to + 8 * i, v[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(to + 8 * i + 1, v[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+  };
+  using std::integral_constant;
+  if (wv < 4) {  // the other twelve waves choose
+    const bool narrow = nk <= 64;  // four steps a cut
+    if (nt == 1 && narrow) steps(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+    else if (nt == 1) steps(integral_constant<int, 1>{}, integral_constant<int, 8>{});
+    else if (nt == 2 && narrow) steps(integral_constant<int, 2>{}, integral_constant<int, 4>{});
+    else if (nt == 2) steps(integral_constant<int, 2>{}, integral_constant<int, 8>{});
+    else steps(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+    store();
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) {
+    const int last = __hip_atomic_fetch_add(cnt + tb, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 3;
+    if (last) {
+      __hip_atomic_store(cnt + tb, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    s_last = last;
+  }
+  __syncthreads();
+  if (!s_last) return;
+  if (const int r = tid >> 4, q = tid & 15; r < 16 && q < nt * 4) {
+    const float* from = parts + ((long long)tb * 256 + r) * (16 * nt) + 4 * q;
+    f32x4 v[16], s{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 16; ++c) v[c] = *reinterpret_cast<const f32x4*>(from + (long long)c * 256 * nt);
+#pragma unroll
+    for (int c = 0; c < 16; ++c) s += v[c];
+    *reinterpret_cast<f32x4*>(z + r * 64 + 4 * q) = s;
+  }
+  __syncthreads();
+  if (t0 + wv < p.T) {
+    if (p.wsg && lane == 0) p.sg[t0 + wv] = sigmoid(z[wv * 64 + p.E]);
+    pick_lanes(p, z + wv * 64, fix, t0 + wv, lane, GROUP ? sids : nullptr);
+  }
+  if constexpr (GROUP) {
+    __syncthreads();
+    gr.ids = sids;
+    group_rows<1024>(gr, sh);
   }
 }
 
@@ -832,14 +960,25 @@ int route_go(const RouteArgs& a, const GroupArgs& g, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? 0 : 4;
 }
 
+template <bool GROUP>
+int split_go(const RouteArgs& a, const GroupArgs& g, void* ws, long long ws_floats, void* cnt, int cnt_n, hipStream_t s) {
+  const int n = a.E + (a.wsg ? 1 : 0), blocks = (a.T + 15) / 16;
+  if (n > 64 || a.T > 1024 || !cnt || cnt_n < blocks || !al16(ws) || ws_floats < blocks * 256ll * ((n + 15) / 16 * 16)) return 6;
+  hipLaunchKernelGGL(route_split_kernel<GROUP>, dim3(blocks * 4), dim3(1024), 0, s, a, g, (float*)ws, (unsigned*)cnt);
+  return hipGetLastError() == hipSuccess ? 0 : 4;
+}
+
 }  // namespace
 
-// dtype: 0 fp32, 1 bf16
+// dtype: 0 fp32, 1 bf16. ws: the split kernel (bf16, d % 8 == 0, up to 64 outputs with the shared gate and 1024 tokens), with
+// ceil(T / 16) * 256 * (outputs rounded up to 16) floats there and ceil(T / 16) zeroed counters at cnt (left zeroed)
 KCA_API int kca_moe_route(int dtype, const void* h, const void* wr, const void* wsg, void* ids, void* wts, void* sg,
-                          int T, int d, int E, int top, int softmax, const void* fix, int groups, int keep, hipStream_t s) {
+                          int T, int d, int E, int top, int softmax, const void* fix, int groups, int keep, void* ws,
+                          long long ws_floats, void* cnt, int cnt_n, hipStream_t s) {
   const RouteArgs a{h, wr, wsg, (int*)ids, (float*)wts, (float*)sg, T, d, E, top, softmax, groups, keep, (const float*)fix};
   if (!route_ok(a)) return 1;
   if (dtype == 1 && d % 8 == 0 && al16(h) && al16(wr) && al16(wsg)) {
+    if (ws) return split_go<false>(a, GroupArgs{}, ws, ws_floats, cnt, cnt_n, s);
     if (T <= 1024 && route_lds<16, false>(a) <= MAX_LDS) return route_go<16, false>(a, GroupArgs{}, s);
     if (route_lds<8, false>(a) <= MAX_LDS) return route_go<8, false>(a, GroupArgs{}, s);
   }
@@ -867,12 +1006,14 @@ KCA_API int kca_moe_group(const void* ids, int n, int E, int mt, void* perm, voi
 // Both in one launch: bf16, at most 16 tokens (10: shape outside it). E: router outputs, the first `real` with weights
 KCA_API int kca_moe_route_group(const void* h, const void* wr, const void* wsg, void* ids, void* wts, void* sg, int T,
                                 int d, int E, int real, int top, int softmax, const void* fix, int groups, int keep, int mt, void* perm,
-                                void* inv, void* tiles, int max_tiles, void* ntiles, hipStream_t s) {
+                                void* inv, void* tiles, int max_tiles, void* ntiles, void* ws, long long ws_floats, void* cnt,
+                                int cnt_n, hipStream_t s) {
   const RouteArgs a{h, wr, wsg, (int*)ids, (float*)wts, (float*)sg, T, d, E, top, softmax, groups, keep, (const float*)fix};
   if (!route_ok(a) || real < 1 || real > E) return 1;
   if (T > 16 || top > 64 || d % 8 || !al16(h) || !al16(wr) || !al16(wsg) || route_lds<16, true>(a) > MAX_LDS) return 10;
   const GroupArgs g{(const int*)ids, T * top, real, mt, (int*)perm, (int*)inv, (int*)tiles, (int*)ntiles};
   if (!group_ok(g, max_tiles)) return 1;
+  if (ws) return split_go<true>(a, g, ws, ws_floats, cnt, cnt_n, s);
   return route_go<16, true>(a, g, s);
 }
 

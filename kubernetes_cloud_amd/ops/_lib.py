@@ -121,9 +121,9 @@ _SIGS.update({
     "kca_rms_shift": [I, P, P, P, P, LL, P, P, I, F, P, I, F, P, P, P, P, P, P, P, P, P, P, P, I, I, I, P],
     "kca_gated_scan": [I, P, LL, P, P, P, LL, P, P, LL, P, I, I, I, P],
     "kca_gated_step": [I, P, LL, P, P, P, LL, P, P, P, I, I, P],
-    "kca_moe_route": [I, P, P, P, P, P, P, I, I, I, I, I, P, I, I, P],
+    "kca_moe_route": [I, P, P, P, P, P, P, I, I, I, I, I, P, I, I, P, LL, P, I, P],
     "kca_moe_group": [P, I, I, I, P, P, P, I, P, P],
-    "kca_moe_route_group": [P, P, P, P, P, P, I, I, I, I, I, I, P, I, I, I, P, P, P, I, P, P],
+    "kca_moe_route_group": [P, P, P, P, P, P, I, I, I, I, I, I, P, I, I, I, P, P, P, I, P, P, LL, P, I, P],
     "kca_moe_expert": [I, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P, P, P, I, I, I, I, P],
     "kca_rows_mm": [I, P, P, P, P, P, P, LL, I, I, I, I, I, P],
     "kca_act_rows": [I, I, P, LL, P, P, P, LL, I, I, F, P],
@@ -246,11 +246,22 @@ def stream() -> int:
     return _raw_stream(_current_device())
 
 
-def stream_on(device: torch.device) -> int:
-    """The current stream's handle on a device (``stream``: on the current one)."""
-    if _raw_stream is None or device.index is None:
-        return torch.cuda.current_stream(device).cuda_stream
-    return _raw_stream(device.index)
+_COUNTERS: dict = {}
+
+
+def counters(device: torch.device, n: int) -> torch.Tensor:
+    """At least ``n`` zeroed int32 counters for a launch on the current stream that leaves them zeroed: one small tensor a
+    stream, whose launches are ordered. Within a capture they are the graph's own, cleared by it: its replays may run
+    beside other work."""
+    if torch.cuda.is_current_stream_capturing():
+        return torch.zeros(n, device=device, dtype=torch.int32)
+    key = (device.index, stream())
+    c = _COUNTERS.get(key)
+    if c is None or c.numel() < n:
+        if len(_COUNTERS) >= 256:  # (memory of its stream: what takes it next is ordered after what reads it now)
+            _COUNTERS.clear()
+        c = _COUNTERS[key] = torch.zeros(max(n, 1024), device=device, dtype=torch.int32)
+    return c
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

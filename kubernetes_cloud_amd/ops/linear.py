@@ -179,7 +179,6 @@ def _k_slices(n: int, k: int) -> int:
 
 def _rows_mm(x2: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor | None:
     """The product of up to FEW_ROWS rows on the weight-streaming kernel; None: sizes or alignment it does not take."""
-    from .skinny_mm import _workspace
     rows, k = x2.shape
     n = weight.shape[0]
     if (n % 16 or k % 64 or k == 0 or 2 * n * k >= 1 << 32 or not weight.is_contiguous() or x2.data_ptr() % 16
@@ -188,7 +187,8 @@ def _rows_mm(x2: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) 
     ks, ws, cnt = _k_slices(n, k), None, None
     if ks > 1:
         blocks = -(-n // 64)
-        ws, cnt = _workspace(x2.device, blocks * ks * 64 * (32 if rows <= 32 else 64 if rows <= 64 else 128), blocks)
+        ws = torch.empty(blocks * ks * 64 * (32 if rows <= 32 else 64 if rows <= 64 else 128), device=x2.device, dtype=torch.float32)
+        cnt = _lib.counters(x2.device, blocks)
     y = torch.empty(rows, n, device=x2.device, dtype=x2.dtype)
     _lib.call("kca_rows_mm", 1 if x2.dtype == torch.bfloat16 else 2, x2.data_ptr(), weight.data_ptr(), _lib.ptr(bias),
               y.data_ptr(), _lib.ptr(ws), _lib.ptr(cnt), 0 if ws is None else ws.numel(), 0 if cnt is None else cnt.numel(),

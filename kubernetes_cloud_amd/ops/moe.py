@@ -59,9 +59,29 @@ def route(h: torch.Tensor, router: torch.Tensor, top: int, shared_gate: torch.Te
     ids = torch.empty(T, top, device=h.device, dtype=torch.int32)
     w = torch.empty(T, top, device=h.device, dtype=torch.float32)
     sg = torch.empty(T, device=h.device, dtype=torch.float32) if shared_gate is not None else None
+    space = _split_space(h, E, shared_gate, code)  # (held until the launch is on the stream)
     _lib.call("kca_moe_route", code, h.data_ptr(), router.data_ptr(), _lib.ptr(shared_gate), ids.data_ptr(),
-              w.data_ptr(), _lib.ptr(sg), T, d, E, top, *_rule_args(rule, E), _lib.stream())
+              w.data_ptr(), _lib.ptr(sg), T, d, E, top, *_rule_args(rule, E), *_space_args(*space), _lib.stream())
     return ids, w, sg
+
+
+def _split_space(h: torch.Tensor, E: int, shared_gate: torch.Tensor | None, code: int) -> tuple:
+    """Workspace and counters of the router kernel whose cuts of K run in four workgroups, or none: the kernel of one
+    workgroup a token block. That serves more than 64 outputs (a token's choice there takes a wave's whole time, and the
+    last of four workgroups has four waves), more than 1024 tokens (blocks enough to fill the chip) and captures
+    (whose counters would be cleared by a launch of their own)."""
+    T, d = h.shape
+    n = E + (shared_gate is not None)
+    if (code != 1 or n > 64 or T > 1024 or d % 8 or h.data_ptr() % 16 or torch.cuda.is_current_stream_capturing()
+            or h.get_device() != torch.cuda.current_device()):
+        return None, None
+    blocks = -(-T // 16)
+    ws = torch.empty(blocks * 256 * (-(-n // 16) * 16), device=h.device, dtype=torch.float32)
+    return ws, _lib.counters(h.device, blocks)
+
+
+def _space_args(ws: torch.Tensor | None, cnt: torch.Tensor | None) -> tuple:
+    return (None, 0, None, 0) if ws is None else (ws.data_ptr(), ws.numel(), cnt.data_ptr(), cnt.numel())
 
 
 def _rule_args(rule: Router, E: int) -> tuple:
@@ -136,9 +156,10 @@ def route_group(h: torch.Tensor, router: torch.Tensor, top: int, shared_gate: to
         w = torch.empty(T, top, device=h.device, dtype=torch.float32)
         sg = torch.empty(T, device=h.device, dtype=torch.float32) if shared_gate is not None else None
         assert h.is_contiguous() and router.is_contiguous() and router.shape[1] == d
+        space = _split_space(h, E, shared_gate, 1)  # (held until the launch is on the stream)
         _lib.call("kca_moe_route_group", h.data_ptr(), router.data_ptr(), _lib.ptr(shared_gate), ids.data_ptr(),
                   w.data_ptr(), _lib.ptr(sg), T, d, E, real, top, *_rule_args(rule, E), mt, g.perm.data_ptr(), g.inv.data_ptr(),
-                  g.tiles.data_ptr(), g.tiles.shape[0], g.ntiles.data_ptr(), _lib.stream())
+                  g.tiles.data_ptr(), g.tiles.shape[0], g.ntiles.data_ptr(), *_space_args(*space), _lib.stream())
         return ids, w, sg, g
     ids, w, sg = route(h, router, top, shared_gate, rule)
     return ids, w, sg, group(ids, real, mt)

@@ -177,7 +177,7 @@ def job(parts, N: int, y: torch.Tensor, bias=None, act: int = 0, res=None, stats
 
 
 def _workspace(device, floats: int, nblk: int):
-    key = (device, _lib.stream_on(device))
+    key = (str(device), torch.cuda.current_stream(device).cuda_stream)
     ws = _WS.get(key)
     if ws is None or ws[0].numel() < floats or ws[1].numel() < nblk:
         if torch.cuda.is_current_stream_capturing():

@@ -1,0 +1,74 @@
+"""The router whose cuts of K run in four workgroups gives the bits of the one-workgroup kernel, also across streams."""
+import pytest
+import torch
+
+from kubernetes_cloud_amd.ops import moe
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(T, d, E, gate, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    h = torch.empty(T, d, device="cuda", dtype=torch.bfloat16).normal_(generator=g)
+    r = torch.empty(E, d, device="cuda", dtype=torch.bfloat16).normal_(std=d ** -0.5, generator=g)
+    return h, r, torch.empty(d, device="cuda", dtype=torch.bfloat16).normal_(std=d ** -0.5, generator=g) if gate else None
+
+
+def _rule(E, soft, identity):
+    if not soft:
+        return moe.SIGMOID
+    fix = torch.linspace(-0.01, 0.01, E, device="cuda")
+    return moe.Router(softmax=True, correction=fix, groups=4, keep=3, identity=identity)
+
+
+def _unsplit(monkeypatch, *a):
+    with monkeypatch.context() as m:
+        m.setattr(moe, "_split_space", lambda *_: (None, None))
+        return moe.route_group(*a)
+
+
+@pytest.mark.parametrize("T", [1, 3, 16, 17, 31, 50, 1023, 1024])
+@pytest.mark.parametrize("d,E,top,gate,soft", [(64, 8, 2, False, False), (2048, 32, 4, True, False), (2056, 63, 6, True, False),
+                                               (4096, 16, 2, False, False), (4104, 64, 64, False, False),
+                                               (2048, 32, 5, False, True), (4096, 20, 3, False, True), (512, 64, 8, False, True)])
+def test_same_bits_as_one_workgroup(monkeypatch, T, d, E, top, gate, soft):
+    if top > E // 4 * 3 and soft:
+        pytest.skip("fewer experts than choices in the kept groups")
+    h, r, sg = _inputs(T, d, E, gate)
+    a = (h, r, top, sg, 8, _rule(E, soft, E // 4 if soft else 0))
+    assert moe._split_space(h, E, sg, 1)[0] is not None
+    ids, w, s, g = moe.route_group(*a)
+    ids0, w0, s0, g0 = _unsplit(monkeypatch, *a)
+    assert torch.equal(ids, ids0) and torch.equal(w, w0) and (s is None or torch.equal(s, s0))
+    assert torch.equal(g.ntiles, g0.ntiles)
+    k = int(g.ntiles)
+    assert torch.equal(g.tiles[:k], g0.tiles[:k])
+    # (the order of an expert's rows is free) every assignment has its own row, of its expert
+    for q in (g, g0):
+        rows = q.inv.reshape(-1)
+        real = rows >= 0
+        assert torch.equal(q.perm[rows[real].long()].long(), real.nonzero().reshape(-1))
+    assert torch.equal(g.inv >= 0, g0.inv >= 0)
+
+
+def test_streams_and_captures(monkeypatch):
+    h, r, sg = _inputs(300, 2048, 32, True)
+    a = (h, r, 4, sg, 8)
+    ids0, w0, _, _ = _unsplit(monkeypatch, *a)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    outs = []
+    for _ in range(20):
+        for st in streams:
+            with torch.cuda.stream(st):
+                outs.append(moe.route_group(*a)[:2])
+    torch.cuda.synchronize()
+    assert all(torch.equal(i, ids0) and torch.equal(w, w0) for i, w in outs)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=streams[0]):
+        ids, w, _, _ = moe.route_group(*a)
+    for _ in range(3):
+        ids.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(ids, ids0) and torch.equal(w, w0) and torch.equal(moe.route_group(*a)[0], ids0)
