@@ -1272,39 +1272,44 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 3 : 1) attn_
   row_bases<D>(l32, hh, be, bo);
   tr_bases<D>(lane, b1, b2);
 
-#define KCA_DKDV_LOAD(it_)                                                                     \
-  {                                                                                            \
-    const int hq_ = hk * grp + (it_) / nqt, qt_ = q_lo + ((it_) % nqt) * BQ;                   \
-    if (grp > 1) stg.set_base(p.q + b * p.q_sb + hq_ * p.q_sh, p.dout + b * p.do_sb + hq_ * p.do_sh, qn, gn); \
-    stg.load(sq, sg, p.q + b * p.q_sb + hq_ * p.q_sh, p.dout + b * p.do_sb + hq_ * p.do_sh, qt_,   \
-             p.q_st, p.do_st);                                                                 \
-    if (tid < 64) {                                                                            \
-      const int qr_ = qt_ + (tid & 31);                                                        \
-      const long long li_ = ((long long)b * p.H + hq_) * p.Sq + (G ? min(qr_, p.Sq - 1) : qr_); \
-      lreg = tid < 32 ? p.lse[li_] * kLog2e : p.delta[li_];                                    \
-      if (G && qr_ >= p.Sq) lreg = tid < 32 ? INFINITY : 0.f;  /* P = 0 */                     \
-    }                                                                                          \
-  }
-#define KCA_DKDV_STORE(buf_)                                                                   \
-  {                                                                                            \
-    stg.store(sq, sg, smem + (buf_) * 2 * TILE);                                               \
-    if (tid < 64) reinterpret_cast<float*>(smem + LOFF)[(buf_) * 64 + tid] = lreg;             \
-  }
+  // Tile (nh, nq): query head and q tile of the next step, counted instead of divided out of the step number. The 64 lse /
+  // delta values go to LDS as they come: anything done to them here would wait for the whole tile's loads, in one wave
+  // that the others then wait for at the barrier. The scaling (and G's end of the rows) is done where they are stored.
+  int hcur = 0, qcur = 0;  // the current step's
+  auto load_tile = [&](int nh, int nq) {
+    const int hq = hk * grp + nh, qt = q_lo + nq * BQ;
+    const bf16_t *qb = p.q + b * p.q_sb + hq * p.q_sh, *gb = p.dout + b * p.do_sb + hq * p.do_sh;
+    if (grp > 1) stg.set_base(qb, gb, qn, gn);
+    stg.load(sq, sg, qb, gb, qt, p.q_st, p.do_st);
+    if (tid < 64) {
+      const int qr = qt + (tid & 31);
+      const long long li = ((long long)b * p.H + hq) * p.Sq + (G ? min(qr, p.Sq - 1) : qr);
+      lreg = (tid < 32 ? p.lse : p.delta)[li];
+    }
+  };
+  auto store_tile = [&](int buf, int nq) {
+    stg.store(sq, sg, smem + buf * 2 * TILE);
+    if (tid < 64) {
+      float v = tid < 32 ? lreg * kLog2e : lreg;
+      if (G && q_lo + nq * BQ + (tid & 31) >= p.Sq) v = tid < 32 ? INFINITY : 0.f;  // P = 0
+      reinterpret_cast<float*>(smem + LOFF)[buf * 64 + tid] = v;
+    }
+  };
 
   if (total > 0) {
-    KCA_DKDV_LOAD(0);
-    KCA_DKDV_STORE(0);
+    load_tile(0, 0);
+    store_tile(0, 0);
   }
   __syncthreads();
   ASTAMP(0);
   auto tile_step = [&](int it, auto masked) {
     constexpr bool MASKED = decltype(masked)::value;
-    const int qt = q_lo + (it % nqt) * BQ;
+    const int qt = q_lo + qcur * BQ, hq = hk * grp + hcur;
     const char* Qs = smem + (it & 1) * 2 * TILE;
     const char* Gs = Qs + TILE;
     const float* ls = reinterpret_cast<const float*>(smem + LOFF) + (it & 1) * 64;
-    const int nx = min(it + 1, total - 1);
-    KCA_DKDV_LOAD(nx);
+    if (it + 1 < total && ++qcur == nqt) qcur = 0, ++hcur;  // (the last step loads its own tile again)
+    load_tile(hcur, qcur);
     asm volatile("" ::: "memory");
     ASTAMP(1);
     // No skip of the (at most 3 per head) q tiles that lie wholly above this
@@ -1349,7 +1354,7 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 3 : 1) attn_
     const int ul = G && p.window > 0 ? key + p.window - off - qt - 4 * hh : 1 << 30;  // G: and 8g + j < ul
     float slope = 0.f, b0 = 0.f;
     if constexpr (G == 2) {
-      slope = p.alibi[hk * grp + it / nqt] * kLog2e;
+      slope = p.alibi[hq] * kLog2e;
       b0 = slope * (float)(key - qt - off - 4 * hh);
     }
     bf16x8 p0, p1, s0, s1;
@@ -1404,7 +1409,7 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 3 : 1) attn_
     }
     ASTAMP(4);
     asm volatile("" ::: "memory");
-    if (it + 1 < total) KCA_DKDV_STORE((it + 1) & 1);
+    if (it + 1 < total) store_tile((it + 1) & 1, qcur);
     __syncthreads();
     ASTAMP(5);
   };
@@ -1412,8 +1417,6 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 3 : 1) attn_
   // splitting into masked / mask-free bodies -- by a per-tile branch or by
   // two loops per head -- pushed the 256 dK/dV accumulators into spills.
   for (int it = 0; it < total; ++it) tile_step(it, std::integral_constant<bool, (CAUSAL || G > 0)>{});
-#undef KCA_DKDV_LOAD
-#undef KCA_DKDV_STORE
   if constexpr (D == 96) {  // the LDS staging's registers push this one past 256 (2 -> 1 wave per SIMD)
     if (!G || key < p.Sk) {
       store_acc_t<D>(p.dk + b * p.dk_sb + hk * p.dk_sh + (long long)key * p.dk_st, dk, hh, p.scale);
