@@ -180,6 +180,12 @@ struct Stager<D, true> {
       sv[i] = *reinterpret_cast<const u32x4*>(&b);
     }
   }
+  // one of the 2 CPT loads
+  __device__ __forceinline__ void load_one(int j, u32x4 (&sk)[CPT], u32x4 (&sv)[CPT], int sok, int sov) const {
+    const auto a = j < CPT ? __builtin_amdgcn_raw_buffer_load_b128(rk_, vok_[j < CPT ? j : 0], sok, 0)
+                           : __builtin_amdgcn_raw_buffer_load_b128(rv_, vov_[j < CPT ? 0 : j - CPT], sov, 0);
+    (j < CPT ? sk[j < CPT ? j : 0] : sv[j < CPT ? 0 : j - CPT]) = *reinterpret_cast<const u32x4*>(&a);
+  }
   __device__ __forceinline__ void store(const u32x4 (&sk)[CPT], const u32x4 (&sv)[CPT], char* buf) const {
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
@@ -232,6 +238,12 @@ struct Stager<D, false> {
       sv[i] = *reinterpret_cast<const u32x4*>(&b);
     }
   }
+  // one of the 2 CPT loads
+  __device__ __forceinline__ void load_one(int j, u32x4 (&sk)[CPT], u32x4 (&sv)[CPT], int sok, int sov) const {
+    const auto a = j < CPT ? __builtin_amdgcn_raw_buffer_load_b128(rk_, vok_[j < CPT ? j : 0], sok, 0)
+                           : __builtin_amdgcn_raw_buffer_load_b128(rv_, vov_[j < CPT ? 0 : j - CPT], sov, 0);
+    (j < CPT ? sk[j < CPT ? j : 0] : sv[j < CPT ? 0 : j - CPT]) = *reinterpret_cast<const u32x4*>(&a);
+  }
   __device__ __forceinline__ void store(const u32x4 (&sk)[CPT], const u32x4 (&sv)[CPT], char* buf) const {
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
@@ -277,6 +289,12 @@ struct StagerNarrow {
     const auto b = __builtin_amdgcn_raw_buffer_load_b128(rv_, vov_[0], sov, 0);
     sk[0] = *reinterpret_cast<const u32x4*>(&a);
     sv[0] = *reinterpret_cast<const u32x4*>(&b);
+  }
+  // one of the 2 CPT loads
+  __device__ __forceinline__ void load_one(int j, u32x4 (&sk)[1], u32x4 (&sv)[1], int sok, int sov) const {
+    const auto a = j < CPT ? __builtin_amdgcn_raw_buffer_load_b128(rk_, vok_[j < CPT ? j : 0], sok, 0)
+                           : __builtin_amdgcn_raw_buffer_load_b128(rv_, vov_[j < CPT ? 0 : j - CPT], sov, 0);
+    (j < CPT ? sk[j < CPT ? j : 0] : sv[j < CPT ? 0 : j - CPT]) = *reinterpret_cast<const u32x4*>(&a);
   }
   __device__ __forceinline__ void store(const u32x4 (&sk)[1], const u32x4 (&sv)[1], char* buf) const {
     if (on_) {
@@ -1028,6 +1046,7 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 4 : 1) attn_
   constexpr int TILE = BN * D * 2;
   using Stg = StagerFor<D, DS>;
   constexpr int CPT = Stg::CPT;
+  constexpr bool SPREAD = D == 256;  // the next tile's loads, one a step among the products (as in the dK/dV kernel)
   constexpr int KSD = DS / 16;  // contraction steps over the stored columns
   __shared__ __attribute__((aligned(16))) char smem[4 * TILE];
   ASTAMP_DECL
@@ -1055,6 +1074,13 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 4 : 1) attn_
   const int qr = G ? min(qrow, p.Sq - 1) : qrow;
   const bf16_t* qp = p.q + b * p.q_sb + h * p.q_sh + (long long)qr * p.q_st;
   const bf16_t* gp = p.dout + b * p.do_sb + h * p.do_sh + (long long)qr * p.do_st;
+  const bf16_t* kst = p.k + b * p.k_sb + hk * p.k_sh;
+  const bf16_t* vst = p.v + b * p.v_sb + hk * p.v_sh;
+  Stg stg(tid, p.k_st, p.v_st);
+  if constexpr (G > 0) stg.bind(kst, vst, p.k_st, p.v_st, rows_bytes(kv_end, p.k_st, D), rows_bytes(kv_end, p.v_st, D));
+  else stg.bind(kst, vst, p.k_st, p.v_st);
+  u32x4 sk[CPT], sv[CPT];
+  stg.load(sk, sv, kst, vst, t0 * BN, p.k_st, p.v_st);  // (flies with the query rows)
   bf16x8 qf[KSD], gf[KSD];
 #pragma unroll
   for (int s = 0; s < KSD; ++s) {
@@ -1082,12 +1108,6 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 4 : 1) attn_
 #pragma unroll
     for (int r = 0; r < 16; ++r) dq[i][r] = 0.f;
 
-  const bf16_t* kst = p.k + b * p.k_sb + hk * p.k_sh;
-  const bf16_t* vst = p.v + b * p.v_sb + hk * p.v_sh;
-  Stg stg(tid, p.k_st, p.v_st);
-  if constexpr (G > 0) stg.bind(kst, vst, p.k_st, p.v_st, rows_bytes(kv_end, p.k_st, D), rows_bytes(kv_end, p.v_st, D));
-  else stg.bind(kst, vst, p.k_st, p.v_st);
-  u32x4 sk[CPT], sv[CPT];
   int be, bo, b1, b2;
   row_bases<D>(l32, hh, be, bo);
   tr_bases<D>(lane, b1, b2);
@@ -1099,7 +1119,6 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 4 : 1) attn_
     }
   }
 
-  stg.load(sk, sv, kst, vst, t0 * BN, p.k_st, p.v_st);
   stg.store(sk, sv, smem + (t0 & 1) * 2 * TILE);
   __syncthreads();
   ASTAMP(0);
@@ -1113,7 +1132,9 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 4 : 1) attn_
     // (a second register set of loads in flight -- as the forward's PF2 -- only moved this kernel's
     // wait from the LDS store to the load issue: the K/V stream is throughput-bound per CU,
     // profiles/attn_stamps_r2.md)
-    stg.load(sk, sv, kst, vst, min(k0 + BN, (ntiles - 1) * BN), p.k_st, p.v_st);
+    const int kn = min(k0 + BN, (ntiles - 1) * BN);
+    const int sok = __builtin_amdgcn_readfirstlane((int)(kn * p.k_st * 2)), sov = __builtin_amdgcn_readfirstlane((int)(kn * p.v_st * 2));
+    if constexpr (!SPREAD) stg.load(sk, sv, kst, vst, kn, p.k_st, p.v_st);
     asm volatile("" ::: "memory");
     ASTAMP(1);
     f32x16 st, dpt;
@@ -1134,6 +1155,10 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 4 : 1) attn_
           fk[(s + 2) % 3] = row_frag<D>(Ks, be, bo, s + 2);
           fv[(s + 2) % 3] = row_frag<D>(Vs, be, bo, s + 2);
           __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        }
+        if (SPREAD && s < 2 * CPT) {
+          stg.load_one(s, sk, sv, sok, sov);
+          __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);
         }
         st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fk[s % 3], qf[s], st, 0, 0, 0);
         dpt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fv[s % 3], gf[s], dpt, 0, 0, 0);
@@ -1208,6 +1233,10 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 3 : 1) attn_
   using Stg = StagerFor<D, DS>;
   constexpr int NCH = D / 8, NCS = DS / 8, CPT = Stg::CPT;
   constexpr int KSD = DS / 16;                      // contraction steps over the stored columns
+  // The next tile's loads, together before the products or one a step among the first ones. Together they hold the
+  // wave, alone on its SIMD, up for 700 of a tile's 5000 cycles at D = 256 (backward of 2 x 2048 x 16 heads 411 -> 394 us); at
+  // smaller D a tile is short and the time that they fly is what counts (dK/dV, D = 64: 88 us together, 91 spread; 128: 114, 116).
+  constexpr bool SPREAD = D == 256;
   constexpr int VOFF = 4 * TILE;                    // V images of the 4 waves
   constexpr int LOFF = VOFF + 4 * TILE;             // lse/delta: [buf][64] floats
   __shared__ __attribute__((aligned(16))) char smem[LOFF + 2 * 64 * 4];
@@ -1225,36 +1254,6 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 3 : 1) attn_
   const int key = kw + l32;
   const int kv_end = G ? batch_keys(p.kv_len, b, p.Sk) : p.Sk;
   const float sl2 = p.scale * kLog2e;
-
-  const bf16_t* kp = p.k + b * p.k_sb + hk * p.k_sh;
-  const bf16_t* vp = p.v + b * p.v_sb + hk * p.v_sh;
-  bf16x8 kf[KSD];
-#pragma unroll
-  for (int s = 0; s < KSD; ++s) {
-    kf[s] = *reinterpret_cast<const bf16x8*>(kp + (long long)(G ? min(key, p.Sk - 1) : key) * p.k_st + 16 * s + 8 * hh);
-    if (G && key >= kv_end) kf[s] = bf16x8{};
-  }
-  // this wave's 32 V rows -> its own image (read back by rows for dP; pad chunks zero)
-  char* vimg = smem + VOFF + wave * TILE;
-#pragma unroll
-  for (int i = 0; i < 32 * NCH / 64; ++i) {
-    const int idx = lane + 64 * i, row = idx / NCH, ch = idx % NCH;
-    *reinterpret_cast<u32x4*>(vimg + img_off<D>(row, ch)) =
-        ch < NCS && (!G || kw + row < kv_end) ? *reinterpret_cast<const u32x4*>(vp + (long long)(kw + row) * p.v_st + ch * 8)
-                                              : u32x4{0, 0, 0, 0};
-  }
-  if constexpr (DS < D) {  // Q / dO image chunks DS/8.. are never loaded: zero them in both buffers once
-    constexpr int PC = NCH - NCS, NZ = 2 * 2 * 32 * PC;
-    for (int i = tid; i < NZ; i += 256) {
-      const int img = i / (32 * PC), row = (i / PC) % 32, ch = NCS + i % PC;
-      *reinterpret_cast<u32x4*>(smem + img * TILE + img_off<D>(row, ch)) = u32x4{0, 0, 0, 0};
-    }
-  }
-  f32x16 dk[D / 32], dv[D / 32];
-#pragma unroll
-  for (int i = 0; i < D / 32; ++i)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) { dk[i][r] = 0.f; dv[i][r] = 0.f; }
 
   int q_lo = 0;
   if (CAUSAL) q_lo = max(0, kb * BK - off) & ~(BQ - 1);
@@ -1276,11 +1275,11 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 3 : 1) attn_
   // delta values go to LDS as they come: anything done to them here would wait for the whole tile's loads, in one wave
   // that the others then wait for at the barrier. The scaling (and G's end of the rows) is done where they are stored.
   int hcur = 0, qcur = 0;  // the current step's
-  auto load_tile = [&](int nh, int nq) {
+  int soq = 0, sog = 0;  // byte offsets of the tile being loaded
+  auto aim_tile = [&](int nh, int nq) {
     const int hq = hk * grp + nh, qt = q_lo + nq * BQ;
-    const bf16_t *qb = p.q + b * p.q_sb + hq * p.q_sh, *gb = p.dout + b * p.do_sb + hq * p.do_sh;
-    if (grp > 1) stg.set_base(qb, gb, qn, gn);
-    stg.load(sq, sg, qb, gb, qt, p.q_st, p.do_st);
+    if (grp > 1) stg.set_base(p.q + b * p.q_sb + hq * p.q_sh, p.dout + b * p.do_sb + hq * p.do_sh, qn, gn);
+    soq = __builtin_amdgcn_readfirstlane((int)(qt * p.q_st * 2)), sog = __builtin_amdgcn_readfirstlane((int)(qt * p.do_st * 2));
     if (tid < 64) {
       const int qr = qt + (tid & 31);
       const long long li = ((long long)b * p.H + hq) * p.Sq + (G ? min(qr, p.Sq - 1) : qr);
@@ -1296,10 +1295,46 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 3 : 1) attn_
     }
   };
 
-  if (total > 0) {
-    load_tile(0, 0);
-    store_tile(0, 0);
+  if (total > 0) {  // (flies with the key and value rows)
+    aim_tile(0, 0);
+#pragma unroll
+    for (int j = 0; j < 2 * CPT; ++j) stg.load_one(j, sq, sg, soq, sog);
   }
+  const bf16_t* kp = p.k + b * p.k_sb + hk * p.k_sh;
+  const bf16_t* vp = p.v + b * p.v_sb + hk * p.v_sh;
+  bf16x8 kf[KSD];
+#pragma unroll
+  for (int s = 0; s < KSD; ++s) {
+    kf[s] = *reinterpret_cast<const bf16x8*>(kp + (long long)(G ? min(key, p.Sk - 1) : key) * p.k_st + 16 * s + 8 * hh);
+    if (G && key >= kv_end) kf[s] = bf16x8{};
+  }
+  // this wave's 32 V rows -> its own image (read back by rows for dP; pad chunks zero)
+  char* vimg = smem + VOFF + wave * TILE;
+  u32x4 vr[32 * NCH / 64];
+#pragma unroll
+  for (int i = 0; i < 32 * NCH / 64; ++i) {
+    const int idx = lane + 64 * i, row = idx / NCH, ch = idx % NCH;
+    vr[i] = *reinterpret_cast<const u32x4*>(vp + (long long)(G ? min(kw + row, p.Sk - 1) : kw + row) * p.v_st + min(ch, NCS - 1) * 8);
+  }
+#pragma unroll
+  for (int i = 0; i < 32 * NCH / 64; ++i) {
+    const int idx = lane + 64 * i, row = idx / NCH, ch = idx % NCH;
+    *reinterpret_cast<u32x4*>(vimg + img_off<D>(row, ch)) = ch < NCS && (!G || kw + row < kv_end) ? vr[i] : u32x4{0, 0, 0, 0};
+  }
+  if constexpr (DS < D) {  // Q / dO image chunks DS/8.. are never loaded: zero them in both buffers once
+    constexpr int PC = NCH - NCS, NZ = 2 * 2 * 32 * PC;
+    for (int i = tid; i < NZ; i += 256) {
+      const int img = i / (32 * PC), row = (i / PC) % 32, ch = NCS + i % PC;
+      *reinterpret_cast<u32x4*>(smem + img * TILE + img_off<D>(row, ch)) = u32x4{0, 0, 0, 0};
+    }
+  }
+  f32x16 dk[D / 32], dv[D / 32];
+#pragma unroll
+  for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) { dk[i][r] = 0.f; dv[i][r] = 0.f; }
+
+  if (total > 0) store_tile(0, 0);
   __syncthreads();
   ASTAMP(0);
   auto tile_step = [&](int it, auto masked) {
@@ -1309,7 +1344,11 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 3 : 1) attn_
     const char* Gs = Qs + TILE;
     const float* ls = reinterpret_cast<const float*>(smem + LOFF) + (it & 1) * 64;
     if (it + 1 < total && ++qcur == nqt) qcur = 0, ++hcur;  // (the last step loads its own tile again)
-    load_tile(hcur, qcur);
+    aim_tile(hcur, qcur);
+    if constexpr (!SPREAD) {
+#pragma unroll
+      for (int j = 0; j < 2 * CPT; ++j) stg.load_one(j, sq, sg, soq, sog);
+    }
     asm volatile("" ::: "memory");
     ASTAMP(1);
     // No skip of the (at most 3 per head) q tiles that lie wholly above this
@@ -1340,6 +1379,10 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 3 : 1) attn_
           ng = row_frag<D>(Gs, be, bo, s + 1);
           nv = row_frag<D>(vimg, be, bo, s + 1);
           __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+        }
+        if (SPREAD && s < 2 * CPT) {
+          stg.load_one(s, sq, sg, soq, sog);
+          __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);
         }
         sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cq, kf[s], sacc, 0, 0, 0);
         dpacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cg, cv, dpacc, 0, 0, 0);
