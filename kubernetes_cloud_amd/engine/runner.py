@@ -682,7 +682,7 @@ class ModelRunner(StepRunner):
         # run without their padding (_prefill_packed)
         self._append_ok = (on_gpu and self.dtype in (torch.bfloat16, torch.float16) and not self.multi_device
                            and self.D % 8 == 0 and self.D <= 256)
-        self._packed_ok = self._append_ok and self.dtype == torch.bfloat16
+        self._packed_ok = self._append_ok
         # parallel-residual models (GPT-J, NeoX): the MLP branch does not depend on attention, so at
         # decode its two weight-streaming GEMVs run on a side stream while the latency-bound attention
         # chain (split-K attention, combine, out-proj) runs on the main one -- both captured into the

@@ -19,6 +19,7 @@ import sys
 import threading
 
 import torch
+from torch.autograd import forward_ad
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_DIR = os.path.join(os.path.dirname(_HERE), "_lib")
@@ -68,7 +69,7 @@ _SIGS = {
     "kca_clip_coef": [P, F, F, P, P, P, P],
     "kca_attn_fwd": [P] * 5 + [LL] * 12 + [I] * 7 + [F, P, P, I, P, I, I, P, P],
     "kca_attn_bwd": [P] * 10 + [LL] * 24 + [I] * 7 + [F, P, P, I, P, P],
-    "kca_attn_fwd_packed": [P] * 4 + [LL] * 8 + [I] * 6 + [F, P, I, P, P, P],
+    "kca_attn_fwd_packed": [I] + [P] * 4 + [LL] * 8 + [I] * 6 + [F, P, I, P, P, P],
     "kca_rope_append": [I, P, P, P] + [LL] * 6 + [I] * 6 + [P] * 7 + [I, P],
     "kca_attn_fwd_wide": [P] * 5 + [LL] * 12 + [I] * 6 + [F, P, P],
     "kca_attn_set_tiled": [I],
@@ -266,6 +267,25 @@ def counters(device: torch.device, n: int) -> torch.Tensor:
 
 def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
+
+
+def inference(*tensors: torch.Tensor | None) -> bool:
+    """An eager call without gradients, tangents, transforms, tracing or autocast, on plain tensors of the current device:
+    it may go to a kernel that autograd knows nothing of."""
+    if (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or torch._C._are_functorch_transforms_active()
+            or forward_ad._current_level >= 0 or torch.jit.is_tracing() or torch.compiler.is_compiling()):
+        return False
+    dev = None
+    for t in tensors:
+        if t is None:
+            continue
+        if not t.is_cuda or type(t) not in (torch.Tensor, torch.nn.Parameter):
+            return False
+        if dev is None:
+            dev = torch.cuda.current_device()
+        if t.get_device() != dev:
+            return False
+    return True
 
 
 def native_f16(*tensors: torch.Tensor | None) -> bool:

@@ -133,11 +133,11 @@ def _bwd(q, k, v, o, do, lse, dq, dk, dv, causal, scale, kv_len, alibi, window: 
               int(window), _lib.ptr(_masks(kv_len)[1]), _lib.stream())
 
 
-def _check(q, k, v):
+def _check(q, k, v, dtype=torch.bfloat16):
     for t in (q, k, v):
         if t.dim() != 4 or t.stride(-1) != 1:
             raise ValueError("attention expects [B, S, H, D] views with unit last stride")
-        if t.dtype != torch.bfloat16:
+        if t.dtype != dtype:
             raise ValueError("native attention is bf16")
     D = q.shape[-1]
     if D % 8 or D > 256:
@@ -204,18 +204,20 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: b
 def packed_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu: torch.Tensor, max_len: int,
                      scale: float | None = None, alibi: torch.Tensor | None = None, window: int = 0) -> torch.Tensor:
     """Causal self-attention of sequences that lie one after another in [T, H, D] rows (inference): sequence i is rows
-    ``cu[i]`` .. ``cu[i + 1]`` (int32, on the device), none longer than ``max_len``."""
+    ``cu[i]`` .. ``cu[i + 1]`` (int32, on the device), none longer than ``max_len``. bf16, or fp16 with softmax weights of 22
+    bits."""
     T, H, D = q.shape
-    _check(*(t.unsqueeze(0) for t in (q, k, v)))
+    f16 = q.dtype == torch.float16
+    _check(*(t.unsqueeze(0) for t in (q, k, v)), dtype=torch.float16 if f16 else torch.bfloat16)
     n = cu.shape[0] - 1
     o = torch.empty(T, H, D, device=q.device, dtype=q.dtype)
-    flags = torch.empty(4 * ((max_len + 127) // 128) * n * H, device=q.device, dtype=torch.int32)
+    flags = None if f16 else torch.empty(4 * ((max_len + 127) // 128) * n * H, device=q.device, dtype=torch.int32)
     scale = scale if scale is not None else 1.0 / math.sqrt(D)
     if alibi is not None:
         alibi = alibi.to(device=q.device, dtype=torch.float32).contiguous()
-    _lib.call("kca_attn_fwd_packed", q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), q.stride(0), q.stride(1),
+    _lib.call("kca_attn_fwd_packed", 2 if f16 else 1, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), q.stride(0), q.stride(1),
               k.stride(0), k.stride(1), v.stride(0), v.stride(1), o.stride(0), o.stride(1), n, max_len, H, k.shape[1], D,
-              1, float(scale), _lib.ptr(alibi), int(window), cu.data_ptr(), flags.data_ptr(), _lib.stream())
+              1, float(scale), _lib.ptr(alibi), int(window), cu.data_ptr(), _lib.ptr(flags), _lib.stream())
     return o
 
 

@@ -16,7 +16,6 @@ import math
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
-from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -196,10 +195,6 @@ def _rows_mm(x2: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) 
     return y
 
 
-def _like(t: torch.Tensor, x: torch.Tensor) -> bool:
-    return t.dtype == x.dtype and t.device == x.device and type(t) in (torch.Tensor, nn.Parameter)
-
-
 def linear_rows(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     """``F.linear`` without gradients: up to FEW_ROWS rows on the weight-streaming kernel, more in one product or two
     (``wave_rows``). ``F.linear`` itself for all else (a gradient or a tangent recorded, a transform or autocast at work,
@@ -213,11 +208,8 @@ def linear_rows(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None
     # Past 128 rows it is faster everywhere (the blocks would be half as wide: 200 rows of 12288 x 4096 39.9 : 52.5)
     few = rows <= (FEW_ROWS if n <= 64 * _CUS else 24)
     first = rows if few else wave_rows(rows, n, k)
-    if ((first == rows and not few) or not x.is_contiguous() or type(x) is not torch.Tensor
-            or (bias is not None and bias.shape != (n,))
-            or not _like(weight, x) or not (bias is None or _like(bias, x)) or x.get_device() != torch.cuda.current_device()
-            or torch.is_autocast_enabled("cuda") or torch._C._are_functorch_transforms_active()
-            or forward_ad._current_level >= 0 or torch.jit.is_tracing() or torch.compiler.is_compiling()):
+    if ((first == rows and not few) or not x.is_contiguous() or weight.dtype != x.dtype
+            or (bias is not None and (bias.shape != (n,) or bias.dtype != x.dtype)) or not _lib.inference(x, weight, bias)):
         return F.linear(x, weight, bias)
     x2 = x.view(rows, k)
     if few:

@@ -64,6 +64,13 @@ class _LayerNormFn(torch.autograd.Function):
         return dx, dw, db, None, g1, g2
 
 
+def _rows_f16(x, weight, bias, residual) -> bool:
+    d = x.shape[-1]
+    return (_lib.native_f16(x, weight, bias, *residual) and d % 8 == 0 and 0 < d <= 16384 and x.numel() > 0
+            and weight.shape == (d,) and (bias is None or bias.shape == (d,)) and all(r.shape == x.shape for r in residual)
+            and all(t is None or (t.is_contiguous() and t.data_ptr() % 16 == 0) for t in (x, weight, bias, *residual)))
+
+
 def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
                eps: float = 1e-5, residual: tuple = ()):
     """LayerNorm over the last dim, optionally of ``x + sum(residual)``.
@@ -78,6 +85,14 @@ def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
     if _lib.use_native(x):
         y, h = _LayerNormFn.apply(x, weight, bias, eps, r1, r2)
         return (y, h) if residual else y
+    if (weight is not None and _lib.native_f16(x) and _lib.inference(x, weight, bias, *residual)
+            and _rows_f16(x, weight, bias, residual)):
+        # fp16 inference: the decode steps' rows kernel (eager it is a pass to fp32 and back around torch's kernel, after a
+        # rounded pass a residual: 5400 x 4096 with two residuals 260 us, here 31)
+        from .gemv import ln_rows
+        d = x.shape[-1]
+        y, h = ln_rows(x.reshape(-1, d), weight, bias, eps, tuple(r.reshape(-1, d) for r in residual))
+        return (y.view(x.shape), h.view(x.shape)) if residual else y.view(x.shape)
     h = x
     for r in residual:
         h = h + r
