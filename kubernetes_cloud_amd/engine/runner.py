@@ -678,11 +678,10 @@ class ModelRunner(StepRunner):
             tunable.ensure(tunable.DECODE_FILE)
         if self.multi_device:
             self.use_graphs = False  # one graph cannot span devices; the split path runs eagerly
-        # prompts' rotation and page writes in one launch a layer (what ops.rope_append takes); new bf16 prompts also
+        # prompts' rotation and page writes in one launch a layer (what ops.rope_append takes); new prompts also
         # run without their padding (_prefill_packed)
         self._append_ok = (on_gpu and self.dtype in (torch.bfloat16, torch.float16) and not self.multi_device
                            and self.D % 8 == 0 and self.D <= 256)
-        self._packed_ok = self._append_ok
         # parallel-residual models (GPT-J, NeoX): the MLP branch does not depend on attention, so at
         # decode its two weight-streaming GEMVs run on a side stream while the latency-bound attention
         # chain (split-K attention, combine, out-proj) runs on the main one -- both captured into the
@@ -787,7 +786,7 @@ class ModelRunner(StepRunner):
                 self.cache.release(s_)  # a reused slot starts empty
             self.cache.reserve(s_, p0 + L)
         self.cache.sync()
-        if self._packed_ok and not cont and len(set(slots)) == n:
+        if self._append_ok and not cont and len(set(slots)) == n:
             return self._prefill_packed(ids, slots, lens)
         ids = ids.to(self.device)
         plan = where = None

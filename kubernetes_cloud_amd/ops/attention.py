@@ -64,10 +64,10 @@ def attention_reference(q, k, v, causal: bool, scale: float | None = None,
 
 
 def set_tiled_path(enable: bool) -> None:
-    """Toggle the full-tile fast kernels (csrc/kernels/attention_tiled.hip) used
-    for head_dim 128/256 when Sq % 128 == 0 and Sk % 32 (fwd) / 128 (bwd) == 0
-    and there is no ALiBi / key-length mask. On by default; off forces the
-    generic kernels (A/B measurement, tests)."""
+    """Toggle the tiled kernels (csrc/kernels/attention_tiled.hip): head sizes 64, 96, 128, 160 and 256 with 16-byte rows,
+    any lengths, key lengths and windows, ALiBi with a causal mask; head sizes between, key bitmaps and causal calls
+    with fewer keys than queries run the generic kernels. On by default; off forces the generic kernels (A/B measurement,
+    tests)."""
     _lib.call("kca_attn_set_tiled", int(bool(enable)))
 
 
