@@ -33,7 +33,8 @@ def gelu(u: torch.Tensor, approximate: str = "tanh") -> torch.Tensor:
     approx = approximate == "tanh"
     if _lib.use_native(u) and u.numel() % 8 == 0:
         return _GeluFn.apply(u, approx)
-    if _lib.native_f16(u) and _lib.inference(u) and u.numel() and u.numel() % 8 == 0 and u.is_contiguous() and u.data_ptr() % 16 == 0:
+    if (_lib.native_f16(u) and _lib.inference(u) and u.numel() and u.numel() % 8 == 0 and u.is_contiguous()
+            and u.data_ptr() % 16 == 0 and _lib.has("kca_gelu_fwd_f16")):
         y = torch.empty_like(u)  # (fp16 inference: the decode steps' kernel)
         _lib.call("kca_gelu_fwd_f16", u.data_ptr(), y.data_ptr(), u.numel(), int(approx), _lib.stream())
         return y

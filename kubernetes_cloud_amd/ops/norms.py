@@ -66,7 +66,7 @@ class _LayerNormFn(torch.autograd.Function):
 
 def _rows_f16(x, weight, bias, residual) -> bool:
     d = x.shape[-1]
-    return (_lib.native_f16(x, weight, bias, *residual) and d % 8 == 0 and 0 < d <= 16384 and x.numel() > 0
+    return (_lib.has("kca_ln_rows_f16") and _lib.native_f16(x, weight, bias, *residual) and d % 8 == 0 and 0 < d <= 16384 and x.numel() > 0
             and weight.shape == (d,) and (bias is None or bias.shape == (d,)) and all(r.shape == x.shape for r in residual)
             and all(t is None or (t.is_contiguous() and t.data_ptr() % 16 == 0) for t in (x, weight, bias, *residual)))
 
