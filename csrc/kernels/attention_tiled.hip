@@ -351,8 +351,9 @@ __device__ __forceinline__ void store_tile_lds(bf16_t* row0, long long st, const
 // G > 0 walks the tiles from the last to the first: every row's last visible key -- with ALiBi the one with the
 // least bias, with a window or a length one that surely exists -- then lies in one of the first, masked tiles,
 // whose row max is the reference (below).
+// (two waves a SIMD to D = 160, which spills 0 to 9 registers for it: 4 x 4096 x 8 238 -> 226 us)
 template <int D, bool CAUSAL, int OC = -1, int DS = D, int MC = -1, int G = 0>
-__global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1)) attn_fwd_tiled_kernel(FastFwdParams p) {
+__global__ void __launch_bounds__(256, (D <= 160 ? 2 : 1)) attn_fwd_tiled_kernel(FastFwdParams p) {
   static_assert(G == 0 || (OC < 0 && MC < 0 && DS == D && D < 256), "general form: plain heads");
   constexpr int BM = 128, BN = 32;
   constexpr int TILE = BN * D * 2;           // bytes per K or V tile (LDS image)
@@ -1040,8 +1041,10 @@ __device__ __forceinline__ void store_acc_t(bf16_t* rowp, const f32x16 (&acc)[D 
 // steps, the dQ (dK, dV) tiles are stored DS wide.
 // 64-wide heads without a causal mask (SD): registers capped for 4 waves per SIMD instead of 3 (a 16-byte
 // spill in the 48-wide form; DreamBooth +1.5-2.8 % same box, profiles/decode_launch_structure_ab_r5.txt)
+// (other forms: 3 waves at D = 64, without a spill; 2 at 96 and 128; at D = 160 two waves spill 15 registers, 4 x 1000 x 8
+// 103 -> 115 us for the backward)
 template <int D, bool CAUSAL, int DS = D, int G = 0>
-__global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 4 : 1) attn_bwd_dq_tiled_kernel(FastBwdParams p) {
+__global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 4 : D <= 64 ? 3 : D <= 128 ? 2 : 1) attn_bwd_dq_tiled_kernel(FastBwdParams p) {
   constexpr int BM = 128, BN = 32;
   constexpr int TILE = BN * D * 2;
   using Stg = StagerFor<D, DS>;
@@ -1223,11 +1226,13 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 4 : 1) attn_
   ASTAMP_FLUSH(16);
 }
 
-// 64-wide heads without a causal mask (SD-1.5's 40-wide heads in narrow storage): registers capped for
-// 3 waves per SIMD (165 VGPRs, no spill) instead of 2 -- DreamBooth 61.1 -> 62.3 samples/s same box
-// (the causal D = 64 form spills at that cap and keeps 2)
+// Registers capped for 3 waves a SIMD at D = 64 and 2 at 96 and 128: a wave waits for its loads, its barrier and its own
+// softmax, and what another wave computes meanwhile is worth more than the 2 to 15 registers spilled, or, at D = 96, the
+// accumulators' copies out of the upper half of the file. Backward (with dQ's caps), us, without and with:
+// 8 x 1024 x 12 of 64 123 -> 92, 8 x 1000 with lengths 136 -> 102, 1500 x 64 of 96 211 -> 187, 2 x 2048 x 20 of 128 276 -> 231, 2048 x
+// 14 of 128 with ALiBi 168 -> 157. D = 160 and 256 take more than half of the file.
 template <int D, bool CAUSAL, int DS = D, int G = 0>
-__global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 3 : 1) attn_bwd_dkdv_tiled_kernel(FastBwdParams p) {
+__global__ void __launch_bounds__(256, D <= 64 ? 3 : D <= 128 ? 2 : 1) attn_bwd_dkdv_tiled_kernel(FastBwdParams p) {
   constexpr int BK = 128, BQ = 32;
   constexpr int TILE = BQ * D * 2;                  // one 32-row image
   using Stg = StagerFor<D, DS>;
@@ -1460,7 +1465,7 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 3 : 1) attn_
   // splitting into masked / mask-free bodies -- by a per-tile branch or by
   // two loops per head -- pushed the 256 dK/dV accumulators into spills.
   for (int it = 0; it < total; ++it) tile_step(it, std::integral_constant<bool, (CAUSAL || G > 0)>{});
-  if constexpr (D == 96) {  // the LDS staging's registers push this one past 256 (2 -> 1 wave per SIMD)
+  if constexpr (D == 96) {  // (the LDS staging took this one past 256 registers)
     if (!G || key < p.Sk) {
       store_acc_t<D>(p.dk + b * p.dk_sb + hk * p.dk_sh + (long long)key * p.dk_st, dk, hh, p.scale);
       store_acc_t<D>(p.dv + b * p.dv_sb + hk * p.dv_sh + (long long)key * p.dv_st, dv, hh, 1.f);
