@@ -1240,7 +1240,8 @@ __global__ void __launch_bounds__(256, D <= 64 ? 3 : D <= 128 ? 2 : 1) attn_bwd_
   constexpr int KSD = DS / 16;                      // contraction steps over the stored columns
   // The next tile's loads, together before the products or one a step among the first ones. Together they hold the
   // wave, alone on its SIMD, up for 700 of a tile's 5000 cycles at D = 256 (backward of 2 x 2048 x 16 heads 411 -> 394 us); at
-  // smaller D a tile is short and the time that they fly is what counts (dK/dV, D = 64: 88 us together, 91 spread; 128: 114, 116).
+  // smaller D a tile is short and the time that they fly is what counts (backward of 6 x 1000 x 20 heads of 128: 216 us together,
+  // 224 spread; 8 x 1000 x 12 of 64: 98, 99).
   constexpr bool SPREAD = D == 256;
   constexpr int VOFF = 4 * TILE;                    // V images of the 4 waves
   constexpr int LOFF = VOFF + 4 * TILE;             // lse/delta: [buf][64] floats
