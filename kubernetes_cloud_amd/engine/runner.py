@@ -37,6 +37,7 @@ from ..ops import decode as dops
 from ..ops import _lib
 from ..ops import skinny_mm as smm
 from ..ops.gemv import embed_ln_rows, ln_rows, ln_skinny_linear, skinny_linear
+from ..utils import capture
 
 # decode steps: each row's RoPE angles and page-table row travel with the step's packed inputs (fixed
 # device addresses), so every layer's attention chain loads them in its first memory round trip
@@ -621,10 +622,7 @@ class StepRunner:
         if self._pool is None:
             self._pool = torch.cuda.graph_pool_handle()
         g = torch.cuda.CUDAGraph()
-        # thread-local capture: the RCCL process-group watchdog thread polls its work events while a
-        # capture runs; under the default global mode that query fails ("operation not permitted when
-        # stream is capturing") and the watchdog aborts the process
-        with torch.cuda.graph(g, pool=self._pool, stream=s, capture_error_mode="thread_local"):
+        with capture.graph(g, pool=self._pool, stream=s):
             self._step_body(st, Bb, Kb, mc)
         self._graphs[(Bb, Kb, mc)] = g
         return g

@@ -20,6 +20,7 @@ import os
 
 import torch
 
+from ..utils import capture
 from .clip_text import CLIPTextConfig, CLIPTextModel
 from .schedulers import load_scheduler, sd_scheduler_config
 from .unet import UNet2DConditionModel, UNetConfig, to_channels_last
@@ -125,7 +126,7 @@ class UNetGraph:
                     self.unet(sx, st, sc)
             torch.cuda.current_stream().wait_stream(side)
             graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(graph, capture_error_mode="thread_local"):  # see engine/runner.py _capture
+            with capture.graph(graph):
                 out = self.unet(sx, st, sc)
             from .unet import pad_generation
             self.pad_gen = pad_generation()

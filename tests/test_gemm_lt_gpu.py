@@ -5,6 +5,7 @@ import torch
 
 from kubernetes_cloud_amd.ops import _lib
 from kubernetes_cloud_amd.ops.linear import linear_residual
+from kubernetes_cloud_amd.utils import capture
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -50,7 +51,7 @@ def test_linear_residual_channels_last_view_and_graph():
         s = torch.cuda.Stream()
         s.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(s):
-            with torch.cuda.graph(g):
+            with capture.graph(g):
                 og = linear_residual(t, w, b, res.permute(0, 2, 3, 1))
         torch.cuda.current_stream().wait_stream(s)
         res.mul_(2)  # replay reads the live residual

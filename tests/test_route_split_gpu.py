@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from kubernetes_cloud_amd.ops import moe
+from kubernetes_cloud_amd.utils import capture
 
 pytestmark = pytest.mark.gpu
 
@@ -65,7 +66,7 @@ def test_streams_and_captures(monkeypatch):
     torch.cuda.synchronize()
     assert all(torch.equal(i, ids0) and torch.equal(w, w0) for i, w in outs)
     graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph, stream=streams[0]):
+    with capture.graph(graph, stream=streams[0]):
         ids, w, _, _ = moe.route_group(*a)
     for _ in range(3):
         ids.zero_()

@@ -5,6 +5,7 @@ import torch.nn.functional as F
 
 from kubernetes_cloud_amd.ops import _lib
 from kubernetes_cloud_amd.ops.linear import _k_slices, _rows_mm, linear_rows
+from kubernetes_cloud_amd.utils import capture
 
 pytestmark = pytest.mark.gpu
 
@@ -52,7 +53,7 @@ def test_slices_under_capture_and_on_streams(rows, n, k):
         assert all(torch.equal(o, outs[0]) for o in outs) and _close(outs[0], ref)
         for s in (main, torch.cuda.Stream()):  # a stream with a workspace, and one that has none yet
             graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(graph, stream=s):
+            with capture.graph(graph, stream=s):
                 y = linear_rows(x, w, b)
             for _ in range(3):
                 y.zero_()

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from kubernetes_cloud_amd.ops import skinny_mm as sm
+from kubernetes_cloud_amd.utils import capture
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -242,7 +243,7 @@ def test_split_counters_live_outside_a_graphs_pool():
         pool, graphs, outs = torch.cuda.graph_pool_handle(), [], []
         for i in range(3):
             graphs.append(torch.cuda.CUDAGraph())
-            with torch.cuda.graph(graphs[-1], pool=pool, stream=s):
+            with capture.graph(graphs[-1], pool=pool, stream=s):
                 noise = [torch.full((n,), 7.0, device=DEV) for n in (64, 4096, 1 << 20)] if i != 1 else []
                 outs.append(sm.mm(x, w))
                 del noise
