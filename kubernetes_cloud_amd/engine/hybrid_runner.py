@@ -20,6 +20,8 @@ its start, because a portion's first and last rows are handled by different work
 """
 from __future__ import annotations
 
+import weakref
+
 import numpy as np
 import torch
 import torch.nn.functional as F
@@ -69,9 +71,13 @@ class HybridRunner(StepRunner):
             raise ValueError("these layers need the paged cache (page_size >= 16)")
         if self.dtype == torch.float32 and self.device.type == "cuda":
             torch.backends.cuda.matmul.allow_tf32 = False
+        # (the mixers' way back is weak, and no bound method is kept: a runner in a cycle would hold its cache, graphs and
+        # pinned buffers until a collection)
+        me = weakref.ref(self)
+        linear = lambda *args, **kw: me()._linear(*args, **kw)  # noqa: E731
         self.mixers, first = [], {}  # one per layer run
         for r, i in enumerate(cfg.runs):
-            self.mixers.append(make_mixer(model.layers[i], cfg, r, self._linear, first.get(i)))
+            self.mixers.append(make_mixer(model.layers[i], cfg, r, linear, first.get(i)))
             first.setdefault(i, self.mixers[-1])
         shapes, widths = [], {"shift": (len(cfg.runs), d)} if cfg.block == "parallel" else {}
         members = [m for mx in self.mixers for m in mx.members()]
@@ -85,8 +91,8 @@ class HybridRunner(StepRunner):
         for mx in members:
             mx.cache, mx.state = self.cache, self.state
         self._members = members
-        self._forward_layers = {"parallel": self._parallel, "sandwich": self._sandwich, "prenorm": self._prenorm,
-                                "postnorm": self._postnorm}[cfg.block]
+        self._forward_layers = {"parallel": HybridRunner._parallel, "sandwich": HybridRunner._sandwich,
+                                "prenorm": HybridRunner._prenorm, "postnorm": HybridRunner._postnorm}[cfg.block]
         self._rules = [None if not isinstance(L.spec.mlp, MoESpec) else moe.Router(
             L.spec.mlp.score == "softmax", L.correction.float() if L.spec.mlp.correction else None, L.spec.mlp.groups,
             L.spec.mlp.keep, L.spec.mlp.identity) for L in model.layers]
@@ -150,7 +156,7 @@ class HybridRunner(StepRunner):
     def _forward(self, b: _Batch, want: torch.Tensor | None, layers_out: list | None = None) -> torch.Tensor:
         """Logits of the rows in ``want`` (None: every row). ``layers_out`` collects the residual stream after
         every layer run."""
-        logits = self._linear(self._forward_layers(b, want, layers_out), self.model.head_weight)
+        logits = self._linear(self._forward_layers(self, b, want, layers_out), self.model.head_weight)
         cap = self.cfg.logit_softcap
         return moe.act_rows(logits, logits, False, act="softcap", cap=cap) if cap else logits
 

@@ -95,3 +95,25 @@ def test_a_collector_that_is_off_stays_off():
         assert not gc.isenabled()
     finally:
         gc.enable()
+
+
+@pytest.mark.parametrize("family", ["megusun", "rezusun", "begopel", "gibipel"])
+def test_runners_go_with_their_last_reference(family):
+    """No cycle holds a runner's cache, graphs and pinned buffers until a collection."""
+    import importlib
+    import weakref
+
+    from kubernetes_cloud_amd.engine.llm_engine import LLMEngine, SamplingParams
+    t = importlib.import_module("tests.test_" + family)
+    for name in t.CFGS:
+        m = t.make(t.CFGS[name] if family == "megusun" else name, "cpu", torch.float32)[0]
+        gc.collect()
+        gc.disable()
+        try:
+            e = LLMEngine(m, max_slots=2, max_len=64)
+            e.generate([[1, 2, 3]], SamplingParams(max_new_tokens=3, do_sample=False))
+            left = weakref.ref(e.runner)
+            del e
+            assert left() is None, name
+        finally:
+            gc.enable()
