@@ -247,7 +247,7 @@ KCA_API int kca_rows_mm(int dtype, const void* x, const void* w, const void* bia
       ks > K / SK)
     return 1;
   if (!al16(x) || !al16(w) || (uintptr_t)y % 8) return 2;
-  if (2ll * N * K >= 1ll << 32) return 3;  // (32-bit byte offsets)
+  if (2ll * (N > M ? N : M) * K >= 1ll << 32) return 3;  // (32-bit byte offsets into W and x)
   const long long blocks = (N + NB - 1) / NB, xr = M <= 32 ? 32 : M <= 64 ? 64 : 128;
   if (blocks * ks >= 1ll << 31) return 3;
   if (ks > 1 && (!ws || !cnt || !al16(ws) || ws_floats < blocks * ks * NB * xr || cnt_n < blocks)) return 6;

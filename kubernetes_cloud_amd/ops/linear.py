@@ -180,7 +180,7 @@ def _rows_mm(x2: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) 
     """The product of up to FEW_ROWS rows on the weight-streaming kernel; None: sizes or alignment it does not take."""
     rows, k = x2.shape
     n = weight.shape[0]
-    if (n % 16 or k % 64 or k == 0 or 2 * n * k >= 1 << 32 or not weight.is_contiguous() or x2.data_ptr() % 16
+    if (n % 16 or k % 64 or k == 0 or 2 * max(n, rows) * k >= 1 << 32 or not weight.is_contiguous() or x2.data_ptr() % 16
             or weight.data_ptr() % 16 or (bias is not None and not bias.is_contiguous()) or not _lib.has("kca_rows_mm")):
         return None
     ks, ws, cnt = _k_slices(n, k), None, None
