@@ -15,7 +15,7 @@ def test_parts_cover_the_rows(n, k):
         if first < rows:
             assert rows > 2048 and k >= 2048
             blocks = first // 256 * -(-n // 256)
-            assert first % 256 == 0 and (blocks % 256 == 0 or 1536 < rows - first)
+            assert first % 256 == 0 and blocks % 256 == 0 and not 1536 < rows - first < 2048
 
 
 def test_other_calls_stay_one_product(monkeypatch):
