@@ -730,8 +730,9 @@ __global__ void __launch_bounds__(256, 2) expert_stream_kernel(ExpertArgs p) {
 // 16 experts of 3 x 4096 x 2048, top 3: 764 -> 541; 1000 tokens, 32 experts of 3 x 2048 x 1024, top 4: 148 -> 116.
 constexpr int GBK = 64, GN = 256, GM = 256, GEMM_LDS = 2 * (GN + GM) * GBK * 2;
 
-// WN x WM waves, each with AI runs of 32 weight rows and BJ of 32 rows
-template <bool UP, int WN, int AI, int WM, int BJ>
+// WN x WM waves, each with AI runs of 32 weight rows and BJ of 32 rows. FAR: addresses of 64 bits, for activations or an expert's
+// weights that 32-bit byte offsets do not span
+template <bool UP, int WN, int AI, int WM, int BJ, bool FAR = false>
 __device__ __forceinline__ void expert_gemm_tile(const ExpertArgs& p, bf16_t* gl, int ex, int lo, int nr, int n0) {
   constexpr int WP = WN * AI, RP = WM * BJ, NP = WP + RP;  // staging passes of 32 rows: weights, activations
   constexpr int STG = NP * 32 * GBK;                       // one stage (elements)
@@ -741,10 +742,11 @@ __device__ __forceinline__ void expert_gemm_tile(const ExpertArgs& p, bf16_t* gl
   const int K = p.K, N = p.N;
   // staging: thread tid owns the 16-byte piece tid % 8 of rows tid / 8 + 32 i
   const int ch = tid & 7, sr = tid >> 3;
-  const __amdgpu_buffer_rsrc_t rw =
-      uniform_rsrc(reinterpret_cast<const bf16_t*>(p.w) + (long long)ex * (UP ? 2 * N : N) * K);
+  const bf16_t* wb = reinterpret_cast<const bf16_t*>(p.w) + (long long)ex * (UP ? 2 * N : N) * K;
+  const bf16_t* xb = reinterpret_cast<const bf16_t*>(p.x) + (UP ? 0ll : (long long)lo * K);
   constexpr unsigned OUT = 1u << 31;  // past the activations: a stage past K multiplies zeros
-  const __amdgpu_buffer_rsrc_t rx = uniform_rsrc(reinterpret_cast<const bf16_t*>(p.x) + (UP ? 0ll : (long long)lo * K), OUT);
+  const __amdgpu_buffer_rsrc_t rw = uniform_rsrc(wb), rx = uniform_rsrc(xb, OUT);
+  const unsigned rb = FAR ? 1u : (unsigned)K * 2;  // FAR: wo and xo are row numbers
   unsigned wo[WP], xo[RP];
 #pragma unroll
   for (int i = 0; i < WP; ++i) {
@@ -752,17 +754,23 @@ __device__ __forceinline__ void expert_gemm_tile(const ExpertArgs& p, bf16_t* gl
     // (up: a wave's rows are AI / 2 runs of 32 gate rows, then the same up rows)
     const int run = r / 32, wrun = run % AI, base = run / AI * (AI / 2) * 32;
     const int n = UP ? (wrun < AI / 2 ? 0 : N) + min(n0 + base + wrun % (AI / 2) * 32 + (r & 31), N - 1) : min(n0 + r, N - 1);
-    wo[i] = (unsigned)n * K * 2;
+    wo[i] = (unsigned)n * rb;
   }
 #pragma unroll
   for (int i = 0; i < RP; ++i) {
     const int xr = min(sr + 32 * i, nr - 1);
-    xo[i] = (unsigned)(UP ? p.perm[lo + xr] / p.top : xr) * K * 2;
+    xo[i] = (unsigned)(UP ? p.perm[lo + xr] / p.top : xr) * rb;
   }
   u32x4 ra[2][NP];
   const int so = sr * GBK + ((ch ^ ((sr >> 1) & 7)) << 3);  // 16 rows x one piece cover all 64 banks
   auto load = [&](int t, int i, u32x4 (&r)[NP]) {
     const int k = t * GBK + ch * 8;
+    if constexpr (FAR) {
+      const bf16_t* row = i < WP ? wb + (long long)wo[i < WP ? i : 0] * K : xb + (long long)xo[i < WP ? 0 : i - WP] * K;
+      const unsigned keep = i < WP || k < K ? ~0u : 0u;
+      r[i] = *reinterpret_cast<const u32x4*>(row + min(k, K - 8)) & u32x4{keep, keep, keep, keep};
+      return;
+    }
     const unsigned kw = min(k, K - 8) * 2, kx = k < K ? k * 2 : OUT;
     const auto v = i < WP ? __builtin_amdgcn_raw_buffer_load_b128(rw, wo[i < WP ? i : 0] + kw, 0, 0)
                           : __builtin_amdgcn_raw_buffer_load_b128(rx, xo[i < WP ? 0 : i - WP] + kx, 0, 0);
@@ -876,8 +884,8 @@ __device__ __forceinline__ void expert_gemm_tile(const ExpertArgs& p, bf16_t* gl
   }
 }
 
-// NARROW: tiles of up to 192 rows x 128 weight rows
-template <bool UP, bool NARROW>
+// NARROW: tiles of up to 192 rows x 128 weight rows (FAR: 128 rows)
+template <bool UP, bool NARROW, bool FAR = false>
 __global__ void __launch_bounds__(256, NARROW ? 2 : 1) expert_gemm_kernel(ExpertArgs p) {
   extern __shared__ __attribute__((aligned(16))) bf16_t gl[];  // [2][weight rows, then activation rows][GBK]
   // order: an XCD works a contiguous run of (expert, weight block, row tile), so the row tiles that share a
@@ -890,7 +898,9 @@ __global__ void __launch_bounds__(256, NARROW ? 2 : 1) expert_gemm_kernel(Expert
   const int in = id - t0[3] * nb, tile = t0[3] + in % t0[4], bn = in / t0[4];
   const int* tl = p.tiles + tile * 5;
   const int nr = tl[2], n0 = bn * NB;
-  if constexpr (NARROW) {
+  if constexpr (FAR) {
+    expert_gemm_tile<UP, 2, 2, 2, 2, true>(p, gl, tl[0], tl[1], nr, n0);
+  } else if constexpr (NARROW) {
     if (nr > 128) expert_gemm_tile<UP, 2, 2, 2, 3>(p, gl, tl[0], tl[1], nr, n0);
     else if (nr > 64) expert_gemm_tile<UP, 2, 2, 2, 2>(p, gl, tl[0], tl[1], nr, n0);
     else expert_gemm_tile<UP, 2, 2, 2, 1>(p, gl, tl[0], tl[1], nr, n0);
@@ -904,10 +914,10 @@ __global__ void __launch_bounds__(256, NARROW ? 2 : 1) expert_gemm_kernel(Expert
   }
 }
 
-template <bool UP, bool NARROW>
+template <bool UP, bool NARROW, bool FAR = false>
 int gemm_go(const ExpertArgs& a, int max_tiles, hipStream_t s) {
   constexpr int NB = (NARROW ? 128 : 256) / (UP ? 2 : 1), LDS = NARROW ? GEMM_LDS / 8 * 5 : GEMM_LDS;
-  auto kern = expert_gemm_kernel<UP, NARROW>;
+  auto kern = expert_gemm_kernel<UP, NARROW, FAR>;
   if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess) return 5;
   hipLaunchKernelGGL(kern, dim3((a.N + NB - 1) / NB * max_tiles), dim3(256), LDS, s, a);
   return hipGetLastError() == hipSuccess ? 0 : 4;
@@ -1018,7 +1028,9 @@ KCA_API int kca_moe_route_group(const void* h, const void* wr, const void* wsg, 
 }
 
 // One expert product of every tile. mt: the tiles' row limit (1, 2, 4, 8: gemv; 32: stream, bf16 with K % 64 == 0 and
-// N % 16 == 0; 128, 192, 256: gemm, bf16 with K % 8 == 0 and N % 4 == 0). x_rows: rows of x. ws: a shared expert's product over all tokens beside them (gemv; nullable).
+// N % 16 == 0; 128, 192, 256: gemm, bf16 with K % 8 == 0 and N % 4 == 0). x_rows: rows of x. Where the rows that a tile gathers span
+// 2 GiB or an expert's weights 4 GiB, gemm tiles have up to 128 rows. ws: a shared expert's product over all tokens beside
+// them (gemv; nullable).
 KCA_API int kca_moe_expert(int dtype, const void* x, const void* w, void* y, const void* perm, const void* wts,
                            const void* tiles, const void* ntiles, int max_tiles, int mt, int top, int N, int K, int up,
                            int scale, const void* xs, const void* ws, void* ys, int tokens, int Ns, int Ks, int x_rows,
@@ -1027,17 +1039,15 @@ KCA_API int kca_moe_expert(int dtype, const void* x, const void* w, void* y, con
   if (ws && (!xs || !ys || tokens < 1 || tokens > 32767 || Ns < 1 || Ks < 1 || mt > 8)) return 1;
   const ExpertArgs a{x, w, y, (const int*)perm, (const float*)wts, (const int*)tiles, (const int*)ntiles, top, N, K, up, scale,
                      xs, ws, ys, tokens, Ns, Ks};
+  const bool far = (up ? 4ll : 2ll) * N * K >= 1ll << 32 || 2ll * (up ? x_rows : mt) * K >= 1ll << 31;  // (32-bit byte offsets)
   if (mt == GM || mt == 128 || mt == 192) {
-    if (dtype != 1 || K % 8 || N % 4 || !al16(x) || !al16(w) || (uintptr_t)y % 8 || 2ll * (up ? 2 * N : N) * K >= 1ll << 32 ||
-        (up && 2ll * x_rows * K >= 1ll << 31))  // (32-bit byte offsets)
-      return 10;
+    if (dtype != 1 || K % 8 || N % 4 || !al16(x) || !al16(w) || (uintptr_t)y % 8 || (far && mt != 128)) return 10;
+    if (far) return up ? gemm_go<true, true, true>(a, max_tiles, s) : gemm_go<false, true, true>(a, max_tiles, s);
     if (mt == GM) return up ? gemm_go<true, false>(a, max_tiles, s) : gemm_go<false, false>(a, max_tiles, s);
     return up ? gemm_go<true, true>(a, max_tiles, s) : gemm_go<false, true>(a, max_tiles, s);
   }
   if (mt == SROWS) {
-    if (dtype != 1 || K % SK || N % 16 || !al16(x) || !al16(w) || (uintptr_t)y % 8 || 2ll * (up ? 2 * N : N) * K >= 1ll << 32 ||
-        (up && 2ll * x_rows * K >= 1ll << 31))  // (32-bit byte offsets)
-      return 10;
+    if (dtype != 1 || K % SK || N % 16 || !al16(x) || !al16(w) || (uintptr_t)y % 8 || far) return 10;
     const void* kern = up ? (const void*)expert_stream_kernel<true> : (const void*)expert_stream_kernel<false>;
     if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, STREAM_LDS) != hipSuccess) return 5;
     if (up) hipLaunchKernelGGL(expert_stream_kernel<true>, dim3((N + SWN / 2 - 1) / (SWN / 2) * max_tiles), dim3(256), STREAM_LDS, s, a);

@@ -124,8 +124,12 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
     alone on its CU and pays its ramps in full: it needs a long contraction, or many rows."""
     n = T * top
     used = min(E, n)
-    fits = 4 * F * d < 2 ** 32 and 2 * T * d < 2 ** 31  # 32-bit offsets into an expert's weights and the token rows
-    if dtype == torch.bfloat16 and d % 8 == 0 and F % 8 == 0 and fits:
+    # 32-bit offsets into an expert's weights and the rows of a tile (elsewhere only 128-row tiles have longer ones)
+    near = 4 * F * d < 2 ** 32 and 2 * T * d < 2 ** 31 and 2 * GEMM_ROWS * F < 2 ** 31
+    gemm = dtype == torch.bfloat16 and d % 8 == 0 and F % 8 == 0
+    if gemm and not near and n > 16 * used:
+        return 128
+    if gemm and near:
         stream = d % 64 == 0 and F % 64 == 0
         r, short, full = n / used, min(d, F), used * (F // 64) >= 512
         if r > ((16 if full else 64) if stream else 4):

@@ -39,3 +39,32 @@ def test_products(mt, scale_in, counts, top, d, F):
     a = (torch.nn.functional.silu(u[..., :F]) * u[..., F:]).bfloat16().float()
     want = torch.einsum("tkf,tkdf->tkd", a, dn.float()[e]) * (1 if scale_in else w)
     assert (y.float() - want).norm() <= TOL * want.norm()
+
+
+def _far(T, d, F, E):
+    """Sizes past the 32-bit offsets, and some tokens' outputs in fp32."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    r = lambda *s, std=1.0: torch.empty(s, device="cuda", dtype=torch.bfloat16).normal_(0, std, generator=g)  # noqa: E731
+    h, gu, dn = r(T, d), r(E, 2 * F, d, std=d ** -0.5), r(E, d, F, std=F ** -0.5)
+    ids = torch.randint(0, E, (T, 1), device="cuda", generator=g).int()
+    wts = torch.rand(T, 1, device="cuda", generator=g)
+    mt = moe.tile_rows(T, 1, E, d, F, torch.bfloat16)
+    assert mt == 128
+    groups = moe.group(ids, E, mt)
+    y = moe.experts(h, ids, wts, gu, dn, groups, True)
+    at = torch.cat([torch.arange(T)[:20], torch.arange(T)[-20:], torch.randint(0, T, (40,), generator=torch.Generator().manual_seed(2))]).cuda()
+    got = y[groups.inv.view(-1)[at].long()].float()
+    want = torch.empty_like(got)
+    for e in range(E):
+        k = ids[at, 0] == e
+        u = (h[at[k]].float() @ gu[e].float().T) * wts[at[k]]
+        want[k] = (torch.nn.functional.silu(u[:, :F]) * u[:, F:]).bfloat16().float() @ dn[e].float().T
+    assert (got - want).norm() <= TOL * want.norm()
+
+
+def test_activations_past_2_gib():
+    _far(130960, 8200, 72, 4)
+
+
+def test_expert_weights_past_4_gib():
+    _far(40, 16384, 65536, 1)
