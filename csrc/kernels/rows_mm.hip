@@ -69,7 +69,8 @@ __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
 }
 
 // Bound by the weight stream. A block is 64 weight rows x all activation rows (rounded up to XR); a stage's weights and
-// activations, 64 of K each, go straight to LDS (no registers), so 60 to 64 KiB a workgroup and two workgroups a CU are in flight;
+// activations, 64 of K each, go straight to LDS (no registers), so 60, 64 or 48 KiB a workgroup (XR 32, 64, 128) and two workgroups
+// a CU are in flight;
 // the products (weights as the A operand: a lane holds one activation row and four outputs) hide under it. Blocks of 64 rows
 // rather than 128 keep the CUs busy with fewer slices of K, whose partial sums (4 bytes beside 2 of a weight, for every
 // activation row) cost more than reading the activations once a block from L2: 61 rows of 12288 x 4096 26.5 us against 30.1,
@@ -83,12 +84,13 @@ __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
 //     64    25.3 : 26.8    33.0 : 32.4   15.4 : 13.0   39.1 : 33.8
 //    128    32.2 : 34.2    36.3 : 38.0   24.4 : 17.6   81.5 : 42.2
 // A call costs the host 14 us, the library's through the tuned table 20 to 26: four GPT-J layers on 61 tokens 944 -> 769 us.
+// Which sizes run here: few_rows in ops/linear.py.
 // XR activation rows; 4 waves, WM of them across the activation rows; SNB stages.
 template <bool F16, int XR, int WM, int SNB>
 __global__ void __launch_bounds__(256, 2) rows_mm_kernel(RowsArgs p) {
   constexpr int WN = 4 / WM, A = NB / WN / 16, B = XR / WM / 16;  // a wave's runs of 16 weight and activation rows
   constexpr int STG = (NB + XR) * SK * 2, WI = NB / 32, XI = XR / 32, PER = WI + XI;
-  extern __shared__ __attribute__((aligned(1024))) char sl[];  // [SNB][128 weight rows | XR activation rows][128 B]
+  extern __shared__ __attribute__((aligned(1024))) char sl[];  // [SNB][NB weight rows | XR activation rows][128 B]
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wn = wv % WN, wm = wv / WN;
   const int r16 = lane & 15, g = lane >> 4;
   const int id = xcd_remap(blockIdx.x, gridDim.x);  // the slices of a block on one XCD, beside their partial sums

@@ -168,6 +168,28 @@ def wave_rows(rows: int, n: int, k: int) -> int:
 FEW_ROWS = 128
 
 
+def few_rows(rows: int, n: int, k: int, captured: bool = False) -> bool:
+    """Whether a product of few rows goes to the weight-streaming kernel. us, hipBLASLt : the kernel, weights cold:
+
+    Up to 64 rows: 12288 x 4096, 8 / 32 rows 27.3 : 21.9, 23.9 : 23.1; 4096 x 4096, 8 / 64 15.8 : 11.3, 15.2 : 13.0; 4096 x 16384,
+    64 39.4 : 34.0; 5120 x 20480, 16 115 : 41; 2048 x 8192, 64 22.5 : 14.0. Where the library is the faster one it is by less than
+    the 6 to 12 us that its call costs the host more: 4096 x 16384, 16 rows 30.7 : 32.3, 12288 x 4096, 64 25.8 : 26.9, 768 x 768,
+    16 4.9 : 5.3, 1280 x 1280, 48 6.6 : 8.5.
+    65 to 128 rows: the kernel has one workgroup's LDS for twice the activations, and reads them once a block: only for up to
+    96 blocks of large weights, 96 rows of 4096 x 16384 68.7 : 41.3, of 4096 x 4096 22.4 : 17.2, of 5120 x 5120 27.6 : 22.1 (the
+    least 112 of 4096 x 4096 16.6 : 17.3), not 12288 x 4096 30.5 : 33.6, 8192 x 2048 14.6 : 15.6, 1024 x 4096 9.0 : 15.2. More rows:
+    the library (the blocks would be half as wide: 200 rows of 12288 x 4096 39.9 : 52.5).
+    Beyond one block a CU: 16 rows 18432 x 6144 102 : 63, 24576 x 6144 66.4 : 68.1; 24 rows 58.0 : 64.4, 20480 x 5120 44 : 54.
+    In a capture there is no host time to save, and products cut over K take 1.6 to 2 us more, a fill of the graph's own
+    counters: 16 rows of 4096 x 16384 30.7 : 34.3, of 1024 x 1024 6.0 : 8.3, of 5120 x 5120 15.2 : 17.3; 32 and 64 rows of large
+    weights 34.6 : 34.1, 39.4 : 35.7 and 18.1 : 17.4, 21.7 : 19.8."""
+    if n > 64 * _CUS:
+        return rows <= 16
+    if rows > 64:
+        return rows <= FEW_ROWS and n <= 6144 and n * k >= 1 << 24
+    return not captured or _k_slices(n, k) == 1 or (rows > 24 and n * k >= 1 << 24)
+
+
 def _k_slices(n: int, k: int) -> int:
     """Slices of K for the few-rows kernel's blocks of 64 weight rows: about one block a CU, of 512 or more of K each."""
     return max(1, min(_CUS // -(-n // 64), k // 512))
@@ -193,7 +215,7 @@ def _rows_mm(x2: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) 
 
 
 def linear_rows(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
-    """``F.linear`` without gradients: up to FEW_ROWS rows on the weight-streaming kernel, more in one product or two
+    """``F.linear`` without gradients: few rows on the weight-streaming kernel (``few_rows``), many in one product or two
     (``wave_rows``). ``F.linear`` itself for all else (a gradient or a tangent recorded, a transform or autocast at work,
     tensor subclasses, strided rows, other types)."""
     n, k = weight.shape
@@ -201,9 +223,7 @@ def linear_rows(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None
             or x.shape[-1] != k):
         return F.linear(x, weight, bias)
     rows = x.numel() // k
-    # beyond one block a CU the library is faster from 25 rows on: 50400 x 4096, 24 rows 89.8 us : 89.6 here, 64 rows 85.9 : 102.5.
-    # Past 128 rows it is faster everywhere (the blocks would be half as wide: 200 rows of 12288 x 4096 39.9 : 52.5)
-    few = rows <= (FEW_ROWS if n <= 64 * _CUS else 24)
+    few = rows <= FEW_ROWS and few_rows(rows, n, k, torch.cuda.is_current_stream_capturing())
     first = rows if few else wave_rows(rows, n, k)
     if ((first == rows and not few) or not x.is_contiguous() or weight.dtype != x.dtype
             or (bias is not None and (bias.shape != (n,) or bias.dtype != x.dtype)) or not _lib.inference(x, weight, bias)):

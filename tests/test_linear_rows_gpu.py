@@ -3,7 +3,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from kubernetes_cloud_amd.ops.linear import TLinear, linear_rows, wave_rows
+from kubernetes_cloud_amd.ops.linear import FEW_ROWS, TLinear, few_rows, linear_rows, wave_rows
 
 
 @pytest.mark.parametrize("n,k", [(4096, 4096), (4096, 16384), (12288, 4096), (16384, 4096), (8192, 2048), (6144, 2048),
@@ -16,6 +16,17 @@ def test_parts_cover_the_rows(n, k):
             assert rows > 2048 and k >= 2048
             blocks = first // 256 * -(-n // 256)
             assert first % 256 == 0 and blocks % 256 == 0 and not 1536 < rows - first < 2048
+
+
+@pytest.mark.parametrize("n,k", [(64, 64), (1280, 1280), (4096, 4096), (4096, 16384), (6144, 6144), (12288, 4096), (16384, 4096),
+                                 (18432, 6144), (50400, 4096)])
+def test_few_rows(n, k):
+    # more rows never go back to the kernel once the library has them, but for a capture's products cut over K; a capture
+    # takes no more of them
+    eager, graph = ([few_rows(r, n, k, c) for r in range(1, 200)] for c in (False, True))
+    assert eager == sorted(eager, reverse=True) and all(e or not g for e, g in zip(eager, graph))
+    last = sum(eager)
+    assert last == (16 if n > 16384 else 128 if n <= 6144 and n * k >= 1 << 24 else 64) <= FEW_ROWS
 
 
 def test_other_calls_stay_one_product(monkeypatch):

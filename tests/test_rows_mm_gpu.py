@@ -4,7 +4,7 @@ import torch
 import torch.nn.functional as F
 
 from kubernetes_cloud_amd.ops import _lib
-from kubernetes_cloud_amd.ops.linear import _k_slices, _rows_mm, linear_rows
+from kubernetes_cloud_amd.ops.linear import _k_slices, _rows_mm, few_rows, linear_rows
 from kubernetes_cloud_amd.utils import capture
 
 pytestmark = pytest.mark.gpu
@@ -31,15 +31,15 @@ def test_rows_against_float32(dtype, rows, n, k, bias):
     x, w, b, ref = _inputs(rows, n, k, dtype, bias)
     before = _lib.LAUNCHES[0]
     with torch.no_grad():
-        y = linear_rows(x, w, b)
-        again = linear_rows(x, w, b)
+        y = _rows_mm(x, w, b)
+        again = _rows_mm(x, w, b)
     assert _lib.LAUNCHES[0] == before + 2 and _close(y, ref) and torch.equal(y, again)
 
 
-@pytest.mark.parametrize("rows,n,k", [(61, 4096, 4096), (128, 2048, 2048)])
+@pytest.mark.parametrize("rows,n,k", [(61, 4096, 4096), (128, 4096, 4096)])
 def test_slices_under_capture_and_on_streams(rows, n, k):
     """The slices' counters: two streams at once, and a graph beside eager calls of its stream."""
-    assert _k_slices(n, k) > 1
+    assert _k_slices(n, k) > 1 and few_rows(rows, n, k) and few_rows(rows, n, k, True)
     x, w, b, ref = _inputs(rows, n, k, torch.bfloat16, True)
     main, side = torch.cuda.Stream(), torch.cuda.Stream()
     torch.cuda.synchronize()
