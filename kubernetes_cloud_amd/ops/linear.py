@@ -155,12 +155,14 @@ def wave_rows(rows: int, n: int, k: int) -> int:
 
     Left in one launch: up to 2048 rows (1700 of 16384 x 4096 165 : 172), k below 2048 (a second launch costs as
     much as the idle CUs), widths whose blocks fill a wave only at more rows (6144 and 2048 wide: 8192; there a
-    first part of nearly whole waves loses, 7344 rows of 6144 x 2048 134 : 142), and rests of 1536 to 2048 rows: the
-    library runs 1600 to 1850 rows of 4096 x 16384 at 560 TFLOP/s (5888 rows: 570 in one launch, 755 as 4096 + 1792)."""
+    first part of nearly whole waves loses, 7344 rows of 6144 x 2048 134 : 142), and rests of 1536 to 2048 rows where a
+    wave is no more than that (they fill it nearly: 3948 rows of 8192 x 2048 95 : 98, 3588 of 8192 x 4096 170 : 179) or k is long
+    (1600 to 1850 rows of 4096 x 16384 run at 560 TFLOP/s: 5888 rows 575 : 752, though 5636 883 : 723). Elsewhere such rests
+    gain as others do: 5996 rows of 12288 x 4096 543 : 409, 5636 432 : 392, of 4096 x 4096 172 : 154."""
     across = -(-n // _TILE)
     wave = _TILE * (_CUS // math.gcd(across, _CUS))  # the fewest rows whose blocks fill whole waves
     first = rows // wave * wave
-    if first < 2048 or first == rows or k < 2048 or 1536 < rows - first < 2048:
+    if first < 2048 or first == rows or k < 2048 or (1536 < rows - first < 2048 and (wave <= 2048 or k > 8192)):
         return rows
     return first
 

@@ -15,7 +15,7 @@ def test_parts_cover_the_rows(n, k):
         if first < rows:
             assert rows > 2048 and k >= 2048
             blocks = first // 256 * -(-n // 256)
-            assert first % 256 == 0 and blocks % 256 == 0 and not 1536 < rows - first < 2048
+            assert first % 256 == 0 and blocks % 256 == 0
 
 
 @pytest.mark.parametrize("n,k", [(64, 64), (1280, 1280), (4096, 4096), (4096, 16384), (6144, 6144), (12288, 4096), (16384, 4096),
