@@ -115,6 +115,9 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
                                     600: 128 rows 226, 192 rows 197    1500: 309, 312, wide 332    4096: 645, 634, 558
         2048, 32, 5, 768    tokens   12: vector 53, stream 51       32: 83, 61               250: -, 70, narrow 77
                                     400: stream 76, narrow 79      600: 94, 128 rows 77      8192: -, 382, wide 445
+        widths that are no multiple of 64 have no stream; rows an expert, vector against narrow blocks:
+        4104, 16, 2, 2056   3: 179, 154   4: 209, 176   8: 335, 180   16: 605, 186     1032, 16, 2, 520   4: 34, 22   16: 89, 22
+        4104, 16, 2, 4104   3: 334, 337   4: 376, 329   8: 590, 335   16: 1099, 347    2056, 32, 4, 1032  4: 134, 101
 
     The stream takes over at about 3 rows, at 2 where a row is short (a vector wave's reduction is then a larger part of
     its work), but up to 16 tokens the vector product also carries the shared expert. A stream tile holds 32 rows, past
