@@ -219,6 +219,8 @@ def experts(h: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, gate_up: 
             y[pos] = (ff(h[a // top].float(), gate_up[e], down[e], w if scale_in else 1.0) * (1.0 if scale_in else w)).to(h.dtype)
         return y if shared is None else (y, torch.stack([ff(r.float(), *shared).to(h.dtype) for r in h]))
     assert h.is_contiguous() and gate_up.is_contiguous() and down.is_contiguous() and down.shape == (E, d, F)
+    if g.mt > 8:  # (16-byte loads; the vector product, which calls of up to 16 rows an expert once took, has any address)
+        h, gate_up, down = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (h, gate_up, down))
     act = torch.empty(n, F, device=h.device, dtype=h.dtype)
     y = torch.empty(n, d, device=h.device, dtype=h.dtype)
     mx = g.tiles.shape[0]

@@ -68,3 +68,19 @@ def test_activations_past_2_gib():
 
 def test_expert_weights_past_4_gib():
     _far(40, 16384, 65536, 1)
+
+
+@pytest.mark.parametrize("mt", [moe.STREAM_ROWS, 128])
+def test_rows_off_16_bytes(mt):
+    """Tokens or weights that 16-byte loads do not fit."""
+    h, ids, wts, gu, dn = _case([20, 0, 33, 19], 2, 128, 192)
+    g = moe.group(ids, 4, mt)
+    want = moe.experts(h, ids, wts, gu, dn, g, True)
+
+    def off(t):
+        big = torch.empty(t.numel() + 8, device="cuda", dtype=t.dtype)
+        return big[1:1 + t.numel()].view(t.shape).copy_(t)
+
+    for args in ((off(h), gu, dn), (h, off(gu), dn), (h, gu, off(dn))):
+        y = moe.experts(args[0], ids, wts, *args[1:], g, True)
+        assert torch.equal(y, want)
