@@ -109,10 +109,11 @@ __device__ __forceinline__ int rows_bytes(int rows, long long st, int D) {
 }
 
 // The 32-key tiles of a workgroup's query rows [r0, r0 + BM) in the general forms: it walks tiles [lo, hi),
-// of which [f_lo, f_hi] need no mask. A row's last visible key lies in a tile above f_hi. At least one tile,
+// of which [f_lo, f_hi] need no mask. A row's last visible key lies in a tile above f_hi. For a row's first one, f_lo counts
+// EDGE more tiles: 1, f_lo > lo and it lies in a tile below f_lo or at the start of f_lo; 2, below f_lo. At least one tile,
 // also where no key is visible (a length of 0): its mask gives zeros.
 struct TileSpan { int lo, hi, f_lo, f_hi; };
-template <int BM, bool CAUSAL>
+template <int BM, bool CAUSAL, int EDGE = 0>
 __device__ __forceinline__ TileSpan tile_span(int r0, int off, int kv_end, int window) {
   TileSpan s;
   s.hi = max(1, ((CAUSAL ? min(kv_end, r0 + BM + off) : kv_end) + 31) / 32);
@@ -120,8 +121,9 @@ __device__ __forceinline__ TileSpan tile_span(int r0, int off, int kv_end, int w
   s.lo = s.f_lo = 0;
   if (window > 0) {
     s.lo = min(s.hi - 1, max(0, r0 + off - window + 1) / 32);
-    s.f_lo = max(0, r0 + BM + off - window + 31) / 32;
+    s.f_lo = max(0, r0 + BM + off - window + (EDGE < 2 ? 31 : 32)) / 32;
   }
+  if (EDGE) s.f_lo = max(s.f_lo, s.lo + 1);
   return s;
 }
 __device__ __forceinline__ int batch_keys(const int* kv_len, int b, int Sk) {
@@ -348,9 +350,13 @@ __device__ __forceinline__ void store_tile_lds(bf16_t* row0, long long st, const
 // column MC set to 1.0 (the SD UNet folds both into its padded QKV weights), and the kernel writes
 // -m into Q's column MC in registers once m is known, so the S MFMAs return s * log2(e) - m and
 // P = exp2(S) needs no per-element FMA: the D <= 64 loop is bound by that VALU work, not the MFMAs.
-// G > 0 walks the tiles from the last to the first: every row's last visible key -- with ALiBi the one with the
-// least bias, with a window or a length one that surely exists -- then lies in one of the first, masked tiles,
-// whose row max is the reference (below).
+// The reference (below) of G > 0 is the row max of the row's first tile with a visible key, which is a masked one. G = 1 walks
+// the tiles from the first, as G = 0 and the generic kernels do, and takes the next tile's scores into the reference: the
+// weight that it belongs to is exactly 1, so the more keys it is the largest of, the less is rounded (a row's last tile holds
+// 16 of its keys on average: error against 64 bits, 8 x 1000 x 12 of 64, 0.00210 from there, 0.00208 from the first tile as the
+// generic kernel has it, 0.00206 from two; us, from the last tile and so: 37.5, 37.8, 2 x 2048 x 20 of 128 with a window of 256
+// 38.2, 39.4, prompts of 256 packed 97.4, 100.4). G = 2 walks them from the last, where ALiBi's bias is least: from the first,
+// later scores would pass the reference by the whole bias (0.00196 in the generic kernel, 0.00192 here, 2048 x 14 of 128).
 // (two waves a SIMD to D = 160, which spills 0 to 9 registers for it: 4 x 4096 x 8 238 -> 226 us)
 template <int D, bool CAUSAL, int OC = -1, int DS = D, int MC = -1, int G = 0>
 __global__ void __launch_bounds__(256, (D <= 160 ? 2 : 1)) attn_fwd_tiled_kernel(FastFwdParams p) {
@@ -388,9 +394,9 @@ __global__ void __launch_bounds__(256, (D <= 160 ? 2 : 1)) attn_fwd_tiled_kernel
   int kv_hi = kv_end;
   if (CAUSAL) kv_hi = min(kv_hi, qb * BM + BM + off);
   TileSpan sp{};
-  if constexpr (G > 0) sp = tile_span<BM, CAUSAL>(qb * BM, off, kv_end, p.window);
+  if constexpr (G > 0) sp = tile_span<BM, CAUSAL, G == 1>(qb * BM, off, kv_end, p.window);  // (a tile's successor is at hand)
   const int ntiles = G ? sp.hi - sp.lo : kv_hi > 0 ? (kv_hi + BN - 1) / BN : 0;
-  auto key0 = [&](int t) { return G ? (sp.hi - 1 - t) * BN : t * BN; };  // first key of the t-th tile walked
+  auto key0 = [&](int t) { return (G == 2 ? sp.hi - 1 - t : G ? sp.lo + t : t) * BN; };  // first key of the t-th tile walked
   static_assert(MC < 0 || (!CAUSAL && OC >= 0 && MC < DS), "max column: non-causal, with the row-sum column");
   const float sl2 = MC >= 0 ? 1.f : p.scale * kLog2e;
 
@@ -514,10 +520,11 @@ __global__ void __launch_bounds__(256, (D <= 160 ? 2 : 1)) attn_fwd_tiled_kernel
     for (int r = 0; r < 16; ++r) sa[r] -= m;
   }
   float nm = G ? 0.f : -m;
+  bool begun = false;  // G == 1: a tile with a visible key of this row has been walked
   ASTAMP(0);
 
   auto tile_step = [&](int t, auto masked, auto par) {
-    constexpr bool MASKED = decltype(masked)::value;
+    constexpr bool MASKED = decltype(masked)::value, HEAD = decltype(masked)::value == 2;
     const char* Vs = smem + (t % 3) * 2 * TILE + TILE;
     const char* Kn = smem + ((t + 1) % 3) * 2 * TILE;
     // PF2: tile t+3 is requested into one register set while the other (tile t+2, requested an
@@ -544,14 +551,24 @@ __global__ void __launch_bounds__(256, (D <= 160 ? 2 : 1)) attn_fwd_tiled_kernel
     }
     if constexpr (MASKED) mask(sa, key0(t));
     if constexpr (G > 0 && MASKED) {
-      float mt = -INFINITY;
+      float mt = -INFINITY, m_here = -INFINITY;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         sa[r] = G == 2 ? fmaf(sa[r], sl2, bias[r]) : sa[r] * sl2;
         mt = fmaxf(mt, sa[r]);
       }
+      if constexpr (HEAD) {  // (the next tile's scores are at hand; stale ones lie past the last key)
+        m_here = fmaxf(mt, __shfl_xor(mt, 32, 64));
+        const int lim = last - key0(t + 1) - 4 * hh, lo = before - key0(t + 1) - 4 * hh;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int c = (r & 3) + 8 * (r >> 2);
+          mt = fmaxf(mt, c > lim || c <= lo ? -INFINITY : sb[r] * sl2);
+        }
+      }
       mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-      m = m == -INFINITY ? mt : m;
+      m = m == -INFINITY || (HEAD && !begun) ? mt : m;
+      if constexpr (HEAD) begun = begun || m_here > -INFINITY;
       nm = m == -INFINITY ? 0.f : -m;
       sl = 1.f;
     }
@@ -615,6 +632,11 @@ __global__ void __launch_bounds__(256, (D <= 160 ? 2 : 1)) attn_fwd_tiled_kernel
     tile_step(t + 1, std::true_type{}, std::true_type{});
   }
   if (t < ntiles) tile_step(t, std::true_type{}, std::false_type{});
+  } else if constexpr (G == 1) {
+    const int low = min(ntiles, max(0, sp.f_lo - sp.lo)), top = max(low, min(ntiles, sp.f_hi + 1 - sp.lo));
+    for (int t = 0; t < low; ++t) tile_step(t, std::integral_constant<int, 2>{}, std::false_type{});
+    for (int t = low; t < top; ++t) tile_step(t, std::false_type{}, std::false_type{});
+    for (int t = top; t < ntiles; ++t) tile_step(t, std::true_type{}, std::false_type{});
   } else if constexpr (G > 0) {
     const int top = min(ntiles, sp.hi - 1 - sp.f_hi), low = max(top, min(ntiles, sp.hi - sp.f_lo));
     for (int t = 0; t < top; ++t) tile_step(t, std::true_type{}, std::false_type{});
@@ -763,10 +785,10 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
   const int kv_end = G ? batch_keys(p.kv_len, b, p.Sk) : p.Sk;
   int kv_hi = kv_end;
   if (CAUSAL) kv_hi = min(kv_hi, qb * BM + BM + off);
-  TileSpan sp{}, own{};  // G: of the workgroup, of this wave's rows (which walk the same order, tile_span)
+  TileSpan sp{}, own{};  // G: of the workgroup, of this wave's rows (which walk attn_fwd_tiled_kernel's order)
   if constexpr (G > 0) {
     sp = tile_span<BM, CAUSAL>(qb * BM, off, kv_end, p.window);
-    own = tile_span<32, CAUSAL>(q0, off, kv_end, p.window);
+    own = tile_span<32, CAUSAL, G == 1 ? 2 : 0>(q0, off, kv_end, p.window);
     if (q0 >= p.Sq) own.hi = 0;
   }
   const int ntiles = G ? sp.hi - sp.lo : kv_hi / BN;
@@ -803,7 +825,7 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
   lds_char* lsm = (lds_char*)smem;
   auto issue = [&](int tile, int buf) {
     int kt = min(tile, ntiles - 1);  // clamped: the last tiles re-load a tile nobody reads
-    if constexpr (G > 0) kt = sp.hi - 1 - kt;
+    if constexpr (G > 0) kt = G == 2 ? sp.hi - 1 - kt : sp.lo + kt;
     const int sok = __builtin_amdgcn_readfirstlane(kt * BN * (int)p.k_st * 2);
     const int sov = __builtin_amdgcn_readfirstlane(kt * BN * (int)p.v_st * 2);
 #if defined(__HIP_DEVICE_COMPILE__)  // (the host pass drops the launch stub over this builtin)
@@ -823,6 +845,7 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[i][r] = 0.f;
   float m = G ? -INFINITY : 0.f, lsum = 0.f;
+  float rsum = 0.f;  // G == 1 with a window: sum of the weights as they are multiplied with V, rounded
   const float slope = G == 2 ? p.alibi[h] * kLog2e : 0.f;
 
   // per-lane LDS read bases (bytes, relative to a stage)
@@ -869,7 +892,7 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         if ((r & 3) + 8 * (r >> 2) > lim) sa[r] = -INFINITY;
-      if (G && t < own.f_lo) {
+      if (G && p.window > 0 && t < own.f_lo) {
         const int lo = qrow + off - p.window - t * BN - 4 * hh;
 #pragma unroll
         for (int r = 0; r < 16; ++r)
@@ -877,7 +900,7 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
       }
     }
     // reference max = the first tile's row max (see attn_fwd_tiled_kernel)
-    if (G ? t > own.f_hi : t == 0) {
+    if (G == 2 ? t > own.f_hi : G ? t < own.f_lo : t == 0) {
       float mt = sa[0];
 #pragma unroll
       for (int r = 1; r < 16; ++r) mt = fmaxf(mt, sa[r]);
@@ -895,6 +918,12 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
       pf1[r] = (__bf16)e1;
     }
     lsum += ps;
+    if (G == 1 && p.window > 0) {
+      float pr = 0.f;
+#pragma unroll
+      for (int r = 0; r < 8; ++r) pr += (float)pf0[r] + (float)pf1[r];
+      rsum += pr;
+    }
     ASTAMP(4);
   };
   // O^T += V^T.P^T of the tile in `buf`: the V^T reads of d-block db+1 in flight under block db's MFMAs
@@ -942,7 +971,7 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
   constexpr auto CM = std::integral_constant<bool, (CAUSAL || G > 0)>{};
   for (int t = 0; t < ntiles; ++t) {
     sync_issue(t);
-    const int tile = sp.hi - 1 - t;
+    const int tile = G == 2 ? sp.hi - 1 - t : sp.lo + t;
     if (G ? tile < own.hi && tile >= own.lo : t < mytiles) {
       sm_part(t % NBUF, CM, G ? tile : t);
       pv_part(t % NBUF);
@@ -953,7 +982,11 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
   const bool bad = !(ltot < 1.2676506e30f) && (!G || qrow < p.Sq);
   const int any_bad = __any(bad);
   if (lane == 0 && (!G || qb128 < nqb128)) *flag = any_bad;
-  const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
+  // With a window a row's first tile holds 16 of its keys on average: the reference is its largest weight less often than
+  // elsewhere (attn_fwd_tiled_kernel). Dividing by the rounded weights makes up for it: error against 64 bits of 2 x 1000 x 16
+  // heads, window 256, 0.00213 -> 0.00210 (generic kernel 0.00212). lse keeps the sum of the unrounded ones.
+  const float div = G == 1 && p.window > 0 ? rsum + __shfl_xor(rsum, 32, 64) : ltot;
+  const float inv = ltot > 0.f ? 1.f / div : 0.f;
   if (hh == 0 && p.lse && (!G || qrow < p.Sq))
     p.lse[((long long)b * p.H + h) * p.Sq + qrow] = ltot > 0.f ? (m + log2f(ltot)) * kLn2 : INFINITY;
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // the clamped tail DMAs

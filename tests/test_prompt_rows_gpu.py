@@ -30,15 +30,19 @@ def test_packed_attention(D, alibi, window):
         assert (o[a:b].float() - r).norm() <= TOL * r.norm()
 
 
-def test_packed_attention_overflowing_rows():
+@pytest.mark.parametrize("early", [60.0, -60.0])
+@pytest.mark.parametrize("D", [128, 256])
+@pytest.mark.parametrize("alibi", [False, True])
+def test_packed_attention_overflowing_rows(early, D, alibi):
     """Rows whose reference is 2^100 below a later score are recomputed in their own sequence."""
     lens = [40, 200]
-    q = torch.zeros(240, 1, 128, device="cuda", dtype=torch.bfloat16)
-    k, v = torch.zeros_like(q), torch.randn(240, 1, 128, device="cuda").bfloat16()
-    q[..., 0], k[45, 0, 0], k[230, 0, 0] = 40.0, 60.0, -60.0
+    q = torch.zeros(240, 1, D, device="cuda", dtype=torch.bfloat16)
+    k, v = torch.zeros_like(q), torch.randn(240, 1, D, device="cuda").bfloat16()
+    q[..., 0], k[45, 0, 0], k[230, 0, 0] = 40.0, early, -early
     cu = torch.tensor([0, 40, 240], device="cuda", dtype=torch.int32)
-    o = ops.packed_attention(q, k, v, cu, 200)
-    r = attention_reference(q[None, 40:], k[None, 40:], v[None, 40:], True)[0][0].float()
+    sl = torch.full((1,), 0.25, device="cuda") if alibi else None
+    o = ops.packed_attention(q, k, v, cu, 200, alibi=sl)
+    r = attention_reference(q[None, 40:], k[None, 40:], v[None, 40:], True, None, None, sl)[0][0].float()
     assert (o[40:].float() - r).norm() <= TOL * r.norm()
 
 
