@@ -178,16 +178,20 @@ __device__ __forceinline__ f32x16 mma16(bf16x8 a, bf16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// eight floats as the sum of two fp16 (22 bits)
-__device__ __forceinline__ void split_f16x8(const float* x, bf16x8& hi, bf16x8& lo) {
-  f16x8 h, l;
+// eight floats as sums of three fp16: all 24 bits, down to 2^-25
+__device__ __forceinline__ void split_f16x8(const float* x, bf16x8 (&part)[3]) {
+  f16x8 p[3];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    h[i] = (_Float16)x[i];
-    l[i] = (_Float16)(x[i] - (float)h[i]);
+    float rest = x[i];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      p[j][i] = (_Float16)rest;
+      rest -= (float)p[j][i];
+    }
   }
-  hi = __builtin_bit_cast(bf16x8, h);
-  lo = __builtin_bit_cast(bf16x8, l);
+#pragma unroll
+  for (int j = 0; j < 3; ++j) part[j] = __builtin_bit_cast(bf16x8, p[j]);
 }
 
 // Deferred-rescale threshold (log2 units): O / l are rescaled only when a row's
@@ -195,9 +199,9 @@ __device__ __forceinline__ void split_f16x8(const float* x, bf16x8& hi, bf16x8& 
 #define RESCALE_THR 8.0f
 
 // ============================================================== forward
-// F16: fp16 rows (packed prompts of fp16 servers; no lse). Softmax weights keep 22 bits, as two fp16 whose products with V
-// are added (the general way beside it, fp32 matrices of all scores, keeps 24), and are held 2^7 up, so that what fp16
-// cannot hold is below 2^-21 of a row's largest. 5400 rows of 6 prompts, 16 heads of 256: 352 us, the general way 3.2 ms.
+// F16: fp16 rows (packed prompts of fp16 servers; no lse). Softmax weights keep their 24 bits, as three fp16 whose products
+// with V are added, and are held 2^7 up, so that what fp16 cannot hold is below 2^-32 of a row's largest. 5400 rows of 6
+// prompts, 16 heads of 256: 307 us (284 with two parts, 22 bits); the general way, fp32 matrices of all scores, 3.2 ms.
 template <int D, bool CAUSAL, bool F16 = false>
 __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1)) attn_fwd_kernel(AttnParams p) {
   using L = FwdLds<D>;
@@ -336,12 +340,11 @@ __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1)) attn_fwd_kernel(AttnP
         ps += x[r];
       }
       lsum += ps;
-      bf16x8 pf[2], pl[2];
-      if constexpr (F16) {
-        split_f16x8(x, pf[0], pl[0]);
-        split_f16x8(x + 8, pf[1], pl[1]);
-      } else {
-        pf[0] = to_bf16x8(x), pf[1] = to_bf16x8(x + 8);
+      bf16x8 pf[2][F16 ? 3 : 1];
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        if constexpr (F16) split_f16x8(x + 8 * s, pf[s]);
+        else pf[s][0] = to_bf16x8(x + 8 * s);
       }
 #pragma unroll
       for (int db = 0; db < D / 32; ++db) {
@@ -350,8 +353,8 @@ __global__ void __launch_bounds__(256, (D <= 128 ? 2 : 1)) attn_fwd_kernel(AttnP
           const int row = 16 * s + 4 * hh + (gi >> 2);
           const bf16_t* vb = Vs + row * L::VSTR + db * 32 + dcol;
           bf16x8 a = cat44(tr_read(vb), tr_read(vb + 8 * L::VSTR));
-          oacc[db] = mma16<F16>(a, pf[s], oacc[db]);
-          if constexpr (F16) oacc[db] = mma16<F16>(a, pl[s], oacc[db]);
+#pragma unroll
+          for (int j = 0; j < (F16 ? 3 : 1); ++j) oacc[db] = mma16<F16>(a, pf[s][j], oacc[db]);
         }
       }
     }

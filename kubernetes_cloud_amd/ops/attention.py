@@ -204,7 +204,7 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: b
 def packed_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu: torch.Tensor, max_len: int,
                      scale: float | None = None, alibi: torch.Tensor | None = None, window: int = 0) -> torch.Tensor:
     """Causal self-attention of sequences that lie one after another in [T, H, D] rows (inference): sequence i is rows
-    ``cu[i]`` .. ``cu[i + 1]`` (int32, on the device), none longer than ``max_len``. bf16, or fp16 with softmax weights of 22
+    ``cu[i]`` .. ``cu[i + 1]`` (int32, on the device), none longer than ``max_len``. bf16, or fp16 with softmax weights of 24
     bits."""
     T, H, D = q.shape
     f16 = q.dtype == torch.float16

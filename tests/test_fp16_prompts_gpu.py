@@ -1,4 +1,4 @@
-"""fp16 prompts on the native kernels: packed attention with softmax weights of 22 bits, LayerNorm rows and GELU against
+"""fp16 prompts on the native kernels: packed attention with softmax weights of 24 bits, LayerNorm rows and GELU against
 float64 or float32, and the gradient, strided and odd calls that stay torch's."""
 import pytest
 import torch
@@ -30,7 +30,7 @@ def test_packed_attention(D, alibi, window):
         seen = (i[None] <= i[:, None]) & ((i[None] > i[:, None] - window) if window else True)
         p = z.masked_fill(~seen, -torch.inf).softmax(-1)
         want = torch.einsum("hqk,khd->qhd", p, v[a:b].double())
-        # the result's rounding; scores in 32 bits (products of up to 256 terms) and weights of 22 bits under it
+        # the result's rounding; scores in 32 bits (products of up to 256 terms) and weights of 24 bits under it
         size = torch.einsum("hqk,khd->qhd", p, v[a:b].double().abs())
         assert ((o[a:b].double() - want).abs() <= EPS * want.abs() + 2.0 ** -17 * size + 2.0 ** -24).all()
 
