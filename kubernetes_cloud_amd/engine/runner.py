@@ -784,11 +784,12 @@ class ModelRunner(StepRunner):
                 self.cache.release(s_)  # a reused slot starts empty
             self.cache.reserve(s_, p0 + L)
         self.cache.sync()
-        if self._append_ok and not cont and len(set(slots)) == n:
-            return self._prefill_packed(ids, slots, lens)
+        append = self._append_ok and len(set(slots)) == n  # (rows that share a slot are written one after another)
+        if append and not cont:
+            return self._prefill_packed(ids if ids.device.type == "cpu" else ids.to(self.device), slots, lens)
         ids = ids.to(self.device)
         plan = where = None
-        if self._append_ok:  # one launch a layer rotates and fills the pages (padding rows: page -1)
+        if append:  # one launch a layer rotates and fills the pages (padding rows: page -1)
             at = np.concatenate([np.arange(i * T, i * T + L) for i, L in enumerate(lens)])
             where = np.zeros((3, n * T), dtype=np.int32)
             where[0] = -1

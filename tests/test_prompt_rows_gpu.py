@@ -109,3 +109,14 @@ def test_runner_packs_prompts(name, on_gpu):
             for s, n in zip(slots, lens)]
     a, b = r.decode(rows), one.decode(rows)
     assert max(abs(x - y) for x, y in zip(a[1], b[1])) < 0.05
+
+
+def test_prompts_that_share_a_slot():
+    """The later row's keys and values stay (without pages they are written one prompt after another)."""
+    m = build_model(LMConfig.from_hf(TINY["gptj"]), device="cuda", dtype=torch.bfloat16, seed=1)
+    ids = torch.randint(0, 512, (8, 64), generator=torch.Generator().manual_seed(0))
+    r, one = (ModelRunner(m, max_slots=2, max_len=96, page_size=0) for _ in range(2))
+    r.prefill(ids, [1] * 8)
+    one.prefill(ids[7:], [1])
+    for a, b in zip(r.cache.k + r.cache.v, one.cache.k + one.cache.v):
+        assert (a[1, :, :64].float() - b[1, :, :64].float()).norm() <= 2e-2 * b[1, :, :64].float().norm()
