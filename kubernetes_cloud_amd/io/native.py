@@ -63,6 +63,13 @@ def load():
         return lib
 
 
+def settle(device) -> None:
+    """Waits for what the current stream still does with the destinations: a cast into them, or the work of tensors whose memory
+    they took over. The streamers copy on streams of their own, which wait for nothing."""
+    import torch
+    torch.cuda.current_stream(device).synchronize()
+
+
 def available() -> bool:
     try:
         load()

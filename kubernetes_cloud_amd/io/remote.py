@@ -208,6 +208,7 @@ def _stream(r: Remote, offs, lens, ptrs, device, threads: int = 16, chunk: int =
     dev = -1
     if device.type == "cuda":
         dev = device.index if device.index is not None else torch.cuda.current_device()
+        native.settle(device)
     rc = lib.kca_http_stream(r.host.encode(), r.port, int(r.tls), int(r.verify), r.path.encode(),
                              r.headers.encode(), n, a_off, a_len, a_ptr, dev, threads, chunk, r.timeout_s, stats)
     if rc != 0:

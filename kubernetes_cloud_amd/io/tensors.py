@@ -107,6 +107,7 @@ def _stream(path: str, offs, lens, ptrs, device: torch.device, threads: int, chu
     stats = (ctypes.c_double * 4)()
     lib = native.load()
     if device.type == "cuda":
+        native.settle(device)
         rc = lib.kca_stream_to_device(path.encode(), n, a_off, a_len, a_ptr,
                                       device.index if device.index is not None else torch.cuda.current_device(),
                                       threads, chunk, int(odirect), stats)

@@ -115,3 +115,26 @@ def test_dataset_tokenizer_cli_and_packing(tmp_path):
           "-sampling", "50"])
     n2 = np.fromfile(out2, dtype="<u2").size // 32
     assert n2 == (len(ds) + 1) // 2 or n2 == len(ds) // 2
+
+
+@pytest.mark.parametrize("remote", [False, True])
+def test_streams_wait_for_the_destinations(monkeypatch, remote):
+    """Before a byte is copied on the streamer's own streams, what the current one does with the memory is done."""
+    from types import SimpleNamespace
+
+    from kubernetes_cloud_amd.io import remote as rm
+    from kubernetes_cloud_amd.io import tensors
+    done = []
+
+    def entry(name):
+        return lambda *a: done.append(name) or 0
+
+    monkeypatch.setattr(native, "load", lambda: SimpleNamespace(kca_stream_to_device=entry("copy"), kca_http_stream=entry("copy")))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d=None: SimpleNamespace(synchronize=lambda: done.append("wait")))
+    dev = torch.device("cuda", 0)
+    if remote:
+        r = SimpleNamespace(host="h", port=1, tls=0, verify=0, path="/", headers="", timeout_s=1.0, url="u")
+        rm._stream(r, [0], [8], [0], dev)
+    else:
+        tensors._stream("x", [0], [8], [0], dev, 1, 1 << 20, False)
+    assert done == ["wait", "copy"]
