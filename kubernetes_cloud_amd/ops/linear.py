@@ -171,25 +171,31 @@ FEW_ROWS = 128
 
 
 def few_rows(rows: int, n: int, k: int, captured: bool = False) -> bool:
-    """Whether a product of few rows goes to the weight-streaming kernel. us, hipBLASLt : the kernel, weights cold:
+    """Whether a product of few rows goes to the weight-streaming kernel. On the GPU, us, hipBLASLt : the kernel, weights cold:
 
-    Up to 64 rows: 12288 x 4096, 8 / 32 rows 27.3 : 21.9, 23.9 : 23.1; 4096 x 4096, 8 / 64 15.8 : 11.3, 15.2 : 13.0; 4096 x 16384,
-    64 39.4 : 34.0; 5120 x 20480, 16 115 : 41; 2048 x 8192, 64 22.5 : 14.0. Where the library is the faster one it is by less than
-    the 6 to 12 us that its call costs the host more: 4096 x 16384, 16 rows 30.7 : 32.3, 12288 x 4096, 64 25.8 : 26.9, 768 x 768,
-    16 4.9 : 5.3, 1280 x 1280, 48 6.6 : 8.5.
-    65 to 128 rows: the kernel has one workgroup's LDS for twice the activations, and reads them once a block: only for up to
-    96 blocks of large weights, 96 rows of 4096 x 16384 68.7 : 41.3, of 4096 x 4096 22.4 : 17.2, of 5120 x 5120 27.6 : 22.1 (the
-    least 112 of 4096 x 4096 16.6 : 17.3), not 12288 x 4096 30.5 : 33.6, 8192 x 2048 14.6 : 15.6, 1024 x 4096 9.0 : 15.2. More rows:
-    the library (the blocks would be half as wide: 200 rows of 12288 x 4096 39.9 : 52.5).
-    Beyond one block a CU: 16 rows 18432 x 6144 102 : 63, 24576 x 6144 66.4 : 68.1; 24 rows 58.0 : 64.4, 20480 x 5120 44 : 54.
-    In a capture there is no host time to save, and products cut over K take 1.6 to 2 us more, a fill of the graph's own
-    counters: 16 rows of 4096 x 16384 30.7 : 34.3, of 1024 x 1024 6.0 : 8.3, of 5120 x 5120 15.2 : 17.3; 32 and 64 rows of large
+        12288 x 4096   8 rows 27.3 : 21.9    32: 23.9 : 23.1    64: 25.8 : 26.9    96: 30.5 : 33.6    128: 32.4 : 34.4
+        4096 x 4096           15.8 : 11.3        13.4 : 11.7        15.2 : 13.0        22.4 : 17.2         24.8 : 17.7
+        4096 x 16384          30.4 : 32.4        34.6 : 32.2        39.4 : 34.0        68.7 : 41.3         81.5 : 42.9
+        8192 x 2048           13.2 : 10.8        13.2 : 11.1        13.9 : 12.2        14.6 : 15.6         16.1 : 16.3
+        1024 x 4096           11.4 : 8.7          8.9 : 9.0         12.2 : 10.5         9.0 : 15.2          9.5 : 15.5
+        5120 x 20480           113 : 40           122 : 42           130 : 49           141 : 60            148 : 63
+        14336 x 14336         82.5 : 84.3        84.6 : 84.8        96.1 : 96.5       107.3 : 118.3       119.4 : 127.1
+
+    A call costs the host 6 to 12 us less, and a layer of a short prompt is issued in about the time that it runs in. So an eager
+    call takes the kernel also where it is a little slower: four GPT-J layers of 4096, 100 tokens, 1030 us with the library from 65
+    rows on for 12288 and 16384 outputs, 900 without it; of 2048, 980 and 735. Not past 2^27 weights and 64 rows, unless few
+    blocks leave the library's products without CUs; and for more blocks than CUs up to 24 rows (50400 x 4096 89.8 : 89.6,
+    24576 x 6144 72.5 : 69.0, 20480 x 5120 44 : 54; 64 rows 85.9 : 102.5). More than 128 rows: the library (the blocks would be
+    half as wide: 200 rows of 12288 x 4096 39.9 : 52.5).
+    In a capture there is no host time to save, and a product cut over K takes 1.6 to 2 us more, a fill of the graph's own
+    counters: 16 rows of 4096 x 16384 30.7 : 34.3, of 1024 x 1024 6.0 : 8.3, of 5120 x 5120 15.2 : 17.3, 32 and 64 rows of large
     weights 34.6 : 34.1, 39.4 : 35.7 and 18.1 : 17.4, 21.7 : 19.8."""
     if n > 64 * _CUS:
-        return rows <= 16
-    if rows > 64:
-        return rows <= FEW_ROWS and n <= 6144 and n * k >= 1 << 24
-    return not captured or _k_slices(n, k) == 1 or (rows > 24 and n * k >= 1 << 24)
+        return rows <= (16 if captured else 24)
+    if captured:
+        large = n * k >= 1 << 24
+        return rows <= FEW_ROWS and (n <= 6144 and large if rows > 64 else _k_slices(n, k) == 1 or (rows > 24 and large))
+    return rows <= 64 or (rows <= FEW_ROWS and (n <= 6144 or n * k <= 1 << 27))
 
 
 def _k_slices(n: int, k: int) -> int:

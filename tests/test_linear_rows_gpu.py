@@ -18,15 +18,13 @@ def test_parts_cover_the_rows(n, k):
             assert first % 256 == 0 and blocks % 256 == 0
 
 
-@pytest.mark.parametrize("n,k", [(64, 64), (1280, 1280), (4096, 4096), (4096, 16384), (6144, 6144), (12288, 4096), (16384, 4096),
-                                 (18432, 6144), (50400, 4096)])
-def test_few_rows(n, k):
-    # more rows never go back to the kernel once the library has them, but for a capture's products cut over K; a capture
-    # takes no more of them
+@pytest.mark.parametrize("n,k,last", [(64, 64, 128), (1280, 1280, 128), (4096, 16384, 128), (12288, 4096, 128), (16384, 4096, 128),
+                                      (14336, 14336, 64), (6144, 24576, 128), (18432, 6144, 24), (50400, 4096, 24)])
+def test_few_rows(n, k, last):
+    # eager calls up to a number of rows; a capture takes no other ones
     eager, graph = ([few_rows(r, n, k, c) for r in range(1, 200)] for c in (False, True))
-    assert eager == sorted(eager, reverse=True) and all(e or not g for e, g in zip(eager, graph))
-    last = sum(eager)
-    assert last == (16 if n > 16384 else 128 if n <= 6144 and n * k >= 1 << 24 else 64) <= FEW_ROWS
+    assert eager == [r <= last for r in range(1, 200)] and last <= FEW_ROWS
+    assert all(e or not g for e, g in zip(eager, graph))
 
 
 def test_other_calls_stay_one_product(monkeypatch):

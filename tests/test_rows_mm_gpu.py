@@ -31,8 +31,8 @@ def test_rows_against_float32(dtype, rows, n, k, bias):
     x, w, b, ref = _inputs(rows, n, k, dtype, bias)
     before = _lib.LAUNCHES[0]
     with torch.no_grad():
-        y = _rows_mm(x, w, b)
-        again = _rows_mm(x, w, b)
+        y = linear_rows(x, w, b)
+        again = linear_rows(x, w, b)
     assert _lib.LAUNCHES[0] == before + 2 and _close(y, ref) and torch.equal(y, again)
 
 
