@@ -1089,11 +1089,14 @@ static int attn_fwd_go(AttnParams p, int rowsum_col, int max_col, int* workspace
   if (p.d_real % 8 || p.H % p.Hkv || p.window < 0) return 1;
   const int D = pick_d(p.d_real);
   p.km_words = (p.Sk + 31) / 32;
-  if (g_attn_tiled && workspace && !p.key_mask &&
-      kca_attn_fwd_tiled(p.q, p.k, p.v, p.o, p.lse, p.q_sb, p.q_st, p.q_sh, p.k_sb, p.k_st, p.k_sh, p.v_sb, p.v_st,
-                         p.v_sh, p.o_sb, p.o_st, p.o_sh, p.B, p.Sq, p.Sk, p.H, p.Hkv, p.d_real, p.causal, p.scale,
-                         p.alibi, p.kv_len, p.window, p.cu, rowsum_col, max_col, workspace, stream) == 0)
-    p.fix_flags = workspace;  // fixup launch below: only flagged blocks do work
+  if (g_attn_tiled && workspace && !p.key_mask) {
+    const int rc =
+        kca_attn_fwd_tiled(p.q, p.k, p.v, p.o, p.lse, p.q_sb, p.q_st, p.q_sh, p.k_sb, p.k_st, p.k_sh, p.v_sb, p.v_st,
+                           p.v_sh, p.o_sb, p.o_st, p.o_sh, p.B, p.Sq, p.Sk, p.H, p.Hkv, p.d_real, p.causal, p.scale,
+                           p.alibi, p.kv_len, p.window, p.cu, rowsum_col, max_col, workspace, stream);
+    if (rc < 0) return 0;  // no row is left to another kernel
+    if (rc == 0) p.fix_flags = workspace;  // fixup launch below: only flagged blocks do work
+  }
   dim3 grid(((p.Sq + 127) / 128) * p.B * p.H);
   ATTN_D_DISPATCH(D, {
     if (p.causal)

@@ -1,0 +1,368 @@
+// Flash attention for calls whose 128-row blocks leave the chip idle: the keys of a block are split over the wave groups
+// of its workgroup.
+//
+// What bounds these calls. attn_fwd_tiled_kernel gives a workgroup 128 rows and a wave 32 of them; a call of few heads and
+// rows then has less than one workgroup a CU, so a SIMD runs one wave whose products, softmax, LDS reads and barriers follow
+// each other, and under a causal mask the call waits for the block that sees all keys: 2048 tokens x 14 heads of 128 are 224
+// workgroups on 256 CUs, 52 us for the 64 tiles of the longest one. Here a workgroup has RW * 32 rows and KG groups of RW
+// waves; group g walks tiles g, g + KG, ... with LDS buffers of its own and the partial sums meet in LDS at the end. Blocks
+// are half as tall, so there are twice as many, each 1 / KG as long, and a SIMD has two waves to run.
+//
+// The forms of a mask are attention_tiled.hip's general ones (1: lengths, windows, any sizes; 2: ALiBi) and every call takes
+// one of them. Blocks are taken longest first over all heads (block number = row block * heads + head).
+//
+// Tiles in LDS: two buffers of K and V a group. A step computes S of the group's next tile while it takes the softmax of this
+// one, so K runs a tile ahead of V: K(i + 2) goes where K(i) was and V(i + 1) where V(i - 1) was, which all waves have read
+// before the last barrier.
+//
+// Softmax reference: as in attn_fwd_tiled_kernel the row's maximum over the first tile with a visible key, here of each
+// group; the groups' sums are scaled to the largest reference when they meet. Rows whose sum passes 2^100 (a later score far
+// above the first tile's) are computed again in the same launch with the row's true maximum.
+#include "attn_fast.h"
+
+#include <type_traits>
+
+namespace {
+
+constexpr int kNoTile = 1 << 29;  // first "key" of a tile past the end of a group's walk: masks everything
+
+// A 32-row x D tile staged by the NT threads of a group: chunk idx = thread + NT * j is (row idx / NCH, 16-byte chunk idx % NCH);
+// the last round may be the first waves' alone.
+template <int D, int NT>
+struct GroupStager {
+  static constexpr int NCH = D / 8, TOT = 32 * NCH, CPT = (TOT + NT - 1) / NT;
+  static constexpr bool EVEN = NT % NCH == 0 && TOT % NT == 0;  // chunk column the same for all j: rows a scalar offset apart
+  static_assert(TOT % 64 == 0, "whole waves");
+  int vo_[EVEN ? 1 : CPT], lds_[CPT];
+  int step_;
+  bool tail_;  // this thread owns a chunk in the last round
+  __device__ __forceinline__ GroupStager(int t, long long st) {
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) {
+      const int idx = min(t + NT * j, TOT - 1), row = idx / NCH, ch = idx % NCH;
+      if (j == 0 || !EVEN) vo_[EVEN ? 0 : j] = (int)(((long long)row * st + ch * 8) * 2);
+      lds_[j] = img_off<D>(row, ch);
+    }
+    step_ = __builtin_amdgcn_readfirstlane((int)(NT / NCH * st * 2));
+    tail_ = t + NT * (CPT - 1) < TOT;
+  }
+  __device__ __forceinline__ void load(u32x4 (&x)[CPT], __amdgpu_buffer_rsrc_t r, int so) const {
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) {  // (a chunk past the last one is a valid one, never stored)
+      const auto a = __builtin_amdgcn_raw_buffer_load_b128(r, vo_[EVEN ? 0 : j], EVEN ? so + j * step_ : so, 0);
+      x[j] = *reinterpret_cast<const u32x4*>(&a);
+    }
+  }
+  __device__ __forceinline__ void store(const u32x4 (&x)[CPT], char* img) const {
+#pragma unroll
+    for (int j = 0; j < CPT; ++j)
+      if (TOT % NT == 0 || j < CPT - 1 || tail_) *reinterpret_cast<u32x4*>(img + lds_[j]) = x[j];
+  }
+};
+
+template <int D>
+__device__ __forceinline__ void clear(f32x16 (&acc)[D / 32]) {
+#pragma unroll
+  for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
+}
+
+template <int D, int G, int RW, int KG, int WPS>
+__global__ void __launch_bounds__(64 * RW * KG, WPS) attn_fwd_split_kernel(FastFwdParams p) {
+  constexpr int BM = 32 * RW, BN = 32, NTG = 64 * RW;
+  constexpr int TILE = BN * D * 2, KS = D / 16;
+  using Stg = GroupStager<D, NTG>;
+  constexpr int CPT = Stg::CPT;
+  constexpr int PART = 32 * D * 4;  // a wave's partial sums
+  static_assert((KG - 1) * RW * PART <= KG * 4 * TILE, "the partial sums take the tiles' place");
+  __shared__ __attribute__((aligned(16))) char smem[KG * 4 * TILE];  // per group [K 0 | K 1 | V 0 | V 1]
+  __shared__ float stat[KG][RW][32][2];                              // reference, sum of each row and group
+  __shared__ int again;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = wave / RW, rw = wave % RW;
+  const int l32 = lane & 31, hh = lane >> 5, gi = lane & 15;
+  const int nqb = (p.Sq + BM - 1) / BM, heads = p.B * p.H;
+  const auto [qi, bh] = block_of<true>(nqb, heads);
+  const int qb = nqb - 1 - qi;
+  const int b = bh / p.H, h = bh % p.H;
+  const int hk = h / (p.H / p.Hkv);
+  if (p.cu) {
+    own_sequence(p, b);
+    if (qb * BM >= p.Sq) return;
+  }
+  const int off = p.Sk - p.Sq;
+  const int q0 = qb * BM + rw * 32, qrow = q0 + l32;
+  const int kv_end = batch_keys(p.kv_len, b, p.Sk);
+  const TileSpan sp = tile_span<BM, true, G == 1 ? 2 : 0>(qb * BM, off, kv_end, p.window);
+  const int ntiles = sp.hi - sp.lo, nsteps = (ntiles + KG - 1) / KG;
+  auto index = [&](int i) { return KG * i + g; };                      // the group's i-th tile, counted along the walk
+  auto key0 = [&](int i) {                                             // its first key
+    const int n = min(index(i), ntiles - 1);
+    return (G == 2 ? sp.hi - 1 - n : sp.lo + n) * BN;
+  };
+  auto mkey0 = [&](int i) { return index(i) < ntiles ? key0(i) : kNoTile; };  // as the mask sees it
+  const float sl2 = p.scale * kLog2e;
+
+  const bf16_t* qp = p.q + b * p.q_sb + h * p.q_sh;
+  const __amdgpu_buffer_rsrc_t rk = head_rsrc(p.k + b * p.k_sb + hk * p.k_sh, rows_bytes(kv_end, p.k_st, D));
+  const __amdgpu_buffer_rsrc_t rv = head_rsrc(p.v + b * p.v_sb + hk * p.v_sh, rows_bytes(kv_end, p.v_st, D));
+  const Stg stk(tid % NTG, p.k_st), stv(tid % NTG, p.v_st);
+  const int kst2 = (int)p.k_st * 2, vst2 = (int)p.v_st * 2;
+  auto at = [](int k0, int st2) { return __builtin_amdgcn_readfirstlane(k0 * st2); };
+  char* const kbuf = smem + g * 4 * TILE;
+  char* const vbuf = kbuf + 2 * TILE;
+  u32x4 xk[CPT], xv[CPT];
+  stk.load(xk, rk, at(key0(0), kst2));  // (flies with the query rows)
+  stv.load(xv, rv, at(key0(0), vst2));
+  bf16x8 qf[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s)
+    qf[s] = *reinterpret_cast<const bf16x8*>(qp + (long long)min(qrow, p.Sq - 1) * p.q_st + 16 * s + 8 * hh);
+
+  const int xr = (l32 >> 2) & 3;
+  const int kb_e = (l32 >> 3) * 16 * D + 64 * (l32 & 7) + 16 * (hh ^ xr);
+  const int kb_o = (l32 >> 3) * 16 * D + 64 * (l32 & 7) + 16 * ((2 + hh) ^ xr);
+  const int c3 = 2 * ((lane >> 4) & 1) + ((gi & 3) >> 1);
+  const int vb_1 = 64 * (4 * hh + (gi >> 2)) + 16 * (c3 ^ hh) + 8 * (gi & 1);
+  const int vb_2 = 16 * D + 64 * (4 * hh + (gi >> 2)) + 16 * (c3 ^ hh ^ 2) + 8 * (gi & 1);
+  auto qk = [&](const char* Ks) {
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    bf16x8 fa[3];  // K fragments two k-steps ahead of their MFMA (pinned)
+    fa[0] = lds_b128(Ks, kb_e);
+    fa[1] = lds_b128(Ks, kb_o);
+    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      if (s + 2 < KS) {
+        fa[(s + 2) % 3] = lds_b128(Ks, (((s + 2) & 1) ? kb_o : kb_e) + 512 * ((s + 2) >> 1));
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[s % 3], qf[s], acc, 0, 0, 0);
+      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+    }
+    return acc;
+  };
+  const int last = min(qrow + off, kv_end - 1);              // row's last visible key
+  const int before = p.window > 0 ? qrow + off - p.window : -(1 << 30);            // key before its first
+  auto mask = [&](f32x16& acc, int k0) {
+    const int lim = last - k0 - 4 * hh, lo = before - k0 - 4 * hh;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int c = (r & 3) + 8 * (r >> 2);
+      if (c > lim || c <= lo) acc[r] = -INFINITY;
+    }
+  };
+  const float slope = G == 2 ? p.alibi[h] * kLog2e : 0.f;
+  auto biased = [&](float s, int r, int k0) {  // score in log2 units
+    return G == 2 ? fmaf(s, sl2, fmaf(slope, (float)((r & 3) + 8 * (r >> 2)), slope * (float)(k0 + 4 * hh - qrow - off))) : s * sl2;
+  };
+
+  if (tid == 0) again = 0;
+  f32x16 oacc[D / 32];
+  float m = -INFINITY, lsum = 0.f;
+  bool begun = false;  // G == 1: a tile with a visible key of this row has been walked
+  for (int pass = 0;; ++pass) {
+    if (pass > 0) {  // a sum passed 2^100: the group's true maximum first
+      m = -INFINITY;
+      begun = true;
+      for (int i = 0; i < nsteps; ++i) {
+        stk.load(xk, rk, at(key0(i), kst2));
+        stk.store(xk, kbuf);
+        __syncthreads();
+        f32x16 s = qk(kbuf);
+        mask(s, mkey0(i));
+#pragma unroll
+        for (int r = 0; r < 16; ++r) m = fmaxf(m, s[r] == -INFINITY ? -INFINITY : biased(s[r], r, key0(i)));
+        __syncthreads();
+      }
+      m = fmaxf(m, __shfl_xor(m, 32, 64));
+      stk.load(xk, rk, at(key0(0), kst2));
+      stv.load(xv, rv, at(key0(0), vst2));
+    }
+    clear<D>(oacc);
+    lsum = 0.f;
+    float nm = pass == 0 || m == -INFINITY ? 0.f : -m;
+    stk.store(xk, kbuf);
+    stv.store(xv, vbuf);
+    stk.load(xk, rk, at(key0(1), kst2));
+    stk.store(xk, kbuf + TILE);
+    __syncthreads();
+    f32x16 sa = qk(kbuf);
+
+    auto step = [&](int i, auto masked) {
+      constexpr bool MASKED = decltype(masked)::value, HEAD = decltype(masked)::value == 2;
+      const int k0 = key0(i), mk0 = mkey0(i);
+      stk.load(xk, rk, at(key0(i + 2), kst2));
+      stv.load(xv, rv, at(key0(i + 1), vst2));
+      asm volatile("" ::: "memory");  // (the loads stay above the products, their LDS stores below)
+      f32x16 sb = qk(kbuf + ((i + 1) & 1) * TILE);  // S of the group's next tile (unused after the last)
+      float sl = sl2, bias[16];  // P = exp2(s * sl + bias)
+      if constexpr (G == 2) {
+        const float b0 = slope * (float)(k0 + 4 * hh - qrow - off) + (MASKED ? 0.f : nm);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) bias[r] = fmaf(slope, (float)((r & 3) + 8 * (r >> 2)), b0);
+      }
+      if constexpr (MASKED) {
+        mask(sa, mk0);
+        float mt = -INFINITY, m_here = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          sa[r] = G == 2 ? fmaf(sa[r], sl2, bias[r]) : sa[r] * sl2;
+          mt = fmaxf(mt, sa[r]);
+        }
+        if constexpr (HEAD) {  // (the next tile's scores are at hand and may be the row's largest)
+          m_here = fmaxf(mt, __shfl_xor(mt, 32, 64));
+          const int nk0 = mkey0(i + 1), lim = last - nk0 - 4 * hh, lo = before - nk0 - 4 * hh;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int c = (r & 3) + 8 * (r >> 2);
+            mt = fmaxf(mt, c > lim || c <= lo ? -INFINITY : sb[r] * sl2);
+          }
+        }
+        mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+        m = m == -INFINITY || (HEAD && !begun) ? mt : m;
+        if constexpr (HEAD) begun = begun || m_here > -INFINITY;
+        nm = m == -INFINITY ? 0.f : -m;
+        sl = 1.f;
+      }
+      if constexpr (G < 2 || MASKED) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) bias[r] = nm;
+      }
+      float ps = 0.f;
+      bf16x8 pf0, pf1;
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const float e0 = __builtin_amdgcn_exp2f(fmaf(sa[r], sl, bias[r]));
+        const float e1 = __builtin_amdgcn_exp2f(fmaf(sa[r + 8], sl, bias[r + 8]));
+        ps += e0 + e1;
+        pf0[r] = (__bf16)e0;
+        pf1[r] = (__bf16)e1;
+      }
+      lsum += ps;
+      const char* Vs = vbuf + (i & 1) * TILE;
+      auto vfrag = [&](int db, int s) {
+        return cat8(lds_tr4(Vs, vb_1 + 2 * s * 16 * D + 512 * db), lds_tr4(Vs, vb_2 + 2 * s * 16 * D + 512 * db));
+      };
+      bf16x8 va[2], vb[2];
+      va[0] = vfrag(0, 0);
+      vb[0] = vfrag(0, 1);
+      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+      for (int db = 0; db < D / 32; ++db) {
+        if (db + 1 < D / 32) {
+          va[(db + 1) & 1] = vfrag(db + 1, 0);
+          vb[(db + 1) & 1] = vfrag(db + 1, 1);
+          __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+        }
+        oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[db & 1], pf0, oacc[db], 0, 0, 0);
+        oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vb[db & 1], pf1, oacc[db], 0, 0, 0);
+        __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
+      }
+      sa = sb;
+      asm volatile("" ::: "memory");
+      stk.store(xk, kbuf + (i & 1) * TILE);
+      stv.store(xv, vbuf + ((i + 1) & 1) * TILE);
+      __syncthreads();
+    };
+    if constexpr (G == 1) {
+      // Steps whose KG tiles may hold a row's first visible key of their group: below f_lo the rows' first ones, up to
+      // KG - 1 tiles on the other groups'. Free ones lie whole at or below f_hi.
+      const int head = min(nsteps, (sp.f_lo - sp.lo + 2 * KG - 2) / KG);
+      const int top = max(head, min(nsteps, (min(sp.f_hi + 1, sp.hi) - sp.lo) / KG));
+      for (int i = 0; i < head; ++i) step(i, std::integral_constant<int, 2>{});
+      for (int i = head; i < top; ++i) step(i, std::false_type{});
+      for (int i = top; i < nsteps; ++i) step(i, std::true_type{});
+    } else {
+      // from the last tile down: a row's last visible key lies above f_hi, another group's up to KG - 1 tiles below
+      const int top = min(nsteps, (sp.hi - 1 - sp.f_hi + 2 * KG - 2) / KG);
+      const int low = max(top, min(sp.hi - sp.f_lo, ntiles) / KG);
+      for (int i = 0; i < top; ++i) step(i, std::true_type{});
+      for (int i = top; i < low; ++i) step(i, std::false_type{});
+      for (int i = low; i < nsteps; ++i) step(i, std::true_type{});
+    }
+
+    // the groups' sums meet (the tiles are no longer read: the last step's barrier)
+    const float ltot = lsum + __shfl_xor(lsum, 32, 64);
+    const bool bad = !(ltot < 1.2676506e30f) && qrow < p.Sq;
+    if (pass == 0 && __any(bad) && lane == 0) again = 1;
+    if constexpr (KG > 1) {
+      if (g > 0) put_partial<D>(smem + ((g - 1) * RW + rw) * PART, oacc, lane);
+      if (hh == 0) {
+        stat[g][rw][l32][0] = m;
+        stat[g][rw][l32][1] = ltot;
+      }
+    }
+    lsum = ltot;
+    __syncthreads();
+    if (pass > 0 || !__builtin_amdgcn_readfirstlane(again)) break;
+  }
+  if (KG > 1 && g > 0) return;
+  float mm = m, l = lsum;
+  if constexpr (KG > 1) {
+#pragma unroll
+    for (int i = 1; i < KG; ++i) mm = fmaxf(mm, stat[i][rw][l32][0]);
+    auto weight = [&](float x) { return x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(x - mm); };
+    const float w0 = weight(m);
+    l *= w0;
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) oacc[db][r] *= w0;
+#pragma unroll
+    for (int i = 1; i < KG; ++i) {
+      const float w = weight(stat[i][rw][l32][0]);
+      l = fmaf(stat[i][rw][l32][1], w, l);
+      add_partial<D>(smem + ((i - 1) * RW + rw) * PART, oacc, lane, w);
+    }
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  if (hh == 0 && p.lse && qrow < p.Sq) p.lse[((long long)b * p.H + h) * p.Sq + qrow] = l > 0.f ? (mm + log2f(l)) * kLn2 : INFINITY;
+  asm volatile("" ::: "memory");  // (the image lies on the partial sums that this wave alone has read)
+  store_tile_lds<D, D, true>(p.o + b * p.o_sb + h * p.o_sh + (long long)q0 * p.o_st, p.o_st, oacc, lane, inv, smem + rw * (KG > 1 ? PART : PART / 2),
+                             p.Sq - q0);
+}
+
+}  // namespace
+
+// Which calls are split in two groups (two waves of 32 rows each, 4 waves a workgroup), the others in blocks of 128 rows and
+// one group. One MI355X, us, one group against two; blocks: 128-row blocks of all heads.
+//   forward, 64 wide:   2 x 889 x 16 heads (224 blocks) 19.4, 14.8; 1 x 4000 x 12 (384) 61.6, 45.8; 15 x 256 x 16 (480) 11.9, 15.3;
+//                       2 x 2688 x 12 (504) 45.3, 41.8; 3 x 2048 x 12 (576) 39.2, 35.2; 10 x 577 x 12 (600) 18.3, 21.9
+//   96 wide:            1 x 700 x 32 (192) 19.4, 16.0; 5 x 256 x 32 (320) 14.3, 18.4; 1 x 1403 x 32 (352) 33.8, 31.2; 768: 51, 61
+//   128 wide:           1 x 2048 x 14 with ALiBi (224) 48.7, 41.2; 2 x 896 x 20 (280) 27.9, 24.6; 2 x 1346 x 20 (440) 37.1, 43.0
+static bool split_rows(long long blocks, int d, int rows) {
+  return blocks <= (d == 64 ? (rows >= 1536 ? 640 : 448) : d == 96 ? (rows >= 1024 ? 400 : 256) : 320);
+}
+
+template <class F>
+static int with_form(int d, bool alibi, F&& f) {
+  auto mask = [&](auto D) {
+    if (alibi) f(D, std::integral_constant<int, 2>{});
+    else f(D, std::integral_constant<int, 1>{});
+  };
+  switch (d) {
+    case 64: mask(std::integral_constant<int, 64>{}); break;
+    case 96: mask(std::integral_constant<int, 96>{}); break;
+    case 128: mask(std::integral_constant<int, 128>{}); break;
+    default: return 1;
+  }
+  return hipGetLastError() == hipSuccess ? 0 : 3;
+}
+
+// Causal calls of 64, 96 and 128 wide heads with 16-byte rows; 1: another head size.
+int attn_fwd_split(const FastFwdParams& p, int d, hipStream_t stream) {
+  const long long blocks = (long long)((p.Sq + 127) / 128) * p.B * p.H;
+  const bool two = split_rows(blocks, d, p.Sq);
+  return with_form(d, p.alibi, [&](auto D_, auto G_) {
+    constexpr int D = decltype(D_)::value, G = decltype(G_)::value, W = D == 64 ? 3 : 2;
+    if (two)
+      hipLaunchKernelGGL((attn_fwd_split_kernel<D, G, 2, 2, W>), dim3((p.Sq + 63) / 64 * p.B * p.H), dim3(256), 0, stream, p);
+    else
+      hipLaunchKernelGGL((attn_fwd_split_kernel<D, G, 4, 1, W>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
+  });
+}

@@ -23,12 +23,13 @@
 // tile's global loads in flight under the current tile's MFMAs (T14); online
 // softmax lane-local (query on the lane), max/row-sum in exp2 units with the
 // scale folded into one FMA, deferred rescale (T13, threshold 8).
-#include "attn_tile.h"
+#include "attn_fast.h"
 
 #include <type_traits>
 
-namespace {
+int attn_fwd_split(const FastFwdParams& p, int d, hipStream_t stream);  // attention_split.hip
 
+namespace {
 
 // Diagnostic build only (-DKCA_ATTN_STAMPS, bench/attn_stamps.py): per-wave s_memtime segment
 // sums of the main loops, added into g_attn_stamps once per wave at the end (fwd slots 0..7,
@@ -68,67 +69,6 @@ __device__ __forceinline__ unsigned long long ast_now() {
   } while (0)
 #endif
 
-
-struct FastFwdParams {
-  const bf16_t* q; const bf16_t* k; const bf16_t* v;
-  bf16_t* o; float* lse;
-  int* flags;  // [grid * 4]: 1 = this wave's rows overflowed -> fixup kernel
-  long long q_sb, q_st, q_sh, k_sb, k_st, k_sh, v_sb, v_st, v_sh;
-  long long o_sb, o_st, o_sh;
-  int B, Sq, Sk, H, Hkv;
-  float scale;
-  const float* alibi;  // [H] slopes (G = 2)
-  const int* kv_len;   // [B] or null (G > 0)
-  int window;          // > 0: key visible only if key > q + off - window (G > 0)
-  const int* cu;       // [B + 1] or null (G > 0): packed sequences -- batch b is rows cu[b] .. cu[b + 1], the batch
-                       // strides are 0, Sq is the longest's length and lse null
-};
-
-__device__ __forceinline__ void own_sequence(FastFwdParams& p, int b) {
-  const int c0 = p.cu[b];
-  p.Sq = p.Sk = p.cu[b + 1] - c0;
-  p.q += c0 * p.q_st;
-  p.k += c0 * p.k_st;
-  p.v += c0 * p.v_st;
-  p.o += c0 * p.o_st;
-}
-
-constexpr int kAllRows = 0x7fffffff;
-
-// buffer resource over one (batch, head) slice; the base is workgroup-uniform (readfirstlane'd so
-// the descriptor is provably scalar: no waterfall loop, T20). `bytes`: loads at or past it return zeros.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t head_rsrc(const bf16_t* b, int bytes = kAllRows) {
-  const unsigned long long a = (unsigned long long)b;
-  const unsigned long long au = ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(a >> 32)) << 32) |
-                                (unsigned)__builtin_amdgcn_readfirstlane((unsigned)a);
-  return __builtin_amdgcn_make_buffer_rsrc((void*)au, (short)0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
-}
-// bytes of `rows` rows of D elements, `st` elements apart
-__device__ __forceinline__ int rows_bytes(int rows, long long st, int D) {
-  return rows > 0 ? (int)(((rows - 1) * st + D) * 2) : 0;
-}
-
-// The 32-key tiles of a workgroup's query rows [r0, r0 + BM) in the general forms: it walks tiles [lo, hi),
-// of which [f_lo, f_hi] need no mask. A row's last visible key lies in a tile above f_hi. For a row's first one, f_lo counts
-// EDGE more tiles: 1, f_lo > lo and it lies in a tile below f_lo or at the start of f_lo; 2, below f_lo. At least one tile,
-// also where no key is visible (a length of 0): its mask gives zeros.
-struct TileSpan { int lo, hi, f_lo, f_hi; };
-template <int BM, bool CAUSAL, int EDGE = 0>
-__device__ __forceinline__ TileSpan tile_span(int r0, int off, int kv_end, int window) {
-  TileSpan s;
-  s.hi = max(1, ((CAUSAL ? min(kv_end, r0 + BM + off) : kv_end) + 31) / 32);
-  s.f_hi = (CAUSAL ? min(r0 + off, kv_end - 1) : kv_end - 1) / 32 - 1;
-  s.lo = s.f_lo = 0;
-  if (window > 0) {
-    s.lo = min(s.hi - 1, max(0, r0 + off - window + 1) / 32);
-    s.f_lo = max(0, r0 + BM + off - window + (EDGE < 2 ? 31 : 32)) / 32;
-  }
-  if (EDGE) s.f_lo = max(s.f_lo, s.lo + 1);
-  return s;
-}
-__device__ __forceinline__ int batch_keys(const int* kv_len, int b, int Sk) {
-  return kv_len ? max(0, min(Sk, kv_len[b])) : Sk;
-}
 
 // Staging of a 32-row x D tile by the 256 threads of a workgroup: chunk idx = tid + 256*i is
 // (row idx / NCH, 16-B chunk idx % NCH). D = 96 / 160 serve SD-1.5's 80-wide heads (padded to
@@ -309,38 +249,6 @@ struct StagerNarrow {
 template <int D, int DS>
 using StagerFor = std::conditional_t<DS == D, Stager<D>, StagerNarrow<D, DS>>;
 
-// Epilogue through LDS (cdna_hip_programming.md T21): the wave's 32 x D accumulator tile (row =
-// lane & 31) goes into a wave-private [32][D] bf16 LDS image -- 16-B chunks rotated by the row,
-// so the per-lane 8-B writes and the row-contiguous 16-B reads are both conflict-free -- and every
-// store instruction then writes two whole rows with 16-B stores, instead of 8-B stores that each
-// touch 64 rows. `mul` is the lane's row scale. The LDS must be free (after the loop's barrier).
-// EDGE: only the first `rows` rows exist.
-template <int D, int DS = D, bool EDGE = false>
-__device__ __forceinline__ void store_tile_lds(bf16_t* row0, long long st, const f32x16 (&acc)[D / 32], int lane,
-                                               float mul, char* lds, int rows = 32) {
-  constexpr int NCH = D / 8, RB = D * 2, NCS = DS / 8;  // NCS: stored chunks per row
-  const int l32 = lane & 31, hh = lane >> 5;
-#pragma unroll
-  for (int db = 0; db < D / 32; ++db) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      uint2 w;
-      w.x = pk_bf16(acc[db][4 * g] * mul, acc[db][4 * g + 1] * mul);
-      w.y = pk_bf16(acc[db][4 * g + 2] * mul, acc[db][4 * g + 3] * mul);
-      *reinterpret_cast<uint2*>(lds + l32 * RB + ((4 * db + g + l32) % NCH) * 16 + hh * 8) = w;
-    }
-  }
-  asm volatile("" ::: "memory");  // the wave's LDS accesses execute in order: reads see its writes
-  static_assert((32 * NCS) % 64 == 0, "whole-wave epilogue rounds");
-#pragma unroll
-  for (int j = 0; j < 32 * NCS / 64; ++j) {
-    const int idx = j * 64 + lane, r = idx / NCS, c = idx % NCS;
-    const uint4 v = *reinterpret_cast<const uint4*>(lds + r * RB + ((c + r) % NCH) * 16);
-    if (!EDGE || r < rows) *reinterpret_cast<uint4*>(row0 + (long long)r * st + c * 8) = v;
-  }
-  asm volatile("" ::: "memory");
-}
-
 // OC >= 0 ("ones column"): V's zero-padded column OC holds 1.0 for every key (the SD UNet's
 // padded QKV GEMM writes it through its bias), so O^T row OC accumulates the softmax row sum
 // sum_k bf16(P) on the matrix pipe: the per-element f32 adds of the row sum leave the VALU, which
@@ -372,10 +280,9 @@ __global__ void __launch_bounds__(256, (D <= 160 ? 2 : 1)) attn_fwd_tiled_kernel
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5, gi = lane & 15;
   const int nqb = (p.Sq + BM - 1) / BM;
-  const int lid = xcd_remap(blockIdx.x, gridDim.x);
-  const int qi = lid % nqb;
+  const auto [qi, bh] = block_of<CAUSAL>(nqb, p.B * p.H);
+  const int lid = bh * nqb + qi;  // (the order of the fixup kernel's flags)
   const int qb = CAUSAL ? (nqb - 1 - qi) : qi;
-  const int bh = lid / nqb;
   const int b = bh / p.H, h = bh % p.H;
   const int hk = h / (p.H / p.Hkv);
   if constexpr (G > 0) {
@@ -741,46 +648,46 @@ __device__ __forceinline__ bf16x8 as_bf8(u32x2 lo, u32x2 hi) {
 // SIMD, O^T = 256 registers, Q^T fragments 128; two 64-KiB stages, the next tile's DMA in flight
 // under the current tile). Inference only: the overflow flags go back to the caller, which has no
 // generic D = 512 kernel to fix rows up with and reruns flagged calls on the GEMM path.
-template <int D, bool CAUSAL, int NW = 8, int NBUF = 4, int G = 0>
+template <int D, bool CAUSAL, int NW = 8, int NBUF = 4, int G = 0, int KG = 1>
 __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p) {
-  constexpr int BM = NW * 32, BN = 32;
+  constexpr int RW = NW / KG;                 // waves a group: its 32-row slices
+  constexpr int BM = RW * 32, BN = 32;
   constexpr int TILE = BN * D * 2;            // one K or V image
   constexpr int STAGE = 2 * TILE;
   constexpr int KS = D / 16;
   constexpr int PIECES = TILE / 1024;         // 1-KiB LDS-DMA pieces per image
   constexpr int PPW = PIECES / NW;            // per wave per image
-  constexpr int LEAD = NBUF - 1;                  // tiles issued ahead of the one computed
-  constexpr int INFLIGHT = (LEAD - 1) * 2 * PPW;  // DMA instructions issued after tile t when t is waited
+  constexpr int LEAD = NBUF / KG - 1;                  // steps (of KG tiles) issued ahead of the one computed
+  constexpr int INFLIGHT = (LEAD - 1) * KG * 2 * PPW;  // DMA instructions issued after a step's when it is waited for
+  constexpr bool AGAIN = D != 512;                     // overflowed rows are computed again here
   static_assert(((D == 256 || D == 128) && NW == 8) || (D == 512 && NW == 4 && NBUF == 2 && !CAUSAL),
                 "multi-wave LDS-DMA forward: 8 waves at D = 128 / 256, 4 waves at D = 512");
   static_assert(PPW >= 1 && PIECES % NW == 0, "whole pieces per wave");
+  static_assert(NBUF % KG == 0 && LEAD >= 1 && (KG == 1 || G > 0), "groups: general forms, two steps of buffers");
   constexpr int SMEM = (NBUF * STAGE > NW * 32 * D * 2) ? NBUF * STAGE : NW * 32 * D * 2;
+  constexpr int PART = 32 * D * 4;  // a wave's partial sums
+  static_assert((KG - 1) * RW * PART <= SMEM, "the partial sums take the tiles' place");
   __shared__ __attribute__((aligned(1024))) char smem[SMEM];  // [buf][K|V]; epilogue: [wave][32][D]
+  __shared__ float stat[KG > 1 ? KG : 1][RW][32][2];          // reference, sum of each row and group
+  __shared__ int again;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hh = lane >> 5;
+  const int g = KG > 1 ? wave / RW : 0, rw = KG > 1 ? wave % RW : wave;
   const int nqb = (p.Sq + BM - 1) / BM;
-  const int lid = xcd_remap(blockIdx.x, gridDim.x);
-  const int qi = lid % nqb;
+  const auto [qi, bh] = block_of<CAUSAL>(nqb, p.B * p.H);
   const int qb = CAUSAL ? (nqb - 1 - qi) : qi;
-  const int bh = lid / nqb;
   const int b = bh / p.H, h = bh % p.H;
   const int hk = h / (p.H / p.Hkv);
-  // overflow flags in the 4-wave kernel's layout (4 per 128-row block, lid order of the generic fixup)
-  const int nqb128 = (p.Sq + 127) / 128, qb128 = (qb * BM + wave * 32) / 128;
-  int* flag = p.flags + (bh * nqb128 + (CAUSAL ? nqb128 - 1 - qb128 : qb128)) * 4 + wave % 4;
   if constexpr (G > 0) {
     if (p.cu) {
       own_sequence(p, b);
-      if (qb * BM >= p.Sq) {
-        if (lane == 0 && qb128 < nqb128) *flag = 0;
-        return;
-      }
+      if (qb * BM >= p.Sq) return;
     }
   }
   const int off = p.Sk - p.Sq;
-  const int q0 = qb * BM + wave * 32;
+  const int q0 = qb * BM + rw * 32;
   const int qrow = q0 + l32;
   const int kv_end = G ? batch_keys(p.kv_len, b, p.Sk) : p.Sk;
   int kv_hi = kv_end;
@@ -823,8 +730,9 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
   }
   typedef __attribute__((address_space(3))) char lds_char;
   lds_char* lsm = (lds_char*)smem;
-  auto issue = [&](int tile, int buf) {
-    int kt = min(tile, ntiles - 1);  // clamped: the last tiles re-load a tile nobody reads
+  auto issue = [&](int n) {  // n-th tile walked
+    const int buf = n % NBUF;
+    int kt = min(n, ntiles - 1);  // clamped: the last tiles re-load a tile nobody reads
     if constexpr (G > 0) kt = G == 2 ? sp.hi - 1 - kt : sp.lo + kt;
     const int sok = __builtin_amdgcn_readfirstlane(kt * BN * (int)p.k_st * 2);
     const int sov = __builtin_amdgcn_readfirstlane(kt * BN * (int)p.v_st * 2);
@@ -859,12 +767,16 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
   const unsigned vb_2 = TILE + 16 * D + 64 * (4 * hh + (gi >> 2)) + 16 * (c3 ^ hh ^ 2) + 8 * (gi & 1);
 
   ASTAMP_DECL
+  const int nsteps = (ntiles + KG - 1) / KG;
+  auto issue_step = [&](int i) {
 #pragma unroll
-  for (int t = 0; t < LEAD; ++t) issue(t, t);
+    for (int j = 0; j < KG; ++j) issue(KG * i + j);
+  };
+  int pass = 0;  // 1: once more, with the rows' true maxima
 
   bf16x8 pf0, pf1;  // P^T of the tile in flight (softmax -> PV)
-  // S^T = K.Q^T of tile t (K row fragments two k-steps ahead of their MFMA), softmax into pf0/pf1
-  auto sm_part = [&](int buf, auto masked, int t) {
+  // S^T = K.Q^T of tile t (K row fragments two k-steps ahead of their MFMA)
+  auto scores = [&](int buf, auto masked, int t) {
     constexpr bool MASKED = decltype(masked)::value;
     const unsigned st0 = sbase + buf * STAGE;
     const unsigned ke = st0 + kb_e, ko = st0 + kb_o;
@@ -899,8 +811,13 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
           if ((r & 3) + 8 * (r >> 2) <= lo) sa[r] = -INFINITY;
       }
     }
-    // reference max = the first tile's row max (see attn_fwd_tiled_kernel)
-    if (G == 2 ? t > own.f_hi : G ? t < own.f_lo : t == 0) {
+    return sa;
+  };
+  // softmax into pf0/pf1
+  auto sm_part = [&](int buf, auto masked, int t) {
+    f32x16 sa = scores(buf, masked, t);
+    // reference max = the first tile's row max (see attn_fwd_tiled_kernel; of a group: up to KG - 1 tiles on)
+    if (G == 2 ? t > own.f_hi - (KG - 1) : G ? t < own.f_lo + KG - 1 : t == 0 && pass == 0) {
       float mt = sa[0];
 #pragma unroll
       for (int r = 1; r < 16; ++r) mt = fmaxf(mt, sa[r]);
@@ -958,41 +875,98 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
   // t+LEAD, compute. Measured and not kept (same-box A/B, GPT-J fwd): a ping-pong schedule (waves 4-7
   // one PV behind, so the two waves of a SIMD never sit in softmax together; two tiles ahead) 5 %
   // slower; two tiles per barrier (vmcnt(0), one superstep ahead) 3-5 % slower.
-  auto sync_issue = [&](int t) {
+  auto sync_issue = [&](int i) {
     ASTAMP(0);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(INFLIGHT) : "memory");
     __builtin_amdgcn_s_barrier();
     ASTAMP(1);
-    issue(t + LEAD, (t + LEAD) % NBUF);
+    issue_step(i + LEAD);
     ASTAMP(2);
   };
   // causal: the mask is applied on every tile (16 selects that change nothing before the diagonal):
   // separate masked / mask-free bodies made hipcc spill ~170 registers
   constexpr auto CM = std::integral_constant<bool, (CAUSAL || G > 0)>{};
-  for (int t = 0; t < ntiles; ++t) {
-    sync_issue(t);
-    const int tile = G == 2 ? sp.hi - 1 - t : sp.lo + t;
-    if (G ? tile < own.hi && tile >= own.lo : t < mytiles) {
-      sm_part(t % NBUF, CM, G ? tile : t);
-      pv_part(t % NBUF);
+  auto walk = [&](auto&& f) {  // f(buffer, tile) for this wave's tiles
+#pragma unroll
+    for (int t = 0; t < LEAD; ++t) issue_step(t);
+    for (int i = 0; i < nsteps; ++i) {
+      sync_issue(i);
+      const int n = KG * i + g;
+      const int tile = G == 2 ? sp.hi - 1 - n : sp.lo + n;
+      if (G ? n < ntiles && tile < own.hi && tile >= own.lo : n < mytiles) f(n % NBUF, G ? tile : n);
     }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // the clamped tail DMAs
+  };
+  float ltot;
+  if (AGAIN && tid == 0) again = 0;
+  for (;; ++pass) {
+    walk([&](int buf, int tile) {
+      sm_part(buf, CM, tile);
+      pv_part(buf);
+    });
+    ltot = lsum + __shfl_xor(lsum, 32, 64);
+    const bool bad = !(ltot < 1.2676506e30f) && (!G || qrow < p.Sq);
+    const int any_bad = __any(bad);
+    if constexpr (!AGAIN) {
+      // overflow flags, 4 per 128-row block
+      if (lane == 0) p.flags[(bh * nqb + qi) * 4 + wave] = any_bad;
+      break;
+    }
+    if (pass == 0 && any_bad && lane == 0) again = 1;
+    __syncthreads();  // (the tiles are read)
+    if (pass > 0 || !__builtin_amdgcn_readfirstlane(again)) break;
+    m = -INFINITY;
+    walk([&](int buf, int tile) {
+      const f32x16 sa = scores(buf, CM, tile);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) m = fmaxf(m, G == 2 ? sa[r] : sa[r] * sl2);
+    });
+    m = fmaxf(m, __shfl_xor(m, 32, 64));
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) oacc[i][r] = 0.f;
+    lsum = rsum = 0.f;
   }
 
-  const float ltot = lsum + __shfl_xor(lsum, 32, 64);
-  const bool bad = !(ltot < 1.2676506e30f) && (!G || qrow < p.Sq);
-  const int any_bad = __any(bad);
-  if (lane == 0 && (!G || qb128 < nqb128)) *flag = any_bad;
+  float rtot = G == 1 && p.window > 0 ? rsum + __shfl_xor(rsum, 32, 64) : ltot;
+  if constexpr (KG > 1) {  // the groups' sums meet (attention_split.hip)
+    if (g > 0) put_partial<D>(smem + ((g - 1) * RW + rw) * PART, oacc, lane);
+    if (hh == 0) {
+      stat[g][rw][l32][0] = m;
+      stat[g][rw][l32][1] = ltot;
+    }
+    __syncthreads();
+    if (g > 0) return;
+    const float m0 = m;
+#pragma unroll
+    for (int i = 1; i < KG; ++i) m = fmaxf(m, stat[i][rw][l32][0]);
+    auto weight = [&](float x) { return x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(x - m); };
+    const float w0 = weight(m0);
+    ltot *= w0;
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) oacc[db][r] *= w0;
+#pragma unroll
+    for (int i = 1; i < KG; ++i) {
+      const float w = weight(stat[i][rw][l32][0]);
+      ltot = fmaf(stat[i][rw][l32][1], w, ltot);
+      add_partial<D>(smem + ((i - 1) * RW + rw) * PART, oacc, lane, w);
+    }
+    rtot = ltot;
+  }
   // With a window a row's first tile holds 16 of its keys on average: the reference is its largest weight less often than
   // elsewhere (attn_fwd_tiled_kernel). Dividing by the rounded weights makes up for it: error against 64 bits of 2 x 1000 x 16
   // heads, window 256, 0.00213 -> 0.00210 (generic kernel 0.00212). lse keeps the sum of the unrounded ones.
-  const float div = G == 1 && p.window > 0 ? rsum + __shfl_xor(rsum, 32, 64) : ltot;
-  const float inv = ltot > 0.f ? 1.f / div : 0.f;
+  const float inv = ltot > 0.f ? 1.f / rtot : 0.f;
   if (hh == 0 && p.lse && (!G || qrow < p.Sq))
     p.lse[((long long)b * p.H + h) * p.Sq + qrow] = ltot > 0.f ? (m + log2f(ltot)) * kLn2 : INFINITY;
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // the clamped tail DMAs
-  __syncthreads();  // the tile buffers become the epilogue images
+  if constexpr (!AGAIN) __syncthreads();  // the tile buffers become the epilogue images
+  asm volatile("" ::: "memory");
   store_tile_lds<D, D, (G > 0)>(p.o + b * p.o_sb + h * p.o_sh + (long long)q0 * p.o_st, p.o_st, oacc, lane, inv,
-                                smem + wave * 32 * D * 2, p.Sq - q0);
+                                smem + rw * (KG > 1 ? PART : PART / 2), p.Sq - q0);
   ASTAMP(6);
   ASTAMP_FLUSH(48);
 }
@@ -1013,46 +987,6 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
 //                tiles (and the query heads of its KV head for GQA).
 //                S = Q.K^T, dP = dO.V^T (key on the lane), dV^T += dO^T.P,
 //                dK^T += Q^T.dS with dO^T, Q^T by transposed reads.
-struct FastBwdParams {
-  const bf16_t* q; const bf16_t* k; const bf16_t* v; const bf16_t* dout;
-  bf16_t* dq; bf16_t* dk; bf16_t* dv;
-  const float* lse; float* delta;
-  long long q_sb, q_st, q_sh, k_sb, k_st, k_sh, v_sb, v_st, v_sh, do_sb, do_st, do_sh;
-  long long dq_sb, dq_st, dq_sh, dk_sb, dk_st, dk_sh, dv_sb, dv_st, dv_sh;
-  int B, Sq, Sk, H, Hkv;
-  float scale;
-  const float* alibi;  // as in FastFwdParams
-  const int* kv_len;
-  int window;
-  const bf16_t* o;
-  long long o_sb, o_st, o_sh;
-};
-
-// A operand (32 rows x 16 k) read by rows from an image: lane (row l32, half hh)
-// takes chunk 2s+hh of its row. Returns the two per-lane bases (s even / odd).
-template <int D>
-__device__ __forceinline__ void row_bases(int l32, int hh, int& e, int& o) {
-  const int xr = (l32 >> 2) & 3;
-  e = (l32 >> 3) * 16 * D + 64 * (l32 & 7) + 16 * (hh ^ xr);
-  o = (l32 >> 3) * 16 * D + 64 * (l32 & 7) + 16 * ((2 + hh) ^ xr);
-}
-// transposed A operand (32 columns x 16 permuted rows) from an image
-template <int D>
-__device__ __forceinline__ void tr_bases(int lane, int& b1, int& b2) {
-  const int hh = lane >> 5, gi = lane & 15;
-  const int c3 = 2 * ((lane >> 4) & 1) + ((gi & 3) >> 1);
-  b1 = 64 * (4 * hh + (gi >> 2)) + 16 * (c3 ^ hh) + 8 * (gi & 1);
-  b2 = 16 * D + 64 * (4 * hh + (gi >> 2)) + 16 * (c3 ^ hh ^ 2) + 8 * (gi & 1);
-}
-template <int D>
-__device__ __forceinline__ bf16x8 tr_frag(const char* img, int b1, int b2, int s, int db) {
-  return cat8(lds_tr4(img, b1 + 2 * s * 16 * D + 512 * db), lds_tr4(img, b2 + 2 * s * 16 * D + 512 * db));
-}
-template <int D>
-__device__ __forceinline__ bf16x8 row_frag(const char* img, int be, int bo, int s) {
-  return lds_b128(img, ((s & 1) ? bo : be) + 512 * (s >> 1));
-}
-
 // store a D/32 x f32x16 transposed accumulator (row d, column = lane token) as
 // bf16 row `tok` of a [.., D] tensor, times `mul`
 template <int D>
@@ -1090,10 +1024,8 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 4 : D <= 64 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5;
   const int nqb = (p.Sq + BM - 1) / BM;
-  const int lid = xcd_remap(blockIdx.x, gridDim.x);
-  const int qi = lid % nqb;
+  const auto [qi, bh] = block_of<CAUSAL>(nqb, p.B * p.H);
   const int qb = CAUSAL ? (nqb - 1 - qi) : qi;
-  const int bh = lid / nqb;
   const int b = bh / p.H, h = bh % p.H;
   const int hk = h / (p.H / p.Hkv);
   const int off = p.Sk - p.Sq;
@@ -1284,8 +1216,7 @@ __global__ void __launch_bounds__(256, D <= 64 ? 3 : D <= 128 ? 2 : 1) attn_bwd_
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5;
   const int nkb = (p.Sk + BK - 1) / BK;
-  const int lid = xcd_remap(blockIdx.x, gridDim.x);
-  const int kb = lid % nkb, bh = lid / nkb;
+  const auto [kb, bh] = block_of<CAUSAL>(nkb, p.B * p.Hkv);
   const int b = bh / p.Hkv, hk = bh % p.Hkv;
   const int grp = p.H / p.Hkv;
   const int off = p.Sk - p.Sq;
@@ -1572,6 +1503,12 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
                   B, Sq, Sk, H, Hkv, scale, alibi, kv_len, window, cu};
   dim3 grid(((Sq + 127) / 128) * B * H);
   (void)hipGetLastError();
+  const bool aligned = rows16(q, q_sb, q_st, q_sh) && rows16(k, k_sb, k_st, k_sh) && rows16(v, v_sb, v_st, v_sh) &&
+                       rows16(o, o_sb, o_st, o_sh);
+  if (causal && aligned && rowsum_col < 0 && max_col < 0) {
+    const int rc = attn_fwd_split(p, d, stream);
+    if (rc != 1) return rc ? rc : -1;
+  }
   // The general forms against the generic kernels, which took these calls before (one MI355X; forward, forward's and
   // backward's kernels in us, generic -> general):
   //   2 x 2048, 14 heads of 128, ALiBi       198 -> 80, 345 -> 303    1 x 1500, 64 heads of 96       177 -> 66, 366 -> 234
@@ -1579,19 +1516,26 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
   //   4 x 2048, 16 heads of 256, lengths     528 -> 203, 1870 -> 815  2 x 2048, 20 of 128, window 256  68 -> 39, 148 -> 137
   // Full tiles without another mask keep the plain form, whose loops have no edge to test: 4 x 2048 of 256 179 us
   // against 203 forward and 760 against 815 backward, 8 x 1024 of 64 36 and 137 against 36 and 146.
-  if (alibi || kv_len || window || cu || Sq % 128 || Sk % 32) {
-    if (!rows16(q, q_sb, q_st, q_sh) || !rows16(k, k_sb, k_st, k_sh) || !rows16(v, v_sb, v_st, v_sh) ||
-        !rows16(o, o_sb, o_st, o_sh))
-      return 1;
+  bool whole = false;  // the kernel leaves no row to the fixup launch
+  // D = 256 under a causal mask: blocks of 128 rows, their keys in two groups, where blocks of 256 leave CUs idle (us, 256 rows and
+  // one group against it; blocks of 256 rows: 1 x 1024 x 16 heads (64) 47, 40; 1 x 2048 (128) 89, 73; 1 x 3000 with ALiBi (192) 143,
+  // 107; 2 x 2048 (256) 103, 106; 1 x 4096 (256) 179, 168; 4 x 1100 (320) 65, 80; 1 x 61 9.2, 11.6)
+  const bool two = d == 256 && causal && aligned && Sq > 256 && (long long)((Sq + 255) / 256) * B * H <= 192;
+  if (alibi || kv_len || window || cu || Sq % 128 || Sk % 32 || two) {
+    if (!aligned) return 1;
     const bool done = general_form(d, causal, alibi, [&](auto D_, auto C_, auto G_) {
       constexpr int D = decltype(D_)::value, G = decltype(G_)::value;
       constexpr bool C = decltype(C_)::value;
-      if constexpr (D == 256)
-        hipLaunchKernelGGL((attn_fwd_w8_kernel<D, C, 8, 4, G>), dim3(((Sq + 255) / 256) * B * H), dim3(512), 0, stream, p);
-      else
+      if constexpr (D == 256) {
+        if constexpr (C)
+          if (two) hipLaunchKernelGGL((attn_fwd_w8_kernel<D, C, 8, 4, G, 2>), grid, dim3(512), 0, stream, p);
+        if (!two)
+          hipLaunchKernelGGL((attn_fwd_w8_kernel<D, C, 8, 4, G>), dim3(((Sq + 255) / 256) * B * H), dim3(512), 0, stream, p);
+        whole = true;
+      } else if constexpr (!C || D == 160)  // (the other causal ones: attention_split.hip)
         hipLaunchKernelGGL((attn_fwd_tiled_kernel<D, C, -1, D, -1, G>), grid, dim3(256), 0, stream, p);
     });
-    return !done ? 1 : hipGetLastError() == hipSuccess ? 0 : 3;
+    return !done ? 1 : hipGetLastError() != hipSuccess ? 3 : whole ? -1 : 0;
   }
   if ((d != 48 && d != 64 && d != 96 && d != 128 && d != 160 && d != 256)) return 1;
   if (max_col >= 0 && (max_col != 40 || rowsum_col != 40 || d != 48)) return 1;  // instantiated variant
@@ -1601,6 +1545,7 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
     dim3 g8((Sq / 256) * B * H);
     if (causal) hipLaunchKernelGGL((attn_fwd_w8_kernel<256, true>), g8, dim3(512), 0, stream, p);
     else hipLaunchKernelGGL((attn_fwd_w8_kernel<256, false>), g8, dim3(512), 0, stream, p);
+    whole = true;
   } else if (d == 256) {
     if (causal) hipLaunchKernelGGL((attn_fwd_tiled_kernel<256, true>), grid, dim3(256), 0, stream, p);
     else hipLaunchKernelGGL((attn_fwd_tiled_kernel<256, false>), grid, dim3(256), 0, stream, p);
@@ -1624,7 +1569,7 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
   }
   // a failed launch leaves the flags unwritten: report it so the caller runs
   // the generic kernel on every block instead of trusting stale flags
-  return hipGetLastError() == hipSuccess ? 0 : 3;
+  return hipGetLastError() != hipSuccess ? 3 : whole ? -1 : 0;
 }
 
 // The VAE's single 512-wide head (non-causal, no masks): 0 = launched (flags[4 * (Sq/128) * B * H]
@@ -1665,11 +1610,11 @@ KCA_API int kca_attn_bwd_tiled(const void* q, const void* k, const void* v, cons
                   dq_sb, dq_st, dq_sh, dk_sb, dk_st, dk_sh, dv_sb, dv_st, dv_sh,
                   B, Sq, Sk, H, Hkv, scale, alibi, kv_len, window, (const bf16_t*)o, o_sb, o_st, o_sh};
   dim3 g1(((Sk + 127) / 128) * B * Hkv), g2(((Sq + 127) / 128) * B * H);
+  const bool aligned = rows16(q, q_sb, q_st, q_sh) && rows16(k, k_sb, k_st, k_sh) && rows16(v, v_sb, v_st, v_sh) &&
+                       rows16(o, o_sb, o_st, o_sh) && rows16(dout, do_sb, do_st, do_sh) && rows16(dq, dq_sb, dq_st, dq_sh) &&
+                       rows16(dk, dk_sb, dk_st, dk_sh) && rows16(dv, dv_sb, dv_st, dv_sh);
   if (alibi || kv_len || window || Sq % 128 || Sk % 128) {
-    if (!rows16(q, q_sb, q_st, q_sh) || !rows16(k, k_sb, k_st, k_sh) || !rows16(v, v_sb, v_st, v_sh) ||
-        !rows16(o, o_sb, o_st, o_sh) || !rows16(dout, do_sb, do_st, do_sh) || !rows16(dq, dq_sb, dq_st, dq_sh) || !rows16(dk, dk_sb, dk_st, dk_sh) ||
-        !rows16(dv, dv_sb, dv_st, dv_sh))
-      return 1;
+    if (!aligned) return 1;
     const bool done = general_form(d, causal, alibi, [&](auto D_, auto C_, auto G_) {
       constexpr int D = decltype(D_)::value, G = decltype(G_)::value;
       constexpr bool C = decltype(C_)::value;

@@ -1,0 +1,78 @@
+"""Attention whose blocks split their keys over wave groups, and the same kernels with one group, which calls of many blocks
+take: odd sizes around the tiles of 32, the blocks of 64 and 128 rows and the groups' strides, against the fp32 reference
+(bounds as in test_attention_edges_gpu.py)."""
+import pytest
+import torch
+
+from kubernetes_cloud_amd.ops.attention import _fwd, attention_reference, flash_attention
+
+from .test_attention_edges_gpu import _check, _close
+
+pytestmark = pytest.mark.gpu
+FEW, MANY = (2, 3), (13, 48)  # batch, heads: of MANY every size here has more blocks than the split calls
+
+
+@pytest.mark.parametrize("D", [64, 96, 128])
+@pytest.mark.parametrize("S", [32, 65, 96, 130, 161])
+def test_one_group(D, S):
+    B, H = MANY
+    _check(B, S, S, H, H, D, True)
+
+
+@pytest.mark.parametrize("D", [64, 96, 128, 256])
+def test_one_group_masks(D):
+    B, H = MANY
+    _check(B, 150, 150, H, H, D, True, lens=[150, 33, 0, 1, 64, 65, 31, 32, 150, 149, 128, 129, 96])
+    _check(B, 170, 170, H, H, D, True, window=40)
+    _check(B, 140, 140, H, H, D, True, alibi=True, window=70)
+    _check(B, 40, 171, H, H, D, True)
+    _check(B, 130, 130, H, H // 3, D, True, alibi=True)
+
+
+@pytest.mark.parametrize("D", [64, 96, 128, 256])
+@pytest.mark.parametrize("S", [63, 97, 193, 290, 417])
+def test_two_groups(D, S):
+    B, H = FEW
+    _check(B, S, S, H, H, D, True, window=33)
+    _check(B, S, S, H, H, D, True, alibi=True, lens=[S, S - 40])
+    _check(B, S, S + 37, H, 1, D, True)
+
+
+def test_eight_waves_dkdv():
+    """128-wide heads between the two: dK/dV of 128 keys in two groups of four waves."""
+    _check(9, 300, 300, 10, 10, 128, True)
+    _check(9, 300, 300, 10, 10, 128, True, alibi=True, window=150)
+    _check(9, 200, 330, 20, 10, 128, True, lens=[330, 0, 1, 329, 128, 127, 129, 31, 300])
+
+
+@pytest.mark.parametrize("D", [64, 96, 128, 256])
+@pytest.mark.parametrize("many", [False, True])
+@pytest.mark.parametrize("alibi", [False, True])
+def test_rows_far_above_their_first_tile(D, many, alibi):
+    """A late key that scores 2^900 times above a row's first tile: the rows are computed again with their true maximum, in the
+    same launch, and the rows beside them keep their results."""
+    S = 333
+    B, H = (MANY if many else FEW)
+    g = torch.Generator(device="cuda").manual_seed(D)
+    q, k, v = (torch.randn(B, S, H, D, device="cuda", generator=g) * 0.3 for _ in range(3))
+    k[0, 200, 1] = q[0, 320, 1] * 40.0
+    q, k, v = (t.bfloat16() for t in (q, k, v))
+    sl = torch.full((H,), 0.25, device="cuda") if alibi else None
+    o, lse = _fwd(q, k, v, True, D ** -0.5, None, sl)
+    r, want = attention_reference(*(t[:1, :, :2].float() for t in (q, k, v)), True, None, None, None if sl is None else sl[:2])
+    _close(o[:1, :, :2], r)
+    # sums of up to 256 products in fp32, in another order: 16 roundings of 2^-24 on average, four times that
+    torch.testing.assert_close(lse[:1, :2], want, rtol=2.0 ** -18, atol=2.0 ** -16)
+
+
+@pytest.mark.parametrize("D", [64, 256])
+def test_not_a_number_stays_in_its_rows(D):
+    q, k, v = (torch.randn(1, 300, 2, D, device="cuda", generator=torch.Generator(device="cuda").manual_seed(i)).bfloat16()
+               for i in range(3))
+    want = flash_attention(q, k, v, causal=True)
+    q[0, 70, 1] = float("nan")
+    o = flash_attention(q, k, v, causal=True)
+    assert torch.isnan(o[0, 70, 1]).all()
+    o[0, 70, 1] = want[0, 70, 1]
+    # (the row's block takes its true maxima: other rows of it are rounded relative to another weight)
+    _close(o, want)
