@@ -1,5 +1,5 @@
-// Flash attention for calls whose 128-row blocks leave the chip idle: the keys of a block are split over the wave groups
-// of its workgroup.
+// Flash attention for calls whose 128-row blocks leave the chip idle: the keys (dK/dV: the queries) of a block are split over
+// the wave groups of its workgroup.
 //
 // What bounds these calls. attn_fwd_tiled_kernel gives a workgroup 128 rows and a wave 32 of them; a call of few heads and
 // rows then has less than one workgroup a CU, so a SIMD runs one wave whose products, softmax, LDS reads and barriers follow
@@ -327,6 +327,386 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_fwd_split_kernel(FastF
                              p.Sq - q0);
 }
 
+// dQ: as the forward, a group walks every KG-th key tile of its 32 RW query rows; the groups' dQ add up in LDS.
+template <int D, int G, int RW, int KG, int WPS>
+__global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dq_split_kernel(FastBwdParams p) {
+  constexpr int BM = 32 * RW, BN = 32, NTG = 64 * RW;
+  constexpr int TILE = BN * D * 2, KS = D / 16;
+  using Stg = GroupStager<D, NTG>;
+  constexpr int CPT = Stg::CPT;
+  constexpr int PART = 32 * D * 4;
+  static_assert((KG - 1) * RW * PART <= KG * 4 * TILE, "the partial sums take the tiles' place");
+  __shared__ __attribute__((aligned(16))) char smem[KG * 4 * TILE];  // per group [buf 0 | 1][K | V]
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = wave / RW, rw = wave % RW;
+  const int l32 = lane & 31, hh = lane >> 5;
+  const int nqb = (p.Sq + BM - 1) / BM, heads = p.B * p.H;
+  const auto [qi, bh] = block_of<true>(nqb, heads);
+  const int qb = nqb - 1 - qi;
+  const int b = bh / p.H, h = bh % p.H;
+  const int hk = h / (p.H / p.Hkv);
+  const int off = p.Sk - p.Sq;
+  const int q0 = qb * BM + rw * 32, qrow = q0 + l32;
+  const int kv_end = batch_keys(p.kv_len, b, p.Sk);
+  const TileSpan sp = tile_span<BM, true>(qb * BM, off, kv_end, p.window);
+  const int ntiles = sp.hi - sp.lo, nsteps = (ntiles + KG - 1) / KG;
+  auto key0 = [&](int i) { return (sp.lo + min(KG * i + g, ntiles - 1)) * BN; };
+  const float sl2 = p.scale * kLog2e;
+
+  const int qr = min(qrow, p.Sq - 1);
+  const bf16_t* qp = p.q + b * p.q_sb + h * p.q_sh + (long long)qr * p.q_st;
+  const bf16_t* gp = p.dout + b * p.do_sb + h * p.do_sh + (long long)qr * p.do_st;
+  const __amdgpu_buffer_rsrc_t rk = head_rsrc(p.k + b * p.k_sb + hk * p.k_sh, rows_bytes(kv_end, p.k_st, D));
+  const __amdgpu_buffer_rsrc_t rv = head_rsrc(p.v + b * p.v_sb + hk * p.v_sh, rows_bytes(kv_end, p.v_st, D));
+  const Stg stk(tid % NTG, p.k_st), stv(tid % NTG, p.v_st);
+  const int kst2 = (int)p.k_st * 2, vst2 = (int)p.v_st * 2;
+  auto at = [](int k0, int st2) { return __builtin_amdgcn_readfirstlane(k0 * st2); };
+  char* const own = smem + g * 4 * TILE;
+  u32x4 xk[CPT], xv[CPT];
+  stk.load(xk, rk, at(key0(0), kst2));  // (flies with the query rows)
+  stv.load(xv, rv, at(key0(0), vst2));
+  bf16x8 qf[KS], gf[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    qf[s] = *reinterpret_cast<const bf16x8*>(qp + 16 * s + 8 * hh);
+    gf[s] = *reinterpret_cast<const bf16x8*>(gp + 16 * s + 8 * hh);
+  }
+  const float slope = G == 2 ? p.alibi[h] * kLog2e : 0.f;
+  const long long li = ((long long)b * p.H + h) * p.Sq + qr;
+  const float nlse = -p.lse[li] * kLog2e;
+  float dl = 0.f;  // delta = rowsum(dO * O), left for the dK/dV kernel too
+  {
+    const bf16_t* op = p.o + b * p.o_sb + h * p.o_sh + (long long)qr * p.o_st;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const bf16x8 of = *reinterpret_cast<const bf16x8*>(op + 16 * s + 8 * hh);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) dl = fmaf((float)of[j], (float)gf[s][j], dl);
+    }
+    dl += __shfl_xor(dl, 32, 64);
+    if (g == 0 && hh == 0 && qrow < p.Sq) p.delta[li] = dl;
+  }
+  f32x16 dq[D / 32];
+  clear<D>(dq);
+  int be, bo, b1, b2;
+  row_bases<D>(l32, hh, be, bo);
+  tr_bases<D>(lane, b1, b2);
+  const int last = min(qrow + off, kv_end - 1);    // row's last visible key
+  const int before = p.window > 0 ? qrow + off - p.window : -(1 << 30);  // key before its first
+
+  stk.store(xk, own);
+  stv.store(xv, own + TILE);
+  __syncthreads();
+  auto step = [&](int i, auto masked) {
+    constexpr bool MASKED = decltype(masked)::value;
+    const int k0 = key0(i);
+    const char* Ks = own + (i & 1) * 2 * TILE;
+    const char* Vs = Ks + TILE;
+    stk.load(xk, rk, at(key0(i + 1), kst2));
+    stv.load(xv, rv, at(key0(i + 1), vst2));
+    asm volatile("" ::: "memory");
+    f32x16 st, dpt;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) { st[r] = 0.f; dpt[r] = 0.f; }
+    {  // K / V row fragments two k-steps ahead of their MFMAs (pinned)
+      bf16x8 fk[3], fv[3];
+      fk[0] = row_frag<D>(Ks, be, bo, 0);
+      fv[0] = row_frag<D>(Vs, be, bo, 0);
+      fk[1] = row_frag<D>(Ks, be, bo, 1);
+      fv[1] = row_frag<D>(Vs, be, bo, 1);
+      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        if (s + 2 < KS) {
+          fk[(s + 2) % 3] = row_frag<D>(Ks, be, bo, s + 2);
+          fv[(s + 2) % 3] = row_frag<D>(Vs, be, bo, s + 2);
+          __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        }
+        st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fk[s % 3], qf[s], st, 0, 0, 0);
+        dpt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fv[s % 3], gf[s], dpt, 0, 0, 0);
+        __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
+      }
+    }
+    // visible key offsets (r&3)+8(r>>2): lo < offset <= lim
+    const int mk0 = KG * i + g < ntiles ? k0 : kNoTile;
+    const int lim = last - mk0 - 4 * hh, lo = before - mk0 - 4 * hh;
+    const float b0 = G == 2 ? fmaf(slope, (float)(k0 + 4 * hh - qrow - off), nlse) : nlse;
+    bf16x8 d0, d1;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int c = (r & 3) + 8 * (r >> 2);
+      float p0 = __builtin_amdgcn_exp2f(fmaf(st[r], sl2, G == 2 ? fmaf(slope, (float)c, b0) : b0));
+      float p1 = __builtin_amdgcn_exp2f(fmaf(st[r + 8], sl2, G == 2 ? fmaf(slope, (float)(c + 16), b0) : b0));
+      if constexpr (MASKED) {
+        if (c > lim || c <= lo) p0 = 0.f;
+        if (c + 16 > lim || c + 16 <= lo) p1 = 0.f;
+      }
+      d0[r] = (__bf16)(p0 * (dpt[r] - dl));
+      d1[r] = (__bf16)(p1 * (dpt[r + 8] - dl));
+    }
+    {
+      bf16x8 t0[2], t1[2];
+      t0[0] = tr_frag<D>(Ks, b1, b2, 0, 0);
+      t1[0] = tr_frag<D>(Ks, b1, b2, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+      for (int db = 0; db < D / 32; ++db) {
+        if (db + 1 < D / 32) {
+          t0[(db + 1) & 1] = tr_frag<D>(Ks, b1, b2, 0, db + 1);
+          t1[(db + 1) & 1] = tr_frag<D>(Ks, b1, b2, 1, db + 1);
+          __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+        }
+        dq[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t0[db & 1], d0, dq[db], 0, 0, 0);
+        dq[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t1[db & 1], d1, dq[db], 0, 0, 0);
+        __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
+      }
+    }
+    asm volatile("" ::: "memory");
+    if (i + 1 < nsteps) {
+      stk.store(xk, own + ((i + 1) & 1) * 2 * TILE);
+      stv.store(xv, own + ((i + 1) & 1) * 2 * TILE + TILE);
+    }
+    __syncthreads();
+  };
+  const int low = min(nsteps, (max(0, sp.f_lo - sp.lo) + KG - 1) / KG);
+  const int top = max(low, min(nsteps, (min(sp.f_hi + 1, sp.hi) - sp.lo) / KG));
+  for (int i = 0; i < low; ++i) step(i, std::true_type{});
+  for (int i = low; i < top; ++i) step(i, std::false_type{});
+  for (int i = top; i < nsteps; ++i) step(i, std::true_type{});
+
+  if constexpr (KG > 1) {
+    if (g > 0) put_partial<D>(smem + ((g - 1) * RW + rw) * PART, dq, lane);
+    __syncthreads();
+    if (g > 0) return;
+#pragma unroll
+    for (int i = 1; i < KG; ++i) add_partial<D>(smem + ((i - 1) * RW + rw) * PART, dq, lane, 1.f);
+    asm volatile("" ::: "memory");
+  }
+  store_tile_lds<D, D, true>(p.dq + b * p.dq_sb + h * p.dq_sh + (long long)q0 * p.dq_st, p.dq_st, dq, lane, p.scale,
+                             smem + rw * (KG > 1 ? PART : PART / 2), p.Sq - q0);
+}
+
+// dK/dV: a wave has 32 keys of the workgroup's 32 RW and its group every KG-th 32-row tile of Q and dO (of all the query heads
+// of a KV head); the groups' dV, then their dK add up in LDS.
+template <int D, int G, bool WIN, int RW, int KG, int WPS>
+__global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(FastBwdParams p) {
+  constexpr int BK = 32 * RW, BQ = 32, NTG = 64 * RW;
+  constexpr int TILE = BQ * D * 2, KS = D / 16, NCH = D / 8;
+  using Stg = GroupStager<D, NTG>;
+  constexpr int CPT = Stg::CPT;
+  constexpr int PART = 32 * D * 4;
+  static_assert((KG - 1) * RW * PART <= KG * 4 * TILE, "the partial sums take the tiles' place");
+  constexpr int VOFF = KG * 4 * TILE;  // V images of the RW key blocks, the groups' alike
+  constexpr int LOFF = VOFF + RW * TILE;
+  __shared__ __attribute__((aligned(16))) char smem[LOFF + KG * 2 * 64 * 4];  // lse / delta: [group][buf][64] floats
+
+  const int tid = threadIdx.x, lane = tid & 63, gt = tid % NTG;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = wave / RW, rw = wave % RW;
+  const int l32 = lane & 31, hh = lane >> 5;
+  const int heads = p.B * p.Hkv;
+  const auto [kb, bh] = block_of<true>((p.Sk + BK - 1) / BK, heads);
+  const int b = bh / p.Hkv, hk = bh % p.Hkv;
+  const int grp = p.H / p.Hkv;
+  const int off = p.Sk - p.Sq;
+  const int kw = kb * BK + rw * 32, key = kw + l32;
+  const int kv_end = batch_keys(p.kv_len, b, p.Sk);
+  const float sl2 = p.scale * kLog2e;
+
+  const int q_lo = max(0, kb * BK - off) & ~(BQ - 1);
+  // no query sees a block past the length; past the last key's window no query sees the block
+  const int q_end = WIN ? min(p.Sq, kb * BK + BK - 1 - off + p.window) : p.Sq;
+  const int nqt = max(0, q_end - q_lo + BQ - 1) / BQ;
+  const int total = kb * BK < kv_end ? nqt * grp : 0, nsteps = (total + KG - 1) / KG;
+  const int qn = rows_bytes(p.Sq, p.q_st, D), gn = rows_bytes(p.Sq, p.do_st, D);
+
+  const Stg stq(gt, p.q_st), sto(gt, p.do_st);
+  char* const own = smem + g * 4 * TILE;
+  float* const stat = reinterpret_cast<float*>(smem + LOFF) + g * 128;
+  u32x4 xq[CPT], xg[CPT];
+  float lreg = 0.f;
+  int be, bo, b1, b2;
+  row_bases<D>(l32, hh, be, bo);
+  tr_bases<D>(lane, b1, b2);
+
+  // The group's current tile: query head hcur of the KV head, q tile qcur; past its last one the tile stays and is masked.
+  int hcur = 0, qcur = 0, tile = g;
+  auto settle = [&] {  // (after qcur moved on)
+    while (qcur >= nqt && hcur < grp - 1) qcur -= nqt, ++hcur;
+    qcur = min(qcur, nqt - 1);
+  };
+  auto load_tile = [&] {
+    const int hq = hk * grp + hcur, qt = q_lo + qcur * BQ;
+    const __amdgpu_buffer_rsrc_t rq = head_rsrc(p.q + b * p.q_sb + hq * p.q_sh, qn);
+    const __amdgpu_buffer_rsrc_t rg = head_rsrc(p.dout + b * p.do_sb + hq * p.do_sh, gn);
+    if (gt < 64) {  // as they come: the scaling waits until they are stored
+      const long long li = ((long long)b * p.H + hq) * p.Sq + min(qt + (gt & 31), p.Sq - 1);
+      lreg = (gt < 32 ? p.lse : p.delta)[li];
+    }
+    stq.load(xq, rq, __builtin_amdgcn_readfirstlane((int)(qt * p.q_st * 2)));
+    sto.load(xg, rg, __builtin_amdgcn_readfirstlane((int)(qt * p.do_st * 2)));
+  };
+  auto store_tile = [&](int buf) {
+    stq.store(xq, own + buf * 2 * TILE);
+    sto.store(xg, own + buf * 2 * TILE + TILE);
+    if (gt < 64) {
+      float v = gt < 32 ? lreg * kLog2e : lreg;
+      if (q_lo + qcur * BQ + (gt & 31) >= p.Sq) v = gt < 32 ? INFINITY : 0.f;  // P = 0
+      stat[buf * 64 + gt] = v;
+    }
+  };
+  if (total > 0) {  // (flies with the key and value rows)
+    qcur = g;
+    settle();
+    load_tile();
+  }
+  const bf16_t* kp = p.k + b * p.k_sb + hk * p.k_sh;
+  const bf16_t* vp = p.v + b * p.v_sb + hk * p.v_sh;
+  bf16x8 kf[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    kf[s] = *reinterpret_cast<const bf16x8*>(kp + (long long)min(key, p.Sk - 1) * p.k_st + 16 * s + 8 * hh);
+    if (key >= kv_end) kf[s] = bf16x8{};
+  }
+  // V rows -> the images (read back by rows for dP), 32 RW rows over all threads
+  constexpr int NT = NTG * KG;
+  char* const vimg = smem + VOFF + rw * TILE;
+#pragma unroll
+  for (int i = 0; i < (BK * NCH + NT - 1) / NT; ++i) {
+    const int idx = tid + NT * i, row = idx / NCH, ch = idx % NCH;
+    if (BK * NCH % NT == 0 || idx < BK * NCH) {
+      const u32x4 x = *reinterpret_cast<const u32x4*>(vp + (long long)min(kb * BK + row, p.Sk - 1) * p.v_st + ch * 8);
+      *reinterpret_cast<u32x4*>(smem + VOFF + (row / 32) * TILE + img_off<D>(row % 32, ch)) =
+          kb * BK + row < kv_end ? x : u32x4{0, 0, 0, 0};
+    }
+  }
+  f32x16 dk[D / 32], dv[D / 32];
+  clear<D>(dk);
+  clear<D>(dv);
+
+  if (total > 0) store_tile(0);
+  __syncthreads();
+  for (int i = 0; i < nsteps; ++i) {
+    const int qt = q_lo + qcur * BQ, hq = hk * grp + hcur;
+    const bool gone = tile >= total;
+    // Tiles below the diagonal and inside the window skip the mask. (D = 64 has no registers for two ways through the softmax at
+    // 3 waves a SIMD; two bodies of the whole step spill at every D. 1 x 1500 x 64 heads of 96: 150 -> 142 us with dQ.)
+    const bool plain = D > 64 && !gone && kb * BK + BK <= kv_end && kb * BK + BK - 1 <= qt + off &&
+                       (!WIN || kb * BK > qt + BQ - 1 + off - p.window);
+    const char* Qs = own + (i & 1) * 2 * TILE;
+    const char* Gs = Qs + TILE;
+    const float* ls = stat + (i & 1) * 64;
+    tile += KG;
+    qcur += KG;
+    settle();
+    load_tile();
+    asm volatile("" ::: "memory");
+    f32x16 sacc, dpacc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) { sacc[r] = 0.f; dpacc[r] = 0.f; }
+    {  // S = Q.K^T, dP = dO.V^T, the three fragments of k-step s + 1 before the MFMAs of step s (pinned)
+      bf16x8 fq[2], fg[2], fv[2];
+      fq[0] = row_frag<D>(Qs, be, bo, 0), fg[0] = row_frag<D>(Gs, be, bo, 0), fv[0] = row_frag<D>(vimg, be, bo, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        if (s + 1 < KS) {
+          fq[(s + 1) & 1] = row_frag<D>(Qs, be, bo, s + 1);
+          fg[(s + 1) & 1] = row_frag<D>(Gs, be, bo, s + 1);
+          fv[(s + 1) & 1] = row_frag<D>(vimg, be, bo, s + 1);
+          __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+        }
+        sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fq[s & 1], kf[s], sacc, 0, 0, 0);
+        dpacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fg[s & 1], fv[s & 1], dpacc, 0, 0, 0);
+        __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
+      }
+    }
+    // rows q = qt + 8g + 4hh + j (g = r>>2, j = r&3) that see the key: lim <= 8g + j < ul
+    int lim = key - qt - off - 4 * hh;
+    if (key >= kv_end || gone) lim = 1 << 30;
+    const int ul = WIN ? key + p.window - off - qt - 4 * hh : 0;
+    float slope = 0.f, b0 = 0.f;
+    if constexpr (G == 2) {
+      slope = p.alibi[hq] * kLog2e;
+      b0 = slope * (float)(key - qt - off - 4 * hh);
+    }
+    float pr[16];
+#pragma unroll
+    for (int gg = 0; gg < 4; ++gg) {
+      const f32x4 lq = *reinterpret_cast<const f32x4*>(ls + 8 * gg + 4 * hh);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float bl = G == 2 ? fmaf(-slope, (float)(8 * gg + j), b0) - lq[j] : -lq[j];
+        pr[4 * gg + j] = __builtin_amdgcn_exp2f(fmaf(sacc[4 * gg + j], sl2, bl));
+      }
+    }
+    if (!plain) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int c = 8 * (r >> 2) + (r & 3);
+        if (c < lim || (WIN && c >= ul)) pr[r] = 0.f;
+      }
+    }
+    bf16x8 p0, p1, s0, s1;
+#pragma unroll
+    for (int gg = 0; gg < 4; ++gg) {
+      const f32x4 dq4 = *reinterpret_cast<const f32x4*>(ls + 32 + 8 * gg + 4 * hh);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int r = 4 * gg + j;
+        const float ds = pr[r] * (dpacc[r] - dq4[j]);
+        if (r < 8) { p0[r] = (__bf16)pr[r]; s0[r] = (__bf16)ds; }
+        else { p1[r - 8] = (__bf16)pr[r]; s1[r - 8] = (__bf16)ds; }
+      }
+    }
+    {  // dV^T += dO^T.P, dK^T += Q^T.dS: the reads of d-block db + 1 under the MFMAs of block db (pinned)
+      bf16x8 fr[2][4];
+      auto get = [&](int db) {
+        fr[db & 1][0] = tr_frag<D>(Gs, b1, b2, 0, db), fr[db & 1][1] = tr_frag<D>(Gs, b1, b2, 1, db);
+        fr[db & 1][2] = tr_frag<D>(Qs, b1, b2, 0, db), fr[db & 1][3] = tr_frag<D>(Qs, b1, b2, 1, db);
+        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+      };
+      get(0);
+#pragma unroll
+      for (int db = 0; db < D / 32; ++db) {
+        if (db + 1 < D / 32) get(db + 1);
+        dv[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[db & 1][0], p0, dv[db], 0, 0, 0);
+        dv[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[db & 1][1], p1, dv[db], 0, 0, 0);
+        dk[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[db & 1][2], s0, dk[db], 0, 0, 0);
+        dk[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[db & 1][3], s1, dk[db], 0, 0, 0);
+        __builtin_amdgcn_sched_group_barrier(0x8, 4, 0);
+      }
+    }
+    asm volatile("" ::: "memory");
+    if (i + 1 < nsteps) store_tile((i + 1) & 1);
+    __syncthreads();
+  }
+  // group 0 adds dV up and stores it, then the last group dK
+  if constexpr (KG > 1) {
+    if (g > 0) put_partial<D>(smem + ((g - 1) * RW + rw) * PART, dv, lane);
+    __syncthreads();
+    if (g == 0) {
+#pragma unroll
+      for (int i = 1; i < KG; ++i) add_partial<D>(smem + ((i - 1) * RW + rw) * PART, dv, lane, 1.f);
+    }
+    __syncthreads();
+    if (g < KG - 1) put_partial<D>(smem + (g * RW + rw) * PART, dk, lane);
+    __syncthreads();
+    if (g == KG - 1) {
+#pragma unroll
+      for (int i = 0; i < KG - 1; ++i) add_partial<D>(smem + (i * RW + rw) * PART, dk, lane, 1.f);
+    }
+    asm volatile("" ::: "memory");
+  }
+  if (KG > 1 && g > 0 && g < KG - 1) return;
+  // (images of this wave's own: KG = 1, in the tiles; else group 0's in the V images, the last group's on what it has read)
+  char* const img = KG == 1 ? smem + rw * (PART / 2) : g == 0 ? vimg : smem + rw * PART;
+  if (g == 0)
+    store_tile_lds<D, D, true>(p.dv + b * p.dv_sb + hk * p.dv_sh + (long long)kw * p.dv_st, p.dv_st, dv, lane, 1.f, img, p.Sk - kw);
+  if (g == KG - 1)
+    store_tile_lds<D, D, true>(p.dk + b * p.dk_sb + hk * p.dk_sh + (long long)kw * p.dk_st, p.dk_st, dk, lane, p.scale, img, p.Sk - kw);
+}
+
 }  // namespace
 
 // Which calls are split in two groups (two waves of 32 rows each, 4 waves a workgroup), the others in blocks of 128 rows and
@@ -335,6 +715,7 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_fwd_split_kernel(FastF
 //                       2 x 2688 x 12 (504) 45.3, 41.8; 3 x 2048 x 12 (576) 39.2, 35.2; 10 x 577 x 12 (600) 18.3, 21.9
 //   96 wide:            1 x 700 x 32 (192) 19.4, 16.0; 5 x 256 x 32 (320) 14.3, 18.4; 1 x 1403 x 32 (352) 33.8, 31.2; 768: 51, 61
 //   128 wide:           1 x 2048 x 14 with ALiBi (224) 48.7, 41.2; 2 x 896 x 20 (280) 27.9, 24.6; 2 x 1346 x 20 (440) 37.1, 43.0
+//   dQ follows the same line (gains of 1 to 17 us below it, losses of 1 to 23 above).
 static bool split_rows(long long blocks, int d, int rows) {
   return blocks <= (d == 64 ? (rows >= 1536 ? 640 : 448) : d == 96 ? (rows >= 1024 ? 400 : 256) : 320);
 }
@@ -364,5 +745,36 @@ int attn_fwd_split(const FastFwdParams& p, int d, hipStream_t stream) {
       hipLaunchKernelGGL((attn_fwd_split_kernel<D, G, 2, 2, W>), dim3((p.Sq + 63) / 64 * p.B * p.H), dim3(256), 0, stream, p);
     else
       hipLaunchKernelGGL((attn_fwd_split_kernel<D, G, 4, 1, W>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
+  });
+}
+
+// dK/dV, one group against two, us with dQ: 64 wide, 4 x 948 x 16 heads (512 blocks) 60.6, 55.3; 9 x 409 x 16 (576) 38.8, 41.8; 3 x
+// 2048 x 16 (768) 148, 140; 96 wide, 1 x 1403 x 32 (352) 101, 80; 11 x 146 x 32 (704) 45, 48. At 128 wide two groups of two waves
+// take 81 KB of LDS, one workgroup a CU; two of four (8 waves, 128 keys) are the better ones from 200 blocks on: 1 x 651 x 20 (120
+// blocks) 56.9, 51.1, 53.3; 2 x 896 x 20 (280) 84.7, 84.1, 72.8; 1 x 2944 x 20 (460) 246, 275, 209; 4 x 1408 x 14 (616) 137, 185, 145.
+int attn_bwd_split(const FastBwdParams& p, int d, hipStream_t stream) {
+  const long long qblocks = (long long)((p.Sq + 127) / 128) * p.B * p.H, kblocks = (long long)((p.Sk + 127) / 128) * p.B * p.Hkv;
+  const bool two = split_rows(qblocks, d, p.Sq);
+  const bool two_kv = kblocks <= (d == 64 ? (p.Sk >= 1536 ? 768 : 512) : d == 96 ? 400 : 200);
+  const bool wide_kv = !two_kv && d == 128 && kblocks <= 512;
+  return with_form(d, p.alibi, [&](auto D_, auto G_) {
+    constexpr int D = decltype(D_)::value, G = decltype(G_)::value, W = D == 64 ? 3 : 2;
+    if (two)
+      hipLaunchKernelGGL((attn_bwd_dq_split_kernel<D, G, 2, 2, W>), dim3((p.Sq + 63) / 64 * p.B * p.H), dim3(256), 0, stream, p);
+    else
+      hipLaunchKernelGGL((attn_bwd_dq_split_kernel<D, G, 4, 1, W>), dim3((unsigned)qblocks), dim3(256), 0, stream, p);
+    auto dkdv = [&](auto WIN_) {
+      constexpr bool WIN = decltype(WIN_)::value;
+      if (two_kv)
+        hipLaunchKernelGGL((attn_bwd_dkdv_split_kernel<D, G, WIN, 2, 2, W>), dim3((p.Sk + 63) / 64 * p.B * p.Hkv), dim3(256), 0,
+                           stream, p);
+      else if (!wide_kv)
+        hipLaunchKernelGGL((attn_bwd_dkdv_split_kernel<D, G, WIN, 4, 1, W>), dim3((unsigned)kblocks), dim3(256), 0, stream, p);
+      if constexpr (D == 128)
+        if (wide_kv)
+          hipLaunchKernelGGL((attn_bwd_dkdv_split_kernel<D, G, WIN, 4, 2, 2>), dim3((unsigned)kblocks), dim3(512), 0, stream, p);
+    };
+    if (p.window > 0) dkdv(std::true_type{});
+    else dkdv(std::false_type{});
   });
 }
