@@ -14,9 +14,11 @@ implementations in each op module (that is what the CPU test-suite runs).
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import sys
 import threading
+import warnings
 
 import torch
 from torch.autograd import forward_ad
@@ -165,6 +167,30 @@ def _load():
             fn.restype = ctypes.c_int
         _lib = lib
         return _lib
+
+
+_torch_ext: list = []
+
+
+def torch_ext():
+    """The extension module ``kca_torch`` (autograd functions in C++) bound to the loaded kernel library, or None where it is
+    not built, does not fit this torch, or launches are synchronised one by one: callers then take the same function in Python."""
+    if not _torch_ext:
+        lib = _load()
+        with _lock:
+            if not _torch_ext:
+                m = None
+                path = os.path.join(LIB_DIR, "kca_torch.so")
+                if lib is not None and hasattr(lib, "kca_attn_bwd") and not SYNC_LAUNCH and os.path.exists(path):
+                    spec = importlib.util.spec_from_file_location("kca_torch", path)
+                    try:
+                        m = importlib.util.module_from_spec(spec)
+                        m.init(*(ctypes.cast(f, P).value for f in (lib.kca_attn_fwd, lib.kca_attn_bwd)))
+                    except ImportError as e:  # pragma: no cover - another torch than it was built for
+                        warnings.warn(f"{path}: {e}")
+                        m = None
+                _torch_ext.append(m)
+    return _torch_ext[0]
 
 
 def ensure_built(sources) -> None:

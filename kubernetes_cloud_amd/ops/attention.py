@@ -196,7 +196,15 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: b
     if max_col >= 0:
         raise ValueError("max_col needs rowsum_col and the native inference path")
     if _lib.use_native(q, k, v):
-        return _FlashAttnFn.apply(q, k, v, causal, scale, native_mask(kv_len, q.device), alibi, int(window))
+        mask, window = native_mask(kv_len, q.device), int(window)
+        ext = _lib.torch_ext()
+        if ext is not None and not torch.compiler.is_compiling():
+            # the same function in C++, for plain tensors in plain eager mode (csrc/torch/attention_autograd.cpp); None otherwise
+            o = ext.attention(q, k, v, causal, scale, mask, alibi, window)
+            if o is not None:
+                _lib.LAUNCHES[0] += 1
+                return o
+        return _FlashAttnFn.apply(q, k, v, causal, scale, mask, alibi, window)
     o, _ = attention_reference(q, k, v, causal, scale, kv_len, alibi, window)
     return o
 

@@ -8,7 +8,10 @@
   ``.tensors`` weight streamer, the BPE tokenizer / context packer and the
   shared-memory control channel of the TP serving engine (``csrc/runtime``).
 
-Both are plain C-ABI shared objects loaded with ctypes *after* ``import
+* ``kca_torch.so``      -- autograd functions in C++ (``csrc/torch``), a Python extension module against the installed torch;
+  its kernels are those of the library that ``ops/_lib.py`` has loaded.
+
+The first two are plain C-ABI shared objects loaded with ctypes *after* ``import
 torch`` so that the HIP runtime torch already mapped (soname
 ``libamdhip64.so.7``) is the one the kernels register with.
 
@@ -159,6 +162,33 @@ def build_host(jobs: int = 8, verbose: bool = False) -> str | None:
     return out
 
 
+def build_torch(verbose: bool = False) -> str:
+    """The extension module of ``csrc/torch``, compiled against the torch of this interpreter."""
+    import sysconfig
+
+    import torch
+    base = os.path.dirname(torch.__file__)
+    obj_dir = os.path.join(BUILD, "torch")
+    os.makedirs(obj_dir, exist_ok=True)
+    os.makedirs(OUT_DIR, exist_ok=True)
+    flags = ["-O2", "-fPIC", "-std=c++17", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-DKCA_TORCH=\"{torch.__version__}\"",
+             f"-I{base}/include", f"-I{base}/include/torch/csrc/api/include", f"-I{ROCM}/include",
+             f"-I{sysconfig.get_paths()['include']}"]
+    cxx = shutil.which("g++") or "g++"
+    objs = [_compile([cxx], s, [], obj_dir, flags) for s in _sources("torch", (".cpp",))]
+    out = os.path.join(OUT_DIR, "kca_torch.so")
+    cmd = [cxx, "-shared", "-fPIC", "-o", out + ".tmp"] + objs + [
+        f"-L{base}/lib", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"link failed: {' '.join(cmd)}\n{r.stderr}")
+    os.replace(out + ".tmp", out)
+    if verbose:
+        print(f"built {out}")
+    return out
+
+
 SANITIZE_FLAGS = ["-fsanitize=address,undefined", "-fno-sanitize-recover=all", "-fno-omit-frame-pointer", "-g", "-O1",
                   "-std=c++17", "-fopenmp", "-Wall", "-Wno-unused-function"]
 
@@ -186,7 +216,8 @@ def build_sanitize(verbose: bool = False) -> str:
 
 
 def build_all(jobs: int = 8, verbose: bool = False):
-    return build_kernels(jobs, verbose), build_host(jobs, verbose), build_kernels(jobs, verbose, debug=True)
+    return (build_kernels(jobs, verbose), build_host(jobs, verbose), build_torch(verbose),
+            build_kernels(jobs, verbose, debug=True))
 
 
 if __name__ == "__main__":
