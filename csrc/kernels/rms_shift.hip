@@ -86,10 +86,19 @@ __device__ __forceinline__ void stv(bf16_t* p, const float (&v)[VEC]) {
     for (int i = 0; i < VEC; ++i) p[i] = f2bf(v[i]);
 }
 
+// a vector as loaded
+template <typename E, int VEC>
+struct alignas(VEC * sizeof(E)) Pack {
+  E v[VEC];
+  __device__ __forceinline__ float at(int i) const { return ldf(v + i); }
+};
+
 // E: compute type, VEC elements per access (4: d % 4 == 0), NCH accesses per thread. TOP: routed rows per token as a
 // constant, -1: read from the arguments -- with a constant a row's loads, the gathered ones too, are all in flight
 // before the first is used; a loop over them waits once per routed row and access (4096 tokens of 4096, two routed rows
 // each, no shift: 109 -> 61 us, 287 MB).
+// The loads are requested as they lie, without a lane's condition, and converted afterwards: a conversion inside a condition waited
+// for its load (30 tokens of 2048, four routed rows each: 5.9 -> 5.2 us; 4096 tokens as above 60 -> 44, 6.5 TB/s).
 template <typename E, int VEC, int NCH, int TOP>
 __global__ void __launch_bounds__(256) rms_shift_kernel(RmsShiftArgs p) {
   __shared__ float red[4];
@@ -98,57 +107,66 @@ __global__ void __launch_bounds__(256) rms_shift_kernel(RmsShiftArgs p) {
   const E* y = reinterpret_cast<const E*>(p.y);
   const E* gain = reinterpret_cast<const E*>(p.gain);
   const E* mu = reinterpret_cast<const E*>(p.mu);
+  using P = Pack<E, VEC>;
+  const E g1 = *gain;  // (a gain of one number; requested before the rows)
   const int r0 = blockIdx.x * p.R, r1 = min(p.T, r0 + p.R);
 
   // row t -> h (registers); x_out written where `out` >= 0
   auto row = [&](int t, float (&h)[NCH][VEC], bool write_x) {
     float ss = 0.f;
     const long long tok = p.x_in ? 0 : p.tokens[t];
-    const E* yr[TOP > 0 ? TOP : 1];
-    float ws[TOP > 0 ? NCH : 1][TOP > 0 ? TOP : 1][VEC];
+    auto at = [&](int c) { return (c * 256 + tid) * VEC; };
+    auto get = [&](const E* q, int c) { return *reinterpret_cast<const P*>(q + min(at(c), d - VEC)); };
+    int iv[TOP > 0 ? TOP : 1];
+    P yr[TOP > 0 ? NCH : 1][TOP > 0 ? TOP : 1], ar[NCH];
 #pragma unroll
-    for (int k = 0; k < TOP; ++k) yr[k] = y + (long long)p.inv[(long long)t * TOP + k] * d;
+    for (int k = 0; k < TOP; ++k) iv[k] = p.inv[(long long)t * TOP + k];
+    if (p.x_in) {
 #pragma unroll
-    for (int c = 0; c < (TOP > 0 ? NCH : 0); ++c) {
-      const int i = (c * 256 + tid) * VEC;
-      if (i >= d) continue;
+      for (int c = 0; c < NCH; ++c) ldv<VEC>(p.x_in + (long long)t * d + min(at(c), d - VEC), h[c]);
+    } else {
+      P er[NCH];
 #pragma unroll
-      for (int k = 0; k < TOP; ++k) ldv<VEC>(yr[k] + i, ws[c][k]);
+      for (int c = 0; c < NCH; ++c) er[c] = get(reinterpret_cast<const E*>(p.embed) + tok * d, c);
+#pragma unroll
+      for (int c = 0; c < NCH; ++c)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) h[c][e] = er[c].at(e);
     }
+    if (a)
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) ar[c] = get(a + (long long)t * p.lda, c);
+#pragma unroll
+    for (int k = 0; k < TOP; ++k)
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) yr[c][k] = get(y + (long long)iv[k] * d, c);
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
-      const int i = (c * 256 + tid) * VEC;
-      if (i >= d) continue;
-      float x[VEC];
-      if (p.x_in) ldv<VEC>(p.x_in + (long long)t * d + i, x);
-      else ldv<VEC>(reinterpret_cast<const E*>(p.embed) + tok * d + i, x);
+      const int i = at(c);
       float add[VEC];
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) add[e] = 0.f;
-      if (a) ldv<VEC>(a + (long long)t * p.lda + i, add);
+      for (int e = 0; e < VEC; ++e) add[e] = a ? ar[c].at(e) : 0.f;
       if constexpr (TOP > 0) {
 #pragma unroll
         for (int k = 0; k < TOP; ++k)
 #pragma unroll
-          for (int e = 0; e < VEC; ++e) add[e] += ws[c][k][e];
+          for (int e = 0; e < VEC; ++e) add[e] += yr[c][k].at(e);
       } else if (TOP < 0) {
         for (int k = 0; k < p.top; ++k) {
-          float w[VEC];
-          ldv<VEC>(y + (long long)p.inv[(long long)t * p.top + k] * d + i, w);
+          const P w = get(y + (long long)p.inv[(long long)t * p.top + k] * d, c);
 #pragma unroll
-          for (int e = 0; e < VEC; ++e) add[e] += w[e];
+          for (int e = 0; e < VEC; ++e) add[e] += w.at(e);
         }
       }
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
-        x[e] = fmaf(p.m, add[e], x[e]);
-        ss = fmaf(x[e], x[e], ss);
-        h[c][e] = x[e];
+        h[c][e] = fmaf(p.m, add[e], h[c][e]);
+        ss = fmaf(h[c][e], i < d ? h[c][e] : 0.f, ss);
       }
-      if (write_x) stv<VEC>(p.x_out + (long long)t * d + i, x);
+      if (write_x && i < d) stv<VEC>(p.x_out + (long long)t * d + i, h[c]);
     }
     const float rstd = 1.f / sqrtf(block_sum(ss, red) / (float)d + p.eps);
-    const float g0 = p.gain_vec ? 1.f : ldf(gain);
+    const float g0 = p.gain_vec ? 1.f : ldf(&g1);
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
       const int i = (c * 256 + tid) * VEC;
