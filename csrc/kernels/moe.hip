@@ -177,7 +177,8 @@ __device__ __forceinline__ void pick_lanes(const RouteArgs& p, const float* z, f
   float w = sigmoid(s);
   if (p.softmax) w = s / (lanes_reduce<64>(take ? s : 0.f, [](float a, float b) { return a + b; }) + 1e-20f);
   if (take) {
-    p.ids[(long long)t * p.top + rank] = lane;
+    // (written through: route_split_kernel's last workgroup reads what others chose)
+    __hip_atomic_store(p.ids + (long long)t * p.top + rank, lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (ids_lds) ids_lds[t * p.top + rank] = lane;
     p.wts[(long long)t * p.top + rank] = w;
   }
@@ -237,10 +238,21 @@ template <int NT>
 __device__ __forceinline__ void group_rows(const GroupArgs& p, int* sh) {
   const int E = p.E, n = p.n, mt = p.mt, tid = threadIdx.x;
   int *cnt = sh, *off = sh + E, *toff = off + E + 1;
+  constexpr int R = 4;  // a thread's first ids, read once for both passes
+  int first[R];
+#pragma unroll
+  for (int j = 0; j < R; ++j) first[j] = p.ids[min(tid + j * NT, n - 1)];
+  auto each = [&](auto&& f) {
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+      if (tid + j * NT < n) f(tid + j * NT, first[j]);
+    for (int i = tid + R * NT; i < n; i += NT) f(i, p.ids[i]);
+  };
   for (int e = tid; e < E; e += NT) cnt[e] = 0;
   __syncthreads();
-  for (int i = tid; i < n; i += NT)
-    if (p.ids[i] < E) atomicAdd(&cnt[p.ids[i]], 1);
+  each([&](int, int e) {
+    if (e < E) atomicAdd(&cnt[e], 1);
+  });
   __syncthreads();
   if (tid < 64) {  // exclusive sums over the experts, 64 at a time
     int co = 0, to = 0;
@@ -272,11 +284,11 @@ __device__ __forceinline__ void group_rows(const GroupArgs& p, int* sh) {
     cnt[e] = off[e];
   }
   __syncthreads();
-  for (int i = tid; i < n; i += NT) {  // (the order within an expert does not matter: rows are independent)
-    const int e = p.ids[i], pos = e < E ? atomicAdd(&cnt[e], 1) : -1;
+  each([&](int i, int e) {  // (the order within an expert does not matter: rows are independent)
+    const int pos = e < E ? atomicAdd(&cnt[e], 1) : -1;
     if (pos >= 0) p.perm[pos] = i;
     p.inv[i] = pos;
-  }
+  });
 }
 
 __global__ void __launch_bounds__(1024) group_kernel(GroupArgs p) {
@@ -370,10 +382,12 @@ __global__ void __launch_bounds__(NW * 64) route_mfma_kernel(RouteArgs p, GroupA
 // Routing and grouping, us, one workgroup a token block : this (launches back to back; 32 outputs of 2048, 16 of 4096, sigmoid):
 //   1 token 12.4 : 7.2, 8.9 : 7.0; 16 tokens 15.9 : 8.2, 11.9 : 8.1; 128 tokens 17.6 : 10.2, 13.4 : 10.0;
 //   1024 tokens 19.6 : 14.1, 14.5 : 13.0 (the blocks alone come near filling the chip)
-template <bool GROUP>
+// GROUP: 1, the launch is one token block, whose assignments it groups; 2, the last token block to be chosen groups all (cnt has one
+// counter more), which took a launch of its own.
+template <int GROUP>
 __global__ void __launch_bounds__(1024) route_split_kernel(RouteArgs p, GroupArgs gr, float* parts, unsigned* cnt) {
   __shared__ __attribute__((aligned(16))) float z[16 * 64];
-  __shared__ int sids[GROUP ? 16 * 64 : 1], sh[GROUP ? 3 * 64 + 2 : 1], s_last;
+  __shared__ int sids[GROUP == 1 ? 16 * 64 : 1], sh[GROUP ? 3 * 64 + 2 : 1], s_last;
   const int n = p.E + (p.wsg ? 1 : 0), nt = (n + 15) / 16, d = p.d, nk = (d + 31) / 32;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, r16 = lane & 15, g = lane >> 4;
   const int tb = blockIdx.x / 4, cut = blockIdx.x % 4 * 4 + (wv & 3), t0 = tb * 16;
@@ -432,19 +446,24 @@ __global__ void __launch_bounds__(1024) route_split_kernel(RouteArgs p, GroupArg
     else steps(integral_constant<int, 4>{}, integral_constant<int, 4>{});
     store();
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  if (tid == 0) {
-    const int last = __hip_atomic_fetch_add(cnt + tb, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 3;
-    if (last) {
-      __hip_atomic_store(cnt + tb, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // The last of `of` workgroups to arrive at a zeroed counter, which it leaves zeroed, and which then reads what the others have
+  // written through.
+  auto last_of = [&](unsigned* c, unsigned of) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+      const int last = __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == of - 1;
+      if (last) {
+        __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
+      s_last = last;
     }
-    s_last = last;
-  }
-  __syncthreads();
-  if (!s_last) return;
+    __syncthreads();
+    return s_last != 0;
+  };
+  if (!last_of(cnt + tb, 4)) return;
   if (const int r = tid >> 4, q = tid & 15; r < 16 && q < nt * 4) {
     const float* from = parts + ((long long)tb * 256 + r) * (16 * nt) + 4 * q;
     f32x4 v[16], s{0.f, 0.f, 0.f, 0.f};
@@ -457,11 +476,15 @@ __global__ void __launch_bounds__(1024) route_split_kernel(RouteArgs p, GroupArg
   __syncthreads();
   if (t0 + wv < p.T) {
     if (p.wsg && lane == 0) p.sg[t0 + wv] = sigmoid(z[wv * 64 + p.E]);
-    pick_lanes(p, z + wv * 64, fix, t0 + wv, lane, GROUP ? sids : nullptr);
+    pick_lanes(p, z + wv * 64, fix, t0 + wv, lane, GROUP == 1 ? sids : nullptr);
   }
-  if constexpr (GROUP) {
+  if constexpr (GROUP == 1) {
     __syncthreads();
     gr.ids = sids;
+    group_rows<1024>(gr, sh);
+  }
+  if constexpr (GROUP == 2) {
+    if (!last_of(cnt + gridDim.x / 4, gridDim.x / 4)) return;
     group_rows<1024>(gr, sh);
   }
 }
@@ -970,10 +993,10 @@ int route_go(const RouteArgs& a, const GroupArgs& g, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? 0 : 4;
 }
 
-template <bool GROUP>
+template <int GROUP>
 int split_go(const RouteArgs& a, const GroupArgs& g, void* ws, long long ws_floats, void* cnt, int cnt_n, hipStream_t s) {
   const int n = a.E + (a.wsg ? 1 : 0), blocks = (a.T + 15) / 16;
-  if (n > 64 || a.T > 1024 || !cnt || cnt_n < blocks || !al16(ws) || ws_floats < blocks * 256ll * ((n + 15) / 16 * 16)) return 6;
+  if (n > 64 || a.T > 1024 || !cnt || cnt_n < blocks + (GROUP == 2) || !al16(ws) || ws_floats < blocks * 256ll * ((n + 15) / 16 * 16)) return 6;
   hipLaunchKernelGGL(route_split_kernel<GROUP>, dim3(blocks * 4), dim3(1024), 0, s, a, g, (float*)ws, (unsigned*)cnt);
   return hipGetLastError() == hipSuccess ? 0 : 4;
 }
@@ -988,7 +1011,7 @@ KCA_API int kca_moe_route(int dtype, const void* h, const void* wr, const void* 
   const RouteArgs a{h, wr, wsg, (int*)ids, (float*)wts, (float*)sg, T, d, E, top, softmax, groups, keep, (const float*)fix};
   if (!route_ok(a)) return 1;
   if (dtype == 1 && d % 8 == 0 && al16(h) && al16(wr) && al16(wsg)) {
-    if (ws) return split_go<false>(a, GroupArgs{}, ws, ws_floats, cnt, cnt_n, s);
+    if (ws) return split_go<0>(a, GroupArgs{}, ws, ws_floats, cnt, cnt_n, s);
     if (T <= 1024 && route_lds<16, false>(a) <= MAX_LDS) return route_go<16, false>(a, GroupArgs{}, s);
     if (route_lds<8, false>(a) <= MAX_LDS) return route_go<8, false>(a, GroupArgs{}, s);
   }
@@ -1013,17 +1036,18 @@ KCA_API int kca_moe_group(const void* ids, int n, int E, int mt, void* perm, voi
   return hipGetLastError() == hipSuccess ? 0 : 4;
 }
 
-// Both in one launch: bf16, at most 16 tokens (10: shape outside it). E: router outputs, the first `real` with weights
+// Both in one launch: bf16, at most 16 tokens, or with ws (kca_moe_route; one counter more) 1024 (10: shape outside it). E: router
+// outputs, the first `real` with weights
 KCA_API int kca_moe_route_group(const void* h, const void* wr, const void* wsg, void* ids, void* wts, void* sg, int T,
                                 int d, int E, int real, int top, int softmax, const void* fix, int groups, int keep, int mt, void* perm,
                                 void* inv, void* tiles, int max_tiles, void* ntiles, void* ws, long long ws_floats, void* cnt,
                                 int cnt_n, hipStream_t s) {
   const RouteArgs a{h, wr, wsg, (int*)ids, (float*)wts, (float*)sg, T, d, E, top, softmax, groups, keep, (const float*)fix};
   if (!route_ok(a) || real < 1 || real > E) return 1;
-  if (T > 16 || top > 64 || d % 8 || !al16(h) || !al16(wr) || !al16(wsg) || route_lds<16, true>(a) > MAX_LDS) return 10;
+  if (T > (ws ? 1024 : 16) || top > 64 || d % 8 || !al16(h) || !al16(wr) || !al16(wsg) || (!ws && route_lds<16, true>(a) > MAX_LDS)) return 10;
   const GroupArgs g{(const int*)ids, T * top, real, mt, (int*)perm, (int*)inv, (int*)tiles, (int*)ntiles};
   if (!group_ok(g, max_tiles)) return 1;
-  if (ws) return split_go<true>(a, g, ws, ws_floats, cnt, cnt_n, s);
+  if (ws) return T > 16 ? split_go<2>(a, g, ws, ws_floats, cnt, cnt_n, s) : split_go<1>(a, g, ws, ws_floats, cnt, cnt_n, s);
   return route_go<16, true>(a, g, s);
 }
 
