@@ -201,6 +201,10 @@ __device__ __forceinline__ float gelu_tanh(float x) {
   return 0.5f * x * (1.f + fast_tanh(u));
 }
 
+__device__ __forceinline__ float gelu_erf(float x) {
+  return 0.5f * x * (1.f + erff(x * 0.7071067811865476f));
+}
+
 __device__ __forceinline__ float gelu_tanh_grad(float x) {
   const float k0 = 0.7978845608028654f, k1 = 0.044715f;
   float x2 = x * x;

@@ -8,9 +8,6 @@
 // NeoX-20B, BLOOM) or exact erf ("gelu": Pythia). The bias add is fused into
 // the producing hipBLASLt GEMM epilogue (addmm), so the activation kernel only
 // needs the pre-activation.
-__device__ __forceinline__ float gelu_erf(float x) {
-  return 0.5f * x * (1.f + erff(x * 0.7071067811865476f));
-}
 __device__ __forceinline__ float gelu_erf_grad(float x) {
   const float cdf = 0.5f * (1.f + erff(x * 0.7071067811865476f));
   const float pdf = 0.3989422804014327f * __expf(-0.5f * x * x);

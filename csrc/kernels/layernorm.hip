@@ -22,27 +22,27 @@ __global__ void __launch_bounds__(256) ln_fwd_kernel(
     const bf16_t* __restrict__ r2, bf16_t* __restrict__ h_out,
     const bf16_t* __restrict__ gamma, const bf16_t* __restrict__ beta,
     bf16_t* __restrict__ y, float* __restrict__ mean_out,
-    float* __restrict__ rstd_out, int rows, int d, float eps) {
+    float* __restrict__ rstd_out, int rows, int d, float eps, const long long* __restrict__ idx) {
   __shared__ float red[16];
   const int nvec = d >> 3;
   for (int row = blockIdx.x; row < rows; row += gridDim.x) {
-    const size_t base = (size_t)row * d;
+    const size_t base = (size_t)row * d, from = idx ? (size_t)idx[row] * d : base;  // idx: input row of an output row
     float v[NV][8];
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int vi = threadIdx.x + i * blockDim.x;
       if (vi < nvec) {
-        load8(x + base + vi * 8, v[i]);
+        load8(x + from + vi * 8, v[i]);
         if (r1) {
           float t[8];
-          load8(r1 + base + vi * 8, t);
+          load8(r1 + from + vi * 8, t);
 #pragma unroll
           for (int j = 0; j < 8; ++j) v[i][j] += t[j];
         }
         if (r2) {
           float t[8];
-          load8(r2 + base + vi * 8, t);
+          load8(r2 + from + vi * 8, t);
 #pragma unroll
           for (int j = 0; j < 8; ++j) v[i][j] += t[j];
         }
@@ -357,8 +357,21 @@ KCA_API int kca_layernorm_fwd(const void* x, const void* r1, const void* r2,
                                      (const bf16_t*)x, (const bf16_t*)r1,
                                      (const bf16_t*)r2, (bf16_t*)h_out,
                                      (const bf16_t*)gamma, (const bf16_t*)beta,
-                                     (bf16_t*)y, mean, rstd, rows, d, eps));
+                                     (bf16_t*)y, mean, rstd, rows, d, eps, nullptr));
   return 0;
+}
+
+// y[i] = LayerNorm(x[idx[i]] (+ r1[idx[i]]) (+ r2[idx[i]])): a few rows of many, without the sum and the statistics
+KCA_API int kca_layernorm_rows_fwd(const void* x, const void* r1, const void* r2, const long long* idx, const void* gamma,
+                                   const void* beta, void* y, int rows, int d, float eps, hipStream_t stream) {
+  if (d < 8 || d % 8 || rows < 1 || !x || !idx || !gamma || !y) return 1;
+  int nv, threads;
+  ln_geometry(d, nv, threads);
+  const int grid = rows < 65535 * 4 ? rows : 65535 * 4;
+  LN_DISPATCH(nv, hipLaunchKernelGGL((ln_fwd_kernel<NV>), dim3(grid), dim3(threads), 0, stream, (const bf16_t*)x,
+                                     (const bf16_t*)r1, (const bf16_t*)r2, nullptr, (const bf16_t*)gamma, (const bf16_t*)beta,
+                                     (bf16_t*)y, nullptr, nullptr, rows, d, eps, idx));
+  return hipGetLastError() == hipSuccess ? 0 : 4;
 }
 
 // workspace: 2 * nparts * d floats, nparts = kca_layernorm_bwd_parts(rows).

@@ -11,12 +11,18 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int NB = 64, SK = 64, ROWS = 128;  // weight rows a block, K a stage, activation rows at most
 
-struct RowsArgs {
+struct RowsPart {
   const void *x, *w, *bias;
   void* y;
+  int N, K, act;  // act: 0 none, GELU 1 tanh, 2 erf
+};
+struct RowsArgs {
+  // p[0], and beside it p[1] with blocks of its own (beside), or p[1]'s x and W along K: y[0] = x0 W0^T + x1 W1^T + both biases
+  // (p[1].K without beside). p[1].K == 0: one product.
+  RowsPart p[2];
   float* ws;      // ks > 1: [block][slice][product tile][2][256 threads][2]
   unsigned* cnt;  // ks > 1: one arrival counter a block, zero before and after
-  int M, N, K, ks;
+  int M, ks, beside;
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rsrc(const void* p) {
@@ -86,7 +92,8 @@ __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
 // A call costs the host 14 us, the library's through the tuned table 20 to 26: four GPT-J layers on 61 tokens 944 -> 769 us.
 // Which sizes run here: few_rows in ops/linear.py.
 // XR activation rows; 4 waves, WM of them across the activation rows; SNB stages.
-template <bool F16, int XR, int WM, int SNB>
+// TWO: another product beside this one, or more of K (RowsArgs).
+template <bool F16, int XR, int WM, int SNB, bool TWO>
 __global__ void __launch_bounds__(256, 2) rows_mm_kernel(RowsArgs p) {
   constexpr int WN = 4 / WM, A = NB / WN / 16, B = XR / WM / 16;  // a wave's runs of 16 weight and activation rows
   constexpr int STG = (NB + XR) * SK * 2, WI = NB / 32, XI = XR / 32, PER = WI + XI;
@@ -94,34 +101,49 @@ __global__ void __launch_bounds__(256, 2) rows_mm_kernel(RowsArgs p) {
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wn = wv % WN, wm = wv / WN;
   const int r16 = lane & 15, g = lane >> 4;
   const int id = xcd_remap(blockIdx.x, gridDim.x);  // the slices of a block on one XCD, beside their partial sums
-  const int blk = id / p.ks, z = id % p.ks, n0 = blk * NB, K = p.K;
-  const int nk = K / SK, t0 = (int)((long long)nk * z / p.ks), t1 = (int)((long long)nk * (z + 1) / p.ks);
-  const __amdgpu_buffer_rsrc_t rw = uniform_rsrc(p.w), rx = uniform_rsrc(p.x);
-  unsigned wo[WI], xo[XI];
+  const int blk = id / p.ks, z = id % p.ks;
+  const int nb0 = (p.p[0].N + NB - 1) / NB;
+  const bool second = TWO && p.beside && blk >= nb0;
+  const RowsPart q = second ? p.p[1] : p.p[0];
+  const int n0 = (second ? blk - nb0 : blk) * NB;
+  const int K2 = TWO && !p.beside ? p.p[1].K : 0;
+  const int nka = q.K / SK, nk = nka + K2 / SK;
+  const int t0 = (int)((long long)nk * z / p.ks), t1 = (int)((long long)nk * (z + 1) / p.ks);
+  const __amdgpu_buffer_rsrc_t rw = uniform_rsrc(q.w), rx = uniform_rsrc(q.x);
+  const __amdgpu_buffer_rsrc_t rw2 = uniform_rsrc(p.p[1].w), rx2 = uniform_rsrc(p.p[1].x);
+  unsigned wo[WI], xo[XI], wo2[WI], xo2[XI];
+  auto offsets = [&](int K, unsigned (&w)[WI], unsigned (&x)[XI]) {
 #pragma unroll
-  for (int i = 0; i < WI; ++i) {
-    const int r = wv * 8 * WI + 8 * i + (lane >> 3);
-    wo[i] = ((unsigned)min(n0 + r, p.N - 1) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
-  }
+    for (int i = 0; i < WI; ++i) {
+      const int r = wv * 8 * WI + 8 * i + (lane >> 3);
+      w[i] = ((unsigned)min(n0 + r, q.N - 1) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
+    }
 #pragma unroll
-  for (int i = 0; i < XI; ++i) {
-    const int r = wv * 8 * XI + 8 * i + (lane >> 3);
-    xo[i] = ((unsigned)min(r, p.M - 1) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
-  }
+    for (int i = 0; i < XI; ++i) {
+      const int r = wv * 8 * XI + 8 * i + (lane >> 3);
+      x[i] = ((unsigned)min(r, p.M - 1) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
+    }
+  };
+  offsets(q.K, wo, xo);
+  if (TWO) offsets(K2, wo2, xo2);
   typedef __attribute__((address_space(3))) char lds_char;
   lds_char* lsm = (lds_char*)sl;
   auto issue = [&](int t) {
-    const int k = __builtin_amdgcn_readfirstlane(min(t, t1 - 1) * SK * 2);  // the last stages repeat one that nobody reads
+    const int tt = __builtin_amdgcn_readfirstlane(min(t, t1 - 1));  // the last stages repeat one that nobody reads
     lds_char* st = lsm + ((t - t0) % SNB) * STG;
 #if defined(__HIP_DEVICE_COMPILE__)
+    auto fill = [&](__amdgpu_buffer_rsrc_t fw, __amdgpu_buffer_rsrc_t fx, const unsigned (&w)[WI], const unsigned (&x)[XI], int k) {
 #pragma unroll
-    for (int i = 0; i < WI; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (void __attribute__((address_space(3)))*)(st + (wv * WI + i) * 1024), 16,
-                                               wo[i], k, 0, 0);
+      for (int i = 0; i < WI; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(fw, (void __attribute__((address_space(3)))*)(st + (wv * WI + i) * 1024), 16,
+                                                 w[i], k, 0, 0);
 #pragma unroll
-    for (int i = 0; i < XI; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rx, (void __attribute__((address_space(3)))*)(st + (NB / 8 + wv * XI + i) * 1024), 16, xo[i], k, 0, 0);
+      for (int i = 0; i < XI; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            fx, (void __attribute__((address_space(3)))*)(st + (NB / 8 + wv * XI + i) * 1024), 16, x[i], k, 0, 0);
+    };
+    if (!TWO || tt < nka) fill(rw, rx, wo, xo, tt * SK * 2);
+    else fill(rw2, rx2, wo2, xo2, (tt - nka) * SK * 2);
 #endif
   };
   f32x4 acc[A][B];
@@ -200,22 +222,27 @@ __global__ void __launch_bounds__(256, 2) rows_mm_kernel(RowsArgs p) {
 #pragma unroll
   for (int i = 0; i < A; ++i) {
     const int n = n0 + (wn * A + i) * 16 + 4 * g;
-    if (n >= p.N) continue;
+    if (n >= q.N) continue;
     float b[4] = {0.f, 0.f, 0.f, 0.f};
-    if (p.bias) {
+    auto add_bias = [&](const void* bias) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const unsigned short v = reinterpret_cast<const unsigned short*>(p.bias)[n + e];
-        b[e] = F16 ? (float)__builtin_bit_cast(_Float16, v) : bf2f(v);
+        const unsigned short v = reinterpret_cast<const unsigned short*>(bias)[n + e];
+        b[e] += F16 ? (float)__builtin_bit_cast(_Float16, v) : bf2f(v);
       }
-    }
+    };
+    if (q.bias) add_bias(q.bias);
+    if (TWO && K2 && p.p[1].bias) add_bias(p.p[1].bias);
 #pragma unroll
     for (int j = 0; j < B; ++j) {
       const int m = (wm * B + j) * 16 + r16;
       if (m >= p.M) continue;
       float o[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = acc[i][j][e] + b[e];
+      for (int e = 0; e < 4; ++e) {
+        o[e] = acc[i][j][e] + b[e];
+        if (q.act) o[e] = q.act == 1 ? gelu_tanh(o[e]) : gelu_erf(o[e]);
+      }
       uint2 v;
       if constexpr (F16) {
         const _Float16 h[4] = {(_Float16)o[0], (_Float16)o[1], (_Float16)o[2], (_Float16)o[3]};
@@ -223,19 +250,49 @@ __global__ void __launch_bounds__(256, 2) rows_mm_kernel(RowsArgs p) {
       } else {
         v = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
       }
-      *reinterpret_cast<uint2*>(reinterpret_cast<unsigned short*>(p.y) + (long long)m * p.N + n) = v;
+      *reinterpret_cast<uint2*>(reinterpret_cast<unsigned short*>(q.y) + (long long)m * q.N + n) = v;
     }
   }
 }
 
-template <bool F16, int XR, int WM, int SNB>
-int go(const RowsArgs& a, hipStream_t s) {
+template <bool F16, int XR, int WM, int SNB, bool TWO>
+int go_as(const RowsArgs& a, hipStream_t s) {
   constexpr int lds = SNB * (NB + XR) * SK * 2;
-  if (hipFuncSetAttribute((const void*)rows_mm_kernel<F16, XR, WM, SNB>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) !=
+  if (hipFuncSetAttribute((const void*)rows_mm_kernel<F16, XR, WM, SNB, TWO>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) !=
       hipSuccess)
     return 5;
-  hipLaunchKernelGGL((rows_mm_kernel<F16, XR, WM, SNB>), dim3((a.N + NB - 1) / NB * a.ks), dim3(256), lds, s, a);
+  const int blocks = (a.p[0].N + NB - 1) / NB + (a.beside ? (a.p[1].N + NB - 1) / NB : 0);
+  hipLaunchKernelGGL((rows_mm_kernel<F16, XR, WM, SNB, TWO>), dim3(blocks * a.ks), dim3(256), lds, s, a);
   return hipGetLastError() == hipSuccess ? 0 : 4;
+}
+template <bool F16, int XR, int WM, int SNB>
+int go(const RowsArgs& a, hipStream_t s) {
+  return a.p[1].K ? go_as<F16, XR, WM, SNB, true>(a, s) : go_as<F16, XR, WM, SNB, false>(a, s);
+}
+
+// Checks what the kernel asks of its arguments and launches it
+int rows_mm(int dtype, const RowsArgs& a, long long ws_floats, int cnt_n, hipStream_t s) {
+  if ((dtype != 1 && dtype != 2) || a.M < 1 || a.M > ROWS || a.ks < 1) return 1;
+  const int parts = a.p[1].K ? 2 : 1;
+  long long blocks = 0, stages = 0;
+  for (int i = 0; i < parts; ++i) {
+    const RowsPart& q = a.p[i];
+    const bool out = i == 0 || a.beside;  // has rows of its own
+    if (!q.x || !q.w || (out && !q.y) || q.N < 16 || q.N % 16 || q.K < SK || q.K % SK || q.act < 0 || q.act > 2) return 1;
+    if (!out && q.N != a.p[0].N) return 1;
+    if (a.beside && a.ks > q.K / SK) return 1;
+    if (!al16(q.x) || !al16(q.w) || (out && (uintptr_t)q.y % 8)) return 2;
+    if (2ll * (q.N > a.M ? q.N : a.M) * q.K >= 1ll << 32) return 3;  // (32-bit byte offsets into W and x)
+    if (out) blocks += (q.N + NB - 1) / NB;
+    stages += q.K / SK;
+  }
+  if (!a.beside && a.ks > stages) return 1;
+  const long long xr = a.M <= 32 ? 32 : a.M <= 64 ? 64 : 128;
+  if (blocks * a.ks >= 1ll << 31) return 3;
+  if (a.ks > 1 && (!a.ws || !a.cnt || !al16(a.ws) || ws_floats < blocks * a.ks * NB * xr || cnt_n < blocks)) return 6;
+  if (xr == 32) return dtype == 2 ? go<true, 32, 1, 6>(a, s) : go<false, 32, 1, 6>(a, s);
+  if (xr == 64) return dtype == 2 ? go<true, 64, 1, 5>(a, s) : go<false, 64, 1, 5>(a, s);
+  return dtype == 2 ? go<true, 128, 2, 3>(a, s) : go<false, 128, 2, 3>(a, s);
 }
 
 }  // namespace
@@ -245,16 +302,16 @@ int go(const RowsArgs& a, hipStream_t s) {
 // blocks = ceil(N / 64). Other sizes return a status and launch nothing.
 KCA_API int kca_rows_mm(int dtype, const void* x, const void* w, const void* bias, void* y, float* ws, unsigned* cnt,
                         long long ws_floats, int cnt_n, int M, int N, int K, int ks, hipStream_t s) {
-  if ((dtype != 1 && dtype != 2) || !x || !w || !y || M < 1 || M > ROWS || N < 16 || N % 16 || K < SK || K % SK || ks < 1 ||
-      ks > K / SK)
-    return 1;
-  if (!al16(x) || !al16(w) || (uintptr_t)y % 8) return 2;
-  if (2ll * (N > M ? N : M) * K >= 1ll << 32) return 3;  // (32-bit byte offsets into W and x)
-  const long long blocks = (N + NB - 1) / NB, xr = M <= 32 ? 32 : M <= 64 ? 64 : 128;
-  if (blocks * ks >= 1ll << 31) return 3;
-  if (ks > 1 && (!ws || !cnt || !al16(ws) || ws_floats < blocks * ks * NB * xr || cnt_n < blocks)) return 6;
-  const RowsArgs a{x, w, bias, y, ws, cnt, M, N, K, ks};
-  if (xr == 32) return dtype == 2 ? go<true, 32, 1, 6>(a, s) : go<false, 32, 1, 6>(a, s);
-  if (xr == 64) return dtype == 2 ? go<true, 64, 1, 5>(a, s) : go<false, 64, 1, 5>(a, s);
-  return dtype == 2 ? go<true, 128, 2, 3>(a, s) : go<false, 128, 2, 3>(a, s);
+  return rows_mm(dtype, RowsArgs{{{x, w, bias, y, N, K, 0}, {}}, ws, cnt, M, ks, 0}, ws_floats, cnt_n, s);
+}
+
+// One product with a GELU (act: 0 none, 1 tanh, 2 erf) on its fp32 sums (x2 null), or two: beside each other, y2 [M, N2] =
+// act2(x2 W2^T + bias2) in blocks of its own, or (beside 0) along K: y = act(x W^T + x2 W2^T + bias + bias2), N2 == N. Blocks: both
+// products' where they lie beside each other.
+KCA_API int kca_rows_mm_two(int dtype, int beside, const void* x, const void* w, const void* bias, void* y, int N, int K, int act,
+                            const void* x2, const void* w2, const void* bias2, void* y2, int N2, int K2, int act2, float* ws,
+                            unsigned* cnt, long long ws_floats, int cnt_n, int M, int ks, hipStream_t s) {
+  if (x2 && K2 < SK) return 1;
+  return rows_mm(dtype, RowsArgs{{{x, w, bias, y, N, K, act}, {x2, w2, bias2, y2, N2, x2 ? K2 : 0, act2}}, ws, cnt, M, ks, x2 && beside},
+                 ws_floats, cnt_n, s);
 }

@@ -36,7 +36,10 @@ from .. import ops
 from ..ops import decode as dops
 from ..ops import _lib
 from ..ops import skinny_mm as smm
+from ..models.causal_lm import MLP, LayerNorm
 from ..ops.gemv import embed_ln_rows, ln_rows, ln_skinny_linear, skinny_linear
+from ..ops.linear import FEW_ROWS, TLinear, few_rows_beside, few_rows_gelu, few_rows_sum
+from ..ops.norms import layer_norm_rows
 from ..utils import capture
 
 # decode steps: each row's RoPE angles and page-table row travel with the step's packed inputs (fixed
@@ -160,10 +163,17 @@ class KVCache:
         self._dirty = True
 
     def sync(self):
-        """Block-table edits -> device (stream-ordered after the work already queued)."""
+        """Block-table edits -> device (stream-ordered after the work already queued). From a pinned copy, whose memory the
+        allocator holds until the upload is done: from the table itself the host would wait for all that is queued, so a prompt
+        would not be issued while the one before it runs."""
         if self.paged and self._dirty:
-            for t in self.tables.values():
-                t.copy_(self.table_h)
+            for d, t in self.tables.items():
+                if d == self.device and d.type == "cuda" and not torch.cuda.is_current_stream_capturing():
+                    host = torch.empty(self.table_h.shape, dtype=torch.int32, pin_memory=True)
+                    host.copy_(self.table_h)
+                    t.copy_(host, non_blocking=True)
+                else:
+                    t.copy_(self.table_h)
             self._dirty = False
 
     def table_on(self, dev):
@@ -884,22 +894,48 @@ class ModelRunner(StepRunner):
         self.seen.view(-1).index_fill_(0, mark, 1)
         h = m.embed(tok[None], None if m.wpe is None else pos.long())
         pending = ()
+        few = rows <= FEW_ROWS and not torch.cuda.is_current_stream_capturing()
         for li, blk in enumerate(m.h):
             x, h = blk.ln_1(h, residual=pending) if pending else (blk.ln_1(h), h)
-            at = blk.attn
-            q, k, v = at.qkv(x).view(rows, 3, self.H, self.D).unbind(1)
+            at, mlp = blk.attn, blk.mlp
+            # few rows: a launch costs what it streams and some 6 us, so a parallel MLP's products share the attention's
+            pair, plain = None, self._plain_products(blk) if few else None
+            if plain and cfg.parallel_residual:
+                pair = few_rows_beside((x, *plain[0]), (x if blk.ln_2 is None else blk.ln_2(h), *plain[2]), mlp.approx)
+            q, k, v = (at.qkv(x) if pair is None else pair[0]).view(rows, 3, self.H, self.D).unbind(1)
             if not ops.rope_append(q, k, v, self.rot, cfg.rotary_interleaved, self.cos, self.sin, pos, page, off,
                                    self.cache.k[li], self.cache.v[li]):
                 raise RuntimeError("rope_append: the projection's rows are not 16-byte aligned")
-            o = ops.packed_attention(q, k, v, cu, longest, at.scale, at.alibi, at.window)
-            a = at.out(o.view(1, rows, -1))
+            o = ops.packed_attention(q, k, v, cu, longest, at.scale, at.alibi, at.window).view(1, rows, -1)
+            if pair is not None:
+                y = few_rows_sum((pair[1], *plain[3]), (o, *plain[1]))
+                pending = (y,) if y is not None else (at.out(o), mlp.fc_out(pair[1]))
+                continue
+            a = at.out(o)
             if cfg.parallel_residual:
-                pending = (a, blk.mlp(x if blk.ln_2 is None else blk.ln_2(h)))
+                pending = (a, mlp(x if blk.ln_2 is None else blk.ln_2(h)))
             else:
                 x2, h = blk.ln_2(h, residual=(a,))
-                pending = (blk.mlp(x2),)
-        y, _ = m.ln_f(h[:, last], residual=tuple(p_[:, last] for p_ in pending))
+                u = few_rows_gelu(x2, *plain[2], mlp.approx) if plain else None
+                pending = (mlp(x2) if u is None else mlp.fc_out(u),)
+        if type(m.ln_f) is LayerNorm and not (m.ln_f._forward_hooks or m.ln_f._forward_pre_hooks):
+            y = layer_norm_rows(h[0], m.ln_f.weight, m.ln_f.bias, m.ln_f.eps, tuple(p_[0] for p_ in pending), last)[None]
+        else:
+            y, _ = m.ln_f(h[:, last], residual=tuple(p_[:, last] for p_ in pending))
         return m.logits_from_hidden(y)[0]
+
+    @staticmethod
+    def _plain_products(blk):
+        """(weight, bias) of a block's QKV, out, fc_in and fc_out layers where these are plain linear layers without hooks, so
+        that they may be taken apart and put together; else None."""
+        mlp = blk._modules["mlp"]
+        if type(mlp) is not MLP or mlp._forward_hooks or mlp._forward_pre_hooks:
+            return None
+        a, b = blk._modules["attn"]._modules, mlp._modules
+        mods = (a["qkv"], a["out"], b["fc_in"], b["fc_out"])
+        if any(type(x) is not TLinear or x._forward_hooks or x._forward_pre_hooks for x in mods):
+            return None
+        return tuple((x.weight, x.bias) for x in mods)
 
     def _continued_attention(self, li, q, slots, lens, start, at):
         """Chunk queries [start, start + L) of each row against the slot's cached

@@ -250,6 +250,74 @@ def linear_rows(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None
     return y.view(*x.shape[:-1], n)
 
 
+ACTS = {None: 0, "tanh": 1, "none": 2}  # none, GELU (tanh form, erf form)
+
+
+def _few_part(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, rows: int) -> bool:
+    n, k = weight.shape
+    return (few_rows(rows, n, k) and x.dtype in (torch.bfloat16, torch.float16) and x.dtype == weight.dtype
+            and x.numel() == rows * k and x.is_contiguous() and weight.is_contiguous() and n % 16 == 0 and k % 64 == 0
+            and 2 * max(n, rows) * k < 1 << 32 and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+            and (bias is None or (bias.shape == (n,) and bias.dtype == x.dtype and bias.is_contiguous())))
+
+
+def _few_launch(parts, act: int, act2: int, beside: bool, rows: int):
+    """One launch of ``kca_rows_mm_two`` over one or two (x, weight, bias); None: sizes, types or a mode of torch (gradients,
+    transforms, captures, ...) that it does not serve."""
+    x = parts[0][0]
+    if (not 0 < rows <= FEW_ROWS or not x.is_cuda or torch.cuda.is_current_stream_capturing()
+            or not all(p[0].dtype == x.dtype and _few_part(*p, rows) for p in parts)
+            or not _lib.inference(*(t for p in parts for t in p)) or not _lib.has("kca_rows_mm_two")):
+        return None
+    outs = [torch.empty(rows, p[1].shape[0], device=x.device, dtype=x.dtype) for p in (parts if beside else parts[:1])]
+    blocks = sum(-(-y.shape[1] // 64) for y in outs)
+    k = min(p[1].shape[1] for p in parts) if beside else sum(p[1].shape[1] for p in parts)
+    ks, ws, cnt = max(1, min(_CUS // blocks, k // 512)), None, None  # (about one block a CU, as _k_slices)
+    if ks > 1:
+        ws = torch.empty(blocks * ks * 64 * (32 if rows <= 32 else 64 if rows <= 64 else 128), device=x.device, dtype=torch.float32)
+        cnt = _lib.counters(x.device, blocks)
+    a = []
+    for i in range(2):
+        if i < len(parts):
+            px, w, b = parts[i]
+            a += [px.data_ptr(), w.data_ptr(), _lib.ptr(b), outs[i].data_ptr() if i < len(outs) else None, *w.shape, (act, act2)[i]]
+        else:
+            a += [None, None, None, None, 0, 0, 0]
+    _lib.call("kca_rows_mm_two", 1 if x.dtype == torch.bfloat16 else 2, int(beside), *a, _lib.ptr(ws), _lib.ptr(cnt),
+              0 if ws is None else ws.numel(), 0 if cnt is None else cnt.numel(), rows, ks, _lib.stream())
+    return outs
+
+
+def few_rows_gelu(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, approx: str) -> torch.Tensor | None:
+    """gelu(x W^T + bias) of few rows in one launch, the GELU on the fp32 sums; None: a call that ``linear_rows`` and
+    ``ops.gelu`` serve."""
+    rows = x.numel() // x.shape[-1]
+    y = _few_launch([(x, weight, bias)], ACTS[approx], 0, False, rows) if approx in ACTS else None
+    return None if y is None else y[0].view(*x.shape[:-1], -1)
+
+
+def few_rows_beside(first: tuple, second: tuple, approx2: str | None = None):
+    """Two products (x, weight, bias) of the same few rows in one launch, a GELU on the second's fp32 sums -> (y, y2) or None.
+    On the GPU, us, apart and together, 61 rows: 12288 and 16384 x 4096 26.5 + 32.1, 52.0; 6144 and 8192 x 2048 11.4 + 12.4, 16.7 (two
+    blocks a CU 20.8); 128 rows 34.6 + 37.5, 65.1; and a launch and the GELU's less."""
+    x = first[0]
+    rows = x.numel() // x.shape[-1]
+    y = _few_launch([first, second], 0, ACTS[approx2], True, rows) if approx2 in ACTS else None
+    return None if y is None else tuple(t.view(*x.shape[:-1], -1) for t in y)
+
+
+def few_rows_sum(first: tuple, second: tuple) -> torch.Tensor | None:
+    """The sum of two products (x, weight, bias) of the same few rows in one launch, rounded once; or None. On the GPU, us, apart and
+    together, 61 rows: 4096 x 16384 and x 4096 33.9 + 13.1, 37.3 (two blocks a CU 46.9); 2048 x 8192 and x 2048 14.2 + 9.1, 16.2;
+    128 rows 42.6 + 17.8, 50.2."""
+    x = first[0]
+    rows = x.numel() // x.shape[-1]
+    if first[1].shape[0] != second[1].shape[0]:
+        return None
+    y = _few_launch([first, second], 0, 0, False, rows)
+    return None if y is None else y[0].view(*x.shape[:-1], -1)
+
+
 # ---------------------------------------------------------------- split-K weight gradients
 def _wgrad_splits(tokens: int, n: int, k: int) -> int:
     """Token chunks for dW = dY^T X: one hipBLASLt GEMM leaves most CUs idle when the output is

@@ -64,6 +64,14 @@ class _LayerNormFn(torch.autograd.Function):
         return dx, dw, db, None, g1, g2
 
 
+def _plain_rows(x, weight, bias, residual) -> bool:
+    """Inference on contiguous bf16 rows with bf16 parameters."""
+    d = x.shape[-1]
+    return (_lib.inference(x, weight, bias, *residual) and x.numel() > 0 and weight is not None and weight.shape == (d,)
+            and (bias is None or bias.shape == (d,)) and all(r.shape == x.shape for r in residual)
+            and all(t is None or (t.dtype == torch.bfloat16 and t.is_contiguous()) for t in (x, weight, bias, *residual)))
+
+
 def _rows_f16(x, weight, bias, residual) -> bool:
     d = x.shape[-1]
     return (_lib.has("kca_ln_rows_f16") and _lib.native_f16(x, weight, bias, *residual) and d % 8 == 0 and 0 < d <= 16384 and x.numel() > 0
@@ -83,6 +91,12 @@ def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
     if len(residual) > 2:
         raise ValueError("at most two fused residual adds")
     if _lib.use_native(x):
+        if _plain_rows(x, weight, bias, residual):  # no statistics, no node
+            d = x.shape[-1]
+            h, y = torch.empty_like(x) if residual else None, torch.empty_like(x)
+            _lib.call("kca_layernorm_fwd", x.data_ptr(), _lib.ptr(r1), _lib.ptr(r2), _lib.ptr(h), weight.data_ptr(), _lib.ptr(bias),
+                      y.data_ptr(), None, None, x.numel() // d, d, float(eps), _lib.stream())
+            return (y, h) if residual else y
         y, h = _LayerNormFn.apply(x, weight, bias, eps, r1, r2)
         return (y, h) if residual else y
     if (weight is not None and _lib.native_f16(x) and _lib.inference(x, weight, bias, *residual)
@@ -98,6 +112,22 @@ def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
         h = h + r
     y = _ln_ref(h, weight, bias, eps)
     return (y, h) if residual else y
+
+
+def layer_norm_rows(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, eps: float, residual: tuple,
+                    rows: torch.Tensor) -> torch.Tensor:
+    """LayerNorm of rows ``rows`` (int64) of ``x + sum(residual)``, [T, d] each (inference): a prompt's last rows."""
+    if (x.dim() == 2 and _lib.use_native(x) and len(residual) <= 2 and x.shape[-1] % 8 == 0 and rows.numel()
+            and rows.dtype == torch.int64 and rows.is_contiguous() and _plain_rows(x, weight, bias, residual)
+            and rows.device == x.device):
+        d = x.shape[-1]
+        y = torch.empty(rows.numel(), d, device=x.device, dtype=x.dtype)
+        r1, r2 = (*residual, None, None)[:2]
+        _lib.call("kca_layernorm_rows_fwd", x.data_ptr(), _lib.ptr(r1), _lib.ptr(r2), rows.data_ptr(), weight.data_ptr(),
+                  _lib.ptr(bias), y.data_ptr(), rows.numel(), d, float(eps), _lib.stream())
+        return y
+    y = layer_norm(x[rows], weight, bias, eps, tuple(r[rows] for r in residual))
+    return y[0] if residual else y
 
 
 # ------------------------------------------------------------------ GroupNorm
