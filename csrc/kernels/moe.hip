@@ -230,14 +230,26 @@ struct GroupArgs {
   int *perm, *inv, *tiles, *ntiles;
 };
 
+// Whether the last tile of an expert with `c` rows stands after all experts' others (row limits of 128 and more): it is at most half
+// full, and what its weights cost to read again, away from the expert's other tiles, is less than the CUs that it fills: two full
+// tiles before it, or none, or one of 256 rows, which the matrix cores bound, and hardly any rows. Both products, us (width, experts,
+// top, inner size), beside its expert's and last: 2000 tokens, 4096, 16, 2, 4096 652, 608; 4096 of them 934, 910; 3000, 2048, 32, 4,
+// 1024 237, 215; 300, 4096, 16, 3, 2048 218, 199. 1200 of these (one of 128 rows and about 52) 277, 294 with all such tiles last,
+// 282 with those of up to 16 rows.
+__device__ __forceinline__ bool late_tile(int c, int mt) {
+  const int r = c % mt, full = c / mt;
+  return mt >= 128 && r && 2 * r <= mt && (full != 1 || (mt > 128 && 8 * r <= mt));
+}
+
 // n assignments -> perm (sorted position -> assignment), inv (assignment -> sorted position), tiles
 // [ntiles][5] (expert, first sorted position, rows <= mt, first tile and tile count of the expert) and
-// their count. One workgroup of NT threads;
-// sh: 3 E + 2 ints.
+// their count. Late tiles stand after all others, each by itself, so that a product takes them last (expert_gemm_kernel). One workgroup
+// of NT threads;
+// sh: 4 E + 3 ints.
 template <int NT>
 __device__ __forceinline__ void group_rows(const GroupArgs& p, int* sh) {
   const int E = p.E, n = p.n, mt = p.mt, tid = threadIdx.x;
-  int *cnt = sh, *off = sh + E, *toff = off + E + 1;
+  int *cnt = sh, *off = sh + E, *toff = off + E + 1, *soff = toff + E + 1;
   constexpr int R = 4;  // a thread's first ids, read once for both passes
   int first[R];
 #pragma unroll
@@ -255,31 +267,35 @@ __device__ __forceinline__ void group_rows(const GroupArgs& p, int* sh) {
   });
   __syncthreads();
   if (tid < 64) {  // exclusive sums over the experts, 64 at a time
-    int co = 0, to = 0;
+    int co = 0, to = 0, so = 0;
     for (int e0 = 0; e0 < E; e0 += 64) {
-      const int e = e0 + tid, c = e < E ? cnt[e] : 0, t = (c + mt - 1) / mt;
+      const int e = e0 + tid, c = e < E ? cnt[e] : 0, small = late_tile(c, mt), t = (c + mt - 1) / mt - small;
       int cs = c, ts = t;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
         const int a = __shfl_up(cs, o, 64), b = __shfl_up(ts, o, 64);
         if (tid >= o) cs += a, ts += b;
       }
-      if (e < E) off[e] = co + cs - c, toff[e] = to + ts - t;
+      const unsigned long long m = __ballot(small);
+      if (e < E) off[e] = co + cs - c, toff[e] = to + ts - t, soff[e] = so + __popcll(m & ((1ull << tid) - 1));
       co += __shfl(cs, 63, 64);
       to += __shfl(ts, 63, 64);
+      so += __popcll(m);
     }
-    if (tid == 0) off[E] = co, toff[E] = to, *p.ntiles = to;
+    if (tid == 0) off[E] = co, toff[E] = to, *p.ntiles = to + so;
   }
   __syncthreads();
   for (int e = tid; e < E; e += NT) {
-    const int c = cnt[e];
-    for (int j = 0; j * mt < c; ++j) {
-      int* t = p.tiles + (toff[e] + j) * 5;
+    const int c = cnt[e], nt = (c + mt - 1) / mt, small = late_tile(c, mt);
+    for (int j = 0; j < nt; ++j) {
+      const bool last = small && j == nt - 1;  // (it stands alone)
+      const int at = last ? toff[E] + soff[e] : toff[e] + j;
+      int* t = p.tiles + at * 5;
       t[0] = e;
       t[1] = off[e] + j * mt;
       t[2] = min(mt, c - j * mt);
-      t[3] = toff[e];
-      t[4] = (c + mt - 1) / mt;
+      t[3] = last ? at : toff[e];
+      t[4] = last ? 1 : nt - small;
     }
     cnt[e] = off[e];
   }
@@ -387,7 +403,7 @@ __global__ void __launch_bounds__(NW * 64) route_mfma_kernel(RouteArgs p, GroupA
 template <int GROUP>
 __global__ void __launch_bounds__(1024) route_split_kernel(RouteArgs p, GroupArgs gr, float* parts, unsigned* cnt) {
   __shared__ __attribute__((aligned(16))) float z[16 * 64];
-  __shared__ int sids[GROUP == 1 ? 16 * 64 : 1], sh[GROUP ? 3 * 64 + 2 : 1], s_last;
+  __shared__ int sids[GROUP == 1 ? 16 * 64 : 1], sh[GROUP ? 4 * 64 + 3 : 1], s_last;
   const int n = p.E + (p.wsg ? 1 : 0), nt = (n + 15) / 16, d = p.d, nk = (d + 31) / 32;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, r16 = lane & 15, g = lane >> 4;
   const int tb = blockIdx.x / 4, cut = blockIdx.x % 4 * 4 + (wv & 3), t0 = tb * 16;
@@ -497,6 +513,7 @@ struct ExpertArgs {
   const float* wts;     // [n] by assignment
   const int* tiles;
   const int* ntiles;
+  int mt;               // row limit of a tile
   int top, N, K, up, scale;  // up: gate-and-up (x gathered by token, silu product); scale: the weight applies here
   // gemv: a shared expert beside them, `tokens` rows in order, without a weight (ws null: none)
   const void* xs;       // [tokens][Ks]
@@ -916,9 +933,23 @@ __global__ void __launch_bounds__(256, NARROW ? 2 : 1) expert_gemm_kernel(Expert
   constexpr int NB = (NARROW ? 128 : 256) / (UP ? 2 : 1);
   const int nt = *p.ntiles, nb = (p.N + NB - 1) / NB;
   if ((int)blockIdx.x >= nt * nb) return;
-  const int id = xcd_remap(blockIdx.x, nt * nb);
+  // late tiles (late_tile: alone, at most half full, after all others) fill the CUs that the last long blocks leave idle
+  int id = xcd_remap(blockIdx.x, nt * nb);
   const int* t0 = p.tiles + id / nb * 5;
-  const int in = id - t0[3] * nb, tile = t0[3] + in % t0[4], bn = in / t0[4];
+  int first = t0[3], of = t0[4], large = 0;  // (requested with the count's loads; right where there are none)
+  for (int i = 0; i < nt; i += 64) {
+    const int t = i + (threadIdx.x & 63);
+    const int* tl = p.tiles + min(t, nt - 1) * 5;
+    large += __popcll(__ballot(t < nt && !(tl[4] == 1 && 2 * tl[2] <= p.mt)));
+  }
+  large = __builtin_amdgcn_readfirstlane(large);
+  if (large > 0 && large < nt) {
+    const int l = large * nb;
+    id = (int)blockIdx.x < l ? xcd_remap(blockIdx.x, l) : l + xcd_remap(blockIdx.x - l, nt * nb - l);
+    t0 = p.tiles + id / nb * 5;
+    first = t0[3], of = t0[4];
+  }
+  const int in = id - first * nb, tile = first + in % of, bn = in / of;
   const int* tl = p.tiles + tile * 5;
   const int nr = tl[2], n0 = bn * NB;
   if constexpr (FAR) {
@@ -1032,7 +1063,7 @@ KCA_API int kca_moe_group(const void* ids, int n, int E, int mt, void* perm, voi
                           void* ntiles, hipStream_t s) {
   const GroupArgs g{(const int*)ids, n, E, mt, (int*)perm, (int*)inv, (int*)tiles, (int*)ntiles};
   if (!group_ok(g, max_tiles)) return 1;
-  hipLaunchKernelGGL(group_kernel, dim3(1), dim3(1024), (3 * E + 2) * 4, s, g);
+  hipLaunchKernelGGL(group_kernel, dim3(1), dim3(1024), (4 * E + 3) * 4, s, g);
   return hipGetLastError() == hipSuccess ? 0 : 4;
 }
 
@@ -1061,7 +1092,7 @@ KCA_API int kca_moe_expert(int dtype, const void* x, const void* w, void* y, con
                            hipStream_t s) {
   if (max_tiles < 1 || max_tiles > 32767 || N < 1 || K < 1 || top < 1 || !x || !w || !y || !perm || !wts || !tiles || !ntiles) return 1;
   if (ws && (!xs || !ys || tokens < 1 || tokens > 32767 || Ns < 1 || Ks < 1 || mt > 8)) return 1;
-  const ExpertArgs a{x, w, y, (const int*)perm, (const float*)wts, (const int*)tiles, (const int*)ntiles, top, N, K, up, scale,
+  const ExpertArgs a{x, w, y, (const int*)perm, (const float*)wts, (const int*)tiles, (const int*)ntiles, mt, top, N, K, up, scale,
                      xs, ws, ys, tokens, Ns, Ks};
   const bool far = (up ? 4ll : 2ll) * N * K >= 1ll << 32 || 2ll * (up ? x_rows : mt) * K >= 1ll << 31;  // (32-bit byte offsets)
   if (mt == GM || mt == 128 || mt == 192) {

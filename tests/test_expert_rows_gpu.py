@@ -41,6 +41,25 @@ def test_products(mt, scale_in, counts, top, d, F):
     assert (y.float() - want).norm() <= TOL * want.norm()
 
 
+@pytest.mark.parametrize("counts,mt", [([64, 65, 1, 0, 128, 320, 321], 128), ([257, 288, 289, 40, 513, 256, 130], 256), ([5, 70] * 40, 128), ([3] * 70, 192)])
+def test_short_tiles_run_last(counts, mt):
+    """Tiles that are alone and at most half full stand behind the rest; every row has one tile, and the products are right."""
+    h, ids, wts, gu, dn = _case(counts, 1, 64, 64)
+    g = moe.group(ids, len(counts), mt)
+    tiles = g.tiles[:int(g.ntiles)].tolist()
+    late = [t[4] == 1 and 2 * t[2] <= mt for t in tiles]
+    assert late == sorted(late)
+    for i, (e, at, rows, first, n) in enumerate(tiles):
+        assert 0 < rows <= mt and first <= i < first + n and all(t[0] == e and t[3:] == [first, n] for t in tiles[first:first + n])
+    rows = sorted((t[0], t[1] + j) for t in tiles for j in range(t[2]))
+    assert rows == [(e, sum(counts[:e]) + j) for e, c in enumerate(counts) for j in range(c)]
+    y = moe.experts(h, ids, wts, gu, dn, g, False)[g.inv.view(-1).long()]
+    u = torch.bmm(gu.float()[ids.view(-1).long()], h.float()[:, :, None])[..., 0]
+    a = (torch.nn.functional.silu(u[:, :64]) * u[:, 64:]).bfloat16().float()
+    want = torch.bmm(dn.float()[ids.view(-1).long()], a[..., None])[..., 0] * wts
+    assert (y.float() - want).norm() <= TOL * want.norm()
+
+
 def _far(T, d, F, E):
     """Sizes past the 32-bit offsets, and some tokens' outputs in fp32."""
     g = torch.Generator(device="cuda").manual_seed(1)
