@@ -29,6 +29,7 @@
 
 int attn_fwd_split(const FastFwdParams& p, int d, hipStream_t stream);  // attention_split.hip
 int attn_bwd_split(const FastBwdParams& p, int d, hipStream_t stream);
+int attn_bwd_pair(const FastBwdParams& p, int d, bool causal, hipStream_t stream);
 
 namespace {
 
@@ -1614,9 +1615,9 @@ KCA_API int kca_attn_bwd_tiled(const void* q, const void* k, const void* v, cons
   const bool aligned = rows16(q, q_sb, q_st, q_sh) && rows16(k, k_sb, k_st, k_sh) && rows16(v, v_sb, v_st, v_sh) &&
                        rows16(o, o_sb, o_st, o_sh) && rows16(dout, do_sb, do_st, do_sh) && rows16(dq, dq_sb, dq_st, dq_sh) &&
                        rows16(dk, dk_sb, dk_st, dk_sh) && rows16(dv, dv_sb, dv_st, dv_sh);
-  if (causal && aligned) {
+  if (aligned) {
     (void)hipGetLastError();
-    const int rc = attn_bwd_split(p, d, stream);
+    const int rc = d == 256 ? attn_bwd_pair(p, d, causal, stream) : causal ? attn_bwd_split(p, d, stream) : 1;
     if (rc != 1) return rc;
   }
   if (alibi || kv_len || window || Sq % 128 || Sk % 128) {
@@ -1624,7 +1625,7 @@ KCA_API int kca_attn_bwd_tiled(const void* q, const void* k, const void* v, cons
     const bool done = general_form(d, causal, alibi, [&](auto D_, auto C_, auto G_) {
       constexpr int D = decltype(D_)::value, G = decltype(G_)::value;
       constexpr bool C = decltype(C_)::value;
-      if constexpr (!C || D >= 160) {  // (the other causal ones: attention_split.hip)
+      if constexpr (D == 160 || (!C && D != 256)) {  // (the others: attention_split.hip, attention_pair.hip)
         hipLaunchKernelGGL((attn_bwd_dq_tiled_kernel<D, C, D, G>), g2, dim3(256), 0, stream, p);
         hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<D, C, D, G>), g1, dim3(256), 0, stream, p);
       }

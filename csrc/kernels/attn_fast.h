@@ -169,3 +169,45 @@ __device__ __forceinline__ void add_partial(const char* at, f32x16 (&acc)[D / 32
       for (int j = 0; j < 4; ++j) acc[db][4 * g + j] = fmaf(x[j], w, acc[db][4 * g + j]);
     }
 }
+
+// A 32-row x D tile staged by the NT threads of a group: chunk idx = thread + NT * j is (row idx / NCH, 16-byte chunk idx % NCH);
+// the last round may be the first waves' alone.
+template <int D, int NT>
+struct GroupStager {
+  static constexpr int NCH = D / 8, TOT = 32 * NCH, CPT = (TOT + NT - 1) / NT;
+  static constexpr bool EVEN = NT % NCH == 0 && TOT % NT == 0;  // chunk column the same for all j: rows a scalar offset apart
+  static_assert(TOT % 64 == 0, "whole waves");
+  int vo_[EVEN ? 1 : CPT], lds_[CPT];
+  int step_;
+  bool tail_;  // this thread owns a chunk in the last round
+  __device__ __forceinline__ GroupStager(int t, long long st) {
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) {
+      const int idx = min(t + NT * j, TOT - 1), row = idx / NCH, ch = idx % NCH;
+      if (j == 0 || !EVEN) vo_[EVEN ? 0 : j] = (int)(((long long)row * st + ch * 8) * 2);
+      lds_[j] = img_off<D>(row, ch);
+    }
+    step_ = __builtin_amdgcn_readfirstlane((int)(NT / NCH * st * 2));
+    tail_ = t + NT * (CPT - 1) < TOT;
+  }
+  __device__ __forceinline__ void load(u32x4 (&x)[CPT], __amdgpu_buffer_rsrc_t r, int so) const {
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) {  // (a chunk past the last one is a valid one, never stored)
+      const auto a = __builtin_amdgcn_raw_buffer_load_b128(r, vo_[EVEN ? 0 : j], EVEN ? so + j * step_ : so, 0);
+      x[j] = *reinterpret_cast<const u32x4*>(&a);
+    }
+  }
+  __device__ __forceinline__ void store(const u32x4 (&x)[CPT], char* img) const {
+#pragma unroll
+    for (int j = 0; j < CPT; ++j)
+      if (TOT % NT == 0 || j < CPT - 1 || tail_) *reinterpret_cast<u32x4*>(img + lds_[j]) = x[j];
+  }
+};
+
+template <int D>
+__device__ __forceinline__ void clear(f32x16 (&acc)[D / 32]) {
+#pragma unroll
+  for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
+}
