@@ -1519,10 +1519,14 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
   // Full tiles without another mask keep the plain form, whose loops have no edge to test: 4 x 2048 of 256 179 us
   // against 203 forward and 760 against 815 backward, 8 x 1024 of 64 36 and 137 against 36 and 146.
   bool whole = false;  // the kernel leaves no row to the fixup launch
-  // D = 256 under a causal mask: blocks of 128 rows, their keys in two groups, where blocks of 256 leave CUs idle (us, 256 rows and
-  // one group against it; blocks of 256 rows: 1 x 1024 x 16 heads (64) 47, 40; 1 x 2048 (128) 89, 73; 1 x 3000 with ALiBi (192) 143,
-  // 107; 2 x 2048 (256) 103, 106; 1 x 4096 (256) 179, 168; 4 x 1100 (320) 65, 80; 1 x 61 9.2, 11.6)
-  const bool two = d == 256 && causal && aligned && Sq > 256 && (long long)((Sq + 255) / 256) * B * H <= 192;
+  // D = 256 under a causal mask: blocks of 128 rows, their keys in two groups, where blocks of 256 leave half of the CUs idle, and up to
+  // one a CU where the longest walk, which the call waits for, is long (us, 256 rows and one group against it; blocks of 256 rows:
+  // 1 x 1024 x 16 heads (64) 47, 40; 4 x 400 (128) 27.7, 25.3; 1 x 2000 with a window of 256 (128) 35.6, 28.4; 2 x 1500 (192) 75, 62;
+  // 1 x 3300 (208) 147, 116; 3 x 1200 with lengths (240) 63.4, 61.2; 1 x 4096 (256) 181, 166; but 2 x 2048 (256) 101, 104; 6 x 400 (192) 29.7, 38.9; 1 x 3000 with
+  // a window (192) 38.3, 49.0; 3 x 900 (192) 51.1, 52.0; 4 x 1000 (256) 59, 65; 4 x 1100 (320) 65, 80; 1 x 61 9.2, 11.6)
+  const long long blocks256 = (long long)((Sq + 255) / 256) * B * H;
+  const int walk = window > 0 ? min(Sq, window) : Sq;
+  const bool two = d == 256 && causal && aligned && Sq > 256 && blocks256 <= (walk >= 3000 ? 256 : walk >= 1200 ? 240 : 128);
   if (alibi || kv_len || window || cu || Sq % 128 || Sk % 32 || two) {
     if (!aligned) return 1;
     const bool done = general_form(d, causal, alibi, [&](auto D_, auto C_, auto G_) {
