@@ -668,14 +668,49 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
 }  // namespace
 
 // Which calls are split in two groups (two waves of 32 rows each, 4 waves a workgroup), the others in blocks of 128 rows and
-// one group. One MI355X, us, one group against two; blocks: 128-row blocks of all heads.
-//   forward, 64 wide:   2 x 889 x 16 heads (224 blocks) 19.4, 14.8; 1 x 4000 x 12 (384) 61.6, 45.8; 15 x 256 x 16 (480) 11.9, 15.3;
-//                       2 x 2688 x 12 (504) 45.3, 41.8; 3 x 2048 x 12 (576) 39.2, 35.2; 10 x 577 x 12 (600) 18.3, 21.9
-//   96 wide:            1 x 700 x 32 (192) 19.4, 16.0; 5 x 256 x 32 (320) 14.3, 18.4; 1 x 1403 x 32 (352) 33.8, 31.2; 768: 51, 61
-//   128 wide:           1 x 2048 x 14 with ALiBi (224) 48.7, 41.2; 2 x 896 x 20 (280) 27.9, 24.6; 2 x 1346 x 20 (440) 37.1, 43.0
-//   dQ follows the same line (gains of 1 to 17 us below it, losses of 1 to 23 above).
-static bool split_rows(long long blocks, int d, int rows) {
-  return blocks <= (d == 64 ? (rows >= 1536 ? 640 : 448) : d == 96 ? (rows >= 1024 ? 400 : 256) : 320);
+// one group: up to so many 128-row blocks of all heads, the more the longer the longest walk is (keys that a row sees; dK/dV: queries),
+// for a split costs each of its blocks the meeting of the sums. One MI355X, us, one group against two:
+//   forward, 64 wide:   128 rows, 340 blocks 10.5, 10.5, 400 10.6, 13.2; 512 rows, 400 15.3, 15.3, 480 15.2, 18.1; 1024 rows, 400 22.5,
+//                       18.7, 480 22.5, 23.2; 3 x 2048 x 12 (576) 39.2, 35.2; 3000 rows with a window of 256, 336 18.7, 15.0, 408 19.3, 19.7
+//   96 wide:            128 rows, 100 9.5, 8.7, 140 10.0, 10.6; 256 rows, 140 12.6, 11.5, 180 13.0, 13.4; 512 rows, 220 18.3, 16.9, 260
+//                       19.1, 19.3; 1024 rows, 336 28.4, 26.7, 400 28.9, 30.0; 1 x 1403 x 32 (352) 33.8, 31.2
+//   128 wide:           128 rows, 100 10.3, 9.5, 140 10.8, 11.6, 260 14.0, 18.6; 256 rows, 140 13.8, 13.2, 180 14.1, 14.7; 512 rows, 220
+//                       19.7, 19.4, 260 20.4, 21.5; 1024 rows, 304 29.8, 27.9, 336 30.1, 30.6
+//   dQ follows the same lines.
+struct Upto { int walk, blocks; };
+template <int N>
+static int blocks_upto(const Upto (&t)[N], int walk) {
+  int b = 0;
+  for (const Upto& u : t)
+    if (walk >= u.walk) b = u.blocks;
+  return b;
+}
+static bool split_rows(long long blocks, int d, int keys, int window) {
+  static const Upto t64[] = {{0, 340}, {512, 400}, {1536, 640}};
+  static const Upto t96[] = {{65, 100}, {129, 140}, {384, 220}, {768, 300}, {1024, 336}, {1400, 400}};
+  static const Upto t128[] = {{65, 100}, {129, 140}, {384, 180}, {512, 220}, {768, 260}, {1024, 320}};
+  const int walk = window > 0 ? min(keys, window) : keys;
+  return blocks <= (d == 64 ? blocks_upto(t64, walk) : d == 96 ? blocks_upto(t96, walk) : blocks_upto(t128, walk));
+}
+// dK/dV with one group or two, or, 128 wide, 0, 1 or in two groups of four waves (2): there two groups of two take 81 KB of LDS, one
+// workgroup a CU. us, backward with one group, and what two groups (of four waves) take or save:
+//   64 wide:   128 rows, 260 blocks 22.0, +0.2; 256 rows, 340 27.6, -0.8, 400 28.2, +0.9; 512 rows, 480 40.4, -0.8, 560 44.5, +1.9; 1024
+//              rows, 560 68.4, -2.5; 3 x 2048 x 16 (768) 148, -8; a window of 256, 336 41.6, -2.6, 480 43.8, +5.8
+//   96 wide:   128 rows, 220 23.8, -0.4, 260 30.2, +2.5; 512 rows, 300 47.4, -1.7, 340 48.5, +0.3; 1024 rows, 480 80.5, -0.8
+//   128 wide:  128 rows, 100 23.0, -1.0 (+0.6), 140 25.0, +3.6 (+0.7); 256 rows, 140 33.7, -1.3 (-0.4), 180 34.3, +1.2 (0); 512 rows, 180
+//              48.9, -2.8 (-2.0), 260 54.6, +4.5 (-3.8), 340 57.1, +8.0 (+2.3); 1024 rows, 256 80.0, -7.4 (-7.1), 304 87.4, +2.4 (-9.3), 480
+//              99.2, +17 (-3.9), 560 108, +28 (+6.7); 1 x 2944 x 20 (460) 246, +29 (-37); a window of 256, 96 40.2, -7.1 (-2.2), 144 43.1,
+//              +2.5 (-2.3), 264 48.3, +7.8 (+3.0)
+static int split_keys(long long blocks, int d, int rows, int window) {
+  static const Upto t64[] = {{0, 340}, {512, 480}, {768, 560}, {1536, 768}};
+  static const Upto t96[] = {{0, 760}, {65, 220}, {384, 280}, {768, 380}, {1024, 480}};
+  static const Upto t128[] = {{0, 220}, {65, 100}, {129, 140}, {384, 180}, {768, 220}};
+  static const Upto w128[] = {{384, 260}, {512, 300}, {768, 400}, {1024, 512}};
+  const bool win = window > 0 && window < rows;
+  const int walk = win ? window : rows;
+  if (d == 128 && win) return blocks <= 120 ? 1 : blocks <= 220 ? 2 : 0;
+  if (blocks <= (d == 64 ? blocks_upto(t64, walk) : d == 96 ? blocks_upto(t96, walk) : blocks_upto(t128, walk))) return 1;
+  return d == 128 && blocks <= blocks_upto(w128, walk) ? 2 : 0;
 }
 
 template <class F>
@@ -696,7 +731,7 @@ static int with_form(int d, bool alibi, F&& f) {
 // Causal calls of 64, 96 and 128 wide heads with 16-byte rows; 1: another head size.
 int attn_fwd_split(const FastFwdParams& p, int d, hipStream_t stream) {
   const long long blocks = (long long)((p.Sq + 127) / 128) * p.B * p.H;
-  const bool two = split_rows(blocks, d, p.Sq);
+  const bool two = split_rows(blocks, d, p.Sk, p.window);
   return with_form(d, p.alibi, [&](auto D_, auto G_) {
     constexpr int D = decltype(D_)::value, G = decltype(G_)::value, W = D == 64 ? 3 : 2;
     if (two)
@@ -706,15 +741,10 @@ int attn_fwd_split(const FastFwdParams& p, int d, hipStream_t stream) {
   });
 }
 
-// dK/dV, one group against two, us with dQ: 64 wide, 4 x 948 x 16 heads (512 blocks) 60.6, 55.3; 9 x 409 x 16 (576) 38.8, 41.8; 3 x
-// 2048 x 16 (768) 148, 140; 96 wide, 1 x 1403 x 32 (352) 101, 80; 11 x 146 x 32 (704) 45, 48. At 128 wide two groups of two waves
-// take 81 KB of LDS, one workgroup a CU; two of four (8 waves, 128 keys) are the better ones from 200 blocks on: 1 x 651 x 20 (120
-// blocks) 56.9, 51.1, 53.3; 2 x 896 x 20 (280) 84.7, 84.1, 72.8; 1 x 2944 x 20 (460) 246, 275, 209; 4 x 1408 x 14 (616) 137, 185, 145.
 int attn_bwd_split(const FastBwdParams& p, int d, hipStream_t stream) {
   const long long qblocks = (long long)((p.Sq + 127) / 128) * p.B * p.H, kblocks = (long long)((p.Sk + 127) / 128) * p.B * p.Hkv;
-  const bool two = split_rows(qblocks, d, p.Sq);
-  const bool two_kv = kblocks <= (d == 64 ? (p.Sk >= 1536 ? 768 : 512) : d == 96 ? 400 : 200);
-  const bool wide_kv = !two_kv && d == 128 && kblocks <= 512;
+  const bool two = split_rows(qblocks, d, p.Sk, p.window);
+  const int kv = split_keys(kblocks, d, p.Sq, p.window);
   return with_form(d, p.alibi, [&](auto D_, auto G_) {
     constexpr int D = decltype(D_)::value, G = decltype(G_)::value, W = D == 64 ? 3 : 2;
     if (two)
@@ -723,13 +753,13 @@ int attn_bwd_split(const FastBwdParams& p, int d, hipStream_t stream) {
       hipLaunchKernelGGL((attn_bwd_dq_split_kernel<D, G, 4, 1, W>), dim3((unsigned)qblocks), dim3(256), 0, stream, p);
     auto dkdv = [&](auto WIN_) {
       constexpr bool WIN = decltype(WIN_)::value;
-      if (two_kv)
+      if (kv == 1)
         hipLaunchKernelGGL((attn_bwd_dkdv_split_kernel<D, G, WIN, 2, 2, W>), dim3((p.Sk + 63) / 64 * p.B * p.Hkv), dim3(256), 0,
                            stream, p);
-      else if (!wide_kv)
+      else if (kv == 0)
         hipLaunchKernelGGL((attn_bwd_dkdv_split_kernel<D, G, WIN, 4, 1, W>), dim3((unsigned)kblocks), dim3(256), 0, stream, p);
       if constexpr (D == 128)
-        if (wide_kv)
+        if (kv == 2)
           hipLaunchKernelGGL((attn_bwd_dkdv_split_kernel<D, G, WIN, 4, 2, 2>), dim3((unsigned)kblocks), dim3(512), 0, stream, p);
     };
     if (p.window > 0) dkdv(std::true_type{});

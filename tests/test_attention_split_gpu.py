@@ -40,9 +40,9 @@ def test_two_groups(D, S):
 
 def test_eight_waves_dkdv():
     """128-wide heads between the two: dK/dV of 128 keys in two groups of four waves."""
-    _check(9, 300, 300, 10, 10, 128, True)
-    _check(9, 300, 300, 10, 10, 128, True, alibi=True, window=150)
-    _check(9, 200, 330, 20, 10, 128, True, lens=[330, 0, 1, 329, 128, 127, 129, 31, 300])
+    _check(5, 400, 400, 10, 10, 128, True)
+    _check(5, 400, 400, 10, 10, 128, True, alibi=True, window=150)
+    _check(5, 390, 520, 20, 10, 128, True, lens=[520, 0, 1, 129, 511])
 
 
 @pytest.mark.parametrize("D", [64, 96, 128, 256])
