@@ -650,8 +650,9 @@ __device__ __forceinline__ bf16x8 as_bf8(u32x2 lo, u32x2 hi) {
 // SIMD, O^T = 256 registers, Q^T fragments 128; two 64-KiB stages, the next tile's DMA in flight
 // under the current tile). Inference only: the overflow flags go back to the caller, which has no
 // generic D = 512 kernel to fix rows up with and reruns flagged calls on the GEMM path.
+// NW = 4, NBUF = 2, D = 256: blocks of 128 rows, two workgroups a CU, a tile ahead (their rule: kca_attn_fwd_tiled).
 template <int D, bool CAUSAL, int NW = 8, int NBUF = 4, int G = 0, int KG = 1>
-__global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p) {
+__global__ void __launch_bounds__(NW * 64, NW == 4 && D == 256 ? 2 : 1) attn_fwd_w8_kernel(FastFwdParams p) {
   constexpr int RW = NW / KG;                 // waves a group: its 32-row slices
   constexpr int BM = RW * 32, BN = 32;
   constexpr int TILE = BN * D * 2;            // one K or V image
@@ -662,7 +663,7 @@ __global__ void __launch_bounds__(NW * 64, 1) attn_fwd_w8_kernel(FastFwdParams p
   constexpr int LEAD = NBUF / KG - 1;                  // steps (of KG tiles) issued ahead of the one computed
   constexpr int INFLIGHT = (LEAD - 1) * KG * 2 * PPW;  // DMA instructions issued after a step's when it is waited for
   constexpr bool AGAIN = D != 512;                     // overflowed rows are computed again here
-  static_assert(((D == 256 || D == 128) && NW == 8) || (D == 512 && NW == 4 && NBUF == 2 && !CAUSAL),
+  static_assert(((D == 256 || D == 128) && NW == 8) || (D == 256 && NW == 4 && NBUF == 2) || (D == 512 && NW == 4 && NBUF == 2 && !CAUSAL),
                 "multi-wave LDS-DMA forward: 8 waves at D = 128 / 256, 4 waves at D = 512");
   static_assert(PPW >= 1 && PIECES % NW == 0, "whole pieces per wave");
   static_assert(NBUF % KG == 0 && LEAD >= 1 && (KG == 1 || G > 0), "groups: general forms, two steps of buffers");
@@ -1519,14 +1520,28 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
   // Full tiles without another mask keep the plain form, whose loops have no edge to test: 4 x 2048 of 256 179 us
   // against 203 forward and 760 against 815 backward, 8 x 1024 of 64 36 and 137 against 36 and 146.
   bool whole = false;  // the kernel leaves no row to the fixup launch
-  // D = 256 under a causal mask: blocks of 128 rows, their keys in two groups, where blocks of 256 leave half of the CUs idle, and up to
-  // one a CU where the longest walk, which the call waits for, is long (us, 256 rows and one group against it; blocks of 256 rows:
-  // 1 x 1024 x 16 heads (64) 47, 40; 4 x 400 (128) 27.7, 25.3; 1 x 2000 with a window of 256 (128) 35.6, 28.4; 2 x 1500 (192) 75, 62;
-  // 1 x 3300 (208) 147, 116; 3 x 1200 with lengths (240) 63.4, 61.2; 1 x 4096 (256) 181, 166; but 2 x 2048 (256) 101, 104; 6 x 400 (192) 29.7, 38.9; 1 x 3000 with
-  // a window (192) 38.3, 49.0; 3 x 900 (192) 51.1, 52.0; 4 x 1000 (256) 59, 65; 4 x 1100 (320) 65, 80; 1 x 61 9.2, 11.6)
-  const long long blocks256 = (long long)((Sq + 255) / 256) * B * H;
-  const int walk = window > 0 ? min(Sq, window) : Sq;
-  const bool two = d == 256 && causal && aligned && Sq > 256 && blocks256 <= (walk >= 3000 ? 256 : walk >= 1200 ? 240 : 128);
+  // D = 256 under a causal mask, by the blocks of 256 rows of all heads, those of 128 and the longest walk (keys a row sees). us:
+  //   two:  128 rows, 8 waves, their keys in two groups, where a CU has one long walk at most, against 256 rows and one group: 1 x 1024 x
+  //         16 heads (64 blocks of 256) 47, 40; 2 x 1500 (192) 75, 62; 1 x 3300 (208) 147, 116; 1 x 4096 (256) 181, 166; 2 x 2048 (256) 101, 104
+  //   four: 128 rows, 4 waves, two workgroups a CU, one of which computes while the other waits and long blocks run beside short ones:
+  //         48 blocks of 128 rows 14.7, 11.5; 300 31.5, 20.0; 256 rows, 520 blocks 43, 34; 2 x 2048 (512) 102, 98; 9 x 640 (720) 74, 52; 2 x
+  //         2900 with a window of 256 73, 62; against two groups 640 rows, 160 blocks 31.4, 29.2, 1000 rows 42.3, 44.4, 1400 rows 52.7, 57.7.
+  //         Blocks of 256 rows stream half as many tiles: 1000 rows, 600 blocks of 128 66, 69; 2048 rows, 896 134, 136, 1040 162, 187, 2 x 2185 with
+  //         ALiBi (576) 109, 115; 256 rows, 2000 125, 124; whole blocks of 256 that an odd count leaves half empty lose at any count: 640 rows, 2165 236, 188
+  const int n128 = (Sq + 127) / 128;
+  const long long heads = (long long)B * H, blocks256 = (Sq + 255) / 256 * heads, blocks128 = n128 * heads;
+  const int walk = window > 0 ? min(Sk, window) : Sk;
+  const bool c256 = d == 256 && causal && aligned;
+  const bool two = c256 && Sq > 256 && blocks256 <= (walk >= 3000 ? 256 : walk >= 1400 ? 240 : walk >= 900 ? 128 : 0);
+  const bool four = c256 && !two && (walk < Sk || (n128 % 2 && n128 <= 5) || (Sq % 128 == 0 && Sq % 256) ||
+                                     blocks128 <= (walk <= 256 ? 2000 : walk >= 2000 && !alibi ? 768 : 512));
+  if (four) {
+    if (alibi) hipLaunchKernelGGL((attn_fwd_w8_kernel<256, true, 4, 2, 2>), grid, dim3(256), 0, stream, p);
+    else if (kv_len || window || cu || Sq % 128 || Sk % 32)
+      hipLaunchKernelGGL((attn_fwd_w8_kernel<256, true, 4, 2, 1>), grid, dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((attn_fwd_w8_kernel<256, true, 4, 2>), grid, dim3(256), 0, stream, p);
+    return hipGetLastError() != hipSuccess ? 3 : -1;
+  }
   if (alibi || kv_len || window || cu || Sq % 128 || Sk % 32 || two) {
     if (!aligned) return 1;
     const bool done = general_form(d, causal, alibi, [&](auto D_, auto C_, auto G_) {

@@ -1,12 +1,12 @@
-"""Backward of 256-wide heads, whose waves work in pairs: one, two and three tiles a walk, blocks that nobody sees, walks over
-several query heads, against the fp32 reference (bounds as in test_attention_edges_gpu.py)."""
+"""256-wide heads: the backward, whose waves work in pairs -- one, two and three tiles a walk, blocks that nobody sees, walks over
+several query heads -- and the forward with four waves a block, against the fp32 reference (bounds as in
+test_attention_edges_gpu.py)."""
 import pytest
-
 import torch
 
 from kubernetes_cloud_amd.ops import attention as A
 
-from .test_attention_edges_gpu import _check
+from .test_attention_edges_gpu import _check, _close
 
 pytestmark = pytest.mark.gpu
 
@@ -39,3 +39,27 @@ def test_rows_off_16_bytes():
         grads.append((q.grad, k.grad, v.grad))
     for a, b in zip(*grads):
         assert (a.float() - b.float()).norm() <= 3 * 2.0 ** -9 * b.float().norm()
+
+
+@pytest.mark.parametrize("H", [3, 40])
+@pytest.mark.parametrize("S", [128, 129, 256, 330, 384, 600, 640])
+def test_four_waves(S, H):
+    """Forward in blocks of 128 rows, two workgroups a CU: odd and even counts of blocks, edges, masks; and whole blocks of 256."""
+    _check(2, S, S, H, H, 256, True)
+    _check(2, S, S + 31, H, 1, 256, True, window=100)
+    _check(2, S, S, H, H, 256, True, alibi=True, lens=[S, S - 77])
+
+
+@pytest.mark.parametrize("alibi", [False, True])
+def test_four_waves_far_above_their_first_tile(alibi):
+    """A late key far above a row's first tile: the rows are computed again in the same launch."""
+    S, H, D = 640, 8, 256
+    g = torch.Generator(device="cuda").manual_seed(D)
+    q, k, v = (torch.randn(3, S, H, D, device="cuda", generator=g) * 0.3 for _ in range(3))
+    k[0, 200, 1] = q[0, 600, 1] * 40.0
+    q, k, v = (x.bfloat16() for x in (q, k, v))
+    sl = torch.full((H,), 0.25, device="cuda") if alibi else None
+    o, lse = A._fwd(q, k, v, True, D ** -0.5, None, sl)
+    r, want = A.attention_reference(*(t[:1, :, :2].float() for t in (q, k, v)), True, None, None, None if sl is None else sl[:2])
+    _close(o[:1, :, :2], r)
+    torch.testing.assert_close(lse[:1, :2], want, rtol=2.0 ** -18, atol=2.0 ** -16)  # (as in test_attention_split_gpu.py)
