@@ -9,7 +9,7 @@
 // are half as tall, so there are twice as many, each 1 / KG as long, and a SIMD has two waves to run.
 //
 // The forms of a mask are attention_tiled.hip's general ones (1: lengths, windows, any sizes; 2: ALiBi) and every call takes
-// one of them. Blocks are taken longest first over all heads (block number = row block * heads + head).
+// one of them. Blocks are taken longest first over all heads (block_of).
 //
 // Tiles in LDS: two buffers of K and V a group. A step computes S of the group's next tile while it takes the softmax of this
 // one, so K runs a tile ahead of V: K(i + 2) goes where K(i) was and V(i + 1) where V(i - 1) was, which all waves have read
@@ -42,7 +42,7 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_fwd_split_kernel(FastF
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = wave / RW, rw = wave % RW;
   const int l32 = lane & 31, hh = lane >> 5, gi = lane & 15;
   const int nqb = (p.Sq + BM - 1) / BM, heads = p.B * p.H;
-  const auto [qi, bh] = block_of<true>(nqb, heads);
+  const auto [qi, bh] = block_of<true, D == 64 ? 3 : 1>(nqb, heads);
   const int qb = nqb - 1 - qi;
   const int b = bh / p.H, h = bh % p.H;
   const int hk = h / (p.H / p.Hkv);
@@ -300,7 +300,7 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dq_split_kernel(Fa
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = wave / RW, rw = wave % RW;
   const int l32 = lane & 31, hh = lane >> 5;
   const int nqb = (p.Sq + BM - 1) / BM, heads = p.B * p.H;
-  const auto [qi, bh] = block_of<true>(nqb, heads);
+  const auto [qi, bh] = block_of<true, D == 64 ? 3 : 1>(nqb, heads);
   const int qb = nqb - 1 - qi;
   const int b = bh / p.H, h = bh % p.H;
   const int hk = h / (p.H / p.Hkv);
@@ -463,7 +463,7 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = wave / RW, rw = wave % RW;
   const int l32 = lane & 31, hh = lane >> 5;
   const int heads = p.B * p.Hkv;
-  const auto [kb, bh] = block_of<true>((p.Sk + BK - 1) / BK, heads);
+  const auto [kb, bh] = block_of<true, D == 64 ? 3 : 1>((p.Sk + BK - 1) / BK, heads);
   const int b = bh / p.Hkv, hk = bh % p.Hkv;
   const int grp = p.H / p.Hkv;
   const int off = p.Sk - p.Sq;

@@ -31,10 +31,25 @@ __device__ __forceinline__ void own_sequence(FastFwdParams& p, int b) {
 // heads first, so that no long one starts when the others are done (heads a multiple of 8 also stay on their XCD): 2 x 2048 x 16
 // heads of 256, whose 512 backward workgroups are two a CU, one after the other, 398 -> 298 us against head after head, 8 x 512
 // of them with lengths 168 -> 129. Without a mask all are alike, and a head's blocks lie on one XCD, beside its keys and values.
+// PER_CU: workgroups that run on a CU at one time. They start together, a round of 256 after the other, so that the CU with the longest
+// block of the first round had the longest of the next as well: the later rounds are turned so that a CU's blocks add up to about the
+// same (two: the second backwards; three: the second from its middle on, the third in twos backwards). 64-wide heads, 3 a CU, us,
+// forward, dQ, dK/dV: 8 x 1000 x 12 heads 29.0, 36.0, 49.5 -> 26.7, 33.8, 46.4; 3 x 2048 x 16 46.7, 60.6, 91.3 -> 43.2, 56.9, 86.7. Two a
+// CU (96 and 128 wide) gain or lose 3 %: not there.
 struct BlockOf { int block, head; };
-template <bool CAUSAL>
+template <bool CAUSAL, int PER_CU = 1>
 __device__ __forceinline__ BlockOf block_of(int blocks, int heads) {
-  if (CAUSAL) return {(int)blockIdx.x / heads, (int)blockIdx.x % heads};
+  if (CAUSAL) {
+    int n = (int)blockIdx.x;
+    if constexpr (PER_CU == 3) {
+      const int full = min(PER_CU, (int)gridDim.x / 256), round = n / 256, c = n / 8 % 32;  // (c: the CU of its XCD n % 8)
+      if (round > 0 && round < full) {
+        const int d = full == 2 ? 31 - c : round == 1 ? (c + 16) % 32 : c < 16 ? 31 - 2 * c : 62 - 2 * c;
+        n = round * 256 + d * 8 + n % 8;
+      }
+    }
+    return {n / heads, n % heads};
+  }
   const int id = xcd_remap(blockIdx.x, gridDim.x);
   return {id % blocks, id / blocks};
 }
