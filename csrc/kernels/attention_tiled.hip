@@ -1499,6 +1499,7 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
                                float scale, const float* alibi, const int* kv_len, int window, const int* cu,
                                int rowsum_col, int max_col, int* flags, hipStream_t stream) {
   if (Sq <= 0 || Sk <= 0 || H % Hkv || !flags) return 1;
+  if (!(scale > 0.f)) return 1;  // a masked score of -inf times it would not be masked
   if (causal && Sk < Sq) return 1;
   if (!offsets_fit(Sk, k_st) || !offsets_fit(Sk, v_st)) return 1;  // buffer-load byte offsets are 32-bit
   FastFwdParams p{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (bf16_t*)o, lse, flags,
@@ -1641,15 +1642,17 @@ KCA_API int kca_attn_bwd_tiled(const void* q, const void* k, const void* v, cons
   }
   if (alibi || kv_len || window || Sq % 128 || Sk % 128) {
     if (!aligned) return 1;
-    const bool done = general_form(d, causal, alibi, [&](auto D_, auto C_, auto G_) {
+    bool here = false;
+    general_form(d, causal, alibi, [&](auto D_, auto C_, auto G_) {
       constexpr int D = decltype(D_)::value, G = decltype(G_)::value;
       constexpr bool C = decltype(C_)::value;
       if constexpr (D == 160 || (!C && D != 256)) {  // (the others: attention_split.hip, attention_pair.hip)
         hipLaunchKernelGGL((attn_bwd_dq_tiled_kernel<D, C, D, G>), g2, dim3(256), 0, stream, p);
         hipLaunchKernelGGL((attn_bwd_dkdv_tiled_kernel<D, C, D, G>), g1, dim3(256), 0, stream, p);
+        here = true;
       }
     });
-    return done ? 0 : 1;
+    return here ? 0 : 1;
   }
   if (d != 48 && d != 64 && d != 96 && d != 128 && d != 160 && d != 256) return 1;
   if (d == 48 && causal) return 1;  // narrow storage: SD-1.5's (non-causal) 40-wide heads

@@ -76,3 +76,20 @@ def test_not_a_number_stays_in_its_rows(D):
     o[0, 70, 1] = want[0, 70, 1]
     # (the row's block takes its true maxima: other rows of it are rounded relative to another weight)
     _close(o, want)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("scale", [0.0, -0.07, 1e-25, 0.2])
+def test_scales(D, scale):
+    """No scale, a negative one, hardly any (dK's sums start with lse over it) and a large one."""
+    g = torch.Generator(device="cuda").manual_seed(D)
+    q, k, v, do = (torch.randn(13, 130, 48, D, device="cuda", generator=g).bfloat16() for _ in range(4))
+    x = [t[:, :, :6].contiguous().requires_grad_() if D == 128 else t.requires_grad_() for t in (q, k, v)]
+    do = do[:, :, :x[0].shape[2]].contiguous()
+    o = flash_attention(*x, causal=True, scale=scale)
+    gr = torch.autograd.grad(o, x, do)
+    y = [t[:2, :, :3].detach().float().contiguous().requires_grad_() for t in x]
+    r, _ = attention_reference(*y, True, scale)
+    ref = torch.autograd.grad(r, y, do[:2, :, :3].float())
+    for a, b in zip(gr, ref):
+        _close(a[:2, :, :3], b)
