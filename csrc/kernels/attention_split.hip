@@ -450,6 +450,11 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dq_split_kernel(Fa
 template <int D, int G, bool WIN, int RW, int KG, int WPS>
 __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(FastBwdParams p) {
   constexpr int BK = 32 * RW, BQ = 32, NTG = 64 * RW;
+  // The sums start with a row's -lse (over the scale) and -delta: no LDS read is left to wait for behind the products, where no register
+  // is free to hold them, and the subtractions go. dK/dV, us: 64 wide, one group, 8 x 1000 x 12 heads 47.2 -> 41.3, 6 x 1024 x 16 46.8 ->
+  // 42.4, 16 x 380 x 12 21.3 -> 19.6; 128 wide, two groups, 2048 x 14 with ALiBi 75.9 -> 72.2, 700 x 20 25.0 -> 24.3. ALiBi and windows
+  // spill at 64 (51.9 -> 61.2), 64 wide in two groups, 96 wide and 128 wide in one gain and lose 4 %.
+  constexpr bool START = D == 64 ? KG == 1 && G == 1 && !WIN : D == 128 && KG == 2;
   constexpr int TILE = BQ * D * 2, KS = D / 16, NCH = D / 8;
   using Stg = GroupStager<D, NTG>;
   constexpr int CPT = Stg::CPT;
@@ -469,7 +474,7 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
   const int off = p.Sk - p.Sq;
   const int kw = kb * BK + rw * 32, key = kw + l32;
   const int kv_end = batch_keys(p.kv_len, b, p.Sk);
-  const float sl2 = p.scale * kLog2e;
+  const float sl2 = p.scale * kLog2e, inv = 1.f / p.scale;
 
   const int q_lo = max(0, kb * BK - off) & ~(BQ - 1);
   // no query sees a block past the length; past the last key's window no query sees the block
@@ -508,9 +513,9 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
     stq.store(xq, own + buf * 2 * TILE);
     sto.store(xg, own + buf * 2 * TILE + TILE);
     if (gt < 64) {
-      float v = gt < 32 ? lreg * kLog2e : lreg;
+      float v = lreg;
       if (q_lo + qcur * BQ + (gt & 31) >= p.Sq) v = gt < 32 ? INFINITY : 0.f;  // P = 0
-      stat[buf * 64 + gt] = v;
+      stat[buf * 64 + gt] = !START ? (gt < 32 ? v * kLog2e : v) : gt < 32 ? -v * inv : -v;
     }
   };
   if (total > 0) {  // (flies with the key and value rows)
@@ -561,7 +566,17 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
     asm volatile("" ::: "memory");
     f32x16 sacc, dpacc;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) { sacc[r] = 0.f; dpacc[r] = 0.f; }
+    for (int gg = 0; gg < 4; ++gg) {
+      if constexpr (!START) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sacc[4 * gg + j] = dpacc[4 * gg + j] = 0.f;
+        continue;
+      }
+      const f32x4 lq = *reinterpret_cast<const f32x4*>(ls + 8 * gg + 4 * hh), dq4 = *reinterpret_cast<const f32x4*>(ls + 32 + 8 * gg + 4 * hh);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sacc[4 * gg + j] = lq[j], dpacc[4 * gg + j] = dq4[j];
+    }
+    if constexpr (START) __builtin_amdgcn_sched_barrier(0);
     {  // S = Q.K^T, dP = dO.V^T, the three fragments of k-step s + 1 before the MFMAs of step s (pinned)
       bf16x8 fq[2], fg[2], fv[2];
       fq[0] = row_frag<D>(Qs, be, bo, 0), fg[0] = row_frag<D>(Gs, be, bo, 0), fv[0] = row_frag<D>(vimg, be, bo, 0);
@@ -591,11 +606,12 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
     float pr[16];
 #pragma unroll
     for (int gg = 0; gg < 4; ++gg) {
-      const f32x4 lq = *reinterpret_cast<const f32x4*>(ls + 8 * gg + 4 * hh);
+      f32x4 lq{0.f, 0.f, 0.f, 0.f};
+      if constexpr (!START) lq = *reinterpret_cast<const f32x4*>(ls + 8 * gg + 4 * hh);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float bl = G == 2 ? fmaf(-slope, (float)(8 * gg + j), b0) - lq[j] : -lq[j];
-        pr[4 * gg + j] = __builtin_amdgcn_exp2f(fmaf(sacc[4 * gg + j], sl2, bl));
+        pr[4 * gg + j] = __builtin_amdgcn_exp2f(START && G != 2 ? sacc[4 * gg + j] * sl2 : fmaf(sacc[4 * gg + j], sl2, bl));
       }
     }
     if (!plain) {
@@ -608,11 +624,12 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
     bf16x8 p0, p1, s0, s1;
 #pragma unroll
     for (int gg = 0; gg < 4; ++gg) {
-      const f32x4 dq4 = *reinterpret_cast<const f32x4*>(ls + 32 + 8 * gg + 4 * hh);
+      f32x4 dq4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (!START) dq4 = *reinterpret_cast<const f32x4*>(ls + 32 + 8 * gg + 4 * hh);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int r = 4 * gg + j;
-        const float ds = pr[r] * (dpacc[r] - dq4[j]);
+        const float ds = pr[r] * (START ? dpacc[r] : dpacc[r] - dq4[j]);
         if (r < 8) { p0[r] = (__bf16)pr[r]; s0[r] = (__bf16)ds; }
         else { p1[r - 8] = (__bf16)pr[r]; s1[r - 8] = (__bf16)ds; }
       }
@@ -728,7 +745,7 @@ static int with_form(int d, bool alibi, F&& f) {
   return hipGetLastError() == hipSuccess ? 0 : 3;
 }
 
-// Causal calls of 64, 96 and 128 wide heads with 16-byte rows; 1: another head size.
+// Causal calls of 64, 96 and 128 wide heads with 16-byte rows; 1: another head size (or, backward, a scale of nothing).
 int attn_fwd_split(const FastFwdParams& p, int d, hipStream_t stream) {
   const long long blocks = (long long)((p.Sq + 127) / 128) * p.B * p.H;
   const bool two = split_rows(blocks, d, p.Sk, p.window);
@@ -742,6 +759,7 @@ int attn_fwd_split(const FastFwdParams& p, int d, hipStream_t stream) {
 }
 
 int attn_bwd_split(const FastBwdParams& p, int d, hipStream_t stream) {
+  if (!(fabsf(p.scale) >= 1e-30f)) return 1;  // the sums start with lse / scale: the generic kernel's
   const long long qblocks = (long long)((p.Sq + 127) / 128) * p.B * p.H, kblocks = (long long)((p.Sk + 127) / 128) * p.B * p.Hkv;
   const bool two = split_rows(qblocks, d, p.Sk, p.window);
   const int kv = split_keys(kblocks, d, p.Sq, p.window);
