@@ -711,22 +711,25 @@ static bool split_rows(long long blocks, int d, int keys, int window) {
 }
 // dK/dV with one group or two, or, 128 wide, 0, 1 or in two groups of four waves (2): there two groups of two take 81 KB of LDS, one
 // workgroup a CU. us, backward with one group, and what two groups (of four waves) take or save:
-//   64 wide:   128 rows, 260 blocks 22.0, +0.2; 256 rows, 340 27.6, -0.8, 400 28.2, +0.9; 512 rows, 480 40.4, -0.8, 560 44.5, +1.9; 1024
-//              rows, 560 68.4, -2.5; 3 x 2048 x 16 (768) 148, -8; a window of 256, 336 41.6, -2.6, 480 43.8, +5.8
+//   64 wide:   (dK/dV alone, one, two) 256 rows, 192 blocks 11.9, 11.3, 264 13.0, 13.5; 500 rows, 288 19.6, 18.5; 768 rows, 432 28.5, 27.3;
+//              1400 rows, 528 47.0, 45.4; 2048 rows, 576 68.5, 66.1, 768 74.8, 87.0; a window of 256, 288 20.2, 18.2, 336 41.6, -2.6, 480 43.8, +5.8
 //   96 wide:   128 rows, 220 23.8, -0.4, 260 30.2, +2.5; 512 rows, 300 47.4, -1.7, 340 48.5, +0.3; 1024 rows, 480 80.5, -0.8
 //   128 wide:  128 rows, 100 23.0, -1.0 (+0.6), 140 25.0, +3.6 (+0.7); 256 rows, 140 33.7, -1.3 (-0.4), 180 34.3, +1.2 (0); 512 rows, 180
 //              48.9, -2.8 (-2.0), 260 54.6, +4.5 (-3.8), 340 57.1, +8.0 (+2.3); 1024 rows, 256 80.0, -7.4 (-7.1), 304 87.4, +2.4 (-9.3), 480
 //              99.2, +17 (-3.9), 560 108, +28 (+6.7); 1 x 2944 x 20 (460) 246, +29 (-37); a window of 256, 96 40.2, -7.1 (-2.2), 144 43.1,
 //              +2.5 (-2.3), 264 48.3, +7.8 (+3.0)
-static int split_keys(long long blocks, int d, int rows, int window) {
-  static const Upto t64[] = {{0, 340}, {512, 480}, {768, 560}, {1536, 768}};
+static int split_keys(long long blocks, int d, int rows, int window, bool alibi) {
+  static const Upto t64[] = {{0, 200}, {400, 340}, {512, 480}, {768, 560}, {1536, 680}};  // (the form START; with ALiBi or a window:)
+  static const Upto m64[] = {{0, 340}, {512, 480}, {768, 560}, {1536, 768}};
   static const Upto t96[] = {{0, 760}, {65, 220}, {384, 280}, {768, 380}, {1024, 480}};
   static const Upto t128[] = {{0, 220}, {65, 100}, {129, 140}, {384, 180}, {768, 220}};
   static const Upto w128[] = {{384, 260}, {512, 300}, {768, 400}, {1024, 512}};
   const bool win = window > 0 && window < rows;
   const int walk = win ? window : rows;
   if (d == 128 && win) return blocks <= 120 ? 1 : blocks <= 220 ? 2 : 0;
-  if (blocks <= (d == 64 ? blocks_upto(t64, walk) : d == 96 ? blocks_upto(t96, walk) : blocks_upto(t128, walk))) return 1;
+  if (blocks <= (d == 96 ? blocks_upto(t96, walk) : d == 128 ? blocks_upto(t128, walk) : alibi || window > 0 ? blocks_upto(m64, walk)
+                                                                                                  : blocks_upto(t64, walk)))
+    return 1;
   return d == 128 && blocks <= blocks_upto(w128, walk) ? 2 : 0;
 }
 
@@ -762,7 +765,7 @@ int attn_bwd_split(const FastBwdParams& p, int d, hipStream_t stream) {
   if (!(fabsf(p.scale) >= 1e-30f)) return 1;  // the sums start with lse / scale: the generic kernel's
   const long long qblocks = (long long)((p.Sq + 127) / 128) * p.B * p.H, kblocks = (long long)((p.Sk + 127) / 128) * p.B * p.Hkv;
   const bool two = split_rows(qblocks, d, p.Sk, p.window);
-  const int kv = split_keys(kblocks, d, p.Sq, p.window);
+  const int kv = split_keys(kblocks, d, p.Sq, p.window, p.alibi);
   return with_form(d, p.alibi, [&](auto D_, auto G_) {
     constexpr int D = decltype(D_)::value, G = decltype(G_)::value, W = D == 64 ? 3 : 2;
     if (two)
