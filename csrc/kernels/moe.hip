@@ -646,6 +646,13 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rsrc(const void* p, un
   return __builtin_amdgcn_make_buffer_rsrc((void*)u, (short)0, (int)bytes, 0x00020000);
 }
 
+// its words, for inline asm
+__device__ __forceinline__ u32x4 uniform_words(const void* p) {
+  const unsigned long long a = (unsigned long long)p;
+  return u32x4{(unsigned)__builtin_amdgcn_readfirstlane((unsigned)a), (unsigned)__builtin_amdgcn_readfirstlane((unsigned)(a >> 32) & 0xffff), ~0u,
+               0x00020000};
+}
+
 // four 16-byte LDS reads and their wait in one piece (hipcc would drain every LDS-DMA in flight before a read it sees)
 __device__ __forceinline__ void lds_read4(unsigned a0, unsigned a1, unsigned a2, unsigned a3, u32x4& r0, u32x4& r1,
                                           u32x4& r2, u32x4& r3) {
@@ -768,7 +775,40 @@ __global__ void __launch_bounds__(256, 2) expert_stream_kernel(ExpertArgs p) {
 // Narrow blocks (128 weight rows, tiles to 192 rows, two workgroups a CU) fill the chip with a quarter of the work.
 // Both products of 4096 tokens, 16 experts of 3 x 4096 x 4096, top 2: 1143 -> 904 us (913 TFLOP/s without padding);
 // 16 experts of 3 x 4096 x 2048, top 3: 764 -> 541; 1000 tokens, 32 experts of 3 x 2048 x 1024, top 4: 148 -> 116.
-constexpr int GBK = 64, GN = 256, GM = 256, GEMM_LDS = 2 * (GN + GM) * GBK * 2;
+// Full tiles go another way where K allows it: expert_dma_tile.
+constexpr int GBK = 64, GN = 256, GM = 256, GEMM_LDS = 2 * (GN + GM) * GBK * 2, WIDE_LDS = GEMM_LDS / 4 * 5;
+
+// The results of a wave's AI runs of 32 weight rows and BJ of 32 rows
+template <bool UP, int WN, int AI, int WM, int BJ>
+__device__ __forceinline__ void expert_store(const ExpertArgs& p, const f32x16 (&acc)[AI][BJ], int lo, int nr, int n0) {
+  const int lane = threadIdx.x & 63, l32 = lane & 31, hh = lane >> 5, N = p.N;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wn = wv % WN, wm = wv / WN;
+#pragma unroll
+  for (int j = 0; j < BJ; ++j) {
+    const int r = wm * BJ * 32 + j * 32 + l32;
+    if (r >= nr) continue;
+    const float s = p.scale ? p.wts[p.perm[lo + r]] : 1.f;
+    bf16_t* y = reinterpret_cast<bf16_t*>(p.y) + (long long)(lo + r) * N;
+#pragma unroll
+    for (int i = 0; i < (UP ? AI / 2 : AI); ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int n = n0 + (wn * (UP ? AI / 2 : AI) + i) * 32 + 8 * q + 4 * hh;
+        if (n >= N) continue;  // (N % 4 == 0)
+        float o[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (UP) {
+            const float gt = acc[i][j][4 * q + e] * s, up = acc[AI / 2 + i][j][4 * q + e] * s;
+            o[e] = gt * __builtin_amdgcn_rcpf(1.f + __expf(-gt)) * up;
+          } else {
+            o[e] = acc[i][j][4 * q + e] * s;
+          }
+        }
+        *reinterpret_cast<uint2*>(y + n) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+      }
+  }
+}
 
 // WN x WM waves, each with AI runs of 32 weight rows and BJ of 32 rows. FAR: addresses of 64 bits, for activations or an expert's
 // weights that 32-bit byte offsets do not span
@@ -897,31 +937,126 @@ __device__ __forceinline__ void expert_gemm_tile(const ExpertArgs& p, bf16_t* gl
     stage(t, std::integral_constant<int, 0>{});
     stage(t + 1, std::integral_constant<int, 1>{});
   }
+  expert_store<UP, WN, AI, WM, BJ>(p, acc, lo, nr, n0);
+}
+
+// Full tiles (more than 192 rows, K % 64 == 0), staged by the memory system: 16 bytes a lane straight into LDS, in 5 stages of 32. No
+// register holds a piece on its way and no instruction stores one, so that beside the products a wave only reads the next
+// sub-step's fragments and requests stages (pinned behind pairs of products). The barrier stands before a stage's last sub-step, as above:
+// all waves then have the stage in registers. Same sums in the same order as above.
+// A request of 1 KB takes a CU's address path 16 cycles, half of the products' time: bunched behind the barrier they held the products up.
+// What bounds it now: the products 59 % of a block's time, waits for loads and barriers a quarter.
+// A whole sublayer, us, staged through registers and this: 4096 tokens, 16 experts of 3 x 4096 x 4096, top 2 966 -> 928, with another
+// routing 973 -> 884; 3000 tokens, 32 experts of 3 x 2048 x 1024, top 4 257 -> 248; 3500 of 24 of 3 x 2048 x 768, top 5 232 -> 228. The first
+// in four stages, a request a pair behind the barrier 1055, in five with two a pair 1039 (981 through registers). Requests over
+// four sub-steps: the same. Tiles of 129 to 192 rows in blocks of 4 waves x all rows lose (1200 tokens as the first 383 -> 391) or gain
+// 2 % (1450 tokens); of up to 128 the same.
+// A row's four pieces lie turned by (row / 4) % 4, so 16 rows x one piece cover all 64 banks.
+template <bool UP>
+__device__ __forceinline__ void expert_dma_tile(const ExpertArgs& p, bf16_t* gl, int ex, int lo, int nr, int n0) {
+  constexpr int WN = 2, AI = 4, WM = 2, BJ = 4;                  // as above
+  constexpr int WP = WN * AI, RP = WM * BJ, NP = (WP + RP) / 2;  // runs of 32 rows: weights, activations; 1 KB pieces a wave a stage
+  constexpr int DK = 32, NS = 5, STG = (WP + RP) * 32 * DK;      // one stage (elements)
+  constexpr int NM = AI * BJ, NF = AI + BJ, NC = NM / 2;
+  static_assert(NF == NC && NS * STG * 2 <= WIDE_LDS, "two fragments a pair of products, in the first half of them");
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), wn = wv % WN, wm = wv / WN;
+  const int K = p.K, N = p.N, nk = K / DK;
+  const u32x4 rw = uniform_words(reinterpret_cast<const bf16_t*>(p.w) + (long long)ex * (UP ? 2 * N : N) * K);
+  const u32x4 rx = uniform_words(reinterpret_cast<const bf16_t*>(p.x) + (UP ? 0ll : (long long)lo * K));
+  // piece i of wave wv: rows (4 i + wv) 16 + lane / 4
+  const unsigned ch = ((lane & 3) ^ ((lane >> 4) & 3)) * 16, rb = (unsigned)K * 2;
+  unsigned from[NP];
 #pragma unroll
-  for (int j = 0; j < BJ; ++j) {
-    const int r = wm * BJ * 32 + j * 32 + l32;
-    if (r >= nr) continue;
-    const float s = p.scale ? p.wts[p.perm[lo + r]] : 1.f;
-    bf16_t* y = reinterpret_cast<bf16_t*>(p.y) + (long long)(lo + r) * N;
-#pragma unroll
-    for (int i = 0; i < (UP ? AI / 2 : AI); ++i)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int n = n0 + (wn * (UP ? AI / 2 : AI) + i) * 32 + 8 * q + 4 * hh;
-        if (n >= N) continue;  // (N % 4 == 0)
-        float o[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if constexpr (UP) {
-            const float gt = acc[i][j][4 * q + e] * s, up = acc[AI / 2 + i][j][4 * q + e] * s;
-            o[e] = gt * __builtin_amdgcn_rcpf(1.f + __expf(-gt)) * up;
-          } else {
-            o[e] = acc[i][j][4 * q + e] * s;
-          }
-        }
-        *reinterpret_cast<uint2*>(y + n) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
-      }
+  for (int i = 0; i < NP; ++i) {
+    const int r = (4 * i + wv) * 16 + (lane >> 2);
+    if (i < WP / 2) {
+      const int run = r / 32, wrun = run % AI, base = run / AI * (AI / 2) * 32;  // (as above)
+      const int n = UP ? (wrun < AI / 2 ? 0 : N) + min(n0 + base + wrun % (AI / 2) * 32 + (r & 31), N - 1) : min(n0 + r, N - 1);
+      from[i] = (unsigned)n * rb + ch;
+    } else {
+      const int xr = min(r - WP * 32, nr - 1);
+      from[i] = (unsigned)(UP ? p.perm[lo + xr] / p.top : xr) * rb + ch;
+    }
   }
+  const unsigned to = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) char*)gl + wv * 1024);
+  // (in asm: hipcc would let every read of LDS wait for all requests. Nothing is returned to a register, and nothing else here uses m0)
+  auto request = [&](int t, int slot, int i) {
+    const int k = __builtin_amdgcn_readfirstlane(min(t, nk - 1) * DK * 2);  // past the end: the last one, which nobody reads
+    const unsigned at = __builtin_amdgcn_readfirstlane(to + slot * (STG * 2) + i * 4096);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(at), "v"(from[i]),
+                 "s"(i < WP / 2 ? rw : rx), "s"(k));
+  };
+  f32x16 acc[AI][BJ];
+#pragma unroll
+  for (int i = 0; i < AI; ++i)
+#pragma unroll
+    for (int j = 0; j < BJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  const int sw = (l32 >> 2) & 3;
+  const int ar = (wn * AI * 32 + l32) * DK, br = (WP * 32 + wm * BJ * 32 + l32) * DK;
+  bf16x8 a[2][AI], x[2][BJ];
+  auto frag = [&](int slot, int s, int n) {  // fragment n of sub-step s: a run of weights, then one of activations, ...
+    const bf16_t* st = gl + slot * STG + (((2 * s + hh) ^ sw) << 3);
+    if (n % 2 == 0) a[s][n / 2] = *reinterpret_cast<const bf16x8*>(st + ar + n / 2 * 32 * DK);
+    else x[s][n / 2] = *reinterpret_cast<const bf16x8*>(st + br + n / 2 * 32 * DK);
+  };
+  // pair c of sub-step s, and beside it two of the fragments of the next one
+  auto pair = [&](int slot, int s, int c) {
+#pragma unroll
+    for (int n = 2 * c; n < 2 * c + 2 && n < NF; ++n) frag(slot, s ^ 1, n);
+#pragma unroll
+    for (int m = 2 * c; m < 2 * c + 2; ++m)
+      acc[m % AI][m / AI] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s][m % AI], x[s][m / AI], acc[m % AI][m / AI], 0, 0, 0);
+  };
+#pragma unroll
+  for (int t = 0; t < 4; t += 2)
+#pragma unroll
+    for (int i = 0; i < 2 * NP; ++i) request(t + i % 2, t + i % 2, i / 2);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NP) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int n = 0; n < NF; ++n) frag(0, 0, n);
+  int slot = 0;  // of stage t
+  auto after = [](int s) { return s == NS - 1 ? 0 : s + 1; };
+  // Stages t + 4 and t + 5 (t even), a row's two halves together, go into the free place and stage t's: from t's barrier on, evenly
+  // over three sub-steps (a CU takes 16 cycles a request; in one sub-step they held the products up)
+  constexpr auto upto = [](int c) { return c * 2 * NP / (3 * NC); };
+  auto requests = [&](int t, int free, int own, int c) {
+#pragma unroll
+    for (int i = upto(c); i < upto(c + 1); ++i) request(t + 4 + i % 2, i % 2 ? own : free, i / 2);
+  };
+  auto stage = [&](int t, auto odd_) {
+    constexpr bool odd = decltype(odd_)::value;
+    const int next = after(slot), before = slot == 0 ? NS - 1 : slot - 1, before2 = before == 0 ? NS - 1 : before - 1;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      pair(slot, 0, c);
+      if (odd) requests(t - 1, before2, before, NC + c);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // stage t is in all waves' registers, stage t + 1 in LDS (what was requested after it may be on its way)
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(odd ? upto(2 * NC) : 2 * NP) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      pair(next, 1, c);
+      if (odd) requests(t - 1, before2, before, 2 * NC + c);
+      else requests(t, before, slot, c);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    slot = next;
+  };
+  for (int t = 0; t < nk; t += 2) {
+    stage(t, std::false_type{});
+    stage(t + 1, std::true_type{});
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the repeated stages, before the LDS is given back
+  expert_store<UP, WN, AI, WM, BJ>(p, acc, lo, nr, n0);
 }
 
 // NARROW: tiles of up to 192 rows x 128 weight rows (FAR: 128 rows)
@@ -958,6 +1093,8 @@ __global__ void __launch_bounds__(256, NARROW ? 2 : 1) expert_gemm_kernel(Expert
     if (nr > 128) expert_gemm_tile<UP, 2, 2, 2, 3>(p, gl, tl[0], tl[1], nr, n0);
     else if (nr > 64) expert_gemm_tile<UP, 2, 2, 2, 2>(p, gl, tl[0], tl[1], nr, n0);
     else expert_gemm_tile<UP, 2, 2, 2, 1>(p, gl, tl[0], tl[1], nr, n0);
+  } else if (p.K % 64 == 0 && nr > 192) {
+    expert_dma_tile<UP>(p, gl, tl[0], tl[1], nr, n0);
   } else {
     if (nr > 192) expert_gemm_tile<UP, 2, 4, 2, 4>(p, gl, tl[0], tl[1], nr, n0);
     else if (nr > 160) expert_gemm_tile<UP, 4, 2, 1, 6>(p, gl, tl[0], tl[1], nr, n0);
@@ -970,7 +1107,7 @@ __global__ void __launch_bounds__(256, NARROW ? 2 : 1) expert_gemm_kernel(Expert
 
 template <bool UP, bool NARROW, bool FAR = false>
 int gemm_go(const ExpertArgs& a, int max_tiles, hipStream_t s) {
-  constexpr int NB = (NARROW ? 128 : 256) / (UP ? 2 : 1), LDS = NARROW ? GEMM_LDS / 8 * 5 : GEMM_LDS;
+  constexpr int NB = (NARROW ? 128 : 256) / (UP ? 2 : 1), LDS = NARROW ? GEMM_LDS / 8 * 5 : WIDE_LDS;
   auto kern = expert_gemm_kernel<UP, NARROW, FAR>;
   if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess) return 5;
   hipLaunchKernelGGL(kern, dim3((a.N + NB - 1) / NB * max_tiles), dim3(256), LDS, s, a);

@@ -25,7 +25,8 @@ def _case(counts, top, d, F, seed=0):
 @pytest.mark.parametrize("mt", [moe.STREAM_ROWS, 128, 192, moe.GEMM_ROWS])
 @pytest.mark.parametrize("scale_in", [True, False])
 @pytest.mark.parametrize("counts,top,d,F", [([0, 1, 16, 17, 32, 33, 15], 2, 64, 64), ([31, 64, 65, 0, 8], 3, 320, 192),
-                                            ([1], 1, 128, 64), ([129, 127, 256, 2], 2, 192, 320), ([65, 96, 97, 160, 161, 193, 257, 191], 4, 72, 200), ([40, 40], 4, 64, 576)])
+                                            ([1], 1, 128, 64), ([129, 127, 256, 2], 2, 192, 320), ([65, 96, 97, 160, 161, 193, 257, 191], 4, 72, 200), ([40, 40], 4, 64, 576),
+                                            ([193, 256, 225, 255, 512, 449], 2, 128, 192), ([449, 191, 200, 224], 4, 704, 320)])
 def test_products(mt, scale_in, counts, top, d, F):
     if mt == moe.STREAM_ROWS and (d % 64 or F % 64):
         pytest.skip("the stream takes whole stages")
