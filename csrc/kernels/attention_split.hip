@@ -13,7 +13,7 @@
 //
 // Tiles in LDS: two buffers of K and V a group. A step computes S of the group's next tile while it takes the softmax of this
 // one, so K runs a tile ahead of V: K(i + 2) goes where K(i) was and V(i + 1) where V(i - 1) was, which all waves have read
-// before the last barrier.
+// before the last barrier (K(0), which is read before the first step, has one of its own).
 //
 // Softmax reference: as in attn_fwd_tiled_kernel the row's maximum over the first tile with a visible key, here of each
 // group; the groups' sums are scaled to the largest reference when they meet. Rows whose sum passes 2^100 (a later score far
@@ -150,6 +150,7 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_fwd_split_kernel(FastF
     stk.store(xk, kbuf + TILE);
     __syncthreads();
     f32x16 sa = qk(kbuf);
+    __syncthreads();  // all waves have read K(0), for the first step stores K(2) in its place
 
     auto step = [&](int i, auto masked) {
       constexpr bool MASKED = decltype(masked)::value, HEAD = decltype(masked)::value == 2;

@@ -1,0 +1,52 @@
+"""LDS of the attention kernels whose wave groups stage tiles for each other: between two barriers no wave may read what another
+writes. The kernels' own source runs on the host, thread after thread, with a callback at every load and store (lds_trace/)."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CLANG = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "clang++")
+pytestmark = pytest.mark.skipif(not os.path.exists(CLANG), reason="no clang of ROCm")
+
+
+@pytest.fixture(scope="module")
+def trace(tmp_path_factory):
+    d, src = str(tmp_path_factory.mktemp("lds_trace")), os.path.join(ROOT, "tests", "lds_trace")
+    base = [CLANG, "-x", "c++", "-std=c++17", "-w", "-mavx512f", "-I" + src]
+    objs = [os.path.join(d, n) for n in ("trace.o", "kernels.o")]
+    subprocess.run([*base, "-O1", "-c", os.path.join(src, "trace.cpp"), "-o", objs[0]], check=True)
+    subprocess.run([*base, "-O0", "-fsanitize-coverage=func,trace-pc,trace-loads,trace-stores", "-c",
+                    os.path.join(src, "kernels.cpp"), "-o", objs[1]], check=True)
+    exe = os.path.join(d, "trace")
+    subprocess.run([CLANG, *objs, "-o", exe], check=True)
+
+    def run(kernel, *args, **env):
+        r = subprocess.run([exe, kernel, *map(str, args)], capture_output=True, text=True, env=dict(os.environ, **env))
+        assert r.returncode == 0, r.stderr
+        last = dict(line.rsplit(" ", 1) for line in r.stdout.splitlines()[-2:])
+        assert int(last["accesses"]) > 1000
+        return int(last["races"]), r.stdout
+    return run
+
+
+# batch, queries, keys, heads, KV heads: two groups, one group (more blocks than the split calls), and, 128 wide, dK/dV of eight waves
+FEW, MANY, EIGHT = (1, 300, 300, 2, 1), (13, 270, 290, 48, 48), (5, 400, 400, 10, 10)
+MASKS = {"plain": (0, 0, 0), "window": (70, 0, 0), "alibi": (0, 1, 0), "lengths": (0, 0, 1)}
+
+
+@pytest.mark.parametrize("mask", MASKS)
+@pytest.mark.parametrize("shape", [FEW, MANY, EIGHT, (1, 32, 32, 1, 1), (2, 64, 64, 1, 1)])
+@pytest.mark.parametrize("D", [64, 96, 128, 256])
+def test_no_races(trace, D, shape, mask):
+    # the last argument: an ordinary softmax weight, and one whose rows overflow, so that they are computed again
+    for kernel, weight in (("fwd", 1), ("fwd", 1e30), ("bwd", 1)):
+        if D < 256 or kernel == "bwd":
+            races, out = trace(kernel, D, *shape, *MASKS[mask], weight)
+            assert races == 0, out
+
+
+def test_the_trace_sees_exchanges(trace):
+    """Without the barriers every tile that one wave stores and another reads is reported."""
+    for kernel, D in (("fwd", 64), ("bwd", 64), ("bwd", 256)):
+        assert trace(kernel, D, *FEW, *MASKS["plain"], 1, LDS_TRACE_NO_BARRIERS="1")[0] > 1000
