@@ -62,7 +62,8 @@ __global__ void __launch_bounds__(256) rope_append_kernel(AppendArgs a) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float u = to_f<F16>(x.e[2 * i]), w = to_f<F16>(x.e[2 * i + 1]);
-        const bf16_t p = from_f<F16>(u * c[i] - w * n[i]), r = from_f<F16>(w * c[i] + u * n[i]);
+        // (which product is rounded first is written out: the compiler's choice hangs on the code around it)
+        const bf16_t p = from_f<F16>(fmaf(u, c[i], -(w * n[i]))), r = from_f<F16>(fmaf(u, n[i], w * c[i]));
         if (d + 2 * i < a.rot) x.e[2 * i] = p, x.e[2 * i + 1] = r;
       }
     } else {  // pairs (i, i + rot / 2): the partners are read before any lane of the row stores
@@ -84,7 +85,7 @@ __global__ void __launch_bounds__(256) rope_append_kernel(AppendArgs a) {
       }
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const bf16_t r = from_f<F16>(to_f<F16>(x.e[i]) * c[i] + to_f<F16>(y.e[i]) * n[i]);
+        const bf16_t r = from_f<F16>(fmaf(to_f<F16>(x.e[i]), c[i], to_f<F16>(y.e[i]) * n[i]));
         if (d + i < a.rot) x.e[i] = r;
       }
     }

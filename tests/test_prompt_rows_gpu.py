@@ -81,6 +81,32 @@ def test_rope_append(dtype, D, rot, inter, page_size):
     assert torch.equal(c.v[0], ref.v[0])
 
 
+@pytest.mark.parametrize("D,rot,inter", [(256, 64, True), (128, 64, False), (64, 36, False), (64, 20, True)])
+def test_rope_append_rounds_one_product_first(D, rot, inter):
+    """Bit for bit a product in fp32 and a fused multiply-add of the other one (pairs side by side: w c first, then u s). Which of
+    the two comes first shows in one of some 1e5 elements. (fp16 rounds some fused multiply-adds once, some twice.)"""
+    T, H, half, dtype = 3001, 16, rot // 2, torch.bfloat16
+    c = KVCache(1, 1, H, T, D, "cuda", dtype, page_size=0)
+    page, off, pos = (torch.from_numpy(x).cuda() for x in c.rows([0], [T], [0]))
+    qkv = torch.randn(T, 3, H, D, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1)).to(dtype)
+    cos, sin = rope_tables(rot, T, 10000.0, "cuda")
+    want = qkv.clone()
+    x = want[:, :2, :, :rot]
+    u, w = (x[..., 0::2], x[..., 1::2]) if inter else (x[..., :half], x[..., half:])
+    cs, sn = (t[:, None, None].double() for t in (cos, sin))
+    u, w = u.double(), w.double()
+    first = lambda a, b: (a * b).float().double()  # noqa: E731
+    if inter:
+        a, b = u * cs - first(w, sn), u * sn + first(w, cs)
+    else:
+        a, b = u * cs + first(w, -sn), w * cs + first(u, sn)
+    a, b = a.float().to(dtype), b.float().to(dtype)
+    x.copy_(torch.stack([a, b], -1).flatten(-2) if inter else torch.cat([a, b], -1))
+    assert ops.rope_append(*qkv.unbind(1), rot, inter, cos, sin, pos, page, off, c.k[0], c.v[0])
+    assert torch.equal(qkv, want)
+    assert torch.equal(c.k[0][0, :, :T], want[:, 1].transpose(0, 1)) and torch.equal(c.v[0][0, :, :T], want[:, 2].transpose(0, 1))
+
+
 TINY = {
     "gptj": dict(model_type="gptj", vocab_size=512, n_embd=128, n_layer=2, n_head=2, n_positions=512, rotary_dim=32),
     "gpt2": dict(model_type="gpt2", vocab_size=512, n_embd=128, n_layer=2, n_head=2, n_positions=512),
