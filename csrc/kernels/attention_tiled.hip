@@ -1509,7 +1509,8 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
   (void)hipGetLastError();
   const bool aligned = rows16(q, q_sb, q_st, q_sh) && rows16(k, k_sb, k_st, k_sh) && rows16(v, v_sb, v_st, v_sh) &&
                        rows16(o, o_sb, o_st, o_sh);
-  if (causal && aligned && rowsum_col < 0 && max_col < 0) {
+  const bool general = alibi || kv_len || window || cu || Sq % 128 || Sk % 32;  // (these forms take the row sums as everywhere else)
+  if (causal && aligned && (general || (rowsum_col < 0 && max_col < 0))) {
     const int rc = attn_fwd_split(p, d, stream);
     if (rc != 1) return rc ? rc : -1;
   }
@@ -1538,14 +1539,15 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
                                      blocks128 <= (walk <= 256 ? 2000 : walk >= 2000 && !alibi ? 768 : 512));
   if (four) {
     if (alibi) hipLaunchKernelGGL((attn_fwd_w8_kernel<256, true, 4, 2, 2>), grid, dim3(256), 0, stream, p);
-    else if (kv_len || window || cu || Sq % 128 || Sk % 32)
+    else if (general)
       hipLaunchKernelGGL((attn_fwd_w8_kernel<256, true, 4, 2, 1>), grid, dim3(256), 0, stream, p);
     else hipLaunchKernelGGL((attn_fwd_w8_kernel<256, true, 4, 2>), grid, dim3(256), 0, stream, p);
     return hipGetLastError() != hipSuccess ? 3 : -1;
   }
-  if (alibi || kv_len || window || cu || Sq % 128 || Sk % 32 || two) {
+  if (general || two) {
     if (!aligned) return 1;
-    const bool done = general_form(d, causal, alibi, [&](auto D_, auto C_, auto G_) {
+    bool here = false;
+    general_form(d, causal, alibi, [&](auto D_, auto C_, auto G_) {
       constexpr int D = decltype(D_)::value, G = decltype(G_)::value;
       constexpr bool C = decltype(C_)::value;
       if constexpr (D == 256) {
@@ -1553,11 +1555,13 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
           if (two) hipLaunchKernelGGL((attn_fwd_w8_kernel<D, C, 8, 4, G, 2>), grid, dim3(512), 0, stream, p);
         if (!two)
           hipLaunchKernelGGL((attn_fwd_w8_kernel<D, C, 8, 4, G>), dim3(((Sq + 255) / 256) * B * H), dim3(512), 0, stream, p);
-        whole = true;
-      } else if constexpr (!C || D == 160)  // (the other causal ones: attention_split.hip)
+        here = whole = true;
+      } else if constexpr (!C || D == 160) {  // (the other causal ones: attention_split.hip)
         hipLaunchKernelGGL((attn_fwd_tiled_kernel<D, C, -1, D, -1, G>), grid, dim3(256), 0, stream, p);
+        here = true;
+      }
     });
-    return !done ? 1 : hipGetLastError() != hipSuccess ? 3 : whole ? -1 : 0;
+    return !here ? 1 : hipGetLastError() != hipSuccess ? 3 : whole ? -1 : 0;
   }
   if ((d != 48 && d != 64 && d != 96 && d != 128 && d != 160 && d != 256)) return 1;
   if (max_col >= 0 && (max_col != 40 || rowsum_col != 40 || d != 48)) return 1;  // instantiated variant

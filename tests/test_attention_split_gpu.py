@@ -93,3 +93,22 @@ def test_scales(D, scale):
     ref = torch.autograd.grad(r, y, do[:2, :, :3].float())
     for a, b in zip(gr, ref):
         _close(a[:2, :, :3], b)
+
+
+@pytest.mark.parametrize("mask", ["ragged", "keys", "lens", "window", "alibi", "none"])
+@pytest.mark.parametrize("D", [64, 96, 128, 160, 256])
+def test_column_of_ones(D, mask):
+    """A causal call that names V's column of ones has a result of its own whatever the mask and the size."""
+    S = 200 if mask == "ragged" else 256
+    g = torch.Generator(device="cuda").manual_seed(D)
+    q, k, v = (torch.randn(2, S + (40 if mask == "keys" and i else 0), 3, D, device="cuda", generator=g).bfloat16() for i in range(3))
+    v[..., 40] = 1
+    ln = torch.tensor([S, 77], device="cuda", dtype=torch.int32) if mask == "lens" else None
+    sl = 2.0 ** -torch.arange(1, 4, device="cuda").float() if mask == "alibi" else None
+    window = 50 if mask == "window" else 0
+    # (what the allocator hands out next is zero: as overflow marks it leaves no row to the generic kernel)
+    free = [torch.zeros(n, device="cuda", dtype=torch.uint8) for n in (*[512] * 64, *[65536] * 16, *[2 * S * 3 * D * 2] * 4)]
+    del free
+    with torch.no_grad():
+        o = flash_attention(q, k, v, causal=True, kv_len=ln, alibi=sl, window=window, rowsum_col=40)
+    _close(o, attention_reference(q.float(), k.float(), v.float(), True, None, ln, sl, window)[0])
