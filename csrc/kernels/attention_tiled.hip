@@ -671,7 +671,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D == 256 ? 2 : 1) attn_fwd
   constexpr int PART = 32 * D * 4;  // a wave's partial sums
   static_assert((KG - 1) * RW * PART <= SMEM, "the partial sums take the tiles' place");
   __shared__ __attribute__((aligned(1024))) char smem[SMEM];  // [buf][K|V]; epilogue: [wave][32][D]
-  __shared__ float stat[KG > 1 ? KG : 1][RW][32][2];          // reference, sum of each row and group
+  __shared__ float stat[KG > 1 ? KG : 1][RW][32][3];          // reference, sum and divisor of each row and group
   __shared__ int again;
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -939,6 +939,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D == 256 ? 2 : 1) attn_fwd
     if (hh == 0) {
       stat[g][rw][l32][0] = m;
       stat[g][rw][l32][1] = ltot;
+      stat[g][rw][l32][2] = rtot;
     }
     __syncthreads();
     if (g > 0) return;
@@ -947,7 +948,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D == 256 ? 2 : 1) attn_fwd
     for (int i = 1; i < KG; ++i) m = fmaxf(m, stat[i][rw][l32][0]);
     auto weight = [&](float x) { return x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(x - m); };
     const float w0 = weight(m0);
-    ltot *= w0;
+    ltot *= w0, rtot *= w0;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
@@ -956,13 +957,14 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D == 256 ? 2 : 1) attn_fwd
     for (int i = 1; i < KG; ++i) {
       const float w = weight(stat[i][rw][l32][0]);
       ltot = fmaf(stat[i][rw][l32][1], w, ltot);
+      rtot = fmaf(stat[i][rw][l32][2], w, rtot);
       add_partial<D>(smem + ((i - 1) * RW + rw) * PART, oacc, lane, w);
     }
-    rtot = ltot;
   }
   // With a window a row's first tile holds 16 of its keys on average: the reference is its largest weight less often than
   // elsewhere (attn_fwd_tiled_kernel). Dividing by the rounded weights makes up for it: error against 64 bits of 2 x 1000 x 16
-  // heads, window 256, 0.00213 -> 0.00210 (generic kernel 0.00212). lse keeps the sum of the unrounded ones.
+  // heads, window 256, 0.00213 -> 0.00210 (generic kernel 0.00212). lse keeps the sum of the unrounded ones. Two groups, 1 x 2048 x 16,
+  // window 1024: 0.00209 -> 0.00207 (one group 0.00210), 48.1 -> 50.2 us; a row that one far later key dominates is that key's value to the bit.
   const float inv = ltot > 0.f ? 1.f / rtot : 0.f;
   if (hh == 0 && p.lse && (!G || qrow < p.Sq))
     p.lse[((long long)b * p.H + h) * p.Sq + qrow] = ltot > 0.f ? (m + log2f(ltot)) * kLn2 : INFINITY;

@@ -63,3 +63,21 @@ def test_four_waves_far_above_their_first_tile(alibi):
     r, want = A.attention_reference(*(t[:1, :, :2].float() for t in (q, k, v)), True, None, None, None if sl is None else sl[:2])
     _close(o[:1, :, :2], r)
     torch.testing.assert_close(lse[:1, :2], want, rtol=2.0 ** -18, atol=2.0 ** -16)  # (as in test_attention_split_gpu.py)
+
+
+@pytest.mark.parametrize("H", [16, 40])
+def test_a_window_divides_by_the_rounded_weights(H):
+    """One key whose weight is 2^25 times all others' and no row's reference: a row is that key's value to the bit, for the rounding of
+    its weight cancels, with the keys in two groups (16 heads) as in one."""
+    S, D, at = 2048, 256, (500, 1600)
+    q, k, v = (torch.zeros(1, S, H, D, device="cuda") for _ in range(3))
+    q[..., 0] = 1
+    v.copy_(1 + torch.rand(v.shape, device="cuda", generator=torch.Generator(device="cuda").manual_seed(0)))
+    for j in at:
+        k[0, j, :, 0] = 16 * (18 + 0.25 * torch.arange(H, device="cuda"))  # (every head's weight rounds differently)
+    q, k, v = (t.bfloat16() for t in (q, k, v))
+    with torch.no_grad():
+        o = A.flash_attention(q, k, v, causal=True, window=1024)
+    for j in at:
+        end = min(S, j + 1024)
+        assert torch.equal(o[0, j:end], v[0, j].expand(end - j, H, D))
