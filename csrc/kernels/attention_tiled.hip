@@ -1482,7 +1482,8 @@ bool general_form(int d, bool causal, bool alibi, F&& f) {
 
 }  // namespace
 
-// A/B knob for the full-tile kernels: bit 0 = 8-wave D = 256 forward (attn_fwd_w8_kernel).
+// A/B knob for the full-tile kernels: bit 0 = the LDS-DMA forward of D = 256 (attn_fwd_w8_kernel in all its forms; off: full tiles take
+// attn_fwd_tiled_kernel, other causal calls the 8-wave general form).
 // (An LDS-DMA dQ kernel -- four buffers, three K/V tiles in flight, asm LDS reads -- measured
 // 1.5-2.5 % slower on GPT-J fwd+bwd than the register-staged one and was dropped.)
 static int g_attn_variant = 1;
@@ -1535,7 +1536,7 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
   const int n128 = (Sq + 127) / 128;
   const long long heads = (long long)B * H, blocks256 = (Sq + 255) / 256 * heads, blocks128 = n128 * heads;
   const int walk = window > 0 ? min(Sk, window) : Sk;
-  const bool c256 = d == 256 && causal && aligned;
+  const bool c256 = d == 256 && causal && aligned && (g_attn_variant & 1);
   const bool two = c256 && Sq > 256 && blocks256 <= (walk >= 3000 ? 256 : walk >= 1400 ? 240 : walk >= 900 ? 128 : 0);
   const bool four = c256 && !two && (walk < Sk || (n128 % 2 && n128 <= 5) || (Sq % 128 == 0 && Sq % 256) ||
                                      blocks128 <= (walk <= 256 ? 2000 : walk >= 2000 && !alibi ? 768 : 512));

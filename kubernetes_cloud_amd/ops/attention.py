@@ -75,8 +75,8 @@ _VARIANT = [1]
 
 
 def set_variant(v: int) -> int:
-    """Full-tile kernel variants (A/B knob, attention_tiled.hip): bit 0 = the 8-wave D = 256
-    forward (default on). Returns the previous value."""
+    """Full-tile kernel variants (A/B knob, attention_tiled.hip): bit 0 = the D = 256 forward that loads
+    straight into LDS, in its forms of 4 and 8 waves (default on). Returns the previous value."""
     _lib.call("kca_attn_set_variant", int(v))
     old, _VARIANT[0] = _VARIANT[0], int(v)
     return old

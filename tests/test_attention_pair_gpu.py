@@ -81,3 +81,20 @@ def test_a_window_divides_by_the_rounded_weights(H):
     for j in at:
         end = min(S, j + 1024)
         assert torch.equal(o[0, j:end], v[0, j].expand(end - j, H, D))
+
+
+def test_variants_are_two_kernels():
+    """``set_variant(0)`` takes the register-staged forward where the other one walks keys in two groups, whose sums are added in
+    another order: not the same bits."""
+    g = torch.Generator(device="cuda").manual_seed(2)
+    q, k, v = (torch.randn(2, 1024, 3, 256, device="cuda", generator=g).bfloat16() for _ in range(3))
+    outs = []
+    for var in (1, 0):
+        old = A.set_variant(var)
+        try:
+            with torch.no_grad():
+                outs.append(A.flash_attention(q, k, v, causal=True))
+        finally:
+            A.set_variant(old)
+    assert not torch.equal(*outs)
+    _close(*outs)
