@@ -110,7 +110,7 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_dkdv_pair_kernel(FastBwdParam
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), rw = wave % RW;
-  const auto [kb, bh] = block_of<CAUSAL>((p.Sk + BK - 1) / BK, p.B * p.Hkv);
+  const auto [kb, bh] = block_of<CAUSAL, D, BK>((p.Sk + BK - 1) / BK, p.B * p.Hkv);
   const int b = bh / p.Hkv, hk = bh % p.Hkv;
   const int grp = p.H / p.Hkv;
   const int off = p.Sk - p.Sq;
@@ -332,7 +332,7 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_dq_pair_kernel(FastBwdParams 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), rw = wave % RW;
   const int nqb = (p.Sq + BM - 1) / BM;
-  const auto [qi, bh] = block_of<CAUSAL>(nqb, p.B * p.H);
+  const auto [qi, bh] = block_of<CAUSAL, D, BM>(nqb, p.B * p.H);
   const int qb = CAUSAL ? nqb - 1 - qi : qi;
   const int b = bh / p.H, h = bh % p.H, hk = h / (p.H / p.Hkv);
   const int off = p.Sk - p.Sq;

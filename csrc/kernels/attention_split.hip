@@ -42,7 +42,7 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_fwd_split_kernel(FastF
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = wave / RW, rw = wave % RW;
   const int l32 = lane & 31, hh = lane >> 5, gi = lane & 15;
   const int nqb = (p.Sq + BM - 1) / BM, heads = p.B * p.H;
-  const auto [qi, bh] = block_of<true, D == 64 ? 3 : 1>(nqb, heads);
+  const auto [qi, bh] = block_of<true, D, BM, D == 64 ? 3 : 1>(nqb, heads);
   const int qb = nqb - 1 - qi;
   const int b = bh / p.H, h = bh % p.H;
   const int hk = h / (p.H / p.Hkv);
@@ -301,7 +301,7 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dq_split_kernel(Fa
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = wave / RW, rw = wave % RW;
   const int l32 = lane & 31, hh = lane >> 5;
   const int nqb = (p.Sq + BM - 1) / BM, heads = p.B * p.H;
-  const auto [qi, bh] = block_of<true, D == 64 ? 3 : 1>(nqb, heads);
+  const auto [qi, bh] = block_of<true, D, BM, D == 64 ? 3 : 1>(nqb, heads);
   const int qb = nqb - 1 - qi;
   const int b = bh / p.H, h = bh % p.H;
   const int hk = h / (p.H / p.Hkv);
@@ -469,7 +469,7 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = wave / RW, rw = wave % RW;
   const int l32 = lane & 31, hh = lane >> 5;
   const int heads = p.B * p.Hkv;
-  const auto [kb, bh] = block_of<true, D == 64 ? 3 : 1>((p.Sk + BK - 1) / BK, heads);
+  const auto [kb, bh] = block_of<true, D, BK, D == 64 ? 3 : 1>((p.Sk + BK - 1) / BK, heads);
   const int b = bh / p.Hkv, hk = bh % p.Hkv;
   const int grp = p.H / p.Hkv;
   const int off = p.Sk - p.Sq;

@@ -282,7 +282,7 @@ __global__ void __launch_bounds__(256, (D <= 160 ? 2 : 1)) attn_fwd_tiled_kernel
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5, gi = lane & 15;
   const int nqb = (p.Sq + BM - 1) / BM;
-  const auto [qi, bh] = block_of<CAUSAL>(nqb, p.B * p.H);
+  const auto [qi, bh] = block_of<CAUSAL, D, BM>(nqb, p.B * p.H);
   const int lid = bh * nqb + qi;  // (the order of the fixup kernel's flags)
   const int qb = CAUSAL ? (nqb - 1 - qi) : qi;
   const int b = bh / p.H, h = bh % p.H;
@@ -679,7 +679,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D == 256 ? 2 : 1) attn_fwd
   const int l32 = lane & 31, hh = lane >> 5;
   const int g = KG > 1 ? wave / RW : 0, rw = KG > 1 ? wave % RW : wave;
   const int nqb = (p.Sq + BM - 1) / BM;
-  const auto [qi, bh] = block_of<CAUSAL>(nqb, p.B * p.H);
+  const auto [qi, bh] = block_of<CAUSAL, D, BM>(nqb, p.B * p.H);
   const int qb = CAUSAL ? (nqb - 1 - qi) : qi;
   const int b = bh / p.H, h = bh % p.H;
   const int hk = h / (p.H / p.Hkv);
@@ -1029,7 +1029,7 @@ __global__ void __launch_bounds__(256, (D <= 64 && !CAUSAL && !G) ? 4 : D <= 64 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5;
   const int nqb = (p.Sq + BM - 1) / BM;
-  const auto [qi, bh] = block_of<CAUSAL>(nqb, p.B * p.H);
+  const auto [qi, bh] = block_of<CAUSAL, D, BM>(nqb, p.B * p.H);
   const int qb = CAUSAL ? (nqb - 1 - qi) : qi;
   const int b = bh / p.H, h = bh % p.H;
   const int hk = h / (p.H / p.Hkv);
@@ -1221,7 +1221,7 @@ __global__ void __launch_bounds__(256, D <= 64 ? 3 : D <= 128 ? 2 : 1) attn_bwd_
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hh = lane >> 5;
   const int nkb = (p.Sk + BK - 1) / BK;
-  const auto [kb, bh] = block_of<CAUSAL>(nkb, p.B * p.Hkv);
+  const auto [kb, bh] = block_of<CAUSAL, D, BK>(nkb, p.B * p.Hkv);
   const int b = bh / p.Hkv, hk = bh % p.Hkv;
   const int grp = p.H / p.Hkv;
   const int off = p.Sk - p.Sq;

@@ -36,11 +36,37 @@ __device__ __forceinline__ void own_sequence(FastFwdParams& p, int b) {
 // same (two: the second backwards; three: the second from its middle on, the third in twos backwards). 64-wide heads, 3 a CU, us,
 // forward, dQ, dK/dV: 8 x 1000 x 12 heads 29.0, 36.0, 49.5 -> 26.7, 33.8, 46.4; 3 x 2048 x 16 46.7, 60.6, 91.3 -> 43.2, 56.9, 86.7. Two a
 // CU (96 and 128 wide) gain or lose 3 %: not there.
+//
+// Many blocks: then the keys and values of all heads are walked at one time, and no cache holds them. An XCD takes its heads in turn, a
+// head's blocks beside each other, and longest first among the last 1024 blocks alone (heads_in_turn). us, forward and backward, head after
+// head, all heads at once, so: 559 tokens, 640 heads of 256 229, 275, 207 and 827, 814, 728; 300, 1280 of 256 236, 257, 185 and 740,
+// 736, 644; 850, 1280 of 96 386, 464, 382 and 1053, 1178, 1025; 300, 640 of 128 57, 63, 57 and 174, 170, 161; 559, 640 of 64 71, 77, 70 and
+// 214, 200, 188; 16 x 2048 x 16 of 256 634, 642, 607 and 2502, 2471, 2189. Where a head has 2, 4 or 8 blocks a CU meets one length
+// again and again: 256 tokens, 1024 heads of 256 418, 463 in turn, 450 tokens, 1280 of 64 110, 117. 96-wide heads share their 128-byte
+// lines with their neighbours, which then lie on one XCD: short ones are taken so from the first block on (128 tokens, 2048 heads 51, 47 and
+// 147, 138; 300, 640 heads 59, 54; 2048, 128 heads 147, 156).
+// (blocks of 128 rows: of a head, of all)
+template <int D>
+__device__ __forceinline__ bool heads_in_turn(int blocks, int total) {
+  if (total > 8192 && blocks > 1) return true;
+  if (D == 96) return blocks <= 10 || total > 3072;
+  return blocks > 2 && (blocks % 4 || blocks > 8) && total > (blocks < 8 ? 1536 : 3072);
+}
 struct BlockOf { int block, head; };
-template <bool CAUSAL, int PER_CU = 1>
+template <bool CAUSAL, int D, int ROWS, int PER_CU = 1>
 __device__ __forceinline__ BlockOf block_of(int blocks, int heads) {
   if (CAUSAL) {
     int n = (int)blockIdx.x;
+    if (heads_in_turn<D>((blocks * ROWS + 127) / 128, (int)(gridDim.x * (long long)ROWS / 128))) {
+      const int rest = heads % 8, own = heads / 8;  // (the heads that no XCD has for itself come first)
+      if (n < rest * blocks) return {n / rest, 8 * own + n % rest};
+      n -= rest * blocks;
+      const int last = min(own, (128 + blocks - 1) / blocks), first = own - last, h0 = n % 8 * own;
+      n /= 8;
+      if (n < first * blocks) return {n % blocks, h0 + n / blocks};
+      n -= first * blocks;
+      return {n / last, h0 + first + n % last};
+    }
     if constexpr (PER_CU == 3) {
       const int full = min(PER_CU, (int)gridDim.x / 256), round = n / 256, c = n / 8 % 32;  // (c: the CU of its XCD n % 8)
       if (round > 0 && round < full) {

@@ -50,3 +50,11 @@ def test_the_trace_sees_exchanges(trace):
     """Without the barriers every tile that one wave stores and another reads is reported."""
     for kernel, D in (("fwd", 64), ("bwd", 64), ("bwd", 256)):
         assert trace(kernel, D, *FEW, *MASKS["plain"], 1, LDS_TRACE_NO_BARRIERS="1")[0] > 1000
+
+
+def test_every_block_is_taken_once(tmp_path):
+    """The order of the blocks is one of all blocks of all heads."""
+    src, exe = os.path.join(ROOT, "tests", "lds_trace"), str(tmp_path / "order")
+    subprocess.run([CLANG, "-x", "c++", "-std=c++17", "-w", "-mavx512f", "-O1", "-I" + src, os.path.join(src, "order.cpp"), "-o", exe], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
