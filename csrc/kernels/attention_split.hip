@@ -688,8 +688,9 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
 // Which calls are split in two groups (two waves of 32 rows each, 4 waves a workgroup), the others in blocks of 128 rows and
 // one group: up to so many 128-row blocks of all heads, the more the longer the longest walk is (keys that a row sees; dK/dV: queries),
 // for a split costs each of its blocks the meeting of the sums. One MI355X, us, one group against two:
-//   forward, 64 wide:   128 rows, 340 blocks 10.5, 10.5, 400 10.6, 13.2; 512 rows, 400 15.3, 15.3, 480 15.2, 18.1; 1024 rows, 400 22.5,
-//                       18.7, 480 22.5, 23.2; 3 x 2048 x 12 (576) 39.2, 35.2; 3000 rows with a window of 256, 336 18.7, 15.0, 408 19.3, 19.7
+//   forward, 64 wide:   32 rows, 60 blocks 5.0, 5.6, 288 5.9, 6.8 (one tile is nothing to split); 48 rows, 288 7.2, 7.1; 128 rows, 340
+//                       10.5, 10.5, 400 10.6, 13.2; 512 rows, 400 15.3, 15.3, 480 15.2, 18.1; 1024 rows, 400 22.5, 18.7, 480 22.5, 23.2;
+//                       3 x 2048 x 12 (576) 39.2, 35.2; 3000 rows with a window of 256, 336 18.7, 15.0, 408 19.3, 19.7
 //   96 wide:            128 rows, 100 9.5, 8.7, 140 10.0, 10.6; 256 rows, 140 12.6, 11.5, 180 13.0, 13.4; 512 rows, 220 18.3, 16.9, 260
 //                       19.1, 19.3; 1024 rows, 336 28.4, 26.7, 400 28.9, 30.0; 1 x 1403 x 32 (352) 33.8, 31.2
 //   128 wide:           128 rows, 100 10.3, 9.5, 140 10.8, 11.6, 260 14.0, 18.6; 256 rows, 140 13.8, 13.2, 180 14.1, 14.7; 512 rows, 220
@@ -704,7 +705,7 @@ static int blocks_upto(const Upto (&t)[N], int walk) {
   return b;
 }
 static bool split_rows(long long blocks, int d, int keys, int window) {
-  static const Upto t64[] = {{0, 340}, {512, 400}, {1536, 640}};
+  static const Upto t64[] = {{33, 340}, {512, 400}, {1536, 640}};
   static const Upto t96[] = {{65, 100}, {129, 140}, {384, 220}, {768, 300}, {1024, 336}, {1400, 400}};
   static const Upto t128[] = {{65, 100}, {129, 140}, {384, 180}, {512, 220}, {768, 260}, {1024, 320}};
   const int walk = window > 0 ? min(keys, window) : keys;
@@ -712,25 +713,28 @@ static bool split_rows(long long blocks, int d, int keys, int window) {
 }
 // dK/dV with one group or two, or, 128 wide, 0, 1 or in two groups of four waves (2): there two groups of two take 81 KB of LDS, one
 // workgroup a CU. us, backward with one group, and what two groups (of four waves) take or save:
-//   64 wide:   (dK/dV alone, one, two) 256 rows, 192 blocks 11.9, 11.3, 264 13.0, 13.5; 500 rows, 288 19.6, 18.5; 768 rows, 432 28.5, 27.3;
-//              1400 rows, 528 47.0, 45.4; 2048 rows, 576 68.5, 66.1, 768 74.8, 87.0; a window of 256, 288 20.2, 18.2, 336 41.6, -2.6, 480 43.8, +5.8
-//   96 wide:   128 rows, 220 23.8, -0.4, 260 30.2, +2.5; 512 rows, 300 47.4, -1.7, 340 48.5, +0.3; 1024 rows, 480 80.5, -0.8
-//   128 wide:  128 rows, 100 23.0, -1.0 (+0.6), 140 25.0, +3.6 (+0.7); 256 rows, 140 33.7, -1.3 (-0.4), 180 34.3, +1.2 (0); 512 rows, 180
-//              48.9, -2.8 (-2.0), 260 54.6, +4.5 (-3.8), 340 57.1, +8.0 (+2.3); 1024 rows, 256 80.0, -7.4 (-7.1), 304 87.4, +2.4 (-9.3), 480
-//              99.2, +17 (-3.9), 560 108, +28 (+6.7); 1 x 2944 x 20 (460) 246, +29 (-37); a window of 256, 96 40.2, -7.1 (-2.2), 144 43.1,
+//   64 wide:   32 rows, 60 blocks 10.2, +0.3, 340 12.9, +0.6; 64 rows, 120 11.8, -0.4; (dK/dV alone, one, two) 256 rows, 192 11.9, 11.3, 264
+//              13.0, 13.5; 500 rows, 288 19.6, 18.5; 768 rows, 432 28.5, 27.3; 1400 rows, 528 47.0, 45.4; 2048 rows, 576 68.5, 66.1, 768 74.8,
+//              87.0; a window of 256, 288 20.2, 18.2, 336 41.6, -2.6, 480 43.8, +5.8
+//   96 wide:   64 rows, 60 blocks 13.9, -1.3, 1200 50.2, -3.9; 32 rows, 340 15.2, -0.4; a window of 32 or 64, 120 25, -5, 224 28, -2.5, 340 35,
+//              +1, 480 41, +3; 128 rows, 220 23.8, -0.4, 260 30.2, +2.5; 512 rows, 300 47.4, -1.7, 340 48.5, +0.3; 1024 rows, 480 80.5, -0.8
+//   128 wide:  32 rows, 60 blocks 12.7, +0.4; 64 rows, 220 17.5, -0.9, 260 22.1, +3.4; 128 rows, 100 23.0, -1.0 (+0.6), 140 25.0, +3.6 (+0.7);
+//              256 rows, 140 33.7, -1.3 (-0.4), 180 34.3, +1.2 (0); 512 rows, 180 48.9, -2.8 (-2.0), 260 54.6, +4.5 (-3.8), 340 57.1, +8.0
+//              (+2.3); 1024 rows, 256 80.0, -7.4 (-7.1), 304 87.4, +2.4 (-9.3), 480 99.2, +17 (-3.9), 560 108, +28 (+6.7); 1 x 2944 x 20 (460) 246, +29 (-37); a window of 256, 96 40.2, -7.1 (-2.2), 144 43.1,
 //              +2.5 (-2.3), 264 48.3, +7.8 (+3.0)
 static int split_keys(long long blocks, int d, int rows, int window, bool alibi) {
-  static const Upto t64[] = {{0, 200}, {400, 340}, {512, 480}, {768, 560}, {1536, 680}};  // (the form START; with ALiBi or a window:)
-  static const Upto m64[] = {{0, 340}, {512, 480}, {768, 560}, {1536, 768}};
+  static const Upto t64[] = {{33, 200}, {400, 340}, {512, 480}, {768, 560}, {1536, 680}};  // (the form START; with ALiBi or a window:)
+  static const Upto m64[] = {{33, 340}, {512, 480}, {768, 560}, {1536, 768}};
   static const Upto t96[] = {{0, 760}, {65, 220}, {384, 280}, {768, 380}, {1024, 480}};
-  static const Upto t128[] = {{0, 220}, {65, 100}, {129, 140}, {384, 180}, {768, 220}};
+  static const Upto t128[] = {{33, 220}, {65, 100}, {129, 140}, {384, 180}, {768, 220}};
   static const Upto w128[] = {{384, 260}, {512, 300}, {768, 400}, {1024, 512}};
   const bool win = window > 0 && window < rows;
   const int walk = win ? window : rows;
   if (d == 128 && win) return blocks <= 120 ? 1 : blocks <= 220 ? 2 : 0;
-  if (blocks <= (d == 96 ? blocks_upto(t96, walk) : d == 128 ? blocks_upto(t128, walk) : alibi || window > 0 ? blocks_upto(m64, walk)
-                                                                                                  : blocks_upto(t64, walk)))
-    return 1;
+  const int upto = d == 96    ? (win && walk < 65 ? 280 : blocks_upto(t96, walk))
+                   : d == 128 ? blocks_upto(t128, walk)
+                              : alibi || window > 0 ? blocks_upto(m64, walk) : blocks_upto(t64, walk);
+  if (blocks <= upto) return 1;
   return d == 128 && blocks <= blocks_upto(w128, walk) ? 2 : 0;
 }
 

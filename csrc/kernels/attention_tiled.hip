@@ -1528,18 +1528,23 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
   // D = 256 under a causal mask, by the blocks of 256 rows of all heads, those of 128 and the longest walk (keys a row sees). us:
   //   two:  128 rows, 8 waves, their keys in two groups, where a CU has one long walk at most, against 256 rows and one group: 1 x 1024 x
   //         16 heads (64 blocks of 256) 47, 40; 2 x 1500 (192) 75, 62; 1 x 3300 (208) 147, 116; 1 x 4096 (256) 181, 166; 2 x 2048 (256) 101, 104
-  //   four: 128 rows, 4 waves, two workgroups a CU, one of which computes while the other waits and long blocks run beside short ones:
-  //         48 blocks of 128 rows 14.7, 11.5; 300 31.5, 20.0; 256 rows, 520 blocks 43, 34; 2 x 2048 (512) 102, 98; 9 x 640 (720) 74, 52; 2 x
-  //         2900 with a window of 256 73, 62; against two groups 640 rows, 160 blocks 31.4, 29.2, 1000 rows 42.3, 44.4, 1400 rows 52.7, 57.7.
-  //         Blocks of 256 rows stream half as many tiles: 1000 rows, 600 blocks of 128 66, 69; 2048 rows, 896 134, 136, 1040 162, 187, 2 x 2185 with
-  //         ALiBi (576) 109, 115; 256 rows, 2000 125, 124; whole blocks of 256 that an odd count leaves half empty lose at any count: 640 rows, 2165 236, 188
+  //   four: 128 rows, 4 waves, two workgroups a CU, one of which computes while the other waits and long blocks run beside short ones, against
+  //         two groups: 640 rows, 160 blocks 31.4, 29.2, 1000 rows 42.3, 44.4, 1400 rows 52.7, 57.7; against 256 rows and one group, which
+  //         stream half as many tiles but leave half of an odd head's last block empty, time with four over time with eight at 560, 800, 1100,
+  //         1600, 2400, 3200 blocks of 128:
+  //           256 rows  .77 .91 .88 .85 1.11 1.14    512   .86 .97 1.01 1.05 1.08 1.19   1000  .99 .94 1.13 .99 1.15 1.15   1536  1.04 1.20 ..
+  //           384       .79 .75 .96 .83 .76 .76      640   .76 .84 .94 .95 .89 .89       850   .88 1.04 1.10 1.00 .88 .83    1152  1.01 .99 1.08 1.07 1.04 .91
+  //           768       1.09 1.08 1.10 1.05 1.02 1.00    1664  1.06 1.00 1.09 1.09 1.09 .93    2048  1.06 1.06 1.23 ..     2500  .96 1.05 1.12 ..
+  //           windows: 2048 rows, 256 .91 .93 1.00 1.00 .97 .96; 1024, 256 .97 .90 1.02 .96 1.00 1.02, 4800 blocks 1.15 (640, 128 .91); 1500, 700 1.14 1.08 1.06 1.09
+  //           1.07 .99; 4096, 1024, 300 blocks .91, 420 1.13; 300 blocks of any of these .82 to 1.0
   const int n128 = (Sq + 127) / 128;
   const long long heads = (long long)B * H, blocks256 = (Sq + 255) / 256 * heads, blocks128 = n128 * heads;
   const int walk = window > 0 ? min(Sk, window) : Sk;
   const bool c256 = d == 256 && causal && aligned && (g_attn_variant & 1);
   const bool two = c256 && Sq > 256 && blocks256 <= (walk >= 3000 ? 256 : walk >= 1400 ? 240 : walk >= 900 ? 128 : 0);
-  const bool four = c256 && !two && (walk < Sk || (n128 % 2 && n128 <= 5) || (Sq % 128 == 0 && Sq % 256) ||
-                                     blocks128 <= (walk <= 256 ? 2000 : walk >= 2000 && !alibi ? 768 : 512));
+  const int upto = n128 <= 2 ? 2000 : n128 <= 4 ? 1100 : n128 == 7 ? 700 : n128 >= 20 ? 640 : 512;
+  const bool four = c256 && !two && (walk < Sk ? blocks128 <= (walk > 384 ? 400 : n128 % 8 ? 1 << 30 : 4000)
+                                               : blocks128 <= upto || (n128 % 2 && (n128 <= 5 || blocks128 > (n128 <= 7 ? 1400 : 2800))));
   if (four) {
     if (alibi) hipLaunchKernelGGL((attn_fwd_w8_kernel<256, true, 4, 2, 2>), grid, dim3(256), 0, stream, p);
     else if (general)
@@ -1547,7 +1552,7 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
     else hipLaunchKernelGGL((attn_fwd_w8_kernel<256, true, 4, 2>), grid, dim3(256), 0, stream, p);
     return hipGetLastError() != hipSuccess ? 3 : -1;
   }
-  if (general || two) {
+  if (general || two || (c256 && Sq % 256)) {  // (odd full tiles: 256 rows of the general form, 640 rows, 2165 blocks of 128 236 -> 188)
     if (!aligned) return 1;
     bool here = false;
     general_form(d, causal, alibi, [&](auto D_, auto C_, auto G_) {
