@@ -1513,7 +1513,11 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
   const bool aligned = rows16(q, q_sb, q_st, q_sh) && rows16(k, k_sb, k_st, k_sh) && rows16(v, v_sb, v_st, v_sh) &&
                        rows16(o, o_sb, o_st, o_sh);
   const bool general = alibi || kv_len || window || cu || Sq % 128 || Sk % 32;  // (these forms take the row sums as everywhere else)
-  if (causal && aligned && (general || (rowsum_col < 0 && max_col < 0))) {
+  // 64 wide, full tiles of many blocks: the plain form, whose masks are simpler, though its overflowed rows take a launch of their own (us, split,
+  // plain: 128 rows, 960 blocks 19.3, 18.8, 1920 31.7, 30.2, 3840 56.4, 52.8; 384, 1920 38.2, 35.9; 1024, 1920 59.7, 57.6; 480 blocks 13.9, 13.6, 22.5,
+  // 22.7; on the host a launch is some 3). 96 and 128 wide gain and lose 5 %.
+  const bool plain = d == 64 && !general && (long long)(Sq / 128) * B * H >= 1900;
+  if (causal && aligned && !plain && (general || (rowsum_col < 0 && max_col < 0))) {
     const int rc = attn_fwd_split(p, d, stream);
     if (rc != 1) return rc ? rc : -1;
   }
@@ -1647,7 +1651,10 @@ KCA_API int kca_attn_bwd_tiled(const void* q, const void* k, const void* v, cons
   const bool aligned = rows16(q, q_sb, q_st, q_sh) && rows16(k, k_sb, k_st, k_sh) && rows16(v, v_sb, v_st, v_sh) &&
                        rows16(o, o_sb, o_st, o_sh) && rows16(dout, do_sb, do_st, do_sh) && rows16(dq, dq_sb, dq_st, dq_sh) &&
                        rows16(dk, dk_sb, dk_st, dk_sh) && rows16(dv, dv_sb, dv_st, dv_sh);
-  if (aligned) {
+  // 64 wide, full tiles: the plain forms from 300 blocks on (us, split, plain: 128 rows, 120 blocks 14.0, 14.3, 240 17.6, 15.9, 480 26.4, 24.5, 1920 81.9, 75.3;
+  // 384, 240 25.9, 25.8, 960 60.8, 57.5; 1024, 240 46.0, 51.7, 480 60.1, 57.5, 1920 171.7, 164.2; 96 wide lose up to 12 %, 128 wide gain and lose 4 %)
+  const bool plain = d == 64 && !(alibi || kv_len || window || Sq % 128 || Sk % 128) && (long long)(Sq / 128) * B * H >= 300;
+  if (aligned && !plain) {
     (void)hipGetLastError();
     const int rc = d == 256 ? attn_bwd_pair(p, d, causal, stream) : causal ? attn_bwd_split(p, d, stream) : 1;
     if (rc != 1) return rc;

@@ -19,6 +19,13 @@ def test_one_group(D, S):
     _check(B, S, S, H, H, D, True)
 
 
+@pytest.mark.parametrize("Sq,Sk", [(128, 128), (384, 384), (256, 512)])
+def test_full_tiles_of_many_blocks(Sq, Sk):
+    """64-wide heads: the plain forms, forward from 1900 blocks on, backward from 300."""
+    _check(10, Sq, Sk, 20, 10, 64, True)
+    _check(20, Sq, Sk, 96 if Sq == 128 else 48, 48, 64, True)
+
+
 @pytest.mark.parametrize("D", [64, 96, 128, 256])
 def test_one_group_masks(D):
     B, H = MANY
