@@ -31,6 +31,7 @@ import os
 
 import numpy as np
 import torch
+from torch.nn.modules import module as _nn
 
 from .. import ops
 from ..ops import decode as dops
@@ -55,6 +56,15 @@ def _next_pow2(n: int, lo: int = 1) -> int:
     while p < n:
         p *= 2
     return p
+
+
+def _only_forward(cls, *mods) -> bool:
+    """Whether calling these modules is ``cls.forward`` and nothing else: no hooks, of their own or of all modules, no ``forward``
+    of their own, not compiled."""
+    if _nn._global_forward_hooks or _nn._global_forward_pre_hooks:
+        return False
+    return all(type(m) is cls and "forward" not in m.__dict__ and not (m._forward_hooks or m._forward_pre_hooks)
+               and m._compiled_call_impl is None for m in mods)
 
 
 class KVCacheFull(RuntimeError):
@@ -918,7 +928,7 @@ class ModelRunner(StepRunner):
                 x2, h = blk.ln_2(h, residual=(a,))
                 u = few_rows_gelu(x2, *plain[2], mlp.approx) if plain else None
                 pending = (mlp(x2) if u is None else mlp.fc_out(u),)
-        if type(m.ln_f) is LayerNorm and not (m.ln_f._forward_hooks or m.ln_f._forward_pre_hooks):
+        if _only_forward(LayerNorm, m.ln_f):
             y = layer_norm_rows(h[0], m.ln_f.weight, m.ln_f.bias, m.ln_f.eps, tuple(p_[0] for p_ in pending), last)[None]
         else:
             y, _ = m.ln_f(h[:, last], residual=tuple(p_[:, last] for p_ in pending))
@@ -928,12 +938,11 @@ class ModelRunner(StepRunner):
     def _plain_products(blk):
         """(weight, bias) of a block's QKV, out, fc_in and fc_out layers where these are plain linear layers without hooks, so
         that they may be taken apart and put together; else None."""
-        mlp = blk._modules["mlp"]
-        if type(mlp) is not MLP or mlp._forward_hooks or mlp._forward_pre_hooks:
+        mlp, at = blk._modules.get("mlp"), blk._modules.get("attn")
+        if at is None or not _only_forward(MLP, mlp):
             return None
-        a, b = blk._modules["attn"]._modules, mlp._modules
-        mods = (a["qkv"], a["out"], b["fc_in"], b["fc_out"])
-        if any(type(x) is not TLinear or x._forward_hooks or x._forward_pre_hooks for x in mods):
+        mods = (at._modules.get("qkv"), at._modules.get("out"), mlp.fc_in, mlp.fc_out)
+        if not _only_forward(TLinear, *mods):
             return None
         return tuple((x.weight, x.bias) for x in mods)
 

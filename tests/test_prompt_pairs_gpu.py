@@ -111,6 +111,36 @@ def test_short_prompts_of_every_layer_kind(monkeypatch, dtype, name, kw):
     assert (out[0] - out[1]).norm() <= (2e-2 if dtype is torch.bfloat16 else 3e-3) * out[1].norm()
 
 
+@pytest.mark.parametrize("how", ["global hook", "global pre-hook", "own forward", "own hook"])
+@pytest.mark.parametrize("parallel", [True, False])
+def test_hooks_see_short_prompts(how, parallel):
+    """Whatever a caller has put around a layer's call runs for a short prompt as for a long one."""
+    cfg = dict(PRESETS_HF["gpt-j-6b"], n_embd=512, n_head=2, rotary_dim=64) if parallel else dict(PRESETS_HF["gpt2"], n_embd=512, n_head=8)
+    m = build_model(LMConfig.from_hf(dict(cfg, n_layer=2, vocab_size=1024)), device="cuda", dtype=torch.bfloat16, seed=3).requires_grad_(False)
+    r, seen = R.ModelRunner(m, max_slots=1, max_len=256), []
+    names = {x: n for n, x in m.named_modules()}
+    inner = [x for x, n in names.items() if n.endswith(("qkv", "out", "mlp", "fc_in", "fc_out", "ln_f"))]
+    if how.startswith("global"):
+        reg = torch.nn.modules.module.register_module_forward_pre_hook if "pre" in how else torch.nn.modules.module.register_module_forward_hook
+        handles = [reg(lambda x, *a: seen.append(names[x]) if x in inner else None)]
+    elif how == "own hook":
+        handles = [x.register_forward_hook(lambda x, *a: seen.append(names[x])) for x in inner]
+    else:
+        handles = []
+        for x in inner:
+            x.forward = lambda *a, x=x, f=x.forward, **k: seen.append(names[x]) or f(*a, **k)
+    try:
+        calls = []
+        for n in (30, 200):
+            seen.clear()
+            r.prefill(torch.arange(n)[None], [0], [n])
+            calls.append(sorted(seen))
+    finally:
+        for h in handles:
+            h.remove()
+    assert calls[0] == calls[1] == sorted(names[x] for x in inner)
+
+
 def test_block_tables_go_up_in_order():
     """Edits while earlier uploads still wait for the GPU: each launch reads the table of its own time."""
     c = R.KVCache(1, 8, 1, 512, 64, "cuda", page_size=16)
