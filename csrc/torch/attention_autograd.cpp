@@ -145,4 +145,9 @@ PyModuleDef module{PyModuleDef_HEAD_INIT, "kca_torch", nullptr, -1, methods, nul
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_kca_torch() { return PyModule_Create(&module); }
+// `torch`: the version that it was compiled against, whose class layouts are in it (ops/_lib.py looks before it uses the module)
+PyMODINIT_FUNC PyInit_kca_torch() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch", KCA_TORCH) < 0) Py_CLEAR(m);
+  return m;
+}

@@ -187,8 +187,10 @@ def torch_ext():
                     spec = importlib.util.spec_from_file_location("kca_torch", path)
                     try:
                         m = importlib.util.module_from_spec(spec)
+                        if m.torch != torch.__version__:
+                            raise ImportError(f"built for torch {m.torch}, this is {torch.__version__}")
                         m.init(*(ctypes.cast(f, P).value for f in (lib.kca_attn_fwd, lib.kca_attn_bwd)))
-                    except ImportError as e:  # pragma: no cover - another torch than it was built for
+                    except (ImportError, AttributeError) as e:  # another torch than it was built for
                         warnings.warn(f"{path}: {e}")
                         m = None
                 _torch_ext.append(m)
