@@ -980,12 +980,13 @@ __device__ __forceinline__ void expert_dma_tile(const ExpertArgs& p, bf16_t* gl,
     }
   }
   const unsigned to = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) char*)gl + wv * 1024);
-  // (in asm: hipcc would let every read of LDS wait for all requests. Nothing is returned to a register, and nothing else here uses m0)
+  // (in asm: hipcc would let every read of LDS wait for all requests. Nothing is returned to a register)
   auto request = [&](int t, int slot, int i) {
     const int k = __builtin_amdgcn_readfirstlane(min(t, nk - 1) * DK * 2);  // past the end: the last one, which nobody reads
     const unsigned at = __builtin_amdgcn_readfirstlane(to + slot * (STG * 2) + i * 4096);
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(at), "v"(from[i]),
-                 "s"(i < WP / 2 ? rw : rx), "s"(k));
+                 "s"(i < WP / 2 ? rw : rx), "s"(k)
+                 : "m0");
   };
   f32x16 acc[AI][BJ];
 #pragma unroll

@@ -1,6 +1,7 @@
 """LDS of the attention kernels whose wave groups stage tiles for each other: between two barriers no wave may read what another
 writes. The kernels' own source runs on the host, thread after thread, with a callback at every load and store (lds_trace/)."""
 import os
+import re
 import subprocess
 
 import pytest
@@ -58,3 +59,12 @@ def test_every_block_is_taken_once(tmp_path):
     subprocess.run([CLANG, "-x", "c++", "-std=c++17", "-w", "-mavx512f", "-O1", "-I" + src, os.path.join(src, "order.cpp"), "-o", exe], check=True)
     r = subprocess.run([exe], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
+
+
+def test_asm_names_the_registers_that_it_writes():
+    """m0 is written for requests into LDS: the compiler, which uses it too, has to know."""
+    for d in ("kernels", "comm"):
+        for f in os.listdir(os.path.join(ROOT, "csrc", d)):
+            with open(os.path.join(ROOT, "csrc", d, f)) as src:
+                for stmt in re.findall(r"\basm volatile\((?:[^;]|\n)*?\);", src.read()):
+                    assert "s_mov_b32 m0" not in stmt or re.search(r':\s*"m0"', stmt), (f, stmt)
