@@ -902,6 +902,7 @@ __global__ void __launch_bounds__(NW * 64, NW == 4 && D == 256 ? 2 : 1) attn_fwd
   };
   float ltot;
   if (AGAIN && tid == 0) again = 0;
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the walk's barriers do not wait for LDS: it lies there before a wave raises it)
   for (;; ++pass) {
     walk([&](int buf, int tile) {
       sm_part(buf, CM, tile);

@@ -68,3 +68,11 @@ def test_asm_names_the_registers_that_it_writes():
             with open(os.path.join(ROOT, "csrc", d, f)) as src:
                 for stmt in re.findall(r"\basm volatile\((?:[^;]|\n)*?\);", src.read()):
                     assert "s_mov_b32 m0" not in stmt or re.search(r':\s*"m0"', stmt), (f, stmt)
+
+
+def test_a_flag_is_lowered_before_the_first_bare_barrier():
+    """A bare barrier waits for no LDS access: what one wave has written before it and others write after it needs a wait."""
+    with open(os.path.join(ROOT, "csrc", "kernels", "attention_tiled.hip")) as f:
+        src = f.read()
+    lowered = re.findall(r"again = 0;\n(.*)\n", src)
+    assert lowered and all('"s_waitcnt lgkmcnt(0)"' in line for line in lowered)
