@@ -1,5 +1,5 @@
-// What the matrix-core attention kernels of attention_tiled.hip and attention_split.hip share: their parameters, the span of
-// key tiles that a workgroup walks, fragment reads of a tile image, and the store of a wave's accumulator.
+// What the matrix-core attention kernels of attention_tiled.hip, attention_split.hip and attention_pair.hip share: their parameters, the
+// order of the blocks, the span of key tiles that a workgroup walks, fragment reads of a tile image, and the store of a wave's accumulator.
 #pragma once
 #include "attn_tile.h"
 
@@ -42,14 +42,14 @@ __device__ __forceinline__ void own_sequence(FastFwdParams& p, int b) {
 // head, all heads at once, so: 559 tokens, 640 heads of 256 229, 275, 207 and 827, 814, 728; 300, 1280 of 256 236, 257, 185 and 740,
 // 736, 644; 850, 1280 of 96 386, 464, 382 and 1053, 1178, 1025; 300, 640 of 128 57, 63, 57 and 174, 170, 161; 559, 640 of 64 71, 77, 70 and
 // 214, 200, 188; 16 x 2048 x 16 of 256 634, 642, 607 and 2502, 2471, 2189. Where a head has 2, 4 or 8 blocks a CU meets one length
-// again and again: 256 tokens, 1024 heads of 256 418, 463 in turn, 450 tokens, 1280 of 64 110, 117. 96-wide heads share their 128-byte
-// lines with their neighbours, which then lie on one XCD: short ones are taken so from the first block on (128 tokens, 2048 heads 51, 47 and
-// 147, 138; 300, 640 heads 59, 54; 2048, 128 heads 147, 156).
+// again and again: 256 tokens, 1024 heads of 256 418, 463 in turn, 450 tokens, 1280 of 64 110, 117. Heads of 96 and 160 share 128-byte
+// lines with their neighbours, which then lie on one XCD: short ones are taken so from the first block on (96: 128 tokens, 2048 heads 51,
+// 47 and 147, 138; 300, 640 heads 59, 54; 2048, 128 heads 147, 156).
 // (blocks of 128 rows: of a head, of all)
 template <int D>
 __device__ __forceinline__ bool heads_in_turn(int blocks, int total) {
   if (total > 8192 && blocks > 1) return true;
-  if (D == 96) return blocks <= 10 || total > 3072;
+  if (D % 64) return blocks <= 10 || total > 3072;
   return blocks > 2 && (blocks % 4 || blocks > 8) && total > (blocks < 8 ? 1536 : 3072);
 }
 struct BlockOf { int block, head; };
