@@ -1,15 +1,17 @@
-// Flash attention for calls whose 128-row blocks leave the chip idle: the keys (dK/dV: the queries) of a block are split over
-// the wave groups of its workgroup.
+// Flash attention, causal calls of 64, 96 and 128 wide heads with 16-byte rows: blocks of 128 rows and four waves, or, where those leave the
+// chip idle, of 64 rows whose keys (dK/dV: queries) are split over two groups of waves. (Full tiles of 64-wide heads in many blocks stay with
+// attention_tiled.hip's plain forms: kca_attn_fwd_tiled, kca_attn_bwd_tiled.)
 //
-// What bounds these calls. attn_fwd_tiled_kernel gives a workgroup 128 rows and a wave 32 of them; a call of few heads and
-// rows then has less than one workgroup a CU, so a SIMD runs one wave whose products, softmax, LDS reads and barriers follow
+// What bounds these calls. A block of 128 rows gives a wave 32 of them; a call of few heads and rows then has less than one
+// workgroup a CU, so a SIMD runs one wave whose products, softmax, LDS reads and barriers follow
 // each other, and under a causal mask the call waits for the block that sees all keys: 2048 tokens x 14 heads of 128 are 224
 // workgroups on 256 CUs, 52 us for the 64 tiles of the longest one. Here a workgroup has RW * 32 rows and KG groups of RW
-// waves; group g walks tiles g, g + KG, ... with LDS buffers of its own and the partial sums meet in LDS at the end. Blocks
-// are half as tall, so there are twice as many, each 1 / KG as long, and a SIMD has two waves to run.
+// waves; group g walks tiles g, g + KG, ... with LDS buffers of its own and the partial sums meet in LDS at the end. Two groups'
+// blocks are half as tall, so there are twice as many, each half as long, and a SIMD has two waves to run. Many blocks gain from
+// one group too: overflowed rows take no launch of their own, and blocks go longest first.
 //
 // The forms of a mask are attention_tiled.hip's general ones (1: lengths, windows, any sizes; 2: ALiBi) and every call takes
-// one of them. Blocks are taken longest first over all heads (block_of).
+// one of them. The order of the blocks: block_of.
 //
 // Tiles in LDS: two buffers of K and V a group. A step computes S of the group's next tile while it takes the softmax of this
 // one, so K runs a tile ahead of V: K(i + 2) goes where K(i) was and V(i + 1) where V(i - 1) was, which all waves have read
@@ -718,10 +720,11 @@ static bool split_rows(long long blocks, int d, int keys, int window) {
 //              87.0; a window of 256, 288 20.2, 18.2, 336 41.6, -2.6, 480 43.8, +5.8
 //   96 wide:   64 rows, 60 blocks 13.9, -1.3, 1200 50.2, -3.9; 32 rows, 340 15.2, -0.4; a window of 32 or 64, 120 25, -5, 224 28, -2.5, 340 35,
 //              +1, 480 41, +3; 128 rows, 220 23.8, -0.4, 260 30.2, +2.5; 512 rows, 300 47.4, -1.7, 340 48.5, +0.3; 1024 rows, 480 80.5, -0.8
-//   128 wide:  32 rows, 60 blocks 12.7, +0.4; 64 rows, 220 17.5, -0.9, 260 22.1, +3.4; 128 rows, 100 23.0, -1.0 (+0.6), 140 25.0, +3.6 (+0.7);
-//              256 rows, 140 33.7, -1.3 (-0.4), 180 34.3, +1.2 (0); 512 rows, 180 48.9, -2.8 (-2.0), 260 54.6, +4.5 (-3.8), 340 57.1, +8.0
-//              (+2.3); 1024 rows, 256 80.0, -7.4 (-7.1), 304 87.4, +2.4 (-9.3), 480 99.2, +17 (-3.9), 560 108, +28 (+6.7); 1 x 2944 x 20 (460) 246, +29 (-37); a window of 256, 96 40.2, -7.1 (-2.2), 144 43.1,
-//              +2.5 (-2.3), 264 48.3, +7.8 (+3.0)
+//   128 wide:  32 rows, 60 blocks 12.7, +0.4; 64 rows, 220 17.5, -0.9, 260 22.1, +3.4; 128 rows, 100 23.0, -1.0 (+0.6), 140 25.0,
+//              +3.6 (+0.7); 256 rows, 140 33.7, -1.3 (-0.4), 180 34.3, +1.2 (0); 512 rows, 180 48.9, -2.8 (-2.0), 260 54.6, +4.5
+//              (-3.8), 340 57.1, +8.0 (+2.3); 1024 rows, 256 80.0, -7.4 (-7.1), 304 87.4, +2.4 (-9.3), 480 99.2, +17 (-3.9), 560 108,
+//              +28 (+6.7); 1 x 2944 x 20 (460) 246, +29 (-37); a window of 256, 96 40.2, -7.1 (-2.2), 144 43.1, +2.5 (-2.3), 264
+//              48.3, +7.8 (+3.0)
 static int split_keys(long long blocks, int d, int rows, int window, bool alibi) {
   static const Upto t64[] = {{33, 200}, {400, 340}, {512, 480}, {768, 560}, {1536, 680}};  // (the form START; with ALiBi or a window:)
   static const Upto m64[] = {{33, 340}, {512, 480}, {768, 560}, {1536, 768}};

@@ -1514,9 +1514,9 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
   const bool aligned = rows16(q, q_sb, q_st, q_sh) && rows16(k, k_sb, k_st, k_sh) && rows16(v, v_sb, v_st, v_sh) &&
                        rows16(o, o_sb, o_st, o_sh);
   const bool general = alibi || kv_len || window || cu || Sq % 128 || Sk % 32;  // (these forms take the row sums as everywhere else)
-  // 64 wide, full tiles of many blocks: the plain form, whose masks are simpler, though its overflowed rows take a launch of their own (us, split,
-  // plain: 128 rows, 960 blocks 19.3, 18.8, 1920 31.7, 30.2, 3840 56.4, 52.8; 384, 1920 38.2, 35.9; 1024, 1920 59.7, 57.6; 480 blocks 13.9, 13.6, 22.5,
-  // 22.7; on the host a launch is some 3). 96 and 128 wide gain and lose 5 %.
+  // 64 wide, full tiles of many blocks: the plain form, whose masks are simpler, though its overflowed rows take a launch of their own
+  // (us, split, plain: 128 rows, 960 blocks 19.3, 18.8, 1920 31.7, 30.2, 3840 56.4, 52.8; 384, 480 13.9, 13.6, 1920 38.2, 35.9; 1024, 480
+  // 22.5, 22.7, 1920 59.7, 57.6; on the host a launch is some 3). 96 and 128 wide gain and lose 5 %.
   const bool plain = d == 64 && !general && (long long)(Sq / 128) * B * H >= 1900;
   if (causal && aligned && !plain && (general || (rowsum_col < 0 && max_col < 0))) {
     const int rc = attn_fwd_split(p, d, stream);
@@ -1527,8 +1527,9 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
   //   2 x 2048, 14 heads of 128, ALiBi       198 -> 80, 345 -> 303    1 x 1500, 64 heads of 96       177 -> 66, 366 -> 234
   //   4 x 1100, 16 heads of 256              194 -> 77, 685 -> 307    8 x 1000, 12 heads of 64        59 -> 36, 181 -> 145
   //   4 x 2048, 16 heads of 256, lengths     528 -> 203, 1870 -> 815  2 x 2048, 20 of 128, window 256  68 -> 39, 148 -> 137
-  // Full tiles without another mask keep the plain form, whose loops have no edge to test: 4 x 2048 of 256 179 us
-  // against 203 forward and 760 against 815 backward, 8 x 1024 of 64 36 and 137 against 36 and 146.
+  // Full tiles without another mask, where they come here (not causal; 160 wide; 64 wide in many blocks; 256 wide in whole blocks of 256
+  // rows), keep the plain form, whose loops have no edge to test: 4 x 2048 of 256 179 us against 203 forward, 8 x 1024 of 64, not
+  // causal, 36 and 137 with the backward against 36 and 146.
   bool whole = false;  // the kernel leaves no row to the fixup launch
   // D = 256 under a causal mask, by the blocks of 256 rows of all heads, those of 128 and the longest walk (keys a row sees). us:
   //   two:  128 rows, 8 waves, their keys in two groups, where a CU has one long walk at most, against 256 rows and one group: 1 x 1024 x
@@ -1538,10 +1539,11 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
   //         stream half as many tiles but leave half of an odd head's last block empty, time with four over time with eight at 560, 800, 1100,
   //         1600, 2400, 3200 blocks of 128:
   //           256 rows  .77 .91 .88 .85 1.11 1.14    512   .86 .97 1.01 1.05 1.08 1.19   1000  .99 .94 1.13 .99 1.15 1.15   1536  1.04 1.20 ..
-  //           384       .79 .75 .96 .83 .76 .76      640   .76 .84 .94 .95 .89 .89       850   .88 1.04 1.10 1.00 .88 .83    1152  1.01 .99 1.08 1.07 1.04 .91
-  //           768       1.09 1.08 1.10 1.05 1.02 1.00    1664  1.06 1.00 1.09 1.09 1.09 .93    2048  1.06 1.06 1.23 ..     2500  .96 1.05 1.12 ..
-  //           windows: 2048 rows, 256 .91 .93 1.00 1.00 .97 .96; 1024, 256 .97 .90 1.02 .96 1.00 1.02, 4800 blocks 1.15 (640, 128 .91); 1500, 700 1.14 1.08 1.06 1.09
-  //           1.07 .99; 4096, 1024, 300 blocks .91, 420 1.13; 300 blocks of any of these .82 to 1.0
+  //           384       .79 .75 .96 .83 .76 .76      640   .76 .84 .94 .95 .89 .89       850   .88 1.04 1.10 1.00 .88 .83
+  //           768       1.09 1.08 1.10 1.05 1.02 1.00    1152  1.01 .99 1.08 1.07 1.04 .91    1664  1.06 1.00 1.09 1.09 1.09 .93
+  //           2048      1.06 1.06 1.23 ..     2500  .96 1.05 1.12 ..     1000 with ALiBi  1.10 1.06 1.15 ..
+  //         windows: 2048 rows, 256 .91 .93 1.00 1.00 .97 .96; 1024, 256 .97 .90 1.02 .96 1.00 1.02, 4800 blocks 1.15 (640, 128 .91); 1500,
+  //         700 1.14 1.08 1.06 1.09 1.07 .99; 4096, 1024, 300 blocks .91, 420 1.13; 300 blocks of any of these .82 to 1.0
   const int n128 = (Sq + 127) / 128;
   const long long heads = (long long)B * H, blocks256 = (Sq + 255) / 256 * heads, blocks128 = n128 * heads;
   const int walk = window > 0 ? min(Sk, window) : Sk;
@@ -1557,7 +1559,7 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
     else hipLaunchKernelGGL((attn_fwd_w8_kernel<256, true, 4, 2>), grid, dim3(256), 0, stream, p);
     return hipGetLastError() != hipSuccess ? 3 : -1;
   }
-  if (general || two || (c256 && Sq % 256)) {  // (odd full tiles: 256 rows of the general form, 640 rows, 2165 blocks of 128 236 -> 188)
+  if (general || two || (c256 && Sq % 256)) {  // (an odd half block of full tiles: 1920 rows, 1600 blocks of 128 303 plain, 244 in 256 rows)
     if (!aligned) return 1;
     bool here = false;
     general_form(d, causal, alibi, [&](auto D_, auto C_, auto G_) {
@@ -1652,8 +1654,9 @@ KCA_API int kca_attn_bwd_tiled(const void* q, const void* k, const void* v, cons
   const bool aligned = rows16(q, q_sb, q_st, q_sh) && rows16(k, k_sb, k_st, k_sh) && rows16(v, v_sb, v_st, v_sh) &&
                        rows16(o, o_sb, o_st, o_sh) && rows16(dout, do_sb, do_st, do_sh) && rows16(dq, dq_sb, dq_st, dq_sh) &&
                        rows16(dk, dk_sb, dk_st, dk_sh) && rows16(dv, dv_sb, dv_st, dv_sh);
-  // 64 wide, full tiles: the plain forms from 300 blocks on (us, split, plain: 128 rows, 120 blocks 14.0, 14.3, 240 17.6, 15.9, 480 26.4, 24.5, 1920 81.9, 75.3;
-  // 384, 240 25.9, 25.8, 960 60.8, 57.5; 1024, 240 46.0, 51.7, 480 60.1, 57.5, 1920 171.7, 164.2; 96 wide lose up to 12 %, 128 wide gain and lose 4 %)
+  // 64 wide, full tiles: the plain forms from 300 blocks on (us, split, plain: 128 rows, 120 blocks 14.0, 14.3, 240 17.6, 15.9, 480 26.4,
+  // 24.5, 1920 81.9, 75.3; 384, 240 25.9, 25.8, 960 60.8, 57.5; 1024, 240 46.0, 51.7, 480 60.1, 57.5, 1920 171.7, 164.2; 96 wide lose up
+  // to 12 %, 128 wide gain and lose 4 %)
   const bool plain = d == 64 && !(alibi || kv_len || window || Sq % 128 || Sk % 128) && (long long)(Sq / 128) * B * H >= 300;
   if (aligned && !plain) {
     (void)hipGetLastError();
