@@ -74,7 +74,8 @@ def test_eight_waves_compute_rows_again(kind):
     q, k, v = (torch.randn(B, S, H, D, device="cuda", generator=g) * 0.3 for _ in range(3))
     k[1, 700, 2] = q[1, 950, 2] * 40.0
     q, k, v = (t.bfloat16() for t in (q, k, v))
-    kw = {"lens": {"lens": torch.tensor([S, S - 1, 300, S, S], device="cuda", dtype=torch.int32)}, "alibi": {"slopes": torch.full((H,), 0.25, device="cuda")},
+    kw = {"lens": {"lens": torch.tensor([S, S - 1, 300, S, S], device="cuda", dtype=torch.int32)},
+          "alibi": {"slopes": torch.full((H,), 0.25, device="cuda")},
           "window": {"window": 600}}.get(kind, {})
     o, lse = A._fwd(q, k, v, True, D ** -0.5, kw.get("lens"), kw.get("slopes"), window=kw.get("window", 0))
     _compare(q, k, v, o, lse, slice(0, 3), slice(0, 4), **kw)
@@ -117,7 +118,8 @@ def test_two_groups_compute_rows_again(kind):
     q, k, v = (torch.randn(B, S, H, D, device="cuda", generator=g) * 0.3 for _ in range(3))
     k[0, 700, 1] = q[0, 1050, 1] * 40.0
     q, k, v = (t.bfloat16() for t in (q, k, v))
-    kw = {"lens": {"lens": torch.tensor([S - 1, 300], device="cuda", dtype=torch.int32)}, "alibi": {"slopes": torch.full((H,), 0.25, device="cuda")},
+    kw = {"lens": {"lens": torch.tensor([S - 1, 300], device="cuda", dtype=torch.int32)},
+          "alibi": {"slopes": torch.full((H,), 0.25, device="cuda")},
           "window": {"window": 1000}}.get(kind, {})
     o, lse = A._fwd(q, k, v, True, D ** -0.5, kw.get("lens"), kw.get("slopes"), window=kw.get("window", 0))
     _compare(q, k, v, o, lse, **kw)
