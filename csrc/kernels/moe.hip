@@ -230,20 +230,30 @@ struct GroupArgs {
   int *perm, *inv, *tiles, *ntiles;
 };
 
-// Whether the last tile of an expert with `c` rows stands after all experts' others (row limits of 128 and more): it is at most half
+// Whether the last tile of an expert with `c` rows stands after all experts' others (row limits of 128 and 192): it is at most half
 // full, and what its weights cost to read again, away from the expert's other tiles, is less than the CUs that it fills: two full
-// tiles before it, or none, or one of 256 rows, which the matrix cores bound, and hardly any rows. Both products, us (width, experts,
-// top, inner size), beside its expert's and last: 2000 tokens, 4096, 16, 2, 4096 652, 608; 4096 of them 934, 910; 3000, 2048, 32, 4,
-// 1024 237, 215; 300, 4096, 16, 3, 2048 218, 199. 1200 of these (one of 128 rows and about 52) 277, 294 with all such tiles last,
-// 282 with those of up to 16 rows.
+// tiles before it, or none, or one of 192 rows and hardly any rows. Both products, us (width, experts, top, inner size), beside its
+// expert's and last: 3000 tokens, 2048, 32, 4, 1024 237, 215; 300, 4096, 16, 3, 2048 218, 199.
 __device__ __forceinline__ bool late_tile(int c, int mt) {
   const int r = c % mt, full = c / mt;
-  return mt >= 128 && r && 2 * r <= mt && (full != 1 || (mt > 128 && 8 * r <= mt));
+  return mt >= 128 && mt < 256 && r && 2 * r <= mt && (full != 1 || (mt > 128 && 8 * r <= mt));
+}
+
+// Tiles of up to 256 rows: an expert's rows in units of 64 (a product's steps), as evenly over its tiles as they go: `more` tiles of
+// per + 1 units, then the others. (Full tiles and a short last one, whose weights then came from memory once more: sublayer of 4096
+// tokens, 16 experts of 3 x 4096 x 4096, top 2 893 us, evenly 850.) Experts stand by their largest tile: expert_turns_kernel.
+struct Cut {
+  int tiles, per, more;
+};
+__device__ __forceinline__ Cut cut(int c) {
+  const int u = (c + 63) / 64, nt = (u + 3) / 4;
+  return nt ? Cut{nt, u / nt, u % nt} : Cut{0, 0, 0};
 }
 
 // n assignments -> perm (sorted position -> assignment), inv (assignment -> sorted position), tiles
 // [ntiles][5] (expert, first sorted position, rows <= mt, first tile and tile count of the expert) and
-// their count. Late tiles stand after all others, each by itself, so that a product takes them last (expert_gemm_kernel). One workgroup
+// their count. Late tiles (and those of up to 128 rows where the limit is 256) stand after all others, each by itself, so that a
+// product takes them last (expert_gemm_kernel). One workgroup
 // of NT threads;
 // sh: 4 E + 3 ints.
 template <int NT>
@@ -267,33 +277,53 @@ __device__ __forceinline__ void group_rows(const GroupArgs& p, int* sh) {
   });
   __syncthreads();
   if (tid < 64) {  // exclusive sums over the experts, 64 at a time
-    int co = 0, to = 0, so = 0;
+    int co = 0, so = 0;
+    unsigned to = 0, to2 = 0;  // mt 256: four sums in 16 bits each (tiles are fewer than 32768), of experts whose largest tile is 4 .. 1 units
     for (int e0 = 0; e0 < E; e0 += 64) {
-      const int e = e0 + tid, c = e < E ? cnt[e] : 0, small = late_tile(c, mt), t = (c + mt - 1) / mt - small;
-      int cs = c, ts = t;
+      const int e = e0 + tid, c = e < E ? cnt[e] : 0, small = late_tile(c, mt);
+      const Cut k = cut(c);
+      const int b = 4 - k.per - (k.more > 0);
+      const unsigned t = mt == 256 ? (b < 2 ? k.tiles << 16 * b : 0) : (c + mt - 1) / mt - small, t2 = b < 2 ? 0 : k.tiles << 16 * (b & 1);
+      int cs = c;
+      unsigned ts = t, ts2 = t2;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
-        const int a = __shfl_up(cs, o, 64), b = __shfl_up(ts, o, 64);
-        if (tid >= o) cs += a, ts += b;
+        const int a = __shfl_up(cs, o, 64);
+        const unsigned b1 = __shfl_up(ts, o, 64), b2 = __shfl_up(ts2, o, 64);
+        if (tid >= o) cs += a, ts += b1, ts2 += b2;
       }
       const unsigned long long m = __ballot(small);
-      if (e < E) off[e] = co + cs - c, toff[e] = to + ts - t, soff[e] = so + __popcll(m & ((1ull << tid) - 1));
+      if (e < E) {
+        const unsigned u = to + ts - t, u2 = to2 + ts2 - t2;
+        off[e] = co + cs - c;
+        toff[e] = mt == 256 ? (b < 2 ? u : u2) >> 16 * (b & 1) & 0xffff : u;
+        soff[e] = mt == 256 ? b : so + __popcll(m & ((1ull << tid) - 1));
+      }
       co += __shfl(cs, 63, 64);
       to += __shfl(ts, 63, 64);
+      to2 += __shfl(ts2, 63, 64);
       so += __popcll(m);
+    }
+    if (mt == 256) {  // largest tiles first
+      const unsigned n0 = to & 0xffff, n1 = n0 + (to >> 16), n2 = n1 + (to2 & 0xffff);
+      for (int e = tid; e < E; e += 64) toff[e] += soff[e] == 0 ? 0 : soff[e] == 1 ? n0 : soff[e] == 2 ? n1 : n2;
+      to = n2 + (to2 >> 16);
     }
     if (tid == 0) off[E] = co, toff[E] = to, *p.ntiles = to + so;
   }
   __syncthreads();
   for (int e = tid; e < E; e += NT) {
     const int c = cnt[e], nt = (c + mt - 1) / mt, small = late_tile(c, mt);
+    const Cut k = cut(c);
     for (int j = 0; j < nt; ++j) {
       const bool last = small && j == nt - 1;  // (it stands alone)
       const int at = last ? toff[E] + soff[e] : toff[e] + j;
+      const int from = mt == 256 ? 64 * (j * k.per + min(j, k.more)) : j * mt;
+      const int to = min(c, mt == 256 ? from + 64 * (k.per + (j < k.more)) : from + mt);
       int* t = p.tiles + at * 5;
       t[0] = e;
-      t[1] = off[e] + j * mt;
-      t[2] = min(mt, c - j * mt);
+      t[1] = off[e] + from;
+      t[2] = to - from;
       t[3] = last ? at : toff[e];
       t[4] = last ? 1 : nt - small;
     }
@@ -775,7 +805,7 @@ __global__ void __launch_bounds__(256, 2) expert_stream_kernel(ExpertArgs p) {
 // Narrow blocks (128 weight rows, tiles to 192 rows, two workgroups a CU) fill the chip with a quarter of the work.
 // Both products of 4096 tokens, 16 experts of 3 x 4096 x 4096, top 2: 1143 -> 904 us (913 TFLOP/s without padding);
 // 16 experts of 3 x 4096 x 2048, top 3: 764 -> 541; 1000 tokens, 32 experts of 3 x 2048 x 1024, top 4: 148 -> 116.
-// Full tiles go another way where K allows it: expert_dma_tile.
+// Wide blocks where K % 64 == 0 go another way: expert_turns_tile.
 constexpr int GBK = 64, GN = 256, GM = 256, GEMM_LDS = 2 * (GN + GM) * GBK * 2, WIDE_LDS = GEMM_LDS / 4 * 5;
 
 // The results of a wave's AI runs of 32 weight rows and BJ of 32 rows
@@ -940,136 +970,160 @@ __device__ __forceinline__ void expert_gemm_tile(const ExpertArgs& p, bf16_t* gl
   expert_store<UP, WN, AI, WM, BJ>(p, acc, lo, nr, n0);
 }
 
-// Full tiles (more than 192 rows, K % 64 == 0), staged by the memory system: 16 bytes a lane straight into LDS, in 5 stages of 32. No
-// register holds a piece on its way and no instruction stores one, so that beside the products a wave only reads the next
-// sub-step's fragments and requests stages (pinned behind pairs of products). The barrier stands before a stage's last sub-step, as above:
-// all waves then have the stage in registers. Same sums in the same order as above.
-// A request of 1 KB takes a CU's address path 16 cycles, half of the products' time: bunched behind the barrier they held the products up.
-// What bounds it now: the products 59 % of a block's time, waits for loads and barriers a quarter.
-// A whole sublayer, us, staged through registers and this: 4096 tokens, 16 experts of 3 x 4096 x 4096, top 2 966 -> 928, with another
-// routing 973 -> 884; 3000 tokens, 32 experts of 3 x 2048 x 1024, top 4 257 -> 248; 3500 of 24 of 3 x 2048 x 768, top 5 232 -> 228. The first
-// in four stages, a request a pair behind the barrier 1055, in five with two a pair 1039 (981 through registers). Requests over
-// four sub-steps: the same. Tiles of 129 to 192 rows in blocks of 4 waves x all rows lose (1200 tokens as the first 383 -> 391) or gain
-// 2 % (1450 tokens); of up to 128 the same.
-// A row's four pieces lie turned by (row / 4) % 4, so 16 rows x one piece cover all 64 banks.
-template <bool UP>
-__device__ __forceinline__ void expert_dma_tile(const ExpertArgs& p, bf16_t* gl, int ex, int lo, int nr, int n0) {
-  constexpr int WN = 2, AI = 4, WM = 2, BJ = 4;                  // as above
-  constexpr int WP = WN * AI, RP = WM * BJ, NP = (WP + RP) / 2;  // runs of 32 rows: weights, activations; 1 KB pieces a wave a stage
-  constexpr int DK = 32, NS = 5, STG = (WP + RP) * 32 * DK;      // one stage (elements)
-  constexpr int NM = AI * BJ, NF = AI + BJ, NC = NM / 2;
-  static_assert(NF == NC && NS * STG * 2 <= WIDE_LDS, "two fragments a pair of products, in the first half of them");
-  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), wn = wv % WN, wm = wv / WN;
-  const int K = p.K, N = p.N, nk = K / DK;
+// Wide blocks where K % 64 == 0: 8 waves in two groups of four, one of each on a SIMD. While one group multiplies, the other reads its
+// next fragments from LDS and requests stages, and a barrier later they change places, so that a SIMD's matrix core always has a wave that
+// does nothing else. (4 waves of 128 x 128, a wave alone on its SIMD, whose products waited for its loads, barriers and issue: 59 % of
+// a block's time multiplied. Here 92 % of the loop, 80 % of a block; 142 thousand cycles for 64 stages of 256 rows, 131 the products alone.)
+// A group holds half of the block's weight rows (128: two halves of 64; up: gate rows and their up rows), a wave of it a quarter of the
+// rows, in B runs of 16: 64 B rows a tile. A turn is one half of the weight rows over a stage of 64 of K: 8 B products of 16x16x32 after 8
+// fragments of weights and, first half, 2 B of activations, which the second half multiplies again.
+// Stages go straight into LDS in whole 128-byte lines (a request: 8 rows, 16-byte pieces swizzled by row pair on the source address, so 16
+// rows x one piece cover all 64 banks). Weights have three places and are requested two stages ahead; activations, hit in the XCD's cache
+// more often, two places, requested as soon as both groups have read the first half. A turn between products must be shorter than one of
+// products: LDS reads and requests alternate, since each kind alone holds a wave up while the other's path is idle (all reads first 147
+// thousand cycles; requests between the products, which then wait for the address path, 208).
+// A whole sublayer, us, this and four waves before: 4096 tokens, 16 experts of 3 x 4096 x 4096, top 2 882 -> 774, with another routing 969 ->
+// 810; 2000 tokens 589 -> 482, 1200 412 -> 386; 4000 tokens, 16 of 3 x 4096 x 2048, top 3 574 -> 481.
+// What bounds it: rounds of blocks that end half empty (15 % at 4096 tokens), a block's start and results (22 thousand cycles). Blocks
+// that stay and request the next tile before their results gained nothing over the scheduler's choice of the next block.
+template <bool UP, int B>
+__device__ __forceinline__ void expert_turns_tile(const ExpertArgs& p, char* sl, int ex, int lo, int nr, int n0) {
+  constexpr int HALF = 128 * GBK * 2, BST = 64 * B * GBK * 2, BAT = 6 * HALF;  // bytes: 128 weight rows, the activations of a stage, their place
+  static_assert(BAT + 2 * BST <= WIDE_LDS, "three stages of weights and two of activations");
+  const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), wa = wv >> 2, wb = wv & 3;  // wa: the group
+  const int K = p.K, N = p.N, nk = K / GBK;
   const u32x4 rw = uniform_words(reinterpret_cast<const bf16_t*>(p.w) + (long long)ex * (UP ? 2 * N : N) * K);
   const u32x4 rx = uniform_words(reinterpret_cast<const bf16_t*>(p.x) + (UP ? 0ll : (long long)lo * K));
-  // piece i of wave wv: rows (4 i + wv) 16 + lane / 4
-  const unsigned ch = ((lane & 3) ^ ((lane >> 4) & 3)) * 16, rb = (unsigned)K * 2;
-  unsigned from[NP];
+  unsigned from_w[4], from_x[B];
 #pragma unroll
-  for (int i = 0; i < NP; ++i) {
-    const int r = (4 * i + wv) * 16 + (lane >> 2);
-    if (i < WP / 2) {
-      const int run = r / 32, wrun = run % AI, base = run / AI * (AI / 2) * 32;  // (as above)
-      const int n = UP ? (wrun < AI / 2 ? 0 : N) + min(n0 + base + wrun % (AI / 2) * 32 + (r & 31), N - 1) : min(n0 + r, N - 1);
-      from[i] = (unsigned)n * rb + ch;
-    } else {
-      const int xr = min(r - WP * 32, nr - 1);
-      from[i] = (unsigned)(UP ? p.perm[lo + xr] / p.top : xr) * rb + ch;
-    }
+  for (int i = 0; i < 4; ++i) {
+    const int r = (wb * 4 + i) * 8 + (lane >> 3);  // of the half's 128: 64 of either group
+    const int n = UP ? wa * N + min(n0 + r, N - 1) : min(n0 + (r >> 6) * 128 + wa * 64 + (r & 63), N - 1);
+    from_w[i] = ((unsigned)n * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
   }
-  const unsigned to = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) char*)gl + wv * 1024);
+#pragma unroll
+  for (int i = 0; i < B; ++i) {
+    const int r = (wv * B + i) * 8 + (lane >> 3), xr = min(r, nr - 1);
+    from_x[i] = ((unsigned)(UP ? p.perm[lo + xr] / p.top : xr) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
+  }
+  const unsigned base = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) char*)sl);
   // (in asm: hipcc would let every read of LDS wait for all requests. Nothing is returned to a register)
-  auto request = [&](int t, int slot, int i) {
-    const int k = __builtin_amdgcn_readfirstlane(min(t, nk - 1) * DK * 2);  // past the end: the last one, which nobody reads
-    const unsigned at = __builtin_amdgcn_readfirstlane(to + slot * (STG * 2) + i * 4096);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(at), "v"(from[i]),
-                 "s"(i < WP / 2 ? rw : rx), "s"(k)
+  auto request = [&](const u32x4& rsrc, unsigned at, unsigned from, int t) {
+    const int k = __builtin_amdgcn_readfirstlane(min(t, nk - 1) * GBK * 2);  // past the end: the last one, which nobody reads
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(at)),
+                 "v"(from), "s"(rsrc), "s"(k)
                  : "m0");
   };
-  f32x16 acc[AI][BJ];
+  auto weight = [&](int t, int place, int i) { request(rw, base + (2 * place + wa) * HALF + (wb * 4 + i) * 1024, from_w[i], t); };
+  auto row = [&](int t, int place, int i) { request(rx, base + BAT + place * BST + (wv * B + i) * 1024, from_x[i], t); };
+  f32x4 acc[2][4][B];
 #pragma unroll
-  for (int i = 0; i < AI; ++i)
+  for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int j = 0; j < BJ; ++j)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-  const int sw = (l32 >> 2) & 3;
-  const int ar = (wn * AI * 32 + l32) * DK, br = (WP * 32 + wm * BJ * 32 + l32) * DK;
-  bf16x8 a[2][AI], x[2][BJ];
-  auto frag = [&](int slot, int s, int n) {  // fragment n of sub-step s: a run of weights, then one of activations, ...
-    const bf16_t* st = gl + slot * STG + (((2 * s + hh) ^ sw) << 3);
-    if (n % 2 == 0) a[s][n / 2] = *reinterpret_cast<const bf16x8*>(st + ar + n / 2 * 32 * DK);
-    else x[s][n / 2] = *reinterpret_cast<const bf16x8*>(st + br + n / 2 * 32 * DK);
+      for (int j = 0; j < B; ++j) acc[h][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 a[2][4], x[2][B];
+  const int sw = (r16 >> 1) & 7, ar = (wa * 64 + r16) * 128, xr = BAT + (wb * 16 * B + r16) * 128;
+  auto read_w = [&](int place, int h, int s, int i) {
+    a[s][i] = *reinterpret_cast<const bf16x8*>(sl + (2 * place + h) * HALF + ar + ((4 * s + g) ^ sw) * 16 + i * 2048);
   };
-  // pair c of sub-step s, and beside it two of the fragments of the next one
-  auto pair = [&](int slot, int s, int c) {
-#pragma unroll
-    for (int n = 2 * c; n < 2 * c + 2 && n < NF; ++n) frag(slot, s ^ 1, n);
-#pragma unroll
-    for (int m = 2 * c; m < 2 * c + 2; ++m)
-      acc[m % AI][m / AI] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s][m % AI], x[s][m / AI], acc[m % AI][m / AI], 0, 0, 0);
-  };
-#pragma unroll
-  for (int t = 0; t < 4; t += 2)
-#pragma unroll
-    for (int i = 0; i < 2 * NP; ++i) request(t + i % 2, t + i % 2, i / 2);
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NP) : "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-#pragma unroll
-  for (int n = 0; n < NF; ++n) frag(0, 0, n);
-  int slot = 0;  // of stage t
-  auto after = [](int s) { return s == NS - 1 ? 0 : s + 1; };
-  // Stages t + 4 and t + 5 (t even), a row's two halves together, go into the free place and stage t's: from t's barrier on, evenly
-  // over three sub-steps (a CU takes 16 cycles a request; in one sub-step they held the products up)
-  constexpr auto upto = [](int c) { return c * 2 * NP / (3 * NC); };
-  auto requests = [&](int t, int free, int own, int c) {
-#pragma unroll
-    for (int i = upto(c); i < upto(c + 1); ++i) request(t + 4 + i % 2, i % 2 ? own : free, i / 2);
-  };
-  auto stage = [&](int t, auto odd_) {
-    constexpr bool odd = decltype(odd_)::value;
-    const int next = after(slot), before = slot == 0 ? NS - 1 : slot - 1, before2 = before == 0 ? NS - 1 : before - 1;
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      pair(slot, 0, c);
-      if (odd) requests(t - 1, before2, before, NC + c);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    // stage t is in all waves' registers, stage t + 1 in LDS (what was requested after it may be on its way)
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(odd ? upto(2 * NC) : 2 * NP) : "memory");
+  auto read_x = [&](int place, int s, int j) { x[s][j] = *reinterpret_cast<const bf16x8*>(sl + place * BST + xr + ((4 * s + g) ^ sw) * 16 + j * 2048); };
+  auto change = [&] {
+    __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
+  };
+  auto products = [&](int h) {
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      pair(next, 1, c);
-      if (odd) requests(t - 1, before2, before, 2 * NC + c);
-      else requests(t, before, slot, c);
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < B; ++j) acc[h][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s][i], x[s][j], acc[h][i][j], 0, 0, 0);
+    __builtin_amdgcn_s_setprio(0);
+  };
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) weight(t, t, i);
+#pragma unroll
+    for (int i = 0; i < B; ++i) row(t, t, i);
+  }
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 + B) : "memory");
+  change();
+  if (wa) change();  // the second group is one turn behind
+  int pw = 0, px = 0;  // of stage t
+  for (int t = 0; t < nk; ++t) {
+    const int before = pw == 0 ? 2 : pw - 1;  // where stage t - 1 was
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) read_w(pw, 0, s, i);
+#pragma unroll
+      for (int j = 0; j < B; ++j) read_x(px, s, j);
+      __builtin_amdgcn_sched_barrier(0);
+      weight(t + 2, before, s);
       __builtin_amdgcn_sched_barrier(0);
     }
-    slot = next;
-  };
-  for (int t = 0; t < nk; t += 2) {
-    stage(t, std::false_type{});
-    stage(t + 1, std::true_type{});
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    change();
+    products(0);
+    change();
+#pragma unroll
+    for (int i = 0; i < 4 + (B > 2 ? B - 2 : 0); ++i) {
+      if (i < 4) read_w(pw, 1, i / 2, i % 2 * 2), read_w(pw, 1, i / 2, i % 2 * 2 + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (i < 2) weight(t + 2, before, 2 + i);
+      else if (i - 2 < B) row(t + 2, px, i - 2);  // both groups have read them
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(4 + B) : "memory");  // stage t + 1 has landed
+    change();
+    products(1);
+    change();
+    pw = pw == 2 ? 0 : pw + 1;
+    px ^= 1;
   }
+  if (!wa) change();
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the repeated stages, before the LDS is given back
-  expert_store<UP, WN, AI, WM, BJ>(p, acc, lo, nr, n0);
+#pragma unroll
+  for (int j = 0; j < B; ++j) {
+    const int r = (wb * B + j) * 16 + r16;
+    if (r >= nr) continue;
+    const float s = p.scale ? p.wts[p.perm[lo + r]] : 1.f;
+    bf16_t* y = reinterpret_cast<bf16_t*>(p.y) + (long long)(lo + r) * N;
+#pragma unroll
+    for (int h = 0; h < (UP ? 1 : 2); ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int n = n0 + wa * (UP ? 64 : 128) + h * 64 + i * 16 + 4 * g;
+        if (n >= N) continue;  // (N % 4 == 0)
+        float o[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (UP) {
+            const float gt = acc[0][i][j][e] * s, up = acc[1][i][j][e] * s;
+            o[e] = gt * __builtin_amdgcn_rcpf(1.f + __expf(-gt)) * up;
+          } else {
+            o[e] = acc[h][i][j][e] * s;
+          }
+        }
+        *reinterpret_cast<uint2*>(y + n) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+      }
+  }
 }
 
-// NARROW: tiles of up to 192 rows x 128 weight rows (FAR: 128 rows)
-template <bool UP, bool NARROW, bool FAR = false>
-__global__ void __launch_bounds__(256, NARROW ? 2 : 1) expert_gemm_kernel(ExpertArgs p) {
-  extern __shared__ __attribute__((aligned(16))) bf16_t gl[];  // [2][weight rows, then activation rows][GBK]
-  // order: an XCD works a contiguous run of (expert, weight block, row tile), so the row tiles that share a
-  // weight block are on one XCD at one time
-  constexpr int NB = (NARROW ? 128 : 256) / (UP ? 2 : 1);
-  const int nt = *p.ntiles, nb = (p.N + NB - 1) / NB;
-  if ((int)blockIdx.x >= nt * nb) return;
-  // late tiles (late_tile: alone, at most half full, after all others) fill the CUs that the last long blocks leave idle
+// A block's tile and weight block. An XCD works a contiguous run of (expert, weight block, row tile), so the row tiles that share a
+// weight block are on one XCD at one time. Late tiles (late_tile: alone, at most half full, after all others) fill the CUs that the
+// last long blocks leave idle.
+struct GemmPlace {
+  int tile, bn;
+};
+__device__ __forceinline__ GemmPlace gemm_place(const ExpertArgs& p, int nt, int nb) {
   int id = xcd_remap(blockIdx.x, nt * nb);
   const int* t0 = p.tiles + id / nb * 5;
   int first = t0[3], of = t0[4], large = 0;  // (requested with the count's loads; right where there are none)
@@ -1085,17 +1139,66 @@ __global__ void __launch_bounds__(256, NARROW ? 2 : 1) expert_gemm_kernel(Expert
     t0 = p.tiles + id / nb * 5;
     first = t0[3], of = t0[4];
   }
-  const int in = id - first * nb, tile = first + in % of, bn = in / of;
+  const int in = id - first * nb;
+  return {first + in % of, in / of};
+}
+
+// The tiles stand by size, largest first (group_rows). Of each size an XCD takes a run of neighbours, which share weight blocks or rows
+// in its cache, and as much as the others. (One run of all sizes: the XCD of the largest tiles ends last, 4096 tokens above 834 us instead
+// of 774. Rounds of 256 blocks over all XCDs: at 1200 tokens, whose tiles share nothing, eight neighbouring experts' gate and up rows
+// at a time 437 instead of 386.) Returns -1 past the XCD's last.
+__device__ __forceinline__ int turns_place(const ExpertArgs& p, int nt, int nb) {
+  int n[4] = {0, 0, 0, 0};  // tiles of 4 .. 1 runs of 64 rows
+  for (int i = 0; i < nt; i += 64) {
+    const int t = i + (threadIdx.x & 63), u = t < nt ? (p.tiles[t * 5 + 2] + 63) / 64 : 0;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) n[b] += __popcll(__ballot(u == 4 - b));
+  }
+  const int x = blockIdx.x & 7;
+  int y = blockIdx.x >> 3, first = 0;
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const int m = __builtin_amdgcn_readfirstlane(n[b]) * nb, lo = (int)((long long)m * x >> 3), c = (int)((long long)m * (x + 1) >> 3) - lo;
+    if (y < c) return first + lo + y;
+    y -= c;
+    first += m;
+  }
+  return -1;
+}
+
+template <bool UP>
+__global__ void __launch_bounds__(512, 1) expert_turns_kernel(ExpertArgs p) {
+  extern __shared__ __attribute__((aligned(1024))) char sl[];
+  constexpr int NB = GN / (UP ? 2 : 1);
+  const int nt = *p.ntiles, nb = (p.N + NB - 1) / NB;
+  const int id = turns_place(p, nt, nb);
+  if (id < 0) return;
+  const int* t0 = p.tiles + id / nb * 5;
+  const int in = id - t0[3] * nb, tile = t0[3] + in % t0[4], bn = in / t0[4];
   const int* tl = p.tiles + tile * 5;
   const int nr = tl[2], n0 = bn * NB;
+  if (nr > 192) expert_turns_tile<UP, 4>(p, sl, tl[0], tl[1], nr, n0);
+  else if (nr > 128) expert_turns_tile<UP, 3>(p, sl, tl[0], tl[1], nr, n0);
+  else if (nr > 64) expert_turns_tile<UP, 2>(p, sl, tl[0], tl[1], nr, n0);
+  else expert_turns_tile<UP, 1>(p, sl, tl[0], tl[1], nr, n0);
+}
+
+// NARROW: tiles of up to 192 rows x 128 weight rows (FAR: 128 rows)
+template <bool UP, bool NARROW, bool FAR = false>
+__global__ void __launch_bounds__(256, NARROW ? 2 : 1) expert_gemm_kernel(ExpertArgs p) {
+  extern __shared__ __attribute__((aligned(16))) bf16_t gl[];  // [2][weight rows, then activation rows][GBK]
+  constexpr int NB = (NARROW ? 128 : 256) / (UP ? 2 : 1);
+  const int nt = *p.ntiles, nb = (p.N + NB - 1) / NB;
+  if ((int)blockIdx.x >= nt * nb) return;
+  const GemmPlace at = gemm_place(p, nt, nb);
+  const int* tl = p.tiles + at.tile * 5;
+  const int nr = tl[2], n0 = at.bn * NB;
   if constexpr (FAR) {
     expert_gemm_tile<UP, 2, 2, 2, 2, true>(p, gl, tl[0], tl[1], nr, n0);
   } else if constexpr (NARROW) {
     if (nr > 128) expert_gemm_tile<UP, 2, 2, 2, 3>(p, gl, tl[0], tl[1], nr, n0);
     else if (nr > 64) expert_gemm_tile<UP, 2, 2, 2, 2>(p, gl, tl[0], tl[1], nr, n0);
     else expert_gemm_tile<UP, 2, 2, 2, 1>(p, gl, tl[0], tl[1], nr, n0);
-  } else if (p.K % 64 == 0 && nr > 192) {
-    expert_dma_tile<UP>(p, gl, tl[0], tl[1], nr, n0);
   } else {
     if (nr > 192) expert_gemm_tile<UP, 2, 4, 2, 4>(p, gl, tl[0], tl[1], nr, n0);
     else if (nr > 160) expert_gemm_tile<UP, 4, 2, 1, 6>(p, gl, tl[0], tl[1], nr, n0);
@@ -1112,6 +1215,15 @@ int gemm_go(const ExpertArgs& a, int max_tiles, hipStream_t s) {
   auto kern = expert_gemm_kernel<UP, NARROW, FAR>;
   if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess) return 5;
   hipLaunchKernelGGL(kern, dim3((a.N + NB - 1) / NB * max_tiles), dim3(256), LDS, s, a);
+  return hipGetLastError() == hipSuccess ? 0 : 4;
+}
+
+template <bool UP>
+int turns_go(const ExpertArgs& a, int max_tiles, hipStream_t s) {
+  constexpr int NB = GN / (UP ? 2 : 1);
+  auto kern = expert_turns_kernel<UP>;
+  if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, WIDE_LDS) != hipSuccess) return 5;
+  hipLaunchKernelGGL(kern, dim3((a.N + NB - 1) / NB * max_tiles + 32), dim3(512), WIDE_LDS, s, a);  // (an XCD's run of a size is one longer or not)
   return hipGetLastError() == hipSuccess ? 0 : 4;
 }
 
@@ -1236,6 +1348,7 @@ KCA_API int kca_moe_expert(int dtype, const void* x, const void* w, void* y, con
   if (mt == GM || mt == 128 || mt == 192) {
     if (dtype != 1 || K % 8 || N % 4 || !al16(x) || !al16(w) || (uintptr_t)y % 8 || (far && mt != 128)) return 10;
     if (far) return up ? gemm_go<true, true, true>(a, max_tiles, s) : gemm_go<false, true, true>(a, max_tiles, s);
+    if (mt == GM && K % GBK == 0) return up ? turns_go<true>(a, max_tiles, s) : turns_go<false>(a, max_tiles, s);
     if (mt == GM) return up ? gemm_go<true, false>(a, max_tiles, s) : gemm_go<false, false>(a, max_tiles, s);
     return up ? gemm_go<true, true>(a, max_tiles, s) : gemm_go<false, true>(a, max_tiles, s);
   }

@@ -106,15 +106,17 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
     wide ones (256 x 256). Both products of a layer, us (width, experts, top, inner size; - not measured):
 
         4096, 16, 2, 4096   tokens   24: vector 270, stream 273     32: 312, 291             100: 716, 296, narrow 302
-                                    160: stream 298, narrow 296    250: 322, 302             800: 340 - 346, wide 337
-                                   1000: narrow 374, wide 347     2000: 609 - 632, 578      4096: 946, 904
-        2048, 32, 4, 1024   tokens   12: vector 71, stream 74       32: 111, 87, narrow -    100: 265, 89, 91
-                                    250: stream 99, narrow 92     1000: 128 rows 132, 192 rows 116, wide 120
-                                   1500: 143, 162, 140            4096: 302, 267, 301       8192: -, 551, 540
+                                    160: stream 298, narrow 296    300: 339, 305, wide 306  700: narrow 338, wide 322
+                                   1000: narrow 367, wide 333     1300: 377, 339           2500: 610, 505
+        4096, 16, 3, 2048   tokens  300: narrow 182, wide 195     900: 208, 209            1500: 295, 227     3000: 487, 330
+        2048, 32, 4, 1024   tokens   12: vector 71, stream 74       32: 111, 87, narrow -    100: 265, 87, 87
+                                    500: narrow 93, wide 103      1150: 115, 115           3000: 211, 172     8192: 511, 406
         4096, 20, 3, 2048   tokens   24: vector 165, stream 166     32: 190, 172             160: 450 (100), 183, 178
-                                    600: 128 rows 226, 192 rows 197    1500: 309, 312, wide 332    4096: 645, 634, 558
-        2048, 32, 5, 768    tokens   12: vector 53, stream 51       32: 83, 61               250: -, 70, narrow 77
-                                    400: stream 76, narrow 79      600: 94, 128 rows 77      8192: -, 382, wide 445
+                                    900: narrow 271, wide 286     1500: 349, 342           3000: 608, 437
+        2048, 24, 5, 768    tokens  400: narrow 73, wide 83        777: 83, 85              1300: 96, 86      2000: 117, 106
+        (32 outputs, uneven)       3000: 141, 143                  4096: 231, 189
+        2048, 40, 4, 1024   tokens 1200: narrow 142, wide 161     2000: 181, 188           2048, 10, 2, 2048, 600: 84, 90; 2000: 147, 141
+        5120, 8, 2, 2560    tokens  400: narrow 183, wide 156     1200: 275, 283           2000: 386, 333
         widths that are no multiple of 64 have no stream; rows an expert, vector against narrow blocks:
         4104, 16, 2, 2056   3: 179, 154   4: 209, 176   8: 335, 180   16: 605, 186     1032, 16, 2, 520   4: 34, 22   16: 89, 22
         4104, 16, 2, 4104   3: 334, 337   4: 376, 329   8: 590, 335   16: 1099, 347    2056, 32, 4, 1032  4: 134, 101
@@ -123,8 +125,10 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
     its work), but up to 16 tokens the vector product also carries the shared expert. A stream tile holds 32 rows, past
     which weights are read again, so it ends at 16 rows -- at 64 where narrow blocks are too few to fill the chip. A
     narrow tile of 192 rows saves a second tile a little over 128 rows, if there are blocks enough without it, and costs
-    one a little over 192. A wide block is
-    alone on its CU and pays its ramps in full: it needs a long contraction, or many rows."""
+    one a little over 192. A wide block is alone on its CU: it wins where the matrix cores bound the products, from
+    about 150 rows (64 where a contraction is long), if its rounds are well filled (``fill``: the blocks' time over that
+    of the rounds that they take; identity outputs count as experts here, so it is an estimate). Uneven experts cost
+    narrow and wide blocks alike from there on; with fewer rows wide ones wait for the largest expert's."""
     n = T * top
     used = min(E, n)
     # 32-bit offsets into an expert's weights and the rows of a tile (elsewhere only 128-row tiles have longer ones)
@@ -136,7 +140,18 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
         stream = d % 64 == 0 and F % 64 == 0
         r, short, full = n / used, min(d, F), used * (F // 64) >= 512
         if r > ((16 if full else 64) if stream else 4):
-            if r > 96 and (short >= 4096 or (short >= 1024 and r > 512)):
+            if stream:
+                tiles = used * -(-r // GEMM_ROWS)
+                up, down = tiles * -(-F // 128), tiles * -(-d // 256)  # wide blocks of the two products; rounds of one a CU
+                fill = (up * d + down * F) / (256 * (-(-up // 256) * d + -(-down // 256) * F))
+                once = max(up, down) <= 256 and min(up, down) >= 144
+                if r > GEMM_ROWS:
+                    wide = fill >= 0.8 or (fill >= 0.6 and r > 480 and short >= 2048)
+                else:
+                    wide = r > 64 and short >= 4096 or r > 150 and (once or fill >= 0.8) or r > 175 and fill >= 0.6 and short >= 2048
+                if wide:
+                    return GEMM_ROWS
+            elif r > 96 and (short >= 4096 or (short >= 1024 and r > 512)):
                 return GEMM_ROWS
             return 192 if (full and 100 < r <= 160) or r > 240 else 128
         if stream and T > SHARED_ROWS and r > (3 if d > 2048 else 2):

@@ -61,6 +61,32 @@ def test_short_tiles_run_last(counts, mt):
     assert (y.float() - want).norm() <= TOL * want.norm()
 
 
+@pytest.mark.parametrize("counts,d,F", [([250, 64, 577, 1, 0, 129, 300, 65], 128, 320), ([70, 300, 10, 150] * 18, 64, 640), ([130] * 9 + [769, 513], 192, 1152),
+                                        ([257, 320, 63], 1088, 64)])
+def test_wide_tiles(counts, d, F):
+    """Rows of an expert in even tiles, largest first; blocks of all four sizes, fewer than a round, several rounds, 1, 2, 3 and 17 stages, weight
+    rows that end within a block."""
+    h, ids, wts, gu, dn = _case(counts, 1, d, F)
+    g = moe.group(ids, len(counts), moe.GEMM_ROWS)
+    tiles = g.tiles[:int(g.ntiles)].tolist()
+    for e, c in enumerate(counts):
+        units = [-(-t[2] // 64) for t in tiles if t[0] == e]
+        assert sum(t[2] for t in tiles if t[0] == e) == c and len(units) == -(-c // 256) and sum(units) == -(-c // 64)
+        assert not units or max(units) - min(units) <= 1
+    most = [-(-tiles[t[3]][2] // 64) for t in tiles]
+    assert most == sorted(most, reverse=True)
+    for scale_in in (True, False):
+        y = moe.experts(h, ids, wts, gu, dn, g, scale_in)[g.inv.view(-1).long()].float()
+        want = torch.empty_like(y)
+        for e in range(len(counts)):
+            k = ids.view(-1) == e
+            w = wts.view(-1)[k, None]
+            u = h[k].float() @ gu[e].float().T * (w if scale_in else 1)
+            a = (torch.nn.functional.silu(u[:, :F]) * u[:, F:]).bfloat16().float()
+            want[k] = a @ dn[e].float().T * (1 if scale_in else w)
+        assert (y - want).norm() <= TOL * want.norm()
+
+
 def _far(T, d, F, E):
     """Sizes past the 32-bit offsets, and some tokens' outputs in fp32."""
     g = torch.Generator(device="cuda").manual_seed(1)
