@@ -13,9 +13,15 @@
 // The forms of a mask are attention_tiled.hip's general ones (1: lengths, windows, any sizes; 2: ALiBi) and every call takes
 // one of them. The order of the blocks: block_of.
 //
-// Tiles in LDS: two buffers of K and V a group. A step computes S of the group's next tile while it takes the softmax of this
-// one, so K runs a tile ahead of V: K(i + 2) goes where K(i) was and V(i + 1) where V(i - 1) was, which all waves have read
-// before the last barrier (K(0), which is read before the first step, has one of its own).
+// Tiles go from memory straight into LDS (TileRequests), NB of K and NB of V a group in turn: three steps ahead of their use with one group, one
+// or two where two groups' tiles fill the LDS. One barrier a step: behind it a tile has landed for all waves and another has been read by all,
+// whose place is requested at once. A wave requests K or V, not both; a request of 1 KB takes a CU's address path 16 cycles, so those of
+// a step stand between its products. What it replaces, tiles through registers one step ahead, cost their LDS stores, 16 registers and, at a
+// step's end, the wait for memory: a step of 96-wide rows took 1300 cycles alone on its CU, now 1000 (384 of products), and 168
+// registers let a third workgroup run. The forward computes S of the next tile while it takes the softmax of this one, so it reads K a tile ahead.
+// us, before and now: forward 1 x 1500 x 64 x 96 58 -> 48, 4 x 2048 x 32 x 96 160 -> 133, 2 x 2048 x 20 x 128 60 -> 54, 1 x 4000 x 20 x 128 105 -> 91, 3 x 2048
+// x 16 x 64 40.5 -> 38; backward 1 x 1500 x 64 x 96 144 -> 136, 2 x 2048 x 20 x 128 190 -> 169, 2048 x 14 x 128 with ALiBi 112 -> 95,
+// 4 x 2048 x 32 x 96 436 -> 407, 8 x 1000 x 12 x 64 72 -> 71. (The forward's scores are no longer copied from step to step: 3 % of it.)
 //
 // Softmax reference: as in attn_fwd_tiled_kernel the row's maximum over the first tile with a visible key, here of each
 // group; the groups' sums are scaled to the largest reference when they meet. Rows whose sum passes 2^100 (a later score far
@@ -30,13 +36,13 @@ constexpr int kNoTile = 1 << 29;  // first "key" of a tile past the end of a gro
 
 template <int D, int G, int RW, int KG, int WPS>
 __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_fwd_split_kernel(FastFwdParams p) {
-  constexpr int BM = 32 * RW, BN = 32, NTG = 64 * RW;
+  constexpr int BM = 32 * RW, BN = 32;
   constexpr int TILE = BN * D * 2, KS = D / 16;
-  using Stg = GroupStager<D, NTG>;
-  constexpr int CPT = Stg::CPT;
+  constexpr int NB = KG == 1 ? 4 : D == 128 ? 2 : 3;  // tiles of K and of V in LDS, a group
+  using Req = TileRequests<D, RW / 2>;                // (half of a group's waves request K, the others V)
   constexpr int PART = 32 * D * 4;  // a wave's partial sums
-  static_assert((KG - 1) * RW * PART <= KG * 4 * TILE, "the partial sums take the tiles' place");
-  __shared__ __attribute__((aligned(16))) char smem[KG * 4 * TILE];  // per group [K 0 | K 1 | V 0 | V 1]
+  static_assert((KG - 1) * RW * PART <= KG * 2 * NB * TILE, "the partial sums take the tiles' place");
+  __shared__ __attribute__((aligned(16))) char smem[KG * 2 * NB * TILE];  // per group [K's NB tiles | V's]
   __shared__ float stat[KG][RW][32][2];                              // reference, sum of each row and group
   __shared__ int again;
 
@@ -44,7 +50,7 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_fwd_split_kernel(FastF
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = wave / RW, rw = wave % RW;
   const int l32 = lane & 31, hh = lane >> 5, gi = lane & 15;
   const int nqb = (p.Sq + BM - 1) / BM, heads = p.B * p.H;
-  const auto [qi, bh] = block_of<true, D, BM, D == 64 ? 3 : 1>(nqb, heads);
+  const auto [qi, bh] = block_of<true, D, BM, WPS == 3 ? 3 : 1>(nqb, heads);
   const int qb = nqb - 1 - qi;
   const int b = bh / p.H, h = bh % p.H;
   const int hk = h / (p.H / p.Hkv);
@@ -66,16 +72,25 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_fwd_split_kernel(FastF
   const float sl2 = p.scale * kLog2e;
 
   const bf16_t* qp = p.q + b * p.q_sb + h * p.q_sh;
-  const __amdgpu_buffer_rsrc_t rk = head_rsrc(p.k + b * p.k_sb + hk * p.k_sh, rows_bytes(kv_end, p.k_st, D));
-  const __amdgpu_buffer_rsrc_t rv = head_rsrc(p.v + b * p.v_sb + hk * p.v_sh, rows_bytes(kv_end, p.v_st, D));
-  const Stg stk(tid % NTG, p.k_st), stv(tid % NTG, p.v_st);
-  const int kst2 = (int)p.k_st * 2, vst2 = (int)p.v_st * 2;
-  auto at = [](int k0, int st2) { return __builtin_amdgcn_readfirstlane(k0 * st2); };
-  char* const kbuf = smem + g * 4 * TILE;
-  char* const vbuf = kbuf + 2 * TILE;
-  u32x4 xk[CPT], xv[CPT];
-  stk.load(xk, rk, at(key0(0), kst2));  // (flies with the query rows)
-  stv.load(xv, rv, at(key0(0), vst2));
+  const int val = rw / (RW / 2);  // 0: this wave requests keys, 1: values
+  const long long rst = val ? p.v_st : p.k_st;
+  const u32x4 words = val ? head_words(p.v + b * p.v_sb + hk * p.v_sh, rows_bytes(kv_end, p.v_st, D))
+                          : head_words(p.k + b * p.k_sb + hk * p.k_sh, rows_bytes(kv_end, p.k_st, D));
+  const Req req(rw % (RW / 2), lane, rst);
+  char* const kbuf = smem + g * 2 * NB * TILE;
+  char* const vbuf = kbuf + NB * TILE;
+  char* const ring = val ? vbuf : kbuf;
+  auto request = [&](int i, int place, int j) { req(words, ring + place * TILE, __builtin_amdgcn_readfirstlane(key0(i) * (int)rst * 2), j); };
+  auto requests = [&](int i, int place) {
+#pragma unroll
+    for (int j = 0; j < Req::N; ++j) request(i, place, j);
+  };
+  auto first = [&] {  // the places that the first step does not fill
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+      if (i < NB - 1 || !val) requests(i, i);
+  };
+  first();
   bf16x8 qf[KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s)
@@ -87,7 +102,7 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_fwd_split_kernel(FastF
   const int c3 = 2 * ((lane >> 4) & 1) + ((gi & 3) >> 1);
   const int vb_1 = 64 * (4 * hh + (gi >> 2)) + 16 * (c3 ^ hh) + 8 * (gi & 1);
   const int vb_2 = 16 * D + 64 * (4 * hh + (gi >> 2)) + 16 * (c3 ^ hh ^ 2) + 8 * (gi & 1);
-  auto qk = [&](const char* Ks) {
+  auto qk = [&](const char* Ks, auto beside) {  // beside(s): after product s
     f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
@@ -103,6 +118,7 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_fwd_split_kernel(FastF
       }
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[s % 3], qf[s], acc, 0, 0, 0);
       __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+      beside(s);
     }
     return acc;
   };
@@ -130,37 +146,36 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_fwd_split_kernel(FastF
       m = -INFINITY;
       begun = true;
       for (int i = 0; i < nsteps; ++i) {
-        stk.load(xk, rk, at(key0(i), kst2));
-        stk.store(xk, kbuf);
-        __syncthreads();
-        f32x16 s = qk(kbuf);
+        if (!val) requests(i, 0);
+        wait_and_meet<0>();
+        f32x16 s = qk(kbuf, [](int) {});
         mask(s, mkey0(i));
 #pragma unroll
         for (int r = 0; r < 16; ++r) m = fmaxf(m, s[r] == -INFINITY ? -INFINITY : biased(s[r], r, key0(i)));
         __syncthreads();
       }
       m = fmaxf(m, __shfl_xor(m, 32, 64));
-      stk.load(xk, rk, at(key0(0), kst2));
-      stv.load(xv, rv, at(key0(0), vst2));
+      first();
     }
     clear<D>(oacc);
     lsum = 0.f;
     float nm = pass == 0 || m == -INFINITY ? 0.f : -m;
-    stk.store(xk, kbuf);
-    stv.store(xv, vbuf);
-    stk.load(xk, rk, at(key0(1), kst2));
-    stk.store(xk, kbuf + TILE);
-    __syncthreads();
-    f32x16 sa = qk(kbuf);
-    __syncthreads();  // all waves have read K(0), for the first step stores K(2) in its place
+    wait_and_meet<(NB - 1) * Req::N>();
+    f32x16 sa = qk(kbuf, [](int) {});
 
-    auto step = [&](int i, auto masked) {
+    auto step = [&](int i, f32x16& sa, f32x16& sb, auto masked) {
       constexpr bool MASKED = decltype(masked)::value, HEAD = decltype(masked)::value == 2;
       const int k0 = key0(i), mk0 = mkey0(i);
-      stk.load(xk, rk, at(key0(i + 2), kst2));
-      stv.load(xv, rv, at(key0(i + 1), vst2));
-      asm volatile("" ::: "memory");  // (the loads stay above the products, their LDS stores below)
-      f32x16 sb = qk(kbuf + ((i + 1) & 1) * TILE);  // S of the group's next tile (unused after the last)
+      // K(i + 1) and V(i) have landed, and all waves have read K(i) and V(i - 1): the next tiles go there
+      wait_and_meet<(NB - 2) * Req::N>();
+      sb = qk(kbuf + (i + 1) % NB * TILE, [&](int s) {  // S of the group's next tile (unused after the last)
+        constexpr int EACH = KS / Req::N;
+        static_assert(KS % Req::N == 0, "requests at even distances");
+        if (s % EACH) return;
+        __builtin_amdgcn_sched_barrier(0x406);
+        request(i + NB - val, (i + NB - val) % NB, s / EACH);
+        __builtin_amdgcn_sched_barrier(0x406);
+      });
       float sl = sl2, bias[16];  // P = exp2(s * sl + bias)
       if constexpr (G == 2) {
         const float b0 = slope * (float)(k0 + 4 * hh - qrow - off) + (MASKED ? 0.f : nm);
@@ -205,7 +220,7 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_fwd_split_kernel(FastF
         pf1[r] = (__bf16)e1;
       }
       lsum += ps;
-      const char* Vs = vbuf + (i & 1) * TILE;
+      const char* Vs = vbuf + i % NB * TILE;
       auto vfrag = [&](int db, int s) {
         return cat8(lds_tr4(Vs, vb_1 + 2 * s * 16 * D + 512 * db), lds_tr4(Vs, vb_2 + 2 * s * 16 * D + 512 * db));
       };
@@ -224,30 +239,38 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_fwd_split_kernel(FastF
         oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vb[db & 1], pf1, oacc[db], 0, 0, 0);
         __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
       }
+    };
+    f32x16 sb;
+    auto one = [&](int i, auto masked) {
+      step(i, sa, sb, masked);
       sa = sb;
-      asm volatile("" ::: "memory");
-      stk.store(xk, kbuf + (i & 1) * TILE);
-      stv.store(xv, vbuf + ((i + 1) & 1) * TILE);
-      __syncthreads();
+    };
+    auto free = [&](int i, int end) {  // in pairs: no copy of the scores
+      for (; i + 1 < end; i += 2) {
+        step(i, sa, sb, std::false_type{});
+        step(i + 1, sb, sa, std::false_type{});
+      }
+      if (i < end) one(i, std::false_type{});
     };
     if constexpr (G == 1) {
       // Steps whose KG tiles may hold a row's first visible key of their group: below f_lo the rows' first ones, up to
       // KG - 1 tiles on the other groups'. Free ones lie whole at or below f_hi.
       const int head = min(nsteps, (sp.f_lo - sp.lo + 2 * KG - 2) / KG);
       const int top = max(head, min(nsteps, (min(sp.f_hi + 1, sp.hi) - sp.lo) / KG));
-      for (int i = 0; i < head; ++i) step(i, std::integral_constant<int, 2>{});
-      for (int i = head; i < top; ++i) step(i, std::false_type{});
-      for (int i = top; i < nsteps; ++i) step(i, std::true_type{});
+      for (int i = 0; i < head; ++i) one(i, std::integral_constant<int, 2>{});
+      free(head, top);
+      for (int i = top; i < nsteps; ++i) one(i, std::true_type{});
     } else {
       // from the last tile down: a row's last visible key lies above f_hi, another group's up to KG - 1 tiles below
       const int top = min(nsteps, (sp.hi - 1 - sp.f_hi + 2 * KG - 2) / KG);
       const int low = max(top, min(sp.hi - sp.f_lo, ntiles) / KG);
-      for (int i = 0; i < top; ++i) step(i, std::true_type{});
-      for (int i = top; i < low; ++i) step(i, std::false_type{});
-      for (int i = low; i < nsteps; ++i) step(i, std::true_type{});
+      for (int i = 0; i < top; ++i) one(i, std::true_type{});
+      free(top, low);
+      for (int i = low; i < nsteps; ++i) one(i, std::true_type{});
     }
 
-    // the groups' sums meet (the tiles are no longer read: the last step's barrier)
+    // the groups' sums meet where the tiles were
+    wait_and_meet<0>();
     const float ltot = lsum + __shfl_xor(lsum, 32, 64);
     const bool bad = !(ltot < 1.2676506e30f) && qrow < p.Sq;
     if (pass == 0 && __any(bad) && lane == 0) again = 1;
@@ -291,19 +314,19 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_fwd_split_kernel(FastF
 // dQ: as the forward, a group walks every KG-th key tile of its 32 RW query rows; the groups' dQ add up in LDS.
 template <int D, int G, int RW, int KG, int WPS>
 __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dq_split_kernel(FastBwdParams p) {
-  constexpr int BM = 32 * RW, BN = 32, NTG = 64 * RW;
+  constexpr int BM = 32 * RW, BN = 32;
   constexpr int TILE = BN * D * 2, KS = D / 16;
-  using Stg = GroupStager<D, NTG>;
-  constexpr int CPT = Stg::CPT;
+  constexpr int NB = KG == 1 ? 4 : D == 128 ? 2 : 3;  // tiles of K and of V in LDS, a group
+  using Req = TileRequests<D, RW / 2>;                // (half of a group's waves request K, the others V)
   constexpr int PART = 32 * D * 4;
-  static_assert((KG - 1) * RW * PART <= KG * 4 * TILE, "the partial sums take the tiles' place");
-  __shared__ __attribute__((aligned(16))) char smem[KG * 4 * TILE];  // per group [buf 0 | 1][K | V]
+  static_assert((KG - 1) * RW * PART <= KG * 2 * NB * TILE, "the partial sums take the tiles' place");
+  __shared__ __attribute__((aligned(16))) char smem[KG * 2 * NB * TILE];  // per group [K's NB tiles | V's]
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = wave / RW, rw = wave % RW;
   const int l32 = lane & 31, hh = lane >> 5;
   const int nqb = (p.Sq + BM - 1) / BM, heads = p.B * p.H;
-  const auto [qi, bh] = block_of<true, D, BM, D == 64 ? 3 : 1>(nqb, heads);
+  const auto [qi, bh] = block_of<true, D, BM, WPS == 3 ? 3 : 1>(nqb, heads);
   const int qb = nqb - 1 - qi;
   const int b = bh / p.H, h = bh % p.H;
   const int hk = h / (p.H / p.Hkv);
@@ -318,15 +341,19 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dq_split_kernel(Fa
   const int qr = min(qrow, p.Sq - 1);
   const bf16_t* qp = p.q + b * p.q_sb + h * p.q_sh + (long long)qr * p.q_st;
   const bf16_t* gp = p.dout + b * p.do_sb + h * p.do_sh + (long long)qr * p.do_st;
-  const __amdgpu_buffer_rsrc_t rk = head_rsrc(p.k + b * p.k_sb + hk * p.k_sh, rows_bytes(kv_end, p.k_st, D));
-  const __amdgpu_buffer_rsrc_t rv = head_rsrc(p.v + b * p.v_sb + hk * p.v_sh, rows_bytes(kv_end, p.v_st, D));
-  const Stg stk(tid % NTG, p.k_st), stv(tid % NTG, p.v_st);
-  const int kst2 = (int)p.k_st * 2, vst2 = (int)p.v_st * 2;
-  auto at = [](int k0, int st2) { return __builtin_amdgcn_readfirstlane(k0 * st2); };
-  char* const own = smem + g * 4 * TILE;
-  u32x4 xk[CPT], xv[CPT];
-  stk.load(xk, rk, at(key0(0), kst2));  // (flies with the query rows)
-  stv.load(xv, rv, at(key0(0), vst2));
+  const int val = rw / (RW / 2);  // 0: this wave requests keys, 1: values
+  const long long rst = val ? p.v_st : p.k_st;
+  const u32x4 words = val ? head_words(p.v + b * p.v_sb + hk * p.v_sh, rows_bytes(kv_end, p.v_st, D))
+                          : head_words(p.k + b * p.k_sb + hk * p.k_sh, rows_bytes(kv_end, p.k_st, D));
+  const Req req(rw % (RW / 2), lane, rst);
+  char* const kbuf = smem + g * 2 * NB * TILE;
+  char* const vbuf = kbuf + NB * TILE;
+  char* const ring = val ? vbuf : kbuf;
+  auto request = [&](int i, int place, int j) { req(words, ring + place * TILE, __builtin_amdgcn_readfirstlane(key0(i) * (int)rst * 2), j); };
+#pragma unroll
+  for (int i = 0; i < NB - 1; ++i)
+#pragma unroll
+    for (int j = 0; j < Req::N; ++j) request(i, i, j);
   bf16x8 qf[KS], gf[KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
@@ -356,17 +383,13 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dq_split_kernel(Fa
   const int last = min(qrow + off, kv_end - 1);    // row's last visible key
   const int before = p.window > 0 ? qrow + off - p.window : -(1 << 30);  // key before its first
 
-  stk.store(xk, own);
-  stv.store(xv, own + TILE);
-  __syncthreads();
   auto step = [&](int i, auto masked) {
     constexpr bool MASKED = decltype(masked)::value;
     const int k0 = key0(i);
-    const char* Ks = own + (i & 1) * 2 * TILE;
-    const char* Vs = Ks + TILE;
-    stk.load(xk, rk, at(key0(i + 1), kst2));
-    stv.load(xv, rv, at(key0(i + 1), vst2));
-    asm volatile("" ::: "memory");
+    const char* Ks = kbuf + i % NB * TILE;
+    const char* Vs = vbuf + i % NB * TILE;
+    // tile i has landed, and all waves have read tile i - 1: the next one goes there
+    wait_and_meet<(NB - 2) * Req::N>();
     f32x16 st, dpt;
 #pragma unroll
     for (int r = 0; r < 16; ++r) { st[r] = 0.f; dpt[r] = 0.f; }
@@ -387,6 +410,13 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dq_split_kernel(Fa
         st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fk[s % 3], qf[s], st, 0, 0, 0);
         dpt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fv[s % 3], gf[s], dpt, 0, 0, 0);
         __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
+        constexpr int EACH = KS / Req::N;
+        static_assert(KS % Req::N == 0, "requests at even distances");
+        if (s % EACH == 0) {  // (all waves' at once hold the products up)
+          __builtin_amdgcn_sched_barrier(0x406);
+          request(i + NB - 1, (i + NB - 1) % NB, s / EACH);
+          __builtin_amdgcn_sched_barrier(0x406);
+        }
       }
     }
     // visible key offsets (r&3)+8(r>>2): lo < offset <= lim
@@ -423,12 +453,6 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dq_split_kernel(Fa
         __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
       }
     }
-    asm volatile("" ::: "memory");
-    if (i + 1 < nsteps) {
-      stk.store(xk, own + ((i + 1) & 1) * 2 * TILE);
-      stv.store(xv, own + ((i + 1) & 1) * 2 * TILE + TILE);
-    }
-    __syncthreads();
   };
   const int low = min(nsteps, (max(0, sp.f_lo - sp.lo) + KG - 1) / KG);
   const int top = max(low, min(nsteps, (min(sp.f_hi + 1, sp.hi) - sp.lo) / KG));
@@ -436,6 +460,7 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dq_split_kernel(Fa
   for (int i = low; i < top; ++i) step(i, std::false_type{});
   for (int i = top; i < nsteps; ++i) step(i, std::true_type{});
 
+  wait_and_meet<0>();  // what comes next lies where the tiles were
   if constexpr (KG > 1) {
     if (g > 0) put_partial<D>(smem + ((g - 1) * RW + rw) * PART, dq, lane);
     __syncthreads();
@@ -459,8 +484,7 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
   // spill at 64 (51.9 -> 61.2), 64 wide in two groups, 96 wide and 128 wide in one gain and lose 4 %.
   constexpr bool START = D == 64 ? KG == 1 && G == 1 && !WIN : D == 128 && KG == 2;
   constexpr int TILE = BQ * D * 2, KS = D / 16, NCH = D / 8;
-  using Stg = GroupStager<D, NTG>;
-  constexpr int CPT = Stg::CPT;
+  using Req = TileRequests<D, RW / 2>;  // (half of a group's waves request Q, the others dO)
   constexpr int PART = 32 * D * 4;
   static_assert((KG - 1) * RW * PART <= KG * 4 * TILE, "the partial sums take the tiles' place");
   constexpr int VOFF = KG * 4 * TILE;  // V images of the RW key blocks, the groups' alike
@@ -484,12 +508,14 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
   const int q_end = WIN ? min(p.Sq, kb * BK + BK - 1 - off + p.window) : p.Sq;
   const int nqt = max(0, q_end - q_lo + BQ - 1) / BQ;
   const int total = kb * BK < kv_end ? nqt * grp : 0, nsteps = (total + KG - 1) / KG;
-  const int qn = rows_bytes(p.Sq, p.q_st, D), gn = rows_bytes(p.Sq, p.do_st, D);
-
-  const Stg stq(gt, p.q_st), sto(gt, p.do_st);
+  const int grad = rw / (RW / 2);  // 0: this wave requests queries, 1: output gradients
+  const long long rst = grad ? p.do_st : p.q_st, rsh = grad ? p.do_sh : p.q_sh;
+  const bf16_t* const rbase = grad ? p.dout + b * p.do_sb : p.q + b * p.q_sb;
+  const int rbytes = rows_bytes(p.Sq, rst, D);
+  const Req req(rw % (RW / 2), lane, rst);
   char* const own = smem + g * 4 * TILE;
   float* const stat = reinterpret_cast<float*>(smem + LOFF) + g * 128;
-  u32x4 xq[CPT], xg[CPT];
+  char* const ring = own + grad * TILE;
   float lreg = 0.f;
   int be, bo, b1, b2;
   row_bases<D>(l32, hh, be, bo);
@@ -501,20 +527,17 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
     while (qcur >= nqt && hcur < grp - 1) qcur -= nqt, ++hcur;
     qcur = min(qcur, nqt - 1);
   };
-  auto load_tile = [&] {
-    const int hq = hk * grp + hcur, qt = q_lo + qcur * BQ;
-    const __amdgpu_buffer_rsrc_t rq = head_rsrc(p.q + b * p.q_sb + hq * p.q_sh, qn);
-    const __amdgpu_buffer_rsrc_t rg = head_rsrc(p.dout + b * p.do_sb + hq * p.do_sh, gn);
+  auto tile_words = [&] { return head_words(rbase + (hk * grp + hcur) * rsh, rbytes); };
+  auto request = [&](const u32x4& words, int buf, int j) {
+    req(words, ring + buf * 2 * TILE, __builtin_amdgcn_readfirstlane((q_lo + qcur * BQ) * (int)rst * 2), j);
+  };
+  auto load_stat = [&] {
     if (gt < 64) {  // as they come: the scaling waits until they are stored
-      const long long li = ((long long)b * p.H + hq) * p.Sq + min(qt + (gt & 31), p.Sq - 1);
+      const long long li = ((long long)b * p.H + hk * grp + hcur) * p.Sq + min(q_lo + qcur * BQ + (gt & 31), p.Sq - 1);
       lreg = (gt < 32 ? p.lse : p.delta)[li];
     }
-    stq.load(xq, rq, __builtin_amdgcn_readfirstlane((int)(qt * p.q_st * 2)));
-    sto.load(xg, rg, __builtin_amdgcn_readfirstlane((int)(qt * p.do_st * 2)));
   };
-  auto store_tile = [&](int buf) {
-    stq.store(xq, own + buf * 2 * TILE);
-    sto.store(xg, own + buf * 2 * TILE + TILE);
+  auto store_stat = [&](int buf) {
     if (gt < 64) {
       float v = lreg;
       if (q_lo + qcur * BQ + (gt & 31) >= p.Sq) v = gt < 32 ? INFINITY : 0.f;  // P = 0
@@ -524,7 +547,10 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
   if (total > 0) {  // (flies with the key and value rows)
     qcur = g;
     settle();
-    load_tile();
+    const u32x4 words = tile_words();
+#pragma unroll
+    for (int j = 0; j < Req::N; ++j) request(words, 0, j);
+    load_stat();
   }
   const bf16_t* kp = p.k + b * p.k_sb + hk * p.k_sh;
   const bf16_t* vp = p.v + b * p.v_sb + hk * p.v_sh;
@@ -550,8 +576,8 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
   clear<D>(dk);
   clear<D>(dv);
 
-  if (total > 0) store_tile(0);
-  __syncthreads();
+  if (total > 0) store_stat(0);
+  wait_and_meet<0>();
   for (int i = 0; i < nsteps; ++i) {
     const int qt = q_lo + qcur * BQ, hq = hk * grp + hcur;
     const bool gone = tile >= total;
@@ -565,7 +591,8 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
     tile += KG;
     qcur += KG;
     settle();
-    load_tile();
+    load_stat();
+    const u32x4 words = tile_words();
     asm volatile("" ::: "memory");
     f32x16 sacc, dpacc;
 #pragma unroll
@@ -595,6 +622,13 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
         sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fq[s & 1], kf[s], sacc, 0, 0, 0);
         dpacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fg[s & 1], fv[s & 1], dpacc, 0, 0, 0);
         __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
+        constexpr int EACH = KS / Req::N;
+        static_assert(KS % Req::N == 0, "requests at even distances");
+        if (s % EACH == 0) {  // the next tile, where all waves have read the one before (all waves' requests at once hold the products up)
+          __builtin_amdgcn_sched_barrier(0x406);
+          request(words, (i + 1) & 1, s / EACH);
+          __builtin_amdgcn_sched_barrier(0x406);
+        }
       }
     }
     // rows q = qt + 8g + 4hh + j (g = r>>2, j = r&3) that see the key: lim <= 8g + j < ul
@@ -656,8 +690,8 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
       }
     }
     asm volatile("" ::: "memory");
-    if (i + 1 < nsteps) store_tile((i + 1) & 1);
-    __syncthreads();
+    if (i + 1 < nsteps) store_stat((i + 1) & 1);
+    wait_and_meet<0>();
   }
   // group 0 adds dV up and stores it, then the last group dK
   if constexpr (KG > 1) {
@@ -757,6 +791,8 @@ static int with_form(int d, bool alibi, F&& f) {
 }
 
 // Causal calls of 64, 96 and 128 wide heads with 16-byte rows; 1: another head size (or, backward, a scale of nothing).
+// (Three workgroups a CU where the registers of 96-wide rows allow it without spills, ALiBi's dQ does not, and the blocks of a CU are to add up to
+// the same: 1 x 1500 x 64 forward 53 -> 46 us, backward 139 -> 134. Windowed dQ, all blocks alike, is 2 % faster with two.)
 int attn_fwd_split(const FastFwdParams& p, int d, hipStream_t stream) {
   const long long blocks = (long long)((p.Sq + 127) / 128) * p.B * p.H;
   const bool two = split_rows(blocks, d, p.Sk, p.window);
@@ -765,7 +801,7 @@ int attn_fwd_split(const FastFwdParams& p, int d, hipStream_t stream) {
     if (two)
       hipLaunchKernelGGL((attn_fwd_split_kernel<D, G, 2, 2, W>), dim3((p.Sq + 63) / 64 * p.B * p.H), dim3(256), 0, stream, p);
     else
-      hipLaunchKernelGGL((attn_fwd_split_kernel<D, G, 4, 1, W>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((attn_fwd_split_kernel<D, G, 4, 1, (D < 128 ? 3 : 2)>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
   });
 }
 
@@ -778,8 +814,10 @@ int attn_bwd_split(const FastBwdParams& p, int d, hipStream_t stream) {
     constexpr int D = decltype(D_)::value, G = decltype(G_)::value, W = D == 64 ? 3 : 2;
     if (two)
       hipLaunchKernelGGL((attn_bwd_dq_split_kernel<D, G, 2, 2, W>), dim3((p.Sq + 63) / 64 * p.B * p.H), dim3(256), 0, stream, p);
-    else
+    else if (p.window > 0)
       hipLaunchKernelGGL((attn_bwd_dq_split_kernel<D, G, 4, 1, W>), dim3((unsigned)qblocks), dim3(256), 0, stream, p);
+    else
+      hipLaunchKernelGGL((attn_bwd_dq_split_kernel<D, G, 4, 1, D == 96 && G == 1 ? 3 : W>), dim3((unsigned)qblocks), dim3(256), 0, stream, p);
     auto dkdv = [&](auto WIN_) {
       constexpr bool WIN = decltype(WIN_)::value;
       if (kv == 1)

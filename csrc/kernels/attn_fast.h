@@ -211,39 +211,54 @@ __device__ __forceinline__ void add_partial(const char* at, f32x16 (&acc)[D / 32
     }
 }
 
-// A 32-row x D tile staged by the NT threads of a group: chunk idx = thread + NT * j is (row idx / NCH, 16-byte chunk idx % NCH);
-// the last round may be the first waves' alone.
-template <int D, int NT>
-struct GroupStager {
-  static constexpr int NCH = D / 8, TOT = 32 * NCH, CPT = (TOT + NT - 1) / NT;
-  static constexpr bool EVEN = NT % NCH == 0 && TOT % NT == 0;  // chunk column the same for all j: rows a scalar offset apart
-  static_assert(TOT % 64 == 0, "whole waves");
-  int vo_[EVEN ? 1 : CPT], lds_[CPT];
-  int step_;
-  bool tail_;  // this thread owns a chunk in the last round
-  __device__ __forceinline__ GroupStager(int t, long long st) {
+// the words of head_rsrc's descriptor, for inline asm
+__device__ __forceinline__ u32x4 head_words(const bf16_t* b, int bytes) {
+  const unsigned long long a = (unsigned long long)b;
+  return u32x4{(unsigned)__builtin_amdgcn_readfirstlane((unsigned)a), (unsigned)__builtin_amdgcn_readfirstlane((unsigned)(a >> 32) & 0xffff),
+               (unsigned)__builtin_amdgcn_readfirstlane(bytes), 0x00020000};
+}
+
+// A 32-row x D tile that NW waves request from memory straight into an image in LDS, N requests of 1 KB a wave (64 chunks of 16 bytes in the
+// image's order; what lies past the descriptor's bytes becomes zeros). Counted by vmcnt; in asm, for hipcc would let every read of LDS
+// wait for all of them.
+template <int D, int NW>
+struct TileRequests {
+  static constexpr int N = D / 16 / NW;
+  static_assert(N * NW * 16 == D, "whole requests");
+  unsigned from_[N];
+  unsigned at_;
+  __device__ __forceinline__ TileRequests(int wave, int lane, long long st) {
 #pragma unroll
-    for (int j = 0; j < CPT; ++j) {
-      const int idx = min(t + NT * j, TOT - 1), row = idx / NCH, ch = idx % NCH;
-      if (j == 0 || !EVEN) vo_[EVEN ? 0 : j] = (int)(((long long)row * st + ch * 8) * 2);
-      lds_[j] = img_off<D>(row, ch);
+    for (int j = 0; j < N; ++j) {
+      const int q = (wave * N + j) * 64 + lane, sub = q / 32, row = sub / (D / 32) * 8 + q % 32 / 4;
+      const int ch = sub % (D / 32) * 4 + ((q & 3) ^ ((row >> 2) & 3));  // img_off's inverse
+      from_[j] = (unsigned)((row * st + ch * 8) * 2);
     }
-    step_ = __builtin_amdgcn_readfirstlane((int)(NT / NCH * st * 2));
-    tail_ = t + NT * (CPT - 1) < TOT;
+    at_ = wave * N * 1024;
   }
-  __device__ __forceinline__ void load(u32x4 (&x)[CPT], __amdgpu_buffer_rsrc_t r, int so) const {
-#pragma unroll
-    for (int j = 0; j < CPT; ++j) {  // (a chunk past the last one is a valid one, never stored)
-      const auto a = __builtin_amdgcn_raw_buffer_load_b128(r, vo_[EVEN ? 0 : j], EVEN ? so + j * step_ : so, 0);
-      x[j] = *reinterpret_cast<const u32x4*>(&a);
-    }
-  }
-  __device__ __forceinline__ void store(const u32x4 (&x)[CPT], char* img) const {
-#pragma unroll
-    for (int j = 0; j < CPT; ++j)
-      if (TOT % NT == 0 || j < CPT - 1 || tail_) *reinterpret_cast<u32x4*>(img + lds_[j]) = x[j];
+  __device__ __forceinline__ void operator()(const u32x4& words, char* image, int so, int j) const {  // request j
+#if defined(__HIP_DEVICE_COMPILE__)
+    const unsigned to = (unsigned)(size_t)(__attribute__((address_space(3))) char*)image + at_ + j * 1024;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(to)),
+                 "v"(from_[j]), "s"(words), "s"(so)
+                 : "m0");
+#else
+    *reinterpret_cast<u32x4*>(image + at_ + j * 1024 + threadIdx.x % 64 * 16) = u32x4{};  // (what a trace of LDS accesses on the host sees)
+#endif
   }
 };
+
+// All but the wave's last N requests have landed, its LDS reads are done, and so are all other waves'.
+template <int N>
+__device__ __forceinline__ void wait_and_meet() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+#else
+  __syncthreads();
+#endif
+}
 
 template <int D>
 __device__ __forceinline__ void clear(f32x16 (&acc)[D / 32]) {

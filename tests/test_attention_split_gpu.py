@@ -45,6 +45,28 @@ def test_two_groups(D, S):
     _check(B, S, S + 37, H, 1, D, True)
 
 
+@pytest.mark.parametrize("D", [64, 96, 128])
+@pytest.mark.parametrize("S", [127, 193, 225, 257, 290])
+def test_tiles_in_turn(D, S):
+    """Walks of 1 to 10 tiles over the places that they take in turn, one group and two."""
+    for B, H in ((6, 48), (1, 2)):
+        _check(B, S, S, H, H, D, True)
+        _check(B, S, S, H, H, D, True, alibi=True)
+
+
+@pytest.mark.parametrize("D", [64, 96, 128])
+@pytest.mark.parametrize("B,H", [(2, 3), (13, 48)])
+def test_rows_past_the_length_are_not_read(D, B, H):
+    """What lies behind a sequence's length may be anything."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q, k, v = (torch.randn(B, 200, H, D, device="cuda", generator=g).bfloat16() for _ in range(3))
+    ln = torch.tensor([200 - 17 * (b % 12) for b in range(B)], device="cuda", dtype=torch.int32)
+    gone = torch.arange(200, device="cuda")[None] >= ln[:, None]
+    want = flash_attention(q, k, v, causal=True, kv_len=ln)
+    k[gone], v[gone] = float("nan"), float("inf")
+    assert torch.equal(flash_attention(q, k, v, causal=True, kv_len=ln), want)
+
+
 def test_eight_waves_dkdv():
     """128-wide heads between the two: dK/dV of 128 keys in two groups of four waves."""
     _check(5, 400, 400, 10, 10, 128, True)
