@@ -74,13 +74,14 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_fwd_split_kernel(FastF
   const bf16_t* qp = p.q + b * p.q_sb + h * p.q_sh;
   const int val = rw / (RW / 2);  // 0: this wave requests keys, 1: values
   const long long rst = val ? p.v_st : p.k_st;
-  const u32x4 words = val ? head_words(p.v + b * p.v_sb + hk * p.v_sh, rows_bytes(kv_end, p.v_st, D))
-                          : head_words(p.k + b * p.k_sb + hk * p.k_sh, rows_bytes(kv_end, p.k_st, D));
+  const u32x4 words = head_words(val ? p.v + b * p.v_sb + hk * p.v_sh : p.k + b * p.k_sb + hk * p.k_sh, rows_bytes(kv_end, rst, D));
   const Req req(rw % (RW / 2), lane, rst);
   char* const kbuf = smem + g * 2 * NB * TILE;
   char* const vbuf = kbuf + NB * TILE;
   char* const ring = val ? vbuf : kbuf;
-  auto request = [&](int i, int place, int j) { req(words, ring + place * TILE, __builtin_amdgcn_readfirstlane(key0(i) * (int)rst * 2), j); };
+  auto request = [&](int i, int place, int j) {  // (past the walk its last tile, which nobody reads)
+    req(words, ring + place * TILE, __builtin_amdgcn_readfirstlane(key0(i) * (int)rst * 2), j);
+  };
   auto requests = [&](int i, int place) {
 #pragma unroll
     for (int j = 0; j < Req::N; ++j) request(i, place, j);
@@ -343,8 +344,7 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dq_split_kernel(Fa
   const bf16_t* gp = p.dout + b * p.do_sb + h * p.do_sh + (long long)qr * p.do_st;
   const int val = rw / (RW / 2);  // 0: this wave requests keys, 1: values
   const long long rst = val ? p.v_st : p.k_st;
-  const u32x4 words = val ? head_words(p.v + b * p.v_sb + hk * p.v_sh, rows_bytes(kv_end, p.v_st, D))
-                          : head_words(p.k + b * p.k_sb + hk * p.k_sh, rows_bytes(kv_end, p.k_st, D));
+  const u32x4 words = head_words(val ? p.v + b * p.v_sb + hk * p.v_sh : p.k + b * p.k_sb + hk * p.k_sh, rows_bytes(kv_end, rst, D));
   const Req req(rw % (RW / 2), lane, rst);
   char* const kbuf = smem + g * 2 * NB * TILE;
   char* const vbuf = kbuf + NB * TILE;
@@ -722,16 +722,21 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
 }  // namespace
 
 // Which calls are split in two groups (two waves of 32 rows each, 4 waves a workgroup), the others in blocks of 128 rows and
-// one group: up to so many 128-row blocks of all heads, the more the longer the longest walk is (keys that a row sees; dK/dV: queries),
-// for a split costs each of its blocks the meeting of the sums. One MI355X, us, one group against two:
-//   forward, 64 wide:   32 rows, 60 blocks 5.0, 5.6, 288 5.9, 6.8 (one tile is nothing to split); 48 rows, 288 7.2, 7.1; 128 rows, 340
-//                       10.5, 10.5, 400 10.6, 13.2; 512 rows, 400 15.3, 15.3, 480 15.2, 18.1; 1024 rows, 400 22.5, 18.7, 480 22.5, 23.2;
-//                       3 x 2048 x 12 (576) 39.2, 35.2; 3000 rows with a window of 256, 336 18.7, 15.0, 408 19.3, 19.7
-//   96 wide:            128 rows, 100 9.5, 8.7, 140 10.0, 10.6; 256 rows, 140 12.6, 11.5, 180 13.0, 13.4; 512 rows, 220 18.3, 16.9, 260
-//                       19.1, 19.3; 1024 rows, 336 28.4, 26.7, 400 28.9, 30.0; 1 x 1403 x 32 (352) 33.8, 31.2
-//   128 wide:           128 rows, 100 10.3, 9.5, 140 10.8, 11.6, 260 14.0, 18.6; 256 rows, 140 13.8, 13.2, 180 14.1, 14.7; 512 rows, 220
-//                       19.7, 19.4, 260 20.4, 21.5; 1024 rows, 304 29.8, 27.9, 336 30.1, 30.6
-//   dQ follows the same lines.
+// one group: up to so many blocks of 64 rows of all heads, the more the longer the longest walk is (keys that a row sees; dK/dV: queries),
+// for a split costs each of its blocks the meeting of the sums. Past the workgroups that run at one time (768 of 64-wide heads, 512 of
+// others) a last round of a few loses more than it saves. One MI355X, us with one group, and what two take, at so many blocks of 64 rows:
+//   forward, 64 wide:   96 rows, 200 6.8, 6.7, 280 6.9, 7.4; 130 rows, 510 9.2, 8.5; 200 rows, 680 9.9, 10.0, 800 10.1, 12.3; 400 rows, 700 12.4, 11.6;
+//                       768 rows, 684 17.1, 16.7, 804 19.2, 20.3; 1200 rows, 760 20.1, 16.8, 912 20.4, 20.7; 2048 rows, 672 29.7, 26.8, 800 31.2,
+//                       36.0; 2600 rows, 656 34.5, 24.6, 779 36.0, 37.9
+//   96 wide:            96 rows, 200 7.9, 7.9, 280 8.1, 9.3; 200 rows, 280 10.0, 9.9, 360 10.1, 10.6; 320 rows, 500 12.7, 12.3, 565 12.7, 15.8;
+//                       512 rows, 440 14.3, 13.0, 520 14.6, 16.0; 1024 rows, 512 20.6, 17.6, 608 21.4, 22.0; 1500 rows, 528 26.6, 26.3, 600 30.0, 33.4; 2048
+//                       rows, 512 32.4, 25.5, 608 34.4, 41.3
+//   128 wide:           96 rows, 200 8.4, 8.4; 200 rows, 280 10.8, 10.6, 360 11.0, 11.8; 256 rows, 280 12.2, 11.5, 360 12.5, 13.2; 512 rows, 440 17.9,
+//                       17.8, 520 18.8, 20.5; 900 rows, 480 21.7, 17.1; 1024 rows, 608 26.5, 25.9, 672 27.0, 28.0; 2048 rows, 672 42.2, 40.9, 800 45.4, 53.5
+//   dQ, what two save:  64 wide, 96 rows, 200 0.2, 280 -1.0; 400 rows, 700 1.0; 768 rows, 516 1.9, 600 -1.0; 1024 rows, 608 0.6, 672 -0.8; 1200 rows, 760 4.4, 912
+//                       0.9; 2048 rows, 512 10.1, 608 -0.2; 2600 rows, 779 11.5; 96 wide, 200 rows, 200 1.1, 280 -1.3; 512 rows, 440 1.0, 520 -1.8;
+//                       768 rows, 516 2.4, 600 -3.8; 1024 rows, 608 2.7, 672 -1.4; 2048 rows, 672 6.2, 800 0.6; 128 wide, 200 rows, 200 1.0, 280 -0.4;
+//                       512 rows, 440 0.5, 520 -1.1; 1024 rows, 512 3.5, 608 -1.9; 2048 rows, 672 2.6, 800 -4.8
 struct Upto { int walk, blocks; };
 template <int N>
 static int blocks_upto(const Upto (&t)[N], int walk) {
@@ -740,38 +745,49 @@ static int blocks_upto(const Upto (&t)[N], int walk) {
     if (walk >= u.walk) b = u.blocks;
   return b;
 }
-static bool split_rows(long long blocks, int d, int keys, int window) {
-  static const Upto t64[] = {{33, 340}, {512, 400}, {1536, 640}};
-  static const Upto t96[] = {{65, 100}, {129, 140}, {384, 220}, {768, 300}, {1024, 336}, {1400, 400}};
-  static const Upto t128[] = {{65, 100}, {129, 140}, {384, 180}, {512, 220}, {768, 260}, {1024, 320}};
+static long long halves(int rows, int heads) { return (rows + 63ll) / 64 * heads; }
+static bool split_rows(int rows, int heads, int d, int keys, int window, bool dq) {
+  static const Upto f64[] = {{33, 200}, {97, 620}, {640, 700}, {1000, 768}};
+  static const Upto f96[] = {{65, 200}, {97, 260}, {129, 320}, {300, 520}};
+  static const Upto f128[] = {{97, 280}, {256, 320}, {512, 450}, {900, 620}, {1400, 660}};
+  static const Upto q64[] = {{33, 200}, {129, 560}};
+  static const Upto q96[] = {{65, 200}, {97, 260}, {240, 340}, {300, 480}, {640, 520}, {900, 620}, {1400, 700}};
+  static const Upto q128[] = {{65, 200}, {97, 250}, {300, 300}, {440, 480}, {900, 520}, {1400, 670}};
   const int walk = window > 0 ? min(keys, window) : keys;
-  return blocks <= (d == 64 ? blocks_upto(t64, walk) : d == 96 ? blocks_upto(t96, walk) : blocks_upto(t128, walk));
+  const long long n = halves(rows, heads);
+  if (dq) return n <= (d == 64 ? walk > 128 && rows % 128 ? 790 : blocks_upto(q64, walk) : d == 96 ? blocks_upto(q96, walk) : blocks_upto(q128, walk));
+  return n <= (d == 64 ? blocks_upto(f64, walk) : d == 96 ? blocks_upto(f96, walk) : blocks_upto(f128, walk));
 }
-// dK/dV with one group or two, or, 128 wide, 0, 1 or in two groups of four waves (2): there two groups of two take 81 KB of LDS, one
-// workgroup a CU. us, backward with one group, and what two groups (of four waves) take or save:
-//   64 wide:   32 rows, 60 blocks 10.2, +0.3, 340 12.9, +0.6; 64 rows, 120 11.8, -0.4; (dK/dV alone, one, two) 256 rows, 192 11.9, 11.3, 264
-//              13.0, 13.5; 500 rows, 288 19.6, 18.5; 768 rows, 432 28.5, 27.3; 1400 rows, 528 47.0, 45.4; 2048 rows, 576 68.5, 66.1, 768 74.8,
-//              87.0; a window of 256, 288 20.2, 18.2, 336 41.6, -2.6, 480 43.8, +5.8
-//   96 wide:   64 rows, 60 blocks 13.9, -1.3, 1200 50.2, -3.9; 32 rows, 340 15.2, -0.4; a window of 32 or 64, 120 25, -5, 224 28, -2.5, 340 35,
-//              +1, 480 41, +3; 128 rows, 220 23.8, -0.4, 260 30.2, +2.5; 512 rows, 300 47.4, -1.7, 340 48.5, +0.3; 1024 rows, 480 80.5, -0.8
-//   128 wide:  32 rows, 60 blocks 12.7, +0.4; 64 rows, 220 17.5, -0.9, 260 22.1, +3.4; 128 rows, 100 23.0, -1.0 (+0.6), 140 25.0,
-//              +3.6 (+0.7); 256 rows, 140 33.7, -1.3 (-0.4), 180 34.3, +1.2 (0); 512 rows, 180 48.9, -2.8 (-2.0), 260 54.6, +4.5
-//              (-3.8), 340 57.1, +8.0 (+2.3); 1024 rows, 256 80.0, -7.4 (-7.1), 304 87.4, +2.4 (-9.3), 480 99.2, +17 (-3.9), 560 108,
-//              +28 (+6.7); 1 x 2944 x 20 (460) 246, +29 (-37); a window of 256, 96 40.2, -7.1 (-2.2), 144 43.1, +2.5 (-2.3), 264
-//              48.3, +7.8 (+3.0)
-static int split_keys(long long blocks, int d, int rows, int window, bool alibi) {
-  static const Upto t64[] = {{33, 200}, {400, 340}, {512, 480}, {768, 560}, {1536, 680}};  // (the form START; with ALiBi or a window:)
+// dK/dV with one group or two, or, 128 wide, 0, 1 or in two groups of four waves (2, by blocks of 128 rows): there two groups of two take 81 KB of
+// LDS, one workgroup a CU. us, backward with one group, and what two groups (of four waves) take or save:
+//   64 wide:   96 rows, 600 blocks of 64 rows 18.8, -0.5, 680 18.7, +0.2; 200 rows, 680 22.9, -0.7, 800 23.3, +1.1; 512 rows, 800 37.0, -1.4, 960 37.3,
+//              +0.9; 768 rows, 516 42.9, -3.8, 600 43.5, +1.0; 1200 rows, 760 59.1, -5.5, 912 61.3, -2.9; 1500 rows, 960 75.0, -4.9, 1128 83.6, +1.5;
+//              2048 rows, 512 84.0, -12.7, 608 94.1, +0.5; 2600 rows, 943 119, -7.1 (before tiles went straight into LDS:) a window of 256, 576 20.2,
+//              18.2, 672 41.6, -2.6, 960 43.8, +5.8
+//   96 wide:   96 rows, 200 17.4, -0.8, 280 18.0, +0.3; 200 rows, 440 25.0, -0.6, 520 28.7, +1.5; 320 rows, 500 32.5, -3.5, 565 32.3, +2.7; 512 rows, 520
+//              38.8, -0.9, 600 41.2, +0.5; 768 rows, 684 52.8, -0.8, 804 55.7, +2.1; 1024 rows, 672 64.5, -4.5, 800 67.3, -0.9; 1500 rows, 960 96.8,
+//              -1.9, 1128 110, +8; 2048 rows, 800 119, -9, 960 127, +6; (before:) 64 rows, 60 13.9, -1.3, 1200 50.2, -3.9; a window of 32 or 64, 240
+//              25, -5, 448 28, -2.5, 680 35, +1
+//   128 wide:  200 rows, 200 26.0, -1.9 (-1.0), 280 26.9, -0.3 (-0.5); 256 rows, 200 29.3, -2.6 (-1.6), 280 30.5, +1.3 (-1.5), 360 31.9, +2.9 (-1.4), 520
+//              37.4, +10 (+4.7); 512 rows, 280 43.1, -4.8 (-4.1), 360 44.0, -0.9 (-3.8), 520 48.9, +7.8 (-2.2), 600 51.0, +9.7 (+0.6); 768 rows, 960
+//              75.6, +16 (-2.1), 1116 87, +27 (+6); 1024 rows, 352 67.1, -10.6 (-8.7), 448 67.4, -4.7 (-7.6), 672 77.9, +8.5 (-6.6); 1200 rows, 912 94.3,
+//              +18 (-5.4); 2048 rows, 352 116, -22 (-19), 448 117, -16 (-17), 1120 170, +35 (-2.0), 1280 172, +43 (+1.7); (before:) 32 rows, 60 12.7,
+//              +0.4; 64 rows, 220 17.5, -0.9; a window of 256, 192 40.2, -7.1 (-2.2), 288 43.1, +2.5 (-2.3), 528 48.3, +7.8 (+3.0)
+static int split_keys(int keys, int heads, int d, int rows, int window, bool alibi) {
+  static const Upto t64[] = {{33, 320}, {65, 640}, {129, 690}, {256, 900}};  // (the form START; with ALiBi or a window, in blocks of 128 rows:)
   static const Upto m64[] = {{33, 340}, {512, 480}, {768, 560}, {1536, 768}};
-  static const Upto t96[] = {{0, 760}, {65, 220}, {384, 280}, {768, 380}, {1024, 480}};
-  static const Upto t128[] = {{33, 220}, {65, 100}, {129, 140}, {384, 180}, {768, 220}};
-  static const Upto w128[] = {{384, 260}, {512, 300}, {768, 400}, {1024, 512}};
+  static const Upto t96[] = {{0, 760}, {65, 210}, {97, 430}, {256, 510}, {512, 600}, {768, 700}, {1400, 860}};
+  static const Upto t128[] = {{33, 220}, {65, 120}, {97, 250}, {300, 290}, {768, 350}, {1400, 420}};
+  static const Upto w128[] = {{129, 220}, {256, 240}, {384, 260}, {600, 320}, {768, 480}, {1800, 560}};
   const bool win = window > 0 && window < rows;
   const int walk = win ? window : rows;
+  const long long blocks = (keys + 127ll) / 128 * heads, n = halves(keys, heads);
   if (d == 128 && win) return blocks <= 120 ? 1 : blocks <= 220 ? 2 : 0;
-  const int upto = d == 96    ? (win && walk < 65 ? 280 : blocks_upto(t96, walk))
+  if (d == 64 && (alibi || window > 0)) return blocks <= blocks_upto(m64, walk);
+  const int upto = d == 96    ? (win && walk < 65 ? 560 : blocks_upto(t96, walk))
                    : d == 128 ? blocks_upto(t128, walk)
-                              : alibi || window > 0 ? blocks_upto(m64, walk) : blocks_upto(t64, walk);
-  if (blocks <= upto) return 1;
+                              : walk >= 700 && keys % 128 == 0 ? 560 : blocks_upto(t64, walk);
+  if (n <= upto) return 1;
   return d == 128 && blocks <= blocks_upto(w128, walk) ? 2 : 0;
 }
 
@@ -795,7 +811,7 @@ static int with_form(int d, bool alibi, F&& f) {
 // the same: 1 x 1500 x 64 forward 53 -> 46 us, backward 139 -> 134. Windowed dQ, all blocks alike, is 2 % faster with two.)
 int attn_fwd_split(const FastFwdParams& p, int d, hipStream_t stream) {
   const long long blocks = (long long)((p.Sq + 127) / 128) * p.B * p.H;
-  const bool two = split_rows(blocks, d, p.Sk, p.window);
+  const bool two = split_rows(p.Sq, p.B * p.H, d, p.Sk, p.window, false);
   return with_form(d, p.alibi, [&](auto D_, auto G_) {
     constexpr int D = decltype(D_)::value, G = decltype(G_)::value, W = D == 64 ? 3 : 2;
     if (two)
@@ -808,8 +824,8 @@ int attn_fwd_split(const FastFwdParams& p, int d, hipStream_t stream) {
 int attn_bwd_split(const FastBwdParams& p, int d, hipStream_t stream) {
   if (!(fabsf(p.scale) >= 1e-30f)) return 1;  // the sums start with lse / scale: the generic kernel's
   const long long qblocks = (long long)((p.Sq + 127) / 128) * p.B * p.H, kblocks = (long long)((p.Sk + 127) / 128) * p.B * p.Hkv;
-  const bool two = split_rows(qblocks, d, p.Sk, p.window);
-  const int kv = split_keys(kblocks, d, p.Sq, p.window, p.alibi);
+  const bool two = split_rows(p.Sq, p.B * p.H, d, p.Sk, p.window, true);
+  const int kv = split_keys(p.Sk, p.B * p.Hkv, d, p.Sq, p.window, p.alibi);
   return with_form(d, p.alibi, [&](auto D_, auto G_) {
     constexpr int D = decltype(D_)::value, G = decltype(G_)::value, W = D == 64 ? 3 : 2;
     if (two)

@@ -220,7 +220,8 @@ __device__ __forceinline__ u32x4 head_words(const bf16_t* b, int bytes) {
 
 // A 32-row x D tile that NW waves request from memory straight into an image in LDS, N requests of 1 KB a wave (64 chunks of 16 bytes in the
 // image's order; what lies past the descriptor's bytes becomes zeros). Counted by vmcnt; in asm, for hipcc would let every read of LDS
-// wait for all of them.
+// wait for all of them. Five wait states stand before the request: a vector instruction may have written its scalars (readfirstlane, a
+// spilled scalar), and in asm nobody else keeps the distance.
 template <int D, int NW>
 struct TileRequests {
   static constexpr int N = D / 16 / NW;
@@ -239,7 +240,7 @@ struct TileRequests {
   __device__ __forceinline__ void operator()(const u32x4& words, char* image, int so, int j) const {  // request j
 #if defined(__HIP_DEVICE_COMPILE__)
     const unsigned to = (unsigned)(size_t)(__attribute__((address_space(3))) char*)image + at_ + j * 1024;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(to)),
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(to)),
                  "v"(from_[j]), "s"(words), "s"(so)
                  : "m0");
 #else

@@ -1008,10 +1008,11 @@ __device__ __forceinline__ void expert_turns_tile(const ExpertArgs& p, char* sl,
     from_x[i] = ((unsigned)(UP ? p.perm[lo + xr] / p.top : xr) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
   }
   const unsigned base = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) char*)sl);
-  // (in asm: hipcc would let every read of LDS wait for all requests. Nothing is returned to a register)
+  // (in asm: hipcc would let every read of LDS wait for all requests. Nothing is returned to a register. Five wait states after what may be a
+  // vector write of a scalar)
   auto request = [&](const u32x4& rsrc, unsigned at, unsigned from, int t) {
     const int k = __builtin_amdgcn_readfirstlane(min(t, nk - 1) * GBK * 2);  // past the end: the last one, which nobody reads
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(at)),
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(at)),
                  "v"(from), "s"(rsrc), "s"(k)
                  : "m0");
   };

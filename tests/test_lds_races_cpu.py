@@ -70,6 +70,20 @@ def test_asm_names_the_registers_that_it_writes():
                     assert "s_mov_b32 m0" not in stmt or re.search(r':\s*"m0"', stmt), (f, stmt)
 
 
+def test_asm_requests_keep_their_distance():
+    """Five wait states between a vector write of a scalar and a memory request that reads it: in asm the compiler adds none."""
+    seen = 0
+    for d in ("kernels", "comm"):
+        for f in os.listdir(os.path.join(ROOT, "csrc", d)):
+            with open(os.path.join(ROOT, "csrc", d, f)) as src:
+                for stmt in re.findall(r"\basm volatile\((?:[^;]|\n)*?\);", src.read()):
+                    if "buffer_load" in stmt and "lds" in stmt:
+                        seen += 1
+                        before = re.search(r"s_mov_b32 m0, %0.*?s_nop (\d+).*?buffer_load", stmt)
+                        assert before and int(before.group(1)) >= 3, (f, stmt)
+    assert seen >= 2
+
+
 def test_a_flag_is_lowered_before_the_first_bare_barrier():
     """A bare barrier waits for no LDS access: what one wave has written before it and others write after it needs a wait."""
     with open(os.path.join(ROOT, "csrc", "kernels", "attention_tiled.hip")) as f:
