@@ -281,27 +281,38 @@ __device__ __forceinline__ void group_rows(const GroupArgs& p, int* sh) {
     unsigned to = 0, to2 = 0;  // mt 256: four sums in 16 bits each (tiles are fewer than 32768), of experts whose largest tile is 4 .. 1 units
     for (int e0 = 0; e0 < E; e0 += 64) {
       const int e = e0 + tid, c = e < E ? cnt[e] : 0, small = late_tile(c, mt);
-      const Cut k = cut(c);
-      const int b = 4 - k.per - (k.more > 0);
-      const unsigned t = mt == 256 ? (b < 2 ? k.tiles << 16 * b : 0) : (c + mt - 1) / mt - small, t2 = b < 2 ? 0 : k.tiles << 16 * (b & 1);
-      int cs = c;
+      const unsigned before2 = to2;
+      int cs = c, b = 0;
+      unsigned t = (c + mt - 1) / mt - small, t2 = 0;
+      if (mt == 256) {
+        const Cut k = cut(c);
+        b = 4 - k.per - (k.more > 0);
+        t = b < 2 ? k.tiles << 16 * b : 0, t2 = b < 2 ? 0 : k.tiles << 16 * (b & 1);
+      }
       unsigned ts = t, ts2 = t2;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
         const int a = __shfl_up(cs, o, 64);
-        const unsigned b1 = __shfl_up(ts, o, 64), b2 = __shfl_up(ts2, o, 64);
-        if (tid >= o) cs += a, ts += b1, ts2 += b2;
+        const unsigned b1 = __shfl_up(ts, o, 64);
+        if (tid >= o) cs += a, ts += b1;
+      }
+      if (mt == 256) {
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+          const unsigned b2 = __shfl_up(ts2, o, 64);
+          if (tid >= o) ts2 += b2;
+        }
+        to2 += __shfl(ts2, 63, 64);
       }
       const unsigned long long m = __ballot(small);
       if (e < E) {
-        const unsigned u = to + ts - t, u2 = to2 + ts2 - t2;
+        const unsigned u = to + ts - t, u2 = before2 + ts2 - t2;
         off[e] = co + cs - c;
         toff[e] = mt == 256 ? (b < 2 ? u : u2) >> 16 * (b & 1) & 0xffff : u;
         soff[e] = mt == 256 ? b : so + __popcll(m & ((1ull << tid) - 1));
       }
       co += __shfl(cs, 63, 64);
       to += __shfl(ts, 63, 64);
-      to2 += __shfl(ts2, 63, 64);
       so += __popcll(m);
     }
     if (mt == 256) {  // largest tiles first
@@ -314,7 +325,7 @@ __device__ __forceinline__ void group_rows(const GroupArgs& p, int* sh) {
   __syncthreads();
   for (int e = tid; e < E; e += NT) {
     const int c = cnt[e], nt = (c + mt - 1) / mt, small = late_tile(c, mt);
-    const Cut k = cut(c);
+    const Cut k = mt == 256 ? cut(c) : Cut{0, 0, 0};
     for (int j = 0; j < nt; ++j) {
       const bool last = small && j == nt - 1;  // (it stands alone)
       const int at = last ? toff[E] + soff[e] : toff[e] + j;
@@ -657,16 +668,20 @@ __global__ void __launch_bounds__(256) expert_gemv_kernel(ExpertArgs p) {
 }
 
 // ---------------------------------------------------------------------------------------------- stream
-// bf16, tiles of up to 32 rows x 128 weight rows (up: 64 gate rows and the 64 up rows beside them) x 64 per stage,
-// 4 waves of 32 weight rows. Bound by the weight stream: a stage's 16 KiB of weights and 4 KiB of activations go
-// straight to LDS (no registers, so three stages a workgroup and two workgroups a CU are in flight, 120 KiB), and
-// the products (16x16x32 tiles, weights as the A operand: a lane holds one activation row and four outputs) hide
-// under it. Beside the gemv kernel, whose vector products a row cost more than its weights from about 4 rows an
-// expert on, and the gemm, which computes and stages mostly padding: both products of 32 tokens, 16 experts of
-// 3 x 4096 x 2048, top 3: 190 us (gemv), 192 (gemm), 172 (4.7 TB/s); 100 tokens 450, 197, 175 (tile_rows in ops/moe.py).
+// bf16, tiles of up to 32 rows x 32 weight rows (up: 16 gate rows and the 16 up rows beside them), 4 waves, each with every fourth stage
+// of 64 of K; the waves' sums meet in LDS. Bound by the weight stream. How fast memory gives it hangs on how far apart the rows lie that
+// the chip reads at one time: blocks of 64 rows that walk K by themselves have the whole of a weight in flight, 4.7 to 4.9 TB/s (50432 x
+// 4096, loads alone), of 32 rows, K over the waves, 6.0; the number of bytes in flight and the length of a request's rows make no
+// difference. A wave's stages go straight to LDS, weights three stages ahead, activations, in the XCD's cache, two; no wave
+// waits for another before the end, and two workgroups a CU cover each other's ramps. Beside the gemv kernel, whose vector products a row
+// cost more than its weights from about 2 rows an expert on, and the gemm, which computes and stages mostly padding.
+// Both products of a layer, us, blocks of 64 weight rows that walk K by themselves (the form before) and this: 20 outputs, 16 experts of 3 x
+// 4096 x 2048, top 3: 20 tokens 163, 142, 64 173, 143; 32 of 3 x 2048 x 1024, top 4: 64 85, 80; 16 of 3 x 4096 x 4096, top 2: 32 282,
+// 274, 130 295, 278. Workgroups in plain order 149, 87, 281, 307; an XCD a contiguous eighth of the blocks 161, 84, 278, 301; runs of
+// 512 151, 83, 293, 308; a fourth weight stage, one workgroup a CU, 172, 102, 285, 310.
 // K % 64 == 0 and N % 16 == 0; an LDS-DMA instruction fills 8 rows of 128 bytes lane by lane, so the 16-byte pieces
 // are swizzled (by row pair: 16 rows x one piece cover all 64 banks) on the source address.
-constexpr int SROWS = 32, SK = 64, SWN = 128, SST = (SWN + SROWS) * SK * 2, SNB = 4, STREAM_LDS = SNB * SST;
+constexpr int SROWS = 32, SK = 64, SWN = 32;
 
 // `bytes`: loads past them return zeros
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rsrc(const void* p, unsigned bytes = ~0u) {
@@ -683,115 +698,129 @@ __device__ __forceinline__ u32x4 uniform_words(const void* p) {
                0x00020000};
 }
 
-// four 16-byte LDS reads and their wait in one piece (hipcc would drain every LDS-DMA in flight before a read it sees)
-__device__ __forceinline__ void lds_read4(unsigned a0, unsigned a1, unsigned a2, unsigned a3, u32x4& r0, u32x4& r1,
-                                          u32x4& r2, u32x4& r3) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile(
-      "ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %6\n\tds_read_b128 %3, %7\n\ts_waitcnt lgkmcnt(0)"
-      : "=&v"(r0), "=&v"(r1), "=&v"(r2), "=&v"(r3)
-      : "v"(a0), "v"(a1), "v"(a2), "v"(a3)
-      : "memory");
-#endif
-}
-
-template <bool UP>
-__global__ void __launch_bounds__(256, 2) expert_stream_kernel(ExpertArgs p) {
-  extern __shared__ __attribute__((aligned(1024))) char sl[];  // [SNB][128 weight rows | 32 activation rows][128 B]
-  constexpr int NB = UP ? SWN / 2 : SWN;
-  const int nt = *p.ntiles, nb = (p.N + NB - 1) / NB;
-  if ((int)blockIdx.x >= nt * nb) return;
-  const int id = xcd_remap(blockIdx.x, nt * nb);  // the order of expert_gemm_kernel
-  const int* t0 = p.tiles + id / nb * 5;
-  const int in = id - t0[3] * nb, tile = t0[3] + in % t0[4], bn = in / t0[4];
-  const int* tl = p.tiles + tile * 5;
-  const int ex = tl[0], lo = tl[1], nr = tl[2], K = p.K, N = p.N, n0 = bn * NB;
+// rows: 8, 16 or 32 of activations (XI requests a stage)
+template <bool UP, int XI>
+__device__ __forceinline__ void expert_stream_tile(const ExpertArgs& p, char* sl, int ex, int lo, int nr, int n0) {
+  constexpr int XB = XI > 2 ? 2 : 1, NW = 3, NX = 2, OWN = NW * 4096 + NX * XI * 1024;  // runs of 16 rows; places; a wave's bytes
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int r16 = lane & 15, g = lane >> 4;
-  // sources: a wave fills its own 32 weight rows (4 pieces of 8) and 8 of the activation rows
-  const __amdgpu_buffer_rsrc_t rw =
-      uniform_rsrc(reinterpret_cast<const bf16_t*>(p.w) + (long long)ex * (UP ? 2 * N : N) * K);
-  const __amdgpu_buffer_rsrc_t rx = uniform_rsrc(reinterpret_cast<const bf16_t*>(p.x) + (UP ? 0ll : (long long)lo * K));
-  unsigned wo[4], xo;
+  const int r16 = lane & 15, g = lane >> 4, K = p.K, N = p.N;
+  const u32x4 rw = uniform_words(reinterpret_cast<const bf16_t*>(p.w) + (long long)ex * (UP ? 2 * N : N) * K);
+  const u32x4 rx = uniform_words(reinterpret_cast<const bf16_t*>(p.x) + (UP ? 0ll : (long long)lo * K));
+  unsigned wo[4], xo[XI];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int r = 8 * i + (lane >> 3);  // of the wave's 32
-    const int n = UP ? (r < 16 ? 0 : N) + min(n0 + wv * 16 + (r & 15), N - 1) : min(n0 + wv * 32 + r, N - 1);
+    const int r = 8 * i + (lane >> 3), n = UP ? (i < 2 ? 0 : N) + n0 + (r & 15) : min(n0 + r, N - 1);
     wo[i] = ((unsigned)n * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
   }
-  {
-    const int r = wv * 8 + (lane >> 3), xr = min(r, nr - 1);
-    xo = ((unsigned)(UP ? p.perm[lo + xr] / p.top : xr) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
-  }
-  typedef __attribute__((address_space(3))) char lds_char;
-  lds_char* lsm = (lds_char*)sl;
-  const int nk = K / SK;
-  auto issue = [&](int t) {
-    const int k = __builtin_amdgcn_readfirstlane(min(t, nk - 1) * SK * 2);  // the last stages repeat one that nobody reads
-    lds_char* st = lsm + (t % SNB) * SST;
-#if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (void __attribute__((address_space(3)))*)(st + (wv * 4 + i) * 1024), 16,
-                                               wo[i], k, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (void __attribute__((address_space(3)))*)(st + (16 + wv) * 1024), 16, xo,
-                                             k, 0, 0);
-#endif
+  for (int i = 0; i < XI; ++i) {
+    const int r = 8 * i + (lane >> 3), xr = min(r, nr - 1);
+    xo[i] = ((unsigned)(UP ? p.perm[lo + xr] / p.top : xr) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
+  }
+  const int nk = K / SK, last = nk > wv ? (nk - 1 - wv) / 4 * 4 + wv : 0;  // the wave's last stage
+  char* const own = sl + wv * OWN;
+  const unsigned base = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) char*)own);
+  auto request = [&](const u32x4& rsrc, unsigned at, unsigned from, int k) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(at)),
+                 "v"(from), "s"(rsrc), "s"(k)
+                 : "m0");
   };
-  f32x4 acc[2][2];  // [gate, up | two runs of 16 outputs][16 rows]
+  auto stage_k = [&](int t) { return __builtin_amdgcn_readfirstlane(min(4 * t + wv, last) * SK * 2); };  // past the end: one that nobody reads
+  auto weights = [&](int t, int place) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) request(rw, base + place * 4096 + i * 1024, wo[i], stage_k(t));
+  };
+  auto rows = [&](int t, int place) {
+#pragma unroll
+    for (int i = 0; i < XI; ++i) request(rx, base + NW * 4096 + (place * XI + i) * 1024, xo[i], stage_k(t));
+  };
+  f32x4 acc[2][XB];  // [gate, up | two runs of 16 outputs][16 rows]
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < XB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int sw = (r16 >> 1) & 7;
+  rows(0, 0);
+  weights(0, 0);
+  rows(1, 1);
+  weights(1, 1);
+  weights(2, 2);
+  int pw = 0, px = 0;
+  for (int t = 0; 4 * t + wv < nk; ++t) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 + XI) : "memory");  // stage t has landed; weights t + 1, t + 2 and rows t + 1 may be on their way
+    bf16x8 a[2][2], x[2][XB];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[i][j][e] = 0.f;
-  const unsigned base = (unsigned)(size_t)lsm, sw = (r16 >> 1) & 7;
-  const unsigned aw = (wv * 32 + r16) * 128, ax = (SWN + r16) * 128;
+    for (int s = 0; s < 2; ++s) {
+      const int c = ((4 * s + g) ^ sw) * 16;
 #pragma unroll
-  for (int t = 0; t < SNB - 1; ++t) issue(t);
-  for (int t = 0; t < nk; ++t) {
-    // this wave's pieces of stage t have landed (two younger stages may be in flight), then everybody's
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SNB - 2) * 5) : "memory");
-    __builtin_amdgcn_s_barrier();
-    issue(t + SNB - 1);  // into the buffer of stage t - 1, which all waves have left
-    const unsigned st = base + (t % SNB) * SST;
+      for (int i = 0; i < 2; ++i) a[s][i] = *reinterpret_cast<const bf16x8*>(own + pw * 4096 + (16 * i + r16) * 128 + c);
 #pragma unroll
-    for (int s = 0; s < SK / 32; ++s) {
-      const unsigned c = ((4 * s + g) ^ sw) * 16;
-      u32x4 a0, a1, x0, x1;
-      lds_read4(st + aw + c, st + aw + 16 * 128 + c, st + ax + c, st + ax + 16 * 128 + c, a0, a1, x0, x1);
-      const bf16x8 A0 = __builtin_bit_cast(bf16x8, a0), A1 = __builtin_bit_cast(bf16x8, a1);
-      const bf16x8 X0 = __builtin_bit_cast(bf16x8, x0), X1 = __builtin_bit_cast(bf16x8, x1);
-      acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A0, X0, acc[0][0], 0, 0, 0);
-      acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A1, X0, acc[1][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A0, X1, acc[0][1], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A1, X1, acc[1][1], 0, 0, 0);
+      for (int j = 0; j < XB; ++j)  // (8 rows: twice)
+        x[s][j] = *reinterpret_cast<const bf16x8*>(own + NW * 4096 + px * XI * 1024 + (16 * j + (XI == 1 ? r16 & 7 : r16)) * 128 +
+                                                   ((4 * s + g) ^ (XI == 1 ? ((r16 & 7) >> 1) : sw)) * 16);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    rows(t + 2, px);
+    weights(t + 3, pw);
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < XB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s][i], x[s][j], acc[i][j], 0, 0, 0);
+    pw = pw == NW - 1 ? 0 : pw + 1;
+    px ^= 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the repeated stages, before their places are used again
+  __syncthreads();
+  f32x4* const part = reinterpret_cast<f32x4*>(sl);  // [run][rows][wave][lane]
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < XB; ++j) part[((i * XB + j) * 4 + wv) * 64 + lane] = acc[i][j];
+  __syncthreads();
+  auto sum = [&](int i, int j) {  // in the order of the waves
+    f32x4 s = part[(i * XB + j) * 256 + lane];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) s += part[((i * XB + j) * 4 + w) * 64 + lane];
+    return s;
+  };
+  if (wv >= (UP ? XB : 2 * XB)) return;
+  const int j = UP ? wv : wv % XB, i = UP ? 0 : wv / XB, r = 16 * j + r16, n = n0 + 16 * i + 4 * g;
+  if (r >= nr || n >= N) return;
+  const float s = p.scale ? p.wts[p.perm[lo + r]] : 1.f;
+  const f32x4 u = sum(i, j), v = UP ? sum(1, j) : u;
+  float o[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if constexpr (UP) {
+      const float gt = u[e] * s, up = v[e] * s;
+      o[e] = gt * __builtin_amdgcn_rcpf(1.f + __expf(-gt)) * up;
+    } else {
+      o[e] = u[e] * s;
     }
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the repeated stages, before the LDS is given back
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int r = 16 * j + r16;
-    if (r >= nr) continue;
-    const float s = p.scale ? p.wts[p.perm[lo + r]] : 1.f;
-    bf16_t* y = reinterpret_cast<bf16_t*>(p.y) + (long long)(lo + r) * N;
-#pragma unroll
-    for (int i = 0; i < (UP ? 1 : 2); ++i) {
-      const int n = n0 + wv * (UP ? 16 : 32) + 16 * i + 4 * g;
-      if (n >= N) continue;
-      float o[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if constexpr (UP) {
-          const float gt = acc[0][j][e] * s, up = acc[1][j][e] * s;
-          o[e] = gt * __builtin_amdgcn_rcpf(1.f + __expf(-gt)) * up;
-        } else {
-          o[e] = acc[i][j][e] * s;
-        }
-      }
-      *reinterpret_cast<uint2*>(y + n) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
-    }
-  }
+  bf16_t* y = reinterpret_cast<bf16_t*>(p.y) + (long long)(lo + r) * N;
+  *reinterpret_cast<uint2*>(y + n) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+}
+constexpr int STREAM_LDS = 4 * (3 * 4096 + 2 * 4 * 1024);
+
+template <bool UP>
+__global__ void __launch_bounds__(256, 2) expert_stream_kernel(ExpertArgs p) {
+  extern __shared__ __attribute__((aligned(1024))) char sl[];
+  constexpr int NB = UP ? SWN / 2 : SWN;
+  const int nt = *p.ntiles, nb = (p.N + NB - 1) / NB;
+  if ((int)blockIdx.x >= nt * nb) return;
+  // Runs of 64 blocks, eight adjacent ones an XCD: what the chip reads at a time stays compact, and an expert's row tiles share an L2
+  const int b = blockIdx.x, end = nt * nb, c = b & ~63;
+  const int id = c + xcd_remap(b - c, min(64, end - c));
+  const int* t0 = p.tiles + id / nb * 5;
+  const int in = id - t0[3] * nb, tile = t0[3] + in % t0[4], bn = in / t0[4];
+  const int* tl = p.tiles + tile * 5;
+  const int nr = tl[2];
+  if (nr <= 8) expert_stream_tile<UP, 1>(p, sl, tl[0], tl[1], nr, bn * NB);
+  else if (nr <= 16) expert_stream_tile<UP, 2>(p, sl, tl[0], tl[1], nr, bn * NB);
+  else expert_stream_tile<UP, 4>(p, sl, tl[0], tl[1], nr, bn * NB);
 }
 
 // ------------------------------------------------------------------------------------------------ gemm

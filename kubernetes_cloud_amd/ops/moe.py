@@ -105,25 +105,32 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
     weight stream on the matrix cores (32), the prompts' product in narrow blocks (128 or 192 rows x 128 weight rows) or
     wide ones (256 x 256). Both products of a layer, us (width, experts, top, inner size; - not measured):
 
-        4096, 16, 2, 4096   tokens   24: vector 270, stream 273     32: 312, 291             100: 716, 296, narrow 302
-                                    160: stream 298, narrow 296    300: 339, 305, wide 306  700: narrow 338, wide 322
+        4096, 16, 2, 4096   tokens   17: vector 226, stream 240     24: 270, 262             32: 314, 278
+                                    100: stream 275, narrow 292    160: 283, 295            260: 352, 301
+                                    300: narrow 305, wide 306      700: 338, 322
                                    1000: narrow 367, wide 333     1300: 377, 339           2500: 610, 505
-        4096, 16, 3, 2048   tokens  300: narrow 182, wide 195     900: 208, 209            1500: 295, 227     3000: 487, 330
-        2048, 32, 4, 1024   tokens   12: vector 71, stream 74       32: 111, 87, narrow -    100: 265, 87, 87
+        4096, 16, 3, 2048   tokens   17: vector 158, stream 135     32: 195, 142             90: stream 146, narrow 173
+        (20 outputs)               160: stream 165, narrow 177    260: 202, 180            300: narrow 182, wide 195
+                                    900: narrow 208, wide 209     1500: 295, 227           3000: 487, 330
+        2048, 32, 4, 1024   tokens   17: vector 83, stream 73       24: 97, 76               100: stream 83, narrow 87
+                                    128: stream 85, narrow 87      200: 92, 89              300: 112, 90
                                     500: narrow 93, wide 103      1150: 115, 115           3000: 211, 172     8192: 511, 406
-        4096, 20, 3, 2048   tokens   24: vector 165, stream 166     32: 190, 172             160: 450 (100), 183, 178
-                                    900: narrow 271, wide 286     1500: 349, 342           3000: 608, 437
-        2048, 24, 5, 768    tokens  400: narrow 73, wide 83        777: 83, 85              1300: 96, 86      2000: 117, 106
-        (32 outputs, uneven)       3000: 141, 143                  4096: 231, 189
+        4096, 20, 3, 2048   tokens  900: narrow 271, wide 286     1500: 349, 342           3000: 608, 437
+        2048, 24, 5, 768    tokens   17: vector 65, stream 47      100: stream 56, narrow 69   200: 67, 74      300: 81, 73
+        (32 outputs, uneven)       400: narrow 73, wide 83        777: 83, 85              1300: 96, 86      2000: 117, 106
+                                   3000: narrow 141, wide 143     4096: 231, 189
+        5120, 8, 2, 2560    tokens   17: vector 144, stream 109    100: stream 134, narrow 149   160: 170, 154
+        1024, 64, 2, 512    tokens   17: vector 27, stream 26       32: 39, 36               64: 58, 45
         2048, 40, 4, 1024   tokens 1200: narrow 142, wide 161     2000: 181, 188           2048, 10, 2, 2048, 600: 84, 90; 2000: 147, 141
         5120, 8, 2, 2560    tokens  400: narrow 183, wide 156     1200: 275, 283           2000: 386, 333
         widths that are no multiple of 64 have no stream; rows an expert, vector against narrow blocks:
         4104, 16, 2, 2056   3: 179, 154   4: 209, 176   8: 335, 180   16: 605, 186     1032, 16, 2, 520   4: 34, 22   16: 89, 22
         4104, 16, 2, 4104   3: 334, 337   4: 376, 329   8: 590, 335   16: 1099, 347    2056, 32, 4, 1032  4: 134, 101
 
-    The stream takes over at about 3 rows, at 2 where a row is short (a vector wave's reduction is then a larger part of
-    its work), but up to 16 tokens the vector product also carries the shared expert. A stream tile holds 32 rows, past
-    which weights are read again, so it ends at 16 rows -- at 64 where narrow blocks are too few to fill the chip. A
+    The stream takes over where an expert expects more than one row, a little past two where rows are long (the vector
+    product's wave then has the longer walk over which to hide its reduction), but up to 16 tokens the vector product also
+    carries the shared expert. A stream tile holds 32 rows, past which weights are read again and a block has twice the
+    work, so it ends at 20 rows, as experts are uneven -- at 36 where narrow blocks are too few to fill the chip. A
     narrow tile of 192 rows saves a second tile a little over 128 rows, if there are blocks enough without it, and costs
     one a little over 192. A wide block is alone on its CU: it wins where the matrix cores bound the products, from
     about 150 rows (64 where a contraction is long), if its rounds are well filled (``fill``: the blocks' time over that
@@ -139,7 +146,7 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
     if gemm and near:
         stream = d % 64 == 0 and F % 64 == 0
         r, short, full = n / used, min(d, F), used * (F // 64) >= 512
-        if r > ((16 if full else 64) if stream else 4):
+        if r > ((20 if full else 36) if stream else 4):
             if stream:
                 tiles = used * -(-r // GEMM_ROWS)
                 up, down = tiles * -(-F // 128), tiles * -(-d // 256)  # wide blocks of the two products; rounds of one a CU
@@ -154,7 +161,7 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
             elif r > 96 and (short >= 4096 or (short >= 1024 and r > 512)):
                 return GEMM_ROWS
             return 192 if (full and 100 < r <= 160) or r > 240 else 128
-        if stream and T > SHARED_ROWS and r > (3 if d > 2048 else 2):
+        if stream and T > SHARED_ROWS and r > (2.25 if d > 2048 else 1):
             return STREAM_ROWS
     return 1 if T == 1 else 2 if T == 2 else 4 if T <= 4 else 8
 

@@ -42,6 +42,20 @@ def test_products(mt, scale_in, counts, top, d, F):
     assert (y.float() - want).norm() <= TOL * want.norm()
 
 
+@pytest.mark.parametrize("d,F", [(64, 128), (192, 256), (320, 576), (1088, 64), (64, 1216)])
+def test_stream_rows(d, F):
+    """Every number of rows a tile's forms end at, with fewer stages of K than waves, one more, and a remainder of them; row by row."""
+    counts = [1, 7, 8, 9, 15, 16, 0, 17, 31, 32, 33, 65, 2]
+    h, ids, wts, gu, dn = _case(counts, 1, d, F)
+    g = moe.group(ids, len(counts), moe.STREAM_ROWS)
+    y = moe.experts(h, ids, wts, gu, dn, g, False)[g.inv.view(-1).long()].float()
+    e = ids.view(-1).long()
+    u = torch.bmm(gu.float()[e], h.float()[:, :, None])[..., 0]
+    a = (torch.nn.functional.silu(u[:, :F]) * u[:, F:]).bfloat16().float()
+    want = torch.bmm(dn.float()[e], a[..., None])[..., 0] * wts
+    assert ((y - want).norm(dim=1) <= 2 * TOL * want.norm(dim=1)).all()  # (a row has few outputs: twice the whole's bound)
+
+
 @pytest.mark.parametrize("counts,mt", [([64, 65, 1, 0, 128, 320, 321], 128), ([257, 288, 289, 40, 513, 256, 130], 256), ([5, 70] * 40, 128), ([3] * 70, 192)])
 def test_short_tiles_run_last(counts, mt):
     """Tiles that are alone and at most half full stand behind the rest; every row has one tile, and the products are right."""
