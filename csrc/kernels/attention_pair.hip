@@ -9,35 +9,31 @@
 //   dQ:    the first takes S^T = K.Q^T and P, the second dP^T = V.dO^T, dS^T and dQ^T += K^T.dS^T, and leaves delta = rowsum(dO * O).
 // P goes from one to the other through LDS, in fp32 as it was. The second wave runs a tile behind and turns its step around -- dS and
 // its last product of tile t - 1, then dP of tile t -- so that one's softmax lies beside the other's products, and leaves the loads to the
-// first one, which has less to do.
+// first one, which has less to do: requests straight into LDS (TileRequests), two steps ahead, one between two products.
 //
 // Backward, us, one wave and a pair: 2 x 2048 x 16 heads 300, 266; 1 x 2048 225, 184; 1 x 4096 522, 454; 4 x 1100 234, 198; 8 x 512
-// with lengths 128, 108; 1 x 3000 with ALiBi 361, 285; 3 x 300 56, 46; 1 x 61 24.7, 21.8. A tile of dK/dV takes 3200 cycles now, of dQ
-// 2740 (1536 in the matrix cores): the LDS reads of both waves, 2085 of the 3200, and what of a wave's own chain the other does not
-// cover. No gain: deeper rings of fragments, wave priorities, a walk that touches tiles ahead, heads turned over the XCDs.
+// with lengths 128, 108; 1 x 3000 with ALiBi 361, 285; 3 x 300 56, 46; 1 x 61 24.7, 21.8. That was with tiles through the first wave's registers,
+// for which the last quarter of K's fragments had to lie in LDS and be read again at each step; requested into LDS, pairs, before and now:
+// 2 x 2048 254, 245 (dK/dV 160, 148; dQ 130, 122); 1 x 2048 182, 173; 1 x 4096 447, 424; 1 x 3000 with ALiBi 278, 265; 3 x 300 46.7, 45.0.
+// What bounds them: the LDS reads of both waves, 256 KB of a step of dK/dV, 192 of dQ (2048, 1536 cycles at 128 bytes), beside as many cycles in
+// the matrix cores, and what of a wave's own chain the other does not cover. No gain: deeper rings of fragments, wave priorities, a walk that touches
+// tiles ahead, heads turned over the XCDs, dQ's columns half to the first wave, with dS through LDS (130, 137: the reads stay as many).
 #include "attn_fast.h"
 
 #include <type_traits>
 
 namespace {
 
-__device__ __forceinline__ u32x4 buf_b128(__amdgpu_buffer_rsrc_t r, int vo, int so) {
-  const auto a = __builtin_amdgcn_raw_buffer_load_b128(r, vo, so, 0);
-  return *reinterpret_cast<const u32x4*>(&a);
-}
-
 struct Nothing { __device__ void operator()(int) const {} };
 
-// Rows of a tile image times a fixed operand, the reads two steps ahead of their product (pinned), `also(s)` between; the last NF
-// fragments of the operand come from LDS (`far`, a lane's 16 bytes of each 1 KB).
-template <int D, int NF = 0, class Also = Nothing>
-__device__ __forceinline__ f32x16 pair_rows(const char* smem, int img, int be, const bf16x8 (&fix)[D / 16], const char* far = nullptr,
-                                            Also also = {}) {
+// Rows of a tile image times a fixed operand, the reads two steps ahead of their product (pinned), `also(s)` between
+template <int D, class Also = Nothing>
+__device__ __forceinline__ f32x16 pair_rows(const char* smem, int img, int be, const bf16x8 (&fix)[D / 16], Also also = {}) {
   constexpr int KS = D / 16;
   f32x16 x;
 #pragma unroll
   for (int r = 0; r < 16; ++r) x[r] = 0.f;
-  bf16x8 f[3], l[NF ? NF : 1];
+  bf16x8 f[3];
   const int e = be + img, o = e ^ 32;  // (row_bases' second one is made of the first: the registers are full)
   __builtin_amdgcn_sched_barrier(0);  // (earlier reads are not of the groups)
   f[0] = row_frag<D>(smem, e, o, 0), f[1] = row_frag<D>(smem, e, o, 1);
@@ -48,21 +44,17 @@ __device__ __forceinline__ f32x16 pair_rows(const char* smem, int img, int be, c
     if (t < KS) {
       f[t % 3] = row_frag<D>(smem, e, o, t);
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      if (t >= KS - NF) {
-        l[t - KS + NF] = *reinterpret_cast<const bf16x8*>(far + (t - KS + NF) * 1024);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      }
     }
     also(s);
-    x = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[s % 3], s >= KS - NF ? l[max(0, s - KS + NF)] : fix[s], x, 0, 0, 0);
+    x = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[s % 3], fix[s], x, 0, 0, 0);
     __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
   }
   return x;
 }
 
 // acc += a tile image's columns times (x0, x1), read like its rows
-template <int D, class Also = Nothing>
-__device__ __forceinline__ void pair_columns(f32x16 (&acc)[D / 32], const char* smem, int img, int b1, bf16x8 x0, bf16x8 x1, Also also = {}) {
+template <int D>
+__device__ __forceinline__ void pair_columns(f32x16 (&acc)[D / 32], const char* smem, int img, int b1, bf16x8 x0, bf16x8 x1) {
   bf16x8 f[3];
   const int c1 = b1 + img, c2 = (c1 ^ 32) + 16 * D;
   auto get = [&](int n) {
@@ -75,38 +67,20 @@ __device__ __forceinline__ void pair_columns(f32x16 (&acc)[D / 32], const char* 
 #pragma unroll
   for (int n = 0; n < D / 16; ++n) {
     if (n + 2 < D / 16) get(n + 2);
-    also(n);
     acc[n >> 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[n % 3], n & 1 ? x1 : x0, acc[n >> 1], 0, 0, 0);
     __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
   }
 }
 
-// A tile by the first four waves: a wave's lanes take 8 chunks of 8 rows, 128 bytes of each and 1 KB in a row in the image; the next
-// 8 rows lie 16 D bytes on, their low sub-chunk bits turned.
-template <int D>
-struct PairLoader {
-  static_assert(D == 256, "four waves, 8 of 32 chunks each");
-  int vo, step;  // first chunk's byte offset, 8 rows
-  __device__ __forceinline__ PairLoader(int wave, int lane, long long st)
-      : vo((int)(((lane >> 3) * st + (wave * 8 + (lane & 7)) * 8) * 2)), step(__builtin_amdgcn_readfirstlane((int)(8 * st * 2))) {}
-  __device__ __forceinline__ void load(u32x4& x, __amdgpu_buffer_rsrc_t r, int so, int j) const { x = buf_b128(r, vo, so + j * step); }
-  static __device__ __forceinline__ int image(int wave, int lane) { return img_off<D>(lane >> 3, wave * 8 + (lane & 7)); }
-  static __device__ __forceinline__ void put(const u32x4 (&x)[4], char* smem, int at) {  // at: image + the thread's place in it
-#pragma unroll
-    for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4*>(smem + (at ^ (j % 2 * 32)) + j * 16 * D) = x[j];
-  }
-};
-
 template <int D, bool CAUSAL, int G>
 __global__ void __launch_bounds__(512, 2) attn_bwd_dkdv_pair_kernel(FastBwdParams p) {
   constexpr int RW = 4, BK = 32 * RW, BQ = 32;
   constexpr int TILE = BQ * D * 2, KS = D / 16;
-  // Q's tiles t - 1 (dK), t, t + 1 (loads); dO's t, t + 1; P of t - 1, t of each pair; lse and delta of t - 1 .. t + 1; the last NL of
-  // K's KS fragments, for which no register is left
-  constexpr int NL = 4;
-  constexpr int GOFF = 3 * TILE, POFF = GOFF + 2 * TILE, LOFF = POFF + 2 * RW * 4096, FOFF = LOFF + 4 * 64 * 4;
-  __shared__ __attribute__((aligned(16))) char smem[FOFF + NL * RW * 1024];
-  static_assert(FOFF + NL * RW * 1024 >= 2 * RW * TILE, "the epilogue's images take the tiles' place");
+  // Q's tiles t - 1 (dK), t, and t + 1, t + 2 on their way; dO's t to t + 2; P of t - 1, t of each pair; lse and delta of t - 1 .. t + 1
+  constexpr int NQ = 4, NG = 3;
+  constexpr int GOFF = NQ * TILE, POFF = GOFF + NG * TILE, LOFF = POFF + 2 * RW * 4096;
+  __shared__ __attribute__((aligned(1024))) char smem[LOFF + 4 * 64 * 4];
+  static_assert(LOFF >= 2 * RW * TILE, "the epilogue's images take the tiles' place");
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), rw = wave % RW;
@@ -150,67 +124,52 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_dkdv_pair_kernel(FastBwdParam
   };
 
   if (wave < RW) {
-    // The first waves bring the tiles. A step stores Q of the next one, requested in the step before, among its first products,
-    // requests dO of the next one among the rest and stores it behind its softmax, and requests Q of the one after under dV.
+    // The first waves request the tiles, two steps ahead: the second ones wait for loads of their own, which would wait for requests too.
     const float sl2 = p.scale * kLog2e;
     const int qn = rows_bytes(p.Sq, p.q_st, D), gn = rows_bytes(p.Sq, p.do_st, D);
-    const PairLoader<D> lq(wave, lane, p.q_st), lg(wave, lane, p.do_st);
-    const int own = PairLoader<D>::image(wave, lane);
-    const int soq0 = __builtin_amdgcn_readfirstlane(q_top * (int)p.q_st * 2), sog0 = __builtin_amdgcn_readfirstlane(q_top * (int)p.do_st * 2);
-    // the tiles of Q and of dO being loaded: first row, where it lies, query head (counted on: a step has no time to multiply)
-    int qtq = q_top, soq = soq0, headq = hk * grp, qtg = q_top, sog = sog0, headg = hk * grp;
-    __amdgpu_buffer_rsrc_t rq = head_rsrc(p.q + b * p.q_sb + headq * p.q_sh, qn), rg = head_rsrc(p.dout + b * p.do_sb + headg * p.do_sh, gn);
-    auto next_q = [&] {
-      qtq -= BQ, soq -= 4 * lq.step;
-      if (qtq >= q_lo) return;
-      qtq = q_top, soq = soq0, ++headq;
-      rq = head_rsrc(p.q + b * p.q_sb + headq * p.q_sh, qn);
+    using Req = TileRequests<D, RW>;
+    const Req lq(wave, lane, p.q_st), lg(wave, lane, p.do_st);
+    const int stepq = BQ * (int)p.q_st * 2, stepg = BQ * (int)p.do_st * 2;
+    const int soq0 = q_top * (int)p.q_st * 2, sog0 = q_top * (int)p.do_st * 2;
+    // the tile being requested: first row, where it lies, query head (counted on: a step has no time to multiply)
+    int qtr = q_top, soq = soq0, sog = sog0, headr = hk * grp;
+    u32x4 rq, rg;
+    auto words = [&] {
+      rq = head_words(p.q + b * p.q_sb + headr * p.q_sh, qn), rg = head_words(p.dout + b * p.do_sb + headr * p.do_sh, gn);
     };
-    auto next_g = [&] {
-      qtg -= BQ, sog -= 4 * lg.step;
-      if (qtg >= q_lo) return false;
-      qtg = q_top, sog = sog0, ++headg;
-      rg = head_rsrc(p.dout + b * p.do_sb + headg * p.do_sh, gn);
-      return true;
+    auto next = [&] {
+      qtr -= BQ, soq -= stepq, sog -= stepg;
+      if (qtr >= q_lo) return;
+      qtr = q_top, soq = soq0, sog = sog0, ++headr;
+      words();
     };
-    u32x4 xq[4];
-    if (total > 0) {  // (flies with the key rows)
-      u32x4 xg[4];
+    int sq = 0, sg = 0;  // their slots
+    auto request = [&](int j) {
+      if (j < Req::N) lq(rq, smem + sq * TILE, soq, j);
+      else lg(rg, smem + GOFF + sg * TILE, sog, j - Req::N);
+    };
+    auto taken = [&] { sq = sq == NQ - 1 ? 0 : sq + 1, sg = sg == NG - 1 ? 0 : sg + 1; };
+    if (total > 0) {  // (they fly with the key rows)
+      words();
 #pragma unroll
-      for (int j = 0; j < 4; ++j) lq.load(xq[j], rq, soq, j), lg.load(xg[j], rg, sog, j);
+      for (int t = 0; t < 2; ++t) {
+        if (t < total && t > 0) next();
+#pragma unroll
+        for (int j = 0; j < 2 * Req::N; ++j) request(j);
+        taken();
+      }
       load_fix(p.k + b * p.k_sb + hk * p.k_sh, p.k_st);
-#pragma unroll
-      for (int s = KS - NL; s < KS; ++s) *reinterpret_cast<bf16x8*>(smem + FOFF + (rw * NL + s - KS + NL) * 1024 + lane * 16) = fix[s];
-      PairLoader<D>::put(xq, smem, own);
-      PairLoader<D>::put(xg, smem, GOFF + own);
-      if (total > 1) next_q();
-#pragma unroll
-      for (int j = 0; j < 4; ++j) lq.load(xq[j], rq, soq, j);
     }
-    __syncthreads();
-    float next_slope = G == 2 ? p.alibi[headg] * kLog2e : 0.f;
-    int slot = 0;  // of tile i in Q's three
+    wait_and_meet<2 * Req::N>();  // the first tile is there
+    int qt = q_top, head = hk * grp, now = 0, at = 0;
+    float slope = G == 2 ? p.alibi[head] * kLog2e : 0.f;
     for (int i = 0; i < total; ++i) {
-      const int qt = qtg;
-      const float slope = next_slope;
-      // (past the last tile a step loads it again, into the slots that nobody reads)
-      if (i + 1 < total && next_g() && G == 2) next_slope = p.alibi[headg] * kLog2e;
-      if (i + 2 < total) next_q();
-      const int now = slot * TILE;
-      slot = slot == 2 ? 0 : slot + 1;
-      const int then = slot * TILE, at = GOFF + (i & 1) * TILE;
-      u32x4 xg[4];
+      if (i + 2 < total) next();  // (past the last tile a step requests it again, into the slots that nobody reads)
       asm volatile("" ::: "memory");
-      const f32x16 s = pair_rows<D, NL>(smem, now, be, fix, smem + FOFF + rw * NL * 1024 + lane * 16, [&](int s) {
-        if (s == 7) {
-          PairLoader<D>::put(xq, smem, then + own);
-          __builtin_amdgcn_sched_group_barrier(0x200, 4, 0);
-        }
-        if (s >= 8 && s % 2 == 0) {
-          lg.load(xg[s / 2 - 4], rg, sog, s / 2 - 4);
-          __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);
-        }
+      const f32x16 s = pair_rows<D>(smem, now * TILE, be, fix, [&](int s) {
+        if (s % 2 == 1) request(s / 2);
       });
+      taken();
       const int ln = own_lane(), key = kw + (ln & 31), hh = ln >> 5;
       // rows q = qt + 8g + 4hh + j (g = r>>2, j = r&3) that see the key: lim <= 8g + j < ul
       const bool plain = kb * BK + BK <= kv_end && (!CAUSAL || kb * BK + BK - 1 <= qt + off) &&
@@ -243,17 +202,17 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_dkdv_pair_kernel(FastBwdParam
       bf16x8 p0, p1;
 #pragma unroll
       for (int r = 0; r < 8; ++r) p0[r] = (__bf16)pr[r], p1[r] = (__bf16)pr[r + 8];
-      PairLoader<D>::put(xg, smem, GOFF + ((i + 1) & 1) * TILE + own);
       asm volatile("" ::: "memory");
-      pair_columns<D>(acc, smem, at, b1, p0, p1, [&](int n) {
-        if (n % 2 == 0 && n < 8) {
-          lq.load(xq[n / 2], rq, soq, n / 2);
-          __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);
-        }
-      });
-      __syncthreads();
+      pair_columns<D>(acc, smem, GOFF + at * TILE, b1, p0, p1);
+      now = now == NQ - 1 ? 0 : now + 1, at = at == NG - 1 ? 0 : at + 1;
+      qt -= BQ;
+      if (qt < q_lo) {
+        qt = q_top, ++head;
+        if (G == 2 && i + 1 < total) slope = p.alibi[head] * kLog2e;
+      }
+      wait_and_meet<2 * Req::N>();  // the next tile is there
     }
-    __syncthreads();  // the tiles become the epilogue images
+    wait_and_meet<0>();  // the tiles become the epilogue images
     store_tile_lds<D, D, true>(p.dv + b * p.dv_sb + hk * p.dv_sh + (long long)kw * p.dv_st, p.dv_st, acc, lane, 1.f, smem + wave * TILE,
                                p.Sk - kw);
   } else {
@@ -284,7 +243,7 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_dkdv_pair_kernel(FastBwdParam
     for (int g = 0; g < 4; ++g) *reinterpret_cast<f32x4*>(pair + lane * 16 + RW * 4096 + g * 1024) = f32x4{0.f, 0.f, 0.f, 0.f};
     if (rw == 1) stat[3 * 64 + lane] = 0.f;
     __syncthreads();
-    int slot = 0, before = 0;  // slots of tile i and the previous one (at first its own: P is 0)
+    int slot = 0, before = 0, at = 0;  // slots of tile i and the previous one (at first its own: P is 0), and of dO's
     f32x16 dp;
 #pragma unroll
     for (int r = 0; r < 16; ++r) dp[r] = 0.f;
@@ -309,9 +268,9 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_dkdv_pair_kernel(FastBwdParam
       pair_columns<D>(acc, smem, before * TILE, b1, s0, s1);
       before = slot;
       if (i < total) {
-        dp = pair_rows<D>(smem, GOFF + (i & 1) * TILE, be, fix);
+        dp = pair_rows<D>(smem, GOFF + at * TILE, be, fix);
         asm volatile("" ::: "memory");
-        slot = slot == 2 ? 0 : slot + 1;
+        slot = slot == NQ - 1 ? 0 : slot + 1, at = at == NG - 1 ? 0 : at + 1;
         put_stats(x, i + 1);
         __syncthreads();
       }
@@ -326,8 +285,10 @@ template <int D, bool CAUSAL, int G>
 __global__ void __launch_bounds__(512, 2) attn_bwd_dq_pair_kernel(FastBwdParams p) {
   constexpr int RW = 4, BM = 32 * RW, BN = 32;
   constexpr int TILE = BN * D * 2, KS = D / 16;
-  constexpr int VOFF = 3 * TILE, POFF = VOFF + 2 * TILE;  // K's tiles t - 1 (dQ), t, t + 1 (loads); V's t, t + 1; P of t - 1, t of each pair
-  __shared__ __attribute__((aligned(16))) char smem[POFF + 2 * RW * 4096];
+  // K's tiles t - 1 (dQ), t, and t + 1, t + 2 on their way; V's t to t + 2; P of t - 1, t of each pair
+  constexpr int NK = 4, NV = 3;
+  constexpr int VOFF = NK * TILE, POFF = VOFF + NV * TILE;
+  __shared__ __attribute__((aligned(1024))) char smem[POFF + 2 * RW * 4096];
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), rw = wave % RW;
@@ -346,48 +307,40 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_dq_pair_kernel(FastBwdParams 
   row_bases<D>(l32, hh, be, o_);
   tr_bases<D>(lane, b1, o_);
 
+  auto on = [](int& slot, int slots) { slot = slot == slots - 1 ? 0 : slot + 1; };
   bf16x8 fix[KS];  // the rows of Q, or of dO
   if (wave < RW) {
-    const int kn = rows_bytes(kv_end, p.k_st, D), vn = rows_bytes(kv_end, p.v_st, D);
-    const __amdgpu_buffer_rsrc_t rk = head_rsrc(p.k + b * p.k_sb + hk * p.k_sh, kn), rv = head_rsrc(p.v + b * p.v_sb + hk * p.v_sh, vn);
-    const PairLoader<D> lk(wave, lane, p.k_st), lv(wave, lane, p.v_st);
-    const int own = PairLoader<D>::image(wave, lane);
-    // the tile being loaded, a step before it is stored and two before it is read
-    int sok = __builtin_amdgcn_readfirstlane(sp.lo * 4 * lk.step), sov = __builtin_amdgcn_readfirstlane(sp.lo * 4 * lv.step);
-    u32x4 xk[4], xv[4];
-    auto load = [&] {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) lk.load(xk[j], rk, sok, j), lv.load(xv[j], rv, sov, j);
+    using Req = TileRequests<D, RW>;
+    const Req lk(wave, lane, p.k_st), lv(wave, lane, p.v_st);
+    const u32x4 kw = head_words(p.k + b * p.k_sb + hk * p.k_sh, rows_bytes(kv_end, p.k_st, D));
+    const u32x4 vw = head_words(p.v + b * p.v_sb + hk * p.v_sh, rows_bytes(kv_end, p.v_st, D));
+    const int stepk = BN * (int)p.k_st * 2, stepv = BN * (int)p.v_st * 2;
+    int sok = sp.lo * stepk, sov = sp.lo * stepv, sk = 0, sv = 0;  // the tile being requested, two steps ahead, and its slots
+    auto request = [&](int j) {
+      if (j < Req::N) lk(kw, smem + sk * TILE, sok, j);
+      else lv(vw, smem + VOFF + sv * TILE, sov, j - Req::N);
     };
-    load();
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      if (t > 0 && n > 1) sok += stepk, sov += stepv;
+#pragma unroll
+      for (int j = 0; j < 2 * Req::N; ++j) request(j);
+      on(sk, NK), on(sv, NV);
+    }
     const bf16_t* qp = p.q + b * p.q_sb + h * p.q_sh + (long long)qr * p.q_st + 8 * hh;
 #pragma unroll
     for (int s = 0; s < KS; ++s) fix[s] = *reinterpret_cast<const bf16x8*>(qp + 16 * s);
     const float sl2 = p.scale * kLog2e, nlse = -p.lse[li] * kLog2e, slope = G == 2 ? p.alibi[h] * kLog2e : 0.f;
-    PairLoader<D>::put(xk, smem, own);
-    PairLoader<D>::put(xv, smem, VOFF + own);
-    if (n > 1) sok += 4 * lk.step, sov += 4 * lv.step;
-    load();
-    __syncthreads();
-    int slot = 0;  // of tile i in K's three
+    wait_and_meet<2 * Req::N>();  // the first tile is there
+    int now = 0;
     for (int i = 0; i < n; ++i) {
-      const int t = sp.lo + i, k0 = t * BN, now = slot * TILE;
-      slot = slot == 2 ? 0 : slot + 1;
-      const int then = slot * TILE;
-      if (i + 2 < n) sok += 4 * lk.step, sov += 4 * lv.step;  // (past the last tile: it again, into slots that nobody reads)
+      const int t = sp.lo + i, k0 = t * BN;
+      if (i + 2 < n) sok += stepk, sov += stepv;  // (past the last tile: it again, into slots that nobody reads)
       asm volatile("" ::: "memory");
-      const f32x16 s = pair_rows<D>(smem, now, be, fix, nullptr, [&](int s) {
-        if (s == 3 || s == 5) {
-          if (s == 3) PairLoader<D>::put(xk, smem, then + own);
-          else PairLoader<D>::put(xv, smem, VOFF + ((i + 1) & 1) * TILE + own);
-          __builtin_amdgcn_sched_group_barrier(0x200, 4, 0);
-        }
-        if (s >= 8) {
-          if (s % 2 == 0) lk.load(xk[s / 2 - 4], rk, sok, s / 2 - 4);
-          else lv.load(xv[s / 2 - 4], rv, sov, s / 2 - 4);
-          __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);
-        }
+      const f32x16 s = pair_rows<D>(smem, now * TILE, be, fix, [&](int s) {
+        if (s % 2 == 1) request(s / 2);
       });
+      on(now, NK), on(sk, NK), on(sv, NV);
       const float b0 = G == 2 ? fmaf(slope, (float)(k0 + 4 * hh - qrow - off), nlse) : nlse;
       f32x16 pr;
 #pragma unroll
@@ -408,9 +361,9 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_dq_pair_kernel(FastBwdParams 
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         *reinterpret_cast<f32x4*>(pair + (i & 1) * RW * 4096 + g * 1024) = f32x4{pr[4 * g], pr[4 * g + 1], pr[4 * g + 2], pr[4 * g + 3]};
-      __syncthreads();
+      wait_and_meet<2 * Req::N>();  // the next tile is there
     }
-    __syncthreads();  // the second waves' last step reads the tiles
+    wait_and_meet<0>();  // the second waves' last step reads the tiles
     return;
   }
   f32x16 dq[D / 32];
@@ -432,7 +385,7 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_dq_pair_kernel(FastBwdParams 
 #pragma unroll
   for (int g = 0; g < 4; ++g) *reinterpret_cast<f32x4*>(pair + RW * 4096 + g * 1024) = f32x4{0.f, 0.f, 0.f, 0.f};
   __syncthreads();
-  int slot = 0, before = 0;
+  int slot = 0, before = 0, at = 0;
   f32x16 dp;
 #pragma unroll
   for (int r = 0; r < 16; ++r) dp[r] = 0.f;
@@ -452,9 +405,9 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_dq_pair_kernel(FastBwdParams 
     pair_columns<D>(dq, smem, before * TILE, b1, s0, s1);
     before = slot;
     if (i < n) {
-      dp = pair_rows<D>(smem, VOFF + (i & 1) * TILE, be, fix);
+      dp = pair_rows<D>(smem, VOFF + at * TILE, be, fix);
       asm volatile("" ::: "memory");
-      slot = slot == 2 ? 0 : slot + 1;
+      on(slot, NK), on(at, NV);
       __syncthreads();
     }
   }

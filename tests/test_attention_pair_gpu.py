@@ -28,6 +28,24 @@ def test_masks(causal):
         _check(2, 140, 330, 4, 1, 256, True, window=64, alibi=True)
 
 
+@pytest.mark.parametrize("S", [40, 200])
+def test_keys_past_the_length_are_not_read(S):
+    """What lies behind a sequence's length may be anything, and gets no gradient: one tile a walk, and tiles requested ahead of the last."""
+    g = torch.Generator(device="cuda").manual_seed(2)
+    q, k, v, do = (torch.randn(3, S, 2, 256, device="cuda", generator=g).bfloat16() for _ in range(4))
+    ln = torch.tensor([S, S - 37, 1], device="cuda", dtype=torch.int32)
+    gone = torch.arange(S, device="cuda")[None] >= ln[:, None]
+
+    def grads():
+        t = [x.clone().requires_grad_() for x in (q, k, v)]
+        return torch.autograd.grad(A.flash_attention(*t, causal=True, kv_len=ln), t, do)
+    want = grads()
+    k[gone], v[gone] = float("nan"), float("inf")
+    got = grads()
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
+    assert not got[1][gone].any() and not got[2][gone].any()
+
+
 def test_rows_off_16_bytes():
     """Full tiles in rows that 16-byte loads do not fit keep the kernels of one wave a block."""
     g = torch.Generator(device="cuda").manual_seed(1)
