@@ -204,19 +204,29 @@ def _k_slices(n: int, k: int) -> int:
 
 
 def _rows_mm(x2: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor | None:
-    """The product of up to FEW_ROWS rows on the weight-streaming kernel; None: sizes or alignment it does not take."""
+    """The product of up to FEW_ROWS rows on the weight-streaming kernel; None: sizes or alignment it does not take. One row, and two
+    where the vector kernel of the decode steps holds them in registers, go to that: no stage in LDS, no rows that are not there. us, rows'
+    kernel : vector kernel, one row and two: 50400 x 4096 78.9 : 56.4, 78.3 : 59.3; 12288 x 4096 21.2 : 16.2, 21.3 : 17.9; 4096 x 16384 31.4 :
+    21.8, 31.4 : 37.0; 2048 x 8192 11.6 : 7.6, 11.7 : 8.5; 14336 x 14336 75.7 : 59.5; 4096 x 1024 7.0 : 4.8, 7.1 : 5.9; short rows of wide
+    weights stay: 32000 x 1024 14.6 : 16.4, 14.6 : 23.3; 50400 x 768 19.1 : 23.3. Errors against 64 bits are the same."""
     rows, k = x2.shape
     n = weight.shape[0]
     if (n % 16 or k % 64 or k == 0 or 2 * max(n, rows) * k >= 1 << 32 or not weight.is_contiguous() or x2.data_ptr() % 16
             or weight.data_ptr() % 16 or (bias is not None and not bias.is_contiguous()) or not _lib.has("kca_rows_mm")):
         return None
+    bf16 = x2.dtype == torch.bfloat16
+    if (rows == 1 or (rows == 2 and bf16 and k <= 8192)) and (k >= 2048 or n <= 4096):
+        y = torch.empty(rows, n, device=x2.device, dtype=x2.dtype)
+        _lib.call("kca_skinny_gemm" if bf16 else "kca_skinny_gemm_f16", x2.data_ptr(), k, weight.data_ptr(), _lib.ptr(bias), y.data_ptr(),
+                  n, rows, n, k, 0, _lib.stream())
+        return y
     ks, ws, cnt = _k_slices(n, k), None, None
     if ks > 1:
         blocks = -(-n // 64)
         ws = torch.empty(blocks * ks * 64 * (32 if rows <= 32 else 64 if rows <= 64 else 128), device=x2.device, dtype=torch.float32)
         cnt = _lib.counters(x2.device, blocks)
     y = torch.empty(rows, n, device=x2.device, dtype=x2.dtype)
-    _lib.call("kca_rows_mm", 1 if x2.dtype == torch.bfloat16 else 2, x2.data_ptr(), weight.data_ptr(), _lib.ptr(bias),
+    _lib.call("kca_rows_mm", 1 if bf16 else 2, x2.data_ptr(), weight.data_ptr(), _lib.ptr(bias),
               y.data_ptr(), _lib.ptr(ws), _lib.ptr(cnt), 0 if ws is None else ws.numel(), 0 if cnt is None else cnt.numel(),
               rows, n, k, ks, _lib.stream())
     return y

@@ -36,6 +36,25 @@ def test_rows_against_float32(dtype, rows, n, k, bias):
     assert _lib.LAUNCHES[0] == before + 2 and _close(y, ref) and torch.equal(y, again)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [1, 2, 3])
+@pytest.mark.parametrize("n,k", [(16, 64), (4096, 1984), (4112, 1984), (4112, 2048), (1040, 8192), (1040, 8256), (272, 16448)])
+def test_one_and_two_rows(dtype, rows, n, k):
+    """On both sides of the lines between the vector kernel and the rows' one, eager and replayed."""
+    x, w, b, ref = _inputs(rows, n, k, dtype, True)
+    with torch.no_grad():
+        y = linear_rows(x, w, b)
+        assert _close(y, ref) and _close(linear_rows(x, w), F.linear(x.float(), w.float()))
+        graph = torch.cuda.CUDAGraph()
+        with capture.graph(graph, stream=torch.cuda.Stream()):
+            z = linear_rows(x, w, b)
+        for _ in range(3):
+            z.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert _close(z, ref) and torch.equal(linear_rows(x, w, b), y)
+
+
 @pytest.mark.parametrize("rows,n,k", [(61, 4096, 4096), (128, 4096, 4096)])
 def test_slices_under_capture_and_on_streams(rows, n, k):
     """The slices' counters: two streams at once, and a graph beside eager calls of its stream."""
