@@ -127,15 +127,22 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
         4104, 16, 2, 2056   3: 179, 154   4: 209, 176   8: 335, 180   16: 605, 186     1032, 16, 2, 520   4: 34, 22   16: 89, 22
         4104, 16, 2, 4104   3: 334, 337   4: 376, 329   8: 590, 335   16: 1099, 347    2056, 32, 4, 1032  4: 134, 101
 
-    The stream takes over where an expert expects more than one row, a little past two where rows are long (the vector
-    product's wave then has the longer walk over which to hide its reduction), but up to 16 tokens the vector product also
-    carries the shared expert. A stream tile holds 32 rows, past which weights are read again and a block has twice the
-    work, so it ends at 20 rows, as experts are uneven -- at 36 where narrow blocks are too few to fill the chip. A
-    narrow tile of 192 rows saves a second tile a little over 128 rows, if there are blocks enough without it, and costs
-    one a little over 192. A wide block is alone on its CU: it wins where the matrix cores bound the products, from
-    about 150 rows (64 where a contraction is long), if its rounds are well filled (``fill``: the blocks' time over that
-    of the rounds that they take; identity outputs count as experts here, so it is an estimate). Uneven experts cost
-    narrow and wide blocks alike from there on; with fewer rows wide ones wait for the largest expert's."""
+        the vector product in tiles of 8 rows and of 4, 8 and 16 tokens (the last two with a shared expert of 2048, 1024):
+        4096, 16, 3, 2048   98, 91; 143, 128      2048, 32, 4, 1024   55, 49; 81, 66         2048, 24, 5, 768    42, 35; 63, 49
+        4096, 16, 2, 4096   160, 157; 224, 219    5120, 8, 2, 2560    108, 96; 140, 133
+        4096, 16, 3, 2048   112, 106; 170, 155    2048, 32, 4, 1024   59, 53; 89, 73
+
+    The vector product's block holds its tile's rows in LDS, and with 4 of them twice as many blocks run on a CU;
+    weights are read again where an expert has more, from the cache. The stream takes over where an expert expects more
+    than one row, a little past two where rows are long (the vector product's wave then has the longer walk over which
+    to hide its reduction), but up to 16 tokens the vector product also carries the shared expert. A stream tile holds
+    32 rows, past which weights are read again and a block has twice the work, so it ends at 20 rows, as experts are
+    uneven -- at 36 where narrow blocks are too few to fill the chip. A narrow tile of 192 rows saves a second tile a
+    little over 128 rows, if there are blocks enough without it, and costs one a little over 192. A wide block is alone
+    on its CU: it wins where the matrix cores bound the products, from about 150 rows (64 where a contraction is long),
+    if its rounds are well filled (``fill``: the blocks' time over that of the rounds that they take; identity outputs
+    count as experts here, so it is an estimate). Uneven experts cost narrow and wide blocks alike from there on; with
+    fewer rows wide ones wait for the largest expert's."""
     n = T * top
     used = min(E, n)
     # 32-bit offsets into an expert's weights and the rows of a tile (elsewhere only 128-row tiles have longer ones)
@@ -163,6 +170,8 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
             return 192 if (full and 100 < r <= 160) or r > 240 else 128
         if stream and T > SHARED_ROWS and r > (2.25 if d > 2048 else 1):
             return STREAM_ROWS
+    if dtype == torch.bfloat16 and 4 < T and (T <= SHARED_ROWS or n <= 3 * used):
+        return 4
     return 1 if T == 1 else 2 if T == 2 else 4 if T <= 4 else 8
 
 
