@@ -14,7 +14,7 @@
 // Backward, us, one wave and a pair: 2 x 2048 x 16 heads 300, 266; 1 x 2048 225, 184; 1 x 4096 522, 454; 4 x 1100 234, 198; 8 x 512
 // with lengths 128, 108; 1 x 3000 with ALiBi 361, 285; 3 x 300 56, 46; 1 x 61 24.7, 21.8. That was with tiles through the first wave's registers,
 // for which the last quarter of K's fragments had to lie in LDS and be read again at each step; requested into LDS, pairs, before and now:
-// 2 x 2048 254, 245 (dK/dV 160, 148; dQ 130, 122); 1 x 2048 182, 173; 1 x 4096 447, 424; 1 x 3000 with ALiBi 278, 265; 3 x 300 46.7, 45.0.
+// 2 x 2048 254, 241 (dK/dV 160, 146; dQ 130, 120); 1 x 2048 182, 166; 1 x 4096 447, 420; 1 x 3000 with ALiBi 278, 259; 3 x 300 46.7, 44.1.
 // What bounds them: the LDS reads of both waves, 256 KB of a step of dK/dV, 192 of dQ (2048, 1536 cycles at 128 bytes), beside as many cycles in
 // the matrix cores, and what of a wave's own chain the other does not cover. No gain: deeper rings of fragments, wave priorities, a walk that touches
 // tiles ahead, heads turned over the XCDs, dQ's columns half to the first wave, with dS through LDS (130, 137: the reads stay as many).
@@ -151,25 +151,28 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_dkdv_pair_kernel(FastBwdParam
     auto taken = [&] { sq = sq == NQ - 1 ? 0 : sq + 1, sg = sg == NG - 1 ? 0 : sg + 1; };
     if (total > 0) {  // (they fly with the key rows)
       words();
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        if (t < total && t > 0) next();
+      auto tile = [&] {
 #pragma unroll
         for (int j = 0; j < 2 * Req::N; ++j) request(j);
         taken();
-      }
+      };
+      tile();
+      if (total > 1) next(), tile();
       load_fix(p.k + b * p.k_sb + hk * p.k_sh, p.k_st);
     }
-    wait_and_meet<2 * Req::N>();  // the first tile is there
+    // The first tile is there. A tile that has none behind it is waited for with nothing else on its way, so that the walk's end waits for nothing.
+    if (total > 1) wait_and_meet<2 * Req::N>();
+    else wait_and_meet<0>();
     int qt = q_top, head = hk * grp, now = 0, at = 0;
     float slope = G == 2 ? p.alibi[head] * kLog2e : 0.f;
-    for (int i = 0; i < total; ++i) {
-      if (i + 2 < total) next();  // (past the last tile a step requests it again, into the slots that nobody reads)
+    auto step = [&](int i, auto more) {  // more: there is a tile to request
+      if constexpr (more) next();
       asm volatile("" ::: "memory");
       const f32x16 s = pair_rows<D>(smem, now * TILE, be, fix, [&](int s) {
-        if (s % 2 == 1) request(s / 2);
+        if constexpr (more)
+          if (s % 2 == 1) request(s / 2);
       });
-      taken();
+      if constexpr (more) taken();
       const int ln = own_lane(), key = kw + (ln & 31), hh = ln >> 5;
       // rows q = qt + 8g + 4hh + j (g = r>>2, j = r&3) that see the key: lim <= 8g + j < ul
       const bool plain = kb * BK + BK <= kv_end && (!CAUSAL || kb * BK + BK - 1 <= qt + off) &&
@@ -210,9 +213,12 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_dkdv_pair_kernel(FastBwdParam
         qt = q_top, ++head;
         if (G == 2 && i + 1 < total) slope = p.alibi[head] * kLog2e;
       }
-      wait_and_meet<2 * Req::N>();  // the next tile is there
-    }
-    wait_and_meet<0>();  // the tiles become the epilogue images
+      wait_and_meet<more ? 2 * Req::N : 0>();  // the next tile is there
+    };
+    int i = 0;
+    for (; i + 2 < total; ++i) step(i, std::true_type{});
+    for (; i < total; ++i) step(i, std::false_type{});
+    __syncthreads();  // the tiles become the epilogue images
     store_tile_lds<D, D, true>(p.dv + b * p.dv_sb + hk * p.dv_sh + (long long)kw * p.dv_st, p.dv_st, acc, lane, 1.f, smem + wave * TILE,
                                p.Sk - kw);
   } else {
@@ -320,27 +326,29 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_dq_pair_kernel(FastBwdParams 
       if (j < Req::N) lk(kw, smem + sk * TILE, sok, j);
       else lv(vw, smem + VOFF + sv * TILE, sov, j - Req::N);
     };
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      if (t > 0 && n > 1) sok += stepk, sov += stepv;
+    auto tile = [&] {
 #pragma unroll
       for (int j = 0; j < 2 * Req::N; ++j) request(j);
-      on(sk, NK), on(sv, NV);
-    }
+      on(sk, NK), on(sv, NV), sok += stepk, sov += stepv;
+    };
+    tile();
+    if (n > 1) tile();
     const bf16_t* qp = p.q + b * p.q_sb + h * p.q_sh + (long long)qr * p.q_st + 8 * hh;
 #pragma unroll
     for (int s = 0; s < KS; ++s) fix[s] = *reinterpret_cast<const bf16x8*>(qp + 16 * s);
     const float sl2 = p.scale * kLog2e, nlse = -p.lse[li] * kLog2e, slope = G == 2 ? p.alibi[h] * kLog2e : 0.f;
-    wait_and_meet<2 * Req::N>();  // the first tile is there
+    if (n > 1) wait_and_meet<2 * Req::N>();  // the first tile is there (as in dK/dV)
+    else wait_and_meet<0>();
     int now = 0;
-    for (int i = 0; i < n; ++i) {
+    auto step = [&](int i, auto more) {
       const int t = sp.lo + i, k0 = t * BN;
-      if (i + 2 < n) sok += stepk, sov += stepv;  // (past the last tile: it again, into slots that nobody reads)
       asm volatile("" ::: "memory");
       const f32x16 s = pair_rows<D>(smem, now * TILE, be, fix, [&](int s) {
-        if (s % 2 == 1) request(s / 2);
+        if constexpr (more)
+          if (s % 2 == 1) request(s / 2);
       });
-      on(now, NK), on(sk, NK), on(sv, NV);
+      on(now, NK);
+      if constexpr (more) on(sk, NK), on(sv, NV), sok += stepk, sov += stepv;
       const float b0 = G == 2 ? fmaf(slope, (float)(k0 + 4 * hh - qrow - off), nlse) : nlse;
       f32x16 pr;
 #pragma unroll
@@ -361,9 +369,12 @@ __global__ void __launch_bounds__(512, 2) attn_bwd_dq_pair_kernel(FastBwdParams 
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         *reinterpret_cast<f32x4*>(pair + (i & 1) * RW * 4096 + g * 1024) = f32x4{pr[4 * g], pr[4 * g + 1], pr[4 * g + 2], pr[4 * g + 3]};
-      wait_and_meet<2 * Req::N>();  // the next tile is there
-    }
-    wait_and_meet<0>();  // the second waves' last step reads the tiles
+      wait_and_meet<more ? 2 * Req::N : 0>();  // the next tile is there
+    };
+    int i = 0;
+    for (; i + 2 < n; ++i) step(i, std::true_type{});
+    for (; i < n; ++i) step(i, std::false_type{});
+    __syncthreads();  // the second waves' last step reads the tiles
     return;
   }
   f32x16 dq[D / 32];
