@@ -252,12 +252,10 @@ __device__ __forceinline__ Cut cut(int c) {
 
 // n assignments -> perm (sorted position -> assignment), inv (assignment -> sorted position), tiles
 // [ntiles][5] (expert, first sorted position, rows <= mt, first tile and tile count of the expert) and
-// their count. Late tiles (and those of up to 128 rows where the limit is 256) stand after all others, each by itself, so that a
-// product takes them last (expert_gemm_kernel). One workgroup
-// of NT threads;
-// sh: 4 E + 3 ints.
-template <int NT>
-__device__ __forceinline__ void group_rows(const GroupArgs& p, int* sh) {
+// their count. Late tiles stand after all others, each by itself, so that a product takes them last (expert_gemm_kernel); where the limit
+// is 256 (BY_SIZE) the largest tiles stand first. One workgroup of NT threads; sh: 4 E + 3 ints.
+template <int NT, bool BY_SIZE>
+__device__ __forceinline__ void group_as(const GroupArgs& p, int* sh) {
   const int E = p.E, n = p.n, mt = p.mt, tid = threadIdx.x;
   int *cnt = sh, *off = sh + E, *toff = off + E + 1, *soff = toff + E + 1;
   constexpr int R = 4;  // a thread's first ids, read once for both passes
@@ -278,13 +276,13 @@ __device__ __forceinline__ void group_rows(const GroupArgs& p, int* sh) {
   __syncthreads();
   if (tid < 64) {  // exclusive sums over the experts, 64 at a time
     int co = 0, so = 0;
-    unsigned to = 0, to2 = 0;  // mt 256: four sums in 16 bits each (tiles are fewer than 32768), of experts whose largest tile is 4 .. 1 units
+    unsigned to = 0, to2 = 0;  // BY_SIZE: four sums in 16 bits each (tiles are fewer than 32768), of experts whose largest tile is 4 .. 1 units
     for (int e0 = 0; e0 < E; e0 += 64) {
       const int e = e0 + tid, c = e < E ? cnt[e] : 0, small = late_tile(c, mt);
       const unsigned before2 = to2;
       int cs = c, b = 0;
       unsigned t = (c + mt - 1) / mt - small, t2 = 0;
-      if (mt == 256) {
+      if constexpr (BY_SIZE) {
         const Cut k = cut(c);
         b = 4 - k.per - (k.more > 0);
         t = b < 2 ? k.tiles << 16 * b : 0, t2 = b < 2 ? 0 : k.tiles << 16 * (b & 1);
@@ -296,7 +294,7 @@ __device__ __forceinline__ void group_rows(const GroupArgs& p, int* sh) {
         const unsigned b1 = __shfl_up(ts, o, 64);
         if (tid >= o) cs += a, ts += b1;
       }
-      if (mt == 256) {
+      if constexpr (BY_SIZE) {
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
           const unsigned b2 = __shfl_up(ts2, o, 64);
@@ -308,14 +306,14 @@ __device__ __forceinline__ void group_rows(const GroupArgs& p, int* sh) {
       if (e < E) {
         const unsigned u = to + ts - t, u2 = before2 + ts2 - t2;
         off[e] = co + cs - c;
-        toff[e] = mt == 256 ? (b < 2 ? u : u2) >> 16 * (b & 1) & 0xffff : u;
-        soff[e] = mt == 256 ? b : so + __popcll(m & ((1ull << tid) - 1));
+        toff[e] = BY_SIZE ? (b < 2 ? u : u2) >> 16 * (b & 1) & 0xffff : u;
+        soff[e] = BY_SIZE ? b : so + __popcll(m & ((1ull << tid) - 1));
       }
       co += __shfl(cs, 63, 64);
       to += __shfl(ts, 63, 64);
       so += __popcll(m);
     }
-    if (mt == 256) {  // largest tiles first
+    if constexpr (BY_SIZE) {  // largest tiles first
       const unsigned n0 = to & 0xffff, n1 = n0 + (to >> 16), n2 = n1 + (to2 & 0xffff);
       for (int e = tid; e < E; e += 64) toff[e] += soff[e] == 0 ? 0 : soff[e] == 1 ? n0 : soff[e] == 2 ? n1 : n2;
       to = n2 + (to2 >> 16);
@@ -325,12 +323,12 @@ __device__ __forceinline__ void group_rows(const GroupArgs& p, int* sh) {
   __syncthreads();
   for (int e = tid; e < E; e += NT) {
     const int c = cnt[e], nt = (c + mt - 1) / mt, small = late_tile(c, mt);
-    const Cut k = mt == 256 ? cut(c) : Cut{0, 0, 0};
+    const Cut k = BY_SIZE ? cut(c) : Cut{0, 0, 0};
     for (int j = 0; j < nt; ++j) {
       const bool last = small && j == nt - 1;  // (it stands alone)
       const int at = last ? toff[E] + soff[e] : toff[e] + j;
-      const int from = mt == 256 ? 64 * (j * k.per + min(j, k.more)) : j * mt;
-      const int to = min(c, mt == 256 ? from + 64 * (k.per + (j < k.more)) : from + mt);
+      const int from = BY_SIZE ? 64 * (j * k.per + min(j, k.more)) : j * mt;
+      const int to = min(c, BY_SIZE ? from + 64 * (k.per + (j < k.more)) : from + mt);
       int* t = p.tiles + at * 5;
       t[0] = e;
       t[1] = off[e] + from;
@@ -346,6 +344,13 @@ __device__ __forceinline__ void group_rows(const GroupArgs& p, int* sh) {
     if (pos >= 0) p.perm[pos] = i;
     p.inv[i] = pos;
   });
+}
+
+// (the second scan would cost other limits 0.8 us, its branches 0.25)
+template <int NT>
+__device__ __forceinline__ void group_rows(const GroupArgs& p, int* sh) {
+  if (p.mt == 256) group_as<NT, true>(p, sh);
+  else group_as<NT, false>(p, sh);
 }
 
 __global__ void __launch_bounds__(1024) group_kernel(GroupArgs p) {
