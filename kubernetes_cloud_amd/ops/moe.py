@@ -112,6 +112,8 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
         4096, 16, 3, 2048   tokens   17: vector 158, stream 135     32: 195, 142             90: stream 146, narrow 173
         (20 outputs)               160: stream 165, narrow 177    260: 202, 180            300: narrow 182, wide 195
                                     900: narrow 208, wide 209     1500: 295, 227           3000: 487, 330
+            narrow of 128, of 192   330: 180, 193                  400: 199, 189            660: 229, 196     1100: 265, 257
+        2048, 24, 5, 768            650: 78, 83                    777: 83.5, 81.2         1000: 93, 91
         2048, 32, 4, 1024   tokens   17: vector 83, stream 73       24: 97, 76               100: stream 83, narrow 87
                                     128: stream 85, narrow 87      200: 92, 89              300: 112, 90
                                     500: narrow 93, wide 103      1150: 115, 115           3000: 211, 172     8192: 511, 406
@@ -122,7 +124,8 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
         5120, 8, 2, 2560    tokens   17: vector 144, stream 109    100: stream 134, narrow 149   160: 170, 154
         1024, 64, 2, 512    tokens   17: vector 27, stream 26       32: 39, 36               64: 58, 45
         2048, 40, 4, 1024   tokens 1200: narrow 142, wide 161     2000: 181, 188           2048, 10, 2, 2048, 600: 84, 90; 2000: 147, 141
-        5120, 8, 2, 2560    tokens  400: narrow 183, wide 156     1200: 275, 283           2000: 386, 333
+        5120, 8, 2, 2560    tokens  150: narrow 154, wide 134     250: 163, 146            400: 183, 156      600: 208, 177
+                                   1200: 275, 283                 2000: 386, 333
         widths that are no multiple of 64 have no stream; rows an expert, vector against narrow blocks:
         4104, 16, 2, 2056   3: 179, 154   4: 209, 176   8: 335, 180   16: 605, 186     1032, 16, 2, 520   4: 34, 22   16: 89, 22
         4104, 16, 2, 4104   3: 334, 337   4: 376, 329   8: 590, 335   16: 1099, 347    2056, 32, 4, 1032  4: 134, 101
@@ -138,11 +141,13 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
     to hide its reduction), but up to 16 tokens the vector product also carries the shared expert. A stream tile holds
     32 rows, past which weights are read again and a block has twice the work, so it ends at 20 rows, as experts are
     uneven -- at 36 where narrow blocks are too few to fill the chip. A narrow tile of 192 rows saves a second tile a
-    little over 128 rows, if there are blocks enough without it, and costs one a little over 192. A wide block is alone
-    on its CU: it wins where the matrix cores bound the products, from about 150 rows (64 where a contraction is long),
-    if its rounds are well filled (``fill``: the blocks' time over that of the rounds that they take; identity outputs
-    count as experts here, so it is an estimate). Uneven experts cost narrow and wide blocks alike from there on; with
-    fewer rows wide ones wait for the largest expert's."""
+    little over 128 rows (uneven experts have them from 100 expected rows on; from 56 where rows are long and weights
+    cost the most), if there are blocks enough without it, and costs one a little over 192. A wide block is alone on its
+    CU: it wins where the matrix cores bound the products, from about 150 rows (64 where a contraction is long, any
+    where narrow blocks would not fill the chip and wide ones make one round), if its rounds are well filled (``fill``:
+    the blocks' time over that of the rounds that they take; identity outputs count as experts here, so it is an
+    estimate). Uneven experts cost narrow and wide blocks alike from there on; with fewer rows wide ones wait for the
+    largest expert's."""
     n = T * top
     used = min(E, n)
     # 32-bit offsets into an expert's weights and the rows of a tile (elsewhere only 128-row tiles have longer ones)
@@ -152,7 +157,8 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
         return 128
     if gemm and near:
         stream = d % 64 == 0 and F % 64 == 0
-        r, short, full = n / used, min(d, F), used * (F // 64) >= 512
+        r, short, blocks = n / used, min(d, F), used * (F // 64)
+        full = blocks >= 512
         if r > ((20 if full else 36) if stream else 4):
             if stream:
                 tiles = used * -(-r // GEMM_ROWS)
@@ -162,12 +168,14 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
                 if r > GEMM_ROWS:
                     wide = fill >= 0.8 or (fill >= 0.6 and r > 480 and short >= 2048)
                 else:
-                    wide = r > 64 and short >= 4096 or r > 150 and (once or fill >= 0.8) or r > 175 and fill >= 0.6 and short >= 2048
+                    wide = (r > 64 and short >= 4096 or once and not full and short >= 2048 or r > 150 and (once or fill >= 0.8)
+                            or r > 175 and fill >= 0.6 and short >= 2048)
                 if wide:
                     return GEMM_ROWS
             elif r > 96 and (short >= 4096 or (short >= 1024 and r > 512)):
                 return GEMM_ROWS
-            return 192 if (full and 100 < r <= 160) or r > 240 else 128
+            two = r > (56 if short >= 2048 else 100) if full else r > 115 and blocks >= 384  # a 128-row tile is often not enough
+            return 192 if (two and r <= 175) or r > 240 else 128
         if stream and T > SHARED_ROWS and r > (2.25 if d > 2048 else 1):
             return STREAM_ROWS
     if dtype == torch.bfloat16 and 4 < T and (T <= SHARED_ROWS or n <= 3 * used):
