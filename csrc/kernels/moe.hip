@@ -276,7 +276,7 @@ __device__ __forceinline__ void group_as(const GroupArgs& p, int* sh) {
   __syncthreads();
   if (tid < 64) {  // exclusive sums over the experts, 64 at a time
     int co = 0, so = 0;
-    unsigned to = 0, to2 = 0;  // BY_SIZE: four sums in 16 bits each (tiles are fewer than 32768), of experts whose largest tile is 4 .. 1 units
+    unsigned to = 0, to2 = 0;  // BY_SIZE: four sums in 16 bits each (group_rows: no more tiles), of experts whose largest tile is 4 .. 1 units
     for (int e0 = 0; e0 < E; e0 += 64) {
       const int e = e0 + tid, c = e < E ? cnt[e] : 0, small = late_tile(c, mt);
       const unsigned before2 = to2;
@@ -346,10 +346,11 @@ __device__ __forceinline__ void group_as(const GroupArgs& p, int* sh) {
   });
 }
 
-// (the second scan would cost other limits 0.8 us, its branches 0.25)
+// (the second scan would cost other limits 0.8 us, its branches 0.25. Past 65535 tiles a class's count would not fit its 16 bits: in order of
+// the experts then, full tiles and a rest)
 template <int NT>
 __device__ __forceinline__ void group_rows(const GroupArgs& p, int* sh) {
-  if (p.mt == 256) group_as<NT, true>(p, sh);
+  if (p.mt == 256 && min(p.E, p.n) + p.n / 256 <= 0xffff) group_as<NT, true>(p, sh);
   else group_as<NT, false>(p, sh);
 }
 

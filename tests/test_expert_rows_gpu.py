@@ -101,6 +101,28 @@ def test_wide_tiles(counts, d, F):
         assert (y - want).norm() <= TOL * want.norm()
 
 
+@pytest.mark.parametrize("tiles", [65535, 65536, 66000])
+def test_more_tiles_than_16_bits_count(tiles):
+    """Tiles of up to 256 rows: the counts of a size are packed in 16 bits, up to as many."""
+    few = [300, 64, 1, 0, 700]
+    counts = few + [(tiles - len(few) - 1) * 256 - sum(few)]  # (a call's most tiles: experts and whole tiles)
+    n = sum(counts)
+    assert len(counts) + n // 256 == tiles
+    ids = torch.cat([torch.full((c,), e, device="cuda", dtype=torch.int32) for e, c in enumerate(counts)])
+    ids = ids[torch.randperm(n, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))][:, None]
+    g = moe.group(ids, len(counts), moe.GEMM_ROWS)
+    t = g.tiles[:int(g.ntiles)].long()
+    assert len(t) == sum(-(-c // 256) for c in counts) and int(t[:, 2].min()) >= 1 and int(t[:, 2].max()) <= 256
+    assert torch.bincount(t[:, 0], t[:, 2].double(), minlength=len(counts)).long().tolist() == counts
+    t = t[t[:, 1].argsort()]  # the tiles' rows follow each other, by experts
+    assert torch.equal(t[:, 1], t[:, 2].cumsum(0) - t[:, 2]) and (t[1:, 0] >= t[:-1, 0]).all()
+    sorted_ids = ids.view(-1)[g.perm.long()]
+    assert (sorted_ids[1:] >= sorted_ids[:-1]).all() and torch.equal(g.perm[g.inv.view(-1).long()].long(), torch.arange(n, device="cuda"))
+    of = g.tiles[:int(g.ntiles)].long()
+    first = of[:, 3]  # an expert's tiles stand together
+    assert torch.equal(of[first, 0], of[:, 0]) and (torch.arange(len(of), device="cuda") - first < of[:, 4]).all()
+
+
 def _far(T, d, F, E):
     """Sizes past the 32-bit offsets, and some tokens' outputs in fp32."""
     g = torch.Generator(device="cuda").manual_seed(1)
