@@ -673,6 +673,13 @@ __global__ void __launch_bounds__(256) expert_gemv_kernel(ExpertArgs p) {
   }
 }
 
+// A launch's dimension holds less than 2^32 threads: more blocks stand in rows of 2^22 (a multiple of the 8 XCDs)
+constexpr long long ROW_BLOCKS = 1 << 22;
+dim3 block_rows(long long blocks) {
+  return blocks <= ROW_BLOCKS ? dim3((unsigned)blocks) : dim3((unsigned)ROW_BLOCKS, (unsigned)((blocks + ROW_BLOCKS - 1) / ROW_BLOCKS));
+}
+__device__ __forceinline__ int block_number() { return blockIdx.y * (int)ROW_BLOCKS + blockIdx.x; }
+
 // ---------------------------------------------------------------------------------------------- stream
 // bf16, tiles of up to 32 rows x 32 weight rows (up: 16 gate rows and the 16 up rows beside them), 4 waves, each with every fourth stage
 // of 64 of K; the waves' sums meet in LDS. Bound by the weight stream. How fast memory gives it hangs on how far apart the rows lie that
@@ -816,9 +823,9 @@ __global__ void __launch_bounds__(256, 2) expert_stream_kernel(ExpertArgs p) {
   extern __shared__ __attribute__((aligned(1024))) char sl[];
   constexpr int NB = UP ? SWN / 2 : SWN;
   const int nt = *p.ntiles, nb = (p.N + NB - 1) / NB;
-  if ((int)blockIdx.x >= nt * nb) return;
   // Runs of 64 blocks, eight adjacent ones an XCD: what the chip reads at a time stays compact, and an expert's row tiles share an L2
-  const int b = blockIdx.x, end = nt * nb, c = b & ~63;
+  const int b = block_number(), end = nt * nb, c = b & ~63;
+  if (b >= end) return;
   const int id = c + xcd_remap(b - c, min(64, end - c));
   const int* t0 = p.tiles + id / nb * 5;
   const int in = id - t0[3] * nb, tile = t0[3] + in % t0[4], bn = in / t0[4];
@@ -1392,8 +1399,12 @@ KCA_API int kca_moe_expert(int dtype, const void* x, const void* w, void* y, con
     if (dtype != 1 || K % SK || N % 16 || !al16(x) || !al16(w) || (uintptr_t)y % 8 || far) return 10;
     const void* kern = up ? (const void*)expert_stream_kernel<true> : (const void*)expert_stream_kernel<false>;
     if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, STREAM_LDS) != hipSuccess) return 5;
-    if (up) hipLaunchKernelGGL(expert_stream_kernel<true>, dim3((N + SWN / 2 - 1) / (SWN / 2) * max_tiles), dim3(256), STREAM_LDS, s, a);
-    else hipLaunchKernelGGL(expert_stream_kernel<false>, dim3((N + SWN - 1) / SWN * max_tiles), dim3(256), STREAM_LDS, s, a);
+    const int nb = up ? SWN / 2 : SWN;
+    const long long blocks = (N + nb - 1ll) / nb * max_tiles;
+    if (blocks >= 1ll << 31) return 10;
+    const dim3 grid = block_rows(blocks);
+    if (up) hipLaunchKernelGGL(expert_stream_kernel<true>, grid, dim3(256), STREAM_LDS, s, a);
+    else hipLaunchKernelGGL(expert_stream_kernel<false>, grid, dim3(256), STREAM_LDS, s, a);
     return hipGetLastError() == hipSuccess ? 0 : 4;
   }
   const int v = dtype == 1 ? 8 : 4;

@@ -123,6 +123,20 @@ def test_more_tiles_than_16_bits_count(tiles):
     assert torch.equal(of[first, 0], of[:, 0]) and (torch.arange(len(of), device="cuda") - first < of[:, 4]).all()
 
 
+def test_more_blocks_than_a_dimension_holds():
+    """The stream's launch for 21900 tiles of 12288 outputs: 16.8 million blocks of 256 threads; the rows of the last ones."""
+    T, F = 32 * 21900, 12288
+    h, ids, wts, gu, dn = _case([T], 1, 64, F)
+    g = moe.group(ids, 1, moe.STREAM_ROWS)
+    y = moe.experts(h, ids, wts, gu, dn, g, False)
+    for rows in (slice(0, 64), slice(T // 2, T // 2 + 64), slice(T - 64, T)):
+        t = g.perm[rows].long()
+        u = h[t].float() @ gu[0].float().T
+        a = (torch.nn.functional.silu(u[:, :F]) * u[:, F:]).bfloat16().float()
+        want = a @ dn[0].float().T * wts[t]
+        assert (y[rows].float() - want).norm() <= TOL * want.norm()
+
+
 def _far(T, d, F, E):
     """Sizes past the 32-bit offsets, and some tokens' outputs in fp32."""
     g = torch.Generator(device="cuda").manual_seed(1)
