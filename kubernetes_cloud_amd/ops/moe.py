@@ -268,7 +268,13 @@ def experts(h: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, gate_up: 
             y[pos] = (ff(h[a // top].float(), gate_up[e], down[e], w if scale_in else 1.0) * (1.0 if scale_in else w)).to(h.dtype)
         return y if shared is None else (y, torch.stack([ff(r.float(), *shared).to(h.dtype) for r in h]))
     assert h.is_contiguous() and gate_up.is_contiguous() and down.is_contiguous() and down.shape == (E, d, F)
-    if g.mt > 8:  # (16-byte loads; the vector product, which calls of up to 16 rows an expert once took, has any address)
+    if (g.mt == STREAM_ROWS and shared is None and n <= (3 if d > 2048 else 2) * E
+            and (gate_up.data_ptr() % 16 or down.data_ptr() % 16)):
+        # weights that the stream's loads do not fit, few rows of each: the vector product reads them where they are, in its own order
+        own = group(ids, E, 8)
+        y = experts(h, ids, weights, gate_up, down, own, scale_in)
+        return y[own.inv.view(-1)[g.perm.clamp(0, n - 1).long()].clamp(min=0).long()]
+    if g.mt > 8:  # (16-byte loads; the vector product has any address)
         h, gate_up, down = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (h, gate_up, down))
     act = torch.empty(n, F, device=h.device, dtype=h.dtype)
     y = torch.empty(n, d, device=h.device, dtype=h.dtype)

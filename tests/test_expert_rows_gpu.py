@@ -180,3 +180,23 @@ def test_rows_off_16_bytes(mt):
     for args in ((off(h), gu, dn), (h, off(gu), dn), (h, gu, off(dn))):
         y = moe.experts(args[0], ids, wts, *args[1:], g, True)
         assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("scale_in", [True, False])
+@pytest.mark.parametrize("which", ["gate_up", "down"])
+def test_few_rows_of_weights_off_16_bytes(which, scale_in):
+    """One to two rows an expert: no copy of the stacks, the vector product's results in the order of the stream's groups; identity experts too."""
+    E, d, F = 32, 256, 512
+    h, ids, wts, gu, dn = _case([1, 2, 3, 0] * 8 + [9], 3, d, F)  # (the last id has no weights)
+    gu, dn = gu[:E].contiguous(), dn[:E].contiguous()
+    off = lambda t: torch.empty(t.numel() + 8, device="cuda", dtype=t.dtype)[1:1 + t.numel()].view(t.shape).copy_(t)  # noqa: E731
+    gu, dn = (off(gu), dn) if which == "gate_up" else (gu, off(dn))
+    g, own = moe.group(ids, E, moe.STREAM_ROWS), moe.group(ids, E, 8)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    y = moe.experts(h, ids, wts, gu, dn, g, scale_in)
+    assert torch.cuda.max_memory_allocated() - before < dn.numel()  # (half of the smaller stack's bytes)
+    want = moe.experts(h, ids, wts, gu, dn, own, scale_in)
+    i, j = g.inv.view(-1), own.inv.view(-1)
+    assert torch.equal(i < 0, j < 0) and torch.equal(y[i[i >= 0].long()], want[j[j >= 0].long()])
