@@ -135,8 +135,13 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
         4096, 16, 2, 4096   160, 157; 224, 219    5120, 8, 2, 2560    108, 96; 140, 133
         4096, 16, 3, 2048   112, 106; 170, 155    2048, 32, 4, 1024   59, 53; 89, 73
 
-    The vector product's block holds its tile's rows in LDS, and with 4 of them twice as many blocks run on a CU;
-    weights are read again where an expert has more, from the cache. The stream takes over where an expert expects more
+        few experts, no shared one: 4096, 2, 2, 4096: 5 tokens 57, 67; 8: 68, 73; 16: 119, 130     4096, 2, 1, 8192: 5: 72, 70; 16: 133, 143
+        4096, 8, 4, 4096: 6: 145, 136; 8: 168, 171; 16: 257, 281     4096, 16, 6, 2048: 8: 151, 139; 16: 218, 219
+        2048, 4, 4, 2048: 5: 37, 38; 16: 76, 72     2048, 16, 8, 1024: 5: 50, 43; 16: 94, 79     1024, 8, 8, 512: 16: 39, 32
+
+    The vector product's block holds its tile's rows in LDS, and with 4 of them twice as many blocks run on a CU; an expert
+    with more rows streams its weights again, which costs more where rows of weights are longer than the 2048 that a block takes
+    at one time. The stream takes over where an expert expects more
     than one row, a little past two where rows are long (the vector product's wave then has the longer walk over which
     to hide its reduction), but up to 16 tokens the vector product also carries the shared expert. A stream tile holds
     32 rows, past which weights are read again and a block has twice the work, so it ends at 20 rows, as experts are
@@ -178,7 +183,7 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
             return 192 if (two and r <= 175) or r > 240 else 128
         if stream and T > SHARED_ROWS and r > (2.25 if d > 2048 else 1):
             return STREAM_ROWS
-    if dtype == torch.bfloat16 and 4 < T and (T <= SHARED_ROWS or n <= 3 * used):
+    if dtype == torch.bfloat16 and T > 4 and (n <= 3 * used or (T <= SHARED_ROWS and max(d, F) <= 2048)):
         return 4
     return 1 if T == 1 else 2 if T == 2 else 4 if T <= 4 else 8
 
