@@ -101,58 +101,49 @@ class Groups:
 
 
 def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
-    """Row limit of an expert tile, by the rows ``r`` that an expert expects: a streaming vector product (1 .. 8), the
-    weight stream on the matrix cores (32), the prompts' product in narrow blocks (128 or 192 rows x 128 weight rows) or
-    wide ones (256 x 256). Both products of a layer, us (width, experts, top, inner size; - not measured):
+    """Row limit of an expert tile, by the rows ``r`` that an expert expects (``n`` over the experts): a streaming vector product (1
+    .. 8), the weight stream on the matrix cores (32), the prompts' product in narrow blocks (128 or 192 rows x 128 weight rows)
+    or wide ones (256 x 256). The lines, with both products of a layer in us on either side (width, experts, top, inner size:
+    tokens; weights from memory, uneven routing):
 
-        4096, 16, 2, 4096   tokens   17: vector 226, stream 240     24: 270, 262             32: 314, 278
-                                    100: stream 275, narrow 292    160: 283, 295            260: 352, 301
-                                    300: narrow 305, wide 306      700: 338, 322
-                                   1000: narrow 367, wide 333     1300: 377, 339           2500: 610, 505
-        4096, 16, 3, 2048   tokens   17: vector 158, stream 135     32: 195, 142             90: stream 146, narrow 173
-        (20 outputs)               160: stream 165, narrow 177    260: 202, 180            300: narrow 182, wide 195
-                                    900: narrow 208, wide 209     1500: 295, 227           3000: 487, 330
-            narrow of 128, of 192   330: 180, 193                  400: 199, 189            660: 229, 196     1100: 265, 257
-        2048, 24, 5, 768            650: 78, 83                    777: 83.5, 81.2         1000: 93, 91
-        2048, 32, 4, 1024   tokens   17: vector 83, stream 73       24: 97, 76               100: stream 83, narrow 87
-                                    128: stream 85, narrow 87      200: 92, 89              300: 112, 90
-                                    500: narrow 93, wide 103      1150: 115, 115           3000: 211, 172     8192: 511, 406
-        4096, 20, 3, 2048   tokens  900: narrow 271, wide 286     1500: 349, 342           3000: 608, 437
-        2048, 24, 5, 768    tokens   17: vector 65, stream 47      100: stream 56, narrow 69   200: 67, 74      300: 81, 73
-        (32 outputs, uneven)       400: narrow 73, wide 83        777: 83, 85              1300: 96, 86      2000: 117, 106
-                                   3000: narrow 141, wide 143     4096: 231, 189
-        5120, 8, 2, 2560    tokens   17: vector 144, stream 109    100: stream 134, narrow 149   160: 170, 154
-        1024, 64, 2, 512    tokens   17: vector 27, stream 26       32: 39, 36               64: 58, 45
-        2048, 40, 4, 1024   tokens 1200: narrow 142, wide 161     2000: 181, 188           2048, 10, 2, 2048, 600: 84, 90; 2000: 147, 141
-        5120, 8, 2, 2560    tokens  150: narrow 154, wide 134     250: 163, 146            400: 183, 156      600: 208, 177
-                                   1200: 275, 283                 2000: 386, 333
-        widths that are no multiple of 64 have no stream; rows an expert, vector against narrow blocks:
-        4104, 16, 2, 2056   3: 179, 154   4: 209, 176   8: 335, 180   16: 605, 186     1032, 16, 2, 520   4: 34, 22   16: 89, 22
-        4104, 16, 2, 4104   3: 334, 337   4: 376, 329   8: 590, 335   16: 1099, 347    2056, 32, 4, 1032  4: 134, 101
-
-        the vector product in tiles of 8 rows and of 4, 8 and 16 tokens (the last two with a shared expert of 2048, 1024):
-        4096, 16, 3, 2048   98, 91; 143, 128      2048, 32, 4, 1024   55, 49; 81, 66         2048, 24, 5, 768    42, 35; 63, 49
-        4096, 16, 2, 4096   160, 157; 224, 219    5120, 8, 2, 2560    108, 96; 140, 133
-        4096, 16, 3, 2048   112, 106; 170, 155    2048, 32, 4, 1024   59, 53; 89, 73
-
-        few experts, no shared one: 4096, 2, 2, 4096: 5 tokens 57, 67; 8: 68, 73; 16: 119, 130     4096, 2, 1, 8192: 5: 72, 70; 16: 133, 143
+    Vector product in tiles of 8 rows or of 4. Its block holds the tile's rows in LDS, and with 4 of them twice as many blocks
+    run on a CU; an expert with more rows streams its weights again, which costs more where rows of weights are longer than the
+    2048 that a block takes at one time. 4 up to 3 rows, and for weights of up to 2048 as far as it goes (8, 4):
         4096, 8, 4, 4096: 6: 145, 136; 8: 168, 171; 16: 257, 281     4096, 16, 6, 2048: 8: 151, 139; 16: 218, 219
-        2048, 4, 4, 2048: 5: 37, 38; 16: 76, 72     2048, 16, 8, 1024: 5: 50, 43; 16: 94, 79     1024, 8, 8, 512: 16: 39, 32
-
-    The vector product's block holds its tile's rows in LDS, and with 4 of them twice as many blocks run on a CU; an expert
-    with more rows streams its weights again, which costs more where rows of weights are longer than the 2048 that a block takes
-    at one time. The stream takes over where an expert expects more
-    than one row, a little past two where rows are long (the vector product's wave then has the longer walk over which
-    to hide its reduction), but up to 16 tokens the vector product also carries the shared expert. A stream tile holds
-    32 rows, past which weights are read again and a block has twice the work, so it ends at 20 rows, as experts are
-    uneven -- at 36 where narrow blocks are too few to fill the chip. A narrow tile of 192 rows saves a second tile a
-    little over 128 rows (uneven experts have them from 100 expected rows on; from 56 where rows are long and weights
-    cost the most), if there are blocks enough without it, and costs one a little over 192. A wide block is alone on its
-    CU: it wins where the matrix cores bound the products, from about 150 rows (64 where a contraction is long, any
-    where narrow blocks would not fill the chip and wide ones make one round), if its rounds are well filled (``fill``:
-    the blocks' time over that of the rounds that they take; identity outputs count as experts here, so it is an
-    estimate). Uneven experts cost narrow and wide blocks alike from there on; with fewer rows wide ones wait for the
-    largest expert's."""
+        4096, 2, 2, 4096: 5: 57, 67; 16: 119, 130                    4096, 2, 1, 8192: 5: 72, 70; 16: 133, 143
+        2048, 4, 4, 2048: 5: 37, 38; 16: 76, 72                      2048, 16, 8, 1024: 5: 50, 43; 16: 94, 79
+        with a shared expert: 4096, 16, 3, 2048: 8: 112, 106; 16: 170, 155    4096, 8, 4, 4096: 16: 311, 337
+    Vector, stream: from 1 row on, 2.25 where rows are longer than 2048 (the vector product's wave then has the longer walk over
+    which to hide its reduction). Up to 16 tokens the vector product also carries the shared expert:
+        4096, 16, 2, 4096: 17: 226, 240; 24: 270, 262      4096, 16, 3, 2048: 17: 158, 135
+        2048, 32, 4, 1024: 17: 83, 73; 24: 97, 76          1024, 64, 2, 512: 17: 27, 26; 32: 39, 36
+    Stream, narrow: a stream tile holds 32 rows, past which weights are read again, so it ends at 20 rows, as experts are uneven
+    -- at 36 where narrow blocks (``blocks`` of 64 weight rows) are fewer than the 512 that run at one time:
+        4096, 16, 2, 4096: 160: 283, 295; 260: 352, 301    2048, 32, 4, 1024: 128: 85, 87; 200: 92, 89
+        2048, 24, 5, 768: 200: 67, 74; 300: 81, 73         5120, 8, 2, 2560: 100: 134, 149; 160: 170, 154
+    without it (widths that are no multiple of 64) vector, narrow: 4 rows:
+        4104, 16, 2, 2056: r 3: 179, 154; 8: 335, 180      1032, 16, 2, 520: r 4: 34, 22      4104, 16, 2, 4104: r 3: 334, 337; 4: 376, 329
+    Narrow, 128 rows or 192: the larger tile saves a second one a little over 128 rows and costs one over 192; uneven experts
+    have more than 128 from some 100 on, and where rows are long it costs nothing from 56 on (4096, 16, 3, 2048 of 20 outputs, the largest
+    expert at twice the mean: 400: 200, 191; 467: 218, 187; 600: 212, 194; five layers with other routing .99 to 1.02). Without
+    so many blocks two thirds of the 512 places have to be taken, or a tile's length counts for more than
+    their number: time of 192 rows over that of 128 at 115 to 175 rows (even, uneven and very uneven routing) of 256 to 320 blocks
+    0.98 to 1.07 (8 layers; 2048, 28, 4, 640: 1.00, 1.03, 1.03; 1024, 64, 6, 320: .93, 1.03, 1.01), of 352 (1536, 32, 4, 704) .97, .91,
+    .91, of 384 .96, .92, .91; .92, .97, .97; .97, .94, .97; .95, .90, .99 (2048, 24, 4, 1024; 2048, 32, 5, 768; 3072, 24, 4, 1024; 4096, 16, 3,
+    1536), of 432 to 480 .85 to .90, .93 to 1.02, 1.0 to 1.06; at 90 to 105 rows 1.0 to 1.04.
+    Narrow, wide: a wide block is alone on its CU. It wins where the matrix cores bound the products, from about 150 rows (64
+    where a contraction is long), if its rounds are well filled (``fill``: the blocks' time over that of the rounds that they
+    take; identity outputs count as experts here, so it is an estimate):
+        4096, 16, 2, 4096: 300: 305, 306; 700: 338, 322; 2500: 610, 505    2048, 32, 4, 1024: 500: 93, 103; 1150: 115, 115; 3000: 211, 172
+        4096, 16, 3, 2048: 900: 208, 209; 1500: 295, 227                   2048, 24, 5, 768: 777: 83, 85; 1300: 96, 86; 4096: 231, 189
+        2048, 40, 4, 1024: 1200: 142, 161; 2000: 181, 188                  2048, 10, 2, 2048: 600: 84, 90; 2000: 147, 141
+    or with any rows where narrow blocks do not fill the chip and wide ones of both products are one round on more than half of
+    the CUs (blocks of the products; r 40, 80, 110; narrow, wide):
+        4608, 8, 2, 2304 (144, 144): 140, 124; 141, 144; 156, 155     5120, 8, 2, 2560 (160, 160): 161, 138; 173, 161; 179, 187
+        5632, 6, 2, 2816 (132, 132): 166, 143; 173, 159; 187, 180     4352, 8, 2, 2176 (136, 136): 135, 117; 131, 152; 141, 153
+        3072, 12, 2, 2304 (216, 144): 123, 113; 131, 131; 142, 146    5120, 8, 2, 3840 (240, 160): 201, 180; 225, 210; 247, 218
+        4096, 8, 2, 2560 (160, 128): 129, 130; 143, 154; 153, 161     4096, 8, 2, 2048 (128, 128): 100, 109; 106, 124; 108, 132
+        6144, 8, 2, 2048 (128, 192): 148, 169; 154, 179; 194, 189     5120, 6, 2, 5120 (240, 120): 184, 194"""
     n = T * top
     used = min(E, n)
     # 32-bit offsets into an expert's weights and the rows of a tile (elsewhere only 128-row tiles have longer ones)
@@ -169,7 +160,7 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
                 tiles = used * -(-r // GEMM_ROWS)
                 up, down = tiles * -(-F // 128), tiles * -(-d // 256)  # wide blocks of the two products; rounds of one a CU
                 fill = (up * d + down * F) / (256 * (-(-up // 256) * d + -(-down // 256) * F))
-                once = max(up, down) <= 256 and min(up, down) >= 144
+                once = max(up, down) <= 256 and min(up, down) > 128
                 if r > GEMM_ROWS:
                     wide = fill >= 0.8 or (fill >= 0.6 and r > 480 and short >= 2048)
                 else:
@@ -179,7 +170,7 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
                     return GEMM_ROWS
             elif r > 96 and (short >= 4096 or (short >= 1024 and r > 512)):
                 return GEMM_ROWS
-            two = r > (56 if short >= 2048 else 100) if full else r > 115 and blocks >= 384  # a 128-row tile is often not enough
+            two = r > (56 if short >= 2048 else 100) if full else r > 115 and 3 * blocks >= 2 * 512  # a 128-row tile is often not enough
             return 192 if (two and r <= 175) or r > 240 else 128
         if stream and T > SHARED_ROWS and r > (2.25 if d > 2048 else 1):
             return STREAM_ROWS
