@@ -721,83 +721,52 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
 
 }  // namespace
 
-// Which calls are split in two groups (two waves of 32 rows each, 4 waves a workgroup), the others in blocks of 128 rows and
-// one group: up to so many blocks of 64 rows of all heads, the more the longer the longest walk is (keys that a row sees; dK/dV: queries),
-// for a split costs each of its blocks the meeting of the sums. Past the workgroups that run at one time (768 of 64-wide heads, 512 of
-// others) a last round of a few loses more than it saves. One MI355X, us with one group, and what two take, at so many blocks of 64 rows:
-//   forward, 64 wide:   96 rows, 200 6.8, 6.7, 280 6.9, 7.4; 130 rows, 510 9.2, 8.5; 200 rows, 680 9.9, 10.0, 800 10.1, 12.3; 400 rows, 700 12.4, 11.6;
-//                       768 rows, 684 17.1, 16.7, 804 19.2, 20.3; 1200 rows, 760 20.1, 16.8, 912 20.4, 20.7; 2048 rows, 672 29.7, 26.8, 800 31.2,
-//                       36.0; 2600 rows, 656 34.5, 24.6, 779 36.0, 37.9, 820 36.5, 30.7, 984 37.8, 34.3; 3500 rows, 825 46.4, 39.0, 990 48.2, 43.4, 1155 52.1,
-//                       59.2; 4096 rows, 1152 59.0, 55.8 (the longer the walk, the more the longest ones alone at the end, halved by a split, weigh)
-//   96 wide:            96 rows, 200 7.9, 7.9, 280 8.1, 9.3; 200 rows, 280 10.0, 9.9, 360 10.1, 10.6; 320 rows, 500 12.7, 12.3, 565 12.7, 15.8;
-//                       512 rows, 440 14.3, 13.0, 520 14.6, 16.0; 1024 rows, 512 20.6, 17.6, 608 21.4, 22.0; 1500 rows, 528 26.6, 26.3, 600 30.0, 33.4; 2048
-//                       rows, 512 32.4, 25.5, 608 34.4, 41.3; 3000 rows, 611 46.0, 38.6, 799 49.3, 52.8; 4096 rows, 768 63.3, 57.0, 896 66.4, 69.8
-//   128 wide:           96 rows, 200 8.4, 8.4; 200 rows, 280 10.8, 10.6, 360 11.0, 11.8; 256 rows, 280 12.2, 11.5, 360 12.5, 13.2; 512 rows, 440 17.9,
-//                       17.8, 520 18.8, 20.5; 900 rows, 480 21.7, 17.1; 1024 rows, 608 26.5, 25.9, 672 27.0, 28.0; 2048 rows, 672 42.2, 40.9, 800 45.4, 53.5;
-//                       3500 rows, 715 64.6, 59.6, 825 68.4, 69.3; 4096 rows, 896 80.7, 76.7, 1152 89.9, 99
-//   dQ, what two save:  64 wide, 96 rows, 200 0.2, 280 -1.0; 400 rows, 700 1.0; 768 rows, 516 1.9, 600 -1.0; 1024 rows, 608 0.6, 672 -0.8; 1200 rows, 760 4.4, 912
-//                       0.9; 2048 rows, 512 10.1, 608 -0.2; 2600 rows, 779 11.5; 96 wide, 200 rows, 200 1.1, 280 -1.3; 512 rows, 440 1.0, 520 -1.8;
-//                       768 rows, 516 2.4, 600 -3.8; 1024 rows, 608 2.7, 672 -1.4; 2048 rows, 672 6.2, 800 0.6; 128 wide, 200 rows, 200 1.0, 280 -0.4;
-//                       512 rows, 440 0.5, 520 -1.1; 1024 rows, 512 3.5, 608 -1.9; 2048 rows, 672 2.6, 800 -4.8; 64 wide, 3500 rows, 990 11, 1320 3.2; 4096
-//                       rows, 576 21, 704 0.4; 96 wide, 3500 rows, 990 5.8, 1155 -11; 128 wide, 3500 rows, 880 6.7, 1155 -18; 4096 rows, 1024 6.5, 1152 0
+// Which calls are split in two groups (two waves of 32 rows each, 4 waves a workgroup) and which take blocks of 128 rows and one group.
+// A split costs each of its blocks the meeting of the sums, so it wins as long as all of its blocks of 64 rows run at one time (three
+// workgroups a CU of 64-wide heads, 768 in all, two of others, 512); with walks of up to three tiles only while they are one a CU. Past
+// that, a causal call's longest blocks stand alone at the end, the more the longer they are, and a split halves them: the line rises with the
+// longest walk (keys that a row sees; dK/dV: queries). dK/dV in two groups has short tiles to itself and gains further out. One MI355X, random
+// calls of 24 to 5400 rows (none, ALiBi, lengths, windows), 12 000 in all: the form that these lines pick is 0.03 to 0.3 % slower than the
+// better of the two on average. us with one group and with two at so many blocks of 64 rows:
+//   forward, 64 wide:  128 rows, 640 10.2, 9.5; 784 11.7, 14.2; 320 rows, 784 9.9, 10.8; 1280 rows, 800 22.0, 19.2; 1280, 1080 24.5, 25.2; 2304, 1152 42, 40; 1296 47, 47
+//   96 wide:           192 rows, 288 9.3, 10.1; 512 rows, 440 14.3, 13.0; 520 14.6, 16.0; 1024, 512 20.6, 17.6; 608 21.4, 22.0; 2048, 720 43, 41
+//   128 wide:          256 rows, 280 12.2, 11.5; 512, 512 18.6, 16.4; 640 21, 24; 1111, 504 27, 23; 1152, 648 27.2, 26.3; 1280, 720 30, 33; 1838, 638 42, 36
+// Windows: a block of 128 rows sees as many keys more. All their blocks have as much to do, so none stands alone at the end. (With the
+// window alone as the walk, 4 x 320 rows of 12 heads of 64 with a window of 69 took 10.8 us in one group; two take 8.0.)
 struct Upto { int walk, blocks; };
 template <int N>
 static int blocks_upto(const Upto (&t)[N], int walk) {
-  int b = 0;
+  int b = -1;
   for (const Upto& u : t)
     if (walk >= u.walk) b = u.blocks;
   return b;
 }
+static int longest_walk(int rows, int window) { return window > 0 && window < rows ? min(rows, min(window + 128, 512)) : rows; }
 static long long halves(int rows, int heads) { return (rows + 63ll) / 64 * heads; }
 static bool split_rows(int rows, int heads, int d, int keys, int window, bool dq) {
-  static const Upto f64[] = {{33, 200}, {97, 620}, {640, 700}, {1000, 768}, {2300, 1000}, {3800, 1200}};
-  static const Upto f96[] = {{65, 200}, {97, 260}, {129, 320}, {300, 520}, {1400, 490}, {1900, 520}, {2300, 720}, {3800, 800}};
-  static const Upto f128[] = {{97, 280}, {256, 320}, {512, 450}, {900, 620}, {1400, 660}, {1900, 720}, {2300, 780}, {3800, 900}};
-  static const Upto q64[] = {{33, 200}, {129, 560}, {2000, 610}}, odd64[] = {{129, 790}, {1400, 920}, {2300, 1150}};  // (rows % 128 == 0; others)
-  static const Upto q96[] = {{65, 200}, {97, 260}, {240, 340}, {300, 480}, {640, 520}, {900, 620}, {1400, 680}, {1900, 720}, {2300, 1000}};
-  static const Upto q128[] = {{65, 200}, {97, 250}, {300, 300}, {440, 480}, {900, 520}, {1400, 670}, {1900, 720}, {2300, 880}, {3400, 1024}};
-  const int walk = window > 0 ? min(keys, window) : keys;
-  const long long n = halves(rows, heads);
-  if (dq)
-    return n <= (d == 64 ? (walk > 128 && rows % 128 ? blocks_upto(odd64, walk) : blocks_upto(q64, walk))
-                 : d == 96 ? blocks_upto(q96, walk)
-                           : blocks_upto(q128, walk));
-  return n <= (d == 64 ? blocks_upto(f64, walk) : d == 96 ? blocks_upto(f96, walk) : blocks_upto(f128, walk));
+  static const Upto f64[] = {{33, 260}, {97, 790}, {1000, 880}, {1900, 1200}}, q64[] = {{65, 260}, {256, 800}, {900, 1000}, {1400, 1200}};
+  static const Upto f96[] = {{65, 270}, {129, 520}, {900, 600}, {1400, 640}, {1900, 740}, {3000, 840}};
+  static const Upto q96[] = {{65, 260}, {256, 512}, {700, 640}, {1000, 800}, {2300, 950}};
+  static const Upto f128[] = {{33, 258}, {129, 514}, {1000, 640}, {1400, 720}, {2300, 800}, {3500, 900}};
+  static const Upto q128[] = {{65, 260}, {256, 500}, {700, 600}, {1000, 800}, {2300, 1000}};
+  const int walk = longest_walk(keys, window);
+  const int upto = d == 64   ? (dq ? blocks_upto(q64, walk) : blocks_upto(f64, walk))
+                   : d == 96 ? (dq ? blocks_upto(q96, walk) : blocks_upto(f96, walk))
+                             : (dq ? blocks_upto(q128, walk) : blocks_upto(f128, walk));
+  return halves(rows, heads) <= upto;
 }
 // dK/dV with one group or two, or, 128 wide, 0, 1 or in two groups of four waves (2, by blocks of 128 rows): there two groups of two take 81 KB of
 // LDS, one workgroup a CU. us, backward with one group, and what two groups (of four waves) take or save:
-//   64 wide:   96 rows, 600 blocks of 64 rows 18.8, -0.5, 680 18.7, +0.2; 200 rows, 680 22.9, -0.7, 800 23.3, +1.1; 512 rows, 800 37.0, -1.4, 960 37.3,
-//              +0.9; 768 rows, 516 42.9, -3.8, 600 43.5, +1.0; 1200 rows, 760 59.1, -5.5, 912 61.3, -2.9; 1500 rows, 960 75.0, -4.9, 1128 83.6, +1.5;
-//              2048 rows, 512 84.0, -12.7, 608 94.1, +0.5; 2600 rows, 943 119, -7.1; 3500 rows, 1320 170, -5.2, 1485 188, +5.3; 4096 rows, 576 163, -21, 704
-//              179, 0 (before tiles went straight into LDS:) a window of 256, 576 20.2,
-//              18.2, 672 41.6, -2.6, 960 43.8, +5.8
-//   96 wide:   96 rows, 200 17.4, -0.8, 280 18.0, +0.3; 200 rows, 440 25.0, -0.6, 520 28.7, +1.5; 320 rows, 500 32.5, -3.5, 565 32.3, +2.7; 512 rows, 520
-//              38.8, -0.9, 600 41.2, +0.5; 768 rows, 684 52.8, -0.8, 804 55.7, +2.1; 1024 rows, 672 64.5, -4.5, 800 67.3, -0.9; 1500 rows, 960 96.8,
-//              -1.9, 1128 110, +8; 2048 rows, 800 119, -9, 960 127, +6; 3500 rows, 880 190, -19, 990 203, +9; (before:)
-//              64 rows, 60 13.9, -1.3, 1200 50.2, -3.9; a window of 32 or 64, 240
-//              25, -5, 448 28, -2.5, 680 35, +1
-//   128 wide:  200 rows, 200 26.0, -1.9 (-1.0), 280 26.9, -0.3 (-0.5); 256 rows, 200 29.3, -2.6 (-1.6), 280 30.5, +1.3 (-1.5), 360 31.9, +2.9 (-1.4), 520
-//              37.4, +10 (+4.7); 512 rows, 280 43.1, -4.8 (-4.1), 360 44.0, -0.9 (-3.8), 520 48.9, +7.8 (-2.2), 600 51.0, +9.7 (+0.6); 768 rows, 960
-//              75.6, +16 (-2.1), 1116 87, +27 (+6); 1024 rows, 352 67.1, -10.6 (-8.7), 448 67.4, -4.7 (-7.6), 672 77.9, +8.5 (-6.6); 1200 rows, 912 94.3,
-//              +18 (-5.4); 2048 rows, 352 116, -22 (-19), 448 117, -16 (-17), 1120 170, +35 (-2.0), 1280 172, +43 (+1.7); 3000 rows, 1128 223, +40
-//              (-10), 1316 244, +54 (+8); 4096 rows, 512 226, -40 (-37), 1280 315, +54 (-7), 1472 346, +112 (+20); (before:) 32 rows, 60 12.7,
-//              +0.4; 64 rows, 220 17.5, -0.9; a window of 256, 192 40.2, -7.1 (-2.2), 288 43.1, +2.5 (-2.3), 528 48.3, +7.8 (+3.0)
-static int split_keys(int keys, int heads, int d, int rows, int window, bool alibi) {
-  static const Upto t64[] = {{33, 320}, {65, 640}, {129, 690}, {256, 900}, {2300, 1320}};  // (the form START; with ALiBi or a window, in blocks of 128 rows:)
-  static const Upto m64[] = {{33, 340}, {512, 480}, {768, 560}, {1536, 768}};
-  static const Upto t96[] = {{0, 760}, {65, 210}, {97, 430}, {256, 510}, {512, 600}, {768, 700}, {1400, 860}, {1900, 900}};
-  static const Upto t128[] = {{33, 220}, {65, 120}, {97, 250}, {300, 290}, {768, 350}, {1400, 420}};
-  static const Upto w128[] = {{129, 220}, {256, 240}, {384, 260}, {600, 320}, {768, 480}, {1800, 560}, {2300, 600}, {3400, 680}};
-  const bool win = window > 0 && window < rows;
-  const int walk = win ? window : rows;
-  const long long blocks = (keys + 127ll) / 128 * heads, n = halves(keys, heads);
-  if (d == 128 && win) return blocks <= 120 ? 1 : blocks <= 220 ? 2 : 0;
-  if (d == 64 && (alibi || window > 0)) return blocks <= blocks_upto(m64, walk);
-  const int upto = d == 96    ? (win && walk < 65 ? 560 : blocks_upto(t96, walk))
-                   : d == 128 ? blocks_upto(t128, walk)
-                              : walk >= 700 && keys % 128 == 0 ? (walk < 2300 ? 560 : 600) : blocks_upto(t64, walk);
-  if (n <= upto) return 1;
-  return d == 128 && blocks <= blocks_upto(w128, walk) ? 2 : 0;
+//   64 wide:   200 rows, 680 blocks of 64 rows 22.9, -0.7; 800 23.3, +1.1; 768, 600 43.5, +1.0; 1200, 912 61.3, -2.9; 3500, 1320 170, -5.2; 1485 188, +5.3
+//   96 wide:   64 rows, 1200 50.2, -3.9; 200, 440 25.0, -0.6; 520 28.7, +1.5; 768, 684 52.8, -0.8; 804 55.7, +2.1; 1500, 960 96.8, -1.9; 1128 110, +8
+//   128 wide:  200 rows, 200 26.0, -1.9 (-1.0); 512, 280 43.1, -4.8 (-4.1); 360 44.0, -0.9 (-3.8); 520 48.9, +7.8 (-2.2); 600 51.0, +9.7 (+0.6); 1024, 672 77.9,
+//              +8.5 (-6.6); 2048, 448 117, -16 (-17); 1120 170, +35 (-2.0); 1280 172, +43 (+1.7); 4096, 512 226, -40 (-37); 1280 315, +54 (-7)
+static int split_keys(int keys, int heads, int d, int rows, int window) {
+  static const Upto t64[] = {{33, 1 << 30}, {65, 800}, {400, 970}, {900, 1400}}, t96[] = {{0, 1 << 30}, {65, 516}, {400, 700}, {700, 860}, {1700, 1100}};
+  static const Upto t128[] = {{33, 258}, {700, 360}, {1700, 450}}, w128[] = {{97, 260}, {640, 553}};
+  const int walk = longest_walk(rows, window);
+  if (halves(keys, heads) <= (d == 64 ? blocks_upto(t64, walk) : d == 96 ? blocks_upto(t96, walk) : blocks_upto(t128, walk))) return 1;
+  return d == 128 && (keys + 127ll) / 128 * heads <= blocks_upto(w128, walk) ? 2 : 0;
 }
 
 template <class F>
@@ -816,8 +785,9 @@ static int with_form(int d, bool alibi, F&& f) {
 }
 
 // Causal calls of 64, 96 and 128 wide heads with 16-byte rows; 1: another head size (or, backward, a scale of nothing).
-// (Three workgroups a CU where the registers of 96-wide rows allow it without spills, ALiBi's dQ does not, and the blocks of a CU are to add up to
-// the same: 1 x 1500 x 64 forward 53 -> 46 us, backward 139 -> 134. Windowed dQ, all blocks alike, is 2 % faster with two.)
+// 96-wide rows in one group: three workgroups a CU where there are more than two, though their registers are then tight (1 x 1500 x 64 forward 53
+// -> 46 us, backward 139 -> 134; up to 512 blocks of 128 rows the third never runs, and the forward takes 1 to 2 % longer, the whole
+// backward 2 to 3 %). ALiBi's dQ would spill.
 int attn_fwd_split(const FastFwdParams& p, int d, hipStream_t stream) {
   const long long blocks = (long long)((p.Sq + 127) / 128) * p.B * p.H;
   const bool two = split_rows(p.Sq, p.B * p.H, d, p.Sk, p.window, false);
@@ -825,8 +795,10 @@ int attn_fwd_split(const FastFwdParams& p, int d, hipStream_t stream) {
     constexpr int D = decltype(D_)::value, G = decltype(G_)::value, W = D == 64 ? 3 : 2;
     if (two)
       hipLaunchKernelGGL((attn_fwd_split_kernel<D, G, 2, 2, W>), dim3((p.Sq + 63) / 64 * p.B * p.H), dim3(256), 0, stream, p);
+    else if (D == 96 && blocks > 512)
+      hipLaunchKernelGGL((attn_fwd_split_kernel<D, G, 4, 1, D == 96 ? 3 : W>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
     else
-      hipLaunchKernelGGL((attn_fwd_split_kernel<D, G, 4, 1, (D < 128 ? 3 : 2)>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((attn_fwd_split_kernel<D, G, 4, 1, W>), dim3((unsigned)blocks), dim3(256), 0, stream, p);
   });
 }
 
@@ -834,15 +806,15 @@ int attn_bwd_split(const FastBwdParams& p, int d, hipStream_t stream) {
   if (!(fabsf(p.scale) >= 1e-30f)) return 1;  // the sums start with lse / scale: the generic kernel's
   const long long qblocks = (long long)((p.Sq + 127) / 128) * p.B * p.H, kblocks = (long long)((p.Sk + 127) / 128) * p.B * p.Hkv;
   const bool two = split_rows(p.Sq, p.B * p.H, d, p.Sk, p.window, true);
-  const int kv = split_keys(p.Sk, p.B * p.Hkv, d, p.Sq, p.window, p.alibi);
+  const int kv = split_keys(p.Sk, p.B * p.Hkv, d, p.Sq, p.window);
   return with_form(d, p.alibi, [&](auto D_, auto G_) {
     constexpr int D = decltype(D_)::value, G = decltype(G_)::value, W = D == 64 ? 3 : 2;
     if (two)
       hipLaunchKernelGGL((attn_bwd_dq_split_kernel<D, G, 2, 2, W>), dim3((p.Sq + 63) / 64 * p.B * p.H), dim3(256), 0, stream, p);
-    else if (p.window > 0)
-      hipLaunchKernelGGL((attn_bwd_dq_split_kernel<D, G, 4, 1, W>), dim3((unsigned)qblocks), dim3(256), 0, stream, p);
-    else
+    else if (D == 96 && G == 1 && qblocks > 512)
       hipLaunchKernelGGL((attn_bwd_dq_split_kernel<D, G, 4, 1, D == 96 && G == 1 ? 3 : W>), dim3((unsigned)qblocks), dim3(256), 0, stream, p);
+    else
+      hipLaunchKernelGGL((attn_bwd_dq_split_kernel<D, G, 4, 1, W>), dim3((unsigned)qblocks), dim3(256), 0, stream, p);
     auto dkdv = [&](auto WIN_) {
       constexpr bool WIN = decltype(WIN_)::value;
       if (kv == 1)

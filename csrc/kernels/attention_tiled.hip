@@ -1514,11 +1514,7 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
   const bool aligned = rows16(q, q_sb, q_st, q_sh) && rows16(k, k_sb, k_st, k_sh) && rows16(v, v_sb, v_st, v_sh) &&
                        rows16(o, o_sb, o_st, o_sh);
   const bool general = alibi || kv_len || window || cu || Sq % 128 || Sk % 32;  // (these forms take the row sums as everywhere else)
-  // 64 wide, full tiles of many blocks: the plain form, whose masks are simpler, though its overflowed rows take a launch of their own
-  // (us, split, plain: 128 rows, 960 blocks 19.3, 18.8, 1920 31.7, 30.2, 3840 56.4, 52.8; 384, 480 13.9, 13.6, 1920 38.2, 35.9; 1024, 480
-  // 22.5, 22.7, 1920 59.7, 57.6; on the host a launch is some 3). 96 and 128 wide gain and lose 5 %.
-  const bool plain = d == 64 && !general && (long long)(Sq / 128) * B * H >= 1900;
-  if (causal && aligned && !plain && (general || (rowsum_col < 0 && max_col < 0))) {
+  if (causal && aligned && (general || (rowsum_col < 0 && max_col < 0))) {
     const int rc = attn_fwd_split(p, d, stream);
     if (rc != 1) return rc ? rc : -1;
   }
@@ -1527,7 +1523,7 @@ KCA_API int kca_attn_fwd_tiled(const void* q, const void* k, const void* v, void
   //   2 x 2048, 14 heads of 128, ALiBi       198 -> 80, 345 -> 303    1 x 1500, 64 heads of 96       177 -> 66, 366 -> 234
   //   4 x 1100, 16 heads of 256              194 -> 77, 685 -> 307    8 x 1000, 12 heads of 64        59 -> 36, 181 -> 145
   //   4 x 2048, 16 heads of 256, lengths     528 -> 203, 1870 -> 815  2 x 2048, 20 of 128, window 256  68 -> 39, 148 -> 137
-  // Full tiles without another mask, where they come here (not causal; 160 wide; 64 wide in many blocks; 256 wide in whole blocks of 256
+  // Full tiles without another mask, where they come here (not causal; 160 wide; 256 wide in whole blocks of 256
   // rows), keep the plain form, whose loops have no edge to test: 4 x 2048 of 256 179 us against 203 forward, 8 x 1024 of 64, not
   // causal, 36 and 137 with the backward against 36 and 146.
   bool whole = false;  // the kernel leaves no row to the fixup launch
@@ -1654,10 +1650,10 @@ KCA_API int kca_attn_bwd_tiled(const void* q, const void* k, const void* v, cons
   const bool aligned = rows16(q, q_sb, q_st, q_sh) && rows16(k, k_sb, k_st, k_sh) && rows16(v, v_sb, v_st, v_sh) &&
                        rows16(o, o_sb, o_st, o_sh) && rows16(dout, do_sb, do_st, do_sh) && rows16(dq, dq_sb, dq_st, dq_sh) &&
                        rows16(dk, dk_sb, dk_st, dk_sh) && rows16(dv, dv_sb, dv_st, dv_sh);
-  // 64 wide, full tiles: the plain forms from 300 blocks on (us, split, plain: 128 rows, 120 blocks 14.0, 14.3, 240 17.6, 15.9, 480 26.4,
-  // 24.5, 1920 81.9, 75.3; 384, 240 25.9, 25.8, 960 60.8, 57.5; 1024, 240 46.0, 51.7, 480 60.1, 57.5, 1920 171.7, 164.2; 96 wide lose up
-  // to 12 %, 128 wide gain and lose 4 %)
-  const bool plain = d == 64 && !(alibi || kv_len || window || Sq % 128 || Sk % 128) && (long long)(Sq / 128) * B * H >= 300;
+  // 64 wide, full tiles of a few keys: the plain forms, whose masks are simpler, where the split ones are not in two groups (plain over split,
+  // blocks of 128 rows: 128 rows 260 1.02, 380 .96, 700 .94, 2400 .99; 256 rows 300 1.04, 420 .98, 1000 .96; 384 rows 380 1.07, 420 .97, 1000 .98; 512 rows 500
+  // 1.03, 1000 1.01; 1024 and more 300 1.34, 500 1.10, 1000 1.04. Forward, split forms are 2 to 11 % faster with any number of blocks)
+  const bool plain = d == 64 && !(alibi || kv_len || window || Sq % 128 || Sk % 128) && Sk <= 384 && (long long)(Sq / 128) * B * H > 400;
   if (aligned && !plain) {
     (void)hipGetLastError();
     const int rc = d == 256 ? attn_bwd_pair(p, d, causal, stream) : causal ? attn_bwd_split(p, d, stream) : 1;

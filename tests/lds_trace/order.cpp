@@ -25,6 +25,6 @@ int check() {
 }
 
 int main() {
-  return check<true, 64, 64, 3>() + check<true, 64, 128, 3>() + check<true, 96, 64, 1>() + check<true, 96, 128, 1>() + check<true, 160, 128, 1>() + check<true, 128, 128, 1>() +
+  return check<true, 64, 64, 3>() + check<true, 64, 128, 3>() + check<true, 96, 64, 1>() + check<true, 96, 128, 1>() + check<true, 96, 128, 3>() + check<true, 160, 128, 1>() + check<true, 128, 128, 1>() +
          check<true, 256, 128, 1>() + check<true, 256, 256, 1>() + check<false, 64, 128, 1>() != 0;
 }

@@ -21,7 +21,7 @@ def test_one_group(D, S):
 
 @pytest.mark.parametrize("Sq,Sk", [(128, 128), (384, 384), (256, 512)])
 def test_full_tiles_of_many_blocks(Sq, Sk):
-    """64-wide heads: the plain forms, forward from 1900 blocks on, backward from 300."""
+    """64-wide heads: the plain forms of the backward, up to 384 keys and from 400 blocks on, and the split ones beside them."""
     _check(10, Sq, Sk, 20, 10, 64, True)
     _check(20, Sq, Sk, 96 if Sq == 128 else 48, 48, 64, True)
 
@@ -141,3 +141,20 @@ def test_column_of_ones(D, mask):
     with torch.no_grad():
         o = flash_attention(q, k, v, causal=True, kv_len=ln, alibi=sl, window=window, rowsum_col=40)
     _close(o, attention_reference(q.float(), k.float(), v.float(), True, None, ln, sl, window)[0])
+
+
+@pytest.mark.parametrize("D,B,S,H,window,groups", [
+    (64, 4, 320, 12, 69, 2), (64, 5, 228, 20, 49, 2), (128, 1, 360, 14, 92, 2), (128, 2, 320, 14, 91, 2), (96, 8, 251, 12, 96, 2),  # few blocks
+    (64, 10, 320, 32, 69, 1), (128, 5, 832, 14, 159, 1), (96, 1, 2419, 20, 134, 1),                                                # many
+    (64, 1, 1600, 32, 0, 2), (64, 1, 1280, 64, 0, 1), (64, 12, 97, 12, 0, 2), (64, 40, 97, 12, 0, 1), (96, 1, 2048, 20, 0, 2), (96, 16, 181, 12, 0, 1),
+    (128, 1, 1280, 30, 0, 2), (128, 1, 1280, 40, 0, 1)])
+def test_which_calls_are_split(D, B, S, H, window, groups):
+    """A windowed call is split by the keys that its blocks see, not by the window alone; results in either form."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q, k, v = (torch.randn(B, S, H, D, device="cuda", generator=g).bfloat16() for _ in range(3))
+    with torch.no_grad(), torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        o = flash_attention(q, k, v, causal=True, window=window)
+        torch.cuda.synchronize()
+    names = [e.key for e in prof.key_averages() if "attn_fwd_split_kernel" in e.key]
+    assert len(names) == 1 and f"<{D}, 1, {4 // groups}, {groups}, " in names[0], names
+    _close(o, attention_reference(q.float(), k.float(), v.float(), causal=True, window=window)[0])
