@@ -744,7 +744,7 @@ static int blocks_upto(const Upto (&t)[N], int walk) {
 static int longest_walk(int rows, int window) { return window > 0 && window < rows ? min(rows, min(window + 128, 512)) : rows; }
 static long long halves(int rows, int heads) { return (rows + 63ll) / 64 * heads; }
 static bool split_rows(int rows, int heads, int d, int keys, int window, bool dq) {
-  static const Upto f64[] = {{33, 260}, {97, 790}, {1000, 880}, {1900, 1200}}, q64[] = {{65, 260}, {256, 800}, {900, 1000}, {1400, 1200}};
+  static const Upto f64[] = {{33, 260}, {97, 768}, {400, 790}, {1000, 880}, {1900, 1200}}, q64[] = {{65, 260}, {256, 768}, {900, 1000}, {1400, 1200}};
   static const Upto f96[] = {{65, 270}, {129, 520}, {900, 600}, {1400, 640}, {1900, 740}, {3000, 840}};
   static const Upto q96[] = {{65, 260}, {256, 512}, {700, 640}, {1000, 800}, {2300, 950}};
   static const Upto f128[] = {{33, 258}, {129, 514}, {1000, 640}, {1400, 720}, {2300, 800}, {3500, 900}};
@@ -762,7 +762,7 @@ static bool split_rows(int rows, int heads, int d, int keys, int window, bool dq
 //   128 wide:  200 rows, 200 26.0, -1.9 (-1.0); 512, 280 43.1, -4.8 (-4.1); 360 44.0, -0.9 (-3.8); 520 48.9, +7.8 (-2.2); 600 51.0, +9.7 (+0.6); 1024, 672 77.9,
 //              +8.5 (-6.6); 2048, 448 117, -16 (-17); 1120 170, +35 (-2.0); 1280 172, +43 (+1.7); 4096, 512 226, -40 (-37); 1280 315, +54 (-7)
 static int split_keys(int keys, int heads, int d, int rows, int window) {
-  static const Upto t64[] = {{33, 1 << 30}, {65, 800}, {400, 970}, {900, 1400}}, t96[] = {{0, 1 << 30}, {65, 516}, {400, 700}, {700, 860}, {1700, 1100}};
+  static const Upto t64[] = {{33, 1 << 30}, {65, 770}, {400, 970}, {900, 1400}}, t96[] = {{0, 1 << 30}, {65, 516}, {400, 700}, {700, 860}, {1700, 1100}};
   static const Upto t128[] = {{33, 258}, {700, 360}, {1700, 450}}, w128[] = {{97, 260}, {640, 553}};
   const int walk = longest_walk(rows, window);
   if (halves(keys, heads) <= (d == 64 ? blocks_upto(t64, walk) : d == 96 ? blocks_upto(t96, walk) : blocks_upto(t128, walk))) return 1;

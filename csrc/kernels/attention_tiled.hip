@@ -1651,9 +1651,9 @@ KCA_API int kca_attn_bwd_tiled(const void* q, const void* k, const void* v, cons
                        rows16(o, o_sb, o_st, o_sh) && rows16(dout, do_sb, do_st, do_sh) && rows16(dq, dq_sb, dq_st, dq_sh) &&
                        rows16(dk, dk_sb, dk_st, dk_sh) && rows16(dv, dv_sb, dv_st, dv_sh);
   // 64 wide, full tiles of a few keys: the plain forms, whose masks are simpler, where the split ones are not in two groups (plain over split,
-  // blocks of 128 rows: 128 rows 260 1.02, 380 .96, 700 .94, 2400 .99; 256 rows 300 1.04, 420 .98, 1000 .96; 384 rows 380 1.07, 420 .97, 1000 .98; 512 rows 500
-  // 1.03, 1000 1.01; 1024 and more 300 1.34, 500 1.10, 1000 1.04. Forward, split forms are 2 to 11 % faster with any number of blocks)
-  const bool plain = d == 64 && !(alibi || kv_len || window || Sq % 128 || Sk % 128) && Sk <= 384 && (long long)(Sq / 128) * B * H > 400;
+  // blocks of 128 rows: 128 rows 384 1.00, 432 .94, 1000 .96, 2400 .99; 256 rows 320 1.08, 384 1.02, 400 .92, 1000 .96; 384 rows 384 1.08, 420 .96, 1000 .98; 512
+  // rows 384 1.14, 512 1.02, 1000 1.01; 1024 and more 300 1.34, 500 1.10, 1000 1.04. Forward, split forms are 2 to 11 % faster with any number of blocks)
+  const bool plain = d == 64 && !(alibi || kv_len || window || Sq % 128 || Sk % 128) && Sk <= 384 && (long long)(Sq / 128) * B * H > 384;
   if (aligned && !plain) {
     (void)hipGetLastError();
     const int rc = d == 256 ? attn_bwd_pair(p, d, causal, stream) : causal ? attn_bwd_split(p, d, stream) : 1;

@@ -21,7 +21,7 @@ def test_one_group(D, S):
 
 @pytest.mark.parametrize("Sq,Sk", [(128, 128), (384, 384), (256, 512)])
 def test_full_tiles_of_many_blocks(Sq, Sk):
-    """64-wide heads: the plain forms of the backward, up to 384 keys and from 400 blocks on, and the split ones beside them."""
+    """64-wide heads: the plain forms of the backward, up to 384 keys and past 384 blocks, and the split ones beside them."""
     _check(10, Sq, Sk, 20, 10, 64, True)
     _check(20, Sq, Sk, 96 if Sq == 128 else 48, 48, 64, True)
 
@@ -158,3 +158,16 @@ def test_which_calls_are_split(D, B, S, H, window, groups):
     names = [e.key for e in prof.key_averages() if "attn_fwd_split_kernel" in e.key]
     assert len(names) == 1 and f"<{D}, 1, {4 // groups}, {groups}, " in names[0], names
     _close(o, attention_reference(q.float(), k.float(), v.float(), causal=True, window=window)[0])
+
+
+@pytest.mark.parametrize("B,S,H,plain", [(10, 256, 20, True), (16, 256, 12, False), (11, 384, 12, True), (4, 384, 32, False), (10, 512, 20, False), (4, 1024, 20, False)])
+def test_which_backwards_are_plain(B, S, H, plain):
+    """64-wide heads, full tiles."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q, k, v = (torch.randn(B, S, H, 64, device="cuda", generator=g).bfloat16().requires_grad_() for _ in range(3))
+    o = flash_attention(q, k, v, causal=True)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        o.backward(torch.ones_like(o))
+        torch.cuda.synchronize()
+    names = [e.key for e in prof.key_averages() if "attn_bwd_dq" in e.key or "attn_bwd_dkdv" in e.key]
+    assert len(names) == 2 and all(("_tiled_" if plain else "_split_") in n for n in names), names
