@@ -243,8 +243,8 @@ struct TileRequests {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(to)),
                  "v"(from_[j]), "s"(words), "s"(so)
                  : "m0");
-#else
-    *reinterpret_cast<u32x4*>(image + at_ + j * 1024 + threadIdx.x % 64 * 16) = u32x4{};  // (what a trace of LDS accesses on the host sees)
+#elif defined(LDS_TRACE)  // (a host build that follows requests and accesses)
+    lds_request(image + at_ + j * 1024 + threadIdx.x % 64 * 16);
 #endif
   }
 };
@@ -256,7 +256,8 @@ __device__ __forceinline__ void wait_and_meet() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-#else
+#elif defined(LDS_TRACE)
+  lds_wait(N);
   __syncthreads();
 #endif
 }

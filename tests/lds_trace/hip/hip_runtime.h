@@ -30,7 +30,11 @@ typedef int hipError_t;
 constexpr int hipSuccess = 0;
 static inline int hipGetLastError() { return 0; }
 
-void barrier();                           // trace.cpp
+// trace.cpp
+#define LDS_TRACE
+void barrier();
+void lds_request(void* p);  // 16 bytes that memory writes there until a wait retires the request
+void lds_wait(int newest);  // all of the thread's requests but its newest ones are retired
 void run(dim3 grid, dim3 block, void (*thread)(void*), void* what);
 extern float trace_weight;                      // what exp2 gives: large, and all sums of softmax weights overflow
 static inline void __syncthreads() { barrier(); }

@@ -5,7 +5,7 @@
 #include "../../csrc/kernels/attention_split.hip"
 #include "../../csrc/kernels/attention_pair.hip"
 
-extern long long trace_accesses, trace_races;
+extern long long trace_accesses, trace_requests, trace_races;
 
 int main(int argc, char** argv) {
   if (argc != 12) return 2;
@@ -37,6 +37,6 @@ int main(int argc, char** argv) {
     p.do_sh = p.dq_sh = p.dk_sh = p.dv_sh = D;
     rc = D == 256 ? attn_bwd_pair(p, D, true, nullptr) : attn_bwd_split(p, D, nullptr);
   }
-  printf("accesses %lld\nraces %lld\n", trace_accesses, trace_races);
+  printf("accesses %lld\nrequests %lld\nraces %lld\n", trace_accesses, trace_requests, trace_races);
   return rc;
 }

@@ -25,8 +25,8 @@ def trace(tmp_path_factory):
     def run(kernel, *args, **env):
         r = subprocess.run([exe, kernel, *map(str, args)], capture_output=True, text=True, env=dict(os.environ, **env))
         assert r.returncode == 0, r.stderr
-        last = dict(line.rsplit(" ", 1) for line in r.stdout.splitlines()[-2:])
-        assert int(last["accesses"]) > 1000
+        last = dict(line.rsplit(" ", 1) for line in r.stdout.splitlines()[-3:])
+        assert int(last["accesses"]) > 1000 and int(last["requests"]) > 1000
         return int(last["races"]), r.stdout
     return run
 
@@ -51,6 +51,13 @@ def test_the_trace_sees_exchanges(trace):
     """Without the barriers every tile that one wave stores and another reads is reported."""
     for kernel, D in (("fwd", 64), ("bwd", 64), ("bwd", 256)):
         assert trace(kernel, D, *FEW, *MASKS["plain"], 1, LDS_TRACE_NO_BARRIERS="1")[0] > 1000
+
+
+@pytest.mark.parametrize("kernel,D", [("fwd", 64), ("fwd", 96), ("fwd", 128), ("bwd", 64), ("bwd", 96), ("bwd", 128), ("bwd", 256)])
+@pytest.mark.parametrize("shape", [FEW, MANY, EIGHT])
+def test_every_wait_is_needed_in_full(trace, kernel, D, shape):
+    """With waits that leave one request more on its way, tiles are read that may not have come."""
+    assert trace(kernel, D, *shape, *MASKS["plain"], 1, LDS_TRACE_LAX="1")[0] > 100
 
 
 def test_every_block_is_taken_once(tmp_path):
