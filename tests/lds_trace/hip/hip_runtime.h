@@ -34,6 +34,8 @@ static inline int hipGetLastError() { return 0; }
 #define LDS_TRACE
 void barrier();
 void lds_request(void* p);  // 16 bytes that memory writes there until a wait retires the request
+unsigned lds_offset(const void* p);
+void lds_request_at(unsigned at);  // the same by its offset
 void lds_wait(int newest);  // all of the thread's requests but its newest ones are retired
 void run(dim3 grid, dim3 block, void (*thread)(void*), void* what);
 extern float trace_weight;                      // what exp2 gives: large, and all sums of softmax weights overflow
@@ -65,6 +67,9 @@ struct __amdgpu_buffer_rsrc_t {};
 #define __builtin_amdgcn_make_buffer_rsrc(...) __amdgpu_buffer_rsrc_t()
 #define __builtin_amdgcn_raw_buffer_load_b128(...) v4u(0)
 #define __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, ...) ((void)(a), (void)(b), (c))
+#define __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, ...) ((void)(a), (void)(b), (c))
+#define __builtin_amdgcn_s_barrier() barrier()
+#define __builtin_amdgcn_s_setprio(x) ((void)0)
 #define __builtin_amdgcn_fdot2(a, b, c, ...) (c)
 #define __builtin_amdgcn_fdot2_f32_bf16(a, b, c, ...) (c)
 static inline v4b __builtin_amdgcn_ds_read_tr16_b64_v4bf16(const __attribute__((address_space(3))) v4b* p) {

@@ -88,8 +88,10 @@ void barrier() {
   epoch += count;
 }
 
-void lds_request(void* p) {
-  const long long at = (const char*)p - &__start_lds;
+unsigned lds_offset(const void* p) { return (unsigned)((const char*)p - &__start_lds); }
+void lds_request(void* p) { lds_request_at(lds_offset(p)); }
+void lds_request_at(unsigned offset) {
+  const long long at = offset;
   if (at < 0 || at % 16 || at + 16 > lds_bytes()) abort();
   pending.push_back({at, epoch, ++event});
 }

@@ -1,4 +1,4 @@
-"""LDS of the attention kernels whose wave groups stage tiles for each other: between two barriers no wave may read what another
+"""LDS of the attention kernels and expert tiles whose waves stage tiles for each other: between two barriers no wave may read what another
 writes. The kernels' own source runs on the host, thread after thread, with a callback at every load and store (lds_trace/)."""
 import os
 import re
@@ -15,14 +15,15 @@ pytestmark = pytest.mark.skipif(not os.path.exists(CLANG), reason="no clang of R
 def trace(tmp_path_factory):
     d, src = str(tmp_path_factory.mktemp("lds_trace")), os.path.join(ROOT, "tests", "lds_trace")
     base = [CLANG, "-x", "c++", "-std=c++17", "-w", "-mavx512f", "-I" + src]
-    objs = [os.path.join(d, n) for n in ("trace.o", "kernels.o")]
-    subprocess.run([*base, "-O1", "-c", os.path.join(src, "trace.cpp"), "-o", objs[0]], check=True)
-    subprocess.run([*base, "-O0", "-fsanitize-coverage=func,trace-pc,trace-loads,trace-stores", "-c",
-                    os.path.join(src, "kernels.cpp"), "-o", objs[1]], check=True)
-    exe = os.path.join(d, "trace")
-    subprocess.run([CLANG, *objs, "-o", exe], check=True)
+    obj = lambda n: os.path.join(d, n + ".o")  # noqa: E731
+    subprocess.run([*base, "-O1", "-c", os.path.join(src, "trace.cpp"), "-o", obj("trace")], check=True)
+    for name in ("kernels", "experts"):
+        subprocess.run([*base, "-O0", "-fsanitize-coverage=func,trace-pc,trace-loads,trace-stores", "-c",
+                        os.path.join(src, name + ".cpp"), "-o", obj(name)], check=True)
+        subprocess.run([CLANG, obj("trace"), obj(name), "-o", os.path.join(d, name)], check=True)
 
     def run(kernel, *args, **env):
+        exe = os.path.join(d, "experts" if kernel in ("stream", "turns") else "kernels")
         r = subprocess.run([exe, kernel, *map(str, args)], capture_output=True, text=True, env=dict(os.environ, **env))
         assert r.returncode == 0, r.stderr
         last = dict(line.rsplit(" ", 1) for line in r.stdout.splitlines()[-3:])
@@ -58,6 +59,17 @@ def test_the_trace_sees_exchanges(trace):
 def test_every_wait_is_needed_in_full(trace, kernel, D, shape):
     """With waits that leave one request more on its way, tiles are read that may not have come."""
     assert trace(kernel, D, *shape, *MASKS["plain"], 1, LDS_TRACE_LAX="1")[0] > 100
+
+
+@pytest.mark.parametrize("kernel,rows", [("stream", 5), ("stream", 16), ("stream", 32), ("turns", 40), ("turns", 128), ("turns", 192), ("turns", 250)])
+@pytest.mark.parametrize("up", [0, 1])
+def test_expert_tiles(trace, kernel, rows, up):
+    """Numbers of stages around those that are requested ahead, and around the four waves of the stream."""
+    for stages in (1, 2, 3, 4, 5, 8, 9, 17):
+        races, out = trace(kernel, up, rows, stages)
+        assert races == 0, (stages, out)
+    assert trace(kernel, up, rows, 9, LDS_TRACE_LAX="1")[0] > 100
+    assert trace(kernel, up, rows, 9, LDS_TRACE_NO_BARRIERS="1")[0] > 100
 
 
 def test_every_block_is_taken_once(tmp_path):
