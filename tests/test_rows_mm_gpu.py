@@ -38,21 +38,31 @@ def test_rows_against_float32(dtype, rows, n, k, bias):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows", [1, 2, 3])
-@pytest.mark.parametrize("n,k", [(16, 64), (4096, 1984), (4112, 1984), (4112, 2048), (1040, 8192), (1040, 8256), (272, 16448)])
-def test_one_and_two_rows(dtype, rows, n, k):
-    """On both sides of the lines between the vector kernel and the rows' one, eager and replayed."""
+@pytest.mark.parametrize("n,k", [(16, 64), (4096, 1984), (4112, 1984), (4112, 2048), (1040, 8192), (1040, 8256), (272, 16448),
+                                 (16384, 1984), (16384, 2048), (12288, 4096)])
+def test_one_and_two_rows(dtype, rows, n, k, monkeypatch):
+    """On both sides of the lines between the vector kernel and the rows' one; eager, and replayed where a capture takes them (the others are
+    the library's there)."""
     x, w, b, ref = _inputs(rows, n, k, dtype, True)
+    call, names = _lib.call, []
+    monkeypatch.setattr(_lib, "call", lambda name, *a: (names.append(name), call(name, *a))[1])
+    bf16 = dtype == torch.bfloat16
+    vector = (rows == 1 or (rows == 2 and bf16 and k <= 8192)) and (k >= 2048 or n <= 4096)
+    own = ("kca_skinny_gemm" if bf16 else "kca_skinny_gemm_f16") if vector else "kca_rows_mm"
+    captured = few_rows(rows, n, k, True)
+    assert captured == ((n, k) in [(16, 64), (16384, 1984), (16384, 2048), (12288, 4096)])
     with torch.no_grad():
         y = linear_rows(x, w, b)
-        assert _close(y, ref) and _close(linear_rows(x, w), F.linear(x.float(), w.float()))
+        assert _close(y, ref) and _close(linear_rows(x, w), F.linear(x.float(), w.float())) and names == [own] * 2
         graph = torch.cuda.CUDAGraph()
         with capture.graph(graph, stream=torch.cuda.Stream()):
             z = linear_rows(x, w, b)
+        assert names == [own] * (3 if captured else 2)
         for _ in range(3):
             z.zero_()
             graph.replay()
             torch.cuda.synchronize()
-            assert _close(z, ref) and torch.equal(linear_rows(x, w, b), y)
+            assert _close(z, ref) and torch.equal(linear_rows(x, w, b), y) and (not captured or torch.equal(z, y))
 
 
 @pytest.mark.parametrize("rows,n,k", [(61, 4096, 4096), (128, 4096, 4096)])
