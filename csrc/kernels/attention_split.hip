@@ -763,7 +763,7 @@ static bool split_rows(int rows, int heads, int d, int keys, int window, bool dq
 //              +8.5 (-6.6); 2048, 448 117, -16 (-17); 1120 170, +35 (-2.0); 1280 172, +43 (+1.7); 4096, 512 226, -40 (-37); 1280 315, +54 (-7)
 static int split_keys(int keys, int heads, int d, int rows, int window) {
   static const Upto t64[] = {{33, 1 << 30}, {65, 770}, {400, 970}, {900, 1400}}, t96[] = {{0, 1 << 30}, {65, 516}, {400, 700}, {700, 860}, {1700, 1100}};
-  static const Upto t128[] = {{33, 258}, {700, 360}, {1700, 450}}, w128[] = {{97, 260}, {640, 553}};
+  static const Upto t128[] = {{33, 258}, {700, 340}, {1200, 384}, {1700, 416}, {2600, 450}}, w128[] = {{97, 260}, {640, 553}};
   const int walk = longest_walk(rows, window);
   if (halves(keys, heads) <= (d == 64 ? blocks_upto(t64, walk) : d == 96 ? blocks_upto(t96, walk) : blocks_upto(t128, walk))) return 1;
   return d == 128 && (keys + 127ll) / 128 * heads <= blocks_upto(w128, walk) ? 2 : 0;
