@@ -125,12 +125,13 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
         4104, 16, 2, 2056: r 3: 179, 154; 8: 335, 180      1032, 16, 2, 520: r 4: 34, 22      4104, 16, 2, 4104: r 3: 334, 337; 4: 376, 329
     Narrow, 128 rows or 192: the larger tile saves a second one a little over 128 rows and costs one over 192; uneven experts
     have more than 128 from some 100 on, and where rows are long it costs nothing from 56 on (4096, 16, 3, 2048 of 20 outputs, the largest
-    expert at twice the mean: 400: 200, 191; 467: 218, 187; 600: 212, 194; five layers with other routing .99 to 1.02). Without
-    so many blocks two thirds of the 512 places have to be taken, or a tile's length counts for more than
-    their number: time of 192 rows over that of 128 at 115 to 175 rows (even, uneven and very uneven routing) of 256 to 320 blocks
-    0.98 to 1.07 (8 layers; 2048, 28, 4, 640: 1.00, 1.03, 1.03; 1024, 64, 6, 320: .93, 1.03, 1.01), of 352 (1536, 32, 4, 704) .97, .91,
-    .91, of 384 .96, .92, .91; .92, .97, .97; .97, .94, .97; .95, .90, .99 (2048, 24, 4, 1024; 2048, 32, 5, 768; 3072, 24, 4, 1024; 4096, 16, 3,
-    1536), of 432 to 480 .85 to .90, .93 to 1.02, 1.0 to 1.06; at 90 to 105 rows 1.0 to 1.04.
+    expert at twice the mean: 400: 200, 191; 467: 218, 187; 600: 212, 194; five layers with other routing .99 to 1.02). Without so
+    many blocks two thirds of the 512 places have to be taken, or a tile's length counts for more than their number, and r has to be
+    past 130, as identity outputs count as experts here. Time of 192 rows over that of 128 at 115 to 175 rows (even, uneven
+    and very uneven routing), 256 to 320 blocks .98 to 1.07 (8 layers; 2048, 28, 4, 640: 1.00, 1.03, 1.03), 352 (1536, 32, 4, 704) .97, .91, .91,
+    384 (four layers) .92 to .97, .90 to .97, .91 to .99, 432 to 480 .85 to .90, .93 to 1.02, 1.0 to 1.06; with a quarter of identity outputs:
+        2048, 24, 5, 768: r 104: 82, 83; 121: 84, 82; 136: 86, 84     2048, 30, 5, 704: 121: 93, 99; 136: 103, 102; 145: 105, 101
+        2048, 24, 4, 896: 121: 86, 89; 136: 103, 92                   2048, 36, 5, 640: 121: 91, 99; 136: 95, 100; 145: 103, 101
     Narrow, wide: a wide block is alone on its CU. It wins where the matrix cores bound the products, from about 150 rows (64
     where a contraction is long), if its rounds are well filled (``fill``: the blocks' time over that of the rounds that they
     take; identity outputs count as experts here, so it is an estimate):
@@ -170,7 +171,7 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
                     return GEMM_ROWS
             elif r > 96 and (short >= 4096 or (short >= 1024 and r > 512)):
                 return GEMM_ROWS
-            two = r > (56 if short >= 2048 else 100) if full else r > 115 and 3 * blocks >= 2 * 512  # a 128-row tile is often not enough
+            two = r > (56 if short >= 2048 else 100) if full else r > 130 and 3 * blocks >= 2 * 512  # a 128-row tile is often not enough
             return 192 if (two and r <= 175) or r > 240 else 128
         if stream and T > SHARED_ROWS and r > (2.25 if d > 2048 else 1):
             return STREAM_ROWS

@@ -17,10 +17,10 @@ def test_few_tokens(T, top, E, d, F, rows):
 
 
 @pytest.mark.parametrize("top,E,d,F,r,rows", [
-    (5, 32, 2048, 768, 121, 192), (4, 32, 1536, 704, 121, 192), (6, 64, 1024, 448, 121, 192), (2, 12, 4096, 1920, 121, 192),
-    (4, 40, 2048, 512, 121, 128), (4, 28, 2048, 640, 121, 128), (5, 32, 2048, 768, 110, 128), (5, 32, 2048, 768, 180, 256)])
+    (5, 32, 2048, 768, 136, 192), (4, 32, 1536, 704, 136, 192), (6, 64, 1024, 448, 136, 192), (2, 12, 4096, 1920, 136, 192),
+    (4, 40, 2048, 512, 136, 128), (4, 28, 2048, 640, 136, 128), (5, 32, 2048, 768, 121, 128), (5, 32, 2048, 768, 180, 256)])
 def test_larger_tiles_by_blocks(top, E, d, F, r, rows):
-    """Tiles of 192 rows from 115 expected rows on where the blocks of 64 weight rows take two thirds of the 512 places."""
+    """Tiles of 192 rows past 130 expected rows where the blocks of 64 weight rows take two thirds of the 512 places."""
     assert tile_rows(round(r * E / top), top, E, d, F, torch.bfloat16) == rows
 
 
