@@ -897,11 +897,22 @@ __device__ __forceinline__ GemmPlace gemm_place(const ExpertArgs& p, int nt, int
 // at a time 437 instead of 386.) Returns -1 past the XCD's last.
 __device__ __forceinline__ int turns_place(const ExpertArgs& p, int nt, int nb) {
   int n[4] = {0, 0, 0, 0};  // tiles of 4 .. 1 runs of 64 rows
-  for (int i = 0; i < nt; i += 64) {
-    const int t = i + (threadIdx.x & 63), u = t < nt ? (p.tiles[t * 5 + 2] + 63) / 64 : 0;
+  const int lane = threadIdx.x & 63;
+  auto count = [&](int rows) {
 #pragma unroll
-    for (int b = 0; b < 4; ++b) n[b] += __popcll(__ballot(u == 4 - b));
+    for (int b = 0; b < 4; ++b) n[b] += __popcll(__ballot((rows + 63) / 64 == 4 - b));
+  };
+  int i = 0;
+  // Many tiles: eight loads at one time, as the block has nothing else to do. (One by one, both products of 1.9 million tokens, top 4, 16 experts of 3 x
+  // 512 x 512, 29695 tiles, 126.6 ms, 120.7 in the four waves' blocks that were here before; so 42. 262144 tokens, 4111 tiles 6.4 -> 4.7.)
+  for (; i + 512 <= nt; i += 512) {
+    int rows[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) rows[j] = p.tiles[(i + 64 * j + lane) * 5 + 2];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) count(rows[j]);
   }
+  for (; i < nt; i += 64) count(i + lane < nt ? p.tiles[(i + lane) * 5 + 2] : 0);
   const int x = blockIdx.x & 7;
   int y = blockIdx.x >> 3, first = 0;
 #pragma unroll

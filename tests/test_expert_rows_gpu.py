@@ -101,6 +101,23 @@ def test_wide_tiles(counts, d, F):
         assert (y - want).norm() <= TOL * want.norm()
 
 
+@pytest.mark.parametrize("tiles", [511, 512, 513, 577, 1088])
+def test_many_wide_tiles(tiles):
+    """Blocks count the tiles of each size 512 and 64 at a time; one size ends within the last of them, or all stand past the first 512."""
+    few = [250, 64, 577, 1, 0, 129, 300]
+    counts = few + [(tiles - sum(-(-c // 256) for c in few)) * 256 - 100]
+    d, F = 64, 128
+    h, ids, wts, gu, dn = _case(counts, 1, d, F)
+    g = moe.group(ids, len(counts), moe.GEMM_ROWS)
+    assert int(g.ntiles) == tiles
+    y = moe.experts(h, ids, wts, gu, dn, g, False)[g.inv.view(-1).long()].float()
+    for e in range(len(counts)):
+        k = ids.view(-1) == e
+        u = h[k].float() @ gu[e].float().T
+        want = (torch.nn.functional.silu(u[:, :F]) * u[:, F:]).bfloat16().float() @ dn[e].float().T * wts.view(-1)[k, None]
+        assert (y[k] - want).norm() <= TOL * want.norm() and torch.isfinite(y[k]).all()
+
+
 @pytest.mark.parametrize("tiles", [65535, 65536, 66000])
 def test_more_tiles_than_16_bits_count(tiles):
     """Tiles of up to 256 rows: the counts of a size are packed in 16 bits, up to as many."""
