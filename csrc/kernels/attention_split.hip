@@ -728,8 +728,8 @@ __global__ void __launch_bounds__(64 * RW * KG, WPS) attn_bwd_dkdv_split_kernel(
 // longest walk (keys that a row sees; dK/dV: queries). dK/dV in two groups has short tiles to itself and gains further out. One MI355X, random
 // calls of 24 to 5400 rows (none, ALiBi, lengths, windows), 12 000 in all: the form that these lines pick is 0.03 to 0.3 % slower than the
 // better of the two on average. us with one group and with two at so many blocks of 64 rows:
-//   forward, 64 wide:  128 rows, 640 10.2, 9.5; 784 11.7, 14.2; 320 rows, 784 9.9, 10.8; 1280 rows, 800 22.0, 19.2; 1280, 1080 24.5, 25.2; 2304, 1152 42, 40; 1296 47, 47
-//   96 wide:           192 rows, 288 9.3, 10.1; 512 rows, 440 14.3, 13.0; 520 14.6, 16.0; 1024, 512 20.6, 17.6; 608 21.4, 22.0; 2048, 720 43, 41
+//   forward, 64 wide:  128 rows, 640 10.2, 9.5; 784 11.7, 14.2; 512 rows, 768 12.9, 12.0; 784 13.4, 14.6; 600 rows, 780 14.4, 16.4; 1280 rows, 800 22.0, 19.2; 1280, 1080 24.5, 25.2; 2304, 1152 42, 40; 1296 47, 47
+//   96 wide:           192 rows, 252 (168 of 128 rows) 8.8, 8.5; 264 (176) 9.0, 9.7; 396 (264) 11.4, 10.7; 512 rows, 440 14.3, 13.0; 520 14.6, 16.0; 1024, 512 20.6, 17.6; 608 21.4, 22.0; 2048, 720 43, 41
 //   128 wide:          256 rows, 280 12.2, 11.5; 512, 512 18.6, 16.4; 640 21, 24; 1111, 504 27, 23; 1152, 648 27.2, 26.3; 1280, 720 30, 33; 1838, 638 42, 36
 // Windows: a block of 128 rows sees as many keys more. All their blocks have as much to do, so none stands alone at the end. (With the
 // window alone as the walk, 4 x 320 rows of 12 heads of 64 with a window of 69 took 10.8 us in one group; two take 8.0.)
@@ -744,7 +744,7 @@ static int blocks_upto(const Upto (&t)[N], int walk) {
 static int longest_walk(int rows, int window) { return window > 0 && window < rows ? min(rows, min(window + 128, 512)) : rows; }
 static long long halves(int rows, int heads) { return (rows + 63ll) / 64 * heads; }
 static bool split_rows(int rows, int heads, int d, int keys, int window, bool dq) {
-  static const Upto f64[] = {{33, 260}, {97, 768}, {400, 790}, {1000, 880}, {1900, 1200}}, q64[] = {{65, 260}, {256, 768}, {900, 1000}, {1400, 1200}};
+  static const Upto f64[] = {{33, 260}, {97, 768}, {850, 790}, {1000, 880}, {1900, 1200}}, q64[] = {{65, 260}, {256, 768}, {900, 1000}, {1400, 1200}};
   static const Upto f96[] = {{65, 270}, {129, 520}, {900, 600}, {1400, 640}, {1900, 740}, {3000, 840}};
   static const Upto q96[] = {{65, 260}, {256, 512}, {700, 640}, {1000, 800}, {2300, 950}};
   static const Upto f128[] = {{33, 258}, {129, 514}, {1000, 640}, {1400, 720}, {2300, 800}, {3500, 900}};
@@ -753,6 +753,10 @@ static bool split_rows(int rows, int heads, int d, int keys, int window, bool dq
   const int upto = d == 64   ? (dq ? blocks_upto(q64, walk) : blocks_upto(f64, walk))
                    : d == 96 ? (dq ? blocks_upto(q96, walk) : blocks_upto(f96, walk))
                              : (dq ? blocks_upto(q128, walk) : blocks_upto(f128, walk));
+  // Two blocks of few tiles a head, forward: one group, too, while its blocks are one a CU and those of 64 rows would be two. (Not windows, whose
+  // blocks have less to do each: 8 x 300 rows of 8 heads of 96, a window of 16 to 90, two take .80 to .89 of one's time.)
+  const long long blocks = (rows + 127ll) / 128 * heads;
+  if (d != 64 && !dq && keys > 128 && keys <= 220 && blocks > 170 && blocks <= 256 && !(window > 0 && window < keys)) return false;
   return halves(rows, heads) <= upto;
 }
 // dK/dV with one group or two, or, 128 wide, 0, 1 or in two groups of four waves (2, by blocks of 128 rows): there two groups of two take 81 KB of

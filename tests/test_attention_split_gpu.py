@@ -147,7 +147,8 @@ def test_column_of_ones(D, mask):
     (64, 4, 320, 12, 69, 2), (64, 5, 228, 20, 49, 2), (128, 1, 360, 14, 92, 2), (128, 2, 320, 14, 91, 2), (96, 8, 251, 12, 96, 2),  # few blocks
     (64, 10, 320, 32, 69, 1), (128, 5, 832, 14, 159, 1), (96, 1, 2419, 20, 134, 1),                                                # many
     (64, 1, 1600, 32, 0, 2), (64, 1, 1280, 64, 0, 1), (64, 12, 97, 12, 0, 2), (64, 40, 97, 12, 0, 1), (96, 1, 2048, 20, 0, 2), (96, 16, 181, 12, 0, 1),
-    (128, 1, 1280, 30, 0, 2), (128, 1, 1280, 40, 0, 1)])
+    (128, 1, 1280, 30, 0, 2), (128, 1, 1280, 40, 0, 1), (64, 12, 512, 8, 0, 2), (64, 6, 600, 13, 0, 1),
+    (96, 7, 192, 12, 0, 2), (96, 11, 192, 8, 0, 1), (96, 11, 192, 12, 0, 2), (128, 11, 192, 8, 0, 1), (128, 5, 220, 25, 0, 1), (128, 8, 221, 12, 0, 2), (96, 11, 192, 8, 60, 2)])
 def test_which_calls_are_split(D, B, S, H, window, groups):
     """A windowed call is split by the keys that its blocks see, not by the window alone; results in either form."""
     g = torch.Generator(device="cuda").manual_seed(1)
