@@ -14,7 +14,7 @@
 // Backward, us, one wave and a pair: 2 x 2048 x 16 heads 300, 266; 1 x 2048 225, 184; 1 x 4096 522, 454; 4 x 1100 234, 198; 8 x 512
 // with lengths 128, 108; 1 x 3000 with ALiBi 361, 285; 3 x 300 56, 46; 1 x 61 24.7, 21.8. That was with tiles through the first wave's registers,
 // for which the last quarter of K's fragments had to lie in LDS and be read again at each step; requested into LDS, pairs, before and now:
-// 2 x 2048 254, 241 (dK/dV 160, 146; dQ 130, 120); 1 x 2048 182, 166; 1 x 4096 447, 420; 1 x 3000 with ALiBi 278, 259; 3 x 300 46.7, 44.1.
+// 2 x 2048 254, 241 (dK/dV 137, 129; dQ 114, 108); 1 x 2048 182, 166; 1 x 4096 447, 420; 1 x 3000 with ALiBi 278, 259; 3 x 300 46.7, 44.1.
 // What bounds them: the LDS reads of both waves, 256 KB of a step of dK/dV, 192 of dQ (2048, 1536 cycles at 128 bytes), beside as many cycles in
 // the matrix cores, and what of a wave's own chain the other does not cover. No gain: deeper rings of fragments, wave priorities, a walk that touches
 // tiles ahead, heads turned over the XCDs, dQ's columns half to the first wave, with dS through LDS (130, 137: the reads stay as many).
