@@ -195,6 +195,89 @@ __device__ __forceinline__ void expert_stream_tile(const ExpertArgs& p, char* sl
 }
 constexpr int STREAM_LDS = 4 * (3 * 4096 + 2 * 4 * 1024);
 
+// The same tiles x 128 weight rows (up: 64 gate rows and the 64 up rows beside them) that walk K by themselves, 32 of them a wave; all waves read a
+// stage's activations, requested once: 20 KB a stage, three stages ahead, two workgroups a CU. It has a quarter of the blocks, starts and
+// sums over waves, and half as many requests a weight row where tiles have more than 16 rows, but its weights come at 4.7 to 4.9 TB/s. So it is the
+// better one where the walk is short for its rows (stream_block).
+constexpr int BWN = 128, BSTAGE = (BWN + SROWS) * SK * 2;
+static_assert(4 * BSTAGE == STREAM_LDS, "four stages");
+template <bool UP>
+__device__ __forceinline__ void expert_block_tile(const ExpertArgs& p, char* sl, int ex, int lo, int nr, int n0) {
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, g = lane >> 4, K = p.K, N = p.N, nk = K / SK;
+  const u32x4 rw = uniform_words(reinterpret_cast<const bf16_t*>(p.w) + (long long)ex * (UP ? 2 * N : N) * K);
+  const u32x4 rx = uniform_words(reinterpret_cast<const bf16_t*>(p.x) + (UP ? 0ll : (long long)lo * K));
+  // a wave requests its own 32 weight rows and 8 of the activations'
+  unsigned wo[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = 8 * i + (lane >> 3), n = UP ? (i < 2 ? 0 : N) + min(n0 + wv * 16 + (r & 15), N - 1) : min(n0 + wv * 32 + r, N - 1);
+    wo[i] = ((unsigned)n * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
+  }
+  const int xr = wv * 8 + (lane >> 3), row = min(xr, nr - 1);
+  const unsigned xo = ((unsigned)(UP ? p.perm[lo + row] / p.top : row) * K + 8 * ((lane & 7) ^ ((xr >> 1) & 7))) * 2;
+  const unsigned base = __builtin_amdgcn_readfirstlane(lds_address(sl));
+  auto request = [&](int t) {
+    const int k = __builtin_amdgcn_readfirstlane(min(t, nk - 1) * SK * 2);  // past the end: the last one, which nobody reads
+    const unsigned at = base + t % 4 * BSTAGE;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) request_into_lds(rw, at + (wv * 4 + i) * 1024, wo[i], k);
+    request_into_lds(rx, at + (16 + wv) * 1024, xo, k);
+  };
+  f32x4 acc[2][2];  // [gate, up | two runs of 16 outputs][16 rows]
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int sw = (r16 >> 1) & 7;
+#pragma unroll
+  for (int t = 0; t < 3; ++t) request(t);
+  for (int t = 0; t < nk; ++t) {
+    wait_requests_and_reads<10>();  // the wave's pieces of stage t have landed and it has read stage t - 1; so have all others'
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    request(t + 3);  // where stage t - 1 was
+    const char* const st = sl + t % 4 * BSTAGE;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int c = ((4 * s + g) ^ sw) * 16;
+      bf16x8 a[2], x[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) a[i] = *reinterpret_cast<const bf16x8*>(st + (wv * 32 + 16 * i + r16) * 128 + c);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) x[j] = *reinterpret_cast<const bf16x8*>(st + (BWN + 16 * j + r16) * 128 + c);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], x[j], acc[i][j], 0, 0, 0);
+    }
+  }
+  wait_requests<0>();  // the repeated stages, before the LDS is given back
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int r = 16 * j + r16;
+    if (r >= nr) continue;
+    const float s = p.scale ? p.wts[p.perm[lo + r]] : 1.f;
+    bf16_t* y = reinterpret_cast<bf16_t*>(p.y) + (long long)(lo + r) * N;
+#pragma unroll
+    for (int i = 0; i < (UP ? 1 : 2); ++i) {
+      const int n = n0 + wv * (UP ? 16 : 32) + 16 * i + 4 * g;
+      if (n >= N) continue;
+      float o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (UP) {
+          const float gt = acc[0][j][e] * s, up = acc[1][j][e] * s;
+          o[e] = gt * __builtin_amdgcn_rcpf(1.f + __expf(-gt)) * up;
+        } else {
+          o[e] = acc[i][j][e] * s;
+        }
+      }
+      *reinterpret_cast<uint2*>(y + n) = make_uint2(pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3]));
+    }
+  }
+}
+
 // ------------------------------------------------------------------------------------------------ turns
 constexpr int GBK = 64, GN = 256, GM = 256, GEMM_LDS = 2 * (GN + GM) * GBK * 2, WIDE_LDS = GEMM_LDS / 4 * 5;
 

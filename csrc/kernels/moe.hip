@@ -682,6 +682,34 @@ __global__ void __launch_bounds__(256, 2) expert_stream_kernel(ExpertArgs p) {
   else expert_stream_tile<UP, 4>(p, sl, tl[0], tl[1], nr, bn * NB);
 }
 
+template <bool UP>
+__global__ void __launch_bounds__(256, 2) expert_block_kernel(ExpertArgs p) {
+  extern __shared__ __attribute__((aligned(1024))) char sl[];
+  constexpr int NB = UP ? BWN / 2 : BWN;
+  const int nt = *p.ntiles, nb = (p.N + NB - 1) / NB, b = block_number();
+  if (b >= nt * nb) return;
+  const int id = xcd_remap(b, nt * nb);  // the order of expert_gemm_kernel
+  const int* t0 = p.tiles + id / nb * 5;
+  const int in = id - t0[3] * nb, tile = t0[3] + in % t0[4], bn = in / t0[4];
+  const int* tl = p.tiles + tile * 5;
+  expert_block_tile<UP>(p, sl, tl[0], tl[1], tl[2], bn * NB);
+}
+
+// Whether a product of up to 32 rows a tile goes to blocks of 128 weight rows: past (K - 704) / 48 rows an expert, or, where blocks of 32 run all
+// at one time, (K - 256) / 64; at most 30. One product, us, blocks of 32 weight rows and of 128 (outputs x K, experts):
+//   down 1024 x 512, 64: 5 rows 15.4, 13.1; 16 rows 22.1, 18.2
+//   down 2048 x 768, 24: 3 rows 15.7, 17.0; 5 rows 18.4, 18.4; 12 rows 21.6, 19.4; 20 rows 23.8, 19.1
+//   down 2048 x 1024, 32: 5 rows 19.9, 20.8; 12 rows 28.2, 24.1; 26 rows 37.9, 34.3
+//   up 512 x 1024, 16: 5 rows 9.2, 10.4; 12 rows 10.9, 11.3; 16 rows 13.5, 11.4; 26 rows 13.7, 11.1
+//   up 704 x 1536, 32: 8 rows 25.6, 27.7; 16 rows 32.3, 31.5; 20 rows 35.1, 32.7
+//   up 1024 x 2048, 32: 20 rows 57.9, 62.6; 26 rows 62.1, 61.7; 34 rows 67.8, 60.9    down 4096 x 4096, 8: 20 rows 57.4, 71.4; 34 rows 67.0, 67.2
+static bool stream_block(int up, int N, int K, int top, int x_rows, int max_tiles) {
+  const long long n = up ? (long long)x_rows * top : x_rows;
+  const long long used = max_tiles - n / SROWS > 1 ? max_tiles - n / SROWS : 1;  // (max_tiles: experts and whole tiles)
+  const bool once = used * ((N + (up ? SWN / 2 : SWN) - 1) / (up ? SWN / 2 : SWN)) <= 512;
+  return n > 30 * used || (once ? 64 * n > (K - 256ll) * used : 48 * n > (K - 704ll) * used);
+}
+
 // ------------------------------------------------------------------------------------------------ gemm
 // bf16, tiles of up to 256 rows x 256 weight rows (up: 128 gate rows and the 128 up rows beside them) x 64 per stage;
 // weights are the A operand, so a lane holds one activation row and runs of four outputs.
@@ -1113,14 +1141,13 @@ KCA_API int kca_moe_expert(int dtype, const void* x, const void* w, void* y, con
   }
   if (mt == SROWS) {
     if (dtype != 1 || K % SK || N % 16 || !al16(x) || !al16(w) || (uintptr_t)y % 8 || far) return 10;
-    const void* kern = up ? (const void*)expert_stream_kernel<true> : (const void*)expert_stream_kernel<false>;
-    if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, STREAM_LDS) != hipSuccess) return 5;
-    const int nb = up ? SWN / 2 : SWN;
+    const bool block = stream_block(up, N, K, top, x_rows, max_tiles);
+    auto kern = block ? (up ? expert_block_kernel<true> : expert_block_kernel<false>) : (up ? expert_stream_kernel<true> : expert_stream_kernel<false>);
+    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, STREAM_LDS) != hipSuccess) return 5;
+    const int nb = (block ? BWN : SWN) / (up ? 2 : 1);
     const long long blocks = (N + nb - 1ll) / nb * max_tiles;
     if (blocks >= 1ll << 31) return 10;
-    const dim3 grid = block_rows(blocks);
-    if (up) hipLaunchKernelGGL(expert_stream_kernel<true>, grid, dim3(256), STREAM_LDS, s, a);
-    else hipLaunchKernelGGL(expert_stream_kernel<false>, grid, dim3(256), STREAM_LDS, s, a);
+    hipLaunchKernelGGL(kern, block_rows(blocks), dim3(256), STREAM_LDS, s, a);
     return hipGetLastError() == hipSuccess ? 0 : 4;
   }
   const int v = dtype == 1 ? 8 : 4;

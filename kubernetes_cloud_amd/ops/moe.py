@@ -118,9 +118,11 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
         4096, 16, 2, 4096: 17: 226, 240; 24: 270, 262      4096, 16, 3, 2048: 17: 158, 135
         2048, 32, 4, 1024: 17: 83, 73; 24: 97, 76          1024, 64, 2, 512: 17: 27, 26; 32: 39, 36
     Stream, narrow: a stream tile holds 32 rows, past which weights are read again, so it ends at 20 rows, as experts are uneven
-    -- at 36 where narrow blocks (``blocks`` of 64 weight rows) are fewer than the 512 that run at one time:
-        4096, 16, 2, 4096: 160: 283, 295; 260: 352, 301    2048, 32, 4, 1024: 128: 85, 87; 200: 92, 89
-        2048, 24, 5, 768: 200: 67, 74; 300: 81, 73         5120, 8, 2, 2560: 100: 134, 149; 160: 170, 154
+    -- at 36 where narrow blocks (``blocks`` of 64 weight rows) are fewer than the 512 that run at one time, at 52 where they are less
+    than half as many (stream tiles then have more of the chip):
+        4096, 16, 2, 4096: 160: 283, 295; 260: 352, 301    2048, 32, 4, 1024: 128: 86, 94; 200: 96, 94; 240: 99, 94
+        2048, 24, 5, 768: 153: 66, 71; 192: 73, 73         1536, 32, 4, 704: 256: 56, 58; 320: 65, 59
+        5120, 8, 2, 2560: 100: 134, 149; 160: 170, 154     1024, 16, 2, 512: 384: 20, 22; 448: 25, 26; 2048, 16, 4, 512: 192: 33, 34; 224: 45, 40
     without it (widths that are no multiple of 64) vector, narrow: 4 rows:
         4104, 16, 2, 2056: r 3: 179, 154; 8: 335, 180      1032, 16, 2, 520: r 4: 34, 22      4104, 16, 2, 4104: r 3: 334, 337; 4: 376, 329
     Narrow, 128 rows or 192: the larger tile saves a second one a little over 128 rows and costs one over 192; uneven experts
@@ -156,7 +158,7 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
         stream = d % 64 == 0 and F % 64 == 0
         r, short, blocks = n / used, min(d, F), used * (F // 64)
         full = blocks >= 512
-        if r > ((20 if full else 36) if stream else 4):
+        if r > ((20 if full else 36 if blocks >= 256 else 52) if stream else 4):
             if stream:
                 tiles = used * -(-r // GEMM_ROWS)
                 up, down = tiles * -(-F // 128), tiles * -(-d // 256)  # wide blocks of the two products; rounds of one a CU

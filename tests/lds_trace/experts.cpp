@@ -1,5 +1,5 @@
-// The expert tiles' own source for the host, every load and store with a callback (trace.cpp). Arguments: "stream" or "turns", 1 for gate and
-// up, rows, stages of 64 of K.
+// The expert tiles' own source for the host, every load and store with a callback (trace.cpp). Arguments: "stream", "block" or "turns", 1 for gate
+// and up, rows, stages of 64 of K.
 #include <stdlib.h>
 
 #include "../../csrc/kernels/expert_tiles.h"
@@ -11,6 +11,11 @@ void stream(ExpertArgs p, int rows) {
   __shared__ __attribute__((aligned(1024))) char sl[STREAM_LDS];
   expert_stream_tile<UP, XI>(p, sl, 0, 0, rows, 16);
 }
+template <bool UP>
+void block(ExpertArgs p, int rows) {
+  __shared__ __attribute__((aligned(1024))) char sl[STREAM_LDS];
+  expert_block_tile<UP>(p, sl, 0, 0, rows, 0);
+}
 template <bool UP, int B>
 void turns(ExpertArgs p, int rows) {
   __shared__ __attribute__((aligned(1024))) char sl[WIDE_LDS];
@@ -18,9 +23,10 @@ void turns(ExpertArgs p, int rows) {
 }
 
 template <bool UP>
-void block(bool wide, const ExpertArgs& p, int rows) {
+void tile(char form, const ExpertArgs& p, int rows) {
   auto go = [&](auto f, int threads) { hipLaunchKernelGGL(f, dim3(1), dim3(threads), 0, nullptr, p, rows); };
-  if (wide) rows > 192 ? go(turns<UP, 4>, 512) : rows > 128 ? go(turns<UP, 3>, 512) : rows > 64 ? go(turns<UP, 2>, 512) : go(turns<UP, 1>, 512);
+  if (form == 't') rows > 192 ? go(turns<UP, 4>, 512) : rows > 128 ? go(turns<UP, 3>, 512) : rows > 64 ? go(turns<UP, 2>, 512) : go(turns<UP, 1>, 512);
+  else if (form == 'b') go(block<UP>, 256);
   else rows > 16 ? go(stream<UP, 4>, 256) : rows > 8 ? go(stream<UP, 2>, 256) : go(stream<UP, 1>, 256);
 }
 
@@ -31,9 +37,8 @@ int main(int argc, char** argv) {
   for (int i = 0; i < rows; ++i) perm[i] = i;
   ExpertArgs p{};
   p.perm = perm, p.wts = (float*)calloc(rows, 4), p.y = calloc(rows * N, 2), p.top = 1, p.N = N, p.K = 64 * atoi(argv[4]), p.scale = 1;
-  const bool wide = argv[1][0] == 't';
-  if (atoi(argv[2])) block<true>(wide, p, rows);
-  else block<false>(wide, p, rows);
+  if (atoi(argv[2])) tile<true>(argv[1][0], p, rows);
+  else tile<false>(argv[1][0], p, rows);
   printf("accesses %lld\nrequests %lld\nraces %lld\n", trace_accesses, trace_requests, trace_races);
   return 0;
 }

@@ -101,6 +101,33 @@ def test_wide_tiles(counts, d, F):
         assert (y - want).norm() <= TOL * want.norm()
 
 
+@pytest.mark.parametrize("d,F,counts,kernels", [
+    (64, 128, [1, 5, 8, 9, 16, 17, 31, 32, 33, 0, 64, 65], "bb"), (640, 576, [3, 4, 2, 0, 33, 2, 1], "bb"), (192, 64, [2, 1, 3], "bb"),
+    (1088, 64, [3, 8, 1, 9, 2, 0, 33, 16], "sb"), (1152, 1088, [8, 9, 16, 17, 1, 0, 7, 12], "ss"), (512, 1216, [9, 5, 31, 8, 12, 7], "bs"), (1024, 8256, [8, 9, 7, 6, 5], "bs"),
+    (1024, 8256, [8, 1, 7, 6, 5], "ss"), (2112, 1984, [0, 1, 8, 9, 16, 17, 32, 33, 40, 64], "ss")])
+def test_stream_and_blocks(d, F, counts, kernels):
+    """The two kernels of up to 32 rows a tile, which the rows of an expert and the length of the walk choose between; 1 to 33 stages, weight rows that
+    end within a block of 128."""
+    h, ids, wts, gu, dn = _case(counts, 1, d, F)
+    g = moe.group(ids, len(counts), moe.STREAM_ROWS)
+    for scale_in in (True, False):
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+            y = moe.experts(h, ids, wts, gu, dn, g, scale_in)
+            torch.cuda.synchronize()
+        names = [e.key for e in prof.key_averages() if "expert_" in e.key]
+        for up, k in zip(("true", "false"), kernels):
+            assert any(f"expert_{'block' if k == 'b' else 'stream'}_kernel<{up}>" in n for n in names), names
+        y = y[g.inv.view(-1).long()].float()
+        want = torch.empty_like(y)
+        for e in range(len(counts)):
+            k = ids.view(-1) == e
+            w = wts.view(-1)[k, None]
+            u = h[k].float() @ gu[e].float().T * (w if scale_in else 1)
+            a = (torch.nn.functional.silu(u[:, :F]) * u[:, F:]).bfloat16().float()
+            want[k] = a @ dn[e].float().T * (1 if scale_in else w)
+        assert (y - want).norm() <= TOL * want.norm()
+
+
 @pytest.mark.parametrize("tiles", [511, 512, 513, 577, 1088])
 def test_many_wide_tiles(tiles):
     """Blocks count the tiles of each size 512 and 64 at a time; one size ends within the last of them, or all stand past the first 512."""

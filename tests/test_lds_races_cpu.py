@@ -23,7 +23,7 @@ def trace(tmp_path_factory):
         subprocess.run([CLANG, obj("trace"), obj(name), "-o", os.path.join(d, name)], check=True)
 
     def run(kernel, *args, **env):
-        exe = os.path.join(d, "experts" if kernel in ("stream", "turns") else "kernels")
+        exe = os.path.join(d, "experts" if kernel in ("stream", "block", "turns") else "kernels")
         r = subprocess.run([exe, kernel, *map(str, args)], capture_output=True, text=True, env=dict(os.environ, **env))
         assert r.returncode == 0, r.stderr
         last = dict(line.rsplit(" ", 1) for line in r.stdout.splitlines()[-3:])
@@ -61,7 +61,7 @@ def test_every_wait_is_needed_in_full(trace, kernel, D, shape):
     assert trace(kernel, D, *shape, *MASKS["plain"], 1, LDS_TRACE_LAX="1")[0] > 100
 
 
-@pytest.mark.parametrize("kernel,rows", [("stream", 5), ("stream", 16), ("stream", 32), ("turns", 40), ("turns", 128), ("turns", 192), ("turns", 250)])
+@pytest.mark.parametrize("kernel,rows", [("stream", 5), ("stream", 16), ("stream", 32), ("block", 9), ("block", 32), ("turns", 40), ("turns", 128), ("turns", 192), ("turns", 250)])
 @pytest.mark.parametrize("up", [0, 1])
 def test_expert_tiles(trace, kernel, rows, up):
     """Numbers of stages around those that are requested ahead, and around the four waves of the stream."""
