@@ -139,14 +139,12 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
     take; identity outputs count as experts here, so it is an estimate):
         4096, 16, 2, 4096: 300: 305, 306; 700: 338, 322; 2500: 610, 505    2048, 32, 4, 1024: 500: 93, 103; 1150: 115, 115; 3000: 211, 172
         4096, 16, 3, 2048: 900: 208, 209; 1500: 295, 227                   2048, 24, 5, 768: 777: 83, 85; 1300: 96, 86; 4096: 231, 189
-        2048, 40, 4, 1024: 1200: 142, 161; 2000: 181, 188                  2048, 10, 2, 2048: 600: 84, 90; 2000: 147, 141
     or with any rows where narrow blocks do not fill the chip and wide ones of both products are one round on more than half of
-    the CUs (blocks of the products; r 40, 80, 110; narrow, wide):
-        4608, 8, 2, 2304 (144, 144): 140, 124; 141, 144; 156, 155     5120, 8, 2, 2560 (160, 160): 161, 138; 173, 161; 179, 187
-        5632, 6, 2, 2816 (132, 132): 166, 143; 173, 159; 187, 180     4352, 8, 2, 2176 (136, 136): 135, 117; 131, 152; 141, 153
-        3072, 12, 2, 2304 (216, 144): 123, 113; 131, 131; 142, 146    5120, 8, 2, 3840 (240, 160): 201, 180; 225, 210; 247, 218
-        4096, 8, 2, 2560 (160, 128): 129, 130; 143, 154; 153, 161     4096, 8, 2, 2048 (128, 128): 100, 109; 106, 124; 108, 132
-        6144, 8, 2, 2048 (128, 192): 148, 169; 154, 179; 194, 189     5120, 6, 2, 5120 (240, 120): 184, 194"""
+    the CUs. Wide over narrow at 40 to 100 rows, 5 layers: even routing .86 to .96, uneven .81 to 1.2, very uneven .87 to 1.3 (blocks of the
+    products; r 40, 80, 110; narrow, wide):
+        5120, 8, 2, 2560 (160, 160): 161, 138; 173, 161; 179, 187     5632, 6, 2, 2816 (132, 132): 166, 143; 173, 159; 187, 180
+        4352, 8, 2, 2176 (136, 136): 135, 117; 131, 152; 141, 153     5120, 8, 2, 3840 (240, 160): 201, 180; 225, 210; 247, 218
+        4096, 8, 2, 2560 (160, 128): 129, 130; 143, 154; 153, 161     5120, 6, 2, 5120 (240, 120): 184, 194"""
     n = T * top
     used = min(E, n)
     # 32-bit offsets into an expert's weights and the rows of a tile (elsewhere only 128-row tiles have longer ones)
