@@ -9,7 +9,7 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int NB = 64, SK = 64, ROWS = 128;  // weight rows a block, K a stage, activation rows at most
+constexpr int SK = 64, ROWS = 128;  // K a stage, activation rows at most
 
 struct RowsPart {
   const void *x, *w, *bias;
@@ -20,7 +20,7 @@ struct RowsArgs {
   // p[0], and beside it p[1] with blocks of its own (beside), or p[1]'s x and W along K: y[0] = x0 W0^T + x1 W1^T + both biases
   // (p[1].K without beside). p[1].K == 0: one product.
   RowsPart p[2];
-  float* ws;      // ks > 1: [block][slice][product tile][2][256 threads][2]
+  float* ws;      // ks > 1: [block][slice][product tile][2][threads][2]
   unsigned* cnt;  // ks > 1: one arrival counter a block, zero before and after
   int M, ks, beside;
 };
@@ -66,6 +66,10 @@ __device__ __forceinline__ void read_frags(unsigned a0, unsigned a1, u32x4 (&r)[
 #endif
 }
 
+// A block's first stage of its walk: neighbours at neighbouring ones, so that they find each other's activations in L2 (spread over all of K
+// 128 rows of 4096 x 16384 40.5, 49.6 us), groups of 8 turned (16384 x 4096, a block a CU: 25.6; one after another 27.4)
+__device__ __forceinline__ int walk_start(int blk, int stages) { return (blk ^ (blk >> 3)) % stages; }
+
 template <bool F16>
 __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
   if constexpr (F16)
@@ -74,29 +78,34 @@ __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// Bound by the weight stream. A block is 64 weight rows x all activation rows (rounded up to XR); a stage's weights and
-// activations, 64 of K each, go straight to LDS (no registers), so 60, 64 or 48 KiB a workgroup (XR 32, 64, 128) and two workgroups
-// a CU are in flight;
+// Bound by the weight stream. A block is NB weight rows x all activation rows (rounded up to XR); a stage's weights and
+// activations, 64 of K each, go straight to LDS (no registers), 64 to 96 KiB a workgroup;
 // the products (weights as the A operand: a lane holds one activation row and four outputs) hide under it. Blocks of 64 rows
-// rather than 128 keep the CUs busy with fewer slices of K, whose partial sums (4 bytes beside 2 of a weight, for every
-// activation row) cost more than reading the activations once a block from L2: 61 rows of 12288 x 4096 26.5 us against 30.1,
-// of 16384 x 4096 32.2 : 36.1, of 4096 x 4096 13.0 : 16.6. Where the blocks are fewer than the CUs, slices of K write partial
-// sums and the last to arrive adds them in slice order. Deeper pipelines with one workgroup a CU were slower (33.2, 27.6).
+// where they are no more than the CUs, or K is sliced: partial sums (4 bytes beside 2 of a weight, for every activation row) cost
+// more than reading the activations once a block from L2 (61 rows of 16384 x 4096 25.4 us, of 4096 x 4096 12.9; blocks of 128 in twice
+// the slices 29.2, 16.2). Where 64 rows make more blocks than CUs, 128 halve what the activations cost (`wide`).
+// Blocks start their walks of K at different stages (`walk_start`): from the same one they read the same columns of all rows, 2K bytes
+// apart, at one time, which few of the memory's channels hold. 61 rows, us, from the first stage and this: 12288 x 4096 26.3, 24.3;
+// 16384 x 4096 32.1, 25.6; 4096 x 16384 34.3, 30.0; 14336 x 14336 93.1, 86.0; loads alone of 16384 x 4096 30.2, 23.8. Weights packed so that a
+// stage is one piece of memory come to the same (24.4). The order of the sums follows from the block, the same at every run.
+// Where the blocks are fewer than the CUs, slices of K write partial sums and the last to arrive adds them in slice order.
 // An LDS-DMA instruction fills 8 rows of 128 bytes lane by lane, so the 16-byte pieces are swizzled (by row pair: 16 rows x one
 // piece cover all 64 banks) on the source address.
-// us, hipBLASLt : this (weights cold; at the copy rate 20.9, 27.8, 7.0, 27.8):
-//   rows   12288 x 4096   16384 x 4096   4096 x 4096   4096 x 16384
-//     16    27.2 : 22.3    31.6 : 30.0   15.6 : 11.5   29.9 : 32.1
-//     64    25.3 : 26.8    33.0 : 32.4   15.4 : 13.0   39.1 : 33.8
-//    128    32.2 : 34.2    36.3 : 38.0   24.4 : 17.6   81.5 : 42.2
-// A call costs the host 14 us, the library's through the tuned table 20 to 26: four GPT-J layers on 61 tokens 944 -> 769 us.
+// us, hipBLASLt : this (weights cold, both in a captured graph; at the copy rate 20.9, 27.8, 7.0, 27.8, 86):
+//   rows   12288 x 4096   16384 x 4096   4096 x 4096   4096 x 16384   50400 x 4096
+//     16    25.8 : 19.3    31.7 : 25.3   15.5 : 14.0   30.1 : 29.6    88.9 : 79.6
+//     64    26.2 : 24.7    31.9 : 25.7   15.4 : 15.2   41.0 : 31.9    90.4 : 81.4
+//    128    32.1 : 34.1    35.4 : 34.5   24.5 : 19.3   79.1 : 42.2    98.8 : 98.3
+// A call costs the host 14 us, the library's through the tuned table 20 to 26.
 // Which sizes run here: few_rows in ops/linear.py.
-// XR activation rows; 4 waves, WM of them across the activation rows; SNB stages.
+// XR activation rows; W waves, WM of them across the activation rows (8 rather than 4 read less from LDS: 61 rows of 2048 x 8192 and x 2048
+// 16.7, 15.9); SNB stages.
 // TWO: another product beside this one, or more of K (RowsArgs).
-template <bool F16, int XR, int WM, int SNB, bool TWO>
-__global__ void __launch_bounds__(256, 2) rows_mm_kernel(RowsArgs p) {
-  constexpr int WN = 4 / WM, A = NB / WN / 16, B = XR / WM / 16;  // a wave's runs of 16 weight and activation rows
-  constexpr int STG = (NB + XR) * SK * 2, WI = NB / 32, XI = XR / 32, PER = WI + XI;
+template <bool F16, int NB, int W, int XR, int WM, int SNB, bool TWO>
+__global__ void __launch_bounds__(64 * W, 2) rows_mm_kernel(RowsArgs p) {
+  constexpr int WN = W / WM, A = NB / WN / 16, B = XR / WM / 16;  // a wave's runs of 16 weight and activation rows
+  constexpr int STG = (NB + XR) * SK * 2, WI = NB / 8 / W, XI = XR / 8 / W, PER = WI + XI;
+  static_assert(WI > 0 && XI > 0 && A > 0 && B > 0);
   extern __shared__ __attribute__((aligned(1024))) char sl[];  // [SNB][NB weight rows | XR activation rows][128 B]
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wn = wv % WN, wm = wv / WN;
   const int r16 = lane & 15, g = lane >> 4;
@@ -128,22 +137,22 @@ __global__ void __launch_bounds__(256, 2) rows_mm_kernel(RowsArgs p) {
   if (TWO) offsets(K2, wo2, xo2);
   typedef __attribute__((address_space(3))) char lds_char;
   lds_char* lsm = (lds_char*)sl;
-  auto issue = [&](int t) {
-    const int tt = __builtin_amdgcn_readfirstlane(min(t, t1 - 1));  // the last stages repeat one that nobody reads
-    lds_char* st = lsm + ((t - t0) % SNB) * STG;
+  const int first = t0 + walk_start(blk, t1 - t0);
+  auto issue = [&](int t) {  // the walk's stage t: the last ones repeat one that nobody reads
+    const int at = first + min(t, t1 - t0 - 1), tt = __builtin_amdgcn_readfirstlane(at < t1 ? at : at - (t1 - t0));
+    lds_char* st = lsm + t % SNB * STG;
 #if defined(__HIP_DEVICE_COMPILE__)
-    auto fill = [&](__amdgpu_buffer_rsrc_t fw, __amdgpu_buffer_rsrc_t fx, const unsigned (&w)[WI], const unsigned (&x)[XI], int k) {
+    const bool one = !TWO || tt < nka;
+    const int k = (one ? tt : tt - nka) * SK * 2;
+    const __amdgpu_buffer_rsrc_t fw = one ? rw : rw2, fx = one ? rx : rx2;
 #pragma unroll
-      for (int i = 0; i < WI; ++i)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(fw, (void __attribute__((address_space(3)))*)(st + (wv * WI + i) * 1024), 16,
-                                                 w[i], k, 0, 0);
+    for (int i = 0; i < WI; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(fw, (void __attribute__((address_space(3)))*)(st + (wv * WI + i) * 1024), 16,
+                                               one ? wo[i] : wo2[i], k, 0, 0);
 #pragma unroll
-      for (int i = 0; i < XI; ++i)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            fx, (void __attribute__((address_space(3)))*)(st + (NB / 8 + wv * XI + i) * 1024), 16, x[i], k, 0, 0);
-    };
-    if (!TWO || tt < nka) fill(rw, rx, wo, xo, tt * SK * 2);
-    else fill(rw2, rx2, wo2, xo2, (tt - nka) * SK * 2);
+    for (int i = 0; i < XI; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(fx, (void __attribute__((address_space(3)))*)(st + (NB / 8 + wv * XI + i) * 1024), 16,
+                                               one ? xo[i] : xo2[i], k, 0, 0);
 #endif
   };
   f32x4 acc[A][B];
@@ -155,13 +164,13 @@ __global__ void __launch_bounds__(256, 2) rows_mm_kernel(RowsArgs p) {
   const unsigned aw = (wn * A * 16 + r16) * 128, ax = (NB + wm * B * 16 + r16) * 128;
   const unsigned c0 = (g ^ sw) * 16, c1 = ((4 + g) ^ sw) * 16;
 #pragma unroll
-  for (int t = 0; t < SNB - 1; ++t) issue(t0 + t);
-  for (int t = t0; t < t1; ++t) {
+  for (int t = 0; t < SNB - 1; ++t) issue(t);
+  for (int t = 0; t < t1 - t0; ++t) {
     // this wave's pieces of stage t have landed (SNB - 2 younger stages may be in flight), then everybody's
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SNB - 2) * PER) : "memory");
     __builtin_amdgcn_s_barrier();
     issue(t + SNB - 1);  // into the buffer of stage t - 1, which all waves have left
-    const unsigned st = base + ((t - t0) % SNB) * STG;
+    const unsigned st = base + t % SNB * STG;
     u32x4 wf[2][A], xf[2][B];
     read_frags(st + aw + c0, st + aw + c1, wf);
     read_frags(st + ax + c0, st + ax + c1, xf);
@@ -174,14 +183,14 @@ __global__ void __launch_bounds__(256, 2) rows_mm_kernel(RowsArgs p) {
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the repeated stages, before the LDS is given back
   if (p.ks > 1) {
-    unsigned long long* part = reinterpret_cast<unsigned long long*>(p.ws) + (long long)blk * p.ks * A * B * 512 + threadIdx.x;
+    unsigned long long* part = reinterpret_cast<unsigned long long*>(p.ws) + (long long)blk * p.ks * A * B * (128 * W) + threadIdx.x;
 #pragma unroll
     for (int i = 0; i < A; ++i)
 #pragma unroll
       for (int j = 0; j < B; ++j)
 #pragma unroll
         for (int h = 0; h < 2; ++h)
-          __hip_atomic_store(part + (z * A * B + i * B + j) * 512 + h * 256,
+          __hip_atomic_store(part + (z * A * B + i * B + j) * (128 * W) + h * (64 * W),
                              __builtin_bit_cast(unsigned long long, f32x2{acc[i][j][2 * h], acc[i][j][2 * h + 1]}),
                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -209,8 +218,8 @@ __global__ void __launch_bounds__(256, 2) rows_mm_kernel(RowsArgs p) {
       for (int i = 0; i < A; ++i)
 #pragma unroll
         for (int j = 0; j < B; ++j) {
-          const auto* q = part + (s * A * B + i * B + j) * 512;
-          const f32x2 lo = __builtin_bit_cast(f32x2, q[0]), hi = __builtin_bit_cast(f32x2, q[256]);
+          const auto* q = part + (s * A * B + i * B + j) * (128 * W);
+          const f32x2 lo = __builtin_bit_cast(f32x2, q[0]), hi = __builtin_bit_cast(f32x2, q[64 * W]);
           sum[i][j] += f32x4{lo[0], lo[1], hi[0], hi[1]};
         }
     }
@@ -255,19 +264,28 @@ __global__ void __launch_bounds__(256, 2) rows_mm_kernel(RowsArgs p) {
   }
 }
 
-template <bool F16, int XR, int WM, int SNB, bool TWO>
+int blocks_of(const RowsArgs& a, int nb) { return (a.p[0].N + nb - 1) / nb + (a.beside ? (a.p[1].N + nb - 1) / nb : 0); }
+
+template <bool F16, int NB, int W, int XR, int WM, int SNB, bool TWO>
 int go_as(const RowsArgs& a, hipStream_t s) {
   constexpr int lds = SNB * (NB + XR) * SK * 2;
-  if (hipFuncSetAttribute((const void*)rows_mm_kernel<F16, XR, WM, SNB, TWO>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) !=
+  if (hipFuncSetAttribute((const void*)rows_mm_kernel<F16, NB, W, XR, WM, SNB, TWO>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) !=
       hipSuccess)
     return 5;
-  const int blocks = (a.p[0].N + NB - 1) / NB + (a.beside ? (a.p[1].N + NB - 1) / NB : 0);
-  hipLaunchKernelGGL((rows_mm_kernel<F16, XR, WM, SNB, TWO>), dim3(blocks * a.ks), dim3(256), lds, s, a);
+  hipLaunchKernelGGL((rows_mm_kernel<F16, NB, W, XR, WM, SNB, TWO>), dim3(blocks_of(a, NB) * a.ks), dim3(64 * W), lds, s, a);
   return hipGetLastError() == hipSuccess ? 0 : 4;
 }
-template <bool F16, int XR, int WM, int SNB>
+template <bool F16, int NB, int W, int XR, int WM, int SNB>
 int go(const RowsArgs& a, hipStream_t s) {
-  return a.p[1].K ? go_as<F16, XR, WM, SNB, true>(a, s) : go_as<F16, XR, WM, SNB, false>(a, s);
+  return a.p[1].K ? go_as<F16, NB, W, XR, WM, SNB, true>(a, s) : go_as<F16, NB, W, XR, WM, SNB, false>(a, s);
+}
+
+// Blocks of 128 weight rows: where 64 make more blocks than CUs and 128 fill whole rounds of them better. us, 61 rows, 64 and 128 a block
+// (x 4096): 18432 44.0, 35.2; 24576 46.9, 37.7; 12288 and 16384 beside each other 51, 41.7; 32768 48.9, 46.1; 50400 93, 80.6; 57344 99.5, 88.6; a
+// second round of a few blocks loses: 36864 70.5, 73.9; 43008 71.9, 77.1; not for 128 rows, whose products cost as much as their weights: 91.8, 88.6.
+bool wide(const RowsArgs& a, int xr) {
+  const int n = blocks_of(a, 128);
+  return a.ks == 1 && blocks_of(a, 64) > 256 && (n <= 256 || n > 384 || xr == 128);
 }
 
 // Checks what the kernel asks of its arguments and launches it
@@ -283,16 +301,22 @@ int rows_mm(int dtype, const RowsArgs& a, long long ws_floats, int cnt_n, hipStr
     if (a.beside && a.ks > q.K / SK) return 1;
     if (!al16(q.x) || !al16(q.w) || (out && (uintptr_t)q.y % 8)) return 2;
     if (2ll * (q.N > a.M ? q.N : a.M) * q.K >= 1ll << 32) return 3;  // (32-bit byte offsets into W and x)
-    if (out) blocks += (q.N + NB - 1) / NB;
+    if (out) blocks += (q.N + 63) / 64;
     stages += q.K / SK;
   }
   if (!a.beside && a.ks > stages) return 1;
-  const long long xr = a.M <= 32 ? 32 : a.M <= 64 ? 64 : 128;
+  const int xr = a.M <= 32 ? 32 : a.M <= 64 ? 64 : 128;
   if (blocks * a.ks >= 1ll << 31) return 3;
-  if (a.ks > 1 && (!a.ws || !a.cnt || !al16(a.ws) || ws_floats < blocks * a.ks * NB * xr || cnt_n < blocks)) return 6;
-  if (xr == 32) return dtype == 2 ? go<true, 32, 1, 6>(a, s) : go<false, 32, 1, 6>(a, s);
-  if (xr == 64) return dtype == 2 ? go<true, 64, 1, 5>(a, s) : go<false, 64, 1, 5>(a, s);
-  return dtype == 2 ? go<true, 128, 2, 3>(a, s) : go<false, 128, 2, 3>(a, s);
+  if (a.ks > 1 && (!a.ws || !a.cnt || !al16(a.ws) || ws_floats < blocks * a.ks * 64 * xr || cnt_n < blocks)) return 6;
+  const bool f16 = dtype == 2;
+  if (wide(a, xr)) {
+    if (xr == 32) return f16 ? go<true, 128, 4, 32, 1, 4>(a, s) : go<false, 128, 4, 32, 1, 4>(a, s);
+    if (xr == 64) return f16 ? go<true, 128, 8, 64, 2, 4>(a, s) : go<false, 128, 8, 64, 2, 4>(a, s);
+    return f16 ? go<true, 128, 8, 128, 2, 3>(a, s) : go<false, 128, 8, 128, 2, 3>(a, s);
+  }
+  if (xr == 32) return f16 ? go<true, 64, 4, 32, 1, 6>(a, s) : go<false, 64, 4, 32, 1, 6>(a, s);
+  if (xr == 64) return f16 ? go<true, 64, 8, 64, 2, 4>(a, s) : go<false, 64, 8, 64, 2, 4>(a, s);
+  return f16 ? go<true, 64, 8, 128, 2, 3>(a, s) : go<false, 64, 8, 128, 2, 3>(a, s);
 }
 
 }  // namespace

@@ -171,27 +171,26 @@ FEW_ROWS = 128
 
 
 def few_rows(rows: int, n: int, k: int, captured: bool = False) -> bool:
-    """Whether a product of few rows goes to the weight-streaming kernel. On the GPU, us, hipBLASLt : the kernel, weights cold:
+    """Whether a product of few rows goes to the weight-streaming kernel. On the GPU, us, hipBLASLt : the kernel, weights cold, in captures
+    (where a product cut over K takes 1.6 to 2 us more, a fill of the graph's own counters):
 
-        12288 x 4096   8 rows 27.3 : 21.9    32: 23.9 : 23.1    64: 25.8 : 26.9    96: 30.5 : 33.6    128: 32.4 : 34.4
-        4096 x 4096           15.8 : 11.3        13.4 : 11.7        15.2 : 13.0        22.4 : 17.2         24.8 : 17.7
-        4096 x 16384          30.4 : 32.4        34.6 : 32.2        39.4 : 34.0        68.7 : 41.3         81.5 : 42.9
-        8192 x 2048           13.2 : 10.8        13.2 : 11.1        13.9 : 12.2        14.6 : 15.6         16.1 : 16.3
-        1024 x 4096           11.4 : 8.7          8.9 : 9.0         12.2 : 10.5         9.0 : 15.2          9.5 : 15.5
-        5120 x 20480           113 : 40           122 : 42           130 : 49           141 : 60            148 : 63
-        14336 x 14336         82.5 : 84.3        84.6 : 84.8        96.1 : 96.5       107.3 : 118.3       119.4 : 127.1
+        12288 x 4096   8 rows 26.1 : 19.3    32: 23.2 : 20.5    64: 26.2 : 24.7    96: 30.5 : 32.5    128: 32.1 : 34.1
+        16384 x 4096          31.9 : 25.4        30.5 : 24.0        31.9 : 25.7        34.0 : 32.8         35.4 : 34.5
+        4096 x 4096           15.9 : 14.0        14.0 : 14.5        15.4 : 15.2        22.3 : 18.7         24.5 : 19.3
+        4096 x 16384          29.6 : 29.6        32.9 : 29.5        41.0 : 31.9        66.4 : 40.7         79.1 : 42.2
+        8192 x 2048           14.7 : 13.3        13.4 : 13.3        13.9 : 14.6        15.0 : 18.2         16.1 : 18.8
+        5120 x 20480           110 : 43           117 : 43           128 : 49           138 : 62            145 : 64
+        14336 x 14336         82.5 : 73.8        81.2 : 74.1        93.0 : 86.2       100.9 : 110.1       117.0 : 115.0
+        50400 x 4096          88.9 : 77.7        86.3 : 78.7        90.4 : 81.4        93.7 : 94.5         98.8 : 98.3
 
     A call costs the host 6 to 12 us less, and a layer of a short prompt is issued in about the time that it runs in. So an eager
     call takes the kernel also where it is a little slower: four GPT-J layers of 4096, 100 tokens, 1030 us with the library from 65
     rows on for 12288 and 16384 outputs, 900 without it; of 2048, 980 and 735. Not past 2^27 weights and 64 rows, unless few
-    blocks leave the library's products without CUs; and for more blocks than CUs up to 24 rows (50400 x 4096 89.8 : 89.6,
-    24576 x 6144 72.5 : 69.0, 20480 x 5120 44 : 54; 64 rows 85.9 : 102.5). More than 128 rows: the library (the blocks would be
-    half as wide: 200 rows of 12288 x 4096 39.9 : 52.5).
-    In a capture there is no host time to save, and a product cut over K takes 1.6 to 2 us more, a fill of the graph's own
-    counters: 16 rows of 4096 x 16384 30.7 : 34.3, of 1024 x 1024 6.0 : 8.3, of 5120 x 5120 15.2 : 17.3, 32 and 64 rows of large
-    weights 34.6 : 34.1, 39.4 : 35.7 and 18.1 : 17.4, 21.7 : 19.8."""
+    blocks leave the library's products without CUs; and up to 24 rows where blocks of 64 weight rows are more than the CUs (24: 20480 x 5120
+    45.5 : 44.1, 24576 x 6144 71 : 55; 64: 47.8 : 51.0, 74 : 64). More than 128 rows: the library (200 rows of 12288 x 4096 39.9 : 52.5).
+    In a capture there is no host time to save: 16 rows of 1024 x 1024 6.0 : 8.3, of 5120 x 5120 15.2 : 17.3."""
     if n > 64 * _CUS:
-        return rows <= (16 if captured else 24)
+        return rows <= 24
     if captured:
         large = n * k >= 1 << 24
         return rows <= FEW_ROWS and (n <= 6144 and large if rows > 64 else _k_slices(n, k) == 1 or (rows > 24 and large))
@@ -308,8 +307,8 @@ def few_rows_gelu(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | No
 
 def few_rows_beside(first: tuple, second: tuple, approx2: str | None = None):
     """Two products (x, weight, bias) of the same few rows in one launch, a GELU on the second's fp32 sums -> (y, y2) or None.
-    On the GPU, us, apart and together, 61 rows: 12288 and 16384 x 4096 26.5 + 32.1, 52.0; 6144 and 8192 x 2048 11.4 + 12.4, 16.7 (two
-    blocks a CU 20.8); 128 rows 34.6 + 37.5, 65.1; and a launch and the GELU's less."""
+    On the GPU, us, apart and together, 61 rows: 12288 and 16384 x 4096 24.3 + 25.6, 41.7; 6144 and 8192 x 2048 11.4 + 12.4, 15.6;
+    128 rows 33.3 + 34.4, 49.1; and a launch and the GELU's less."""
     x = first[0]
     rows = x.numel() // x.shape[-1]
     y = _few_launch([first, second], 0, ACTS[approx2], True, rows) if approx2 in ACTS else None
@@ -318,8 +317,8 @@ def few_rows_beside(first: tuple, second: tuple, approx2: str | None = None):
 
 def few_rows_sum(first: tuple, second: tuple) -> torch.Tensor | None:
     """The sum of two products (x, weight, bias) of the same few rows in one launch, rounded once; or None. On the GPU, us, apart and
-    together, 61 rows: 4096 x 16384 and x 4096 33.9 + 13.1, 37.3 (two blocks a CU 46.9); 2048 x 8192 and x 2048 14.2 + 9.1, 16.2;
-    128 rows 42.6 + 17.8, 50.2."""
+    together, 61 rows: 4096 x 16384 and x 4096 29.9 + 13.2, 36.4; 2048 x 8192 and x 2048 14.0 + 9.1, 15.9;
+    128 rows 40.3 + 16.9, 49.2."""
     x = first[0]
     rows = x.numel() // x.shape[-1]
     if first[1].shape[0] != second[1].shape[0]:

@@ -4,7 +4,7 @@ import torch
 import torch.nn.functional as F
 
 from kubernetes_cloud_amd.ops import _lib
-from kubernetes_cloud_amd.ops.linear import _k_slices, _rows_mm, few_rows, linear_rows
+from kubernetes_cloud_amd.ops.linear import _k_slices, _rows_mm, few_rows, few_rows_beside, linear_rows
 from kubernetes_cloud_amd.utils import capture
 
 pytestmark = pytest.mark.gpu
@@ -104,3 +104,26 @@ def test_what_it_does_not_take():
     assert linear_rows(x, p, b).requires_grad
     with pytest.raises(RuntimeError):
         _lib.call("kca_rows_mm", 1, x.data_ptr(), w.data_ptr(), None, x.data_ptr(), None, None, 0, 0, 129, 96, 128, 1, _lib.stream())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [3, 32, 33, 64, 65, 128])
+@pytest.mark.parametrize("n,k", [(16384, 320), (16400, 64), (16400, 192), (24560, 448), (32768, 320), (32784, 128), (49152, 64), (49168, 576)])
+def test_blocks_of_64_and_128_weight_rows(dtype, rows, n, k):
+    """On both sides of the lines between the blocks, their last ones partly filled, in walks shorter and longer than the stages in LDS that
+    start at any of them."""
+    x, w, b, ref = _inputs(rows, n, k, dtype, True)
+    with torch.no_grad():
+        y = _rows_mm(x, w, b)
+        assert _close(y, ref) and torch.equal(y, _rows_mm(x, w, b))
+        assert _close(_rows_mm(x, w, None), F.linear(x.float(), w.float()))
+
+
+@pytest.mark.parametrize("rows", [5, 61, 100])
+@pytest.mark.parametrize("n,k,n2,k2", [(12304, 192, 4096, 640), (8192, 64, 8208, 320), (16384, 320, 16, 64)])
+def test_two_products_in_wide_blocks(rows, n, k, n2, k2):
+    x, w, b, ref = _inputs(rows, n, k, torch.bfloat16, True)
+    x2, w2, b2, ref2 = _inputs(rows, n2, k2, torch.bfloat16, True, 4)
+    with torch.no_grad():
+        y, y2 = few_rows_beside((x, w, b), (x2, w2, b2), None)
+    assert _close(y, ref) and _close(y2, ref2)
