@@ -39,7 +39,7 @@ from ..ops import _lib
 from ..ops import skinny_mm as smm
 from ..models.causal_lm import MLP, LayerNorm
 from ..ops.gemv import embed_ln_rows, ln_rows, ln_skinny_linear, skinny_linear
-from ..ops.linear import FEW_ROWS, TLinear, few_rows_beside, few_rows_gelu, few_rows_sum
+from ..ops.linear import (FEW_ROWS, TLinear, few_rows_beside, few_rows_gelu, few_rows_head, few_rows_scratch, few_rows_sum)
 from ..ops.norms import layer_norm_rows
 from ..utils import capture
 
@@ -766,17 +766,23 @@ class ModelRunner(StepRunner):
         self._batched_ok = (self._fused_ok and self.dtype in (torch.bfloat16, torch.float16)
                             and d_model % 64 == 0 and d_model <= 16384
                             and os.environ.get("KCA_DECODE_FUSED_BATCHED", "1") not in ("0", "false"))
+        # GPT-J layers at batch 2 to FEW_ROWS: two launches of the weight-streaming kernel, attention and a norm a layer
+        # (_layers_decode_rows). Four layers, us a step, this and before it (2 to 16 rows: the matrix-core layer; more: one launch a
+        # product, the feed-forward's on a side stream): 4096 wide, 400 tokens behind, 2 rows 492, 514; 5 535, 559; 8 543, 581; 16 589, 636;
+        # 24 of 100 558, 623; 32 of 700 795, 830; 64 of 300 948, 1077; 128 of 200 2066, 2220; 2048 wide, 100 behind, 2 rows 248, 262;
+        # 16 272, 303; 64 435, 520
+        self._rows_ok = self._batched_ok and self._embed_head and self._layer_kind == "gptj" and not tp and model.emb_ln is None
+        self.rows_steps = 0
         # largest batch bucket the matrix-core layer takes, per layer kind, from same-box A/Bs against the
         # per-projection path (hipBLASLt + the fused LN / GELU / all-reduce launches,
-        # profiles/decode_suite_r6_batched_vs_unfused.jsonl): GPT-J 3.49 vs 3.88 ms at B=16 but 4.63 vs
-        # 4.27 at 32 (the per-projection step overlaps the MLP GEMMs with the attention on a side stream);
-        # BLOOM TP=8 rank 11.46 vs 12.58 at 16, 14.25 vs 13.50 at 32 (hipBLASLt streams the 14336-wide
-        # shapes faster from M = 32); NeoX wins at every batch (12.84 vs 15.86 at 32, 25.9 vs 28.3 at 64)
+        # profiles/decode_suite_r6_batched_vs_unfused.jsonl): BLOOM TP=8 rank 11.46 vs 12.58 at 16, 14.25 vs 13.50 at 32
+        # (hipBLASLt streams the 14336-wide shapes faster from M = 32); NeoX wins at every batch (12.84 vs 15.86 at 32, 25.9
+        # vs 28.3 at 64)
         # fp16 takes the same caps since the per-projection path's LayerNorm / GELU run their fp16
-        # instantiations (ln_rows, kca_gelu_fwd_f16) instead of eager kernels: B=32 GPT-J 4.40 vs 4.65 ms,
-        # BLOOM rank 13.38 vs 14.84 per-projection vs matrix-core layer (profiles/decode_fp16_cap_ab_r6.jsonl)
+        # instantiations (ln_rows, kca_gelu_fwd_f16) instead of eager kernels: BLOOM rank 13.38 vs 14.84 per-projection
+        # vs matrix-core layer at 32 (profiles/decode_fp16_cap_ab_r6.jsonl)
         self._batched_max_b = int(os.environ.get("KCA_DECODE_BATCHED_MAX_B", "0")) or \
-            {"gptj": 16, "seq": 16}.get(self._layer_kind, 64)
+            {"gptj": 1 if self._rows_ok else 16, "seq": 16}.get(self._layer_kind, 64)
 
     # ------------------------------------------------------------- prefill
     @torch.no_grad()
@@ -1195,6 +1201,38 @@ class ModelRunner(StepRunner):
             logits = gather_last_dim(logits, grp)
         return logits
 
+    def _layers_decode_rows(self, tokens, pos, slots, kv_lens, max_kv, ws, obuf):
+        """Decode step of GPT-J layers at batch 2 to FEW_ROWS (see _rows_ok): QKV and fc_in (GELU on its sums) in one launch of the
+        weight-streaming kernel, attention, then fc_out and out in one, and the norm that adds their sum. One queue: the
+        feed-forward on a side stream beside the attention costs a fork and a join a layer (32 rows, 700 behind 824 us, this 793).
+        None: sizes or a mode that the kernel does not serve; nothing has run then but the step's head."""
+        m, cfg = self.model, self.cfg
+        B = tokens.shape[0]
+        sc = self._fz.get(("rows", B))
+        if sc is None:
+            sc = self._fz["rows", B] = few_rows_scratch(B, self.device)
+        chain, prev = self._chain_src if self._chain_src is not None else (None, None)
+        ln = m.h[0].ln_1
+        xn, h = embed_ln_rows(m.wte.weight, tokens, ln.weight, ln.bias, ln.eps, chain=chain, prev=prev)
+        cos, sin, tbl, by_row = self._desc_args(self.cos, self.sin, self.cache.table_on(self.device))
+        for li, blk in enumerate(m.h):
+            at, mlp = blk.attn, blk.mlp
+            pair = few_rows_beside((xn, at.qkv.weight, at.qkv.bias), (xn, mlp.fc_in.weight, mlp.fc_in.bias), mlp.approx, sc)
+            if pair is None:
+                if li == 0:
+                    return None
+                raise RuntimeError("decode layer of few rows: shape support changed between layers")
+            o = dops.decode_prep_attention(pair[0], self.H, self.Hkv, self.D, self.rot, cfg.rotary_interleaved, cos, sin, pos, slots,
+                                           self.cache.k[li], self.cache.v[li], kv_lens, max_kv, at.scale, at.alibi, out=obuf, ws=ws,
+                                           block_table=tbl, window=at.window, by_row=by_row)
+            y = few_rows_sum((pair[1], mlp.fc_out.weight, mlp.fc_out.bias), (o, at.out.weight, at.out.bias), sc)
+            if y is None:
+                y = skinny_linear(o, at.out.weight, at.out.bias).add_(skinny_linear(pair[1], mlp.fc_out.weight, mlp.fc_out.bias))
+            ln = m.h[li + 1].ln_1 if li + 1 < len(m.h) else m.ln_f
+            xn, h = ln_rows(h, ln.weight, ln.bias, ln.eps, (y,))
+        w, b, _ = self._head_weight()
+        return few_rows_head(xn, w, b)
+
     def _layers_decode(self, tokens, pos, slots, kv_lens, max_kv, ws, obuf):
         m, cfg = self.model, self.cfg
         if self._fused_ok and tokens.shape[0] == 1 and obuf is not None:
@@ -1205,6 +1243,11 @@ class ModelRunner(StepRunner):
         if (self._batched_ok and 2 <= tokens.shape[0] <= min(smm.MAX_M, self._batched_max_b) and obuf is not None
                 and (self._chain_src is None or self._embed_head)):
             return self._layers_decode_batched(tokens, pos, slots, kv_lens, max_kv, ws, obuf)
+        if self._rows_ok and 1 < tokens.shape[0] <= FEW_ROWS and obuf is not None:
+            y = self._layers_decode_rows(tokens, pos, slots, kv_lens, max_kv, ws, obuf)
+            if y is not None:
+                self.rows_steps += 1
+                return y
         if self._chain_src is not None and obuf is not None:  # chained rows not resolved by a fused head
             chain, prev = self._chain_src
             tokens = torch.where(chain[:tokens.shape[0]] >= 0, prev[chain[:tokens.shape[0]].clamp(min=0).long()],

@@ -270,11 +270,18 @@ def _few_part(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, 
             and (bias is None or (bias.shape == (n,) and bias.dtype == x.dtype and bias.is_contiguous())))
 
 
-def _few_launch(parts, act: int, act2: int, beside: bool, rows: int):
+def few_rows_scratch(rows: int, device: torch.device) -> tuple[torch.Tensor, torch.Tensor]:
+    """What the products of up to ``rows`` rows need for their slices of K (some 256 blocks' partial sums and arrival counters, left
+    zeroed), for launches that follow one another on one stream."""
+    return (torch.empty(_CUS * 64 * (32 if rows <= 32 else 64 if rows <= 64 else 128), device=device, dtype=torch.float32),
+            torch.zeros(_CUS, device=device, dtype=torch.int32))
+
+
+def _few_launch(parts, act: int, act2: int, beside: bool, rows: int, scratch=None):
     """One launch of ``kca_rows_mm_two`` over one or two (x, weight, bias); None: sizes, types or a mode of torch (gradients,
-    transforms, captures, ...) that it does not serve."""
+    transforms, captures without ``few_rows_scratch``, ...) that it does not serve."""
     x = parts[0][0]
-    if (not 0 < rows <= FEW_ROWS or not x.is_cuda or torch.cuda.is_current_stream_capturing()
+    if (not 0 < rows <= FEW_ROWS or not x.is_cuda or (scratch is None and torch.cuda.is_current_stream_capturing())
             or not all(p[0].dtype == x.dtype and _few_part(*p, rows) for p in parts)
             or not _lib.inference(*(t for p in parts for t in p)) or not _lib.has("kca_rows_mm_two")):
         return None
@@ -282,7 +289,9 @@ def _few_launch(parts, act: int, act2: int, beside: bool, rows: int):
     blocks = sum(-(-y.shape[1] // 64) for y in outs)
     k = min(p[1].shape[1] for p in parts) if beside else sum(p[1].shape[1] for p in parts)
     ks, ws, cnt = max(1, min(_CUS // blocks, k // 512)), None, None  # (about one block a CU, as _k_slices)
-    if ks > 1:
+    if ks > 1 and scratch is not None:
+        ws, cnt = scratch
+    elif ks > 1:
         ws = torch.empty(blocks * ks * 64 * (32 if rows <= 32 else 64 if rows <= 64 else 128), device=x.device, dtype=torch.float32)
         cnt = _lib.counters(x.device, blocks)
     a = []
@@ -305,17 +314,17 @@ def few_rows_gelu(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | No
     return None if y is None else y[0].view(*x.shape[:-1], -1)
 
 
-def few_rows_beside(first: tuple, second: tuple, approx2: str | None = None):
+def few_rows_beside(first: tuple, second: tuple, approx2: str | None = None, scratch=None):
     """Two products (x, weight, bias) of the same few rows in one launch, a GELU on the second's fp32 sums -> (y, y2) or None.
     On the GPU, us, apart and together, 61 rows: 12288 and 16384 x 4096 24.3 + 25.6, 41.7; 6144 and 8192 x 2048 11.4 + 12.4, 15.6;
     128 rows 33.3 + 34.4, 49.1; and a launch and the GELU's less."""
     x = first[0]
     rows = x.numel() // x.shape[-1]
-    y = _few_launch([first, second], 0, ACTS[approx2], True, rows) if approx2 in ACTS else None
+    y = _few_launch([first, second], 0, ACTS[approx2], True, rows, scratch) if approx2 in ACTS else None
     return None if y is None else tuple(t.view(*x.shape[:-1], -1) for t in y)
 
 
-def few_rows_sum(first: tuple, second: tuple) -> torch.Tensor | None:
+def few_rows_sum(first: tuple, second: tuple, scratch=None) -> torch.Tensor | None:
     """The sum of two products (x, weight, bias) of the same few rows in one launch, rounded once; or None. On the GPU, us, apart and
     together, 61 rows: 4096 x 16384 and x 4096 29.9 + 13.2, 36.4; 2048 x 8192 and x 2048 14.0 + 9.1, 15.9;
     128 rows 40.3 + 16.9, 49.2."""
@@ -323,7 +332,7 @@ def few_rows_sum(first: tuple, second: tuple) -> torch.Tensor | None:
     rows = x.numel() // x.shape[-1]
     if first[1].shape[0] != second[1].shape[0]:
         return None
-    y = _few_launch([first, second], 0, 0, False, rows)
+    y = _few_launch([first, second], 0, 0, False, rows, scratch)
     return None if y is None else y[0].view(*x.shape[:-1], -1)
 
 
@@ -509,3 +518,16 @@ def linear_residual(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | 
               r2.data_ptr(), r2.stride(0), out.data_ptr(), N, M, N, K, 1.0, _lib.ptr(ws),
               _WS_BYTES if ws is not None else 0, _lib.stream())
     return out.view(res.shape)
+
+
+def few_rows_head(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
+    """Logits [rows, n] of a decode step's rows: past ``few_rows``' 24 rows of more blocks of 64 weight rows than CUs too, where blocks of 128
+    are on most CUs (table of ``few_rows``; 48 rows of 50400 x 2048 50.6 : 42.9, of 20480 x 5120, 160 blocks, 47.1 : 48.9)."""
+    (rows, k), n = x.shape, weight.shape[0]
+    if (n > 64 * _CUS and rows <= (64 if n >= 96 * _CUS else 32) and k >= 1024 and x.dtype in (torch.bfloat16, torch.float16)
+            and x.dtype == weight.dtype and x.is_contiguous() and (bias is None or (bias.shape == (n,) and bias.dtype == x.dtype))
+            and _lib.inference(x, weight, bias)):
+        y = _rows_mm(x, weight, bias)
+        if y is not None:
+            return y
+    return linear_rows(x, weight, bias)

@@ -1046,3 +1046,47 @@ def test_engine_emulated_rank_runs_real_tp_tails(dtype):
     assert eng.runner.step_launches  # launches per step recorded for the bench
     for p, o in zip([prompts[0]] + prompts, outs):
         _check_against_forward(m, p, o)
+
+
+@pytest.mark.parametrize("dtype,B,width", [(torch.bfloat16, 2, 1024), (torch.float16, 17, 512), (torch.bfloat16, 33, 1024), (torch.bfloat16, 70, 512)])
+def test_engine_gptj_rows_layer(dtype, B, width):
+    """GPT-J decode steps of 2 and more rows on the weight-streaming products (runner._layers_decode_rows), with step graphs: in each
+    class of rows that the kernel rounds up to, every row's greedy tokens match a full forward of its own continuation."""
+    from kubernetes_cloud_amd.engine.llm_engine import LLMEngine, SamplingParams
+    from kubernetes_cloud_amd.models.causal_lm import build_model
+    from kubernetes_cloud_amd.models.config import PRESETS_HF, LMConfig
+    cfg = dict(PRESETS_HF["gpt-j-6b"])
+    cfg.update(n_embd=width, n_layer=2, n_head=width // 256, rotary_dim=64, n_positions=512)
+    m = build_model(LMConfig.from_hf(cfg), device=dev, dtype=dtype, seed=0)
+    g = torch.Generator().manual_seed(B)
+    prompts = [[int(x) for x in torch.randint(0, 1000, (int(n),), generator=g)] for n in torch.randint(8, 90, (B,), generator=g)]
+    eng = LLMEngine(m, max_slots=B, max_len=256, use_graphs=True)
+    outs = [r.output for r in eng.generate(prompts, SamplingParams(max_new_tokens=8, do_sample=False))]
+    assert eng.runner.rows_steps > 0 and eng.runner.batched_steps == 0 and not eng.runner._packs
+    for p, o in zip(prompts, outs):
+        _check_against_forward(m, p, o)
+
+
+@pytest.mark.parametrize("rows", [2, 32, 33, 64, 65])
+@pytest.mark.parametrize("n,k", [(16400, 1024), (24576, 1024), (24560, 1088), (4096, 512)])
+def test_decode_logits_of_few_rows(rows, n, k):
+    """Around the lines of the head's rule, eager and replayed."""
+    from kubernetes_cloud_amd.ops.linear import few_rows_head
+    from kubernetes_cloud_amd.utils import capture
+    g = torch.Generator(device=dev).manual_seed(rows)
+    x = torch.empty(rows, k, device=dev, dtype=torch.bfloat16).normal_(generator=g)
+    w = torch.empty(n, k, device=dev, dtype=torch.bfloat16).normal_(std=k ** -0.5, generator=g)
+    b = torch.empty(n, device=dev, dtype=torch.bfloat16).normal_(generator=g)
+    ref = torch.nn.functional.linear(x.float(), w.float(), b.float())
+    with torch.no_grad():
+        y = few_rows_head(x, w, b)
+        graph = torch.cuda.CUDAGraph()
+        with capture.graph(graph, stream=torch.cuda.Stream()):
+            z = few_rows_head(x, w, b)
+    # one rounding to the type; the 32-bit sums of terms of size k^-1/2 are good to well below 1e-4
+    for _ in range(2):
+        z.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for t in (y, z):
+            assert ((t.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4).all()
