@@ -350,19 +350,27 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
   };
   load_qkv_rows();
   // per-step RoPE row (by_row bit 0): the angles do not wait for the length
-  const bool pre_rope = (p.by_row & 1) && p.fused && p.rot > 0;
+  const bool rope = p.fused && p.rot > 0;
+  const bool angles = rope && (PF || (p.by_row & 1));  // in rc and rs
   float rc[8], rs[8];
-  if (pre_rope && dact) rope_tab8(p.cos_t, p.sin_t, b, dslot * 8, p.rot, p.interleaved, rc, rs);
+  if ((p.by_row & 1) && rope && dact) rope_tab8(p.cos_t, p.sin_t, b, dslot * 8, p.rot, p.interleaved, rc, rs);
   // paged: this split's page ids staged in LDS (chunk <= 1024 tokens, pages >= 16 tokens), so a
   // token's address costs an LDS read instead of a dependent global load in front of every K/V
   // load; the whole chunk's range is staged (clipped to the table row), independent of the length
-  __shared__ int pg[1024 / 16 + 2];
+  __shared__ long long pg[1024 / 16 + 2];  // (offsets of the pages)
   const int pg0 = c0 >> p.ps_shift;
+  int npg = 0, page = 0;
   if constexpr (PAGED) {
-    const int npg = min(((c0 + p.chunk - 1) >> p.ps_shift) - pg0 + 1, p.tbl_stride - pg0);
+    npg = min(((c0 + p.chunk - 1) >> p.ps_shift) - pg0 + 1, p.tbl_stride - pg0);
     KCA_DASSERT(npg <= 1024 / 16 + 2);
     const int trow = (p.by_row & 2) ? b : seq;  // per-step page rows: no wait for the slot
-    for (int i = tid; i < npg; i += 256) pg[i] = p.tbl[(long long)trow * p.tbl_stride + pg0 + i];
+    if (tid < npg) page = p.tbl[(long long)trow * p.tbl_stride + pg0 + tid];
+  }
+  // the angles at the new token's position are requested beside the page ids (not beside a batch-1 step's GEMV, whose step brings
+  // its angles: the choice alone costs its attention 1 us of 25)
+  if (PF && !(p.by_row & 1) && rope && dact) rope_tab8(p.cos_t, p.sin_t, max(L - 1, 0), dslot * 8, p.rot, p.interleaved, rc, rs);
+  if constexpr (PAGED) {
+    if (tid < npg) pg[tid] = (long long)page * p.cs_slot;
   }
   const int c1 = min(c0 + p.chunk, L);
   // sliding window: positions below L - window are never read (splits left of it are empty)
@@ -387,12 +395,12 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
     if (dact) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) q[g][j] = e2f<DT>(qraw[g].v[j]);
-      if (pre_rope) {
+      if (angles) {
         float raw[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) raw[j] = q[g][j];
         rope8_reg<DT>(p.q + b * p.q_bs + (long long)(hk * G + g) * D, dslot * 8, q[g], raw, rc, rs, p.rot, p.interleaved);
-      } else if (p.fused && p.rot > 0) {
+      } else if (rope) {
         rope8<DT>(p.q + b * p.q_bs + (long long)(hk * G + g) * D, dslot * 8, q[g], pnew, p.rot, p.interleaved, p.cos_t,
               p.sin_t);
       }
@@ -418,7 +426,7 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
   // offset of token t inside this sequence's storage
   auto toff = [&](int t) -> long long {
     if constexpr (PAGED)
-      return (long long)pg[(t >> p.ps_shift) - pg0] * p.cs_slot + (long long)(t & ((1 << p.ps_shift) - 1)) * p.cs_pos;
+      return pg[(t >> p.ps_shift) - pg0] + (long long)((unsigned)(t & ((1 << p.ps_shift) - 1)) * (unsigned long long)p.cs_pos);
     return (long long)t * p.cs_pos;
   };
 
@@ -437,12 +445,12 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
       kx[j] = e2f<DT>(knraw.v[j]);
       vx[j] = e2f<DT>(vnraw.v[j]);
     }
-    if (pre_rope) {  // tid < ND <= LPT: this lane's dslot is tid, its angles are rc / rs
+    if (angles) {  // tid < ND <= LPT: this lane's dslot is tid, its angles are rc / rs
       float raw[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) raw[j] = kx[j];
       rope8_reg<DT>(krow, tid * 8, kx, raw, rc, rs, p.rot, p.interleaved);
-    } else if (p.rot > 0) {
+    } else if (rope) {
       rope8<DT>(krow, tid * 8, kx, pnew, p.rot, p.interleaved, p.cos_t, p.sin_t);
     }
     const long long o = toff(pnew) + hk * p.cs_head + tid * 8;  // toff: offset inside the sequence
@@ -490,27 +498,22 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
   auto load_kv = [&](int tb, U16x8 (&kk)[U], U16x8 (&vv)[U]) {
     long long o[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) o[u] = toff(min(tb + u * TPB, ce - 1)) + dfix;
+    for (int u = 0; u < U; ++u) o[u] = toff(min(tb + u * TPB, max(ce - 1, ca))) + dfix;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       kk[u] = *reinterpret_cast<const U16x8*>(kb + o[u]);
       vv[u] = *reinterpret_cast<const U16x8*>(vb + o[u]);
     }
-  };
-  // PF (long splits, the standalone launch): the next iteration's K / V rows are requested before this
-  // iteration's scores, so a split of many iterations streams instead of paying one round trip each
-  U16x8 kr[U], vr[U];
-  if (PF && ca + wid * TPW + tsub < ce) load_kv(ca + wid * TPW + tsub, kr, vr);
-  for (int t0 = ca + wid * TPW + tsub; t0 < ce; t0 += TPB * U) {
-    U16x8 kn[U], vn[U];
-    if constexpr (PF) {
-      if (t0 + TPB * U < ce) load_kv(t0 + TPB * U, kn, vn);
-    } else {
-      load_kv(t0, kr, vr);
+    if constexpr (PF) {  // hipcc moves loads that only the next round of a loop uses into that round, or behind the other set's sums
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
     }
-    // the U scores of this iteration are independent (their lane-group sums overlap), then ONE
-    // online-softmax update folds them in: the dependent chain per iteration is one reduction and
-    // one rescale, not U of each. Token t0 (u = 0) is always valid, so the running max is finite.
+  };
+  // the U scores of an iteration are independent (their lane-group sums overlap), then ONE
+  // online-softmax update folds them in: the dependent chain per iteration is one reduction and
+  // one rescale, not U of each. Token t0 (u = 0) of the first one is always valid, so the running max is finite;
+  // a later iteration without a valid token changes nothing.
+  auto fold = [&](int t0, const U16x8 (&kr)[U], const U16x8 (&vr)[U]) {
     float sv[G][U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -547,12 +550,27 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
       }
       m[g] = mn;
     }
-    if constexpr (PF) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        kr[u] = kn[u];
-        vr[u] = vn[u];
-      }
+  };
+  const int ts = ca + wid * TPW + tsub;
+  if constexpr (PF) {
+    // Long splits, the standalone launch: bound by the cache's stream and, where it is short, by round trips. Two iterations' rows are
+    // on their way, in registers of their own: moved from one set to the other, the move waits for rows that have only just been
+    // requested, and the next request for them. 16 heads of 256, cold, us, with the move and so: 32 sequences of 700 to 917 95, 86 (4.9 TB/s);
+    // 24 of 100 to 261 27.3, 23.5; 16 of 400 to 505 35.1, 29.9; 13 of 60 to 144 16.8, 12.6; 64 of 300 to 741 124, 111.
+    U16x8 kx0[U], vx0[U], kx1[U], vx1[U];
+    load_kv(ts, kx0, vx0);
+    load_kv(ts + TPB * U, kx1, vx1);
+    for (int t0 = ts; t0 < ce; t0 += 2 * TPB * U) {
+      fold(t0, kx0, vx0);
+      load_kv(t0 + 2 * TPB * U, kx0, vx0);
+      fold(t0 + TPB * U, kx1, vx1);
+      load_kv(t0 + 3 * TPB * U, kx1, vx1);
+    }
+  } else {
+    for (int t0 = ts; t0 < ce; t0 += TPB * U) {
+      U16x8 kr[U], vr[U];
+      load_kv(t0, kr, vr);
+      fold(t0, kr, vr);
     }
   }
   DSTAMP(4);

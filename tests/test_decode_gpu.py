@@ -467,6 +467,35 @@ def test_decode_prep_attention_fused_equals_two_kernels(D, rot, inter, G, PS, CH
     assert torch.equal(q2, qkv)  # the fused kernel leaves the QKV buffer untouched
 
 
+@pytest.mark.parametrize("D,Hkv,G,PS", [(256, 3, 1, 64), (256, 2, 1, 0), (96, 3, 1, 16), (64, 2, 2, 32)])
+@pytest.mark.parametrize("window", [0, 5, 37, 96])
+def test_decode_one_pass_walk_edges(D, Hkv, G, PS, window):
+    """The one-pass kernel's walk, two rounds of requests on their way: lengths and windows about one, two and three rounds of a
+    workgroup (32 tokens at 256, 64 at 96, 128 at 64 dims), a split whose only token is the new one, starts off a round's tokens."""
+    lens = [1, 2, 9, 31, 32, 33, 34, 63, 64, 65, 66, 96, 97, 98, 128, 129, 130, 193, 257, 258, 300, 385]
+    torch.manual_seed(D + window)
+    B, L, H = len(lens), 448, Hkv * G
+    kc = torch.randn(B, Hkv, L, D, device=dev).to(torch.bfloat16)
+    vc = torch.randn_like(kc)
+    q = torch.randn(B, H * D, device=dev).to(torch.bfloat16)
+    want = torch.empty(B, H, D, dtype=torch.float64)
+    for i, n in enumerate(lens):
+        lo = max(0, n - window) if window else 0
+        k, v = (x[i, :, lo:n].double().cpu().repeat_interleave(G, 0) for x in (kc, vc))
+        p = torch.softmax((k @ q[i].double().cpu().view(H, D, 1))[..., 0] * D ** -0.5, -1)
+        want[i] = (p[:, None] @ v)[:, 0]
+    tbl = None
+    if PS:
+        kc, tbl = _paginate(kc, PS, 3)
+        vc, _ = _paginate(vc, PS, 3)
+    slots = torch.arange(B, device=dev, dtype=torch.int32)
+    kl = torch.tensor(lens, device=dev, dtype=torch.int32)
+    for chunk in (448, 256):
+        got = dops.decode_attention(q, kc, vc, slots, kl, H, L, chunk=chunk, block_table=tbl, window=window)
+        # half a unit of the result's last place, and scores whose fp32 sums are off by some 1e-5 of values of up to 4
+        assert ((got.double().cpu().view(B, H, D) - want).abs() <= want.abs() * 2 ** -8 + 1e-4).all()
+
+
 _FANIN_CASE = """
 import sys, torch
 from kubernetes_cloud_amd.ops import decode as dops
