@@ -312,6 +312,14 @@ __device__ void fanin_combine(const DecodeParams& p, int b, int hk, int nsplit) 
   }
 }
 
+// Cached rows are read once a step, and a layer's are back only after all others and the weights. Non-temporal, as the weights' (standalone
+// launch, 16 heads of 256, us: 32 sequences of 700 to 917 86.5, 78.4 (5.4 TB/s); 24 of 100 to 261 23.4, 21.1; 3 of 900 22.2, 20.6; 64 of 300 to 741
+// 110, 100; 16 of 1900 114, 104)
+typedef unsigned u32x4_once __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ U16x8 load_once(const bf16_t* p) {
+  return __builtin_bit_cast(U16x8, __builtin_nontemporal_load(reinterpret_cast<const u32x4_once*>(p)));
+}
+
 // LPT lanes cooperate on one token row (8 dims per lane); TPW = 64/LPT tokens per
 // wave step; G query heads share each K/V row (GQA group).
 // (the workgroup's (split, kv-head, sequence) coordinates are arguments: decode_attn_kernel passes
@@ -501,8 +509,8 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
     for (int u = 0; u < U; ++u) o[u] = toff(min(tb + u * TPB, max(ce - 1, ca))) + dfix;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      kk[u] = *reinterpret_cast<const U16x8*>(kb + o[u]);
-      vv[u] = *reinterpret_cast<const U16x8*>(vb + o[u]);
+      kk[u] = load_once(kb + o[u]);
+      vv[u] = load_once(vb + o[u]);
     }
     if constexpr (PF) {  // hipcc moves loads that only the next round of a loop uses into that round, or behind the other set's sums
       asm volatile("" ::: "memory");
