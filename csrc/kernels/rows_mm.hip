@@ -145,10 +145,13 @@ __global__ void __launch_bounds__(64 * W, 2) rows_mm_kernel(RowsArgs p) {
     const bool one = !TWO || tt < nka;
     const int k = (one ? tt : tt - nka) * SK * 2;
     const __amdgpu_buffer_rsrc_t fw = one ? rw : rw2, fx = one ? rx : rx2;
+    // (the weights non-temporal: no other block reads them. 32 rows, cold, us: 12288 and 16384 x 4096 42.6, 37.8 (6.2 TB/s); 4096 x 16384 and x 4096
+    // 34.7, 30.2; 50400 x 4096 82.8, 75.6; 61 rows 43.8, 40.1; 38.6, 37.2; 86.5, 81.7. Called again with nothing between, weights that the last
+    // cache would hold come slower: 50400 x 1024 19.5, 21.9)
 #pragma unroll
     for (int i = 0; i < WI; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(fw, (void __attribute__((address_space(3)))*)(st + (wv * WI + i) * 1024), 16,
-                                               one ? wo[i] : wo2[i], k, 0, 0);
+                                               one ? wo[i] : wo2[i], k, 0, 2);
 #pragma unroll
     for (int i = 0; i < XI; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(fx, (void __attribute__((address_space(3)))*)(st + (NB / 8 + wv * XI + i) * 1024), 16,
