@@ -41,15 +41,24 @@ __device__ __forceinline__ unsigned lds_address(const char* p) {
 #endif
 }
 
-// 16 bytes a lane, 1 KB in a row at `at`, from `from` + k bytes on. (In asm: hipcc would let every read of LDS wait for all requests. Nothing is
+// 16 bytes a lane, 1 KB in a row at `at`, from `from` + k bytes on. ONCE: non-temporal, for the weights of an expert that has one tile, which no other
+// block reads. One layer, cold, us, without and with: 16 experts of 3 x 4096 x 4096, top 2, 32 tokens 300, 287 (stream, 5.6 TB/s), 100 308, 293; 777 372,
+// 350 (wide blocks of up to 192 rows; those of 256, bound by the products, gain nothing: not there), 1200 406, 392; 3 x 4096 x 2048, top 3, 32 175, 166; 130 189, 177
+// (blocks of 128 weight rows). (In asm: hipcc would let every read of LDS wait for all requests. Nothing is
 // returned to a register. Five wait states after what may be a vector write of a scalar)
+template <bool ONCE = false>
 __device__ __forceinline__ void request_into_lds(const u32x4& rsrc, unsigned at, unsigned from, int k) {
 #if defined(LDS_TRACE)
   lds_request_at(at + threadIdx.x % 64 * 16);
 #else
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(at)),
-               "v"(from), "s"(rsrc), "s"(k)
-               : "m0");
+  if constexpr (ONCE)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(__builtin_amdgcn_readfirstlane(at)),
+                 "v"(from), "s"(rsrc), "s"(k)
+                 : "m0");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(at)),
+                 "v"(from), "s"(rsrc), "s"(k)
+                 : "m0");
 #endif
 }
 
@@ -94,7 +103,7 @@ __device__ __forceinline__ void wait_reads() {
 constexpr int SROWS = 32, SK = 64, SWN = 32;
 
 // rows: 8, 16 or 32 of activations (XI requests a stage)
-template <bool UP, int XI>
+template <bool UP, int XI, bool ONCE = false>
 __device__ __forceinline__ void expert_stream_tile(const ExpertArgs& p, char* sl, int ex, int lo, int nr, int n0) {
   constexpr int XB = XI > 2 ? 2 : 1, NW = 3, NX = 2, OWN = NW * 4096 + NX * XI * 1024;  // runs of 16 rows; places; a wave's bytes
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -118,7 +127,7 @@ __device__ __forceinline__ void expert_stream_tile(const ExpertArgs& p, char* sl
   auto stage_k = [&](int t) { return __builtin_amdgcn_readfirstlane(min(4 * t + wv, last) * SK * 2); };  // past the end: one that nobody reads
   auto weights = [&](int t, int place) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) request_into_lds(rw, base + place * 4096 + i * 1024, wo[i], stage_k(t));
+    for (int i = 0; i < 4; ++i) request_into_lds<ONCE>(rw, base + place * 4096 + i * 1024, wo[i], stage_k(t));
   };
   auto rows = [&](int t, int place) {
 #pragma unroll
@@ -201,7 +210,7 @@ constexpr int STREAM_LDS = 4 * (3 * 4096 + 2 * 4 * 1024);
 // better one where the walk is short for its rows (stream_block).
 constexpr int BWN = 128, BSTAGE = (BWN + SROWS) * SK * 2;
 static_assert(4 * BSTAGE == STREAM_LDS, "four stages");
-template <bool UP>
+template <bool UP, bool ONCE = false>
 __device__ __forceinline__ void expert_block_tile(const ExpertArgs& p, char* sl, int ex, int lo, int nr, int n0) {
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g = lane >> 4, K = p.K, N = p.N, nk = K / SK;
@@ -221,7 +230,7 @@ __device__ __forceinline__ void expert_block_tile(const ExpertArgs& p, char* sl,
     const int k = __builtin_amdgcn_readfirstlane(min(t, nk - 1) * SK * 2);  // past the end: the last one, which nobody reads
     const unsigned at = base + t % 4 * BSTAGE;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) request_into_lds(rw, at + (wv * 4 + i) * 1024, wo[i], k);
+    for (int i = 0; i < 4; ++i) request_into_lds<ONCE>(rw, at + (wv * 4 + i) * 1024, wo[i], k);
     request_into_lds(rx, at + (16 + wv) * 1024, xo, k);
   };
   f32x4 acc[2][2];  // [gate, up | two runs of 16 outputs][16 rows]
@@ -297,7 +306,7 @@ constexpr int GBK = 64, GN = 256, GM = 256, GEMM_LDS = 2 * (GN + GM) * GBK * 2, 
 // 810; 2000 tokens 589 -> 482, 1200 412 -> 386; 4000 tokens, 16 of 3 x 4096 x 2048, top 3 574 -> 481.
 // What bounds it: rounds of blocks that end half empty (15 % at 4096 tokens), a block's start and results (22 thousand cycles). Blocks
 // that stay and request the next tile before their results gained nothing over the scheduler's choice of the next block.
-template <bool UP, int B>
+template <bool UP, int B, bool ONCE = false>
 __device__ __forceinline__ void expert_turns_tile(const ExpertArgs& p, char* sl, int ex, int lo, int nr, int n0) {
   constexpr int HALF = 128 * GBK * 2, BST = 64 * B * GBK * 2, BAT = 6 * HALF;  // bytes: 128 weight rows, the activations of a stage, their place
   static_assert(BAT + 2 * BST <= WIDE_LDS, "three stages of weights and two of activations");
@@ -319,11 +328,11 @@ __device__ __forceinline__ void expert_turns_tile(const ExpertArgs& p, char* sl,
     from_x[i] = ((unsigned)(UP ? p.perm[lo + xr] / p.top : xr) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
   }
   const unsigned base = __builtin_amdgcn_readfirstlane(lds_address(sl));
-  auto request = [&](const u32x4& rsrc, unsigned at, unsigned from, int t) {
-    request_into_lds(rsrc, at, from, __builtin_amdgcn_readfirstlane(min(t, nk - 1) * GBK * 2));  // past the end: the last one, which nobody reads
+  auto request = [&](auto once, const u32x4& rsrc, unsigned at, unsigned from, int t) {
+    request_into_lds<decltype(once)::value>(rsrc, at, from, __builtin_amdgcn_readfirstlane(min(t, nk - 1) * GBK * 2));  // past the end: the last one, which nobody reads
   };
-  auto weight = [&](int t, int place, int i) { request(rw, base + (2 * place + wa) * HALF + (wb * 4 + i) * 1024, from_w[i], t); };
-  auto row = [&](int t, int place, int i) { request(rx, base + BAT + place * BST + (wv * B + i) * 1024, from_x[i], t); };
+  auto weight = [&](int t, int place, int i) { request(std::integral_constant<bool, ONCE>{}, rw, base + (2 * place + wa) * HALF + (wb * 4 + i) * 1024, from_w[i], t); };
+  auto row = [&](int t, int place, int i) { request(std::false_type{}, rx, base + BAT + place * BST + (wv * B + i) * 1024, from_x[i], t); };
   f32x4 acc[2][4][B];
 #pragma unroll
   for (int h = 0; h < 2; ++h)

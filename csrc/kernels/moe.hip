@@ -662,6 +662,15 @@ dim3 block_rows(long long blocks) {
 }
 __device__ __forceinline__ int block_number() { return blockIdx.y * (int)ROW_BLOCKS + blockIdx.x; }
 
+// Whether an expert's weights are read by one tile, and come non-temporal then (request_into_lds). In the gemm, of two tiles that share a
+// cache, the second finds what the first has read: 24 experts of 3 x 2048 x 768, top 5, 500 tokens, us, ordinary 101.3, non-temporal all 102.2, so 97.3;
+// 777 112.3, 114.4, 110.4; 16 of 3 x 4096 x 2048, top 3, 300 210.5, 192, 192.5; 777 267, 253, 250.6.
+template <typename F>
+__device__ __forceinline__ void once_or_again(int tiles, F&& f) {
+  if (tiles == 1) f(std::true_type{});
+  else f(std::false_type{});
+}
+
 // ---------------------------------------------------------------------------------------------- stream
 // (the tile: expert_tiles.h)
 template <bool UP>
@@ -677,9 +686,12 @@ __global__ void __launch_bounds__(256, 2) expert_stream_kernel(ExpertArgs p) {
   const int in = id - t0[3] * nb, tile = t0[3] + in % t0[4], bn = in / t0[4];
   const int* tl = p.tiles + tile * 5;
   const int nr = tl[2];
-  if (nr <= 8) expert_stream_tile<UP, 1>(p, sl, tl[0], tl[1], nr, bn * NB);
-  else if (nr <= 16) expert_stream_tile<UP, 2>(p, sl, tl[0], tl[1], nr, bn * NB);
-  else expert_stream_tile<UP, 4>(p, sl, tl[0], tl[1], nr, bn * NB);
+  once_or_again(tl[4], [&](auto once) {
+    constexpr bool ONCE = decltype(once)::value;
+    if (nr <= 8) expert_stream_tile<UP, 1, ONCE>(p, sl, tl[0], tl[1], nr, bn * NB);
+    else if (nr <= 16) expert_stream_tile<UP, 2, ONCE>(p, sl, tl[0], tl[1], nr, bn * NB);
+    else expert_stream_tile<UP, 4, ONCE>(p, sl, tl[0], tl[1], nr, bn * NB);
+  });
 }
 
 template <bool UP>
@@ -692,7 +704,7 @@ __global__ void __launch_bounds__(256, 2) expert_block_kernel(ExpertArgs p) {
   const int* t0 = p.tiles + id / nb * 5;
   const int in = id - t0[3] * nb, tile = t0[3] + in % t0[4], bn = in / t0[4];
   const int* tl = p.tiles + tile * 5;
-  expert_block_tile<UP>(p, sl, tl[0], tl[1], tl[2], bn * NB);
+  once_or_again(tl[4], [&](auto once) { expert_block_tile<UP, decltype(once)::value>(p, sl, tl[0], tl[1], tl[2], bn * NB); });
 }
 
 // Whether a product of up to 32 rows a tile goes to blocks of 128 weight rows: past (K - 704) / 48 rows an expert, or, where blocks of 32 run all
@@ -765,7 +777,7 @@ __device__ __forceinline__ void expert_store(const ExpertArgs& p, const f32x16 (
 
 // WN x WM waves, each with AI runs of 32 weight rows and BJ of 32 rows. FAR: addresses of 64 bits, for activations or an expert's
 // weights that 32-bit byte offsets do not span
-template <bool UP, int WN, int AI, int WM, int BJ, bool FAR = false>
+template <bool UP, int WN, int AI, int WM, int BJ, bool FAR = false, bool ONCE = false>
 __device__ __forceinline__ void expert_gemm_tile(const ExpertArgs& p, bf16_t* gl, int ex, int lo, int nr, int n0) {
   constexpr int WP = WN * AI, RP = WM * BJ, NP = WP + RP;  // staging passes of 32 rows: weights, activations
   constexpr int STG = NP * 32 * GBK;                       // one stage (elements)
@@ -805,7 +817,7 @@ __device__ __forceinline__ void expert_gemm_tile(const ExpertArgs& p, bf16_t* gl
       return;
     }
     const unsigned kw = min(k, K - 8) * 2, kx = k < K ? k * 2 : OUT;
-    const auto v = i < WP ? __builtin_amdgcn_raw_buffer_load_b128(rw, wo[i < WP ? i : 0] + kw, 0, 0)
+    const auto v = i < WP ? __builtin_amdgcn_raw_buffer_load_b128(rw, wo[i < WP ? i : 0] + kw, 0, ONCE ? 2 : 0)
                           : __builtin_amdgcn_raw_buffer_load_b128(rx, xo[i < WP ? 0 : i - WP] + kx, 0, 0);
     r[i] = *reinterpret_cast<const u32x4*>(&v);
   };
@@ -964,10 +976,13 @@ __global__ void __launch_bounds__(512, 1) expert_turns_kernel(ExpertArgs p) {
   const int in = id - t0[3] * nb, tile = t0[3] + in % t0[4], bn = in / t0[4];
   const int* tl = p.tiles + tile * 5;
   const int nr = tl[2], n0 = bn * NB;
-  if (nr > 192) expert_turns_tile<UP, 4>(p, sl, tl[0], tl[1], nr, n0);
-  else if (nr > 128) expert_turns_tile<UP, 3>(p, sl, tl[0], tl[1], nr, n0);
-  else if (nr > 64) expert_turns_tile<UP, 2>(p, sl, tl[0], tl[1], nr, n0);
-  else expert_turns_tile<UP, 1>(p, sl, tl[0], tl[1], nr, n0);
+  once_or_again(tl[4], [&](auto once) {
+    constexpr bool ONCE = decltype(once)::value;
+    if (nr > 192) expert_turns_tile<UP, 4>(p, sl, tl[0], tl[1], nr, n0);
+    else if (nr > 128) expert_turns_tile<UP, 3, ONCE>(p, sl, tl[0], tl[1], nr, n0);
+    else if (nr > 64) expert_turns_tile<UP, 2, ONCE>(p, sl, tl[0], tl[1], nr, n0);
+    else expert_turns_tile<UP, 1, ONCE>(p, sl, tl[0], tl[1], nr, n0);
+  });
 }
 
 // NARROW: tiles of up to 192 rows x 128 weight rows (FAR: 128 rows)
@@ -983,9 +998,12 @@ __global__ void __launch_bounds__(256, NARROW ? 2 : 1) expert_gemm_kernel(Expert
   if constexpr (FAR) {
     expert_gemm_tile<UP, 2, 2, 2, 2, true>(p, gl, tl[0], tl[1], nr, n0);
   } else if constexpr (NARROW) {
-    if (nr > 128) expert_gemm_tile<UP, 2, 2, 2, 3>(p, gl, tl[0], tl[1], nr, n0);
-    else if (nr > 64) expert_gemm_tile<UP, 2, 2, 2, 2>(p, gl, tl[0], tl[1], nr, n0);
-    else expert_gemm_tile<UP, 2, 2, 2, 1>(p, gl, tl[0], tl[1], nr, n0);
+    once_or_again(tl[4], [&](auto once) {
+      constexpr bool ONCE = decltype(once)::value;
+      if (nr > 128) expert_gemm_tile<UP, 2, 2, 2, 3, false, ONCE>(p, gl, tl[0], tl[1], nr, n0);
+      else if (nr > 64) expert_gemm_tile<UP, 2, 2, 2, 2, false, ONCE>(p, gl, tl[0], tl[1], nr, n0);
+      else expert_gemm_tile<UP, 2, 2, 2, 1, false, ONCE>(p, gl, tl[0], tl[1], nr, n0);
+    });
   } else {
     if (nr > 192) expert_gemm_tile<UP, 2, 4, 2, 4>(p, gl, tl[0], tl[1], nr, n0);
     else if (nr > 160) expert_gemm_tile<UP, 4, 2, 1, 6>(p, gl, tl[0], tl[1], nr, n0);
