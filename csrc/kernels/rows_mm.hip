@@ -83,7 +83,7 @@ __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
 // the products (weights as the A operand: a lane holds one activation row and four outputs) hide under it. Blocks of 64 rows
 // where they are no more than the CUs, or K is sliced: partial sums (4 bytes beside 2 of a weight, for every activation row) cost
 // more than reading the activations once a block from L2 (61 rows of 16384 x 4096 25.4 us, of 4096 x 4096 12.9; blocks of 128 in twice
-// the slices 29.2, 16.2). Where 64 rows make more blocks than CUs, 128 halve what the activations cost (`wide`).
+// the slices 29.2, 16.2). Where 64 rows make more blocks than CUs, 128 halve what the activations cost (`block_rows`).
 // Blocks start their walks of K at different stages (`walk_start`): from the same one they read the same columns of all rows, 2K bytes
 // apart, at one time, which few of the memory's channels hold. 61 rows, us, from the first stage and this: 12288 x 4096 26.3, 24.3;
 // 16384 x 4096 32.1, 25.6; 4096 x 16384 34.3, 30.0; 14336 x 14336 93.1, 86.0; loads alone of 16384 x 4096 30.2, 23.8. Weights packed so that a
@@ -104,8 +104,9 @@ __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
 template <bool F16, int NB, int W, int XR, int WM, int SNB, bool TWO>
 __global__ void __launch_bounds__(64 * W, 2) rows_mm_kernel(RowsArgs p) {
   constexpr int WN = W / WM, A = NB / WN / 16, B = XR / WM / 16;  // a wave's runs of 16 weight and activation rows
-  constexpr int STG = (NB + XR) * SK * 2, WI = NB / 8 / W, XI = XR / 8 / W, PER = WI + XI;
-  static_assert(WI > 0 && XI > 0 && A > 0 && B > 0);
+  constexpr int XP = XR / 8, XI = (XP + W - 1) / W;  // pieces of 8 activation rows, requests a wave (7 waves: some of a piece that another one requests)
+  constexpr int STG = (NB + XR) * SK * 2, WI = NB / 8 / W, PER = WI + XI;
+  static_assert(WI * W * 8 == NB && A * WN * 16 == NB && B * WM * 16 == XR);
   extern __shared__ __attribute__((aligned(1024))) char sl[];  // [SNB][NB weight rows | XR activation rows][128 B]
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wn = wv % WN, wm = wv / WN;
   const int r16 = lane & 15, g = lane >> 4;
@@ -129,7 +130,7 @@ __global__ void __launch_bounds__(64 * W, 2) rows_mm_kernel(RowsArgs p) {
     }
 #pragma unroll
     for (int i = 0; i < XI; ++i) {
-      const int r = wv * 8 * XI + 8 * i + (lane >> 3);
+      const int r = 8 * min(wv * XI + i, XP - 1) + (lane >> 3);
       x[i] = ((unsigned)min(r, p.M - 1) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7))) * 2;
     }
   };
@@ -154,7 +155,7 @@ __global__ void __launch_bounds__(64 * W, 2) rows_mm_kernel(RowsArgs p) {
                                                one ? wo[i] : wo2[i], k, 0, 2);
 #pragma unroll
     for (int i = 0; i < XI; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(fx, (void __attribute__((address_space(3)))*)(st + (NB / 8 + wv * XI + i) * 1024), 16,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(fx, (void __attribute__((address_space(3)))*)(st + (NB / 8 + min(wv * XI + i, XP - 1)) * 1024), 16,
                                                one ? xo[i] : xo2[i], k, 0, 0);
 #endif
   };
@@ -286,9 +287,14 @@ int go(const RowsArgs& a, hipStream_t s) {
 // Blocks of 128 weight rows: where 64 make more blocks than CUs and 128 fill whole rounds of them better. us, 61 rows, 64 and 128 a block
 // (x 4096): 18432 44.0, 35.2; 24576 46.9, 37.7; 12288 and 16384 beside each other 51, 41.7; 32768 48.9, 46.1; 50400 93, 80.6; 57344 99.5, 88.6; a
 // second round of a few blocks loses: 36864 70.5, 73.9; 43008 71.9, 77.1; not for 128 rows, whose products cost as much as their weights: 91.8, 88.6.
-bool wide(const RowsArgs& a, int xr) {
-  const int n = blocks_of(a, 128);
-  return a.ks == 1 && blocks_of(a, 64) > 256 && (n <= 256 || n > 384 || xr == 128);
+// Blocks of 112, two a CU, where its most loaded CU has fewer rows then: 32 rows, 128 and 112 a block: 50400 x 4096 75.1, 71.0, x 2048 41.4, 37.0; 57344 78.9,
+// 75.3, 42.1, 39.5; one round of blocks gains nothing (28672 x 4096, 224 blocks and 256, 39.3, 40.0).
+int block_rows(const RowsArgs& a, int xr) {
+  if (a.ks > 1 || blocks_of(a, 64) <= 256) return 64;
+  const int n = blocks_of(a, 128), rounds = (n + 255) / 256;
+  if (xr == 128 || n <= 256) return 128;
+  if (n <= 384) return 64;
+  return (blocks_of(a, 112) + 255) / 256 * 112 < rounds * 128 ? 112 : 128;
 }
 
 // Checks what the kernel asks of its arguments and launches it
@@ -312,7 +318,12 @@ int rows_mm(int dtype, const RowsArgs& a, long long ws_floats, int cnt_n, hipStr
   if (blocks * a.ks >= 1ll << 31) return 3;
   if (a.ks > 1 && (!a.ws || !a.cnt || !al16(a.ws) || ws_floats < blocks * a.ks * 64 * xr || cnt_n < blocks)) return 6;
   const bool f16 = dtype == 2;
-  if (wide(a, xr)) {
+  const int nb = block_rows(a, xr);
+  if (nb == 112) {
+    if (xr == 32) return f16 ? go<true, 112, 7, 32, 1, 4>(a, s) : go<false, 112, 7, 32, 1, 4>(a, s);
+    return f16 ? go<true, 112, 7, 64, 1, 3>(a, s) : go<false, 112, 7, 64, 1, 3>(a, s);
+  }
+  if (nb == 128) {
     if (xr == 32) return f16 ? go<true, 128, 4, 32, 1, 4>(a, s) : go<false, 128, 4, 32, 1, 4>(a, s);
     if (xr == 64) return f16 ? go<true, 128, 8, 64, 2, 4>(a, s) : go<false, 128, 8, 64, 2, 4>(a, s);
     return f16 ? go<true, 128, 8, 128, 2, 3>(a, s) : go<false, 128, 8, 128, 2, 3>(a, s);

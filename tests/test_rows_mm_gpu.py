@@ -119,6 +119,21 @@ def test_blocks_of_64_and_128_weight_rows(dtype, rows, n, k):
         assert _close(_rows_mm(x, w, None), F.linear(x.float(), w.float()))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [3, 32, 33, 64])
+@pytest.mark.parametrize("n,k", [(50400, 320), (51216, 64), (57344, 192), (57360, 128)])
+def test_blocks_of_112_weight_rows(dtype, rows, n, k):
+    """Seven waves, some of which request a piece of the activations that another one requests too; the last one is back at blocks of 128."""
+    x, w, b, ref = _inputs(rows, n, k, dtype, True)
+    x2, w2, b2, ref2 = _inputs(rows, 48, 64, dtype, True, 4)
+    with torch.no_grad():
+        y = _rows_mm(x, w, b)
+        assert _close(y, ref) and torch.equal(y, _rows_mm(x, w, b))
+        if rows <= 24:  # (more rows of so many outputs are the library's beside another product)
+            for got, want in zip(few_rows_beside((x, w, b), (x2, w2, b2), None), (ref, ref2)):
+                assert _close(got, want)
+
+
 @pytest.mark.parametrize("rows", [5, 61, 100])
 @pytest.mark.parametrize("n,k,n2,k2", [(12304, 192, 4096, 640), (8192, 64, 8208, 320), (16384, 320, 16, 64)])
 def test_two_products_in_wide_blocks(rows, n, k, n2, k2):
