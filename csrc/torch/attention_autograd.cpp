@@ -5,6 +5,8 @@
 // Why: a short training call is bound by the host. 1 x 96 tokens x 12 heads of 64, forward and backward, is 20 us of kernels
 // that took 132 us to issue: ctypes converts 33 and 45 arguments (25 us), and the backward pass waits for the interpreter
 // lock in the engine's thread.
+#include "prompt_rows.h"
+
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/DeviceGuard.h>
@@ -140,6 +142,11 @@ PyObject* init(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 PyMethodDef methods[] = {{"attention", (PyCFunction)(void (*)())attention, METH_FASTCALL, nullptr},
                          {"init", (PyCFunction)(void (*)())init, METH_FASTCALL, nullptr},
+                         {"few_rows", (PyCFunction)(void (*)())kca_few_rows, METH_FASTCALL, nullptr},
+                         {"norm_rows", (PyCFunction)(void (*)())kca_norm_rows, METH_FASTCALL, nullptr},
+                         {"rope_append", (PyCFunction)(void (*)())kca_rope_rows, METH_FASTCALL, nullptr},
+                         {"packed_attention", (PyCFunction)(void (*)())kca_packed_rows, METH_FASTCALL, nullptr},
+                         {"init_rows", (PyCFunction)(void (*)())kca_init_rows, METH_FASTCALL, nullptr},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module{PyModuleDef_HEAD_INIT, "kca_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -175,7 +175,7 @@ _torch_ext: list = []
 
 
 def torch_ext():
-    """The extension module ``kca_torch`` (autograd functions in C++) bound to the loaded kernel library, or None where it is
+    """The extension module ``kca_torch`` (autograd functions and a prompt layer's operators in C++) bound to the loaded kernel library, or None where it is
     not built, does not fit this torch, or launches are synchronised one by one: callers then take the same function in Python."""
     if not _torch_ext:
         lib = _load()
@@ -190,11 +190,19 @@ def torch_ext():
                         if m.torch != torch.__version__:
                             raise ImportError(f"built for torch {m.torch}, this is {torch.__version__}")
                         m.init(*(ctypes.cast(f, P).value for f in (lib.kca_attn_fwd, lib.kca_attn_bwd)))
+                        m.init_rows(*(ctypes.cast(f, P).value for f in (
+                            lib.kca_rows_mm_two, lib.kca_layernorm_fwd, lib.kca_ln_rows_f16, lib.kca_rope_append,
+                            lib.kca_attn_fwd_packed)), counters)
                     except (ImportError, AttributeError) as e:  # another torch than it was built for
                         warnings.warn(f"{path}: {e}")
                         m = None
                 _torch_ext.append(m)
     return _torch_ext[0]
+
+
+def plain_ext():
+    """``torch_ext`` for a call whose operator may run there, without gradients; None while torch compiles or records them."""
+    return None if torch.is_grad_enabled() or torch.compiler.is_compiling() else torch_ext()
 
 
 def ensure_built(sources) -> None:

@@ -215,6 +215,12 @@ def packed_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu: torc
     ``cu[i]`` .. ``cu[i + 1]`` (int32, on the device), none longer than ``max_len``. bf16, or fp16 with softmax weights of 24
     bits."""
     T, H, D = q.shape
+    ext = _lib.plain_ext() if q.is_cuda and alibi is None else None
+    if ext is not None:
+        o = ext.packed_attention(q, k, v, cu, max_len, scale if scale is not None else 1.0 / math.sqrt(D), window)
+        if o is not None:
+            _lib.LAUNCHES[0] += 1
+            return o
     f16 = q.dtype == torch.float16
     _check(*(t.unsqueeze(0) for t in (q, k, v)), dtype=torch.float16 if f16 else torch.bfloat16)
     n = cu.shape[0] - 1

@@ -281,6 +281,12 @@ def _few_launch(parts, act: int, act2: int, beside: bool, rows: int, scratch=Non
     """One launch of ``kca_rows_mm_two`` over one or two (x, weight, bias); None: sizes, types or a mode of torch (gradients,
     transforms, captures without ``few_rows_scratch``, ...) that it does not serve."""
     x = parts[0][0]
+    ext = _lib.plain_ext() if scratch is None and x.is_cuda else None
+    if ext is not None and 0 < rows <= FEW_ROWS and all(few_rows(rows, *p[1].shape) for p in parts):
+        y = ext.few_rows(*parts[0], *(parts[1] if len(parts) > 1 else (None, None, None)), act, act2, beside, rows)
+        if y is not None:
+            _lib.LAUNCHES[0] += 1
+            return y
     if (not 0 < rows <= FEW_ROWS or not x.is_cuda or (scratch is None and torch.cuda.is_current_stream_capturing())
             or not all(p[0].dtype == x.dtype and _few_part(*p, rows) for p in parts)
             or not _lib.inference(*(t for p in parts for t in p)) or not _lib.has("kca_rows_mm_two")):

@@ -93,6 +93,12 @@ def rope_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, rot: int, int
     """Prompt rows [T, H, D] (views of a fused projection): rotates q and k in place and writes k and v to row ``off`` of
     page ``page`` (< 0: nowhere) of a cache [pages, Hkv, rows, D]. ``pos``, ``page``, ``off``: int32 [T]. One launch
     (``csrc/kernels/rope_append.hip``); False, and nothing done, for tensors it does not take."""
+    ext = _lib.plain_ext() if q.is_cuda else None
+    if ext is not None:
+        took = ext.rope_append(q, k, v, rot, interleaved, cos, sin, pos, page, off, kc, vc)
+        if took is not None:
+            _lib.LAUNCHES[0] += took
+            return took
     code = {torch.bfloat16: 1, torch.float16: 2}.get(q.dtype)
     T, H, D = q.shape
     if (code is None or not q.is_cuda or any(t.dtype != q.dtype for t in (k, v, kc, vc))

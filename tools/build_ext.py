@@ -176,7 +176,8 @@ def build_torch(verbose: bool = False) -> str:
              f"-I{base}/include", f"-I{base}/include/torch/csrc/api/include", f"-I{ROCM}/include",
              f"-I{sysconfig.get_paths()['include']}"]
     cxx = shutil.which("g++") or "g++"
-    objs = [_compile([cxx], s, [], obj_dir, flags) for s in _sources("torch", (".cpp",))]
+    hdrs = _sources("torch", (".h",))
+    objs = [_compile([cxx], s, hdrs, obj_dir, flags) for s in _sources("torch", (".cpp",))]
     out = os.path.join(OUT_DIR, "kca_torch.so")
     cmd = [cxx, "-shared", "-fPIC", "-o", out + ".tmp"] + objs + [
         f"-L{base}/lib", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
