@@ -89,12 +89,12 @@ __device__ __forceinline__ void wait_reads() {
 // ---------------------------------------------------------------------------------------------- stream
 // bf16, tiles of up to 32 rows x 32 weight rows (up: 16 gate rows and the 16 up rows beside them), 4 waves, each with every fourth stage
 // of 64 of K; the waves' sums meet in LDS. Bound by the weight stream. How fast memory gives it hangs on how far apart the rows lie that
-// the chip reads at one time: blocks of 64 rows that walk K by themselves have the whole of a weight in flight, 4.7 to 4.9 TB/s (50432 x
+// the chip reads at one time: blocks of 64 rows that walk K by themselves have the whole of a weight in flight, ordinary loads 4.7 to 4.9 TB/s (50432 x
 // 4096, loads alone), of 32 rows, K over the waves, 6.0; the number of bytes in flight and the length of a request's rows make no
 // difference. A wave's stages go straight to LDS, weights three stages ahead, activations, in the XCD's cache, two; no wave
 // waits for another before the end, and two workgroups a CU cover each other's ramps. Beside the gemv kernel, whose vector products a row
 // cost more than its weights from about 2 rows an expert on, and the gemm, which computes and stages mostly padding.
-// Both products of a layer, us, blocks of 64 weight rows that walk K by themselves (the form before) and this: 20 outputs, 16 experts of 3 x
+// Both products of a layer, us, ordinary loads, blocks of 64 weight rows that walk K by themselves (the form before) and this: 20 outputs, 16 experts of 3 x
 // 4096 x 2048, top 3: 20 tokens 163, 142, 64 173, 143; 32 of 3 x 2048 x 1024, top 4: 64 85, 80; 16 of 3 x 4096 x 4096, top 2: 32 282,
 // 274, 130 295, 278. Workgroups in plain order 149, 87, 281, 307; an XCD a contiguous eighth of the blocks 161, 84, 278, 301; runs of
 // 512 151, 83, 293, 308; a fourth weight stage, one workgroup a CU, 172, 102, 285, 310.
@@ -206,7 +206,7 @@ constexpr int STREAM_LDS = 4 * (3 * 4096 + 2 * 4 * 1024);
 
 // The same tiles x 128 weight rows (up: 64 gate rows and the 64 up rows beside them) that walk K by themselves, 32 of them a wave; all waves read a
 // stage's activations, requested once: 20 KB a stage, three stages ahead, two workgroups a CU. It has a quarter of the blocks, starts and
-// sums over waves, and half as many requests a weight row where tiles have more than 16 rows, but its weights come at 4.7 to 4.9 TB/s. So it is the
+// sums over waves, and half as many requests a weight row where tiles have more than 16 rows, but its weights come slower (ordinary loads 4.7 to 4.9 TB/s). So it is the
 // better one where the walk is short for its rows (stream_block).
 constexpr int BWN = 128, BSTAGE = (BWN + SROWS) * SK * 2;
 static_assert(4 * BSTAGE == STREAM_LDS, "four stages");

@@ -83,9 +83,9 @@ __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
 // the products (weights as the A operand: a lane holds one activation row and four outputs) hide under it. Blocks of 64 rows
 // where they are no more than the CUs, or K is sliced: partial sums (4 bytes beside 2 of a weight, for every activation row) cost
 // more than reading the activations once a block from L2 (61 rows of 16384 x 4096 25.4 us, of 4096 x 4096 12.9; blocks of 128 in twice
-// the slices 29.2, 16.2). Where 64 rows make more blocks than CUs, 128 halve what the activations cost (`block_rows`).
+// the slices 29.2, 16.2; 64 in twice the slices, 32 rows of 4096 x 16384 and x 4096 30.2, 35.0). Where 64 rows make more blocks than CUs, 128 halve what the activations cost (`block_rows`).
 // Blocks start their walks of K at different stages (`walk_start`): from the same one they read the same columns of all rows, 2K bytes
-// apart, at one time, which few of the memory's channels hold. 61 rows, us, from the first stage and this: 12288 x 4096 26.3, 24.3;
+// apart, at one time, which few of the memory's channels hold. 61 rows, us, ordinary loads, from the first stage and this: 12288 x 4096 26.3, 24.3;
 // 16384 x 4096 32.1, 25.6; 4096 x 16384 34.3, 30.0; 14336 x 14336 93.1, 86.0; loads alone of 16384 x 4096 30.2, 23.8. Weights packed so that a
 // stage is one piece of memory come to the same (24.4). The order of the sums follows from the block, the same at every run.
 // Where the blocks are fewer than the CUs, slices of K write partial sums and the last to arrive adds them in slice order.
@@ -93,10 +93,9 @@ __device__ __forceinline__ f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
 // piece cover all 64 banks) on the source address.
 // us, hipBLASLt : this (weights cold, both in a captured graph; at the copy rate 20.9, 27.8, 7.0, 27.8, 86):
 //   rows   12288 x 4096   16384 x 4096   4096 x 4096   4096 x 16384   50400 x 4096
-//     16    25.8 : 19.3    31.7 : 25.3   15.5 : 14.0   30.1 : 29.6    88.9 : 79.6
-//     64    26.2 : 24.7    31.9 : 25.7   15.4 : 15.2   41.0 : 31.9    90.4 : 81.4
-//    128    32.1 : 34.1    35.4 : 34.5   24.5 : 19.3   79.1 : 42.2    98.8 : 98.3
-// A call costs the host 14 us, the library's through the tuned table 20 to 26.
+//     16    28.1 : 19.4    33.1 : 23.2   15.3 : 11.0   30.1 : 25.0    80.7 : 67.8
+//     64    24.7 : 24.0    32.5 : 25.6   14.8 : 12.5   41.5 : 29.3    82.2 : 76.4
+//    128    31.7 : 33.3    36.6 : 35.1   24.2 : 16.6   80.8 : 41.4    88.1 : 95.5
 // Which sizes run here: few_rows in ops/linear.py.
 // XR activation rows; W waves, WM of them across the activation rows (8 rather than 4 read less from LDS: 61 rows of 2048 x 8192 and x 2048
 // 16.7, 15.9); SNB stages.

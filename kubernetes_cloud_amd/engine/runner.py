@@ -770,7 +770,7 @@ class ModelRunner(StepRunner):
         # (_layers_decode_rows). Four layers, us a step, this and before it (2 to 16 rows: the matrix-core layer; more: one launch a
         # product, the feed-forward's on a side stream): 4096 wide, 400 tokens behind, 2 rows 492, 514; 5 535, 559; 8 543, 581; 16 589, 636;
         # 24 of 100 558, 623; 32 of 700 795, 830; 64 of 300 948, 1077; 128 of 200 2066, 2220; 2048 wide, 100 behind, 2 rows 248, 262;
-        # 16 272, 303; 64 435, 520
+        # 16 272, 303; 64 435, 520; this with weights and cache read non-temporal 427, 451, 468, 512, 496, 700, 942, 1853; 224, 244, 448
         self._rows_ok = self._batched_ok and self._embed_head and self._layer_kind == "gptj" and not tp and model.emb_ln is None
         self.rows_steps = 0
         # largest batch bucket the matrix-core layer takes, per layer kind, from same-box A/Bs against the
@@ -1204,7 +1204,7 @@ class ModelRunner(StepRunner):
     def _layers_decode_rows(self, tokens, pos, slots, kv_lens, max_kv, ws, obuf):
         """Decode step of GPT-J layers at batch 2 to FEW_ROWS (see _rows_ok): QKV and fc_in (GELU on its sums) in one launch of the
         weight-streaming kernel, attention, then fc_out and out in one, and the norm that adds their sum. One queue: the
-        feed-forward on a side stream beside the attention costs a fork and a join a layer (32 rows, 700 behind 824 us, this 793).
+        feed-forward on a side stream beside the attention costs a fork and a join a layer (32 rows, 700 behind 824 us, this 793, both with ordinary loads).
         None: sizes or a mode that the kernel does not serve; nothing has run then but the step's head."""
         m, cfg = self.model, self.cfg
         B = tokens.shape[0]

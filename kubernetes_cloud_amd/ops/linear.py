@@ -172,23 +172,23 @@ FEW_ROWS = 128
 
 def few_rows(rows: int, n: int, k: int, captured: bool = False) -> bool:
     """Whether a product of few rows goes to the weight-streaming kernel. On the GPU, us, hipBLASLt : the kernel, weights cold, in captures
-    (where a product cut over K takes 1.6 to 2 us more, a fill of the graph's own counters):
+    (where a product cut over K takes 1.6 to 2 us more, a fill of the graph's own counters, not counted here):
 
-        12288 x 4096   8 rows 26.1 : 19.3    32: 23.2 : 20.5    64: 26.2 : 24.7    96: 30.5 : 32.5    128: 32.1 : 34.1
-        16384 x 4096          31.9 : 25.4        30.5 : 24.0        31.9 : 25.7        34.0 : 32.8         35.4 : 34.5
-        4096 x 4096           15.9 : 14.0        14.0 : 14.5        15.4 : 15.2        22.3 : 18.7         24.5 : 19.3
-        4096 x 16384          29.6 : 29.6        32.9 : 29.5        41.0 : 31.9        66.4 : 40.7         79.1 : 42.2
-        8192 x 2048           14.7 : 13.3        13.4 : 13.3        13.9 : 14.6        15.0 : 18.2         16.1 : 18.8
-        5120 x 20480           110 : 43           117 : 43           128 : 49           138 : 62            145 : 64
-        14336 x 14336         82.5 : 73.8        81.2 : 74.1        93.0 : 86.2       100.9 : 110.1       117.0 : 115.0
-        50400 x 4096          88.9 : 77.7        86.3 : 78.7        90.4 : 81.4        93.7 : 94.5         98.8 : 98.3
+        12288 x 4096  16 rows 28.1 : 19.4    32: 22.5 : 19.6    64: 24.7 : 24.0    96: 29.5 : 31.6    128: 31.7 : 33.3
+        16384 x 4096          33.1 : 23.2        31.5 : 22.1        32.5 : 25.6        34.7 : 33.7         36.6 : 35.1
+        4096 x 4096           15.3 : 11.0        12.9 : 11.2        14.8 : 12.5        21.8 : 15.8         24.2 : 16.6
+        4096 x 16384          30.1 : 25.0        33.9 : 25.9        41.5 : 29.3        68.0 : 39.2         80.8 : 41.4
+        8192 x 2048           12.8 : 10.1        12.9 : 10.3        13.4 : 11.3        14.3 : 15.0         15.7 : 15.6
+        5120 x 20480           114 : 38           121 : 39           129 : 46           139 : 62            146 : 64
+        14336 x 14336         81.1 : 66.9        80.1 : 68.9        91.2 : 82.3       101.2 : 108.3       118.7 : 112.2
+        50400 x 4096          80.7 : 67.8        77.2 : 71.0        82.2 : 76.4        85.1 : 91.1         88.1 : 95.5
 
     A call costs the host 6 to 12 us less, and a layer of a short prompt is issued in about the time that it runs in. So an eager
     call takes the kernel also where it is a little slower: four GPT-J layers of 4096, 100 tokens, 1030 us with the library from 65
     rows on for 12288 and 16384 outputs, 900 without it; of 2048, 980 and 735. Not past 2^27 weights and 64 rows, unless few
     blocks leave the library's products without CUs; and up to 24 rows where blocks of 64 weight rows are more than the CUs (24: 20480 x 5120
-    45.5 : 44.1, 24576 x 6144 71 : 55; 64: 47.8 : 51.0, 74 : 64). More than 128 rows: the library (200 rows of 12288 x 4096 39.9 : 52.5).
-    In a capture there is no host time to save: 16 rows of 1024 x 1024 6.0 : 8.3, of 5120 x 5120 15.2 : 17.3."""
+    43.1 : 42.4, 24576 x 6144 70.8 : 53.2; 64: 48.1 : 51.1, 73.9 : 59.8). More than 128 rows: the library (200 rows of 12288 x 4096 39.9 : 52.5).
+    In a capture there is no host time to save: 16 rows of 1024 x 1024, cut over K, 7.2 : 6.7 and the fill."""
     if n > 64 * _CUS:
         return rows <= 24
     if captured:
@@ -205,9 +205,9 @@ def _k_slices(n: int, k: int) -> int:
 def _rows_mm(x2: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor | None:
     """The product of up to FEW_ROWS rows on the weight-streaming kernel; None: sizes or alignment it does not take. One row, and two
     where the vector kernel of the decode steps holds them in registers, go to that: no stage in LDS, no rows that are not there. us, rows'
-    kernel : vector kernel, one row and two: 50400 x 4096 78.9 : 56.4, 78.3 : 59.3; 12288 x 4096 21.2 : 16.2, 21.3 : 17.9; 4096 x 16384 31.4 :
-    21.8, 31.4 : 37.0; 2048 x 8192 11.6 : 7.6, 11.7 : 8.5; 14336 x 14336 75.7 : 59.5; 4096 x 1024 7.0 : 4.8, 7.1 : 5.9; short rows of wide
-    weights stay: 32000 x 1024 14.6 : 16.4, 14.6 : 23.3; 50400 x 768 19.1 : 23.3. Errors against 64 bits are the same."""
+    kernel : vector kernel, one row and two: 50400 x 4096 67.6 : 56.4, 59.3; 12288 x 4096 20.2 : 16.2, 17.9; 4096 x 16384 25.7 :
+    21.8, 37.0; 2048 x 8192 11.2 : 7.6, 8.5; 14336 x 14336 67.8 : 59.5; 4096 x 1024 6.9 : 4.8, 5.9; short rows of wide
+    weights stay: 32000 x 1024 13.3 : 16.4, 23.3; 50400 x 768 15.5 : 23.3. Errors against 64 bits are the same."""
     rows, k = x2.shape
     n = weight.shape[0]
     if (n % 16 or k % 64 or k == 0 or 2 * max(n, rows) * k >= 1 << 32 or not weight.is_contiguous() or x2.data_ptr() % 16
@@ -322,8 +322,8 @@ def few_rows_gelu(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | No
 
 def few_rows_beside(first: tuple, second: tuple, approx2: str | None = None, scratch=None):
     """Two products (x, weight, bias) of the same few rows in one launch, a GELU on the second's fp32 sums -> (y, y2) or None.
-    On the GPU, us, apart and together, 61 rows: 12288 and 16384 x 4096 24.3 + 25.6, 41.7; 6144 and 8192 x 2048 11.4 + 12.4, 15.6;
-    128 rows 33.3 + 34.4, 49.1; and a launch and the GELU's less."""
+    On the GPU, us, apart and together, 61 rows: 12288 and 16384 x 4096 24.0 + 25.6, 40.5; 6144 and 8192 x 2048 11.0 + 11.3, 16.5;
+    128 rows 33.3 + 35.1, 54.9; and a launch and the GELU's less."""
     x = first[0]
     rows = x.numel() // x.shape[-1]
     y = _few_launch([first, second], 0, ACTS[approx2], True, rows, scratch) if approx2 in ACTS else None
@@ -332,8 +332,8 @@ def few_rows_beside(first: tuple, second: tuple, approx2: str | None = None, scr
 
 def few_rows_sum(first: tuple, second: tuple, scratch=None) -> torch.Tensor | None:
     """The sum of two products (x, weight, bias) of the same few rows in one launch, rounded once; or None. On the GPU, us, apart and
-    together, 61 rows: 4096 x 16384 and x 4096 29.9 + 13.2, 36.4; 2048 x 8192 and x 2048 14.0 + 9.1, 15.9;
-    128 rows 40.3 + 16.9, 49.2."""
+    together, 61 rows: 4096 x 16384 and x 4096 29.3 + 12.5, 35.3; 2048 x 8192 and x 2048 13.2 + 8.8, 15.2;
+    128 rows 41.4 + 16.6, 49.9."""
     x = first[0]
     rows = x.numel() // x.shape[-1]
     if first[1].shape[0] != second[1].shape[0]:
@@ -528,7 +528,7 @@ def linear_residual(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | 
 
 def few_rows_head(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
     """Logits [rows, n] of a decode step's rows: past ``few_rows``' 24 rows of more blocks of 64 weight rows than CUs too, where blocks of 128
-    are on most CUs (table of ``few_rows``; 48 rows of 50400 x 2048 50.6 : 42.9, of 20480 x 5120, 160 blocks, 47.1 : 48.9)."""
+    are on most CUs (table of ``few_rows``; 48 rows of 43008 x 4096 79.0 : 65.7, of 20480 x 5120, 160 blocks, 47.0 : 48.4)."""
     (rows, k), n = x.shape, weight.shape[0]
     if (n > 64 * _CUS and rows <= (64 if n >= 96 * _CUS else 32) and k >= 1024 and x.dtype in (torch.bfloat16, torch.float16)
             and x.dtype == weight.dtype and x.is_contiguous() and (bias is None or (bias.shape == (n,) and bias.dtype == x.dtype))

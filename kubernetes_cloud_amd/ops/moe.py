@@ -144,7 +144,10 @@ def tile_rows(T: int, top: int, E: int, d: int, F: int, dtype) -> int:
     products; r 40, 80, 110; narrow, wide):
         5120, 8, 2, 2560 (160, 160): 161, 138; 173, 161; 179, 187     5632, 6, 2, 2816 (132, 132): 166, 143; 173, 159; 187, 180
         4352, 8, 2, 2176 (136, 136): 135, 117; 131, 152; 141, 153     5120, 8, 2, 3840 (240, 160): 201, 180; 225, 210; 247, 218
-        4096, 8, 2, 2560 (160, 128): 129, 130; 143, 154; 153, 161     5120, 6, 2, 5120 (240, 120): 184, 194"""
+        4096, 8, 2, 2560 (160, 128): 129, 130; 143, 154; 153, 161     5120, 6, 2, 5120 (240, 120): 184, 194
+    (All with ordinary loads. Non-temporal weights, sublayer, narrow, wide: 4096, 16, 2, 4096: 300: 317, 333; 777: 380, 350; 2048, 32, 4, 1024:
+    500: 118, 127; 900: 137, 138; 1200: 147, 141; 2048, 24, 5, 768: 500: 97, 104; 777: 110, 110; with four identity outputs, which the rule counts as
+    experts, 4096, 16, 3, 2048: 500: 205, 221; 640: 240, 226; 777: 250, 227.)"""
     n = T * top
     used = min(E, n)
     # 32-bit offsets into an expert's weights and the rows of a tile (elsewhere only 128-row tiles have longer ones)
