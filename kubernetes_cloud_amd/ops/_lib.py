@@ -172,6 +172,7 @@ def _load():
 
 
 _torch_ext: list = []
+_ROWS = ("kca_rows_mm_two", "kca_layernorm_fwd", "kca_ln_rows_f16", "kca_rope_append", "kca_attn_fwd_packed")
 
 
 def torch_ext():
@@ -190,9 +191,9 @@ def torch_ext():
                         if m.torch != torch.__version__:
                             raise ImportError(f"built for torch {m.torch}, this is {torch.__version__}")
                         m.init(*(ctypes.cast(f, P).value for f in (lib.kca_attn_fwd, lib.kca_attn_bwd)))
-                        m.init_rows(*(ctypes.cast(f, P).value for f in (
-                            lib.kca_rows_mm_two, lib.kca_layernorm_fwd, lib.kca_ln_rows_f16, lib.kca_rope_append,
-                            lib.kca_attn_fwd_packed)), counters)
+                        m.rows = all(hasattr(lib, n) for n in _ROWS)  # (a library of a few sources may lack some)
+                        if m.rows:
+                            m.init_rows(*(ctypes.cast(getattr(lib, n), P).value for n in _ROWS), counters)
                     except (ImportError, AttributeError) as e:  # another torch than it was built for
                         warnings.warn(f"{path}: {e}")
                         m = None
@@ -202,7 +203,10 @@ def torch_ext():
 
 def plain_ext():
     """``torch_ext`` for a call whose operator may run there, without gradients; None while torch compiles or records them."""
-    return None if torch.is_grad_enabled() or torch.compiler.is_compiling() else torch_ext()
+    if torch.is_grad_enabled() or torch.compiler.is_compiling():
+        return None
+    ext = torch_ext()
+    return ext if ext is not None and ext.rows else None
 
 
 def ensure_built(sources) -> None:

@@ -26,6 +26,25 @@ def test_another_torch(monkeypatch):
     assert _lib.torch_ext().torch == torch.__version__
 
 
+@pytest.mark.skipif(not os.path.exists(os.path.join(_lib.LIB_DIR, "kca_torch.so")) or not _lib.available(), reason="not built")
+def test_a_library_without_prompt_kernels(monkeypatch):
+    """A library of a few sources: attention stays in the module, a prompt layer's operators go to Python."""
+    class Partial:
+        def __getattr__(self, n):
+            if n == "kca_rope_append":
+                raise AttributeError(n)
+            return getattr(lib, n)
+    lib = _lib._load()
+    with torch.no_grad(), monkeypatch.context() as mp:
+        mp.setattr(_lib, "_torch_ext", [])
+        mp.setattr(_lib, "_load", lambda: Partial())
+        assert _lib.torch_ext() is not None and _lib.plain_ext() is None
+    with torch.no_grad(), monkeypatch.context() as mp:
+        mp.setattr(_lib, "_torch_ext", [])
+        assert _lib.plain_ext() is _lib.torch_ext() is not None
+    assert _lib.plain_ext() is None  # gradients
+
+
 def test_a_build_without_it(monkeypatch, capsys):
     monkeypatch.setattr(build_ext, "build_kernels", lambda *a, debug=False, **k: "debug" if debug else "kernels")
     monkeypatch.setattr(build_ext, "build_host", lambda *a: "host")
