@@ -24,6 +24,23 @@ struct ExpertArgs {
   int tokens, Ns, Ks;
 };
 
+// Whether the last tile of an expert with `c` rows stands after all experts' others (row limits of 128 and 192): it is at most half
+// full, and what its weights cost to read again, away from the expert's other tiles, is less than the CUs that it fills: two full
+// tiles before it, or none, or one of 192 rows and hardly any rows. Both products, us (width, experts, top, inner size), beside its
+// expert's and last: 3000 tokens, 2048, 32, 4, 1024 237, 215; 300, 4096, 16, 3, 2048 218, 199.
+__device__ __forceinline__ bool late_tile(int c, int mt) {
+  const int r = c % mt, full = c / mt;
+  return mt >= 128 && mt < 256 && r && 2 * r <= mt && (full != 1 || (mt > 128 && 8 * r <= mt));
+}
+
+// Whether a tile's weights come non-temporal (request_into_lds): no other tile reads them beside it or later. `tiles`: how many stand together. A
+// late one is the last to read its expert's weights, but a full one of 192 rows by itself may have a late one after it, which finds them in the last
+// cache (196 rows an expert, cold, us, both non-temporal, both ordinary, so: 24 experts of 3 x 2048 x 768 120, 104, 103.5; 32 of 3 x 2048 x 1024 210, 193,
+// 179; 16 of 3 x 4096 x 2048 389, 375, 348; of 3 x 4096 x 4096 672, 677, 638).
+// Tiles that stand together: in the gemm the second of two finds what the first has read: 24 experts of 3 x 2048 x 768, top 5, 500 tokens, us, ordinary
+// 101.3, non-temporal all 102.2, so 97.3; 777 112.3, 114.4, 110.4; 16 of 3 x 4096 x 2048, top 3, 300 210.5, 192, 192.5; 777 267, 253, 250.6.
+__device__ __forceinline__ bool read_once(int tiles, int rows, int mt) { return tiles == 1 && !(mt > 128 && rows == mt); }
+
 // the words of a descriptor of everything from p on, for inline asm
 __device__ __forceinline__ u32x4 uniform_words(const void* p) {
   const unsigned long long a = (unsigned long long)p;

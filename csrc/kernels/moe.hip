@@ -229,15 +229,6 @@ struct GroupArgs {
   int *perm, *inv, *tiles, *ntiles;
 };
 
-// Whether the last tile of an expert with `c` rows stands after all experts' others (row limits of 128 and 192): it is at most half
-// full, and what its weights cost to read again, away from the expert's other tiles, is less than the CUs that it fills: two full
-// tiles before it, or none, or one of 192 rows and hardly any rows. Both products, us (width, experts, top, inner size), beside its
-// expert's and last: 3000 tokens, 2048, 32, 4, 1024 237, 215; 300, 4096, 16, 3, 2048 218, 199.
-__device__ __forceinline__ bool late_tile(int c, int mt) {
-  const int r = c % mt, full = c / mt;
-  return mt >= 128 && mt < 256 && r && 2 * r <= mt && (full != 1 || (mt > 128 && 8 * r <= mt));
-}
-
 // Tiles of up to 256 rows: an expert's rows in units of 64 (a product's steps), as evenly over its tiles as they go: `more` tiles of
 // per + 1 units, then the others. (Full tiles and a short last one, whose weights then came from memory once more: sublayer of 4096
 // tokens, 16 experts of 3 x 4096 x 4096, top 2 893 us, evenly 850.) Experts stand by their largest tile: expert_turns_kernel.
@@ -662,12 +653,9 @@ dim3 block_rows(long long blocks) {
 }
 __device__ __forceinline__ int block_number() { return blockIdx.y * (int)ROW_BLOCKS + blockIdx.x; }
 
-// Whether an expert's weights are read by one tile, and come non-temporal then (request_into_lds). In the gemm, of two tiles that share a
-// cache, the second finds what the first has read: 24 experts of 3 x 2048 x 768, top 5, 500 tokens, us, ordinary 101.3, non-temporal all 102.2, so 97.3;
-// 777 112.3, 114.4, 110.4; 16 of 3 x 4096 x 2048, top 3, 300 210.5, 192, 192.5; 777 267, 253, 250.6.
 template <typename F>
-__device__ __forceinline__ void once_or_again(int tiles, F&& f) {
-  if (tiles == 1) f(std::true_type{});
+__device__ __forceinline__ void once_or_again(bool once, F&& f) {
+  if (once) f(std::true_type{});
   else f(std::false_type{});
 }
 
@@ -686,7 +674,7 @@ __global__ void __launch_bounds__(256, 2) expert_stream_kernel(ExpertArgs p) {
   const int in = id - t0[3] * nb, tile = t0[3] + in % t0[4], bn = in / t0[4];
   const int* tl = p.tiles + tile * 5;
   const int nr = tl[2];
-  once_or_again(tl[4], [&](auto once) {
+  once_or_again(read_once(tl[4], tl[2], p.mt), [&](auto once) {
     constexpr bool ONCE = decltype(once)::value;
     if (nr <= 8) expert_stream_tile<UP, 1, ONCE>(p, sl, tl[0], tl[1], nr, bn * NB);
     else if (nr <= 16) expert_stream_tile<UP, 2, ONCE>(p, sl, tl[0], tl[1], nr, bn * NB);
@@ -704,7 +692,7 @@ __global__ void __launch_bounds__(256, 2) expert_block_kernel(ExpertArgs p) {
   const int* t0 = p.tiles + id / nb * 5;
   const int in = id - t0[3] * nb, tile = t0[3] + in % t0[4], bn = in / t0[4];
   const int* tl = p.tiles + tile * 5;
-  once_or_again(tl[4], [&](auto once) { expert_block_tile<UP, decltype(once)::value>(p, sl, tl[0], tl[1], tl[2], bn * NB); });
+  once_or_again(read_once(tl[4], tl[2], p.mt), [&](auto once) { expert_block_tile<UP, decltype(once)::value>(p, sl, tl[0], tl[1], tl[2], bn * NB); });
 }
 
 // Whether a product of up to 32 rows a tile goes to blocks of 128 weight rows: past (K - 704) / 48 rows an expert, or, where blocks of 32 run all
@@ -976,7 +964,7 @@ __global__ void __launch_bounds__(512, 1) expert_turns_kernel(ExpertArgs p) {
   const int in = id - t0[3] * nb, tile = t0[3] + in % t0[4], bn = in / t0[4];
   const int* tl = p.tiles + tile * 5;
   const int nr = tl[2], n0 = bn * NB;
-  once_or_again(tl[4], [&](auto once) {
+  once_or_again(read_once(tl[4], tl[2], p.mt), [&](auto once) {
     constexpr bool ONCE = decltype(once)::value;
     if (nr > 192) expert_turns_tile<UP, 4>(p, sl, tl[0], tl[1], nr, n0);
     else if (nr > 128) expert_turns_tile<UP, 3, ONCE>(p, sl, tl[0], tl[1], nr, n0);
@@ -998,7 +986,7 @@ __global__ void __launch_bounds__(256, NARROW ? 2 : 1) expert_gemm_kernel(Expert
   if constexpr (FAR) {
     expert_gemm_tile<UP, 2, 2, 2, 2, true>(p, gl, tl[0], tl[1], nr, n0);
   } else if constexpr (NARROW) {
-    once_or_again(tl[4], [&](auto once) {
+    once_or_again(read_once(tl[4], nr, p.mt), [&](auto once) {
       constexpr bool ONCE = decltype(once)::value;
       if (nr > 128) expert_gemm_tile<UP, 2, 2, 2, 3, false, ONCE>(p, gl, tl[0], tl[1], nr, n0);
       else if (nr > 64) expert_gemm_tile<UP, 2, 2, 2, 2, false, ONCE>(p, gl, tl[0], tl[1], nr, n0);

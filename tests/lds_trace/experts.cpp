@@ -1,6 +1,8 @@
 // The expert tiles' own source for the host, every load and store with a callback (trace.cpp). Arguments: "stream", "block" or "turns", 1 for gate
-// and up, rows, stages of 64 of K.
+// and up, rows, stages of 64 of K. Or "once": which tiles' weights come non-temporal, for experts of any number of rows.
 #include <stdlib.h>
+
+#include <initializer_list>
 
 #include "../../csrc/kernels/expert_tiles.h"
 
@@ -30,7 +32,24 @@ void tile(char form, const ExpertArgs& p, int rows) {
   else rows > 16 ? go(stream<UP, 4>, 256) : rows > 8 ? go(stream<UP, 2>, 256) : go(stream<UP, 1>, 256);
 }
 
+// An expert's c rows: full tiles side by side, and the rest, among them or after all others. Weights that are read again come through the cache.
+int once() {
+  int wrong = 0, seen = 0;
+  for (int mt : {128, 192})
+    for (int c = 1; c < 1000; ++c) {
+      const int late = late_tile(c, mt), beside = (c + mt - 1) / mt - late;
+      for (int i = 0; i < beside; ++i) {
+        const bool is = read_once(beside, c - i * mt < mt ? c - i * mt : mt, mt);
+        wrong += is && (beside > 1 || late), seen += is;
+      }
+      seen += late && read_once(1, c % mt, mt);
+    }
+  printf("wrong %d\nonce %d\n", wrong, seen);
+  return 0;
+}
+
 int main(int argc, char** argv) {
+  if (argc == 2) return once();
   if (argc != 5) return 2;
   const int rows = atoi(argv[3]), N = 48;
   int* perm = (int*)calloc(rows, 4);

@@ -72,6 +72,16 @@ def test_expert_tiles(trace, kernel, rows, up):
     assert trace(kernel, up, rows, 9, LDS_TRACE_NO_BARRIERS="1")[0] > 100
 
 
+def test_weights_read_again_come_through_the_cache(tmp_path):
+    """No tile's weights come non-temporal where another tile of its expert reads them beside it or after it."""
+    src, exe = os.path.join(ROOT, "tests", "lds_trace"), str(tmp_path / "once")
+    subprocess.run([CLANG, "-x", "c++", "-std=c++17", "-w", "-mavx512f", "-O0", "-I" + src, os.path.join(src, "experts.cpp"), os.path.join(src, "trace.cpp"),
+                    "-o", exe], check=True)
+    r = subprocess.run([exe, "once"], capture_output=True, text=True)
+    got = dict(line.split() for line in r.stdout.splitlines())
+    assert r.returncode == 0 and int(got["wrong"]) == 0 and int(got["once"]) > 300
+
+
 def test_every_block_is_taken_once(tmp_path):
     """The order of the blocks is one of all blocks of all heads."""
     src, exe = os.path.join(ROOT, "tests", "lds_trace"), str(tmp_path / "order")
