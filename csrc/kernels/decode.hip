@@ -519,8 +519,7 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
   };
   // the U scores of an iteration are independent (their lane-group sums overlap), then ONE
   // online-softmax update folds them in: the dependent chain per iteration is one reduction and
-  // one rescale, not U of each. Token t0 (u = 0) of the first one is always valid, so the running max is finite;
-  // a later iteration without a valid token changes nothing.
+  // one rescale, not U of each. Token t0 (u = 0) is always valid, so the running max is finite.
   auto fold = [&](int t0, const U16x8 (&kr)[U], const U16x8 (&vr)[U]) {
     float sv[G][U];
 #pragma unroll
@@ -571,7 +570,7 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
     for (int t0 = ts; t0 < ce; t0 += 2 * TPB * U) {
       fold(t0, kx0, vx0);
       load_kv(t0 + 2 * TPB * U, kx0, vx0);
-      fold(t0 + TPB * U, kx1, vx1);
+      if (t0 + TPB * U < ce) fold(t0 + TPB * U, kx1, vx1);  // (without a token of its own it has one's infinite V times 0)
       load_kv(t0 + 3 * TPB * U, kx1, vx1);
     }
   } else {

@@ -496,6 +496,20 @@ def test_decode_one_pass_walk_edges(D, Hkv, G, PS, window):
         assert ((got.double().cpu().view(B, H, D) - want).abs() <= want.abs() * 2 ** -8 + 1e-4).all()
 
 
+@pytest.mark.parametrize("D,n", [(256, 33), (256, 97), (256, 161), (96, 65), (96, 193), (64, 129), (64, 385), (128, 193)])
+def test_decode_infinite_values(D, n):
+    """An infinite value in the last cached row stays one: no group of lanes has it times the weight 0 of a token that is not there, after an odd number
+    of whole rounds of tokens (32 at 256 dims, 64 at 96 and 128, 128 at 64)."""
+    torch.manual_seed(n)
+    kc = torch.randn(1, 2, 448, D, device=dev).to(torch.bfloat16)
+    vc = torch.randn_like(kc)
+    q = torch.randn(1, 2 * D, device=dev).to(torch.bfloat16)
+    vc[0, 1, n - 2, 5] = float("inf")
+    i32 = dict(device=dev, dtype=torch.int32)
+    o = dops.decode_attention(q, kc, vc, torch.zeros(1, **i32), torch.full((1,), n, **i32), 2, 448, chunk=448).view(2, D)
+    assert o[1, 5] == float("inf") and int(o.isfinite().sum()) == 2 * D - 1
+
+
 _FANIN_CASE = """
 import sys, torch
 from kubernetes_cloud_amd.ops import decode as dops
