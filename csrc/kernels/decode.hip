@@ -312,19 +312,22 @@ __device__ void fanin_combine(const DecodeParams& p, int b, int hk, int nsplit) 
   }
 }
 
-// Cached rows are read once a step, and a layer's are back only after all others and the weights. Non-temporal, as the weights' (standalone
-// launch, 16 heads of 256, us: 32 sequences of 700 to 917 86.5, 78.4 (5.4 TB/s); 24 of 100 to 261 23.4, 21.1; 3 of 900 22.2, 20.6; 64 of 300 to 741
-// 110, 100; 16 of 1900 114, 104)
+// Cached rows as a launch reads them (ONCE): non-temporal, as the weights', or through the caches (`launch_decode` has the lines and the times)
 typedef unsigned u32x4_once __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ U16x8 load_once(const bf16_t* p) {
   return __builtin_bit_cast(U16x8, __builtin_nontemporal_load(reinterpret_cast<const u32x4_once*>(p)));
+}
+template <bool ONCE>
+__device__ __forceinline__ U16x8 load_row(const bf16_t* p) {
+  if constexpr (ONCE) return load_once(p);
+  else return *reinterpret_cast<const U16x8*>(p);
 }
 
 // LPT lanes cooperate on one token row (8 dims per lane); TPW = 64/LPT tokens per
 // wave step; G query heads share each K/V row (GQA group).
 // (the workgroup's (split, kv-head, sequence) coordinates are arguments: decode_attn_kernel passes
 // its block index, the fused decode-layer kernel below a slice of its grid)
-template <int LPT, int G, bool PAGED, bool ONLINE, bool PF = false, int DT = 0>
+template <int LPT, int G, bool PAGED, bool ONLINE, bool PF, int DT, bool ONCE>
 __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const int split, const int hk, const int b,
                                                  const int nsplit) {
   constexpr int TPW = 64 / LPT;
@@ -509,8 +512,8 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
     for (int u = 0; u < U; ++u) o[u] = toff(min(tb + u * TPB, max(ce - 1, ca))) + dfix;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      kk[u] = load_once(kb + o[u]);
-      vv[u] = load_once(vb + o[u]);
+      kk[u] = load_row<ONCE>(kb + o[u]);
+      vv[u] = load_row<ONCE>(vb + o[u]);
     }
     if constexpr (PF) {  // hipcc moves loads that only the next round of a loop uses into that round, or behind the other set's sums
       asm volatile("" ::: "memory");
@@ -799,10 +802,10 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
   if (nsplit > 1 && p.cnt) fanin_combine<G, DT>(p, b, hk, nsplit);
 }
 
-template <int LPT, int G, bool PAGED, bool ONLINE, int DT = 0>
+template <int LPT, int G, bool PAGED, bool ONLINE, int DT, bool ONCE>
 __global__ __launch_bounds__(256) void decode_attn_kernel(DecodeParams p) {
   // G == 1 only: the prefetched rows cost GQA groups a residency step (G = 2: 119 -> 135 VGPRs)
-  decode_attn_body<LPT, G, PAGED, ONLINE, ONLINE && G == 1, DT>(p, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x);
+  decode_attn_body<LPT, G, PAGED, ONLINE, ONLINE && G == 1, DT, ONCE>(p, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x);
 }
 
 // ---------------------------------------------------------------- fused decode layer (batch 1)
@@ -825,14 +828,14 @@ struct GemvM1 {
   int N, K, act;
 };
 
-template <int LPT, int G, bool PAGED, bool ONLINE, int DT = 0>
+template <int LPT, int G, bool PAGED, bool ONLINE, int DT, bool ONCE>
 __global__ __launch_bounds__(256) void decode_attn_gemv_kernel(DecodeParams p, int nsplit, int n_attn, GemvM1 g) {
   constexpr int R = 4;
   __shared__ float part[4][R];
   const int bid = blockIdx.x;
   if (bid < n_attn) {
     const int split = bid % nsplit, rest = bid / nsplit;
-    decode_attn_body<LPT, G, PAGED, ONLINE, false, DT>(p, split, rest % p.Hkv, rest / p.Hkv, nsplit);
+    decode_attn_body<LPT, G, PAGED, ONLINE, false, DT, ONCE>(p, split, rest % p.Hkv, rest / p.Hkv, nsplit);
     DSTAMP(7);
     return;
   }
@@ -963,18 +966,31 @@ KCA_API long long kca_decode_ws_floats(int B, int H, int D, int max_kv, int chun
   return ns > 1 ? fanin_words(B, H) + (long long)B * H * ns * (D + 2) : 0;
 }
 
+// How the one-pass kernel reads the cache. A layer's rows are back only after all other layers' and the weights: non-temporal (16 heads of 256,
+// cold, us, ordinary and so: 32 sequences of 700 to 917 86.5, 78.4 (5.4 TB/s); 24 of 100 to 261 23.4, 21.1; 64 of 300 to 741 110, 100; 16 of 1900
+// 114, 104; 2 and 4 query heads a key head, 8 key heads of 256, 64 of 500 66.3, 58.6; 79, 75). Not with 8 query heads, bound by their products, whose
+// loop in fp16 hipcc then orders worse (8 key heads of 256: 16 of 150 37.5, 48; 32 of 1500 209, 264; in bf16 38.0, 37.7; 312, 311); nor with 2 or 4 and a
+// cache that the last cache holds from step to step, as the weights are read past it (2 of 130 14.0, 15.2; 21.1, 21.9; 16 of 150, 20 MB, 16.3, 15.8; 22.9,
+// 22.4; with one query head 8.9, 8.8).
 template <int LPT, int G, int DT = 0>
 static void launch_decode(const DecodeParams& p, int B, int nsplit, hipStream_t stream) {
   constexpr int TPB = 4 * (64 / LPT), U = 4;
   const dim3 grid(nsplit, p.Hkv, B);
   if (p.chunk > TPB * U) {  // long splits: one pass with online softmax
     const size_t lds = (size_t)4 * G * (2 + p.D) * sizeof(float);
-    if (p.tbl) hipLaunchKernelGGL((decode_attn_kernel<LPT, G, true, true, DT>), grid, dim3(256), lds, stream, p);
-    else hipLaunchKernelGGL((decode_attn_kernel<LPT, G, false, true, DT>), grid, dim3(256), lds, stream, p);
+    const bool once = G == 1 || (G < 8 && (long long)B * p.Hkv * nsplit * p.chunk * p.D * 4 > 4 << 20);
+    constexpr bool MAY = G < 8, MUST = G == 1;
+    if (p.tbl) {
+      if (once) hipLaunchKernelGGL((decode_attn_kernel<LPT, G, true, true, DT, MAY>), grid, dim3(256), lds, stream, p);
+      else hipLaunchKernelGGL((decode_attn_kernel<LPT, G, true, true, DT, MUST>), grid, dim3(256), lds, stream, p);
+    } else {
+      if (once) hipLaunchKernelGGL((decode_attn_kernel<LPT, G, false, true, DT, MAY>), grid, dim3(256), lds, stream, p);
+      else hipLaunchKernelGGL((decode_attn_kernel<LPT, G, false, true, DT, MUST>), grid, dim3(256), lds, stream, p);
+    }
   } else {
     const size_t lds = (size_t)(G * p.chunk + 4 * G * p.D) * sizeof(float);
-    if (p.tbl) hipLaunchKernelGGL((decode_attn_kernel<LPT, G, true, false, DT>), grid, dim3(256), lds, stream, p);
-    else hipLaunchKernelGGL((decode_attn_kernel<LPT, G, false, false, DT>), grid, dim3(256), lds, stream, p);
+    if (p.tbl) hipLaunchKernelGGL((decode_attn_kernel<LPT, G, true, false, DT, false>), grid, dim3(256), lds, stream, p);
+    else hipLaunchKernelGGL((decode_attn_kernel<LPT, G, false, false, DT, false>), grid, dim3(256), lds, stream, p);
   }
 }
 
@@ -1127,21 +1143,28 @@ static int prep_attn_gemv(const void* qkv, long long ld, const void* kc, const v
   const GemvM1 g{(const bf16_t*)gx, (const bf16_t*)gw, (const bf16_t*)gbias, (bf16_t*)gy, gN, gK, gact};
   const int n_attn = nsplit * Hkv * B;
   const dim3 grid(n_attn + (gN + 3) / 4);
-  auto go = [&](auto lpt) {
+  // Ordinary loads of a cache of 2 MB at most: the other weights are read past the last cache, which holds it from step to step, and the fc_in of so
+  // narrow a model does not hide a walk's round trips. Steps of 2048-wide GPT-J layers, us, ordinary and non-temporal, by the bound on a layer's bytes: 2 MB
+  // (100 tokens) 4 layers 182.5, 188.5, 16 565, 578, (250) 4 193.5, 205; 4 MB (300) 194, 197; 617, 609; 8 MB (900) 211, 207; of 4096-wide ones 4 MB (100) 364, 362.5; 8 MB
+  // (500) 376.5, 370.
+  const bool once = (long long)B * Hkv * max_kv * D * 4 > 2 << 20;
+  auto go = [&](auto lpt, auto kind) {
     constexpr int LPT = decltype(lpt)::value;
+    constexpr bool ONCE = decltype(kind)::value;
     constexpr int TPB = 4 * (64 / LPT), U = 4;
     if (p.chunk > TPB * U) {
       const size_t lds = (size_t)4 * (2 + p.D) * sizeof(float);
-      if (p.tbl) hipLaunchKernelGGL((decode_attn_gemv_kernel<LPT, 1, true, true, DT>), grid, dim3(256), lds, stream, p, nsplit, n_attn, g);
-      else hipLaunchKernelGGL((decode_attn_gemv_kernel<LPT, 1, false, true, DT>), grid, dim3(256), lds, stream, p, nsplit, n_attn, g);
+      if (p.tbl) hipLaunchKernelGGL((decode_attn_gemv_kernel<LPT, 1, true, true, DT, ONCE>), grid, dim3(256), lds, stream, p, nsplit, n_attn, g);
+      else hipLaunchKernelGGL((decode_attn_gemv_kernel<LPT, 1, false, true, DT, ONCE>), grid, dim3(256), lds, stream, p, nsplit, n_attn, g);
     } else {
       const size_t lds = (size_t)(p.chunk + 4 * p.D) * sizeof(float);
-      if (p.tbl) hipLaunchKernelGGL((decode_attn_gemv_kernel<LPT, 1, true, false, DT>), grid, dim3(256), lds, stream, p, nsplit, n_attn, g);
-      else hipLaunchKernelGGL((decode_attn_gemv_kernel<LPT, 1, false, false, DT>), grid, dim3(256), lds, stream, p, nsplit, n_attn, g);
+      if (p.tbl) hipLaunchKernelGGL((decode_attn_gemv_kernel<LPT, 1, true, false, DT, false>), grid, dim3(256), lds, stream, p, nsplit, n_attn, g);
+      else hipLaunchKernelGGL((decode_attn_gemv_kernel<LPT, 1, false, false, DT, false>), grid, dim3(256), lds, stream, p, nsplit, n_attn, g);
     }
   };
-  if (nd <= 16) go(std::integral_constant<int, 16>{});
-  else go(std::integral_constant<int, 32>{});
+  auto go_as = [&](auto lpt) { once ? go(lpt, std::true_type{}) : go(lpt, std::false_type{}); };
+  if (nd <= 16) go_as(std::integral_constant<int, 16>{});
+  else go_as(std::integral_constant<int, 32>{});
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 

@@ -510,6 +510,50 @@ def test_decode_infinite_values(D, n):
     assert o[1, 5] == float("inf") and int(o.isfinite().sum()) == 2 * D - 1
 
 
+def _attention_loads(f):
+    """f()'s decode attention launch: whether it read the cache non-temporal."""
+    f()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        f()
+        torch.cuda.synchronize()
+    names = [e.key for e in prof.key_averages() if "decode_attn_" in e.key]
+    assert len(names) == 1 and names[0].split("(")[0].endswith((", true>", ", false>")), names
+    return ", true>" in names[0].split("(")[0][-7:]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("G,L,once", [(1, 448, True), (2, 448, False), (4, 512, False), (2, 768, True), (4, 768, True), (8, 768, False)])
+def test_decode_loads_by_group(dtype, G, L, once):
+    """Many queries a key head, and a few with a cache of 4 MB or less, read it with ordinary loads; the rows are those of the plain form."""
+    torch.manual_seed(G)
+    B, Hkv, D = 3, 2, 256
+    kc = torch.randn(B, Hkv, L, D, device=dev).to(dtype)
+    vc = torch.randn_like(kc)
+    qkv = torch.randn(B, (Hkv * G + 2 * Hkv) * D, device=dev).to(dtype)
+    i32 = dict(device=dev, dtype=torch.int32)
+    slots, kl = torch.arange(B, **i32), torch.tensor([1, 130, 448], **i32)
+    o = torch.empty(B, Hkv * G * D, device=dev, dtype=dtype)
+    assert once == _attention_loads(lambda: dops.decode_prep_attention(qkv, Hkv * G, Hkv, D, 0, False, None, None, kl - 1, slots, kc, vc, kl, L, out=o))
+    want = dops.decode_attention_reference(qkv.float(), kc.float(), vc.float(), slots, kl, Hkv * G, D ** -0.5)  # (the rows that it appended)
+    assert (o.float() - want).abs().max() < 2 ** -8 * 4
+
+
+@pytest.mark.parametrize("max_kv,once", [(256, False), (512, True)])
+def test_decode_loads_by_size(max_kv, once):
+    """A batch-1 step's launch of 2 MB of cache and less reads it with ordinary loads."""
+    H, D, i32 = 8, 256, dict(device=dev, dtype=torch.int32)
+    kc = torch.randn(2, H, max_kv, D, device=dev).to(torch.bfloat16)
+    vc = torch.randn_like(kc)
+    qkv = torch.randn(1, 3 * H * D, device=dev).to(torch.bfloat16)
+    gx, gw = torch.randn(1, H * D, device=dev).to(torch.bfloat16), torch.randn(512, H * D, device=dev).to(torch.bfloat16)
+    kl, slots, out, gy = torch.tensor([200], **i32), torch.zeros(1, **i32), torch.empty(1, H * D, device=dev, dtype=torch.bfloat16), gx.new_empty(1, 512)
+    ws = torch.zeros(dops.decode_ws_floats(1, H, H, D, max_kv) + 1, device=dev)
+    assert once == _attention_loads(lambda: dops.decode_prep_attention_gemv(qkv, H, H, D, 0, False, None, None, kl - 1, slots, kc, vc, kl, max_kv, D ** -0.5,
+                                                                            None, out, ws, None, 0, gx, gw, None, gy, 0))
+    want = dops.decode_prep_attention(qkv, H, H, D, 0, False, None, None, kl - 1, slots, kc, vc, kl, max_kv)
+    assert torch.equal(out, want)
+
+
 _FANIN_CASE = """
 import sys, torch
 from kubernetes_cloud_amd.ops import decode as dops
