@@ -150,6 +150,7 @@ struct DecodeParams {
   // per-step descriptors uploaded with the step's inputs (fused batch-1 decode): bit 0 -- cos_t /
   // sin_t hold row b's RoPE angles at index b (not the position table); bit 1 -- tbl holds row b's
   // page ids at row b (not the slot's). Neither then waits for the length or the slot to arrive.
+  // bit 2 -- sequences share pages (beams, their prefix): launch_decode
   int by_row;
 };
 
@@ -971,7 +972,9 @@ KCA_API long long kca_decode_ws_floats(int B, int H, int D, int max_kv, int chun
 // 114, 104; 2 and 4 query heads a key head, 8 key heads of 256, 64 of 500 66.3, 58.6; 79, 75). Not with 8 query heads, bound by their products, whose
 // loop in fp16 hipcc then orders worse (8 key heads of 256: 16 of 150 37.5, 48; 32 of 1500 209, 264; in bf16 38.0, 37.7; 312, 311); nor with 2 or 4 and a
 // cache that the last cache holds from step to step, as the weights are read past it (2 of 130 14.0, 15.2; 21.1, 21.9; 16 of 150, 20 MB, 16.3, 15.8; 22.9,
-// 22.4; with one query head 8.9, 8.8).
+// 22.4; with one query head 8.9, 8.8); nor up to 128 dims where sequences share pages (DecodeParams::by_row), which one of them then reads for the others
+// (beams over a prefix, non-temporal and so: 14 heads of 128, 8 beams over 1920 28.0, 22.5, 32 over 512 20.1, 17.0; 64 of 96 52, 42; 51.5, 44.2; 12 of 64 17.4,
+// 16.9; 12.7, 12.4; 16 of 256 30.9, 31.8; 26.3, 26.9).
 template <int LPT, int G, int DT = 0>
 static void launch_decode(const DecodeParams& p, int B, int nsplit, hipStream_t stream) {
   constexpr int TPB = 4 * (64 / LPT), U = 4;
@@ -979,10 +982,11 @@ static void launch_decode(const DecodeParams& p, int B, int nsplit, hipStream_t 
   if (p.chunk > TPB * U) {  // long splits: one pass with online softmax
     const size_t lds = (size_t)4 * G * (2 + p.D) * sizeof(float);
     const bool once = G == 1 || (G < 8 && (long long)B * p.Hkv * nsplit * p.chunk * p.D * 4 > 4 << 20);
-    constexpr bool MAY = G < 8, MUST = G == 1;
+    constexpr bool MAY = G < 8, MUST = G == 1, MUST_PAGED = MUST && LPT == 32;
     if (p.tbl) {
-      if (once) hipLaunchKernelGGL((decode_attn_kernel<LPT, G, true, true, DT, MAY>), grid, dim3(256), lds, stream, p);
-      else hipLaunchKernelGGL((decode_attn_kernel<LPT, G, true, true, DT, MUST>), grid, dim3(256), lds, stream, p);
+      if (once && (LPT == 32 || !(p.by_row & 4)))
+        hipLaunchKernelGGL((decode_attn_kernel<LPT, G, true, true, DT, MAY>), grid, dim3(256), lds, stream, p);
+      else hipLaunchKernelGGL((decode_attn_kernel<LPT, G, true, true, DT, MUST_PAGED>), grid, dim3(256), lds, stream, p);
     } else {
       if (once) hipLaunchKernelGGL((decode_attn_kernel<LPT, G, false, true, DT, MAY>), grid, dim3(256), lds, stream, p);
       else hipLaunchKernelGGL((decode_attn_kernel<LPT, G, false, true, DT, MUST>), grid, dim3(256), lds, stream, p);

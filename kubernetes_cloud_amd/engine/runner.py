@@ -189,6 +189,10 @@ class KVCache:
     def table_on(self, dev):
         return self.tables.get(torch.device(dev)) if self.paged else None
 
+    def shares(self, slots: list[int]) -> bool:
+        """Whether some of these sequences may read the same pages: a fork shares a prefix, its first page among it."""
+        return self.paged and len(slots) > 1 and any(self.pages[s] and self.ref[self.pages[s][0]] > 1 for s in slots)
+
     def _per_layer(self, idx: list[int]):
         """``idx`` as a long tensor on every cache device."""
         t = torch.tensor(idx, dtype=torch.long)
@@ -378,6 +382,7 @@ class StepRunner:
     mixed_steps = False    # forward_tokens: prompt portions and decoded tokens in one batch
     multi_device = False
     _embed_head = False    # the step head resolves chained tokens on the device
+    _rows_share = False    # an eager step of beams whose prefix lies in the same pages
 
     def __init__(self, model, max_slots: int, max_len: int | None, use_graphs: bool | None, max_bans: int):
         self.model = model.eval()
@@ -501,7 +506,11 @@ class StepRunner:
         sl = torch.tensor(slots, device=dev, dtype=torch.int32)
         kl = pos + 1
         max_kv = max(positions) + 1
-        logits = self._eager_logits(tok, pos, sl, kl, max_kv)
+        self._rows_share = self.cache.shares(slots)
+        try:
+            logits = self._eager_logits(tok, pos, sl, kl, max_kv)
+        finally:
+            self._rows_share = False
         lp = torch.log_softmax(logits.float(), dim=-1)
         return lp.topk(k, dim=-1)
 
@@ -1296,7 +1305,7 @@ class ModelRunner(StepRunner):
             # only the last `window` positions)
             o = dops.decode_prep_attention(qkv, self.H, self.Hkv, self.D, self.rot, cfg.rotary_interleaved,
                                            cos, sin, pos, slots, kc, vc, kv_lens, max_kv, at.scale, at.alibi,
-                                           out=obuf, ws=ws, block_table=tbl, window=at.window, by_row=by_row)
+                                           out=obuf, ws=ws, block_table=tbl, window=at.window, by_row=by_row, shared=self._rows_share)
             a = self._lin(at.out, o)
             if side_out is not None:  # join
                 cur.wait_stream(self._side)

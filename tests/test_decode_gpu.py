@@ -538,6 +538,24 @@ def test_decode_loads_by_group(dtype, G, L, once):
     assert (o.float() - want).abs().max() < 2 ** -8 * 4
 
 
+@pytest.mark.parametrize("D,once", [(64, False), (96, False), (128, False), (160, True), (256, True)])
+def test_decode_loads_of_shared_pages(D, once):
+    """Beams of up to 128 dims read their common prefix through the caches; the bits are the same."""
+    H, PS, i32 = 24, 32, dict(device=dev, dtype=torch.int32)
+    torch.manual_seed(D)
+    kc = torch.randn(60, H, PS, D, device=dev).to(torch.bfloat16)
+    vc = torch.randn_like(kc)
+    tbl = torch.cat([torch.arange(30).expand(3, 30), 30 + torch.arange(6).view(3, 2)], 1).to(**i32)
+    qkv = torch.randn(3, 3 * H * D, device=dev).to(torch.bfloat16)
+    slots, kl = torch.arange(3, **i32), torch.tensor([970, 961, 1024], **i32)
+    out = torch.empty(2, 3, H * D, device=dev, dtype=torch.bfloat16)
+    for i, shared in enumerate((False, True)):
+        got = _attention_loads(lambda: dops.decode_prep_attention(qkv, H, H, D, 0, False, None, None, kl - 1, slots, kc, vc, kl, 1024, out=out[i],
+                                                                  block_table=tbl, shared=shared))
+        assert got == (once or not shared)
+    assert torch.equal(out[0], out[1])
+
+
 @pytest.mark.parametrize("max_kv,once", [(256, False), (512, True)])
 def test_decode_loads_by_size(max_kv, once):
     """A batch-1 step's launch of 2 MB of cache and less reads it with ordinary loads."""

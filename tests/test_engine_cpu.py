@@ -212,6 +212,22 @@ def test_fork_shares_full_pages_and_copies_tail():
     assert c.free_count() == c.n_pages and all(x == 0 for x in c.ref)
 
 
+@pytest.mark.parametrize("page_size,shared", [(16, True), (64, False), (0, False)])
+def test_beams_say_that_they_share_pages(monkeypatch, page_size, shared):
+    """A prompt of 17 tokens: a whole page of 16 is the beams' own together, of 64 none, and a decode step of unrelated sequences shares nothing."""
+    seen, f = [], dops.decode_prep_attention
+    monkeypatch.setattr(dops, "decode_prep_attention", lambda *a, **k: (seen.append((a[0].shape[0], k.get("shared", False))), f(*a, **k))[1])
+    eng = LLMEngine(tiny("gpt-j-6b"), max_slots=4, max_len=64, page_size=page_size)
+    prompt = [3, 1, 4, 1, 5, 9, 2, 6, 5, 3, 5, 8, 9, 7, 9, 3, 2]
+    eng.generate([prompt, prompt[::-1]], SamplingParams(max_new_tokens=3, do_sample=False))
+    assert seen and not any(s for _, s in seen)
+    seen.clear()
+    eng.beam_generate(prompt, 3, 4)
+    assert seen == [(3, shared)] * len(seen) and seen
+    eng.beam_generate(prompt, 1, 4)
+    assert seen[-1] == (1, False)
+
+
 def test_paged_decode_ops_reference_match_contiguous():
     torch.manual_seed(0)
     H, Hkv, D, PS, L = 4, 2, 8, 16, 64
