@@ -20,6 +20,7 @@ struct RowsArgs {
   // p[0], and beside it p[1] with blocks of its own (beside), or p[1]'s x and W along K: y[0] = x0 W0^T + x1 W1^T + both biases
   // (p[1].K without beside). p[1].K == 0: one product.
   RowsPart p[2];
+  const void* res;  // two products along K: rows [M, N] that are added to their sums, or null
   float* ws;      // ks > 1: [block][slice][product tile][2][threads][2]
   unsigned* cnt;  // ks > 1: one arrival counter a block, zero before and after
   int M, ks, beside;
@@ -185,8 +186,8 @@ __global__ void __launch_bounds__(64 * W, 2) rows_mm_kernel(RowsArgs p) {
         for (int i = 0; i < A; ++i) acc[i][j] = mma<F16>(wf[s][i], xf[s][j], acc[i][j]);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the repeated stages, before the LDS is given back
+  unsigned long long* const part = reinterpret_cast<unsigned long long*>(p.ws) + (long long)blk * p.ks * A * B * (128 * W) + threadIdx.x;
   if (p.ks > 1) {
-    unsigned long long* part = reinterpret_cast<unsigned long long*>(p.ws) + (long long)blk * p.ks * A * B * (128 * W) + threadIdx.x;
 #pragma unroll
     for (int i = 0; i < A; ++i)
 #pragma unroll
@@ -209,6 +210,18 @@ __global__ void __launch_bounds__(64 * W, 2) rows_mm_kernel(RowsArgs p) {
     }
     __syncthreads();
     if (!*(volatile int*)sl) return;
+  }
+  uint2 res[A][B];  // requested before the other slices' sums
+  if (TWO && p.res) {
+#pragma unroll
+    for (int i = 0; i < A; ++i)
+#pragma unroll
+      for (int j = 0; j < B; ++j) {
+        const int n = min(n0 + (wn * A + i) * 16 + 4 * g, q.N - 4), m = min((wm * B + j) * 16 + r16, p.M - 1);
+        res[i][j] = *reinterpret_cast<const uint2*>(reinterpret_cast<const unsigned short*>(p.res) + (long long)m * q.N + n);
+      }
+  }
+  if (p.ks > 1) {
     // all slices in slice order, whichever came last: the sum does not depend on the order of arrival
     f32x4 sum[A][B];
 #pragma unroll
@@ -254,6 +267,13 @@ __global__ void __launch_bounds__(64 * W, 2) rows_mm_kernel(RowsArgs p) {
       for (int e = 0; e < 4; ++e) {
         o[e] = acc[i][j][e] + b[e];
         if (q.act) o[e] = q.act == 1 ? gelu_tanh(o[e]) : gelu_erf(o[e]);
+      }
+      if (TWO && p.res) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const unsigned short v = (e < 2 ? res[i][j].x : res[i][j].y) >> 16 * (e & 1);
+          o[e] += F16 ? (float)__builtin_bit_cast(_Float16, v) : bf2f(v);
+        }
       }
       uint2 v;
       if constexpr (F16) {
@@ -339,16 +359,17 @@ int rows_mm(int dtype, const RowsArgs& a, long long ws_floats, int cnt_n, hipStr
 // blocks = ceil(N / 64). Other sizes return a status and launch nothing.
 KCA_API int kca_rows_mm(int dtype, const void* x, const void* w, const void* bias, void* y, float* ws, unsigned* cnt,
                         long long ws_floats, int cnt_n, int M, int N, int K, int ks, hipStream_t s) {
-  return rows_mm(dtype, RowsArgs{{{x, w, bias, y, N, K, 0}, {}}, ws, cnt, M, ks, 0}, ws_floats, cnt_n, s);
+  return rows_mm(dtype, RowsArgs{{{x, w, bias, y, N, K, 0}, {}}, nullptr, ws, cnt, M, ks, 0}, ws_floats, cnt_n, s);
 }
 
 // One product with a GELU (act: 0 none, 1 tanh, 2 erf) on its fp32 sums (x2 null), or two: beside each other, y2 [M, N2] =
 // act2(x2 W2^T + bias2) in blocks of its own, or (beside 0) along K: y = act(x W^T + x2 W2^T + bias + bias2), N2 == N. Blocks: both
-// products' where they lie beside each other.
+// products' where they lie beside each other. res (along K, no act): rows [M, N] of y's type, 8-byte aligned, added to the fp32 sums; or null.
 KCA_API int kca_rows_mm_two(int dtype, int beside, const void* x, const void* w, const void* bias, void* y, int N, int K, int act,
-                            const void* x2, const void* w2, const void* bias2, void* y2, int N2, int K2, int act2, float* ws,
-                            unsigned* cnt, long long ws_floats, int cnt_n, int M, int ks, hipStream_t s) {
-  if (x2 && K2 < SK) return 1;
-  return rows_mm(dtype, RowsArgs{{{x, w, bias, y, N, K, act}, {x2, w2, bias2, y2, N2, x2 ? K2 : 0, act2}}, ws, cnt, M, ks, x2 && beside},
+                            const void* x2, const void* w2, const void* bias2, void* y2, int N2, int K2, int act2,
+                            const void* res, float* ws, unsigned* cnt, long long ws_floats, int cnt_n, int M, int ks, hipStream_t s) {
+  if ((x2 && K2 < SK) || (res && (!x2 || beside || act))) return 1;
+  if ((uintptr_t)res % 8) return 2;
+  return rows_mm(dtype, RowsArgs{{{x, w, bias, y, N, K, act}, {x2, w2, bias2, y2, N2, x2 ? K2 : 0, act2}}, res, ws, cnt, M, ks, x2 && beside},
                  ws_floats, cnt_n, s);
 }

@@ -27,7 +27,7 @@ typedef long long ll;
 
 // of the kernel library that ops/_lib.py has loaded
 typedef int (*RowsFn)(int, int, const void*, const void*, const void*, void*, int, int, int, const void*, const void*, const void*, void*,
-                      int, int, int, float*, unsigned*, ll, int, int, int, hipStream_t);
+                      int, int, int, const void*, float*, unsigned*, ll, int, int, int, hipStream_t);
 typedef int (*NormFn)(const void*, const void*, const void*, void*, const void*, const void*, void*, float*, float*, int, int, float,
                       hipStream_t);
 typedef int (*NormF16Fn)(const void*, ll, const void*, const void*, void*, ll, const void*, const void*, float, void*, int, int,
@@ -67,17 +67,19 @@ bool bias_fits(PyObject* o, int64_t n, const Tensor& x, int64_t device) {
 
 }  // namespace
 
-// few_rows(x, weight, bias | None, x2 | None, weight2, bias2 | None, act, act2, beside, rows) -> (y,) or (y, y2), or None. The caller has
-// asked few_rows (ops/linear.py) about the sizes.
+// few_rows(x, weight, bias | None, x2 | None, weight2, bias2 | None, act, act2, beside, rows[, res | None]) -> (y,) or (y, y2), or None. The
+// caller has asked few_rows (ops/linear.py) about the sizes.
 PyObject* kca_few_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 10 || !rows_mm) {
-    PyErr_SetString(PyExc_TypeError, "few_rows(x, weight, bias, x2, weight2, bias2, act, act2, beside, rows) after init_rows");
+  if ((n != 10 && n != 11) || !rows_mm) {
+    PyErr_SetString(PyExc_TypeError, "few_rows(x, weight, bias, x2, weight2, bias2, act, act2, beside, rows, res) after init_rows");
     return nullptr;
   }
   const int parts = a[3] == Py_None ? 1 : 2;
+  PyObject* const res = n > 10 ? a[10] : Py_None;
   for (int i = 0; i < parts; ++i)
     if (!is_tensor(a[3 * i]) || !is_tensor(a[3 * i + 1]) || !is_tensor_or_none(a[3 * i + 2])) Py_RETURN_NONE;
+  if (!is_tensor_or_none(res)) Py_RETURN_NONE;
   const long act = PyLong_AsLong(a[6]), act2 = PyLong_AsLong(a[7]), rows = PyLong_AsLong(a[9]);
   const int beside = PyObject_IsTrue(a[8]);
   if (PyErr_Occurred()) return nullptr;
@@ -100,6 +102,12 @@ PyObject* kca_few_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t N = w.size(0), K = w.size(1), N2 = w2.size(0), K2 = w2.size(1);
   const bool two = parts > 1, apart = two && beside;
   if (two && !beside && N != N2) Py_RETURN_NONE;
+  if (res != Py_None) {
+    const Tensor& r = THPVariable_Unpack(res);
+    if (!two || beside || !on(r, device) || r.scalar_type() != x0.scalar_type() || r.numel() != rows * N || !r.is_contiguous() ||
+        reinterpret_cast<uintptr_t>(r.const_data_ptr()) % 8)
+      Py_RETURN_NONE;
+  }
   // (as _few_launch: about one block of 64 weight rows a CU)
   const int64_t blocks = (N + 63) / 64 + (apart ? (N2 + 63) / 64 : 0), k = apart ? std::min(K, K2) : two ? K + K2 : K;
   const int64_t ks = std::max<int64_t>(1, std::min(256 / blocks, k / 512));
@@ -114,7 +122,7 @@ PyObject* kca_few_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int rc = rows_mm(x0.scalar_type() == at::kBFloat16 ? 1 : 2, apart, x0.const_data_ptr(), w.const_data_ptr(), at_or_null(a[2]),
                          y.mutable_data_ptr(), N, K, act, two ? at_or_null(a[3]) : nullptr, two ? w2.const_data_ptr() : nullptr,
                          two ? at_or_null(a[5]) : nullptr, apart ? y2.mutable_data_ptr() : nullptr, two ? N2 : 0, two ? K2 : 0,
-                         two ? act2 : 0, ks > 1 ? ws.mutable_data_ptr<float>() : nullptr,
+                         two ? act2 : 0, at_or_null(res), ks > 1 ? ws.mutable_data_ptr<float>() : nullptr,
                          ks > 1 ? reinterpret_cast<unsigned*>(cnt.mutable_data_ptr<int>()) : nullptr, ks > 1 ? ws.numel() : 0,
                          ks > 1 ? cnt.numel() : 0, rows, ks, stream_of(device));
   TORCH_CHECK(rc == 0, "kca_rows_mm_two returned status ", rc, " (unsupported shape/arguments)");

@@ -130,7 +130,7 @@ _SIGS.update({
     "kca_moe_expert": [I, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P, P, P, I, I, I, I, P],
     "kca_rows_mm": [I, P, P, P, P, P, P, LL, I, I, I, I, I, P],
     "kca_layernorm_rows_fwd": [P] * 7 + [I, I, F, P],
-    "kca_rows_mm_two": [I, I] + [P, P, P, P, I, I, I] * 2 + [P, P, LL, I, I, I, P],
+    "kca_rows_mm_two": [I, I] + [P, P, P, P, I, I, I] * 2 + [P, P, P, LL, I, I, I, P],
     "kca_act_rows": [I, I, P, LL, P, P, P, LL, I, I, F, P],
     "kca_norm_residual": [I, P, P, P, P, LL, P, P, P, P, F, P, P, P, I, I, I, P],
 })

@@ -277,19 +277,21 @@ def few_rows_scratch(rows: int, device: torch.device) -> tuple[torch.Tensor, tor
             torch.zeros(_CUS, device=device, dtype=torch.int32))
 
 
-def _few_launch(parts, act: int, act2: int, beside: bool, rows: int, scratch=None):
+def _few_launch(parts, act: int, act2: int, beside: bool, rows: int, scratch=None, res=None):
     """One launch of ``kca_rows_mm_two`` over one or two (x, weight, bias); None: sizes, types or a mode of torch (gradients,
     transforms, captures without ``few_rows_scratch``, ...) that it does not serve."""
     x = parts[0][0]
     ext = _lib.plain_ext() if scratch is None and x.is_cuda else None
     if ext is not None and 0 < rows <= FEW_ROWS and all(few_rows(rows, *p[1].shape) for p in parts):
-        y = ext.few_rows(*parts[0], *(parts[1] if len(parts) > 1 else (None, None, None)), act, act2, beside, rows)
+        y = ext.few_rows(*parts[0], *(parts[1] if len(parts) > 1 else (None, None, None)), act, act2, beside, rows, res)
         if y is not None:
             _lib.LAUNCHES[0] += 1
             return y
     if (not 0 < rows <= FEW_ROWS or not x.is_cuda or (scratch is None and torch.cuda.is_current_stream_capturing())
             or not all(p[0].dtype == x.dtype and _few_part(*p, rows) for p in parts)
-            or not _lib.inference(*(t for p in parts for t in p)) or not _lib.has("kca_rows_mm_two")):
+            or (res is not None and (res.dtype != x.dtype or res.numel() != rows * parts[0][1].shape[0] or not res.is_contiguous()
+                                     or res.data_ptr() % 8))
+            or not _lib.inference(*(t for p in parts for t in p), res) or not _lib.has("kca_rows_mm_two")):
         return None
     outs = [torch.empty(rows, p[1].shape[0], device=x.device, dtype=x.dtype) for p in (parts if beside else parts[:1])]
     blocks = sum(-(-y.shape[1] // 64) for y in outs)
@@ -307,7 +309,7 @@ def _few_launch(parts, act: int, act2: int, beside: bool, rows: int, scratch=Non
             a += [px.data_ptr(), w.data_ptr(), _lib.ptr(b), outs[i].data_ptr() if i < len(outs) else None, *w.shape, (act, act2)[i]]
         else:
             a += [None, None, None, None, 0, 0, 0]
-    _lib.call("kca_rows_mm_two", 1 if x.dtype == torch.bfloat16 else 2, int(beside), *a, _lib.ptr(ws), _lib.ptr(cnt),
+    _lib.call("kca_rows_mm_two", 1 if x.dtype == torch.bfloat16 else 2, int(beside), *a, _lib.ptr(res), _lib.ptr(ws), _lib.ptr(cnt),
               0 if ws is None else ws.numel(), 0 if cnt is None else cnt.numel(), rows, ks, _lib.stream())
     return outs
 
@@ -330,15 +332,15 @@ def few_rows_beside(first: tuple, second: tuple, approx2: str | None = None, scr
     return None if y is None else tuple(t.view(*x.shape[:-1], -1) for t in y)
 
 
-def few_rows_sum(first: tuple, second: tuple, scratch=None) -> torch.Tensor | None:
-    """The sum of two products (x, weight, bias) of the same few rows in one launch, rounded once; or None. On the GPU, us, apart and
+def few_rows_sum(first: tuple, second: tuple, scratch=None, res: torch.Tensor | None = None) -> torch.Tensor | None:
+    """The sum of two products (x, weight, bias) of the same few rows, and of rows ``res``, in one launch, rounded once; or None. On the GPU, us, apart and
     together, 61 rows: 4096 x 16384 and x 4096 29.3 + 12.5, 35.3; 2048 x 8192 and x 2048 13.2 + 8.8, 15.2;
     128 rows 41.4 + 16.6, 49.9."""
     x = first[0]
     rows = x.numel() // x.shape[-1]
     if first[1].shape[0] != second[1].shape[0]:
         return None
-    y = _few_launch([first, second], 0, 0, False, rows, scratch)
+    y = _few_launch([first, second], 0, 0, False, rows, scratch, res)
     return None if y is None else y[0].view(*x.shape[:-1], -1)
 
 

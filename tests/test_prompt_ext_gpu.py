@@ -47,6 +47,8 @@ def test_few_rows(monkeypatch, dtype, rows, n, k, n2, k2):
     _both(monkeypatch, lambda: L.few_rows_beside(a, b, "tanh"), "few_rows")
     _both(monkeypatch, lambda: L.few_rows_gelu(*a, "none"), "few_rows")
     _both(monkeypatch, lambda: L.few_rows_sum(a, b), "few_rows" if n == n2 else None)
+    res = _rand(rows, n, dtype=dtype)
+    _both(monkeypatch, lambda: L.few_rows_sum(a, b, res=res), "few_rows" if n == n2 else None)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

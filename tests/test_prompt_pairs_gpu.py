@@ -55,6 +55,34 @@ def test_sum(dtype, rows, n, k, k2):
             assert _close(L.few_rows_sum(a, b), _ref(*a) + _ref(*b), 2)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [1, 17, 32, 33, 64, 65, 128])
+@pytest.mark.parametrize("n,k,k2", [(16, 64, 64), (80, 64, 1984), (2048, 64, 2112), (4096, 4096, 1024), (16400, 128, 64)])
+@pytest.mark.parametrize("captured", [False, True])
+def test_sum_and_residual_rows(dtype, rows, n, k, k2, captured):
+    """The residual rows enter the 32-bit sums: one rounding, where the rounded sum of the products was added to them and rounded again."""
+    if not L.few_rows(rows, n, k) or not L.few_rows(rows, n, k2):
+        pytest.skip("the library's")
+    a, b = _part(rows, n, k, dtype, True, 1), _part(rows, n, k2, dtype, n % 32 == 0, 2)
+    res = torch.empty(1, rows, n, device="cuda", dtype=dtype).normal_(std=30, generator=torch.Generator(device="cuda").manual_seed(3))
+    sc = L.few_rows_scratch(rows, torch.device("cuda", 0)) if captured else None  # (with a scratch: the launch from Python)
+    with torch.no_grad():
+        for _ in range(2):
+            y = L.few_rows_sum(a, b, sc, res)
+            assert _close(y, _ref(*a) + _ref(*b) + res[0].double(), 3)
+
+
+def test_residual_rows_they_leave():
+    a, b = _part(8, 96, 128, torch.bfloat16, True, 1), _part(8, 96, 192, torch.bfloat16, True, 2)
+    r = torch.ones(8, 96, device="cuda", dtype=torch.bfloat16)
+    for sc in (None, L.few_rows_scratch(8, torch.device("cuda", 0))):
+        with torch.no_grad():
+            for bad in (r.float(), r.half(), r[:7], torch.ones(8, 192, device="cuda", dtype=torch.bfloat16)[:, ::2], r.cpu(),
+                        torch.ones(769, device="cuda", dtype=torch.bfloat16)[1:].view(8, 96)):
+                assert L.few_rows_sum(a, b, sc, bad) is None
+            assert L.few_rows_sum(a, b, sc, r) is not None
+
+
 def test_what_they_leave():
     a, b = _part(8, 96, 128, torch.bfloat16, True, 1), _part(8, 96, 128, torch.bfloat16, True, 2)
     assert L.few_rows_beside(a, b) is not None if not torch.is_grad_enabled() else L.few_rows_beside(a, b) is None
