@@ -39,7 +39,8 @@ from ..ops import _lib
 from ..ops import skinny_mm as smm
 from ..models.causal_lm import MLP, LayerNorm
 from ..ops.gemv import embed_ln_rows, ln_rows, ln_skinny_linear, skinny_linear
-from ..ops.linear import (FEW_ROWS, TLinear, few_rows_beside, few_rows_gelu, few_rows_head, few_rows_scratch, few_rows_sum)
+from ..ops.linear import (FEW_ROWS, TLinear, few_rows_beside, few_rows_gelu, few_rows_head, few_rows_scratch, few_rows_serve,
+                          few_rows_sum)
 from ..ops.norms import layer_norm_rows
 from ..utils import capture
 
@@ -790,8 +791,10 @@ class ModelRunner(StepRunner):
         # fp16 takes the same caps since the per-projection path's LayerNorm / GELU run their fp16
         # instantiations (ln_rows, kca_gelu_fwd_f16) instead of eager kernels: BLOOM rank 13.38 vs 14.84 per-projection
         # vs matrix-core layer at 32 (profiles/decode_fp16_cap_ab_r6.jsonl)
-        self._batched_max_b = int(os.environ.get("KCA_DECODE_BATCHED_MAX_B", "0")) or \
-            {"gptj": 1 if self._rows_ok else 16, "seq": 16}.get(self._layer_kind, 64)
+        forced = int(os.environ.get("KCA_DECODE_BATCHED_MAX_B", "0"))
+        self._batched_max_b = forced or {"gptj": 1 if self._rows_ok else 16, "seq": 16}.get(self._layer_kind, 64)
+        # where the products of few rows do not serve a step (_rows_serve): as without them
+        self._declined_max_b = 16 if self._rows_ok and not forced else 0
 
     # ------------------------------------------------------------- prefill
     @torch.no_grad()
@@ -1217,12 +1220,22 @@ class ModelRunner(StepRunner):
             logits = gather_last_dim(logits, grp)
         return logits
 
+    def _rows_serve(self, B: int) -> bool:
+        """Whether _layers_decode_rows takes a step of B rows: a matter of the weights' sizes and types and of torch's modes."""
+        if not (self._rows_ok and self._batched_ok and self._batched_max_b < B <= FEW_ROWS):
+            return False
+        for blk in self.model.h:
+            lin = (blk.attn.qkv, blk.attn.out, blk.mlp.fc_in, blk.mlp.fc_out)
+            if not few_rows_serve(B, [(x.weight, x.bias) for x in lin], blk.mlp.approx) or lin[1].weight.shape[0] != lin[3].weight.shape[0]:
+                return False
+        return True
+
     def _layers_decode_rows(self, tokens, pos, slots, kv_lens, max_kv, ws, obuf):
         """Decode step of GPT-J layers at batch 2 to FEW_ROWS (see _rows_ok): QKV and fc_in (GELU on its sums) in one launch of the
         weight-streaming kernel, attention, then fc_out, out and the residual rows in one, rounded once, and the norm. (Error of a step's logits
         against 64 bits, four layers of 4096: 8 rows 0.00647, the matrix-core layer 0.00647, with the residual rows added by the norm 0.00691; 32 rows
         0.00611, a launch a product 0.00682.) One queue: the feed-forward on a side stream beside the attention costs a fork and a join a layer (32 rows, 700 behind 824 us, this 793, both with ordinary loads).
-        None: sizes or a mode that the kernel does not serve; nothing has run then but the step's head."""
+        For steps that _rows_serve takes."""
         m, cfg = self.model, self.cfg
         B = tokens.shape[0]
         sc = self._fz.get(("rows", B))
@@ -1236,15 +1249,13 @@ class ModelRunner(StepRunner):
             at, mlp = blk.attn, blk.mlp
             pair = few_rows_beside((xn, at.qkv.weight, at.qkv.bias), (xn, mlp.fc_in.weight, mlp.fc_in.bias), mlp.approx, sc)
             if pair is None:
-                if li == 0:
-                    return None
-                raise RuntimeError("decode layer of few rows: shape support changed between layers")
+                raise RuntimeError("decode layer of few rows: shape support changed within a step")
             o = dops.decode_prep_attention(pair[0], self.H, self.Hkv, self.D, self.rot, cfg.rotary_interleaved, cos, sin, pos, slots,
                                            self.cache.k[li], self.cache.v[li], kv_lens, max_kv, at.scale, at.alibi, out=obuf, ws=ws,
                                            block_table=tbl, window=at.window, by_row=by_row)
             h = few_rows_sum((pair[1], mlp.fc_out.weight, mlp.fc_out.bias), (o, at.out.weight, at.out.bias), sc, h)
             if h is None:
-                raise RuntimeError("decode layer of few rows: shape support changed within a layer")
+                raise RuntimeError("decode layer of few rows: shape support changed within a step")
             ln = m.h[li + 1].ln_1 if li + 1 < len(m.h) else m.ln_f
             xn, _ = ln_rows(h, ln.weight, ln.bias, ln.eps)
         w, b, _ = self._head_weight()
@@ -1257,14 +1268,12 @@ class ModelRunner(StepRunner):
             if y is not None:
                 self.fused_steps += 1
                 return y
-        if (self._batched_ok and 2 <= tokens.shape[0] <= min(smm.MAX_M, self._batched_max_b) and obuf is not None
+        if tokens.shape[0] > 1 and obuf is not None and self._rows_serve(tokens.shape[0]):
+            self.rows_steps += 1
+            return self._layers_decode_rows(tokens, pos, slots, kv_lens, max_kv, ws, obuf)
+        if (self._batched_ok and 2 <= tokens.shape[0] <= min(smm.MAX_M, max(self._batched_max_b, self._declined_max_b)) and obuf is not None
                 and (self._chain_src is None or self._embed_head)):
             return self._layers_decode_batched(tokens, pos, slots, kv_lens, max_kv, ws, obuf)
-        if self._rows_ok and 1 < tokens.shape[0] <= FEW_ROWS and obuf is not None:
-            y = self._layers_decode_rows(tokens, pos, slots, kv_lens, max_kv, ws, obuf)
-            if y is not None:
-                self.rows_steps += 1
-                return y
         if self._chain_src is not None and obuf is not None:  # chained rows not resolved by a fused head
             chain, prev = self._chain_src
             tokens = torch.where(chain[:tokens.shape[0]] >= 0, prev[chain[:tokens.shape[0]].clamp(min=0).long()],

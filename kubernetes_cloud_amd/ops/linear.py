@@ -262,12 +262,22 @@ def linear_rows(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None
 ACTS = {None: 0, "tanh": 1, "none": 2}  # none, GELU (tanh form, erf form)
 
 
-def _few_part(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, rows: int) -> bool:
+def _few_weight(weight: torch.Tensor, bias: torch.Tensor | None, rows: int) -> bool:
     n, k = weight.shape
-    return (few_rows(rows, n, k) and x.dtype in (torch.bfloat16, torch.float16) and x.dtype == weight.dtype
-            and x.numel() == rows * k and x.is_contiguous() and weight.is_contiguous() and n % 16 == 0 and k % 64 == 0
-            and 2 * max(n, rows) * k < 1 << 32 and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
-            and (bias is None or (bias.shape == (n,) and bias.dtype == x.dtype and bias.is_contiguous())))
+    return (few_rows(rows, n, k) and weight.dtype in (torch.bfloat16, torch.float16) and weight.is_contiguous() and n % 16 == 0
+            and n > 0 < k and k % 64 == 0 and 2 * max(n, rows) * k < 1 << 32 and weight.data_ptr() % 16 == 0
+            and (bias is None or (bias.shape == (n,) and bias.dtype == weight.dtype and bias.is_contiguous())))
+
+
+def _few_part(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, rows: int) -> bool:
+    return (_few_weight(weight, bias, rows) and x.dtype == weight.dtype and x.numel() == rows * weight.shape[1] and x.is_contiguous()
+            and x.data_ptr() % 16 == 0)
+
+
+def few_rows_serve(rows: int, products, approx: str | None = None) -> bool:
+    """Whether these (weight, bias) go to the weight-streaming kernel for ``rows`` fresh rows, with this GELU, before anything is launched."""
+    return (0 < rows <= FEW_ROWS and approx in ACTS and all(_few_weight(w, b, rows) for w, b in products)
+            and _lib.inference(*(t for p in products for t in p)) and _lib.has("kca_rows_mm_two"))
 
 
 def few_rows_scratch(rows: int, device: torch.device) -> tuple[torch.Tensor, torch.Tensor]:

@@ -1036,7 +1036,7 @@ def test_engine_batched_mfma_layer(preset, B):
     previous tail's row statistics, [QKV | fc_in] / K-concatenated out-proj + fc_out launches for the
     parallel-residual kinds, ALiBi + embedding LayerNorm for BLOOM, learned positions and an odd
     vocabulary for GPT-2), HIP graphs on: every row's greedy tokens match a full forward of its own
-    continuation, and so do the per-projection path's."""
+    continuation, and so do the per-projection path's (GPT-J's with the feed-forward on a side stream among them)."""
     from kubernetes_cloud_amd.engine.llm_engine import LLMEngine, SamplingParams
     over = {"gpt-j-6b": dict(n_embd=1024, n_layer=3, n_head=4, rotary_dim=64, n_positions=512)}.get(preset)
     if over:
@@ -1057,7 +1057,7 @@ def test_engine_batched_mfma_layer(preset, B):
         eng.runner._batched_ok = batched
         eng.runner._batched_max_b = 64  # (the layer at every bucket, whatever the per-kind dispatch cap)
         outs = [r.output for r in eng.generate(prompts, sp)]
-        assert (eng.runner.batched_steps > 0) == batched
+        assert (eng.runner.batched_steps > 0) == batched and eng.runner.rows_steps == 0
         for p, o in zip(prompts, outs):
             _check_against_forward(m, p, o)
 
@@ -1066,7 +1066,8 @@ def test_engine_batched_mfma_layer(preset, B):
 def test_engine_fp16_native_decode(preset, monkeypatch):
     """fp16 serving (the precision of BASELINE config 4's FasterTransformer /
     DS-Inference rows) runs the native decode step -- the fused GEMV layer at batch 1, the matrix-core
-    layer at batch > 1, the fp16 attention / LayerNorm-row / embedding-head instantiations and the sampler
+    layer (GPT-J: the products of few rows, and without them the matrix-core layer) at batch > 1, the per-projection
+    path above its cap, the fp16 attention / LayerNorm-row / embedding-head instantiations and the sampler
     reading fp16 logits -- with HIP graphs: the PyTorch fallbacks of the decode attention and the sampler
     are made to fail, greedy tokens match a full fp16 forward, and seeded sampling is reproducible."""
     from kubernetes_cloud_amd.engine.llm_engine import LLMEngine, SamplingParams
@@ -1088,17 +1089,21 @@ def test_engine_fp16_native_decode(preset, monkeypatch):
     from kubernetes_cloud_amd.ops import gemv as gmod
     monkeypatch.setattr(gmod, "_act_ref", boom)  # the per-projection path's GELU: fp16 kernel, not eager
     g = torch.Generator().manual_seed(3)
-    for B in (1, 5, 20):  # 20: above the GPT-J / BLOOM matrix-core cap -> the per-projection path in fp16
+    # 20: above the GPT-J / BLOOM matrix-core cap -> the per-projection path in fp16; GPT-J with and without its products of few rows
+    for B, few in [(1, True), (5, True), (20, True)] + [(5, False), (20, False)] * (preset == "gpt-j-6b"):
         prompts = [[int(x) for x in torch.randint(0, 1000, (30 + 7 * (i % 5),), generator=g)] for i in range(B)]
         eng = LLMEngine(m, max_slots=B, max_len=256, use_graphs=True)
-        assert eng.runner._batched_ok
+        assert eng.runner._batched_ok and eng.runner._rows_ok == (preset == "gpt-j-6b")
+        eng.runner._rows_ok &= few
         outs = [r.output for r in eng.generate(prompts, SamplingParams(max_new_tokens=12, do_sample=False))]
         if B == 1:
             assert eng.runner.fused_steps > 0
-        elif B <= eng.runner._batched_max_b:
-            assert eng.runner.batched_steps > 0
+        elif eng.runner._rows_ok:
+            assert eng.runner.rows_steps > 0 and eng.runner.batched_steps == 0
         else:
-            assert eng.runner.batched_steps == 0
+            cap = max(eng.runner._batched_max_b, eng.runner._declined_max_b)
+            assert (eng.runner.batched_steps > 0) == (B <= cap) and eng.runner.rows_steps == 0
+            assert B <= cap or preset != "gpt-neox-20b"
         for p, o in zip(prompts, outs):
             _check_against_forward(m, p, o)
         sp = SamplingParams(max_new_tokens=8, do_sample=True, temperature=0.9, top_k=40, top_p=0.9, seed=17)
@@ -1170,6 +1175,33 @@ def test_engine_gptj_rows_layer(dtype, B, width):
     assert eng.runner.rows_steps > 0 and eng.runner.batched_steps == 0 and not eng.runner._packs
     for p, o in zip(prompts, outs):
         _check_against_forward(m, p, o)
+
+
+@pytest.mark.parametrize("how,B", [("sizes", 5), ("sizes", 26), ("autocast", 5), ("autocast", 26)])
+def test_gptj_rows_layer_declines(monkeypatch, how, B):
+    """A step that the products of few rows do not serve is known for one before anything is launched, and goes where it went without them:
+    the matrix-core layer up to 16 rows, then a launch a projection. (Outputs past 16384 are theirs up to 24 rows.)"""
+    import contextlib
+
+    from kubernetes_cloud_amd.engine import runner as R
+    from kubernetes_cloud_amd.models.causal_lm import build_model
+    from kubernetes_cloud_amd.models.config import PRESETS_HF, LMConfig
+    cfg = dict(PRESETS_HF["gpt-j-6b"])
+    cfg.update(n_embd=512, n_layer=2, n_head=2, rotary_dim=64, n_positions=512, n_inner=16448 if how == "sizes" else 2048)
+    m = build_model(LMConfig.from_hf(cfg), device=dev, dtype=torch.bfloat16, seed=0).requires_grad_(False)
+    r = R.ModelRunner(m, max_slots=B, max_len=256)
+    ids = torch.randint(0, 1000, (B, 30), generator=torch.Generator().manual_seed(B))
+    r.prefill(ids[:, :29], list(range(B)), [29] * B)
+    heads, f = [], R.embed_ln_rows
+    monkeypatch.setattr(R, "embed_ln_rows", lambda *a, **k: heads.append(1) or f(*a, **k))
+    rows = [dict(token=int(ids[i, 29]), pos=29, slot=i, temperature=0.0, top_k=1, top_p=1.0, rep=1.0, seed=i) for i in range(B)]
+    with torch.autocast("cuda", dtype=torch.bfloat16) if how == "autocast" else contextlib.nullcontext():
+        h = r.decode_async(rows)
+    torch.cuda.synchronize()
+    assert (r.rows_steps > 0) == (how == "sizes" and B <= 24) and (r.batched_steps > 0) == (how == "autocast" and B <= 16)
+    assert len(heads) == r.rows_steps + r.batched_steps
+    for i in range(B):
+        _check_against_forward(m, ids[i].tolist(), [int(h.ids_dev[i])])
 
 
 @pytest.mark.parametrize("rows", [2, 32, 33, 64, 65])
