@@ -195,7 +195,7 @@ __device__ __forceinline__ void rope8(const bf16_t* __restrict__ row, int d0, fl
       sgn = d < half ? -1.f : 1.f;
     }
     const float c = cos_t[(long long)pos * half + fi], sn = sin_t[(long long)pos * half + fi];
-    x[j] = e2f<DT>(f2e<DT>(x[j] * c + sgn * e2f<DT>(row[partner]) * sn));
+    x[j] = e2f<DT>(f2e<DT>(fmaf(x[j], c, sgn * e2f<DT>(row[partner]) * sn)));
   }
 }
 
@@ -215,12 +215,25 @@ __device__ __forceinline__ void rope_tab8(const float* __restrict__ cos_t, const
   }
 }
 
-// rope8 with the angles in registers (rope_tab8); interleaved pairs take the partner from the
-// lane's own raw values, rotate-half partners are read from the unrotated row as rope8 does.
+// The partners of dims [d0, d0+8) of a row whose halves rotate, d0 < rot
+__device__ __forceinline__ U16x8 rope_other8(const bf16_t* __restrict__ row, int d0, int rot) {
+  const int half = rot >> 1;
+  if (half % 8 == 0) return *reinterpret_cast<const U16x8*>(row + (d0 < half ? d0 + half : d0 - half));
+  U16x8 v;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int d = min(d0 + j, rot - 1);
+    v.v[j] = (uint16_t)row[d < half ? d + half : d - half];
+  }
+  return v;
+}
+
+// rope8 with the angles (rope_tab8) and, of rotated halves, the partners (rope_other8) in registers; interleaved pairs take them from the
+// lane's own raw values. (Partners read here, each behind a wait of its own and all behind the angles: 20 sequences of 300 tokens, 16 heads of 64,
+// rot 32, us, all in rope8, angles ahead, both ahead 14.2, 13.3, 11.4; 64 of 700, of 128, 74.9, 64.0, 59.0.)
 template <int DT = 0>
-__device__ __forceinline__ void rope8_reg(const bf16_t* __restrict__ row, int d0, float (&x)[8],
-                                          const float (&raw)[8], const float (&c)[8], const float (&sn)[8],
-                                          int rot, int interleaved) {
+__device__ __forceinline__ void rope8_reg(int d0, float (&x)[8], const float (&raw)[8], const U16x8& other, const float (&c)[8],
+                                          const float (&sn)[8], int rot, int interleaved) {
   const int half = rot >> 1;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
@@ -231,10 +244,10 @@ __device__ __forceinline__ void rope8_reg(const bf16_t* __restrict__ row, int d0
       pv = raw[j ^ 1];
       sgn = (d & 1) ? 1.f : -1.f;
     } else {
-      pv = e2f<DT>(row[d < half ? d + half : d - half]);
+      pv = e2f<DT>(other.v[j]);
       sgn = d < half ? -1.f : 1.f;
     }
-    x[j] = e2f<DT>(f2e<DT>(x[j] * c[j] + sgn * pv * sn[j]));
+    x[j] = e2f<DT>(f2e<DT>(fmaf(x[j], c[j], sgn * pv * sn[j])));  // (as decode_prep_kernel rounds, however it is compiled)
   }
 }
 
@@ -351,6 +364,9 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
   const bf16_t* krow = p.q + b * p.q_bs + (long long)(p.H + hk) * D;
   const bf16_t* vrow = p.q + b * p.q_bs + (long long)(p.H + p.Hkv + hk) * D;
   U16x8 knraw, vnraw;  // the new token's K / V slice of lane tid (< ND), from the fused QKV row
+  const bool rope = p.fused && p.rot > 0;
+  const bool angles = rope && (PF || (p.by_row & 1));  // in rc and rs; rotated halves' partners in qother and kother
+  U16x8 qother[G], kother;
   auto load_qkv_rows = [&]() {
 #pragma unroll
     for (int g = 0; g < G; ++g)
@@ -359,11 +375,14 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
       knraw = *reinterpret_cast<const U16x8*>(krow + tid * 8);
       vnraw = *reinterpret_cast<const U16x8*>(vrow + tid * 8);
     }
+    if (angles && !p.interleaved && dslot * 8 < p.rot) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) qother[g] = rope_other8(p.q + b * p.q_bs + (long long)(hk * G + g) * D, dslot * 8, p.rot);
+      if (tid < ND) kother = rope_other8(krow, dslot * 8, p.rot);
+    }
   };
   load_qkv_rows();
   // per-step RoPE row (by_row bit 0): the angles do not wait for the length
-  const bool rope = p.fused && p.rot > 0;
-  const bool angles = rope && (PF || (p.by_row & 1));  // in rc and rs
   float rc[8], rs[8];
   if ((p.by_row & 1) && rope && dact) rope_tab8(p.cos_t, p.sin_t, b, dslot * 8, p.rot, p.interleaved, rc, rs);
   // paged: this split's page ids staged in LDS (chunk <= 1024 tokens, pages >= 16 tokens), so a
@@ -411,7 +430,7 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
         float raw[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) raw[j] = q[g][j];
-        rope8_reg<DT>(p.q + b * p.q_bs + (long long)(hk * G + g) * D, dslot * 8, q[g], raw, rc, rs, p.rot, p.interleaved);
+        rope8_reg<DT>(dslot * 8, q[g], raw, qother[g], rc, rs, p.rot, p.interleaved);
       } else if (rope) {
         rope8<DT>(p.q + b * p.q_bs + (long long)(hk * G + g) * D, dslot * 8, q[g], pnew, p.rot, p.interleaved, p.cos_t,
               p.sin_t);
@@ -461,7 +480,7 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
       float raw[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) raw[j] = kx[j];
-      rope8_reg<DT>(krow, tid * 8, kx, raw, rc, rs, p.rot, p.interleaved);
+      rope8_reg<DT>(tid * 8, kx, raw, kother, rc, rs, p.rot, p.interleaved);
     } else if (rope) {
       rope8<DT>(krow, tid * 8, kx, pnew, p.rot, p.interleaved, p.cos_t, p.sin_t);
     }
@@ -516,10 +535,6 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
       kk[u] = load_row<ONCE>(kb + o[u]);
       vv[u] = load_row<ONCE>(vb + o[u]);
     }
-    if constexpr (PF) {  // hipcc moves loads that only the next round of a loop uses into that round, or behind the other set's sums
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-    }
   };
   // the U scores of an iteration are independent (their lane-group sums overlap), then ONE
   // online-softmax update folds them in: the dependent chain per iteration is one reduction and
@@ -568,14 +583,20 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
     // on their way, in registers of their own: moved from one set to the other, the move waits for rows that have only just been
     // requested, and the next request for them. 16 heads of 256, cold, us, with the move and so: 32 sequences of 700 to 917 95, 86 (4.9 TB/s);
     // 24 of 100 to 261 27.3, 23.5; 16 of 400 to 505 35.1, 29.9; 13 of 60 to 144 16.8, 12.6; 64 of 300 to 741 124, 111.
+    auto request = [&](int tb, U16x8 (&kk)[U], U16x8 (&vv)[U]) {
+      load_kv(tb, kk, vv);
+      // hipcc moves loads that only the next round of a loop uses into that round, or behind the other set's sums
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    };
     U16x8 kx0[U], vx0[U], kx1[U], vx1[U];
-    load_kv(ts, kx0, vx0);
-    load_kv(ts + TPB * U, kx1, vx1);
+    request(ts, kx0, vx0);
+    request(ts + TPB * U, kx1, vx1);
     for (int t0 = ts; t0 < ce; t0 += 2 * TPB * U) {
       fold(t0, kx0, vx0);
-      load_kv(t0 + 2 * TPB * U, kx0, vx0);
+      request(t0 + 2 * TPB * U, kx0, vx0);
       if (t0 + TPB * U < ce) fold(t0 + TPB * U, kx1, vx1);  // (without a token of its own it has one's infinite V times 0)
-      load_kv(t0 + 3 * TPB * U, kx1, vx1);
+      request(t0 + 3 * TPB * U, kx1, vx1);
     }
   } else {
     for (int t0 = ts; t0 < ce; t0 += TPB * U) {

@@ -496,6 +496,37 @@ def test_decode_one_pass_walk_edges(D, Hkv, G, PS, window):
         assert ((got.double().cpu().view(B, H, D) - want).abs() <= want.abs() * 2 ** -8 + 1e-4).all()
 
 
+@pytest.mark.parametrize("D,rot,inter,G,f16", [(64, 16, False, 1, False), (64, 64, False, 1, True), (96, 24, False, 1, False), (128, 32, False, 1, False),
+                                               (256, 20, False, 1, True), (256, 4, False, 2, False), (256, 64, True, 1, True)])
+def test_decode_rotation_walks(D, rot, inter, G, f16, monkeypatch):
+    """One launch is the rotation's and the attention's two, bit for bit, where a walk takes one round, two or more: halves of 16-byte pieces and of odd
+    sizes, angles by position and by the step's rows."""
+    monkeypatch.setattr(dops, "decode_chunk", lambda *a: 448)
+    torch.manual_seed(D + rot)
+    lens = [1, 2, 31, 33, 64, 65, 66, 127, 128, 129, 130, 257, 258, 385, 448]
+    dt = torch.float16 if f16 else torch.bfloat16
+    B, Hkv, L, H = len(lens), 2, 448, 2 * G
+    kc, tbl = _paginate(torch.randn(B, Hkv, L, D, device=dev).to(dt), 64, 5)
+    vc, _ = _paginate(torch.randn(B, Hkv, L, D, device=dev).to(dt), 64, 5)
+    qkv = torch.randn(B, (H + 2 * Hkv) * D, device=dev).to(dt)
+    slots, kl = torch.arange(B, device=dev, dtype=torch.int32), torch.tensor(lens, device=dev, dtype=torch.int32)
+    cos, sin = rope_tables(rot, L, 10000.0, dev)
+    pos = kl - 1
+    k1, v1, q1 = kc.clone(), vc.clone(), qkv.clone()
+    dops.decode_prep(q1, H, Hkv, D, rot, inter, cos, sin, pos, slots, k1, v1, block_table=tbl)
+    outs = []
+    for by_row in (0, 1):
+        c, s = (cos[pos.long()].contiguous(), sin[pos.long()].contiguous()) if by_row else (cos, sin)
+        k2, v2 = kc.clone(), vc.clone()
+        o = dops.decode_prep_attention(qkv, H, Hkv, D, rot, inter, c, s, pos, slots, k2, v2, kl, L, block_table=tbl, by_row=by_row)
+        outs.append(o)
+        # (fp16's two steps are torch's, which rounds each product: an ulp, where the sum cancels one of the products')
+        assert torch.equal(v1, v2) and (((k1 - k2).abs() <= 2 ** -9 * k1.abs().max()).all() if f16 else torch.equal(k1, k2))
+    assert torch.equal(*outs)
+    if not f16:
+        assert torch.equal(outs[0], dops.decode_attention(q1, k1, v1, slots, kl, H, L, block_table=tbl, chunk=L))
+
+
 @pytest.mark.parametrize("D,n", [(256, 33), (256, 97), (256, 161), (96, 65), (96, 193), (64, 129), (64, 385), (128, 193)])
 def test_decode_infinite_values(D, n):
     """An infinite value in the last cached row stays one: no group of lanes has it times the weight 0 of a token that is not there, after an odd number
