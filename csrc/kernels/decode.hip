@@ -526,14 +526,14 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
   // inactive lanes (dslot >= ND) and tokens past the split read an in-range row instead of branching
   // around their loads: no branch in the loop, so all 2U loads of an iteration are in flight together
   const long long dfix = dact ? 0 : -(long long)dslot * 8;
-  auto load_kv = [&](int tb, U16x8 (&kk)[U], U16x8 (&vv)[U]) {
+  auto load_kv = [&](auto kind, int tb, U16x8 (&kk)[U], U16x8 (&vv)[U]) {
     long long o[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) o[u] = toff(min(tb + u * TPB, max(ce - 1, ca))) + dfix;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      kk[u] = load_row<ONCE>(kb + o[u]);
-      vv[u] = load_row<ONCE>(vb + o[u]);
+      kk[u] = load_row<decltype(kind)::value>(kb + o[u]);
+      vv[u] = load_row<decltype(kind)::value>(vb + o[u]);
     }
   };
   // the U scores of an iteration are independent (their lane-group sums overlap), then ONE
@@ -583,25 +583,37 @@ __device__ __forceinline__ void decode_attn_body(const DecodeParams& p, const in
     // on their way, in registers of their own: moved from one set to the other, the move waits for rows that have only just been
     // requested, and the next request for them. 16 heads of 256, cold, us, with the move and so: 32 sequences of 700 to 917 95, 86 (4.9 TB/s);
     // 24 of 100 to 261 27.3, 23.5; 16 of 400 to 505 35.1, 29.9; 13 of 60 to 144 16.8, 12.6; 64 of 300 to 741 124, 111.
-    auto request = [&](int tb, U16x8 (&kk)[U], U16x8 (&vv)[U]) {
-      load_kv(tb, kk, vv);
-      // hipcc moves loads that only the next round of a loop uses into that round, or behind the other set's sums
-      asm volatile("" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-    };
-    U16x8 kx0[U], vx0[U], kx1[U], vx1[U];
-    request(ts, kx0, vx0);
-    request(ts + TPB * U, kx1, vx1);
-    for (int t0 = ts; t0 < ce; t0 += 2 * TPB * U) {
-      fold(t0, kx0, vx0);
-      request(t0 + 2 * TPB * U, kx0, vx0);
-      if (t0 + TPB * U < ce) fold(t0 + TPB * U, kx1, vx1);  // (without a token of its own it has one's infinite V times 0)
-      request(t0 + 3 * TPB * U, kx1, vx1);
+    // A walk of one or two rounds, whatever the bound that the launch knows, is short of what the two sets request past its end (three of four
+    // are nobody's) and of their code: the plain loop, through the caches, where the lanes that stand on the last row find it. us, one set ahead with moves, two
+    // sets, so, 16 heads: of 64, 64 sequences of 30 tokens 7.3, 9.1, 6.9; of 100 9.0, 10.5, 8.6; of 128, 20 of 60 6.4, 7.3, 6.1; of 256, 64 of 30
+    // 7.5, 10.9, 7.2, of 60 14.4, 13.9, 13.6. Steps of NeoX layers 1024 wide, 8 of them, 64 rows of 100: 547, 594, 542.
+    if (ce - ca <= 2 * TPB * U) {
+      for (int t0 = ts; t0 < ce; t0 += TPB * U) {
+        U16x8 kr[U], vr[U];
+        load_kv(std::false_type{}, t0, kr, vr);
+        fold(t0, kr, vr);
+      }
+    } else {
+      auto request = [&](int tb, U16x8 (&kk)[U], U16x8 (&vv)[U]) {
+        load_kv(std::integral_constant<bool, ONCE>{}, tb, kk, vv);
+        // hipcc moves loads that only the next round of a loop uses into that round, or behind the other set's sums
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      U16x8 kx0[U], vx0[U], kx1[U], vx1[U];
+      request(ts, kx0, vx0);
+      request(ts + TPB * U, kx1, vx1);
+      for (int t0 = ts; t0 < ce; t0 += 2 * TPB * U) {
+        fold(t0, kx0, vx0);
+        request(t0 + 2 * TPB * U, kx0, vx0);
+        if (t0 + TPB * U < ce) fold(t0 + TPB * U, kx1, vx1);  // (without a token of its own it has one's infinite V times 0)
+        request(t0 + 3 * TPB * U, kx1, vx1);
+      }
     }
   } else {
     for (int t0 = ts; t0 < ce; t0 += TPB * U) {
       U16x8 kr[U], vr[U];
-      load_kv(t0, kr, vr);
+      load_kv(std::integral_constant<bool, ONCE>{}, t0, kr, vr);
       fold(t0, kr, vr);
     }
   }
