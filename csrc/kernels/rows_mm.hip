@@ -147,8 +147,11 @@ __global__ void __launch_bounds__(64 * W, 2) rows_mm_kernel(RowsArgs p) {
     const int k = (one ? tt : tt - nka) * SK * 2;
     const __amdgpu_buffer_rsrc_t fw = one ? rw : rw2, fx = one ? rx : rx2;
     // (the weights non-temporal: no other block reads them. 32 rows, cold, us: 12288 and 16384 x 4096 42.6, 37.8 (6.2 TB/s); 4096 x 16384 and x 4096
-    // 34.7, 30.2; 50400 x 4096 82.8, 75.6; 61 rows 43.8, 40.1; 38.6, 37.2; 86.5, 81.7. Called again with nothing between, weights that the last
-    // cache would hold come slower: 50400 x 1024 19.5, 21.9)
+    // 34.7, 30.2; 50400 x 4096 82.8, 75.6; 61 rows 43.8, 40.1; 38.6, 37.2; 86.5, 81.7. Called over and over with nothing
+    // else between, weights that the last cache (256 MB) would hold come slower, 180 MB of 2304 x 768 at 61 rows 6.2, 7.1, of 50304 x 768 16.1, 21.0; cold
+    // they gain nothing below 2048 of width. But whole steps of models that small, which read a cache and logits too, are no faster with ordinary loads
+    // of weights less than 2048 wide: GPT-J layers, 12 of 768 with their head, 16 rows of 100 tokens 404, 390; 64 506, 509; 128 of 200 703, 709; 8 of 1024 317,
+    // 315; 386, 383; 594, 577; GPT-2's prompts of 16 to 120 tokens are bound by the host.)
 #pragma unroll
     for (int i = 0; i < WI; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(fw, (void __attribute__((address_space(3)))*)(st + (wv * WI + i) * 1024), 16,
