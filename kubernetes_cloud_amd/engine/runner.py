@@ -936,15 +936,8 @@ class ModelRunner(StepRunner):
                 raise RuntimeError("rope_append: the projection's rows are not 16-byte aligned")
             o = ops.packed_attention(q, k, v, cu, longest, at.scale, at.alibi, at.window).view(1, rows, -1)
             if pair is not None:
-                # h in the same sums, rounded once (after the last layer, whose norm reads its sum unrounded, apart)
-                res = h if li + 1 < len(m.h) else None
-                y = few_rows_sum((pair[1], *plain[3]), (o, *plain[1]), res=res)
-                if y is None:
-                    pending = (at.out(o), mlp.fc_out(pair[1]))
-                elif res is None:
-                    pending = (y,)
-                else:
-                    h, pending = y, ()
+                y = few_rows_sum((pair[1], *plain[3]), (o, *plain[1]))
+                pending = (y,) if y is not None else (at.out(o), mlp.fc_out(pair[1]))
                 continue
             a = at.out(o)
             if cfg.parallel_residual:
@@ -1232,9 +1225,10 @@ class ModelRunner(StepRunner):
 
     def _layers_decode_rows(self, tokens, pos, slots, kv_lens, max_kv, ws, obuf):
         """Decode step of GPT-J layers at batch 2 to FEW_ROWS (see _rows_ok): QKV and fc_in (GELU on its sums) in one launch of the
-        weight-streaming kernel, attention, then fc_out, out and the residual rows in one, rounded once, and the norm. (Error of a step's logits
-        against 64 bits, four layers of 4096: 8 rows 0.00647, the matrix-core layer 0.00647, with the residual rows added by the norm 0.00691; 32 rows
-        0.00611, a launch a product 0.00682.) One queue: the feed-forward on a side stream beside the attention costs a fork and a join a layer (32 rows, 700 behind 824 us, this 793, both with ordinary loads).
+        weight-streaming kernel, attention, then fc_out and out in one, and the norm. Up to 16 rows the residual rows enter that launch's sums, which
+        are rounded once, as the matrix-core layer has them (error of a step's logits against 64 bits, four layers of 4096, 8 rows: 0.00647, that layer 0.00647, the
+        products' sum rounded before the norm adds the residual rows 0.00691). More rows keep the norm's addition, no less exact than the launch a product that
+        serves them otherwise (32 rows 0.00659, 0.00682). One queue: the feed-forward on a side stream beside the attention costs a fork and a join a layer (32 rows, 700 behind 824 us, this 793, both with ordinary loads).
         For steps that _rows_serve takes."""
         m, cfg = self.model, self.cfg
         B = tokens.shape[0]
@@ -1253,11 +1247,15 @@ class ModelRunner(StepRunner):
             o = dops.decode_prep_attention(pair[0], self.H, self.Hkv, self.D, self.rot, cfg.rotary_interleaved, cos, sin, pos, slots,
                                            self.cache.k[li], self.cache.v[li], kv_lens, max_kv, at.scale, at.alibi, out=obuf, ws=ws,
                                            block_table=tbl, window=at.window, by_row=by_row)
-            h = few_rows_sum((pair[1], mlp.fc_out.weight, mlp.fc_out.bias), (o, at.out.weight, at.out.bias), sc, h)
-            if h is None:
+            y = few_rows_sum((pair[1], mlp.fc_out.weight, mlp.fc_out.bias), (o, at.out.weight, at.out.bias), sc, h if B <= 16 else None)
+            if y is None:
                 raise RuntimeError("decode layer of few rows: shape support changed within a step")
             ln = m.h[li + 1].ln_1 if li + 1 < len(m.h) else m.ln_f
-            xn, _ = ln_rows(h, ln.weight, ln.bias, ln.eps)
+            if B <= 16:
+                h = y
+                xn, _ = ln_rows(h, ln.weight, ln.bias, ln.eps)
+            else:
+                xn, h = ln_rows(h, ln.weight, ln.bias, ln.eps, (y,))
         w, b, _ = self._head_weight()
         return few_rows_head(xn, w, b)
 

@@ -1208,6 +1208,27 @@ def test_engine_gptj_rows_layer(dtype, B, width):
         _check_against_forward(m, p, o)
 
 
+@pytest.mark.parametrize("B,once", [(2, True), (16, True), (17, False), (33, False)])
+def test_gptj_rows_layer_residual(monkeypatch, B, once):
+    """Up to 16 rows a layer's residual rows enter the products' sums, which are rounded once; past them the norm adds them to the rounded sum."""
+    from kubernetes_cloud_amd.engine import runner as R
+    from kubernetes_cloud_amd.models.causal_lm import build_model
+    from kubernetes_cloud_amd.models.config import PRESETS_HF, LMConfig
+    cfg = dict(PRESETS_HF["gpt-j-6b"])
+    cfg.update(n_embd=512, n_layer=2, n_head=2, rotary_dim=64, n_positions=512)
+    m = build_model(LMConfig.from_hf(cfg), device=dev, dtype=torch.bfloat16, seed=0).requires_grad_(False)
+    r = R.ModelRunner(m, max_slots=B, max_len=256, use_graphs=False)
+    ids = torch.randint(0, 1000, (B, 30), generator=torch.Generator().manual_seed(B))
+    r.prefill(ids[:, :29], list(range(B)), [29] * B)
+    res, f = [], R.few_rows_sum
+    monkeypatch.setattr(R, "few_rows_sum", lambda a, b, sc, h: res.append(h is not None) or f(a, b, sc, h))
+    h = r.decode_async([dict(token=int(ids[i, 29]), pos=29, slot=i, temperature=0.0, top_k=1, top_p=1.0, rep=1.0, seed=i) for i in range(B)])
+    torch.cuda.synchronize()
+    assert r.rows_steps > 0 and res == [once] * 2
+    for i in range(B):
+        _check_against_forward(m, ids[i].tolist(), [int(h.ids_dev[i])])
+
+
 @pytest.mark.parametrize("how,B", [("sizes", 5), ("sizes", 26), ("autocast", 5), ("autocast", 26)])
 def test_gptj_rows_layer_declines(monkeypatch, how, B):
     """A step that the products of few rows do not serve is known for one before anything is launched, and goes where it went without them:
