@@ -1067,7 +1067,7 @@ def test_engine_batched_mfma_layer(preset, B):
     previous tail's row statistics, [QKV | fc_in] / K-concatenated out-proj + fc_out launches for the
     parallel-residual kinds, ALiBi + embedding LayerNorm for BLOOM, learned positions and an odd
     vocabulary for GPT-2), HIP graphs on: every row's greedy tokens match a full forward of its own
-    continuation, and so do the per-projection path's (GPT-J's with the feed-forward on a side stream among them)."""
+    continuation, and so do the per-projection path's."""
     from kubernetes_cloud_amd.engine.llm_engine import LLMEngine, SamplingParams
     over = {"gpt-j-6b": dict(n_embd=1024, n_layer=3, n_head=4, rotary_dim=64, n_positions=512)}.get(preset)
     if over:
@@ -1088,7 +1088,7 @@ def test_engine_batched_mfma_layer(preset, B):
         eng.runner._batched_ok = batched
         eng.runner._batched_max_b = 64  # (the layer at every bucket, whatever the per-kind dispatch cap)
         outs = [r.output for r in eng.generate(prompts, sp)]
-        assert (eng.runner.batched_steps > 0) == batched and eng.runner.rows_steps == 0
+        assert (eng.runner.batched_steps > 0) == batched
         for p, o in zip(prompts, outs):
             _check_against_forward(m, p, o)
 
@@ -1097,8 +1097,7 @@ def test_engine_batched_mfma_layer(preset, B):
 def test_engine_fp16_native_decode(preset, monkeypatch):
     """fp16 serving (the precision of BASELINE config 4's FasterTransformer /
     DS-Inference rows) runs the native decode step -- the fused GEMV layer at batch 1, the matrix-core
-    layer (GPT-J: the products of few rows, and without them the matrix-core layer) at batch > 1, the per-projection
-    path above its cap, the fp16 attention / LayerNorm-row / embedding-head instantiations and the sampler
+    layer at batch > 1, the fp16 attention / LayerNorm-row / embedding-head instantiations and the sampler
     reading fp16 logits -- with HIP graphs: the PyTorch fallbacks of the decode attention and the sampler
     are made to fail, greedy tokens match a full fp16 forward, and seeded sampling is reproducible."""
     from kubernetes_cloud_amd.engine.llm_engine import LLMEngine, SamplingParams
@@ -1120,27 +1119,53 @@ def test_engine_fp16_native_decode(preset, monkeypatch):
     from kubernetes_cloud_amd.ops import gemv as gmod
     monkeypatch.setattr(gmod, "_act_ref", boom)  # the per-projection path's GELU: fp16 kernel, not eager
     g = torch.Generator().manual_seed(3)
-    # 20: above the GPT-J / BLOOM matrix-core cap -> the per-projection path in fp16; GPT-J with and without its products of few rows
-    for B, few in [(1, True), (5, True), (20, True)] + [(5, False), (20, False)] * (preset == "gpt-j-6b"):
+    for B in (1, 5, 20):  # 20: above the GPT-J / BLOOM matrix-core cap -> the per-projection path in fp16
         prompts = [[int(x) for x in torch.randint(0, 1000, (30 + 7 * (i % 5),), generator=g)] for i in range(B)]
         eng = LLMEngine(m, max_slots=B, max_len=256, use_graphs=True)
-        assert eng.runner._batched_ok and eng.runner._rows_ok == (preset == "gpt-j-6b")
-        eng.runner._rows_ok &= few
+        assert eng.runner._batched_ok
         outs = [r.output for r in eng.generate(prompts, SamplingParams(max_new_tokens=12, do_sample=False))]
         if B == 1:
             assert eng.runner.fused_steps > 0
-        elif eng.runner._rows_ok:
-            assert eng.runner.rows_steps > 0 and eng.runner.batched_steps == 0
+        elif B <= eng.runner._batched_max_b:
+            assert eng.runner.batched_steps > 0
         else:
-            cap = max(eng.runner._batched_max_b, eng.runner._declined_max_b)
-            assert (eng.runner.batched_steps > 0) == (B <= cap) and eng.runner.rows_steps == 0
-            assert B <= cap or preset != "gpt-neox-20b"
+            assert eng.runner.batched_steps == 0
         for p, o in zip(prompts, outs):
             _check_against_forward(m, p, o)
         sp = SamplingParams(max_new_tokens=8, do_sample=True, temperature=0.9, top_k=40, top_p=0.9, seed=17)
         a = [r.output for r in eng.generate(prompts, sp)]
         b = [r.output for r in eng.generate(prompts, sp)]
         assert a == b and all(len(x) == 8 for x in a)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,layer", [(5, "rows"), (20, "rows"), (5, "matrix cores"), (3, "projections"), (20, "projections")])
+def test_engine_gptj_decode_layers(dtype, B, layer, monkeypatch):
+    """GPT-J steps with graphs on each of their three layers: the products of few rows; without them the matrix-core layer up to 16 rows; and a
+    launch a projection, with the feed-forward on a side stream, where the batched layers are off or the rows are more. No PyTorch GELU."""
+    from kubernetes_cloud_amd.engine.llm_engine import LLMEngine, SamplingParams
+    from kubernetes_cloud_amd.models.causal_lm import build_model
+    from kubernetes_cloud_amd.models.config import PRESETS_HF, LMConfig
+    from kubernetes_cloud_amd.ops import gemv as gmod
+    cfg = dict(PRESETS_HF["gpt-j-6b"])
+    cfg.update(n_embd=1024, n_layer=3, n_head=4, rotary_dim=64, n_positions=512)
+    m = build_model(LMConfig.from_hf(cfg), device=dev, dtype=dtype, seed=0)
+
+    def boom(*a, **k):
+        raise AssertionError("decode fell back to PyTorch")
+    monkeypatch.setattr(gmod, "_act_ref", boom)
+    g = torch.Generator().manual_seed(3)
+    prompts = [[int(x) for x in torch.randint(0, 1000, (30 + 7 * (i % 5),), generator=g)] for i in range(B)]
+    eng = LLMEngine(m, max_slots=B, max_len=256, use_graphs=True)
+    assert eng.runner._batched_ok and eng.runner._rows_ok
+    if layer == "matrix cores":
+        eng.runner._rows_ok = False
+    elif layer == "projections":
+        eng.runner._batched_ok = False
+    outs = [r.output for r in eng.generate(prompts, SamplingParams(max_new_tokens=12, do_sample=False))]
+    assert (eng.runner.rows_steps > 0) == (layer == "rows") and (eng.runner.batched_steps > 0) == (layer == "matrix cores")
+    for p, o in zip(prompts, outs):
+        _check_against_forward(m, p, o)
 
 
 def test_engine_batched_mfma_bloom_tp_emulated_rank():

@@ -50,8 +50,15 @@ def test_few_rows(monkeypatch, dtype, rows, n, k, n2, k2):
     _both(monkeypatch, lambda: L.few_rows_beside(a, b, "tanh"), "few_rows")
     _both(monkeypatch, lambda: L.few_rows_gelu(*a, "none"), "few_rows")
     _both(monkeypatch, lambda: L.few_rows_sum(a, b), "few_rows" if n == n2 else None)
-    res = _rand(rows, n, dtype=dtype)
-    _both(monkeypatch, lambda: L.few_rows_sum(a, b, res=res), "few_rows" if n == n2 else None)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [1, 33, 128])
+@pytest.mark.parametrize("n,k,k2", [(16, 64, 64), (4096, 1024, 4096)])
+def test_few_rows_and_residual_rows(monkeypatch, dtype, rows, n, k, k2):
+    a = _rand(1, rows, k, dtype=dtype), _rand(n, k, dtype=dtype), _rand(n, dtype=dtype)
+    b, res = (_rand(rows, k2, dtype=dtype), _rand(n, k2, dtype=dtype), None), _rand(rows, n, dtype=dtype)
+    _both(monkeypatch, lambda: L.few_rows_sum(a, b, res=res), "few_rows")
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -108,11 +115,21 @@ def test_what_it_leaves(monkeypatch):
         class Sub(torch.Tensor):
             pass
         assert few(x.as_subclass(Sub)) is None and norm(x.as_subclass(Sub)) is None
+        assert torch.func.vmap(lambda t: layer_norm(t, x[0], None))(x[None].float()).shape == (1, 8, 128)
+
+
+def test_modes_it_leaves():
+    """Transforms, tracing, torch's modes and (few_rows) captures, on types that the module's functions take otherwise."""
+    ext = _lib.torch_ext()
+    x, w, b = _rand(8, 128), _rand(96, 128), _rand(96)
+    few = lambda x=x: ext.few_rows(x, w, b, None, None, None, 0, 0, False, 8)  # noqa: E731
+    norm = lambda x=x, w=_rand(128), r=None: ext.norm_rows(x, w, None, 1e-5, r, None)  # noqa: E731
+    with torch.no_grad():
+        assert few() is not None and norm() is not None
 
         def under(t):
             assert few(t) is None and norm(t) is None and norm(r=t) is None
             return t
-        # (the module's own functions, on types that they take otherwise)
         assert torch.equal(torch.func.vmap(under)(x[None]), x[None])
         torch.func.jvp(under, (x,), (x,))
         torch.jit.trace(under, (x,), check_trace=False)
